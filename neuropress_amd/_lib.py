@@ -12,6 +12,7 @@ import os
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libnpamd.so"
+HOST_PATH = LIB_PATH.with_name("npamd_host.so")
 
 F16, BF16, F32 = 0, 1, 2
 GEMV_MAX_M = 32
@@ -98,6 +99,30 @@ def load() -> ctypes.CDLL:
         raise RuntimeError(_load_error) from exc
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The extension module that issues the lowered modules' calls (loaded once; links ``libnpamd.so``)."""
+    global _host
+    if _host is None:
+        import importlib.machinery
+        import importlib.util
+
+        load()
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("npamd_host", os.fspath(HOST_PATH))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("npamd_host", loader))
+            loader.exec_module(module)
+        except ImportError as exc:
+            raise RuntimeError(f"neuropress_amd: cannot load {HOST_PATH}: {exc}; build it with `python -m neuropress_amd.build`") from exc
+        from . import kernels
+
+        module.set_workspaces(kernels._SLICED_WORKSPACES, kernels.drop_sliced_workspace_of)
+        _host = module
+    return _host
 
 
 def is_available() -> bool:

@@ -1,10 +1,12 @@
-"""Build ``libnpamd.so`` (HIP kernels + C ABI) for gfx950 with hipcc.
+"""Build ``libnpamd.so`` (HIP kernels + C ABI) for gfx950 with hipcc, and ``npamd_host.so``.
 
     python -m neuropress_amd.build [--force]
 
 Each ``csrc/*.hip`` is compiled to an object file (in parallel) and the
 objects are linked into ``neuropress_amd/lib/libnpamd.so``.  hipcc
-cross-compiles, so no GPU is needed to build.
+cross-compiles, so no GPU is needed to build.  ``csrc/host/*.cpp`` is host code
+against torch's own headers: the Python extension module that issues the lowered
+modules' calls (``neuropress_amd/lib/npamd_host.so``).
 """
 
 from __future__ import annotations
@@ -13,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -20,6 +23,8 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "lib"
 LIB_PATH = LIB_DIR / "libnpamd.so"
+HOST_PATH = LIB_DIR / "npamd_host.so"
+HOST_SRC = CSRC / "host" / "call_plan.cpp"
 OBJ_DIR = LIB_DIR / "obj"
 
 ARCH = "gfx950"
@@ -61,12 +66,44 @@ def _compile(src: Path, force: bool) -> Path:
     return obj
 
 
+def _compile_host(force: bool) -> Path:
+    """Compile the host extension module (no device code) against torch's headers."""
+    obj = OBJ_DIR / (HOST_SRC.stem + ".o")
+    newest = max(HOST_SRC.stat().st_mtime, _headers_mtime())
+    if not force and obj.exists() and obj.stat().st_mtime >= newest:
+        return obj
+    from torch.utils.cpp_extension import include_paths
+
+    rocm = Path(_hipcc()).resolve().parent.parent
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-I{sysconfig.get_paths()['include']}", f"-I{rocm / 'include'}"]  # fmt: skip
+    cmd += [f"-isystem{p}" for p in include_paths()] + ["-c", os.fspath(HOST_SRC), "-o", os.fspath(obj)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SRC.name}:\n{res.stderr}")
+    return obj
+
+
+def _link_host(obj: Path, force: bool) -> None:
+    if not force and HOST_PATH.exists() and HOST_PATH.stat().st_mtime >= max(obj.stat().st_mtime, LIB_PATH.stat().st_mtime):
+        return
+    import torch
+
+    libs = Path(torch.__file__).resolve().parent / "lib"
+    cmd = [shutil.which("g++") or "g++", "-shared", "-o", os.fspath(HOST_PATH), os.fspath(obj), f"-L{LIB_DIR}", "-l:libnpamd.so",
+           f"-L{libs}", "-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-lc10_hip", "-lc10", "-Wl,-rpath,$ORIGIN"]  # fmt: skip
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link of {HOST_PATH.name} failed:\n{res.stderr}")
+
+
 def build(force: bool = False, jobs: int | None = None) -> Path:
-    """Compile every kernel source and link the shared library; return its path."""
+    """Compile every kernel source and link the shared libraries; return the kernel library's path."""
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     srcs = sources()
-    jobs = jobs or min(len(srcs), os.cpu_count() or 4, 16)
+    jobs = jobs or min(len(srcs) + 1, os.cpu_count() or 4, 16)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_compile_host, force)
         objs = list(pool.map(lambda s: _compile(s, force), srcs))
     if force or not LIB_PATH.exists() or any(o.stat().st_mtime > LIB_PATH.stat().st_mtime for o in objs):
         cmd = [_hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", os.fspath(LIB_PATH)]
@@ -74,6 +111,7 @@ def build(force: bool = False, jobs: int | None = None) -> Path:
         res = subprocess.run(cmd, capture_output=True, text=True)
         if res.returncode != 0:
             raise RuntimeError(f"link failed:\n{res.stderr}")
+    _link_host(host.result(), force)
     return LIB_PATH
 
 

@@ -1,0 +1,611 @@
+// CallPlan: one lowered module's forward call with everything that stays the same from call to call
+// worked out once, issued from native code.
+//
+// What bounds a decode step of small layers is the time to issue its launches, not the kernels: through
+// Python argument checks and ctypes a call took 12-19 us of host time against 3-9 us of kernel.  Through a plan it
+// takes 4.5-5 us, 2.8 of them the HIP launch itself and 1.0 the output's allocation (us per eager call, before / now:
+// 2048 x 640 with a 256-row codebook 14.6 / 4.5, the nine calls of a block with hidden size 2048 128 / 44, residual VQ
+// 4096 x 4096 18.1 / 8.6 and int4 14336 x 4096 12.3 / 8.3, which are then bound by their kernels).  A plan
+// keeps the entry point's constant arguments (addresses, sizes, the kernel that serves a token count) and does
+// per call only what depends on the call: check that nothing it was built from has changed, allocate the output,
+// pass the addresses on.
+//
+// A plan never decides anything: which kernel serves how many tokens, and when a layer's derived tensors are
+// stale, stays the Python module's business.  Whatever a plan has not been told about (a token count, a dtype, a
+// layout, a changed buffer or threshold, an error from the library) makes the call return None, and the module
+// takes its ordinary route, which checks and reports.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <structmember.h>
+
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/index_select.h>
+#include <ATen/ops/linear.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <deque>
+#include <unordered_map>
+#include <vector>
+
+#include "../../../include/npamd.h"
+
+namespace {
+
+enum Kind : int {
+  kSliced = 0,
+  kVqGemv, kVqGemvPerm, kVqTile, kVqDense,
+  kRvqGemv, kRvqTile, kRvqDense,
+  kQGemv, kQTile, kQDense,
+  kRmsNorm, kVqEmbedding, kQEmbedding,
+  kKinds,
+};
+
+// Constant arguments each kind takes, in the order of its entry point (see issue()).
+constexpr int kArgs[kKinds] = {7, 9, 10, 9, 7, 15, 15, 13, 9, 9, 9, 2, 8, 8};
+
+// A dictionary some of whose entries the plan was built from.  CPython stamps a dictionary with a new tag on every
+// change, so an unchanged tag means unchanged entries; after a change the entries themselves are compared.
+struct Guard {
+  PyObject* dict = nullptr;  // borrowed for the module's own __dict__, owned otherwise
+  bool wrappers = false;     // entries that instrumentation replaces: the plan's own calls step aside for them, no more
+  uint64_t tag = 0;
+  std::vector<std::pair<PyObject*, PyObject*>> entries;  // owned
+};
+
+uint64_t dict_tag(PyObject* dict) {
+#if PY_VERSION_HEX < 0x030C0000
+  return reinterpret_cast<PyDictObject*>(dict)->ma_version_tag;
+#else
+  (void)dict;
+  return 0;  // no tag in this interpreter: the entries are compared on every call
+#endif
+}
+
+bool holds(Guard& g, PyObject* dict) {
+  const uint64_t tag = dict_tag(dict);
+  if (tag != 0 && tag == g.tag && dict == g.dict) return true;
+  for (const auto& e : g.entries)
+    if (PyDict_GetItemWithError(dict, e.first) != e.second) {
+      PyErr_Clear();
+      return false;
+    }
+  g.dict = dict;
+  g.tag = tag;
+  return true;
+}
+
+// A buffer the plan's derived tensors were made from: the same tensor, at the same place, not written to since.
+struct Source {
+  at::Tensor tensor;
+  const void* data;
+  int64_t version;  // -1: an inference tensor, which counts no versions
+};
+
+int64_t version_of(const at::Tensor& t) {
+  return t.is_inference() ? -1 : (int64_t)t.unsafeGetTensorImpl()->version_counter().current_version();
+}
+
+struct Template {
+  Kind kind;
+  int64_t n, k;                     // output and input features (embedding lookups: row length, 1)
+  std::vector<int64_t> a;           // constant arguments
+  double f;                         // eps of a norm, scale of an embedding
+  at::ScalarType out;
+  at::Tensor perm;                  // int64 column permutation applied to x first, or undefined
+  at::Tensor bias;                  // bias of the dense product, or undefined
+  std::vector<at::Tensor> keep;     // what the addresses point into
+};
+
+struct Route {
+  int tmpl;
+  int64_t ws;  // bytes of scratch (for kSliced: bytes of the shared zero-filled one)
+};
+
+struct Plan {
+  PyObject_HEAD
+  vectorcallfunc call;
+  PyObject* names;  // dict: what the module calls its templates
+  int device;
+  bool guarded;
+  Guard self;  // entries of the module's own __dict__
+  std::vector<Guard>* guards;
+  std::vector<PyObject*>* held;
+  std::vector<Source>* sources;
+  std::deque<Template>* templates;
+  std::unordered_map<int64_t, Route>* routes;  // key: dtype code << 32 | tokens
+};
+
+PyObject* g_workspaces = nullptr;       // {(device, stream): zero-filled scratch of the slice-list GEMV}
+PyObject* g_drop_workspace = nullptr;   // called as drop(device, stream) after a call that failed part-way
+
+int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kHalf: return NPAMD_F16;
+    case at::kBFloat16: return NPAMD_BF16;
+    case at::kFloat: return NPAMD_F32;
+    case at::kLong: return 3;
+    default: return -1;
+  }
+}
+
+at::ScalarType scalar_type(int code) {
+  return code == NPAMD_F16 ? at::kHalf : code == NPAMD_BF16 ? at::kBFloat16 : at::kFloat;
+}
+
+at::Tensor empty(at::IntArrayRef sizes, at::ScalarType t, int device) {
+  return at::Tensor(at::detail::empty_cuda(sizes, t, c10::Device(c10::kCUDA, (c10::DeviceIndex)device), std::nullopt));
+}
+
+// The slice-list GEMV's scratch on this device and stream, as the Python side allocated it; the last answer is
+// reused while the dictionary is unchanged.
+bool sliced_scratch(int device, hipStream_t stream, int64_t need, void** ptr, int64_t* bytes) {
+  static struct { uint64_t tag; int device; hipStream_t stream; void* ptr; int64_t bytes; } last = {0, -1, nullptr, nullptr, 0};
+  const uint64_t tag = dict_tag(g_workspaces);
+  if (tag == 0 || tag != last.tag || device != last.device || stream != last.stream) {
+    PyObject* key = Py_BuildValue("(in)", device, (Py_ssize_t)(intptr_t)stream);
+    if (!key) { PyErr_Clear(); return false; }
+    PyObject* ws = PyDict_GetItemWithError(g_workspaces, key);
+    Py_DECREF(key);
+    if (!ws || !THPVariable_Check(ws)) { PyErr_Clear(); return false; }
+    const at::Tensor& t = THPVariable_Unpack(ws);
+    last = {tag, device, stream, t.data_ptr(), t.numel() * (int64_t)t.element_size()};
+  }
+  if (last.bytes < need) return false;
+  *ptr = last.ptr;
+  *bytes = last.bytes;
+  return true;
+}
+
+template <class T>
+T ptr(int64_t v) { return reinterpret_cast<T>((uintptr_t)v); }
+
+using U8 = const uint8_t*;
+using F32 = const float*;
+using I32 = const int32_t*;
+
+// Launches template t on x ([m, k], row stride ldx); the output in *out.  False: not issued, or it failed.
+bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m, int64_t ldx, int device, at::Tensor* out) {
+  const std::vector<int64_t>& a = t.a;
+  hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+  at::Tensor x = x_in;
+  if (t.perm.defined()) {
+    x = at::index_select(x_in, -1, t.perm);
+    ldx = t.k;
+  }
+  c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
+  if (t.kind == kVqEmbedding || t.kind == kQEmbedding) sizes.push_back(t.n);
+  else sizes.back() = t.n;
+
+  if (t.kind == kVqDense || t.kind == kRvqDense || t.kind == kQDense) {
+    const int code = dtype_code(t.out);
+    at::Tensor w = empty({t.n, t.k}, t.out, device);
+    int rc;
+    if (t.kind == kVqDense)
+      rc = npamd_vq_dequant(ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], a[6], w.data_ptr(), code, st);
+    else if (t.kind == kRvqDense)
+      rc = npamd_rvq_dequant(ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]), (int)a[7],
+                             ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12], (int)t.n, (int)t.k,
+                             w.data_ptr(), code, st);
+    else
+      rc = npamd_q_dequant(ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), (int)t.n, (int)t.k, (int)a[6], (int)a[7],
+                           w.data_ptr(), code, st);
+    if (rc != NPAMD_OK) return false;
+    *out = at::linear(x, w, t.bias.defined() ? std::optional<at::Tensor>(t.bias) : std::nullopt);
+    return true;
+  }
+
+  void* ws = nullptr;
+  int64_t ws_bytes = 0;
+  at::Tensor scratch;
+  if (t.kind == kSliced) {
+    if (!sliced_scratch(device, st, r.ws, &ws, &ws_bytes)) return false;
+  } else if (r.ws > 0) {
+    scratch = empty({r.ws / 4}, at::kFloat, device);
+    ws = scratch.data_ptr();
+    ws_bytes = r.ws;
+  }
+  at::Tensor y = empty(sizes, t.out, device);
+  const void* xp = x.const_data_ptr();
+  void* yp = y.data_ptr();
+  const int M = (int)m, N = (int)t.n, K = (int)t.k;
+  int rc = NPAMD_ERR_INVALID;
+  switch (t.kind) {
+    case kSliced:
+      rc = npamd_vq_gemv_sliced(xp, ldx, ptr<I32>(a[0]), ptr<const npamd_sliced_header*>(a[1]), ptr<void*>(a[2]), ptr<void*>(a[3]), (int)a[4],
+                                ptr<F32>(a[5]), yp, t.n, M, (int)a[6], ws, ws_bytes, st);
+      if (rc != NPAMD_OK) {  // a launch of a multi-pass call may have run: the shared buffer is not known to be zero
+        PyObject* done = PyObject_CallFunction(g_drop_workspace, "in", device, (Py_ssize_t)(intptr_t)st);
+        if (!done) PyErr_Clear();
+        Py_XDECREF(done);
+      }
+      break;
+    case kVqGemv:
+      rc = npamd_vq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
+                         ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
+      break;
+    case kVqGemvPerm:
+      rc = npamd_vq_gemv_perm(xp, ldx, ptr<I32>(a[9]), ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4],
+                              (int)a[5], (int)a[6], ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
+      break;
+    case kVqTile:
+      rc = npamd_vq_gemm_tile(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
+                              ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], ws, ws_bytes, st);
+      break;
+    case kRvqGemv:
+      rc = npamd_rvq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]), (int)a[7],
+                          ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12], ptr<F32>(a[13]), yp,
+                          t.n, M, N, K, (int)a[14], st);
+      break;
+    case kRvqTile:
+      rc = npamd_rvq_gemm_tile(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]),
+                               (int)a[7], ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12],
+                               ptr<F32>(a[13]), yp, t.n, M, N, K, (int)a[14], ws, ws_bytes, st);
+      break;
+    case kQGemv:
+      rc = npamd_q_gemv(xp, ldx, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), ptr<F32>(a[3]), yp, t.n, M, N, K,
+                        (int)a[6], (int)a[7], (int)a[8], st);
+      break;
+    case kQTile:
+      rc = npamd_q_gemm_tile(xp, ldx, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), ptr<F32>(a[3]), yp, t.n, M, N, K,
+                             (int)a[6], (int)a[7], (int)a[8], ws, ws_bytes, st);
+      break;
+    case kRmsNorm:
+      rc = npamd_rms_norm(xp, ldx, ptr<void*>(a[0]), yp, t.n, M, N, (float)t.f, (int)a[1], st);
+      break;
+    case kVqEmbedding:
+      rc = npamd_vq_embedding((const int64_t*)xp, m, ptr<const int16_t*>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5],
+                              ptr<I32>(a[6]), (float)t.f, yp, (int)a[7], st);
+      break;
+    case kQEmbedding:
+      rc = npamd_q_embedding((const int64_t*)xp, m, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), (int)a[3], (int)a[4],
+                             a[5], N, a[6], (float)t.f, yp, (int)a[7], st);
+      break;
+    default: break;
+  }
+  if (rc != NPAMD_OK) return false;
+  *out = std::move(y);
+  return true;
+}
+
+bool wrapped(Plan* p) {
+  for (Guard& g : *p->guards)
+    if (g.wrappers && !holds(g, g.dict)) return true;
+  return false;
+}
+
+bool stale(Plan* p, PyObject* module) {
+  PyObject** dictp = _PyObject_GetDictPtr(module);
+  if (!dictp || !*dictp || !holds(p->self, *dictp)) return true;
+  for (Guard& g : *p->guards)
+    if (!g.wrappers && !holds(g, g.dict)) return true;
+  for (const Source& s : *p->sources) {
+    if (s.tensor.const_data_ptr() != s.data) return true;
+    if (s.version >= 0 && (int64_t)s.tensor.unsafeGetTensorImpl()->version_counter().current_version() != s.version) return true;
+  }
+  return false;
+}
+
+// Whether x is a stack of contiguous rows at one distance (the last tokens of a batch of prompts, say).
+bool rows_at_one_stride(const at::Tensor& x, int64_t* ldx) {
+  const int64_t dims = x.dim();
+  if (x.stride(-1) != 1) return false;
+  int64_t row = 0, next = 0;  // distance of two rows; stride the next dimension outwards must have
+  for (int64_t d = dims - 2; d >= 0; --d) {
+    if (x.size(d) == 1) continue;
+    if (row == 0) row = x.stride(d);
+    else if (x.stride(d) != next) return false;
+    next = x.stride(d) * x.size(d);
+  }
+  if (row == 0) row = x.size(-1);
+  *ldx = row;
+  return row >= x.size(-1);
+}
+
+PyObject* run(Plan* p, PyObject* xo) {
+  if (!THPVariable_CheckExact(xo)) Py_RETURN_NONE;
+  const at::Tensor& x = THPVariable_Unpack(xo);
+  const int code = dtype_code(x.scalar_type());
+  const int64_t dims = x.dim();
+  if (code < 0 || dims < 1 || !x.is_cuda() || x.get_device() != p->device) Py_RETURN_NONE;
+  const bool ids = code == 3;
+  const int64_t k = ids ? 1 : x.size(-1);
+  if (k == 0) Py_RETURN_NONE;
+  int64_t ldx = k;
+  const int64_t m = x.numel() / k;
+  if (!x.is_contiguous() && (ids || !rows_at_one_stride(x, &ldx))) Py_RETURN_NONE;
+  if (m < 1 || m > INT32_MAX) Py_RETURN_NONE;
+  auto it = p->routes->find(((int64_t)code << 32) | m);
+  if (it == p->routes->end()) {
+    it = p->routes->find((int64_t)code << 32);  // a route for any number of tokens
+    if (it == p->routes->end()) Py_RETURN_NONE;
+  }
+  const Route route = it->second;
+  const Template& t = (*p->templates)[(size_t)route.tmpl];
+  if (t.k != k) Py_RETURN_NONE;
+  try {
+    at::Tensor y;
+    if (!issue(t, route, x, m, ldx, p->device, &y)) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+// plan(module, x)
+PyObject* plan_call(PyObject* self, PyObject* const* args, size_t nargsf, PyObject* kwnames) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  if (PyVectorcall_NARGS(nargsf) != 2 || kwnames) {
+    PyErr_SetString(PyExc_TypeError, "CallPlan(module, x)");
+    return nullptr;
+  }
+  if (!p->guarded || stale(p, args[0]) || wrapped(p)) Py_RETURN_NONE;
+  return run(p, args[1]);
+}
+
+void clear_guard(Guard& g, bool owns_dict) {
+  for (auto& e : g.entries) {
+    Py_XDECREF(e.first);
+    Py_XDECREF(e.second);
+  }
+  g.entries.clear();
+  if (owns_dict) Py_XDECREF(g.dict);
+  g.dict = nullptr;
+}
+
+PyObject* plan_new(PyTypeObject* type, PyObject* args, PyObject*) {
+  int device = 0;
+  if (!PyArg_ParseTuple(args, "i", &device)) return nullptr;
+  PyObject* names = PyDict_New();
+  if (!names) return nullptr;
+  Plan* p = reinterpret_cast<Plan*>(type->tp_alloc(type, 0));
+  if (!p) {
+    Py_DECREF(names);
+    return nullptr;
+  }
+  // tp_alloc has handed the object to the garbage collector: from here to the last member nothing may allocate a
+  // Python object.
+  p->call = plan_call;
+  p->device = device;
+  p->guarded = false;
+  new (&p->self) Guard();
+  p->names = names;
+  p->guards = new std::vector<Guard>();
+  p->held = new std::vector<PyObject*>();
+  p->sources = new std::vector<Source>();
+  p->templates = new std::deque<Template>();
+  p->routes = new std::unordered_map<int64_t, Route>();
+  return reinterpret_cast<PyObject*>(p);
+}
+
+int plan_traverse(PyObject* self, visitproc visit, void* arg) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  for (auto& e : p->self.entries) {
+    Py_VISIT(e.first);
+    Py_VISIT(e.second);
+  }
+  Py_VISIT(p->names);
+  for (PyObject* o : *p->held) Py_VISIT(o);
+  for (Guard& g : *p->guards) {
+    Py_VISIT(g.dict);
+    for (auto& e : g.entries) {
+      Py_VISIT(e.first);
+      Py_VISIT(e.second);
+    }
+  }
+  return 0;
+}
+
+int plan_clear(PyObject* self) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  p->guarded = false;
+  clear_guard(p->self, false);
+  for (Guard& g : *p->guards) clear_guard(g, true);
+  p->guards->clear();
+  Py_CLEAR(p->names);
+  for (PyObject* o : *p->held) Py_DECREF(o);
+  p->held->clear();
+  return 0;
+}
+
+void plan_dealloc(PyObject* self) {
+  PyObject_GC_UnTrack(self);
+  plan_clear(self);
+  Plan* p = reinterpret_cast<Plan*>(self);
+  p->self.~Guard();
+  delete p->guards;
+  delete p->held;
+  delete p->sources;
+  delete p->templates;
+  delete p->routes;
+  Py_TYPE(self)->tp_free(self);
+}
+
+bool fill_guard(Guard& g, PyObject* entries) {
+  PyObject *key, *value;
+  Py_ssize_t at = 0;
+  if (!PyDict_Check(entries)) {
+    PyErr_SetString(PyExc_TypeError, "guard entries must be a dict");
+    return false;
+  }
+  while (PyDict_Next(entries, &at, &key, &value)) {
+    Py_INCREF(key);
+    Py_INCREF(value);
+    g.entries.emplace_back(key, value);
+  }
+  return true;
+}
+
+// guard(dict_or_type, {key: expected}, wrappers)
+PyObject* plan_guard(PyObject* self, PyObject* args) {
+  PyObject *where, *entries;
+  int wrappers;
+  if (!PyArg_ParseTuple(args, "OOp", &where, &entries, &wrappers)) return nullptr;
+  PyObject* dict = PyType_Check(where) ? reinterpret_cast<PyTypeObject*>(where)->tp_dict : where;
+  if (!PyDict_Check(dict)) {
+    PyErr_SetString(PyExc_TypeError, "guard() takes a dict or a class");
+    return nullptr;
+  }
+  Guard g;
+  if (!fill_guard(g, entries)) return nullptr;
+  Py_INCREF(dict);
+  g.dict = dict;
+  g.wrappers = wrappers != 0;
+  reinterpret_cast<Plan*>(self)->guards->push_back(std::move(g));
+  Py_RETURN_NONE;
+}
+
+// guard_module({attribute: expected}): entries of the calling module's __dict__.  The plan keeps no reference to
+// that dictionary (it holds the plan).
+PyObject* plan_guard_module(PyObject* self, PyObject* entries) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  if (!fill_guard(p->self, entries)) return nullptr;
+  p->guarded = true;
+  Py_RETURN_NONE;
+}
+
+// source(tensor or None)
+PyObject* plan_source(PyObject* self, PyObject* t) {
+  if (t == Py_None) Py_RETURN_NONE;
+  if (!THPVariable_Check(t)) {
+    PyErr_SetString(PyExc_TypeError, "source() takes a tensor");
+    return nullptr;
+  }
+  const at::Tensor& v = THPVariable_Unpack(t);
+  reinterpret_cast<Plan*>(self)->sources->push_back({v, v.const_data_ptr(), version_of(v)});
+  Py_RETURN_NONE;
+}
+
+// hold(object): something the template's addresses point into that is not a tensor
+PyObject* plan_hold(PyObject* self, PyObject* o) {
+  Py_INCREF(o);
+  reinterpret_cast<Plan*>(self)->held->push_back(o);
+  Py_RETURN_NONE;
+}
+
+// template(kind, n, k, args, f, out_dtype_code, perm or None, bias or None, keep) -> number
+PyObject* plan_template(PyObject* self, PyObject* args) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  int kind, out_code;
+  long long n, k;
+  double f;
+  PyObject *ints, *perm, *bias, *keep;
+  if (!PyArg_ParseTuple(args, "iLLO!diOOO!", &kind, &n, &k, &PyTuple_Type, &ints, &f, &out_code, &perm, &bias, &PyTuple_Type, &keep))
+    return nullptr;
+  if (kind < 0 || kind >= kKinds || (int)PyTuple_GET_SIZE(ints) > kArgs[kind]) {
+    PyErr_SetString(PyExc_ValueError, "template(): bad kind or argument count");
+    return nullptr;
+  }
+  Template t;
+  t.kind = (Kind)kind;
+  t.n = n;
+  t.k = k;
+  t.f = f;
+  t.out = scalar_type(out_code);
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(ints); ++i) {
+    PyObject* v = PyTuple_GET_ITEM(ints, i);
+    const long long value = v == Py_None ? 0 : PyLong_AsLongLong(v);
+    if (value == -1 && PyErr_Occurred()) return nullptr;
+    t.a.push_back(value);
+  }
+  t.a.resize((size_t)kArgs[kind], 0);
+  if (perm != Py_None) t.perm = THPVariable_Unpack(perm);
+  if (bias != Py_None) t.bias = THPVariable_Unpack(bias);
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(keep); ++i) {
+    PyObject* v = PyTuple_GET_ITEM(keep, i);
+    if (v != Py_None && THPVariable_Check(v)) t.keep.push_back(THPVariable_Unpack(v));
+  }
+  p->templates->push_back(std::move(t));
+  return PyLong_FromSize_t(p->templates->size() - 1);
+}
+
+// route(dtype_code, tokens (0: any number), template, scratch_bytes)
+PyObject* plan_route(PyObject* self, PyObject* args) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  int code, tmpl;
+  long long m, ws;
+  if (!PyArg_ParseTuple(args, "iLiL", &code, &m, &tmpl, &ws)) return nullptr;
+  if (code < 0 || code > 3 || m < 0 || m > INT32_MAX || tmpl < 0 || (size_t)tmpl >= p->templates->size()) {
+    PyErr_SetString(PyExc_ValueError, "route(): out of range");
+    return nullptr;
+  }
+  if (p->routes->size() > 65536) p->routes->clear();  // bounded, whatever token counts a server sees
+  (*p->routes)[((int64_t)code << 32) | m] = Route{tmpl, ws};
+  Py_RETURN_NONE;
+}
+
+PyObject* plan_stale(PyObject* self, PyObject* module) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  return PyBool_FromLong(!p->guarded || stale(p, module));
+}
+
+PyObject* plan_wrapped(PyObject* self, PyObject*) { return PyBool_FromLong(wrapped(reinterpret_cast<Plan*>(self))); }
+
+PyObject* plan_run(PyObject* self, PyObject* x) { return run(reinterpret_cast<Plan*>(self), x); }
+
+// A plan holds addresses: a copied or unpickled module starts without one.
+PyObject* plan_reduce(PyObject*, PyObject*) { return Py_BuildValue("(O())", Py_TYPE(Py_None)); }
+
+PyMethodDef plan_methods[] = {
+    {"guard", plan_guard, METH_VARARGS, "guard(dict_or_class, {key: expected}, wrappers)"},
+    {"guard_module", plan_guard_module, METH_O, "guard_module({attribute: expected})"},
+    {"source", plan_source, METH_O, "source(tensor or None)"},
+    {"hold", plan_hold, METH_O, "hold(object)"},
+    {"template", plan_template, METH_VARARGS, "template(kind, n, k, args, f, out, perm, bias, keep) -> number"},
+    {"route", plan_route, METH_VARARGS, "route(dtype, tokens, template, scratch_bytes)"},
+    {"stale", plan_stale, METH_O, "stale(module): whether anything the plan was built from has changed"},
+    {"wrapped", plan_wrapped, METH_NOARGS, "wrapped(): whether a wrapper function has been replaced"},
+    {"run", plan_run, METH_O, "run(x): the call without the checks of the module"},
+    {"__reduce__", plan_reduce, METH_NOARGS, ""},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyMemberDef plan_members[] = {
+    {"names", T_OBJECT_EX, offsetof(Plan, names), READONLY, "template numbers by the module's names for them"},
+    {nullptr, 0, 0, 0, nullptr},
+};
+
+PyTypeObject plan_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyObject* set_workspaces(PyObject*, PyObject* args) {
+  PyObject *dict, *drop;
+  if (!PyArg_ParseTuple(args, "O!O", &PyDict_Type, &dict, &drop)) return nullptr;
+  Py_INCREF(dict);
+  Py_INCREF(drop);
+  Py_XDECREF(g_workspaces);
+  Py_XDECREF(g_drop_workspace);
+  g_workspaces = dict;
+  g_drop_workspace = drop;
+  Py_RETURN_NONE;
+}
+
+PyMethodDef module_methods[] = {
+    {"set_workspaces", set_workspaces, METH_VARARGS, "set_workspaces(dict, drop): the slice-list GEMV's scratch buffers"},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "npamd_host", nullptr, -1, module_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_npamd_host(void) {
+  plan_type.tp_name = "npamd_host.CallPlan";
+  plan_type.tp_basicsize = sizeof(Plan);
+  plan_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC | Py_TPFLAGS_HAVE_VECTORCALL;
+  plan_type.tp_doc = "One lowered module's forward call, issued from native code.";
+  plan_type.tp_new = plan_new;
+  plan_type.tp_dealloc = plan_dealloc;
+  plan_type.tp_traverse = plan_traverse;
+  plan_type.tp_clear = plan_clear;
+  plan_type.tp_call = PyVectorcall_Call;
+  plan_type.tp_vectorcall_offset = offsetof(Plan, call);
+  plan_type.tp_methods = plan_methods;
+  plan_type.tp_members = plan_members;
+  if (PyType_Ready(&plan_type) < 0) return nullptr;
+  PyObject* m = PyModule_Create(&module_def);
+  if (!m) return nullptr;
+  Py_INCREF(&plan_type);
+  if (PyModule_AddObject(m, "CallPlan", reinterpret_cast<PyObject*>(&plan_type)) < 0) return nullptr;
+  return m;
+}

@@ -1,0 +1,63 @@
+"""What the lowered modules hand to the native call path (``csrc/host/call_plan.cpp``).
+
+A module that has decided which kernel serves a call describes that call here once -- the entry point's constant
+arguments as a *template*, the token counts it serves as *routes* -- and later calls are issued by the plan without
+Python argument checks.  A plan is valid while the module's buffers, the attributes and thresholds that the decision
+read, and the wrapper functions of ``kernels`` are what they were; otherwise it declines and the module decides again.
+"""
+
+from __future__ import annotations
+
+import torch
+
+from .. import _lib
+
+(SLICED, VQ_GEMV, VQ_GEMV_PERM, VQ_TILE, VQ_DENSE, RVQ_GEMV, RVQ_TILE, RVQ_DENSE,
+ Q_GEMV, Q_TILE, Q_DENSE, RMS_NORM, VQ_EMBEDDING, Q_EMBEDDING) = range(14)  # fmt: skip
+
+DTYPE_CODES = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32, torch.int64: 3}
+
+
+def make(module, attributes, thresholds=None, names=(), holders=(), sources=()):
+    """An empty plan for *module*, or None where it cannot have one (a tensor off the module's GPU, or with gaps).
+
+    *attributes*: names in the module's ``__dict__`` the dispatch reads; *thresholds* / *names*: the globals of the
+    module's file it reads; *holders*: further modules whose buffers are used (shared codebooks); *sources*: the
+    buffers themselves.
+    """
+    from .. import kernels
+
+    device = None
+    for t in sources:
+        if t is None:
+            continue
+        if not t.is_cuda or not t.is_contiguous() or (device is not None and t.device != device):
+            return None
+        device = t.device
+    if device is None:
+        return None
+    plan = _lib.host().CallPlan(device.index)
+    own = module.__dict__
+    plan.guard_module({name: own[name] for name in (*attributes, "_buffers") if name in own})
+    for holder in (module, *holders):
+        plan.guard(holder._buffers, dict(holder._buffers), False)
+    if names:
+        plan.guard(thresholds, {name: thresholds[name] for name in names}, False)
+    plan.guard(kernels.__dict__, kernels.WRAPPERS, True)
+    plan.guard(kernels.SlicedCallPlan, {"run": kernels.SLICED_RUN}, True)
+    for t in sources:
+        plan.source(t)
+    return plan
+
+
+def template(plan, kind, n, k, args, dtype, *, f=0.0, perm=None, bias=None):
+    """Template number of one call shape.  *args*: its constant arguments, tensors standing for their addresses (the
+    plan keeps them alive); *dtype*: of the output."""
+    ints = tuple(a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args)
+    keep = tuple(a for a in args if isinstance(a, torch.Tensor))
+    return plan.template(kind, n, k, ints, f, DTYPE_CODES[dtype], perm, bias, keep)
+
+
+def tile_scratch(m: int, n: int, k: int) -> int:
+    """Bytes of scratch a tile GEMM of this shape can use."""
+    return max(0, int(_lib.load().npamd_gemm_tile_workspace_bytes(m, n, k))) // 4 * 4

@@ -155,10 +155,47 @@ class NPEmbedding(nn.Module):
         self.backend = bk
         return self
 
+    _plan = None  # CallPlan of the calls made so far
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        plan = self._plan
+        if plan is not None:  # a call made before, with the same table
+            y = plan(self, x)
+            if y is not None:
+                return y
+        return self._forward(x)
+
+    def _planned(self, ids: torch.Tensor):
+        """Let a plan issue this lookup, whatever the number of ids; None where it cannot."""
+        from ..kernels import plans
+
+        blob, scale, zp = self.u8_blob, self.scale, self.zero_point
+        dtype, dim = self.out_dtype or scale.dtype, self.embedding_dim
+        if ids.dtype != torch.int64 or ids.device != blob.device or dtype not in plans.DTYPE_CODES or blob.dim() != 2 or (
+            scale.dtype != torch.float16 or (zp is not None and zp.dtype != torch.float16)
+            or blob.shape[1] * 8 != dim * self.nbits or scale.numel() * self.group_size != blob.shape[0] * dim
+            or torch.cuda.is_current_stream_capturing()
+        ):  # fmt: skip
+            return None
+        plan = self._plan
+        if plan is None or plan.stale(self):
+            plan = plans.make(self, ("backend", "nbits", "group_size", "padding_idx", "embed_scale", "out_dtype", "zero_point",
+                                     "embedding_dim"), sources=(blob, scale, zp))  # fmt: skip
+            if plan is None:
+                return None
+            pad = -1 if self.padding_idx is None else int(self.padding_idx)
+            args = (blob, scale, zp, self.nbits, self.group_size, blob.shape[0], pad, plans.DTYPE_CODES[dtype])
+            plan.route(3, 0, plans.template(plan, plans.Q_EMBEDDING, dim, 1, args, dtype, f=float(self.embed_scale)), 0)
+            self._plan = plan
+        return None if plan.wrapped() else plan.run(ids)
+
+    def _forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.backend == EmbeddingBackend.CUDA and x.is_cuda and self.u8_blob.is_cuda:
             from .. import kernels
 
+            y = self._planned(x)
+            if y is not None:
+                return y
             return kernels.q_embedding(x, self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point,
                                        self.padding_idx, self.embed_scale, self.out_dtype or self.scale.dtype)  # fmt: skip
         if self.backend == EmbeddingBackend.DEFAULT:

@@ -153,8 +153,17 @@ def _q_dequant_linear(
     return F.linear(x, w.to(x.dtype), bias)
 
 
+# What the choice of a kernel reads besides the buffers: a call plan is valid while these are unchanged.
+_PLAN_ATTRIBUTES = ("backend", "out_features", "in_features", "group_size", "nbits", "zero_point", "bias")
+_PLAN_THRESHOLDS = ("_Q_TILE_MAX_TOKENS", "_Q_TILE_LONG_K_MAX_TOKENS", "_Q_TILE_WIDE_MAX_TOKENS", "_Q_TILE_WIDE_MIN_FEATURES",
+                    "_Q_TILE_MIN_GRID_FRACTION", "_Q_TILE_SPLIT_MAX_TOKENS", "_Q_TILE_SPLIT_LONG_K", "_Q_FUSED_MAX_TOKENS",
+                    "_Q_FUSED_WIDE_MAX_TOKENS", "_Q_FUSED_WIDE_MAX_ACTIVATIONS")  # fmt: skip
+
+
 class NPLinear(nn.Module):
     """Linear layer with a packed n-bit quantized weight and a pluggable backend."""
+
+    _plan = None  # CallPlan of the calls made so far (see forward)
 
     def __init__(
         self,
@@ -203,6 +212,7 @@ class NPLinear(nn.Module):
     def _apply(self, fn, recurse: bool = True):
         result = super()._apply(fn, recurse)
         self._derived = {}
+        self._plan = None
         return result
 
     @classmethod
@@ -280,6 +290,11 @@ class NPLinear(nn.Module):
         return self.bias.to(dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        plan = self._plan
+        if plan is not None:  # a call made before: same token count, dtype and buffers
+            y = plan(self, x)
+            if y is not None:
+                return y
         if self.backend == LinearBackend.CUDA:
             return self._forward_cuda(x)
         # default / compile: the torch-op specification of the layer.
@@ -336,28 +351,14 @@ class NPLinear(nn.Module):
 
         m = x.numel() // self.in_features
         try:
-            # Layers the MFMA kernels do not take (1 / 2 / 8 bits, odd group sizes) would run an
-            # element-wise kernel, slower at every token count than decoding once and calling the
-            # dense GEMM (14336 x 4096, 8 bits: 99 us against 57 us at one token, 452 against 57 at 16).
-            fused_ok = x.dtype in (torch.float16, torch.bfloat16) and self._mfma_layer()
-            gemv_max = self._gemv_max_tokens(m)
-            if fused_ok and m > gemv_max:
-                limit = _Q_TILE_MAX_TOKENS
-                if self.in_features >= _Q_TILE_SPLIT_LONG_K:
-                    limit = max(limit, _Q_TILE_LONG_K_MAX_TOKENS)
-                if limit > 0 and max(self.in_features, self.out_features) >= _Q_TILE_WIDE_MIN_FEATURES:
-                    limit = max(limit, _Q_TILE_WIDE_MAX_TOKENS)
-                fused_ok = m <= limit and self._tile_grid_fills_gpu(x, m)
-            if fused_ok:
-                if m <= gemv_max:
-                    return kernels.q_linear(
-                        x, self.u8_blob, self.scale, self.nbits, self.group_size,
-                        self.zero_point, self._bias_f32(),
-                    )  # fmt: skip
-                return kernels.q_gemm_tile(
-                    x, self.u8_blob, self.scale, self.nbits, self.group_size,
-                    self.zero_point, self._bias_f32(),
-                )  # fmt: skip
+            band = self._band(x, m)
+            if not torch.cuda.is_current_stream_capturing():
+                y = self._planned(x, m, band)
+                if y is not None:
+                    return y
+            if band != "dense":
+                fn = kernels.q_linear if band == "fused" else kernels.q_gemm_tile
+                return fn(x, self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point, self._bias_f32())
             w = kernels.q_dequant(
                 self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point, x.dtype
             )
@@ -367,6 +368,50 @@ class NPLinear(nn.Module):
             kernels.warn_kernel_fallback("q_linear", "torch dequant + matmul", exc)
             return self._forward_compile(x)
         return F.linear(x, w, self._bias_as(x.dtype))
+
+    def _band(self, x: torch.Tensor, m: int) -> str:
+        """Which kernel serves a call of *m* tokens: ``fused`` (GEMV), ``tile`` (fused GEMM) or ``dense`` (decode + GEMM)."""
+        # Layers the MFMA kernels do not take (1 / 2 / 8 bits, odd group sizes) would run an
+        # element-wise kernel, slower at every token count than decoding once and calling the
+        # dense GEMM (14336 x 4096, 8 bits: 99 us against 57 us at one token, 452 against 57 at 16).
+        if x.dtype not in (torch.float16, torch.bfloat16) or not self._mfma_layer():
+            return "dense"
+        if m <= self._gemv_max_tokens(m):
+            return "fused"
+        limit = _Q_TILE_MAX_TOKENS
+        if self.in_features >= _Q_TILE_SPLIT_LONG_K:
+            limit = max(limit, _Q_TILE_LONG_K_MAX_TOKENS)
+        if limit > 0 and max(self.in_features, self.out_features) >= _Q_TILE_WIDE_MIN_FEATURES:
+            limit = max(limit, _Q_TILE_WIDE_MAX_TOKENS)
+        return "tile" if m <= limit and self._tile_grid_fills_gpu(x, m) else "dense"
+
+    def _planned(self, x: torch.Tensor, m: int, band: str):
+        """Add this call to the layer's plan and let the plan issue it; None where it cannot."""
+        from ..kernels import plans
+
+        n, k = self.out_features, self.in_features
+        if m < 1 or x.dtype not in plans.DTYPE_CODES or x.device != self.u8_blob.device or (
+            self.u8_blob.dtype != torch.uint8 or self.scale.dtype != torch.float16
+            or tuple(self.u8_blob.shape) != (n, k * self.nbits // 8) or self.scale.numel() * self.group_size != n * k
+            or (self.zero_point is not None and self.zero_point.numel() != self.scale.numel())
+        ):  # fmt: skip
+            return None
+        plan = self._plan
+        if plan is None or plan.stale(self):
+            plan = plans.make(self, _PLAN_ATTRIBUTES, globals(), _PLAN_THRESHOLDS,
+                              sources=(self.u8_blob, self.scale, self.zero_point, self.bias))  # fmt: skip
+            if plan is None:
+                return None
+        code = plans.DTYPE_CODES[x.dtype]
+        number = plan.names.get((band, x.dtype))
+        if number is None:
+            kind = {"fused": plans.Q_GEMV, "tile": plans.Q_TILE, "dense": plans.Q_DENSE}[band]
+            args = (self.u8_blob, self.scale, self.zero_point, self._bias_f32(), 0, 0, self.nbits, self.group_size, code)
+            number = plan.names[band, x.dtype] = plans.template(
+                plan, kind, n, k, args, x.dtype, bias=self._bias_as(x.dtype) if band == "dense" else None)  # fmt: skip
+        plan.route(code, m, number, plans.tile_scratch(m, n, k) if band == "tile" else 0)
+        self._plan = plan
+        return None if plan.wrapped() else plan.run(x)
 
     def extra_repr(self) -> str:
         return (

@@ -35,12 +35,44 @@ class NPRMSNorm(nn.Module):
         source = self.__dict__.get("_source")
         return None if source is None else source.to(self.weight.device)
 
+    _plan = None  # CallPlan of the calls made so far
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        plan = self._plan
+        if plan is not None:  # a call made before: same dtype and weight
+            y = plan(self, x)
+            if y is not None:
+                return y
+        return self._forward(x)
+
+    def _planned(self, x: torch.Tensor, w: torch.Tensor):
+        """Let a plan issue this norm, whatever the number of rows; None where it cannot."""
+        from ..kernels import plans
+
+        h = self.weight.shape[0]
+        if x.dtype not in plans.DTYPE_CODES or x.device != w.device or w.dim() != 1 or torch.cuda.is_current_stream_capturing():
+            return None
+        plan = self._plan
+        if plan is None or plan.stale(self):
+            plan = plans.make(self, ("eps",), sources=(self.weight,))
+            if plan is None:
+                return None
+        if x.dtype not in plan.names:
+            code = plans.DTYPE_CODES[x.dtype]
+            plan.names[x.dtype] = plans.template(plan, plans.RMS_NORM, h, h, (w, code), x.dtype, f=float(self.eps))
+            plan.route(code, 0, plan.names[x.dtype], 0)
+        self._plan = plan
+        return None if plan.wrapped() else plan.run(x)
+
+    def _forward(self, x: torch.Tensor) -> torch.Tensor:
         *leading, h = x.shape
         w = self.weight if self.weight.dtype == x.dtype else self.weight.to(x.dtype)
         if x.is_cuda:
             from .. import kernels
 
+            y = self._planned(x, w)
+            if y is not None:
+                return y
             return kernels.rms_norm(x.reshape(-1, h), w, self.eps).reshape(*leading, h)
         xf = x.float()  # specification of the kernel, for tensors that are not on a GPU
         return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps) * w.float()).to(x.dtype)

@@ -94,7 +94,39 @@ class NPVQEmbedding(nn.Module):
     def weight(self) -> _WeightProxy:
         return _WeightProxy(self)
 
+    _plan = None  # CallPlan of the calls made so far
+
     def forward(self, input_ids: torch.Tensor) -> torch.Tensor:
+        plan = self._plan
+        if plan is not None:  # a call made before, with the same tables
+            y = plan(self, input_ids)
+            if y is not None:
+                return y
+        return self._forward(input_ids)
+
+    def _planned(self, ids: torch.Tensor, perm: torch.Tensor | None):
+        """Let a plan issue this lookup, whatever the number of ids; None where it cannot."""
+        from ..kernels import plans
+
+        table, cb = self.all_indices, self.proxy.centroids
+        dtype = self.out_dtype or torch.float16
+        if ids.dtype != torch.int64 or ids.device != table.device or dtype not in plans.DTYPE_CODES or table.dim() != 2 or (
+            cb.dtype != torch.float16 or table.shape[1] * cb.shape[1] != self.embedding_dim
+            or torch.cuda.is_current_stream_capturing()
+        ):  # fmt: skip
+            return None
+        plan = self._plan
+        if plan is None or plan.stale(self):
+            plan = plans.make(self, ("proxy", "scale", "out_dtype", "inv_perm", "embedding_dim"), holders=(self.proxy,),
+                              sources=(table, cb, self.inv_perm))  # fmt: skip
+            if plan is None:
+                return None
+            args = (table, table.shape[0], table.shape[1], cb, cb.shape[0], cb.shape[1], perm, plans.DTYPE_CODES[dtype])
+            plan.route(3, 0, plans.template(plan, plans.VQ_EMBEDDING, self.embedding_dim, 1, args, dtype, f=float(self.scale)), 0)
+            self._plan = plan
+        return None if plan.wrapped() else plan.run(ids)
+
+    def _forward(self, input_ids: torch.Tensor) -> torch.Tensor:
         if input_ids.is_cuda and self.all_indices.is_cuda:
             from .. import kernels
 
@@ -104,6 +136,9 @@ class NPVQEmbedding(nn.Module):
                 if perm is None or perm.device != input_ids.device:
                     perm = self.inv_perm.to(device=input_ids.device, dtype=torch.int32).contiguous()
                     self._derived["perm_i32"] = perm
+            y = self._planned(input_ids, perm)
+            if y is not None:
+                return y
             return kernels.vq_embedding(input_ids, self.all_indices, self.proxy.centroids, self.scale, perm,
                                         self.out_dtype)  # fmt: skip
         # torch ops: the specification (reference: np_vq_embedding.py:120-142), indices read as unsigned

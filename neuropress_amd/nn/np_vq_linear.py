@@ -161,6 +161,14 @@ _ALLOW_FALLBACK: bool = os.environ.get("NEUROPRESS_ALLOW_KERNEL_FALLBACK", "").s
 _CODED_BACKENDS = frozenset({VQBackend.CUDA_TIERED, VQBackend.CUDA_NTIER, VQBackend.CUDA_ZERO_ESCAPE})
 _FUSED_BACKENDS = frozenset({VQBackend.CUDA_WMMA, VQBackend.CUDA_LUT, VQBackend.CUDA}) | _CODED_BACKENDS
 
+# What the band decision reads besides the buffers: a call plan is valid while these are unchanged.
+_PLAN_ATTRIBUTES = ("backend", "proxy", "residual_proxy", "out_features", "in_features", "vector_len", "bits", "residual_bits",
+                    "bias", "column_perm", "packed_residual", "row_scale", "row_bias")  # fmt: skip
+_PLAN_THRESHOLDS = ("_FUSED_MAX_TOKENS", "_FUSED_WIDE_MAX_TOKENS", "_FUSED_WIDE_MAX_ACTIVATIONS", "_SLICED_MAX_TOKENS",
+                    "_SLICED_MIN_CENTROIDS", "_SLICED_MIN_INDICES", "_LUT_MAX_TOKENS", "_TILE_MAX_TOKENS", "_TILE_WIDE_MAX_TOKENS",
+                    "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_SMALL_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS", "_TILE_WIDE_SMALL_MAX_TOKENS",
+                    "_TILE_MIN_GRID_FRACTION", "_TILE_SPLIT_MAX_TOKENS", "_TILE_SPLIT_LONG_K", "_tile_failed")  # fmt: skip
+
 # Latched once the tile GEMM fails with fallback allowed, so later calls go
 # straight to decode + GEMM (reference: np_vq_linear.py:91-93).
 _tile_failed: bool = False
@@ -242,15 +250,6 @@ def _vq_dequant_linear(
 # ---------------------------------------------------------------------------
 # VQProxy — shared codebook
 # ---------------------------------------------------------------------------
-
-
-def _versions_of(packed, bias, perm, cent) -> tuple:
-    return (
-        packed._version,
-        cent._version,
-        -1 if bias is None else bias._version,
-        -1 if perm is None else perm._version,
-    )
 
 
 class VQProxy(nn.Module):
@@ -359,6 +358,8 @@ class NPVQLinear(nn.Module):
     each operation rounded to fp16 (the benchmark's residual-VQ configuration; not in the reference).
     """
 
+    _plan = None  # CallPlan of the calls made so far (see forward)
+
     def __init__(
         self,
         proxy: VQProxy,
@@ -446,8 +447,6 @@ class NPVQLinear(nn.Module):
         self._register_optional("row_bias", None if row_bias is None else row_bias.to(torch.float16))
         # Derived, rebuilt on demand: f32 bias for the kernels, widened index stream.
         self._derived: dict = {}
-        # Per activation dtype: the decode call with its constant arguments worked out once (see forward).
-        self._plans: dict = {}
         # load_state_dict() copies into the buffers in place: what was derived from them is stale.
         self.register_load_state_dict_post_hook(NPVQLinear._after_load_state_dict)
 
@@ -512,7 +511,7 @@ class NPVQLinear(nn.Module):
         result = super()._apply(fn, recurse)
         if self._buffer_places() != before:
             self._derived = {}
-        self._plans = {}
+        self._plan = None
         self._bind_proxies()  # a copied or unpickled proxy starts with no users
         self._prepare_after_move()
         return result
@@ -538,7 +537,7 @@ class NPVQLinear(nn.Module):
     @staticmethod
     def _after_load_state_dict(module, incompatible_keys) -> None:
         module._derived = {}
-        module._plans = {}
+        module._plan = None
         module._prepare_after_move()
 
     # ------------------------------------------------------------------
@@ -687,52 +686,33 @@ class NPVQLinear(nn.Module):
     # ------------------------------------------------------------------
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        """Band dispatch by token count (reference: neuropress/nn/np_vq_linear.py:1014-1058)."""
-        entry = self._plans.get(x.dtype)
-        if entry is not None:
-            # A decode call this layer has made before: same buffers, not written to since?  Then the
-            # call is issued with its constant arguments as they were worked out then.
-            plan, packed, bias, perm, cent, versions = entry
-            buffers = self._buffers
-            if (
-                buffers["packed_indices"] is packed
-                and buffers.get("bias") is bias
-                and buffers.get("column_perm") is perm
-                and self.proxy._buffers["centroids"] is cent
-                and (versions is None or versions == _versions_of(packed, bias, perm, cent))
-            ):
-                y = plan.run(x)
-                if y is not None:
-                    return y
-            else:
-                self._plans = {}
-        if self.backend in _FUSED_BACKENDS and x.dtype in (torch.float16, torch.bfloat16):
-            m = x.numel() // self.in_features
-            if m <= min(_SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)) and x.is_cuda:
-                sliced = self._sliced_for(m)
-                if sliced is not None:
-                    return self._forward_sliced(x, sliced)  # applies column_perm inside the kernel
-            if self.column_perm is not None and self._perm_fusable(x, m):
-                return self._fused(x, tile=False, perm=self._perm_i32(x.device))
+        """Band dispatch by token count (reference: neuropress/nn/np_vq_linear.py:1014-1058).
+
+        A call this layer has made before -- same token count, dtype and buffers -- is issued by its plan."""
+        plan = self._plan
+        if plan is not None:
+            y = plan(self, x)
+            if y is not None:
+                return y
+        return self._forward(x)
+
+    def _forward(self, x: torch.Tensor) -> torch.Tensor:
+        m = x.numel() // self.in_features
+        band = self._band(x, m)
+        if x.is_cuda and not torch.cuda.is_current_stream_capturing():
+            y = self._planned(x, m, band)
+            if y is not None:
+                return y
+        if band == "sliced":
+            return self._forward_sliced(x, self._sliced_for(m))  # applies column_perm inside the kernel
+        if band == "gemv_perm":
+            return self._fused(x, tile=False, perm=self._perm_i32(x.device))
         if self.column_perm is not None:
             x = x[..., self.column_perm]
-        if self.backend in _FUSED_BACKENDS:
-            if x.dtype not in (torch.float16, torch.bfloat16):
-                return self._forward_dequant_gemm(x)  # fp32 activations: decode + GEMM
-            if x.is_cuda and not self._mfma_layer():
-                # Shapes without an MFMA kernel (vector lengths other than 8 and 4, K not a
-                # multiple of 64): the element-wise GEMV is slower than decoding once and calling
-                # the dense GEMM at every token count (14336 x 4096: 99 us against 57 us at one token).
-                return self._forward_dequant_gemm(x)
-            m = x.numel() // self.in_features
-            if m > self._gemv_max_tokens(m):
-                if (
-                    self.backend != VQBackend.CUDA_LUT
-                    and m <= self._tile_max_tokens()
-                    and self._tile_band_ok(x, m)
-                ):
-                    return self._forward_tile_gemm(x)
-                return self._forward_dequant_gemm(x)
+        if band == "dense":
+            return self._forward_dequant_gemm(x)
+        if band == "tile":
+            return self._forward_tile_gemm(x)
         if self.backend == VQBackend.CUDA_LUT:
             return self._forward_cuda_lut(x)
         if self.backend == VQBackend.CUDA_WMMA or self.backend in _CODED_BACKENDS:
@@ -742,6 +722,109 @@ class NPVQLinear(nn.Module):
         if self.backend == VQBackend.COMPILE:
             return self._forward_compile(x)
         return self._forward_default(x)
+
+    def _band(self, x: torch.Tensor, m: int) -> str:
+        """Which kernel serves a call of *m* tokens: ``sliced``, ``gemv_perm`` (the GEMV that gathers x's columns),
+        ``fused`` (the backend's GEMV), ``tile``, ``dense`` (decode + GEMM) or ``torch``."""
+        if self.backend not in _FUSED_BACKENDS:
+            return "torch"
+        if x.dtype not in (torch.float16, torch.bfloat16):
+            return "dense"  # fp32 activations: decode + GEMM
+        if m <= min(_SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)) and x.is_cuda and self._sliced_for(m) is not None:
+            return "sliced"
+        if self.column_perm is not None and self._perm_fusable(x, m):
+            return "gemv_perm"
+        if x.is_cuda and not self._mfma_layer():
+            # Shapes without an MFMA kernel (vector lengths other than 8 and 4, K not a
+            # multiple of 64): the element-wise GEMV is slower than decoding once and calling
+            # the dense GEMM at every token count (14336 x 4096: 99 us against 57 us at one token).
+            return "dense"
+        if m > self._gemv_max_tokens(m):
+            if self.backend != VQBackend.CUDA_LUT and m <= self._tile_max_tokens() and self._tile_band_ok(x, m):
+                return "tile"
+            return "dense"
+        return "fused"
+
+    # -- call plan ---------------------------------------------------------
+
+    def _planned(self, x: torch.Tensor, m: int, band: str):
+        """Add this call to the layer's plan and let the plan issue it; None where it cannot."""
+        from .. import kernels
+        from ..kernels import plans
+
+        plan = self._plan
+        if plan is not None and plan.stale(self):
+            self._plan = plan = None
+        if plan is not None and band == "sliced" and (band, x.dtype) in plan.names:
+            return kernels.SlicedCallPlan(plan).run(x)  # the wrapper functions have been replaced
+        if m < 1 or band == "torch" or (band == "tile" and _tile_failed) or x.dtype not in plans.DTYPE_CODES or (
+            x.device != self.packed_indices.device or self.packed_indices.dtype != torch.uint8
+        ):  # fmt: skip
+            return None
+        if plan is None:
+            try:
+                plan = plans.make(
+                    self, _PLAN_ATTRIBUTES, globals(), _PLAN_THRESHOLDS,
+                    holders=[p for p in (self.proxy, self.residual_proxy) if p is not None],
+                    sources=(self.packed_indices, self.proxy.centroids, self.bias, self.column_perm, self.packed_residual,
+                             self.row_scale, self.row_bias, None if self.residual_proxy is None else self.residual_proxy.centroids),
+                )  # fmt: skip
+            except RuntimeError as exc:
+                self._fallback("call_plan", "the Python call path", exc)
+                return None
+            if plan is None:
+                return None
+        self._add_route(plan, x.dtype, m, band)
+        self._plan = plan
+        return None if plan.wrapped() else plan.run(x)
+
+    def _add_route(self, plan, dtype: torch.dtype, m: int, band: str) -> None:
+        from ..kernels import plans
+
+        tile = band == "tile" or (band == "fused" and m > _GEMV_KERNEL_MAX_TOKENS)
+        kind = "tile" if tile else band
+        number = plan.names.get((kind, dtype))
+        if number is None:
+            number = plan.names[kind, dtype] = self._template(plan, dtype, kind)
+        code = plans.DTYPE_CODES[dtype]
+        if band == "sliced":
+            sl, limit = self._derived_hit("sliced", self.packed_indices)
+            for tokens in range(1, min(limit, _SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)) + 1):
+                plan.route(code, tokens, number, sl.workspace_bytes(tokens))
+        else:
+            plan.route(code, m, number, plans.tile_scratch(m, self.out_features, self.in_features) if tile else 0)
+
+    def _template(self, plan, dtype: torch.dtype, kind: str) -> int:
+        from ..kernels import plans
+
+        n, k, vl = self.out_features, self.in_features, self.vector_len
+        code = plans.DTYPE_CODES[dtype]
+        packed, proxy = self.packed_indices.reshape(-1), self.proxy
+        perm = None if self.column_perm is None or kind in ("sliced", "gemv_perm") else self.column_perm
+        if kind == "sliced":
+            sl, _ = self._derived_hit("sliced", self.packed_indices)
+            i32 = None if self.column_perm is None else self._perm_i32(packed.device)
+            plan.hold(sl)  # the plan passes the address of its header
+            args = (i32, sl.header_ptr, sl.blob, proxy.centroids_as(dtype), code, self._bias_f32(), code)
+            return plans.template(plan, plans.SLICED, n, k, args, dtype)
+        if self.is_residual:
+            res = self._res_stream().reshape(-1)
+            cr = self._res_centroids()
+            args = (packed, packed.numel(), self.bits, res, res.numel(), self._res_bits(), proxy.centroids, proxy.num_centroids,
+                    cr, cr.shape[0], self.row_scale, self.row_bias, vl)  # fmt: skip
+            if kind == "dense":
+                return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=self._bias_as(dtype))
+            kind_code = plans.RVQ_TILE if kind == "tile" else plans.RVQ_GEMV
+            return plans.template(plan, kind_code, n, k, (*args, self._bias_f32(), code), dtype, perm=perm)
+        if kind == "dense":
+            args = (packed, packed.numel(), self.bits, proxy.centroids, proxy.num_centroids, vl, self.n_vectors)
+            return plans.template(plan, plans.VQ_DENSE, n, k, args, dtype, perm=perm, bias=self._bias_as(dtype))
+        stream, bits = self._kernel_stream()
+        stream = stream.reshape(-1)
+        args = (stream, stream.numel(), bits, proxy.centroids_as(dtype), code, proxy.num_centroids, vl, self._bias_f32(), code)
+        if kind == "gemv_perm":
+            return plans.template(plan, plans.VQ_GEMV_PERM, n, k, (*args, self._perm_i32(stream.device)), dtype)
+        return plans.template(plan, plans.VQ_TILE if kind == "tile" else plans.VQ_GEMV, n, k, args, dtype, perm=perm)
 
     # -- slice-list GEMV ---------------------------------------------------
 
@@ -768,6 +851,7 @@ class NPVQLinear(nn.Module):
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("NPVQLinear.prepare_sliced() copies to the host and back: call it before the capture")
         self._derive("sliced", self.packed_indices, self._build_sliced)
+        self._plan = None  # it may hold routes of the fused GEMV for the token counts the lists serve
         self.prepare()
         return True
 
@@ -947,26 +1031,7 @@ class NPVQLinear(nn.Module):
             if self.column_perm is not None:
                 x = x[..., self.column_perm]
             return self._forward_dequant_gemm(x)
-        if x.dtype not in self._plans and not torch.cuda.is_current_stream_capturing():
-            self._plan_sliced_calls(x.dtype, sliced, perm)
         return y.reshape(*leading, self.out_features)
-
-    def _plan_sliced_calls(self, dtype: torch.dtype, sliced, perm) -> None:
-        """Remember how the slice-list call for *dtype* activations was made, with the buffers it was
-        made from: forward() reuses it while those are the module's buffers and unwritten."""
-        from .. import kernels
-
-        hit = self._derived_hit("sliced", self.packed_indices)
-        if hit is None or hit[0] is not sliced:
-            return
-        packed, bias, column_perm, cent = self.packed_indices, self.bias, self.column_perm, self.proxy.centroids
-        plan = kernels.SlicedCallPlan(sliced, self.proxy.centroids_as(dtype), self._bias_f32(), perm, dtype,
-                                      min(hit[1], _SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)))  # fmt: skip
-        try:
-            versions = _versions_of(packed, bias, column_perm, cent)
-        except RuntimeError:  # inference tensors count no versions: writes into them go unseen, as for every cache here
-            versions = None
-        self._plans[dtype] = (plan, packed, bias, column_perm, cent, versions)
 
     def _mfma_layer(self) -> bool:
         """Whether the MFMA kernels take this layer's shape (vector length 8, K a multiple of 64)."""

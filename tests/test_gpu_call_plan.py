@@ -1,0 +1,105 @@
+"""The native call path (CallPlan): a layer's later calls give what its first one gives, and the plan steps aside
+when anything it was built from changes."""
+
+import copy
+
+import pytest
+import torch
+
+import neuropress_amd.nn.np_linear as qmod
+import neuropress_amd.nn.np_vq_linear as vqmod
+from neuropress_amd.nn import NPLinear, NPVQLinear, VQProxy
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(kind, gpu, act):
+    n, k = 96, 512
+    if kind == "q4":
+        Q = cases.q4_layer(5, n, k, act=act, bias=True)
+        return NPLinear(Q["blob"], Q["scale"], n, k, 32, 4, "sym", "cuda", bias=Q["bias"]).to(gpu)
+    if kind == "rvq":
+        R = cases.rvq_layer(6, n, k, act=act)
+        layer = NPVQLinear(VQProxy(R["cbm"]), R["pm"], R["bm"], n, k, 8, "cuda_wmma", residual_proxy=VQProxy(R["cbr"]),
+                           packed_residual=R["pr"], row_scale=R["scale"], row_bias=R["wbias"])  # fmt: skip
+    else:
+        nc, bits = {"vq8": (256, 8), "vq16": (20000, 16)}[kind.split("-")[0]]
+        V = cases.vq_layer(7, n, k, nc, bits=bits, act=act, bias=True, std=0.05)
+        perm = torch.randperm(k, generator=cases.gen(8)) if kind.endswith("perm") else None
+        layer = NPVQLinear(VQProxy(V["cb"]), V["packed"], bits, n, k, 8, "cuda_wmma", bias=V["bias"], column_perm=perm)
+    layer.proxy.to(gpu)
+    if layer.residual_proxy is not None:
+        layer.residual_proxy.to(gpu)
+    return layer.to(gpu)
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["vq8", "vq8-perm", "vq16", "vq16-perm", "rvq", "q4"])
+def test_planned_calls_equal_first_calls_and_follow_the_module(gpu, kind, act, monkeypatch):
+    monkeypatch.setattr(vqmod, "_SLICED_MIN_INDICES", 1)
+    monkeypatch.setattr(vqmod, "_TILE_MAX_TOKENS", 64)
+    monkeypatch.setattr(vqmod, "_TILE_MIN_GRID_FRACTION", 0.0)
+    monkeypatch.setattr(qmod, "_Q_TILE_MAX_TOKENS", 64)
+    monkeypatch.setattr(qmod, "_Q_TILE_MIN_GRID_FRACTION", 0.0)
+    layer = _layer(kind, gpu, act)
+    k = layer.in_features
+    for m in (1, 2, 9, 40, 130):  # every band
+        x = torch.randn(m, k, generator=cases.gen(m)).to(act).to(gpu)
+        layer._plan = None
+        first = layer(x)
+        plan = layer._plan
+        assert plan is not None and not plan.stale(layer)
+        assert torch.equal(layer(x), first)
+        assert torch.equal(plan(layer, x), first)  # the plan itself answers
+        assert torch.equal(plan(layer, x.reshape(m, 1, 1, k)), first.reshape(m, 1, 1, -1))
+        wide = torch.zeros(m, 3, k, dtype=act, device=gpu)
+        wide[:, 2] = x
+        strided = plan(layer, wide[:, 2:]).reshape(m, -1)  # rows at a stride; torch's dense product may sum in another order
+        assert torch.equal(strided, first) if m < 130 else torch.allclose(strided, first, rtol=2e-2, atol=2e-2)
+        if m > 1:
+            assert plan(layer, wide[:, :2]) is None  # two row distances: not a stack of rows
+        assert plan(layer, x.cpu()) is None and plan(layer, x.double()) is None and plan(layer, x[:, : k // 2]) is None
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            side.wait_stream(torch.cuda.current_stream())
+            torch.cuda.synchronize()
+            assert torch.equal(layer(x), first) and torch.equal(layer(x), first)
+        torch.cuda.synchronize()
+        copied = copy.deepcopy(layer)
+        assert copied._plan is None  # it may run another kernel: the slice lists are not its buffers'
+        assert torch.allclose(copied(x), first, rtol=2e-2, atol=2e-2)
+        layer.bias = None if layer.bias is None else layer.bias + 1  # another tensor in the buffer's place
+        if layer.bias is not None:
+            assert plan.stale(layer) and plan(layer, x) is None
+            assert not torch.equal(layer(x), first)
+            layer.bias = layer.bias - 1
+        backend, layer.backend = layer.backend, layer.backend.__class__("default")
+        assert plan(layer, x) is None
+        layer(x)
+        layer.backend = backend
+
+
+def test_planned_norm_and_lookups(gpu):
+    from neuropress_amd.nn.np_embedding import NPEmbedding
+    from neuropress_amd.nn.np_rms_norm import NPRMSNorm
+    from neuropress_amd.nn.np_vq_embedding import NPVQEmbedding
+
+    g = cases.gen(9)
+    norm = NPRMSNorm(torch.rand(320, generator=g).half() + 0.5, 1e-5).to(gpu)
+    for m in (1, 77):
+        x = torch.randn(m, 320, generator=g).half().to(gpu)
+        first = norm(x)
+        assert torch.equal(norm._plan(norm, x), first)
+    norm.eps = 1.0
+    assert norm._plan(norm, x) is None and not torch.equal(norm(x), first)
+    Q = cases.q4_layer(10, 300, 256)
+    proxy = VQProxy((torch.randn(1000, 8, generator=g) * 0.05).half()).to(gpu)
+    tab = torch.randint(0, 1000, (300, 32), generator=g)
+    for emb in (NPVQEmbedding(tab, proxy, 256, 8, out_dtype=torch.bfloat16).to(gpu),
+                NPEmbedding(Q["blob"], Q["scale"], 300, 256, 32, 4, "sym", "cuda", padding_idx=3).to(gpu)):  # fmt: skip
+        for shape in ((1,), (3, 5)):
+            ids = torch.randint(0, 300, shape, generator=g).to(gpu)
+            first = emb(ids)
+            assert first.shape == (*shape, 256) and torch.equal(emb._plan(emb, ids), first)
+            assert emb._plan(emb, ids.int()) is None and torch.equal(emb(ids.int()), first)
