@@ -328,7 +328,70 @@ int launch_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
   return check_launch("npamd_q_embedding");
 }
 
+// ---------------------------------------------------------------------------
+// Activations as the MFMA kernels read them: columns permuted and / or rows padded with zeros to a
+// whole number of 64-column chunks, 16-bit elements:
+//   out[m, k] = x[m, perm ? perm[k] : k] for k < K, 0 for K <= k < ldo.
+//
+// Bound by the launch at the token counts of a decode step and by HBM beyond.  A block takes 2048
+// output columns of one row.  With a permutation it first copies the whole row into LDS (one
+// contiguous read) and gathers there with 2-byte reads: through the vector memory path an element
+// gather costs a lane one cycle and a cache line each.  77 x 2184 with a permutation: 2.3 us where
+// torch's gather takes 4.2; 4096 x 3456: see the table of cases in the design notes.
+// ---------------------------------------------------------------------------
+constexpr int kGatherRowMax = 32768;  // elements of a row held in LDS (64 KiB)
+template <bool PERM, bool LDS>
+__global__ void __launch_bounds__(256)
+gather_columns_kernel(const uint16_t* __restrict__ x, int64_t ldx, const int32_t* __restrict__ perm,
+                      uint16_t* __restrict__ out, int64_t ldo, int K, bool vec) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t row_lds[];
+  const uint16_t* xr = x + (int64_t)blockIdx.y * ldx;
+  if constexpr (PERM && LDS) {
+    const int whole = vec ? K >> 3 : 0;
+    for (int i = threadIdx.x; i < whole; i += 256)
+      reinterpret_cast<u32x4*>(row_lds)[i] = reinterpret_cast<const u32x4*>(xr)[i];
+    for (int i = whole * 8 + threadIdx.x; i < K; i += 256) row_lds[i] = xr[i];
+    __syncthreads();
+    xr = row_lds;
+  }
+  const int k0 = (blockIdx.x * 256 + threadIdx.x) * 8;
+  if (k0 >= ldo) return;
+  uint16_t v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int k = k0 + e;
+    v[e] = 0;
+    if (k < K) v[e] = xr[PERM ? perm[k] : k];
+  }
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = (uint32_t)v[2 * e] | ((uint32_t)v[2 * e + 1] << 16);
+  *reinterpret_cast<u32x4*>(out + (int64_t)blockIdx.y * ldo + k0) = o;
+}
+
 }  // namespace
+
+extern "C" int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* out, int64_t ldo, int M, int K,
+                                    void* stream) {
+  NPAMD_REQUIRE(M >= 0 && K >= 0 && ldx >= K && ldo >= K, "npamd_gather_columns: bad shape [%d, %d]", M, K);
+  NPAMD_REQUIRE(ldo % 8 == 0 && ldo <= 0x7FFFFFFF - 2048, "npamd_gather_columns: output row stride must be a multiple of 8");
+  if (M == 0 || ldo == 0) return NPAMD_OK;
+  NPAMD_REQUIRE(x && out && aligned16(out), "npamd_gather_columns: null or unaligned pointer");
+  hipStream_t st = (hipStream_t)stream;
+  const bool vec = aligned16(x) && ldx % 8 == 0;
+  auto xs = (const uint16_t*)x;
+  auto os = (uint16_t*)out;
+  const unsigned segments = (unsigned)((ldo + 2047) / 2048);
+  for (int m0 = 0; m0 < M; m0 += 65535) {
+    const dim3 grid(segments, (unsigned)(M - m0 < 65535 ? M - m0 : 65535));
+    const uint16_t* xm = xs + (int64_t)m0 * ldx;
+    uint16_t* om = os + (int64_t)m0 * ldo;
+    if (!perm) gather_columns_kernel<false, false><<<grid, 256, 0, st>>>(xm, ldx, perm, om, ldo, K, vec);
+    else if (K <= kGatherRowMax) gather_columns_kernel<true, true><<<grid, 256, (K * 2 + 15) & ~15, st>>>(xm, ldx, perm, om, ldo, K, vec);
+    else gather_columns_kernel<true, false><<<grid, 256, 0, st>>>(xm, ldx, perm, om, ldo, K, vec);
+  }
+  return check_launch("npamd_gather_columns");
+}
 
 extern "C" int npamd_rms_norm(const void* x, int64_t ldx, const void* weight, void* out, int64_t ldo, int M, int H,
                               float eps, int dtype, void* stream) {

@@ -88,11 +88,12 @@ int64_t version_of(const at::Tensor& t) {
 
 struct Template {
   Kind kind;
-  int64_t n, k;                     // output and input features (embedding lookups: row length, 1)
+  int64_t n, k;                     // output features, columns the kernel contracts (embedding lookups: row length, 1)
+  int64_t k_in;                     // columns of x: fewer than k where rows are padded to whole 64-column chunks
   std::vector<int64_t> a;           // constant arguments
   double f;                         // eps of a norm, scale of an embedding
   at::ScalarType out;
-  at::Tensor perm;                  // int64 column permutation applied to x first, or undefined
+  at::Tensor perm;                  // column permutation applied to x first, or undefined: int32 (16-bit x) or int64
   at::Tensor bias;                  // bias of the dense product, or undefined
   std::vector<at::Tensor> keep;     // what the addresses point into
 };
@@ -168,12 +169,19 @@ using I32 = const int32_t*;
 bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m, int64_t ldx, int device, at::Tensor* out) {
   const std::vector<int64_t>& a = t.a;
   hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+  c10::SmallVector<int64_t, 6> sizes(x_in.sizes().begin(), x_in.sizes().end());
   at::Tensor x = x_in;
-  if (t.perm.defined()) {
+  if (t.perm.defined() && t.perm.scalar_type() == at::kLong) {
     x = at::index_select(x_in, -1, t.perm);
     ldx = t.k;
+  } else if (t.perm.defined() || t.k_in != t.k) {
+    sizes.back() = t.k;
+    x = empty(sizes, x_in.scalar_type(), device);
+    if (npamd_gather_columns(x_in.const_data_ptr(), ldx, t.perm.defined() ? t.perm.const_data_ptr<int32_t>() : nullptr, x.data_ptr(),
+                             t.k, (int)m, (int)t.k_in, st) != NPAMD_OK)
+      return false;
+    ldx = t.k;
   }
-  c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
   if (t.kind == kVqEmbedding || t.kind == kQEmbedding) sizes.push_back(t.n);
   else sizes.back() = t.n;
 
@@ -322,7 +330,7 @@ PyObject* run(Plan* p, PyObject* xo) {
   }
   const Route route = it->second;
   const Template& t = (*p->templates)[(size_t)route.tmpl];
-  if (t.k != k) Py_RETURN_NONE;
+  if (t.k_in != k) Py_RETURN_NONE;
   try {
     at::Tensor y;
     if (!issue(t, route, x, m, ldx, p->device, &y)) Py_RETURN_NONE;
@@ -484,14 +492,14 @@ PyObject* plan_hold(PyObject* self, PyObject* o) {
   Py_RETURN_NONE;
 }
 
-// template(kind, n, k, args, f, out_dtype_code, perm or None, bias or None, keep) -> number
+// template(kind, n, k, k_in, args, f, out_dtype_code, perm or None, bias or None, keep) -> number
 PyObject* plan_template(PyObject* self, PyObject* args) {
   Plan* p = reinterpret_cast<Plan*>(self);
   int kind, out_code;
-  long long n, k;
+  long long n, k, k_in;
   double f;
   PyObject *ints, *perm, *bias, *keep;
-  if (!PyArg_ParseTuple(args, "iLLO!diOOO!", &kind, &n, &k, &PyTuple_Type, &ints, &f, &out_code, &perm, &bias, &PyTuple_Type, &keep))
+  if (!PyArg_ParseTuple(args, "iLLLO!diOOO!", &kind, &n, &k, &k_in, &PyTuple_Type, &ints, &f, &out_code, &perm, &bias, &PyTuple_Type, &keep))
     return nullptr;
   if (kind < 0 || kind >= kKinds || (int)PyTuple_GET_SIZE(ints) > kArgs[kind]) {
     PyErr_SetString(PyExc_ValueError, "template(): bad kind or argument count");
@@ -501,6 +509,7 @@ PyObject* plan_template(PyObject* self, PyObject* args) {
   t.kind = (Kind)kind;
   t.n = n;
   t.k = k;
+  t.k_in = k_in;
   t.f = f;
   t.out = scalar_type(out_code);
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(ints); ++i) {
@@ -552,7 +561,7 @@ PyMethodDef plan_methods[] = {
     {"guard_module", plan_guard_module, METH_O, "guard_module({attribute: expected})"},
     {"source", plan_source, METH_O, "source(tensor or None)"},
     {"hold", plan_hold, METH_O, "hold(object)"},
-    {"template", plan_template, METH_VARARGS, "template(kind, n, k, args, f, out, perm, bias, keep) -> number"},
+    {"template", plan_template, METH_VARARGS, "template(kind, n, k, k_in, args, f, out, perm, bias, keep) -> number"},
     {"route", plan_route, METH_VARARGS, "route(dtype, tokens, template, scratch_bytes)"},
     {"stale", plan_stale, METH_O, "stale(module): whether anything the plan was built from has changed"},
     {"wrapped", plan_wrapped, METH_NOARGS, "wrapped(): whether a wrapper function has been replaced"},

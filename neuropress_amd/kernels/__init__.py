@@ -847,6 +847,22 @@ def warn_kernel_fallback(kernel: str, fallback: str, exc: BaseException) -> None
 # ---------------------------------------------------------------------------
 
 
+def gather_columns(x: torch.Tensor, perm: torch.Tensor | None, width: int) -> torch.Tensor:
+    """``x[:, perm]`` (``x`` with *perm* None) of a 2-D 16-bit *x*, rows padded with zeros to *width* columns, a
+    multiple of 8 (``npamd_gather_columns``).  *perm*: int32 ``[K]``."""
+    what = "gather_columns"
+    _check_device(what, x, perm)
+    x = _x2d(x, what)
+    if x.element_size() != 2:
+        raise RuntimeError(f"{what}: x must have 16-bit elements, got {x.dtype}")
+    m, k = x.shape
+    if perm is not None and (perm.dtype != torch.int32 or perm.numel() != k or not perm.is_contiguous()):
+        raise RuntimeError(f"{what}: perm must be a contiguous int32 tensor of K={k} entries")
+    out = torch.empty((m, width), device=x.device, dtype=x.dtype)
+    _lib.call("npamd_gather_columns", x.data_ptr(), x.stride(0), _ptr(perm), out.data_ptr(), width, m, k, _stream(x))
+    return out
+
+
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """Fused RMSNorm over the last dimension of a 2-D ``x`` (reference: neuropress/kernels/__init__.py
     ``rms_norm``, kernels/rms_norm.cu:79-118: same checks, same signature)."""

@@ -667,19 +667,34 @@ class NPVQLinear(nn.Module):
     def _kernel_stream(self) -> tuple[torch.Tensor, int]:
         """Index stream and width the fused kernels read.
 
-        Widths outside {4, 8, 12, 16} are widened to a 16-bit stream once per
+        Widths outside {4, 8, 12, 16}, and layers whose K is not a whole number of
+        64-column chunks, are widened to a 16-bit stream once per
         device so they take the vectorised index loads (precedent: the
         reference re-lays index streams out at construction, np_vq_linear.py:644-696).
+        Rows of the latter are padded to :meth:`_kernel_k` columns by repeating their last index:
+        the activations are zero there.
         """
-        if self.bits in _FAST_BITS or self.bits > 16:
+        pad = (self._kernel_k() - self.in_features) // self.vector_len
+        if (self.bits in _FAST_BITS or self.bits > 16) and pad == 0:
             return self.packed_indices, self.bits
         from .. import kernels
 
-        wide = self._derive(
-            "wide", self.packed_indices,
-            lambda: kernels.widen_indices_u16(self.packed_indices, self.n_vectors, self.bits),
-        )  # fmt: skip
-        return wide, 16
+        def widen() -> torch.Tensor:
+            wide = kernels.widen_indices_u16(self.packed_indices, self.n_vectors, self.bits)
+            if pad:
+                rows = wide.view(torch.int16).reshape(self.out_features, -1)
+                wide = torch.cat([rows, rows[:, -1:].expand(-1, pad)], 1).reshape(-1).view(torch.uint8)
+            return wide
+
+        return self._derive("wide", self.packed_indices, widen), 16
+
+    def _kernel_k(self) -> int:
+        """Columns the MFMA kernels contract: K, rounded up to whole 64-column chunks where the layer is otherwise
+        of a form they take (vector length 8 or 4, at most 16 bits per index, no residual stream)."""
+        k = self.in_features
+        if k % 64 == 0 or self.vector_len not in (4, 8) or self.bits > 16 or self.is_residual or self.n_vectors == 0:
+            return k
+        return k + 64 - k % 64
 
     # ------------------------------------------------------------------
     # Forward
@@ -792,7 +807,7 @@ class NPVQLinear(nn.Module):
             for tokens in range(1, min(limit, _SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)) + 1):
                 plan.route(code, tokens, number, sl.workspace_bytes(tokens))
         else:
-            plan.route(code, m, number, plans.tile_scratch(m, self.out_features, self.in_features) if tile else 0)
+            plan.route(code, m, number, plans.tile_scratch(m, self.out_features, self._kernel_k()) if tile else 0)
 
     def _template(self, plan, dtype: torch.dtype, kind: str) -> int:
         from ..kernels import plans
@@ -800,7 +815,9 @@ class NPVQLinear(nn.Module):
         n, k, vl = self.out_features, self.in_features, self.vector_len
         code = plans.DTYPE_CODES[dtype]
         packed, proxy = self.packed_indices.reshape(-1), self.proxy
-        perm = None if self.column_perm is None or kind in ("sliced", "gemv_perm") else self.column_perm
+        perm = None
+        if self.column_perm is not None and kind not in ("sliced", "gemv_perm"):
+            perm = self.column_perm if dtype == torch.float32 else self._perm_i32(packed.device)
         if kind == "sliced":
             sl, _ = self._derived_hit("sliced", self.packed_indices)
             i32 = None if self.column_perm is None else self._perm_i32(packed.device)
@@ -816,15 +833,18 @@ class NPVQLinear(nn.Module):
                 return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=self._bias_as(dtype))
             kind_code = plans.RVQ_TILE if kind == "tile" else plans.RVQ_GEMV
             return plans.template(plan, kind_code, n, k, (*args, self._bias_f32(), code), dtype, perm=perm)
-        if kind == "dense":
-            args = (packed, packed.numel(), self.bits, proxy.centroids, proxy.num_centroids, vl, self.n_vectors)
-            return plans.template(plan, plans.VQ_DENSE, n, k, args, dtype, perm=perm, bias=self._bias_as(dtype))
         stream, bits = self._kernel_stream()
         stream = stream.reshape(-1)
+        if kind == "dense":
+            if self._kernel_k() != k:  # the dense product takes any K: no padding
+                stream, bits = packed, self.bits
+            args = (stream, stream.numel(), bits, proxy.centroids, proxy.num_centroids, vl, self.n_vectors)
+            return plans.template(plan, plans.VQ_DENSE, n, k, args, dtype, perm=perm, bias=self._bias_as(dtype))
         args = (stream, stream.numel(), bits, proxy.centroids_as(dtype), code, proxy.num_centroids, vl, self._bias_f32(), code)
         if kind == "gemv_perm":
             return plans.template(plan, plans.VQ_GEMV_PERM, n, k, (*args, self._perm_i32(stream.device)), dtype)
-        return plans.template(plan, plans.VQ_TILE if kind == "tile" else plans.VQ_GEMV, n, k, args, dtype, perm=perm)
+        kind_code = plans.VQ_TILE if kind == "tile" else plans.VQ_GEMV
+        return plans.template(plan, kind_code, n, self._kernel_k(), args, dtype, k_in=k, perm=perm)
 
     # -- slice-list GEMV ---------------------------------------------------
 
@@ -930,7 +950,8 @@ class NPVQLinear(nn.Module):
                 x = torch.ones(m, self.in_features, dtype=dt, device=dev)
                 ws = torch.zeros(sl.workspace_bytes(m) // 4, dtype=torch.float32, device=dev)
                 t_sliced = timed(lambda: kernels.vq_linear_sliced(x, sl, cb, workspace=ws))
-                t_fused = timed(lambda: kernels.vq_linear(x, stream, cb, bits, self.vector_len, None, self.out_features))
+                xf = kernels.gather_columns(x, None, self._kernel_k()) if self._kernel_k() != self.in_features else x
+                t_fused = timed(lambda: kernels.vq_linear(xf, stream, cb, bits, self.vector_len, None, self.out_features))
                 if t_sliced >= t_fused:
                     break
                 limit = m
@@ -993,7 +1014,7 @@ class NPVQLinear(nn.Module):
             from .. import kernels
 
             rows = max(1, self.proxy.num_centroids * self.vector_len // 8)  # table size in rows of eight
-            hit = (m, kernels.gemv_stages_activations(m, self.out_features, self.in_features, rows))
+            hit = (m, kernels.gemv_stages_activations(m, self.out_features, self._kernel_k(), rows))
             self._derived["stages"] = hit
         return hit[1]
 
@@ -1034,13 +1055,14 @@ class NPVQLinear(nn.Module):
         return y.reshape(*leading, self.out_features)
 
     def _mfma_layer(self) -> bool:
-        """Whether the MFMA kernels take this layer's shape (vector length 8, K a multiple of 64)."""
+        """Whether the MFMA kernels take this layer's shape."""
         ok = self._derived.get("mfma_layer")
         if ok is None:
             from .. import kernels
 
-            bits = self.bits if (self.bits in _FAST_BITS or self.bits > 16) else 16  # as _kernel_stream
-            ok = kernels.vq_fused_supported(self.in_features, self.vector_len, bits)
+            k = self._kernel_k()
+            bits = self.bits if k == self.in_features and (self.bits in _FAST_BITS or self.bits > 16) else 16  # as _kernel_stream
+            ok = kernels.vq_fused_supported(k, self.vector_len, bits)
             self._derived["mfma_layer"] = ok
         return ok
 
@@ -1079,7 +1101,7 @@ class NPVQLinear(nn.Module):
             cus = torch.cuda.get_device_properties(x.device).multi_processor_count
             self._derived["cus"] = cus
         return tile_band_ok(
-            m, self.out_features, self.in_features, cus,
+            m, self.out_features, self._kernel_k(), cus,
             _TILE_MIN_GRID_FRACTION, _TILE_SPLIT_MAX_TOKENS, _TILE_SPLIT_LONG_K,
         )  # fmt: skip
 
@@ -1194,6 +1216,8 @@ class NPVQLinear(nn.Module):
             )  # fmt: skip
         else:
             stream, bits = self._kernel_stream()
+            if self._kernel_k() != self.in_features:
+                x2d = kernels.gather_columns(x2d, None, self._kernel_k())
             cb = self.proxy.centroids_as(x.dtype)
             fn = kernels.vq_gemm_tile if tile else kernels.vq_linear
             if tile:

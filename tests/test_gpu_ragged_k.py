@@ -1,0 +1,58 @@
+"""Layers whose K is not a whole number of 64-column chunks: the index stream is padded once, the activations per
+call (together with the column permutation), and every band then computes with zeros past K."""
+
+import pytest
+import torch
+
+import neuropress_amd.nn.np_vq_linear as vqmod
+from neuropress_amd.nn import NPVQLinear, VQProxy
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("width", [0, 8, 24])
+@pytest.mark.parametrize("k", [8, 40, 1000, 2184, 33000])
+def test_gather_columns(gpu, k, width):
+    from neuropress_amd import kernels
+
+    g = cases.gen(k)
+    wide = (k + 7) // 8 * 8 + width
+    big = torch.randn(3, k + 5, generator=g).half().to(gpu)
+    perm = torch.randperm(k, generator=g).to(gpu)
+    for x in (big[:, :k].contiguous(), big[:, 5:]):  # 16-byte aligned rows, and rows that are not
+        for p in (None, perm):
+            out = kernels.gather_columns(x, None if p is None else p.int(), wide)
+            assert torch.equal(out[:, :k], x if p is None else x[:, p]) and not out[:, k:].any()
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k,nc,vl,perm", [(70, 8, 16, 8, False), (130, 200, 1000, 8, True), (257, 1000, 4096, 4, False),
+                                            (64, 2184, 65536, 8, True), (96, 1544, 300, 8, False)])  # fmt: skip
+def test_ragged_k_runs_the_fused_bands(gpu, n, k, nc, vl, perm, act, monkeypatch):
+    from neuropress_amd import kernels
+
+    monkeypatch.setattr(vqmod, "_TILE_MIN_GRID_FRACTION", 0.0)
+    L = cases.vq_layer(n + k, n, k, nc, vl=vl, bias=True, act=act, std=0.05)
+    cp = torch.randperm(k, generator=cases.gen(k)) if perm else None
+    layer = NPVQLinear(VQProxy(L["cb"]).to(gpu), L["packed"], L["bits"], n, k, vl, "cuda_wmma", bias=L["bias"].float(),
+                       column_perm=cp).to(gpu)  # fmt: skip
+    w = L["cb"][L["idx"]].reshape(n, k).to(act).float()
+    used = []
+    for m in (1, 3, 17, 40, 100, 400):
+        x = torch.randn(m, k, generator=cases.gen(m)).to(act)
+        ref = torch.nn.functional.linear((x if cp is None else x[:, cp]).float(), w, L["bias"].float())
+        for call in range(2):  # the first call and the planned one
+            y = layer(x.to(gpu)).float().cpu()
+            err = (y - ref).abs()
+            assert bool((err <= 1e-2 + 1e-2 * ref.abs()).all()), (m, call, float(err.max()))
+        # rows of x with a stride, and the wrappers in place of the plan
+        with monkeypatch.context() as mp:
+            for name in ("vq_linear", "vq_gemm_tile"):
+                real = getattr(kernels, name)
+                mp.setattr(kernels, name, lambda *a, _r=real, _n=name, **kw: (used.append((m, _n)), _r(*a, **kw))[1])
+            xs = torch.zeros(m, k + 3, dtype=act)
+            xs[:, :k] = x
+            y2 = layer(xs.to(gpu)[:, :k]).float().cpu()
+            assert bool(((y2 - ref).abs() <= 1e-2 + 1e-2 * ref.abs()).all()), m
+    assert used == [(1, "vq_linear"), (3, "vq_linear"), (17, "vq_linear"), (40, "vq_gemm_tile"), (100, "vq_gemm_tile")]
