@@ -400,6 +400,17 @@ int npamd_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
 int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* out, int64_t ldo, int M, int K,
                          void* stream);
 
+/*
+ * Dense product of the decode + GEMM band: y[m, n] = sum_k x[m, k] w[n, k] (+ bias[n]), f32 accumulate, on a weight a
+ * *_dequant entry point has written (the reference calls F.linear there, neuropress/nn/np_vq_linear.py:1148).
+ * x, w, y: act_dtype (NPAMD_F16 or NPAMD_BF16); K a multiple of 64; x and w 16-byte aligned, ldx and ldw multiples of 8.
+ */
+int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
+                     int M, int N, int K, int act_dtype, void* stream);
+
+/* 1 where npamd_dense_gemm is the better choice for this shape against a library GEMM.  Host-only arithmetic. */
+int npamd_dense_gemm_preferred(int M, int N, int K);
+
 #ifdef __cplusplus
 }
 #endif

@@ -59,6 +59,7 @@ static Tuning read_tuning() {
   t.q4_rowwise = env_int("NPAMD_Q4_ROWWISE", 1);
   t.q4_rowwise_bf16 = env_int("NPAMD_Q4_ROWWISE_BF16", 0);
   t.q4_stream = env_int("NPAMD_Q4_STREAM", 1);
+  t.dense_tile = env_int("NPAMD_DENSE_TILE", 0);
   return t;
 }
 

@@ -1,0 +1,336 @@
+// Dense MFMA GEMM of the decode + GEMM band: y = x @ W^T (+ bias) on a weight that the one-pass decode has just
+// written, f32 accumulate.
+//
+// What bounds the band's small and middle shapes in a library GEMM is not the arithmetic: a few dozen output tiles
+// leave most compute units idle, each walks all of K with little in flight, and the call costs the host more than
+// both kernels together.  Here a block keeps one output tile and splits K over groups of waves inside the block
+// (group g takes every KG-th 64-k step): a small tile then has 8 waves and up to 128 KiB of operands on their way,
+// and the groups' sums meet in LDS, in group order, without a second kernel or a workspace.
+//
+// Both operand tiles are loaded straight into LDS (global_load_lds_dwordx4; rows of 128 bytes, 16-byte piece p of
+// row r in slot p ^ ((r >> 1) & 7), so that a read of 32 consecutive rows touches every bank group twice), a ring of
+// kStages steps per group; one in-order counter tracks a wave's loads and the waits are written by hand.  A wave
+// computes 32 MT x 64 of the tile (MFMA 32x32x16), reading the operands of a k group while it multiplies the one
+// before.  The row tiles of a column tile go to one die (workgroups go to the eight dies in turn), so that a die's L2
+// fetches a column tile of W once for all row tiles.
+#include <math.h>
+
+#include <type_traits>
+
+#include "gemm_tile.hpp"
+
+namespace npamd {
+
+namespace {
+
+__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
+}
+// Lane l's 16 bytes land at dst + 16 l; dst is uniform over the wave.  The statement writes m0, which an asm
+// statement cannot declare as clobbered: sound while the compiler keeps nothing of its own in m0 in this kernel.
+__device__ __forceinline__ void lds_load16(uint32_t dst, uint32_t voff, const void* base) {
+  dst = __builtin_amdgcn_readfirstlane(dst);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(base) : "memory");
+}
+
+struct DenseShape {
+  const void* x;
+  const void* w;
+  const float* bias;
+  void* y;
+  int64_t ldx, ldw, ldy;
+  int M, N, steps;   // steps = K / 64
+  int row_tiles, col_tiles, tiles_per_die;
+};
+
+template <int WGM, int WGN, int MT, int KG, int STAGES>
+struct DenseTile {
+  static constexpr int kBM = 32 * MT * WGM, kBN = 64 * WGN;
+  static constexpr int kWaves = WGM * WGN;  // of one K group
+  static constexpr int kThreads = 64 * kWaves * KG;
+  static constexpr int kStageBytes = (kBM + kBN) * 128;
+  static constexpr int kLoadsX = kBM / 8 / kWaves, kLoadsW = kBN / 8 / kWaves;  // per wave and step
+  static constexpr int kRedBytes = (KG - 1) * kBM * kBN * 4;
+  static constexpr int kEpBytes = kBM * kBN * 2;
+  static constexpr int kRingBytes = KG * STAGES * kStageBytes;
+  static constexpr int kLds = kRingBytes > kRedBytes + kEpBytes ? kRingBytes : kRedBytes + kEpBytes;
+  static_assert(kBM / 8 % kWaves == 0 && kBN / 8 % kWaves == 0, "every wave loads whole pieces of one operand at a time");
+  // The first operands of a step are read before its barrier where the ring is deep enough for a step to arrive one
+  // barrier early with two more on their way (128 x 64 tiles, ring of six: 23.0 -> 20.7 us on 384 x 4096 x 4096; 64 x 128
+  // in two groups, ring of three: 19.9 -> 29.3, the loads no longer cover the memory's latency).
+  static constexpr bool kAhead = STAGES >= 5;
+  static_assert(kLds <= kLdsPerBlockMax, "the block's tiles do not fit LDS");
+};
+
+template <int ACT, int WGM, int WGN, int MT, int KG, int STAGES>
+__global__ void __launch_bounds__((DenseTile<WGM, WGN, MT, KG, STAGES>::kThreads))
+dense_gemm_kernel(const DenseShape s) {
+  using T = DenseTile<WGM, WGN, MT, KG, STAGES>;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  // blockIdx.x % 8 names the die; a die takes an eighth of the tiles, counted down the columns
+  const int tile = (blockIdx.x & 7) * s.tiles_per_die + (blockIdx.x >> 3);
+  const int ct = tile / s.row_tiles, rt = tile % s.row_tiles;
+  if (ct >= s.col_tiles) return;
+  const int m0 = rt * T::kBM, n0 = ct * T::kBN;
+
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = wave_all / T::kWaves, wave = wave_all % T::kWaves;
+  const int wm = wave % WGM, wn = wave / WGM;
+  const int c = lane & 31, h = lane >> 5;
+
+  const int steps_g = (s.steps - g + KG - 1) / KG;  // this group's steps: g, g + KG, ...
+  const int base = s.steps / KG;                    // steps every group has
+  const uint8_t* const xb = reinterpret_cast<const uint8_t*>(s.x) + (int64_t)m0 * s.ldx * 2;
+  const uint8_t* const wb = reinterpret_cast<const uint8_t*>(s.w) + (int64_t)n0 * s.ldw * 2;
+  uint32_t voff[T::kLoadsX + T::kLoadsW];
+#pragma unroll
+  for (int i = 0; i < T::kLoadsX + T::kLoadsW; ++i) {
+    const bool is_x = i < T::kLoadsX;
+    const int r = (wave + T::kWaves * (is_x ? i : i - T::kLoadsX)) * 8 + (lane >> 3);
+    const int row = is_x ? min(r, s.M - 1 - m0) : min(r, s.N - 1 - n0);  // rows past the end: a valid row nobody stores
+    voff[i] = (uint32_t)((int64_t)row * (is_x ? s.ldx : s.ldw) * 2) + (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
+  }
+  const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + (uint32_t)(g * STAGES * T::kStageBytes);
+  auto load = [&](int i, int slot, int it) {
+    const bool is_x = i < T::kLoadsX;
+    const uint8_t* src = uniform_ptr((is_x ? xb : wb) + (int64_t)(g + KG * it) * 128);
+    const uint32_t piece = (uint32_t)((is_x ? 0 : T::kBM / 8) + wave + T::kWaves * (is_x ? i : i - T::kLoadsX));
+    lds_load16(ring + (uint32_t)(slot * T::kStageBytes) + piece * 1024u, voff[i], src);
+  };
+
+  f32x16 acc[MT][2];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mt][t][i] = 0.f;
+
+  constexpr int kLoads = T::kLoadsX + T::kLoadsW;
+#pragma unroll
+  for (int p = 0; p < STAGES - 1; ++p)
+    if (p < steps_g) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) load(i, p, p);
+    }
+
+  uint32_t slot_off[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) slot_off[j] = (uint32_t)((((h << 2) | j) ^ ((c >> 1) & 7)) << 4);
+  const uint8_t* const ring_p = lds + g * STAGES * T::kStageBytes;
+  const uint32_t a_off = (uint32_t)((wm * 32 * MT + c) * 128), b_off = (uint32_t)((T::kBM + wn * 64 + c) * 128);
+  u32x4 ao[2][MT], bo[2][2];
+  auto read_ops = [&](int set, const uint8_t* stage, int j) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) bo[set][t] = *reinterpret_cast<const u32x4*>(stage + b_off + t * 4096 + slot_off[j]);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) ao[set][mt] = *reinterpret_cast<const u32x4*>(stage + a_off + mt * 4096 + slot_off[j]);
+  };
+
+  // One step out of ring slot `slot`: the operands of k group j + 1 are read in front of the MFMAs of group j, those of
+  // the next step's first group in front of the last MFMAs (its pieces have arrived one barrier early), and with
+  // LOADS the pieces of step `ahead` are requested behind them, into the slot of the step before this one.
+  auto compute = [&](auto loads, int slot, int ahead) {
+    constexpr bool LOADS = decltype(loads)::value;
+    const uint8_t* const stage = ring_p + slot * T::kStageBytes;
+    const uint8_t* const next = ring_p + (slot == STAGES - 1 ? 0 : slot + 1) * T::kStageBytes;
+    const int into = slot == 0 ? STAGES - 1 : slot - 1;
+    if (!T::kAhead) read_ops(0, stage, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j < 3) read_ops((j + 1) & 1, stage, j + 1);
+      else if (T::kAhead) read_ops(0, next, 0);  // behind the last step: nothing anybody uses
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt][t] = mfma32<ACT>(ao[j & 1][mt], bo[j & 1][t], acc[mt][t]);
+        if constexpr (LOADS) {
+#pragma unroll
+          for (int i = (j * 2 + t) * kLoads / 8; i < (j * 2 + t + 1) * kLoads / 8; ++i) load(i, into, ahead);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // The wave's own pieces of a step have arrived when only those of `young` younger steps are still on their way.
+  // With kAhead every barrier stands for two steps: the one that follows and the one whose first operands that one reads.
+  auto wait_young = [&](int young) {
+    if (young >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * kLoads < 63 ? 3 * kLoads : 63) : "memory");
+    else if (young == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoads) : "memory");
+    else if (young == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+  int slot = 0;
+  auto next_slot = [&] { slot = slot == STAGES - 1 ? 0 : slot + 1; };
+  int it = 0;
+  if constexpr (T::kAhead) {
+    wait_young(min(steps_g, STAGES - 1) - 1);
+    block_sync_lds();
+    read_ops(0, ring_p, 0);
+  }
+  // Steps every group has, while there is something left to request.
+  for (; it < base - (STAGES - 1); ++it) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2 - T::kAhead) * kLoads) : "memory");
+    block_sync_lds();  // everybody's pieces have arrived, and nobody reads the slot of the step before any more
+    compute(std::true_type{}, slot, it + STAGES - 1);
+    next_slot();
+  }
+  for (; it < base; ++it) {
+    wait_young(base - 1 - T::kAhead - it);
+    block_sync_lds();
+    if (it + STAGES - 1 < steps_g) {  // the last step of a group that has one more than the others
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) load(i, slot == 0 ? STAGES - 1 : slot - 1, it + STAGES - 1);
+    }
+    compute(std::false_type{}, slot, 0);
+    next_slot();
+  }
+  if (KG > 1 && s.steps % KG) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    block_sync_lds();
+    if (base < steps_g) compute(std::false_type{}, slot, 0);
+  }
+
+  // The groups' sums meet in group 0, in group order.
+  __syncthreads();
+  if constexpr (KG > 1) {
+    if (g > 0) {
+      float* mine = reinterpret_cast<float*>(lds) + ((size_t)(g - 1) * T::kWaves + wave) * (MT * 2 * 1024) + lane * 4;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<f32x4*>(mine + ((mt * 2 + t) * 4 + q) * 256) =
+                f32x4{acc[mt][t][4 * q], acc[mt][t][4 * q + 1], acc[mt][t][4 * q + 2], acc[mt][t][4 * q + 3]};
+    }
+    __syncthreads();
+    if (g > 0) return;
+#pragma unroll
+    for (int o = 0; o < KG - 1; ++o) {
+      const float* theirs = reinterpret_cast<const float*>(lds) + ((size_t)o * T::kWaves + wave) * (MT * 2 * 1024) + lane * 4;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(theirs + ((mt * 2 + t) * 4 + q) * 256);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[mt][t][4 * q + e] += v[e];
+          }
+    }
+  }
+  store_wave_tile<ACT, MT, 2>(acc, lds + T::kRedBytes + wave * (32 * MT * 128), lane, s.y, s.ldy, m0 + wm * 32 * MT, n0 + wn * 64,
+                              s.M, s.N, s.bias);
+}
+
+template <int ACT, int WGM, int WGN, int MT, int KG, int STAGES>
+int launch_dense_tile(DenseShape s, hipStream_t st) {
+  using T = DenseTile<WGM, WGN, MT, KG, STAGES>;
+  s.row_tiles = (s.M + T::kBM - 1) / T::kBM;
+  s.col_tiles = (s.N + T::kBN - 1) / T::kBN;
+  const int64_t tiles = (int64_t)s.col_tiles * s.row_tiles, blocks = (tiles + 7) / 8 * 8;
+  s.tiles_per_die = (int)(blocks / 8);
+  if (blocks > 0x7FFFFFFF) return fail(NPAMD_ERR_UNSUPPORTED, "npamd_dense_gemm: too many tiles");
+  static LdsLatch latch;
+  const hipError_t e = enable_dynamic_lds(latch, reinterpret_cast<const void*>(&dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES>), T::kLds);
+  if (e != hipSuccess)
+    return fail(NPAMD_ERR_LAUNCH, "npamd_dense_gemm: cannot reserve %d bytes of LDS: %s", T::kLds, hipGetErrorString(e));
+  dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES><<<(unsigned)blocks, T::kThreads, T::kLds, st>>>(s);
+  return check_launch("npamd_dense_gemm");
+}
+
+// The tiles there are and what a launch on each costs, us: fixed + per round of workgroups + hypot(step time, bytes
+// loaded / rate), fitted to 34 shapes of 64 to 4096 rows, 64 to 14336 columns and K of 64 to 14336 (the tile of least
+// estimate is at most 3 % slower than the best of them on every one; the estimates are within 15 % but for the shortest).
+// A round is one tile per compute unit of every die.  What the figures say: a 64-k step of a 64 x 128 tile costs 0.25 us
+// (0.11 of MFMAs, 0.16 to bring 24 KiB at 64 bytes per cycle into LDS), and all of them together load at 22-28 TB/s from the L2s.
+struct DenseCost {
+  int bm, bn, groups;
+  float fixed, per_step, per_mb, per_round;
+};
+constexpr DenseCost kDenseCost[] = {
+    {32, 64, 4, 1.78f, 0.445f, 0.038f, 1.79f},   // 4 waves
+    {64, 64, 2, 1.72f, 0.307f, 0.043f, 2.10f},   // 4 waves
+    {64, 128, 2, 1.48f, 0.499f, 0.036f, 1.97f},  // 8 waves
+    {128, 128, 1, 0.00f, 0.388f, 0.047f, 3.68f}, // 8 waves
+    {128, 128, 1, 0.00f, 0.375f, 0.045f, 4.55f}, // 4 waves
+    {256, 128, 1, 0.00f, 0.622f, 0.053f, 4.39f}, // 8 waves
+};
+constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]);
+
+template <int ACT>
+int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
+  switch (tile) {
+    case 0: return launch_dense_tile<ACT, 1, 1, 1, 4, 3>(s, st);
+    case 1: return launch_dense_tile<ACT, 2, 1, 1, 2, 5>(s, st);
+    case 2: return launch_dense_tile<ACT, 2, 2, 1, 2, 3>(s, st);
+    case 3: return launch_dense_tile<ACT, 4, 2, 1, 1, 5>(s, st);
+    case 4: return launch_dense_tile<ACT, 2, 2, 2, 1, 5>(s, st);
+    default: return launch_dense_tile<ACT, 4, 2, 2, 1, 3>(s, st);
+  }
+}
+
+// The tile of least estimate, and the estimate.
+int plan_dense_tile(int M, int N, int K, float* us) {
+  int best = 0;
+  float best_us = 1e30f;
+  for (int i = 0; i < kDenseTiles; ++i) {
+    const DenseCost& c = kDenseCost[i];
+    const double tiles = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const double rounds = ceil(ceil(tiles / 8) / 32), steps = K / 64;
+    const double walk = rounds * ceil(steps / c.groups) * c.per_step, load = tiles * steps * (c.bm + c.bn) * 128e-6 * c.per_mb;
+    const float t = (float)(c.fixed + rounds * c.per_round + sqrt(walk * walk + load * load));
+    if (t < best_us) {
+      best_us = t;
+      best = i;
+    }
+  }
+  if (us) *us = best_us;
+  return best;
+}
+
+}  // namespace
+}  // namespace npamd
+
+using namespace npamd;
+
+extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
+                                int M, int N, int K, int act_dtype, void* stream) {
+  const char* what = "npamd_dense_gemm";
+  NPAMD_REQUIRE(act_dtype == NPAMD_F16 || act_dtype == NPAMD_BF16, "%s: f16 or bf16 only", what);
+  NPAMD_REQUIRE(M >= 0 && N >= 0 && K >= 64 && K % 64 == 0, "%s: bad shape M=%d N=%d K=%d (K has to be a multiple of 64)", what, M, N, K);
+  NPAMD_REQUIRE(ldx >= K && ldw >= K && ldy >= N && ldx % 8 == 0 && ldw % 8 == 0, "%s: bad row stride", what);
+  if (M == 0 || N == 0) return NPAMD_OK;
+  NPAMD_REQUIRE(x && w && y && (((uintptr_t)x | (uintptr_t)w) & 15) == 0, "%s: null or unaligned pointer", what);
+  NPAMD_REQUIRE(ldx < (1 << 22) && ldw < (1 << 22), "%s: row stride too large", what);
+  const DenseShape s{x, w, bias, y, ldx, ldw, ldy, M, N, K / 64, 0, 0, 0};
+  hipStream_t st = (hipStream_t)stream;
+  const int forced = tuning().dense_tile;
+  const int tile = forced > 0 && forced <= kDenseTiles ? forced - 1 : plan_dense_tile(M, N, K, nullptr);
+  return act_dtype == NPAMD_BF16 ? launch_dense<NPAMD_BF16>(s, tile, st) : launch_dense<NPAMD_F16>(s, tile, st);
+}
+
+// Where this kernel is the better one against the library's product: its estimate against what the library reaches
+// (5 us + 0.85 PFLOP/s; 1.3 once 256 x 256 tiles cover 180 compute units; this kernel's estimates are some 15 % high
+// there) -- or against 16 us, which is what issuing a library product costs the host, so that below it no eager call
+// gains from a faster kernel.  Measured, library / this kernel, us: 171 x 256 x 640
+// 14.6 / 4.8, 77 x 3003 x 2240 13.4 / 8.8, 100 x 14336 x 512 9.7 / 6.7, 384 x 4096 x 4096 23.0 / 20.3, 250 x 11008 x 2048
+// 21.5 / 17.3, 2500 x 3000 x 1024 26.2 / 20.3, 1024 x 4096 x 4096 37.2 / 34.5; but 384 x 14336 x 4096 55.5 / 58.1,
+// 700 x 6000 x 6016 56.8 / 64.8, 4096^3 93 / 124: products of more than 40 GFLOP go to the library.
+extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {
+  if (M < 1 || N < 1 || K < 64 || K % 64) return 0;
+  const int forced = tuning().dense_tile;
+  if (forced) return forced > 0;
+  const double gflop = 2e-9 * M * N * K;
+  float us = 0.f;
+  plan_dense_tile(M, N, K, &us);
+  const double big_tiles = ceil(M / 256.0) * ceil(N / 256.0), rate = big_tiles >= 180 ? 1.3 : 0.85;
+  return gflop <= 40.0 && us <= fmax(16.0, 1.15 * (5.0 + gflop / rate)) ? 1 : 0;
+}

@@ -21,6 +21,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/index_select.h>
 #include <ATen/ops/linear.h>
+#include <c10/core/GradMode.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -94,7 +95,8 @@ struct Template {
   double f;                         // eps of a norm, scale of an embedding
   at::ScalarType out;
   at::Tensor perm;                  // column permutation applied to x first, or undefined: int32 (16-bit x) or int64
-  at::Tensor bias;                  // bias of the dense product, or undefined
+  at::Tensor bias;                  // bias of the dense product, or undefined: float32 for the framework's own
+  bool own;                         // dense kinds: the framework's own product, not the library's
   std::vector<at::Tensor> keep;     // what the addresses point into
 };
 
@@ -187,6 +189,7 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
 
   if (t.kind == kVqDense || t.kind == kRvqDense || t.kind == kQDense) {
     const int code = dtype_code(t.out);
+    if (t.own && (ldx % 8 || ((uintptr_t)x.const_data_ptr() & 15) || (x_in.requires_grad() && c10::GradMode::is_enabled()))) return false;
     at::Tensor w = empty({t.n, t.k}, t.out, device);
     int rc;
     if (t.kind == kVqDense)
@@ -199,6 +202,14 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
       rc = npamd_q_dequant(ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), (int)t.n, (int)t.k, (int)a[6], (int)a[7],
                            w.data_ptr(), code, st);
     if (rc != NPAMD_OK) return false;
+    if (t.own) {
+      at::Tensor y = empty(sizes, t.out, device);
+      if (npamd_dense_gemm(x.const_data_ptr(), ldx, w.data_ptr(), t.k, t.bias.defined() ? t.bias.const_data_ptr<float>() : nullptr,
+                           y.data_ptr(), t.n, (int)m, (int)t.n, (int)t.k, code, st) != NPAMD_OK)
+        return false;
+      *out = std::move(y);
+      return true;
+    }
     *out = at::linear(x, w, t.bias.defined() ? std::optional<at::Tensor>(t.bias) : std::nullopt);
     return true;
   }
@@ -492,14 +503,15 @@ PyObject* plan_hold(PyObject* self, PyObject* o) {
   Py_RETURN_NONE;
 }
 
-// template(kind, n, k, k_in, args, f, out_dtype_code, perm or None, bias or None, keep) -> number
+// template(kind, n, k, k_in, args, f, out_dtype_code, perm or None, bias or None, own, keep) -> number
 PyObject* plan_template(PyObject* self, PyObject* args) {
   Plan* p = reinterpret_cast<Plan*>(self);
-  int kind, out_code;
+  int kind, out_code, own;
   long long n, k, k_in;
   double f;
   PyObject *ints, *perm, *bias, *keep;
-  if (!PyArg_ParseTuple(args, "iLLLO!diOOO!", &kind, &n, &k, &k_in, &PyTuple_Type, &ints, &f, &out_code, &perm, &bias, &PyTuple_Type, &keep))
+  if (!PyArg_ParseTuple(args, "iLLLO!diOOpO!", &kind, &n, &k, &k_in, &PyTuple_Type, &ints, &f, &out_code, &perm, &bias, &own, &PyTuple_Type,
+                        &keep))
     return nullptr;
   if (kind < 0 || kind >= kKinds || (int)PyTuple_GET_SIZE(ints) > kArgs[kind]) {
     PyErr_SetString(PyExc_ValueError, "template(): bad kind or argument count");
@@ -511,6 +523,7 @@ PyObject* plan_template(PyObject* self, PyObject* args) {
   t.k = k;
   t.k_in = k_in;
   t.f = f;
+  t.own = own != 0;
   t.out = scalar_type(out_code);
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(ints); ++i) {
     PyObject* v = PyTuple_GET_ITEM(ints, i);
@@ -561,7 +574,7 @@ PyMethodDef plan_methods[] = {
     {"guard_module", plan_guard_module, METH_O, "guard_module({attribute: expected})"},
     {"source", plan_source, METH_O, "source(tensor or None)"},
     {"hold", plan_hold, METH_O, "hold(object)"},
-    {"template", plan_template, METH_VARARGS, "template(kind, n, k, k_in, args, f, out, perm, bias, keep) -> number"},
+    {"template", plan_template, METH_VARARGS, "template(kind, n, k, k_in, args, f, out, perm, bias, own, keep) -> number"},
     {"route", plan_route, METH_VARARGS, "route(dtype, tokens, template, scratch_bytes)"},
     {"stale", plan_stale, METH_O, "stale(module): whether anything the plan was built from has changed"},
     {"wrapped", plan_wrapped, METH_NOARGS, "wrapped(): whether a wrapper function has been replaced"},

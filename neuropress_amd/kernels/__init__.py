@@ -847,6 +847,31 @@ def warn_kernel_fallback(kernel: str, fallback: str, exc: BaseException) -> None
 # ---------------------------------------------------------------------------
 
 
+def dense_preferred(m: int, n: int, k: int) -> bool:
+    """Whether :func:`dense_linear` is the better choice for this shape against ``F.linear``."""
+    return bool(_lib.load().npamd_dense_gemm_preferred(int(m), int(n), int(k)))
+
+
+def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``x @ w.T (+ bias)`` of a 2-D fp16 / bf16 *x* with a decoded weight of its dtype, K a multiple of 64
+    (``npamd_dense_gemm``): the product of the decode + GEMM band where :func:`dense_preferred` says so."""
+    what = "dense_linear"
+    _check_device(what, x, w, bias)
+    x = _x2d(x, what)
+    if x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype or w.dim() != 2 or w.shape[1] != x.shape[1]:
+        raise RuntimeError(f"{what}: x and w must be float16 or bfloat16 [M, K] and [N, K]")
+    if x.stride(0) % 8 or x.data_ptr() % 16:
+        x = x.contiguous()
+    m, k = x.shape
+    n = w.shape[0]
+    w = w.contiguous()
+    y = torch.empty((m, n), device=x.device, dtype=x.dtype)
+    b32 = _bias_f32(bias)
+    _lib.call("npamd_dense_gemm", x.data_ptr(), x.stride(0), w.data_ptr(), k, _ptr(b32), y.data_ptr(), n, m, n, k,
+              _DT[x.dtype], _stream(x))  # fmt: skip
+    return y
+
+
 def gather_columns(x: torch.Tensor, perm: torch.Tensor | None, width: int) -> torch.Tensor:
     """``x[:, perm]`` (``x`` with *perm* None) of a 2-D 16-bit *x*, rows padded with zeros to *width* columns, a
     multiple of 8 (``npamd_gather_columns``).  *perm*: int32 ``[K]``."""

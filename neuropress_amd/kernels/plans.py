@@ -50,13 +50,13 @@ def make(module, attributes, thresholds=None, names=(), holders=(), sources=()):
     return plan
 
 
-def template(plan, kind, n, k, args, dtype, *, f=0.0, k_in=None, perm=None, bias=None):
+def template(plan, kind, n, k, args, dtype, *, f=0.0, k_in=None, perm=None, bias=None, own=False):
     """Template number of one call shape.  *args*: its constant arguments, tensors standing for their addresses (the
     plan keeps them alive); *dtype*: of the output; *perm*: columns of x to gather first; *k_in*: columns of x where the
-    kernel contracts more (rows padded with zeros)."""
+    kernel contracts more (rows padded with zeros); *own*: the dense product is the package's own (*bias* in float32)."""
     ints = tuple(a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args)
     keep = tuple(a for a in args if isinstance(a, torch.Tensor))
-    return plan.template(kind, n, k, k if k_in is None else k_in, ints, f, DTYPE_CODES[dtype], perm, bias, keep)
+    return plan.template(kind, n, k, k if k_in is None else k_in, ints, f, DTYPE_CODES[dtype], perm, bias, own, keep)
 
 
 def tile_scratch(m: int, n: int, k: int) -> int:

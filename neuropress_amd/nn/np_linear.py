@@ -367,7 +367,15 @@ class NPLinear(nn.Module):
                 raise
             kernels.warn_kernel_fallback("q_linear", "torch dequant + matmul", exc)
             return self._forward_compile(x)
+        if self._own_product(m, x.dtype) and not (x.requires_grad and torch.is_grad_enabled()):
+            return kernels.dense_linear(x.reshape(-1, self.in_features), w, self._bias_f32()).reshape(*x.shape[:-1], self.out_features)
         return F.linear(x, w, self._bias_as(x.dtype))
+
+    def _own_product(self, m: int, dtype: torch.dtype) -> bool:
+        """Whether the dense product of a decode + GEMM call is the package's own kernel."""
+        from .. import kernels
+
+        return dtype in (torch.float16, torch.bfloat16) and kernels.dense_preferred(m, self.out_features, self.in_features)
 
     def _band(self, x: torch.Tensor, m: int) -> str:
         """Which kernel serves a call of *m* tokens: ``fused`` (GEMV), ``tile`` (fused GEMM) or ``dense`` (decode + GEMM)."""
@@ -403,12 +411,14 @@ class NPLinear(nn.Module):
             if plan is None:
                 return None
         code = plans.DTYPE_CODES[x.dtype]
+        if band == "dense" and self._own_product(m, x.dtype):
+            band = "product"
         number = plan.names.get((band, x.dtype))
         if number is None:
-            kind = {"fused": plans.Q_GEMV, "tile": plans.Q_TILE, "dense": plans.Q_DENSE}[band]
+            kind = {"fused": plans.Q_GEMV, "tile": plans.Q_TILE}.get(band, plans.Q_DENSE)
             args = (self.u8_blob, self.scale, self.zero_point, self._bias_f32(), 0, 0, self.nbits, self.group_size, code)
-            number = plan.names[band, x.dtype] = plans.template(
-                plan, kind, n, k, args, x.dtype, bias=self._bias_as(x.dtype) if band == "dense" else None)  # fmt: skip
+            bias = self._bias_as(x.dtype) if band == "dense" else self._bias_f32() if band == "product" else None
+            number = plan.names[band, x.dtype] = plans.template(plan, kind, n, k, args, x.dtype, bias=bias, own=band == "product")
         plan.route(code, m, number, plans.tile_scratch(m, n, k) if band == "tile" else 0)
         self._plan = plan
         return None if plan.wrapped() else plan.run(x)

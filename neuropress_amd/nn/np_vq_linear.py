@@ -797,7 +797,7 @@ class NPVQLinear(nn.Module):
         from ..kernels import plans
 
         tile = band == "tile" or (band == "fused" and m > _GEMV_KERNEL_MAX_TOKENS)
-        kind = "tile" if tile else band
+        kind = "tile" if tile else "product" if band == "dense" and self._own_product(m, dtype) else band
         number = plan.names.get((kind, dtype))
         if number is None:
             number = plan.names[kind, dtype] = self._template(plan, dtype, kind)
@@ -829,17 +829,22 @@ class NPVQLinear(nn.Module):
             cr = self._res_centroids()
             args = (packed, packed.numel(), self.bits, res, res.numel(), self._res_bits(), proxy.centroids, proxy.num_centroids,
                     cr, cr.shape[0], self.row_scale, self.row_bias, vl)  # fmt: skip
-            if kind == "dense":
-                return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=self._bias_as(dtype))
+            if kind in ("dense", "product"):
+                own = kind == "product"
+                bias = self._bias_f32() if own else self._bias_as(dtype)
+                return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=bias, own=own)
             kind_code = plans.RVQ_TILE if kind == "tile" else plans.RVQ_GEMV
             return plans.template(plan, kind_code, n, k, (*args, self._bias_f32(), code), dtype, perm=perm)
         stream, bits = self._kernel_stream()
         stream = stream.reshape(-1)
-        if kind == "dense":
-            if self._kernel_k() != k:  # the dense product takes any K: no padding
+        if kind in ("dense", "product"):
+            own = kind == "product"
+            bias = self._bias_f32() if own else self._bias_as(dtype)
+            width = self._kernel_k() if own else k  # the library's product takes any K: no padding
+            if width == k and self._kernel_k() != k:
                 stream, bits = packed, self.bits
-            args = (stream, stream.numel(), bits, proxy.centroids, proxy.num_centroids, vl, self.n_vectors)
-            return plans.template(plan, plans.VQ_DENSE, n, k, args, dtype, perm=perm, bias=self._bias_as(dtype))
+            args = (stream, stream.numel(), bits, proxy.centroids, proxy.num_centroids, vl, n * (width // vl))
+            return plans.template(plan, plans.VQ_DENSE, n, width, args, dtype, k_in=k, perm=perm, bias=bias, own=own)
         args = (stream, stream.numel(), bits, proxy.centroids_as(dtype), code, proxy.num_centroids, vl, self._bias_f32(), code)
         if kind == "gemv_perm":
             return plans.template(plan, plans.VQ_GEMV_PERM, n, k, (*args, self._perm_i32(stream.device)), dtype)
@@ -1154,21 +1159,36 @@ class NPVQLinear(nn.Module):
         from .. import kernels
 
         try:
+            own = self._own_product(x.numel() // self.in_features, x.dtype) and not (x.requires_grad and torch.is_grad_enabled())
             if self.is_residual:
                 w = kernels.rvq_dequant(
                     self.packed_indices, self.bits, self._res_stream(), self._res_bits(),
                     self.proxy.centroids, self._res_centroids(), self.row_scale, self.row_bias,
                     self.out_features, self.in_features, x.dtype,
                 )  # fmt: skip
+            elif own and self._kernel_k() != self.in_features:
+                stream, bits = self._kernel_stream()
+                w = kernels.vq_dequant(stream, self.proxy.centroids, bits, self.out_features, self._kernel_k(), x.dtype)
             else:
                 w = kernels.vq_dequant(
                     self.packed_indices, self.proxy.centroids, self.bits,
                     self.out_features, self.in_features, x.dtype,
                 )  # fmt: skip
+            if own:
+                x2d = x.reshape(-1, self.in_features)
+                if w.shape[1] != self.in_features:
+                    x2d = kernels.gather_columns(x2d, None, w.shape[1])
+                return kernels.dense_linear(x2d, w, self._bias_f32()).reshape(*x.shape[:-1], self.out_features)
         except RuntimeError as exc:
             self._fallback("vq_dequant", "the gather path", exc)
             return self._forward_compile(x)
         return F.linear(x, w, self._bias_as(x.dtype))
+
+    def _own_product(self, m: int, dtype: torch.dtype) -> bool:
+        """Whether the dense product of a decode + GEMM call is the package's own kernel."""
+        from .. import kernels
+
+        return dtype in (torch.float16, torch.bfloat16) and kernels.dense_preferred(m, self.out_features, self._kernel_k())
 
     def _forward_tile_gemm(self, x: torch.Tensor) -> torch.Tensor:
         """Band (b): MFMA GEMM decoding weight tiles in-kernel.

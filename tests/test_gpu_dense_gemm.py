@@ -1,0 +1,55 @@
+"""The dense product of the decode + GEMM band: every tile at shapes around its edges, ragged rows and columns, one to
+many 64-k steps (fewer than a ring is deep, and counts its groups of waves do not divide)."""
+
+import pytest
+import torch
+
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def dense_tile(monkeypatch):
+    from neuropress_amd import _lib
+
+    def force(tile):
+        monkeypatch.setenv("NPAMD_DENSE_TILE", str(tile))
+        _lib.load().npamd_diag_reload_tuning()
+
+    yield force
+    monkeypatch.delenv("NPAMD_DENSE_TILE", raising=False)
+    _lib.load().npamd_diag_reload_tuning()
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+def test_dense_gemm_tiles(gpu, dense_tile, tile, act):
+    from neuropress_amd import kernels
+
+    dense_tile(tile)
+    for m, n, k in ((1, 1, 64), (31, 63, 128), (33, 65, 192), (64, 128, 256), (65, 129, 320), (127, 200, 448), (129, 257, 704),
+                    (256, 130, 576), (300, 500, 1088), (520, 40, 64)):  # fmt: skip
+        g = cases.gen(m + n + k)
+        x = torch.randn(m, k, generator=g).to(act)
+        w = (torch.randn(n, k, generator=g) * 0.05).to(act)
+        bias = torch.randn(n, generator=g)
+        y = kernels.dense_linear(x.to(gpu), w.to(gpu), bias.to(gpu)).float().cpu()
+        ref = x.double() @ w.double().T + bias.double()
+        tol = 2.0 ** (-10 if act == torch.float16 else -7)  # the rounding of the output, and f32 sums
+        assert bool(((y - ref).abs() <= tol * ref.abs() + 1e-4).all()), (tile, m, n, k, float((y - ref).abs().max()))
+    wide = torch.zeros(70, 200, dtype=act)  # rows of x at a stride; the same bits as dense rows
+    wide[:, :192] = torch.randn(70, 192, generator=cases.gen(1)).to(act)
+    w = (torch.randn(90, 192, generator=cases.gen(2)) * 0.05).to(act).to(gpu)
+    xs = wide.to(gpu)[:, :192]
+    assert torch.equal(kernels.dense_linear(xs, w), kernels.dense_linear(xs.contiguous(), w))
+
+
+def test_dense_gemm_refuses_what_it_does_not_take(gpu):
+    from neuropress_amd import kernels
+
+    x, w = torch.zeros(4, 96, dtype=torch.half, device=gpu), torch.zeros(8, 96, dtype=torch.half, device=gpu)
+    with pytest.raises(RuntimeError, match="multiple of 64"):
+        kernels.dense_linear(x, w)
+    assert not kernels.dense_preferred(4, 8, 96) and not kernels.dense_preferred(4096, 14336, 4096)
+    assert kernels.dense_preferred(171, 256, 640)
