@@ -777,21 +777,26 @@ class NPVQLinear(nn.Module):
         ):  # fmt: skip
             return None
         if plan is None:
-            try:
-                plan = plans.make(
-                    self, _PLAN_ATTRIBUTES, globals(), _PLAN_THRESHOLDS,
-                    holders=[p for p in (self.proxy, self.residual_proxy) if p is not None],
-                    sources=(self.packed_indices, self.proxy.centroids, self.bias, self.column_perm, self.packed_residual,
-                             self.row_scale, self.row_bias, None if self.residual_proxy is None else self.residual_proxy.centroids),
-                )  # fmt: skip
-            except RuntimeError as exc:
-                self._fallback("call_plan", "the Python call path", exc)
-                return None
+            plan = self._new_plan()
             if plan is None:
                 return None
         self._add_route(plan, x.dtype, m, band)
         self._plan = plan
         return None if plan.wrapped() else plan.run(x)
+
+    def _new_plan(self):
+        from ..kernels import plans
+
+        try:
+            return plans.make(
+                self, _PLAN_ATTRIBUTES, globals(), _PLAN_THRESHOLDS,
+                holders=[p for p in (self.proxy, self.residual_proxy) if p is not None],
+                sources=(self.packed_indices, self.proxy.centroids, self.bias, self.column_perm, self.packed_residual,
+                         self.row_scale, self.row_bias, None if self.residual_proxy is None else self.residual_proxy.centroids),
+            )  # fmt: skip
+        except RuntimeError as exc:
+            self._fallback("call_plan", "the Python call path", exc)
+            return None
 
     def _add_route(self, plan, dtype: torch.dtype, m: int, band: str) -> None:
         from ..kernels import plans
@@ -895,6 +900,8 @@ class NPVQLinear(nn.Module):
         if self.is_residual:
             self._res_stream()
             self._res_centroids()
+        if self.backend in _FUSED_BACKENDS and (self._plan is None or self._plan.stale(self)):
+            self._plan = self._new_plan()  # still without routes: every call adds its own
 
     def _build_sliced(self):
         """(slice lists, most tokens for which they beat the fused GEMV on this layer)."""
