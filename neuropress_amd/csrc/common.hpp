@@ -68,6 +68,28 @@ inline hipError_t enable_dynamic_lds(LdsLatch& latch, const void* kernel, int by
     if (!(cond)) return ::npamd::fail(NPAMD_ERR_INVALID, __VA_ARGS__); \
   } while (0)
 
+// Work item of block `block` when each of the GPU's eight dies is to take a contiguous eighth of the items, `per_die`
+// of them (workgroups go to the dies in turn; the grid is per_die * 8 blocks, see DieGrid); per_die 0: items in turn.  The one-pass decodes hand the
+// rows of the weight to the dies as the dense product that follows reads them: a decoded line is then written and
+// read through one L2.  Lines that other dies' L2s still hold from the product before cost a write dearly --
+// decode + product of 33 tokens on a 4096 x 4096 int4 layer, the decoded weight in the same memory every
+// time as an allocator returns it: 31.7 us with the rows dealt to the dies in turn, 20.8 like this; 8192 x 2048 with a
+// 256-row codebook and the library's product, 64 tokens: 33.2 / 19.7.
+__device__ __forceinline__ int64_t die_block(unsigned block, unsigned per_die) {
+  return per_die ? (int64_t)(block & 7u) * per_die + (block >> 3) : (int64_t)block;
+}
+// A decode that writes more than twice what the eight L2s hold (4 MiB each) finds none of its lines in them the next
+// time, and a die that works through one far corner of the weight only loads the memory channels unevenly: rows in turn
+// (14336 x 4096, decode + library product of 4096 tokens: 368 us against 379).
+struct DieGrid {
+  unsigned blocks, per_die;
+  DieGrid(int64_t items, int64_t bytes_written) {
+    const bool by_die = bytes_written <= (int64_t)64 << 20;
+    per_die = by_die ? (unsigned)((items + 7) / 8) : 0;
+    blocks = by_die ? per_die * 8 : (unsigned)items;
+  }
+};
+
 // ---------------------------------------------------------------------------
 // 16-bit float conversions
 // ---------------------------------------------------------------------------

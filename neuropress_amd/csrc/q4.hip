@@ -38,9 +38,9 @@ template <int OUT, bool ASYM>
 __global__ void __launch_bounds__(256)
 q4_dequant_kernel(const uint32_t* __restrict__ w_pack, const uint16_t* __restrict__ scale,
                   const uint16_t* __restrict__ zero_point, int64_t n_words, int words_per_row,
-                  int groups_per_row, int words_per_group, void* __restrict__ out) {
+                  int groups_per_row, int words_per_group, unsigned per_die, void* __restrict__ out) {
 #pragma clang fp contract(off)
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = die_block(blockIdx.x, per_die) * 256 + threadIdx.x;
   if (i >= n_words) return;
   const int64_t n = i / words_per_row;
   const int wr = (int)(i - n * words_per_row);
@@ -77,9 +77,9 @@ template <int NBITS, int OUT>
 __global__ void __launch_bounds__(256)
 qn_dequant_kernel(const uint8_t* __restrict__ w_pack, const uint16_t* __restrict__ scale,
                   const uint16_t* __restrict__ zero_point, int64_t n_octets, int octets_per_row,
-                  int groups_per_row, int octets_per_group, void* __restrict__ out) {
+                  int groups_per_row, int octets_per_group, unsigned per_die, void* __restrict__ out) {
 #pragma clang fp contract(off)
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = die_block(blockIdx.x, per_die) * 256 + threadIdx.x;
   if (i >= n_octets) return;
   const int64_t n = i / octets_per_row;
   const int o = (int)(i - n * octets_per_row);
@@ -725,17 +725,17 @@ extern "C" int npamd_q_dequant(const uint8_t* w_pack, const void* scale_f16, con
                     ptr_aligned(w_pack, 4) && ptr_aligned(out, 16);
   if (fast) {
     const int64_t n_words = total / 8;
-    const unsigned blocks = (unsigned)((n_words + 255) / 256);
+    const DieGrid grid((n_words + 255) / 256, total * (out_dtype == NPAMD_F32 ? 4 : 2));
 #define NPAMD_Q4_LAUNCH(OUT)                                                                              \
   do {                                                                                                    \
     if (zero_point_f16)                                                                                   \
-      q4_dequant_kernel<OUT, true><<<blocks, 256, 0, st>>>(                                               \
+      q4_dequant_kernel<OUT, true><<<grid.blocks, 256, 0, st>>>(                                               \
           (const uint32_t*)w_pack, (const uint16_t*)scale_f16, (const uint16_t*)zero_point_f16, n_words,  \
-          K / 8, K / group_size, group_size / 8, out);                                                    \
+          K / 8, K / group_size, group_size / 8, grid.per_die, out);                                                    \
     else                                                                                                  \
-      q4_dequant_kernel<OUT, false><<<blocks, 256, 0, st>>>(                                              \
+      q4_dequant_kernel<OUT, false><<<grid.blocks, 256, 0, st>>>(                                              \
           (const uint32_t*)w_pack, (const uint16_t*)scale_f16, nullptr, n_words, K / 8, K / group_size,   \
-          group_size / 8, out);                                                                           \
+          group_size / 8, grid.per_die, out);                                                                           \
   } while (0)
     if (out_dtype == NPAMD_F16) NPAMD_Q4_LAUNCH(NPAMD_F16);
     else if (out_dtype == NPAMD_BF16) NPAMD_Q4_LAUNCH(NPAMD_BF16);
@@ -744,11 +744,11 @@ extern "C" int npamd_q_dequant(const uint8_t* w_pack, const void* scale_f16, con
   } else if ((nbits == 8 || nbits == 2 || nbits == 1) && K % 8 == 0 && group_size % 8 == 0 &&
              ptr_aligned(w_pack, nbits) && ptr_aligned(out, 16)) {
     const int64_t n_octets = total / 8;
-    const unsigned blocks = (unsigned)((n_octets + 255) / 256);
+    const DieGrid grid((n_octets + 255) / 256, total * (out_dtype == NPAMD_F32 ? 4 : 2));
 #define NPAMD_QN_LAUNCH(NB, OUT)                                                                       \
-  qn_dequant_kernel<NB, OUT><<<blocks, 256, 0, st>>>(w_pack, (const uint16_t*)scale_f16,               \
+  qn_dequant_kernel<NB, OUT><<<grid.blocks, 256, 0, st>>>(w_pack, (const uint16_t*)scale_f16,               \
                                                      (const uint16_t*)zero_point_f16, n_octets, K / 8, \
-                                                     K / group_size, group_size / 8, out)
+                                                     K / group_size, group_size / 8, grid.per_die, out)
 #define NPAMD_QN_OUT(NB)                                         \
   do {                                                           \
     if (out_dtype == NPAMD_F16) NPAMD_QN_LAUNCH(NB, NPAMD_F16);  \

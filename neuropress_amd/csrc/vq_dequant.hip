@@ -43,8 +43,8 @@ template <int BITS, int OUT>
 __global__ void __launch_bounds__(256)
 vq_dequant_vl8_kernel(const uint8_t* __restrict__ packed, int64_t n_bytes, int bits,
                       const u32x4* __restrict__ codebook, uint32_t nc, void* __restrict__ out,
-                      int64_t n_vectors) {
-  const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
+                      int64_t n_vectors, unsigned per_die) {
+  const int64_t v = die_block(blockIdx.x, per_die) * 256 + threadIdx.x;
   if (v >= n_vectors) return;
   // An index past the codebook is clamped to the last row so a corrupt stream
   // cannot read outside the table.
@@ -71,8 +71,8 @@ template <int BITS, int OUT>
 __global__ void __launch_bounds__(256)
 vq_dequant_vl4_kernel(const uint8_t* __restrict__ packed, int64_t n_bytes, int bits,
                       const u32x2* __restrict__ codebook, uint32_t nc, void* __restrict__ out,
-                      int64_t n_vectors) {
-  const int64_t v0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 2;
+                      int64_t n_vectors, unsigned per_die) {
+  const int64_t v0 = (die_block(blockIdx.x, per_die) * 256 + threadIdx.x) * 2;
   if (v0 >= n_vectors) return;
   const bool both = v0 + 1 < n_vectors;
   const u32x2 c0 = codebook[min(vec_index<BITS>(packed, n_bytes, v0, bits), nc - 1u)];
@@ -89,7 +89,7 @@ template <int BITS, int OUT, int VL>
 __global__ void __launch_bounds__(1024)
 vq_dequant_lds_kernel(const uint8_t* __restrict__ packed, int64_t n_bytes, int bits,
                       const u32x4* __restrict__ codebook, uint32_t nc, void* __restrict__ out,
-                      int64_t n_vectors, int64_t vectors_per_block) {
+                      int64_t n_vectors, int64_t vectors_per_block, unsigned per_die) {
   extern __shared__ __attribute__((aligned(16))) u32x4 cb_lds[];
   const uint32_t vec16 = VL == 8 ? nc : (nc + 1) / 2;  // the allocation behind an odd VL = 4 table is not read past:
   for (uint32_t i = threadIdx.x; i < vec16; i += 1024) {  // its last half-filled unit is fetched as 8 bytes
@@ -101,7 +101,7 @@ vq_dequant_lds_kernel(const uint8_t* __restrict__ packed, int64_t n_bytes, int b
     }
   }
   __syncthreads();
-  const int64_t begin = (int64_t)blockIdx.x * vectors_per_block;
+  const int64_t begin = die_block(blockIdx.x, per_die) * vectors_per_block;
   const int64_t end = min(begin + vectors_per_block, n_vectors);
   if constexpr (VL == 8) {
     for (int64_t v = begin + threadIdx.x; v < end; v += 1024) {
@@ -180,10 +180,10 @@ rvq_dequant_vl8_kernel(const uint8_t* __restrict__ pm, int64_t nbm, int bits_m,
                        const uint8_t* __restrict__ pr, int64_t nbr, int bits_r,
                        const u32x4* __restrict__ cbm, uint32_t ncm, const u32x4* __restrict__ cbr, uint32_t ncr,
                        const uint16_t* __restrict__ row_scale, const uint16_t* __restrict__ row_bias,
-                       int groups, void* __restrict__ out) {
-  const int n = blockIdx.x;
+                       int rows, int groups, unsigned per_die, void* __restrict__ out) {
+  const int n = (int)die_block(blockIdx.x, per_die);
   const int g = blockIdx.y * 256 + threadIdx.x;
-  if (g >= groups) return;
+  if (n >= rows || g >= groups) return;
   const int64_t v = (int64_t)n * groups + g;
   const uint32_t im = min(vec_index<BITS_M>(pm, nbm, v, bits_m), ncm - 1u);
   const uint32_t ir = min(vec_index<BITS_R>(pr, nbr, v, bits_r), ncr - 1u);
@@ -207,6 +207,8 @@ template <int OUT>
 static int launch_vq_dequant(const uint8_t* packed, int64_t n_bytes, int bits, const void* cb,
                              uint32_t nc, int vl, int64_t n_vectors, void* out, hipStream_t st) {
   const unsigned blocks = (unsigned)((n_vectors + 255) / 256);
+  const int64_t bytes = n_vectors * vl * (OUT == NPAMD_F32 ? 4 : 2);
+  const DieGrid grid(blocks, bytes);
   const bool cb_aligned = (reinterpret_cast<uintptr_t>(cb) % 16) == 0;
   const bool out_aligned = (reinterpret_cast<uintptr_t>(out) % 16) == 0;
   // Tables of 16 to 64 KiB on layers large enough to pay for one copy per block.
@@ -216,10 +218,10 @@ static int launch_vq_dequant(const uint8_t* packed, int64_t n_bytes, int bits, c
     const u32x4* c = reinterpret_cast<const u32x4*>(cb);
     const int lds = (int)((table_bytes + 15) / 16 * 16);
     const int64_t per_block = ((n_vectors + 511) / 512 + 1023) / 1024 * 1024;
-    const unsigned grid = (unsigned)((n_vectors + per_block - 1) / per_block);
+    const DieGrid grid((n_vectors + per_block - 1) / per_block, bytes);
     const bool b16 = bits == 16 && (reinterpret_cast<uintptr_t>(packed) % 2) == 0;
 #define NPAMD_VQ_LDS(B, V) \
-  vq_dequant_lds_kernel<B, OUT, V><<<grid, 1024, lds, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, per_block)
+  vq_dequant_lds_kernel<B, OUT, V><<<grid.blocks, 1024, lds, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, per_block, grid.per_die)
     if (vl == 8) {
       if (b16) NPAMD_VQ_LDS(16, 8);
       else NPAMD_VQ_LDS(0, 8);
@@ -233,20 +235,20 @@ static int launch_vq_dequant(const uint8_t* packed, int64_t n_bytes, int bits, c
   if (vl == 8 && cb_aligned && out_aligned) {
     const u32x4* c = reinterpret_cast<const u32x4*>(cb);
     if (bits == 16 && (reinterpret_cast<uintptr_t>(packed) % 2) == 0)
-      vq_dequant_vl8_kernel<16, OUT><<<blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors);
+      vq_dequant_vl8_kernel<16, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
     else if (bits == 8)
-      vq_dequant_vl8_kernel<8, OUT><<<blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors);
+      vq_dequant_vl8_kernel<8, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
     else
-      vq_dequant_vl8_kernel<0, OUT><<<blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors);
+      vq_dequant_vl8_kernel<0, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
   } else if (vl == 4 && (reinterpret_cast<uintptr_t>(cb) % 8) == 0 && out_aligned) {
     const u32x2* c = reinterpret_cast<const u32x2*>(cb);
-    const unsigned blocks = (unsigned)(((n_vectors + 1) / 2 + 255) / 256);  // two vectors per thread
+    const DieGrid grid(((n_vectors + 1) / 2 + 255) / 256, bytes);  // two vectors per thread
     if (bits == 16 && (reinterpret_cast<uintptr_t>(packed) % 2) == 0)
-      vq_dequant_vl4_kernel<16, OUT><<<blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors);
+      vq_dequant_vl4_kernel<16, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
     else if (bits == 8)
-      vq_dequant_vl4_kernel<8, OUT><<<blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors);
+      vq_dequant_vl4_kernel<8, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
     else
-      vq_dequant_vl4_kernel<0, OUT><<<blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors);
+      vq_dequant_vl4_kernel<0, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
   } else {
     vq_dequant_generic_kernel<OUT><<<blocks, 256, 0, st>>>(
         packed, n_bytes, bits, reinterpret_cast<const uint16_t*>(cb), nc, out, n_vectors, vl);
@@ -350,14 +352,15 @@ extern "C" int npamd_rvq_dequant(const uint8_t* packed_main, int64_t n_bytes_mai
   const bool aligned16 = ((reinterpret_cast<uintptr_t>(cb_main_f16) | reinterpret_cast<uintptr_t>(cb_res_f16) |
                            reinterpret_cast<uintptr_t>(out)) % 16) == 0;
   if (vl == 8 && aligned16 && (groups + 255) / 256 <= 65535) {
-    const dim3 grid((unsigned)N, (unsigned)((groups + 255) / 256));
+    const DieGrid rows(N, n_vectors * 8 * (out_dtype == NPAMD_F32 ? 4 : 2));
+    const dim3 grid(rows.blocks, (unsigned)((groups + 255) / 256));
     const bool m16 = bits_main == 16 && (reinterpret_cast<uintptr_t>(packed_main) % 2) == 0;
     const bool r8 = bits_res == 8;
 #define NPAMD_RVQ8_LAUNCH(BM, BR, OUT)                                                               \
   rvq_dequant_vl8_kernel<BM, BR, OUT><<<grid, 256, 0, st>>>(                                         \
       packed_main, n_bytes_main, bits_main, packed_res, n_bytes_res, bits_res, (const u32x4*)cb_main_f16, \
       (uint32_t)nc_main, (const u32x4*)cb_res_f16, (uint32_t)nc_res, (const uint16_t*)row_scale_f16,  \
-      (const uint16_t*)row_bias_f16, (int)groups, out)
+      (const uint16_t*)row_bias_f16, N, (int)groups, rows.per_die, out)
 #define NPAMD_RVQ8_BITS(OUT)                                \
   do {                                                      \
     if (m16 && r8) NPAMD_RVQ8_LAUNCH(16, 8, OUT);           \

@@ -49,10 +49,10 @@ _Q_TILE_WIDE_MIN_FEATURES: int = 8192
 # As for the VQ path: the fused GEMM splits the reduction when the layer has few
 # output features; a layer that still leaves most compute units idle takes decode +
 # GEMM.  Measured (fused vs decode + GEMM): 4096 x 14336 41-57 vs 93-115 us from 128 to
-# 256 tokens; 4096 x 4096 24-31 vs 37-45 us from 128 to 256, 39-41 vs 39-40 us at
-# 320-384; 1024 x 4096 (not enough workgroups even when split) 17-19 vs 16-20 us.
+# 256 tokens; 4096 x 4096 19 vs 22 us at 64, 23 vs 23 at 128, 27 vs 25 at 192, 30 vs 27 at 256;
+# 8192 x 2048 24 vs 21 at 128; 1024 x 4096 (not enough workgroups even when split) 17 vs 14 us at 64.
 _Q_TILE_MIN_GRID_FRACTION: float = 0.7
-_Q_TILE_SPLIT_MAX_TOKENS: int = 256
+_Q_TILE_SPLIT_MAX_TOKENS: int = 144
 _Q_TILE_SPLIT_LONG_K: int = 8192
 _Q_FUSED_MAX_TOKENS: int = 16
 # 17..32 tokens: the GEMV reuses every dequantized operand for two 16-token tiles, and each
@@ -322,7 +322,7 @@ class NPLinear(nn.Module):
             self._derived["cus"] = cus
         return tile_band_ok(
             m, self.out_features, self.in_features, cus,
-            _Q_TILE_MIN_GRID_FRACTION, _Q_TILE_SPLIT_MAX_TOKENS, _Q_TILE_SPLIT_LONG_K,
+            _Q_TILE_MIN_GRID_FRACTION, _Q_TILE_SPLIT_MAX_TOKENS, _Q_TILE_SPLIT_LONG_K, _Q_FUSED_WIDE_MAX_TOKENS,
         )  # fmt: skip
 
     def _gemv_max_tokens(self, m: int) -> int:

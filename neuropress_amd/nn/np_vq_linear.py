@@ -117,15 +117,18 @@ _TILE_MAX_TOKENS: int = _env_int(
 
 # Layers whose codebook LDS does not hold (more than 4096 rows of eight) run the 128-column tile GEMM,
 # which splits the reduction by itself and stays ahead of decode + GEMM up to a token count that goes
-# with the layer's weights (us at 128 / 256 / 384 tokens, tile against decode + GEMM): 14336 x 4096
-# 47 / 59 / 73 against 81 / 96 / 101, 4096 x 14336 53 / 67 / 82 against 114 / 103 / 117; 6144 x 4096
-# 32 / 41 / 56 against 47 / 61 / 55, 4096 x 4096 28 / 34 / 42 against 40 / 38 / 41, 8192 x 2048 28 / 34 / 46
-# against 34 / 40 / 38; 1024 x 4096 18 / 24 / 29 against 20 / 21 / 22, 2048 x 2048 16 / 23 / 28 against 17 / 20 / 20.
+# with the layer's weights (us at 64 / 128 / 256 / 384 tokens, tile against decode + GEMM): 14336 x 4096
+# 42 / 46 / 59 / 70 against 58 / 65 / 75 / 87, 4096 x 14336 44 / 50 / 63 / 80 against 68 / 70 / 85 / 103;
+# 4096 x 4096 23 / 28 / 34 / 42 against 26 / 26 / 30 / 35, 8192 x 2048 22 / 29 / 35 / 46 against 23 / 25 / 30 / 33,
+# 2048 x 8192 27 / 28 / 35 / 44 against 32 / 32 / 33 / 38; 3008 x 2240 15 / 19 / 26 / 31 against 15 / 16 / 18 / 21;
+# 1024 x 4096 15 / 19 / 24 / 28 against 15 / 16 / 17 / 18, 2048 x 2048 13 / 15 / 22 / 28 against 12 / 12 / 13 / 15.
 _TILE_WIDE_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_TILE_WIDE_MAX_TOKENS",), 384)
-_TILE_WIDE_MIN_WEIGHTS: int = 1 << 25  # below: 256 tokens
-_TILE_WIDE_SMALL_WEIGHTS: int = 1 << 24  # below: 128 tokens
-_TILE_WIDE_MID_MAX_TOKENS: int = 256
-_TILE_WIDE_SMALL_MAX_TOKENS: int = 128
+_TILE_WIDE_MIN_WEIGHTS: int = 1 << 25  # below: 80 tokens, on long reductions 160
+_TILE_WIDE_SMALL_WEIGHTS: int = 1 << 24  # below: 64 tokens
+_TILE_WIDE_TINY_WEIGHTS: int = 5_000_000  # below: 32 tokens, where the GEMV ends
+_TILE_WIDE_MID_MAX_TOKENS: int = 80
+_TILE_WIDE_LONG_MAX_TOKENS: int = 160
+_TILE_WIDE_SMALL_MAX_TOKENS: int = 64
 
 # The tile GEMM gives each workgroup 64 output columns (and up to 384 rows).  When
 # that grid covers less than this fraction of the compute units the kernel splits
@@ -138,6 +141,8 @@ _TILE_MIN_GRID_FRACTION: float = 0.7
 # tokens and 82 vs 101 us at 256; 4096 x 4096 layer 25-31 vs 30-39 us up to 128
 # tokens, 39 vs 36 us at 256.
 _TILE_SPLIT_MAX_TOKENS: int = 128
+# Small layers (fewer than 8 M weights) decode in 4-8 us and leave the band earlier; residual ones at 32 tokens.
+_TILE_SMALL_LAYER_MAX_TOKENS: int = 64
 _TILE_SPLIT_LONG_K: int = 8192  # from this many input features on, _TILE_MAX_TOKENS applies
 # Layers of at least this many indices time their slice-list GEMV against the fused one when the
 # lists are built (NPVQLinear._sliced_token_limit).
@@ -166,7 +171,8 @@ _PLAN_ATTRIBUTES = ("backend", "proxy", "residual_proxy", "out_features", "in_fe
                     "bias", "column_perm", "packed_residual", "row_scale", "row_bias")  # fmt: skip
 _PLAN_THRESHOLDS = ("_FUSED_MAX_TOKENS", "_FUSED_WIDE_MAX_TOKENS", "_FUSED_WIDE_MAX_ACTIVATIONS", "_SLICED_MAX_TOKENS",
                     "_SLICED_MIN_CENTROIDS", "_SLICED_MIN_INDICES", "_LUT_MAX_TOKENS", "_TILE_MAX_TOKENS", "_TILE_WIDE_MAX_TOKENS",
-                    "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_SMALL_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS", "_TILE_WIDE_SMALL_MAX_TOKENS",
+                    "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_SMALL_WEIGHTS", "_TILE_WIDE_TINY_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS",
+                    "_TILE_WIDE_LONG_MAX_TOKENS", "_TILE_WIDE_SMALL_MAX_TOKENS", "_TILE_SMALL_LAYER_MAX_TOKENS",
                     "_TILE_MIN_GRID_FRACTION", "_TILE_SPLIT_MAX_TOKENS", "_TILE_SPLIT_LONG_K", "_tile_failed")  # fmt: skip
 
 # Latched once the tile GEMM fails with fallback allowed, so later calls go
@@ -1094,7 +1100,10 @@ class NPVQLinear(nn.Module):
             if weights >= _TILE_WIDE_MIN_WEIGHTS:
                 return max(_TILE_MAX_TOKENS, _TILE_WIDE_MAX_TOKENS)
             if weights >= _TILE_WIDE_SMALL_WEIGHTS:
-                return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_MID_MAX_TOKENS)
+                long = self.in_features >= _TILE_SPLIT_LONG_K
+                return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS if long else _TILE_WIDE_MID_MAX_TOKENS)
+            if weights < _TILE_WIDE_TINY_WEIGHTS and _TILE_MIN_GRID_FRACTION > 0:
+                return min(_TILE_WIDE_MAX_TOKENS, _GEMV_KERNEL_MAX_TOKENS)
             return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_SMALL_MAX_TOKENS)
         return _TILE_MAX_TOKENS
 
@@ -1115,6 +1124,7 @@ class NPVQLinear(nn.Module):
         return tile_band_ok(
             m, self.out_features, self._kernel_k(), cus,
             _TILE_MIN_GRID_FRACTION, _TILE_SPLIT_MAX_TOKENS, _TILE_SPLIT_LONG_K,
+            32 if self.is_residual else _TILE_SMALL_LAYER_MAX_TOKENS,
         )  # fmt: skip
 
     # -- torch-op paths ---------------------------------------------------

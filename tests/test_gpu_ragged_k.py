@@ -32,7 +32,8 @@ def test_gather_columns(gpu, k, width):
 def test_ragged_k_runs_the_fused_bands(gpu, n, k, nc, vl, perm, act, monkeypatch):
     from neuropress_amd import kernels
 
-    monkeypatch.setattr(vqmod, "_TILE_MIN_GRID_FRACTION", 0.0)
+    monkeypatch.setattr(vqmod, "_TILE_MIN_GRID_FRACTION", 0.0)  # small layers: force the tile band
+    monkeypatch.setattr(vqmod, "_TILE_WIDE_SMALL_MAX_TOKENS", 128)
     L = cases.vq_layer(n + k, n, k, nc, vl=vl, bias=True, act=act, std=0.05)
     cp = torch.randperm(k, generator=cases.gen(k)) if perm else None
     layer = NPVQLinear(VQProxy(L["cb"]).to(gpu), L["packed"], L["bits"], n, k, vl, "cuda_wmma", bias=L["bias"].float(),
