@@ -7,6 +7,32 @@ using namespace npamd;
 
 namespace {
 
+// Rows go to the dies in eighths while what a kernel writes may still be in the L2s when its reader runs (lookup + norm
+// of 2048 tokens x 4096: 20.1 us in turn, 16.7 in eighths; of 4096 tokens 27.6 either way, and the norm alone 11.8 / 13.1).
+constexpr int64_t kAuxDieBytes = (int64_t)24 << 20;
+
+// How the lookups split a token's row of `vectors` pieces of eight values: pieces per thread (vpt), blocks per row
+// (segments), and threads per row and block (lanes).  Short rows share a block of up to 256 threads.
+struct TokenGrid {
+  int vpt, segments;
+  unsigned lanes, tokens, threads;
+  TokenGrid(int vectors, int64_t n_ids) {
+    vpt = vectors > 256 && n_ids >= 64 ? 2 : 1;
+    segments = (vectors + 256 * vpt - 1) / (256 * vpt);
+    const unsigned need = (unsigned)((vectors + segments * vpt - 1) / (segments * vpt));
+    lanes = need <= 128 ? need : (need + 63) / 64 * 64;
+    tokens = segments == 1 && lanes <= 128 ? 256 / lanes : 1;
+    threads = tokens == 1 ? (lanes + 63) / 64 * 64 : 256;
+  }
+};
+// The block's token and column of a thread; false for the few threads behind the block's last whole token.
+__device__ __forceinline__ bool token_of_thread(unsigned lanes, unsigned tokens, unsigned per_die, int64_t* t, int* col) {
+  const unsigned sub = tokens == 1 ? 0u : threadIdx.x / lanes;
+  *t = die_block(blockIdx.x, per_die) * tokens + sub;
+  *col = (int)(threadIdx.x - sub * lanes);
+  return sub < tokens && *col < (int)lanes;
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <int DT>
@@ -28,16 +54,19 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 // RMSNorm: out[m, i] = round(x[m, i] * rsqrt(mean_i(x[m, i]^2) + eps) * w[i]),
 // all arithmetic in f32, one rounding at the store.
 //
-// One wave per row; the row stays in registers between the sum of squares and
-// the scaling (NV 16-byte vectors per lane), so x is read from memory once and
-// the only cross-lane traffic is the wave reduction.  Four rows per block.
+// The row stays in registers between the sum of squares and the scaling (NV 16-byte vectors per
+// lane), so x is read from memory once.  Many rows: one wave per row, four rows per block, bound by
+// HBM, an eighth of the rows to each die as the lookups in front of a norm deal them.  Few rows, bound by
+// the launch and one memory round trip: four waves per row (ROW_WAVES), which meet in LDS -- a quarter of
+// the loads and conversions per lane.
 // ---------------------------------------------------------------------------
-template <int DT, int NV>
+template <int DT, int NV, int ROW_WAVES>
 __global__ void __launch_bounds__(256)
 rms_norm_wave_kernel(const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ w,
-                     uint16_t* __restrict__ out, int64_t ldo, int M, int H, float eps) {
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+                     uint16_t* __restrict__ out, int64_t ldo, int M, int H, float eps, unsigned per_die) {
+  constexpr int kLanes = 64 * ROW_WAVES;
+  const int lane = threadIdx.x & (kLanes - 1);
+  const int row = (int)die_block(blockIdx.x, per_die) * (4 / ROW_WAVES) + threadIdx.x / kLanes;
   if (row >= M) return;
   const int n_vec = H >> 3;
   const uint16_t* xr = x + (int64_t)row * ldx;
@@ -45,13 +74,13 @@ rms_norm_wave_kernel(const uint16_t* __restrict__ x, int64_t ldx, const uint16_t
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int p = lane + 64 * i;
+    const int p = lane + kLanes * i;
     v[i] = p < n_vec ? *reinterpret_cast<const u32x4*>(xr + 8 * p) : u32x4{0, 0, 0, 0};
   }
   // the weight does not depend on the reduction: requested now, it arrives while the sum is formed
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int p = lane + 64 * i;
+    const int p = lane + kLanes * i;
     wv[i] = p < n_vec ? *reinterpret_cast<const u32x4*>(w + 8 * p) : u32x4{0, 0, 0, 0};
   }
 #pragma unroll
@@ -62,11 +91,19 @@ rms_norm_wave_kernel(const uint16_t* __restrict__ x, int64_t ldx, const uint16_t
     for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(f[e], f[e], ss);
   }
   ss = wave_reduce_sum(ss);
+  if constexpr (ROW_WAVES > 1) {
+    __shared__ float part[ROW_WAVES];
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < ROW_WAVES; ++i) ss += part[i];
+  }
   const float scale = 1.0f / __builtin_sqrtf(ss / (float)H + eps);
   uint16_t* orow = out + (int64_t)row * ldo;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int p = lane + 64 * i;
+    const int p = lane + kLanes * i;
     if (p >= n_vec) continue;
     float f[8], g[8];
     unpack8<DT>(v[i], f);
@@ -98,6 +135,7 @@ rms_norm_block_kernel(const void* __restrict__ x, int64_t ldx, const void* __res
     store_from_f32<DT>(out, row * ldo + i, load_as_f32<DT>(x, row * ldx + i) * scale * load_as_f32<DT>(w, i));
 }
 
+constexpr int kRmsFewRows = 1024;
 template <int DT>
 int launch_rms_norm(const void* x, int64_t ldx, const void* w, void* out, int64_t ldo, int M, int H, float eps,
                     hipStream_t st) {
@@ -105,16 +143,27 @@ int launch_rms_norm(const void* x, int64_t ldx, const void* w, void* out, int64_
                    aligned16(out) && H <= 8 * 64 * 16;
   if constexpr (DT != NPAMD_F32) {
     if (vec) {
-      const int nv = (H / 8 + 63) / 64;
-      const dim3 grid((M + 3) / 4);
       auto xs = (const uint16_t*)x;
       auto ws = (const uint16_t*)w;
       auto os = (uint16_t*)out;
-      if (nv <= 1) rms_norm_wave_kernel<DT, 1><<<grid, 256, 0, st>>>(xs, ldx, ws, os, ldo, M, H, eps);
-      else if (nv <= 2) rms_norm_wave_kernel<DT, 2><<<grid, 256, 0, st>>>(xs, ldx, ws, os, ldo, M, H, eps);
-      else if (nv <= 4) rms_norm_wave_kernel<DT, 4><<<grid, 256, 0, st>>>(xs, ldx, ws, os, ldo, M, H, eps);
-      else if (nv <= 8) rms_norm_wave_kernel<DT, 8><<<grid, 256, 0, st>>>(xs, ldx, ws, os, ldo, M, H, eps);
-      else rms_norm_wave_kernel<DT, 16><<<grid, 256, 0, st>>>(xs, ldx, ws, os, ldo, M, H, eps);
+#define NPAMD_RMS(NV, RW) \
+  rms_norm_wave_kernel<DT, NV, RW><<<grid.blocks, 256, 0, st>>>(xs, ldx, ws, os, ldo, M, H, eps, grid.per_die)
+      if (M <= kRmsFewRows && H > 512) {
+        const DieGrid grid(M, (int64_t)M * H * 2, kAuxDieBytes);
+        const int nv = (H / 8 + 255) / 256;
+        if (nv <= 1) NPAMD_RMS(1, 4);
+        else if (nv <= 2) NPAMD_RMS(2, 4);
+        else NPAMD_RMS(4, 4);
+      } else {
+        const DieGrid grid((M + 3) / 4, (int64_t)M * H * 2, kAuxDieBytes);
+        const int nv = (H / 8 + 63) / 64;
+        if (nv <= 1) NPAMD_RMS(1, 1);
+        else if (nv <= 2) NPAMD_RMS(2, 1);
+        else if (nv <= 4) NPAMD_RMS(4, 1);
+        else if (nv <= 8) NPAMD_RMS(8, 1);
+        else NPAMD_RMS(16, 1);
+      }
+#undef NPAMD_RMS
       return check_launch("npamd_rms_norm");
     }
   }
@@ -150,37 +199,54 @@ __device__ __forceinline__ void store_embedding8(void* out, int64_t at, const ui
   }
 }
 
-// VL = 8, D % 8 == 0: one thread per eight output elements.
-template <int OUT, bool PERM>
+// VL = 8: a block takes one token's columns (blockIdx.y: VPT vectors of eight per thread; short rows share a
+// block), so no thread divides 64-bit numbers; a thread's VPT table indices are asked for together, then its codebook rows.  Bound by the
+// output stream and, with a codebook larger than L1, by the row lookups.  An eighth of the tokens to each die: whoever
+// reads the rows next (a norm deals them the same way) finds them in its own L2.
+template <int OUT, bool PERM, int VPT>
 __global__ void __launch_bounds__(256)
 vq_embedding_vl8_kernel(const int64_t* __restrict__ ids, int64_t n_ids, const uint16_t* __restrict__ idx,
                         int64_t vocab, int groups, const uint16_t* __restrict__ cb, uint32_t nc_minus_1,
-                        const int32_t* __restrict__ inv_perm, float scale, bool scaled, void* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n_ids * groups) return;
-  const int64_t t = i / groups;
-  const int g8 = (int)(i - t * groups);
+                        const int32_t* __restrict__ inv_perm, float scale, bool scaled, void* __restrict__ out, unsigned lanes,
+                        unsigned tokens, unsigned per_die) {
+  int64_t t;
+  int col;
+  if (!token_of_thread(lanes, tokens, per_die, &t, &col) || t >= n_ids) return;
   int64_t tok = ids[t];
   tok = tok < 0 ? 0 : (tok >= vocab ? vocab - 1 : tok);  // ids are clamped, never followed out of the table
   const uint16_t* trow = idx + tok * groups;
-  uint32_t h[8];
+  const int step = (int)lanes, g0 = blockIdx.y * step * VPT + col;
   if constexpr (PERM) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int src = inv_perm[g8 * 8 + e];
-      const uint32_t c = min((uint32_t)trow[src >> 3], nc_minus_1);
-      h[e] = cb[(int64_t)c * 8 + (src & 7)];
+    for (int j = 0; j < VPT; ++j) {
+      const int g8 = g0 + step * j;
+      if (g8 >= groups) return;
+      uint32_t h[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int src = inv_perm[g8 * 8 + e];
+        const uint32_t c = min((uint32_t)trow[src >> 3], nc_minus_1);
+        h[e] = cb[(int64_t)c * 8 + (src & 7)];
+      }
+      store_embedding8<OUT>(out, (t * groups + g8) * 8, h, scale, scaled);
     }
   } else {
-    const uint32_t c = min((uint32_t)trow[g8], nc_minus_1);
-    const u32x4 v = *reinterpret_cast<const u32x4*>(cb + (int64_t)c * 8);
+    u32x4 v[VPT];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      h[2 * e] = v[e] & 0xFFFFu;
-      h[2 * e + 1] = v[e] >> 16;
+    for (int j = 0; j < VPT; ++j)  // columns past the end look up the last one and are not stored
+      v[j] = *reinterpret_cast<const u32x4*>(cb + (int64_t)min((uint32_t)trow[min(g0 + step * j, groups - 1)], nc_minus_1) * 8);
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      if (g0 + step * j >= groups) return;
+      uint32_t h[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        h[2 * e] = v[j][e] & 0xFFFFu;
+        h[2 * e + 1] = v[j][e] >> 16;
+      }
+      store_embedding8<OUT>(out, (t * groups + g0 + step * j) * 8, h, scale, scaled);
     }
   }
-  store_embedding8<OUT>(out, i * 8, h, scale, scaled);
 }
 
 // Any vector length: one thread per output element.
@@ -208,15 +274,21 @@ int launch_vq_embedding(const int64_t* ids, int64_t n_ids, const uint16_t* idx, 
                         const uint16_t* cb, int nc, int vl, const int32_t* inv_perm, float scale, void* out,
                         hipStream_t st) {
   const bool scaled = scale != 1.0f;
-  if (vl == 8 && aligned16(cb) && aligned16(out)) {
-    const int64_t n = n_ids * groups;
-    const unsigned blocks = (unsigned)((n + 255) / 256);
-    if (inv_perm)
-      vq_embedding_vl8_kernel<OUT, true><<<blocks, 256, 0, st>>>(ids, n_ids, idx, vocab, groups, cb, (uint32_t)nc - 1u,
-                                                                 inv_perm, scale, scaled, out);
-    else
-      vq_embedding_vl8_kernel<OUT, false><<<blocks, 256, 0, st>>>(ids, n_ids, idx, vocab, groups, cb,
-                                                                  (uint32_t)nc - 1u, nullptr, scale, scaled, out);
+  if (vl == 8 && aligned16(cb) && aligned16(out) && n_ids <= 0x7FFFFFF0 && groups <= 256 * 65535) {
+    const TokenGrid tg(groups, n_ids);
+    const DieGrid rows((n_ids + tg.tokens - 1) / tg.tokens, n_ids * groups * 16, kAuxDieBytes);
+    const dim3 grid(rows.blocks, (unsigned)tg.segments);
+#define NPAMD_VQ_EMB(PERM, VPT)                                                                                      \
+  vq_embedding_vl8_kernel<OUT, PERM, VPT><<<grid, tg.threads, 0, st>>>(ids, n_ids, idx, vocab, groups, cb, (uint32_t)nc - 1u, \
+                                                                inv_perm, scale, scaled, out, tg.lanes, tg.tokens, rows.per_die)
+    if (inv_perm) {
+      if (tg.vpt == 2) NPAMD_VQ_EMB(true, 2);
+      else NPAMD_VQ_EMB(true, 1);
+    } else {
+      if (tg.vpt == 2) NPAMD_VQ_EMB(false, 2);
+      else NPAMD_VQ_EMB(false, 1);
+    }
+#undef NPAMD_VQ_EMB
   } else {
     const int64_t n = n_ids * groups * vl;
     vq_embedding_generic_kernel<OUT><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(
@@ -244,47 +316,60 @@ __device__ __forceinline__ void store_q_embedding(void* out, int64_t at, float v
   else store_from_f32<OUT>(out, at, f16_bits_to_f32(h) * embed_scale);
 }
 
-// 4-bit codes, group size a multiple of 8: one thread per eight elements (one 32-bit load of codes).
-template <int OUT>
+// 4-bit codes, group size a multiple of 8: eight elements (one 32-bit load of codes) at a time, VPT of them per thread;
+// blocks and dies as for the VQ lookup.
+template <int OUT, int VPT>
 __global__ void __launch_bounds__(256)
 q4_embedding_kernel(const int64_t* __restrict__ ids, int64_t n_ids, const uint8_t* __restrict__ w_pack,
-                    const uint16_t* __restrict__ scale, const uint16_t* __restrict__ zp, int group_size,
+                    const uint16_t* __restrict__ scale, const uint16_t* __restrict__ zp, int octets_per_group,
                     int64_t vocab, int dim, int64_t padding_idx, float embed_scale, bool scaled,
-                    void* __restrict__ out) {
-  const int per_row = dim >> 3;
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n_ids * per_row) return;
-  const int64_t t = i / per_row;
-  const int j8 = (int)(i - t * per_row);
+                    void* __restrict__ out, unsigned lanes, unsigned tokens, unsigned per_die) {
+  int64_t t;
+  int col;
+  if (!token_of_thread(lanes, tokens, per_die, &t, &col) || t >= n_ids) return;
+  const int per_row = dim >> 3, groups = per_row / octets_per_group;
   const int64_t raw = ids[t];
   const int64_t tok = raw < 0 ? 0 : (raw >= vocab ? vocab - 1 : raw);
-  const uint32_t codes = *reinterpret_cast<const uint32_t*>(w_pack + tok * (dim >> 1) + j8 * 4);
-  const int64_t grp = tok * (dim / group_size) + (j8 * 8) / group_size;
-  const float s = f16_bits_to_f32(scale[grp]);
-  const float z = zp ? f16_bits_to_f32(zp[grp]) : 8.0f;
+  const uint32_t* wrow = reinterpret_cast<const uint32_t*>(w_pack + tok * (dim >> 1));
   const bool pad = raw == padding_idx;
-  if constexpr (OUT == NPAMD_F32) {
+  uint32_t codes[VPT];
+  float s[VPT], z[VPT];
+  const int step = (int)lanes, o0 = blockIdx.y * step * VPT + col;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float q = (float)((codes >> (4 * e)) & 0xFu);
-      store_q_embedding<OUT>(out, i * 8 + e, pad ? 0.f : (q - z) * s, embed_scale, scaled);
-    }
-  } else {
-    // eight 16-bit results leave as one 16-byte store; same roundings as store_q_embedding
-    uint32_t r[8];
+  for (int j = 0; j < VPT; ++j) {  // columns past the end repeat the last one and are not stored
+    const int o = min(o0 + step * j, per_row - 1);
+    const int64_t grp = tok * groups + o / octets_per_group;
+    codes[j] = wrow[o];
+    s[j] = f16_bits_to_f32(scale[grp]);
+    z[j] = zp ? f16_bits_to_f32(zp[grp]) : 8.0f;
+  }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float q = (float)((codes >> (4 * e)) & 0xFu);
-      const uint32_t h = f32_to_f16_bits(pad ? 0.f : (q - z) * s);
-      if constexpr (OUT == NPAMD_F16) {
-        r[e] = scaled ? f32_to_f16_bits(f16_bits_to_f32(h) * embed_scale) : h;
-      } else {
-        const uint32_t b = f32_to_bf16_bits(f16_bits_to_f32(h));
-        r[e] = scaled ? f32_to_bf16_bits(bf16_bits_to_f32(b) * embed_scale) : b;
+  for (int j = 0; j < VPT; ++j) {
+    if (o0 + step * j >= per_row) return;
+    const int64_t i = t * per_row + o0 + step * j;
+    if constexpr (OUT == NPAMD_F32) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float q = (float)((codes[j] >> (4 * e)) & 0xFu);
+        store_q_embedding<OUT>(out, i * 8 + e, pad ? 0.f : (q - z[j]) * s[j], embed_scale, scaled);
       }
+    } else {
+      // eight 16-bit results leave as one 16-byte store; same roundings as store_q_embedding
+      uint32_t r[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float q = (float)((codes[j] >> (4 * e)) & 0xFu);
+        const uint32_t h = f32_to_f16_bits(pad ? 0.f : (q - z[j]) * s[j]);
+        if constexpr (OUT == NPAMD_F16) {
+          r[e] = scaled ? f32_to_f16_bits(f16_bits_to_f32(h) * embed_scale) : h;
+        } else {
+          const uint32_t b = f32_to_bf16_bits(f16_bits_to_f32(h));
+          r[e] = scaled ? f32_to_bf16_bits(bf16_bits_to_f32(b) * embed_scale) : b;
+        }
+      }
+      *reinterpret_cast<u32x4*>((uint16_t*)out + i * 8) =
+          u32x4{r[0] | (r[1] << 16), r[2] | (r[3] << 16), r[4] | (r[5] << 16), r[6] | (r[7] << 16)};
     }
-    *reinterpret_cast<u32x4*>((uint16_t*)out + i * 8) =
-        u32x4{r[0] | (r[1] << 16), r[2] | (r[3] << 16), r[4] | (r[5] << 16), r[6] | (r[7] << 16)};
   }
 }
 
@@ -315,11 +400,16 @@ int launch_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
                        float embed_scale, void* out, hipStream_t st) {
   const bool scaled = embed_scale != 1.0f;
   if (nbits == 4 && group_size % 8 == 0 && dim % 8 == 0 && (reinterpret_cast<uintptr_t>(w_pack) & 3) == 0 &&
-      aligned16(out)) {
-    const int64_t n = n_ids * (dim / 8);
-    q4_embedding_kernel<OUT><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(ids, n_ids, w_pack, scale, zp, group_size,
-                                                                          vocab, dim, padding_idx, embed_scale, scaled,
-                                                                          out);
+      aligned16(out) && n_ids <= 0x7FFFFFF0) {
+    const TokenGrid tg(dim / 8, n_ids);
+    const DieGrid rows((n_ids + tg.tokens - 1) / tg.tokens, n_ids * dim * 2, kAuxDieBytes);
+    const dim3 grid(rows.blocks, (unsigned)tg.segments);
+#define NPAMD_Q4_EMB(VPT)                                                                                            \
+  q4_embedding_kernel<OUT, VPT><<<grid, tg.threads, 0, st>>>(ids, n_ids, w_pack, scale, zp, group_size / 8, vocab, dim,     \
+                                                      padding_idx, embed_scale, scaled, out, tg.lanes, tg.tokens, rows.per_die)
+    if (tg.vpt == 2) NPAMD_Q4_EMB(2);
+    else NPAMD_Q4_EMB(1);
+#undef NPAMD_Q4_EMB
   } else {
     const int64_t n = n_ids * dim;
     q_embedding_generic_kernel<OUT><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(

@@ -83,8 +83,8 @@ __device__ __forceinline__ int64_t die_block(unsigned block, unsigned per_die) {
 // (14336 x 4096, decode + library product of 4096 tokens: 368 us against 379).
 struct DieGrid {
   unsigned blocks, per_die;
-  DieGrid(int64_t items, int64_t bytes_written) {
-    const bool by_die = bytes_written <= (int64_t)64 << 20;
+  DieGrid(int64_t items, int64_t bytes_written, int64_t most = (int64_t)64 << 20) {
+    const bool by_die = bytes_written <= most;
     per_die = by_die ? (unsigned)((items + 7) / 8) : 0;
     blocks = by_die ? per_die * 8 : (unsigned)items;
   }
