@@ -156,75 +156,110 @@ struct T2ProdVq16 {
 };
 
 // ---------------------------------------------------------------------------------------------
-// Producers: int4 / int8 group-affine codes.  Packed bytes and the dword that holds the group's scale
-// (and zero point) go to an LDS staging ring of three steps per column tile (directly, like
-// everything else the kernel loads, so that one in-order counter tracks all of a wave's loads).  Wave
-// w decodes the operand pair J = w / 4 of column tile w % 4; the two waves of a column tile share its
-// ring and request the bytes of alternate steps.  In step t the bytes of step t + 3 are requested,
-// the operands of step t + 1 decoded from registers into the other W slot (ring of two) between
-// the MFMAs, and the bytes of step t + 2 read out of the ring, a barrier ahead of their decoding so
-// that it never waits for LDS.  The arithmetic is the providers' (providers.hpp): bit for bit the
-// one-pass decode.
+// Producers: int4 / int8 group-affine codes.  A column's codes are staged a line at a time: kLine bytes
+// are kSteps steps of it (four of int4, two of int8 in a line of 128 bytes), one load instruction
+// fetches them for eight columns, and the dwords that hold the scales (and zero points) of the same
+// steps come with it.  What the address unit and the L2 spend goes with the lines a load touches, not
+// with its bytes: codes and scales fetched step by step (32 lines per instruction for 32 and 4 bytes
+// of each) kept them as busy as the x tile does, and the two together paced the loop (14336 x 4096
+// int4, 256 / 512 tokens: 48.8 / 79.0 us; by lines 45.4 / 70.8).
+//
+// The two waves of a column tile share its ring of kRing lines, each fetching half of its columns;
+// 16-byte piece p of column r sits in slot p ^ f(r) of its line and dword q of its scales in q ^ g(r), which
+// spreads the reads of 32 columns over the banks.  Wave w decodes the operand pair J = w / 4 of column
+// tile w % 4: in step t the operands of step t + 1 are decoded from registers into the other W slot (ring
+// of two) between the MFMAs, and the bytes of step t + 2 read out of the ring, a barrier ahead of their
+// decoding so that it never waits for LDS.  A line whose last bytes were read in step t - 1 is fetched
+// over from step t on.  The arithmetic is the providers' (providers.hpp): bit for bit the one-pass decode.
 // ---------------------------------------------------------------------------------------------
-template <int ACT, int NBITS, bool ASYM>
+template <int ACT, int NBITS, bool ASYM, int MW>
 struct T2ProdQ {
   using P = typename std::conditional<NBITS == 4, Q4Provider<ACT, ASYM>, Q8Provider<ACT, ASYM>>::type;
   using Args = typename P::Args;
   static constexpr int kWRing = 2;
-  static constexpr int kCodeLoads = NBITS == 4 ? 1 : 2;
-  static constexpr int kSlot = kCodeLoads * 1024 + 256 + (ASYM ? 256 : 0);
   static constexpr int kHandoffBatch = 2;
-  static constexpr int kStageTile = 3 * kSlot;
+  static constexpr int kStepBytes = NBITS * 8;            // of a column
+  static constexpr int kLine = MW == 3 ? 64 : 128;        // beside three row tiles LDS holds half lines
+  static constexpr int kSteps = kLine / kStepBytes;       // steps per line
+  static constexpr int kRing = kSteps == 1 ? 3 : 2;       // lines per column
+  static constexpr int kSlots = kLine / 16;
+  static constexpr int kColsPerLoad = 64 / kSlots;
+  static constexpr int kCodeLoads = 32 / kColsPerLoad / 2;  // per wave and line
+  static constexpr int kScaleLoads = kSteps == 1 ? 1 : kSteps / 2;  // per wave and line (one step: the first wave's)
+  static constexpr int kLoads = kCodeLoads + kScaleLoads * (ASYM ? 2 : 1);
+  static constexpr int kCodeBytes = 32 * kLine;           // of a column tile's line
+  static constexpr int kScaleBytes = 32 * kSteps * 8;     // the dwords of (step, k half) per column
+  static constexpr int kSlot = kCodeBytes + kScaleBytes * (ASYM ? 2 : 1);
+  static constexpr int kStageTile = kRing * kSlot;
   static constexpr int kStageBytes = 4 * kStageTile;
   const Args& a;
   const KWalk& kw;
   const P prov;
-  int tcol, J, lane, h;
+  int tcol, J, lane, c, h, n0t, N;
   uint8_t* ws;
   uint8_t* stage;      // this column tile's ring
   uint32_t stage_lds;
-  uint32_t code_off;   // byte offset of the lane's share of chunk 0 of its row
-  uint32_t scale_row;  // index of the row's first scale
-  int cur = 0;         // step % 3: the ring slot the bytes of step + 3 go to
+  uint32_t code_row[kCodeLoads];    // byte offset of chunk 0 of the row whose codes the lane fetches
+  uint32_t scale_row;  // index of the first scale of the lane's column
   u32x2 raw0, raw1;    // the operand pair being decoded
   uint32_t s2, z;
-  __device__ T2ProdQ(const Args& args, const KWalk& walk, int wave, int lane_, int n0, int N, uint8_t* ws_, uint32_t /*ws_lds*/,
+  __device__ T2ProdQ(const Args& args, const KWalk& walk, int wave, int lane_, int n0, int N_, uint8_t* ws_, uint32_t /*ws_lds*/,
                       uint8_t* stage_, uint32_t stage_lds_)
-      : a(args), kw(walk), prov(args), tcol(wave & 3), J(wave >> 2), lane(lane_), h(lane_ >> 5), ws(ws_),
-        stage(stage_ + (wave & 3) * kStageTile), stage_lds(stage_lds_ + (uint32_t)((wave & 3) * kStageTile)) {
-    const int ncol = min(n0 + 32 * tcol + (lane_ & 31), N - 1);  // columns past N decode a valid row nobody stores
-    code_off = (uint32_t)ncol * (uint32_t)args.chunks * (NBITS == 4 ? 32u : 64u) + (uint32_t)h * (NBITS == 4 ? 16u : 32u);
-    scale_row = (uint32_t)ncol * (uint32_t)args.groups_per_row;
+      : a(args), kw(walk), prov(args), tcol(wave & 3), J(wave >> 2), lane(lane_), c(lane_ & 31), h(lane_ >> 5),
+        n0t(n0 + 32 * (wave & 3)), N(N_), ws(ws_), stage(stage_ + (wave & 3) * kStageTile),
+        stage_lds(stage_lds_ + (uint32_t)((wave & 3) * kStageTile)) {
+#pragma unroll
+    for (int i = 0; i < kCodeLoads; ++i)
+      code_row[i] = row_of(16 * J + kColsPerLoad * i + lane / kSlots) * (uint32_t)args.chunks * (uint32_t)kStepBytes;
+    scale_row = row_of(c) * (uint32_t)args.groups_per_row;
   }
-  __device__ __forceinline__ uint32_t scale_index(int step) const {
-    return scale_row + (uint32_t)((2 * kw.chunk_of(step) + h) >> a.gs_shift_chunks);
+  // The weight row of column r of the tile; columns past N decode a valid row nobody stores.
+  __device__ __forceinline__ uint32_t row_of(int r) const { return (uint32_t)min(n0t + r, N - 1); }
+  static __device__ __forceinline__ int code_swizzle(int r) { return kSlots == 8 ? (r >> 1) & 7 : (r >> 2) & 3; }
+  static __device__ __forceinline__ int scale_swizzle(int r) { return 2 * ((r * kSteps) >> 5); }
+  __device__ __forceinline__ uint32_t group_of(int step, int half) const {
+    return (uint32_t)((2 * kw.chunk_of(step) + half) >> a.gs_shift_chunks);
   }
-  // The packed bytes and scales of `step` into ring slot `slot` (by the wave whose J is the step's parity).
-  __device__ __forceinline__ void request(int step, int slot) const {
-    if ((step & 1) != J) return;
-    const uint32_t dst = stage_lds + (uint32_t)(slot * kSlot);
-    const uint32_t off = code_off + (uint32_t)kw.chunk_of(step) * (NBITS == 4 ? 32u : 64u);
-    lds_load16(dst, off, a.w_pack);
-    if (NBITS == 8) lds_load16(dst + 1024, off + 16u, a.w_pack);
-    const uint32_t sb = (scale_index(step) * 2u) & ~3u;
-    lds_load4(dst + kCodeLoads * 1024, sb, a.scale);
-    if (ASYM) lds_load4(dst + kCodeLoads * 1024 + 256, sb, a.zp);
+  // The wave's share of line `line`.
+  __device__ __forceinline__ void request(int line) const {
+    const uint32_t dst = stage_lds + (uint32_t)((line % kRing) * kSlot);
+#pragma unroll
+    for (int i = 0; i < kCodeLoads; ++i) {
+      const int r = 16 * J + kColsPerLoad * i;  // + lane / kSlots
+      const int piece = (lane % kSlots) ^ code_swizzle(r + lane / kSlots);
+      const uint32_t chunk = (uint32_t)kw.chunk_of(kSteps * line + piece * 16 / kStepBytes);
+      lds_load16(dst + (uint32_t)(r * kLine), code_row[i] + chunk * (uint32_t)kStepBytes + (uint32_t)(piece * 16 % kStepBytes),
+                 a.w_pack);
+    }
+    if (kSteps == 1 && J != 0) return;
+    constexpr int kDwords = 2 * kSteps, kCols = 64 / kDwords;
+#pragma unroll
+    for (int i = 0; i < kScaleLoads; ++i) {
+      const int r0 = kCols * (J * kScaleLoads + i), r = r0 + lane / kDwords;
+      const int q = (lane % kDwords) ^ scale_swizzle(r);
+      const uint32_t index = row_of(r) * (uint32_t)a.groups_per_row + group_of(kSteps * line + (q >> 1), q & 1);
+      const uint32_t sb = (index * 2u) & ~3u, at = dst + (uint32_t)(kCodeBytes + r0 * kDwords * 4);
+      lds_load4(at, sb, a.scale);
+      if (ASYM) lds_load4(at + (uint32_t)kScaleBytes, sb, a.zp);
+    }
   }
-  // Reads the wave's half of the staged bytes of `step` out of ring slot `slot`.
-  __device__ __forceinline__ void fetch(int step, int slot) {
-    const uint8_t* src = stage + slot * kSlot;
+  // Reads the wave's half of the staged bytes of `step` out of the ring.
+  __device__ __forceinline__ void fetch(int step) {
+    const int line = step / kSteps, p = step % kSteps;
+    const uint8_t* src = stage + (line % kRing) * kSlot;
+    const uint8_t* codes = src + c * kLine;
     if (NBITS == 4) {
-      raw0 = *reinterpret_cast<const u32x2*>(src + lane * 16 + J * 8);
-    } else {  // operand O of a lane: dwords 2 (O & 1), 2 (O & 1) + 1 of its 16 bytes in KiB O / 2
-      const u32x4 r = *reinterpret_cast<const u32x4*>(src + J * 1024 + lane * 16);
+      raw0 = *reinterpret_cast<const u32x2*>(codes + (((2 * p + h) ^ code_swizzle(c)) << 4) + J * 8);
+    } else {
+      const u32x4 r = *reinterpret_cast<const u32x4*>(codes + (((4 * p + 2 * h + J) ^ code_swizzle(c)) << 4));
       raw0 = u32x2{r.x, r.y};
       raw1 = u32x2{r.z, r.w};
     }
-    const uint32_t sh = (scale_index(step) & 1u) * 16u;
-    const uint32_t sd = *reinterpret_cast<const uint32_t*>(src + kCodeLoads * 1024 + lane * 4);
-    s2 = ((sd >> sh) & 0xFFFFu) * 0x10001u;
+    const uint32_t sh = ((scale_row + group_of(step, h)) & 1u) * 16u;
+    const uint8_t* sc = src + kCodeBytes + c * (8 * kSteps) + (((2 * p + h) ^ scale_swizzle(c)) << 2);
+    s2 = ((*reinterpret_cast<const uint32_t*>(sc) >> sh) & 0xFFFFu) * 0x10001u;
     z = 0;
-    if (ASYM) z = (*reinterpret_cast<const uint32_t*>(src + kCodeLoads * 1024 + 256 + lane * 4) >> sh) & 0xFFFFu;
+    if (ASYM) z = (*reinterpret_cast<const uint32_t*>(sc + kScaleBytes) >> sh) & 0xFFFFu;
   }
   template <int I>
   __device__ __forceinline__ void decode(int wslot) const {
@@ -234,37 +269,37 @@ struct T2ProdQ {
     *reinterpret_cast<u32x4*>(ws + wslot * kT2WSlotBytes + (tcol * 4 + 2 * J + I) * 1024 + lane * 16) = op;
   }
   __device__ __forceinline__ void prologue_issue() const {
-    request(0, 0);
-    request(1, 1);
-    request(2, 2);
+#pragma unroll
+    for (int i = 0; i < kRing; ++i) request(i);
   }
   // Everything requested has arrived: the W tile of step 0, and the bytes of step 1 in registers.
   __device__ __forceinline__ void prologue_finish() {
-    fetch(0, 0);
+    fetch(0);
     decode<0>(0);
     decode<1>(0);
-    fetch(1, 1);
+    fetch(1);
   }
-  // In step t: the bytes of step t + 3 requested (they are waited for with the x pieces at the end of
-  // the step), the operands of step t + 1 decoded from the registers into the other W slot, and the
-  // bytes of step t + 2 read out of the ring a barrier ahead of their decoding.
+  // The last bytes of line l are read in step kSteps l + kSteps - 3; line l + kRing is requested from the step after
+  // on: one step later where a line is several steps (two steps before its first bytes are read), at once where it is one.
+  static __device__ __forceinline__ bool requests(int step) { return (step + 2) % kSteps == 0; }
   template <int J_, int T>
   __device__ __forceinline__ void work(int step, int wslot, int rem) {
-    if (J_ == 0 && T == 0 && rem >= 2) request(step + 3, cur);
     if (J_ == 1 && T == 0 && rem >= 1) decode<0>(wslot ^ 1);
     if (J_ == 2 && T == 0 && rem >= 1) decode<1>(wslot ^ 1);
-    if (J_ == 3 && T == 1) {
-      if (rem >= 2) fetch(step + 2, cur == 0 ? 2 : cur - 1);
-      cur = cur == 2 ? 0 : cur + 1;
-    }
+    if (J_ == 2 && T == 1 && rem >= 2 && requests(step)) request((step + 2) / kSteps + 1);
+    if (J_ == 3 && T == 1 && rem >= 2) fetch(step + 2);
   }
   __device__ __forceinline__ void work_all(int step, int wslot, int rem) {
-    work<0, 0>(step, wslot, rem);
     work<1, 0>(step, wslot, rem);
     work<2, 0>(step, wslot, rem);
+    work<2, 1>(step, wslot, rem);
     work<3, 1>(step, wslot, rem);
   }
-  __device__ __forceinline__ void wait_step_end(int, int) const { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+  // The x pieces of the next step, requested before a line, have to be there; the line has a step more.
+  __device__ __forceinline__ void wait_step_end(int step, int rem) const {
+    if (kSteps > 1 && rem >= 2 && requests(step)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
 };
 
 template <int ACT, int MW, class Prod>
@@ -313,7 +348,7 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
   KWalk kw;
   kw.chunk0 = bz * s.split_chunks;
   kw.steps = min(s.split_chunks, s.chunks - kw.chunk0);
-  kw.rot = (int)((bx * 7u) % (unsigned)kw.steps);
+  kw.rot = (int)((bx * 7u) % (unsigned)kw.steps) & ~3;  // four steps of codes or indices stay in one line
   const int steps = kw.steps;
 
   const uint32_t xs_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)xs;
@@ -552,8 +587,22 @@ int launch_tile2_mw(const GemmShape& s, const typename Prod::Args& a, const T2Pa
   return check_launch(what);
 }
 
-template <int ACT, class Prod>
-int launch_tile2_prod(GemmShape s, const typename Prod::Args& a, hipStream_t st, const char* what, void* workspace,
+// The producer of a kernel by its row tiles per wave.
+template <int ACT>
+struct T2Vq16Prods {
+  using Args = T2Args;
+  template <int MW>
+  using Of = T2ProdVq16<ACT>;
+};
+template <int ACT, int NBITS, bool ASYM>
+struct T2QProds {
+  using Args = typename T2ProdQ<ACT, NBITS, ASYM, 1>::Args;
+  template <int MW>
+  using Of = T2ProdQ<ACT, NBITS, ASYM, MW>;
+};
+
+template <int ACT, class Prods>
+int launch_tile2_prod(GemmShape s, const typename Prods::Args& a, hipStream_t st, const char* what, void* workspace,
                       int64_t workspace_bytes, int mw) {
   const int splits = plan_tile2_splits(s.M, s.N, s.chunks, mw);
   if (splits > 1 && (!workspace || tile2_workspace_bytes(s.M, s.N, s.chunks, mw) > workspace_bytes)) return 1;
@@ -571,30 +620,30 @@ int launch_tile2_prod(GemmShape s, const typename Prod::Args& a, hipStream_t st,
     pair.call = next_call_number();
   }
   switch (mw) {
-    case 1: return launch_tile2_mw<ACT, 1, Prod>(s, a, pair, st, what);
-    case 2: return launch_tile2_mw<ACT, 2, Prod>(s, a, pair, st, what);
-    default: return launch_tile2_mw<ACT, 3, Prod>(s, a, pair, st, what);
+    case 1: return launch_tile2_mw<ACT, 1, typename Prods::template Of<1>>(s, a, pair, st, what);
+    case 2: return launch_tile2_mw<ACT, 2, typename Prods::template Of<2>>(s, a, pair, st, what);
+    default: return launch_tile2_mw<ACT, 3, typename Prods::template Of<3>>(s, a, pair, st, what);
   }
 }
 
 int launch_tile2(int act, const GemmShape& s, const T2Args& a, hipStream_t st, const char* what, void* workspace,
                  int64_t workspace_bytes) {
   const int mw = plan_tile_mw(s.M);
-  return act == NPAMD_BF16 ? launch_tile2_prod<NPAMD_BF16, T2ProdVq16<NPAMD_BF16>>(s, a, st, what, workspace, workspace_bytes, mw)
-                           : launch_tile2_prod<NPAMD_F16, T2ProdVq16<NPAMD_F16>>(s, a, st, what, workspace, workspace_bytes, mw);
+  return act == NPAMD_BF16 ? launch_tile2_prod<NPAMD_BF16, T2Vq16Prods<NPAMD_BF16>>(s, a, st, what, workspace, workspace_bytes, mw)
+                           : launch_tile2_prod<NPAMD_F16, T2Vq16Prods<NPAMD_F16>>(s, a, st, what, workspace, workspace_bytes, mw);
 }
 
 template <int ACT, int NBITS>
 static int launch_tile2_q_bits(bool asym, const GemmShape& s, const T2QArgs& q, hipStream_t st, const char* what,
                                void* workspace, int64_t workspace_bytes) {
   if (asym) {
-    using Prod = T2ProdQ<ACT, NBITS, true>;
-    const typename Prod::Args a{q.w_pack, q.scale, q.chunks, q.groups_per_row, q.gs_shift_chunks, q.zp};
-    return launch_tile2_prod<ACT, Prod>(s, a, st, what, workspace, workspace_bytes, plan_tile2_q_mw(s.M));
+    using Prods = T2QProds<ACT, NBITS, true>;
+    const typename Prods::Args a{q.w_pack, q.scale, q.chunks, q.groups_per_row, q.gs_shift_chunks, q.zp};
+    return launch_tile2_prod<ACT, Prods>(s, a, st, what, workspace, workspace_bytes, plan_tile2_q_mw(s.M));
   }
-  using Prod = T2ProdQ<ACT, NBITS, false>;
-  const typename Prod::Args a{q.w_pack, q.scale, q.chunks, q.groups_per_row, q.gs_shift_chunks, q.zp};
-  return launch_tile2_prod<ACT, Prod>(s, a, st, what, workspace, workspace_bytes, plan_tile2_q_mw(s.M));
+  using Prods = T2QProds<ACT, NBITS, false>;
+  const typename Prods::Args a{q.w_pack, q.scale, q.chunks, q.groups_per_row, q.gs_shift_chunks, q.zp};
+  return launch_tile2_prod<ACT, Prods>(s, a, st, what, workspace, workspace_bytes, plan_tile2_q_mw(s.M));
 }
 
 int launch_tile2_q(int act, int nbits, const GemmShape& s, const T2QArgs& q, hipStream_t st, const char* what,

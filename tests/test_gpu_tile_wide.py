@@ -212,3 +212,25 @@ def test_wide_tile_gemm_meets_through_a_workspace_nobody_cleared(gpu, tile_wide,
         torch.cuda.synchronize()
         assert torch.equal(y, expect)
         assert torch.equal(kernels.vq_gemm_tile(x, pk, cb, 16, n, bias), expect)  # eager work between the replays
+
+
+@pytest.mark.parametrize("nbits,asym,gs", [(4, False, 32), (4, True, 64), (8, False, 64), (8, True, 32)])
+@pytest.mark.parametrize("m", [100, 256, 300])
+@pytest.mark.parametrize("k", [192, 320, 384, 448, 832])
+def test_wide_tile_gemm_walks_lines_of_codes(gpu, tile_wide, nbits, asym, gs, m, k):
+    """Codes and scales are staged a line of several 64-k steps at a time, in a walk over K that starts elsewhere in
+    every column block: step counts of every remainder, rows that start off a line, the three row-tile
+    counts (half lines with three).  One-hot activations return the one-pass decode exactly."""
+    from neuropress_amd import kernels
+
+    n = 1300
+    Q = cases.q4_layer(70 + k, n, k, nbits=nbits, gs=gs, act=torch.bfloat16, m=1, asym=asym)
+    blob, sc = Q["blob"].to(gpu), Q["scale"].to(gpu)
+    zp = None if Q["zp"] is None else Q["zp"].to(gpu)
+    wt = kernels.q_dequant(blob, sc, nbits, gs, zp, torch.bfloat16).t().contiguous()
+    pick = (torch.arange(m, device=gpu) * 7) % k
+    x = torch.zeros(m, k, dtype=torch.bfloat16, device=gpu)
+    x[torch.arange(m, device=gpu), pick] = 1
+    for splits in (1, 2):
+        tile_wide(2, splits)
+        assert torch.equal(kernels.q_gemm_tile(x, blob, sc, nbits, gs, zp), wt[pick]), f"{splits} splits"
