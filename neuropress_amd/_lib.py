@@ -121,9 +121,12 @@ def host():
             loader.exec_module(module)
         except ImportError as exc:
             raise RuntimeError(f"neuropress_amd: cannot load {HOST_PATH}: {exc}; build it with `python -m neuropress_amd.build`") from exc
+        import torch
+
         from . import kernels
 
         module.set_workspaces(kernels._SLICED_WORKSPACES, kernels.drop_sliced_workspace_of)
+        module.set_module_class(torch.nn.Module, lambda self, *args, **kwargs: torch.nn.Module.__call__(*args, **kwargs))
         _host = module
     return _host
 

@@ -27,10 +27,17 @@ int fail(int code, const char* fmt, ...) {
   return code;
 }
 
+hipError_t& launch_status() {
+  thread_local hipError_t status = hipSuccess;
+  return status;
+}
+
 int check_launch(const char* what) {
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(NPAMD_ERR_LAUNCH, "%s: launch failed: %s", what, hipGetErrorString(e));
-  return NPAMD_OK;
+  const hipError_t e = launch_status();
+  if (e == hipSuccess) return NPAMD_OK;
+  launch_status() = hipSuccess;
+  (void)hipGetLastError();  // reported here: not the next call's
+  return fail(NPAMD_ERR_LAUNCH, "%s: launch failed: %s", what, hipGetErrorString(e));
 }
 
 const char* error_text() { return g_err; }

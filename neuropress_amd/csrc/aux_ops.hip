@@ -147,7 +147,7 @@ int launch_rms_norm(const void* x, int64_t ldx, const void* w, void* out, int64_
       auto ws = (const uint16_t*)w;
       auto os = (uint16_t*)out;
 #define NPAMD_RMS(NV, RW) \
-  rms_norm_wave_kernel<DT, NV, RW><<<grid.blocks, 256, 0, st>>>(xs, ldx, ws, os, ldo, M, H, eps, grid.per_die)
+  launch(rms_norm_wave_kernel<DT, NV, RW>, grid.blocks, 256, 0, st, xs, ldx, ws, os, ldo, M, H, eps, grid.per_die)
       if (M <= kRmsFewRows && H > 512) {
         const DieGrid grid(M, (int64_t)M * H * 2, kAuxDieBytes);
         const int nv = (H / 8 + 255) / 256;
@@ -167,7 +167,7 @@ int launch_rms_norm(const void* x, int64_t ldx, const void* w, void* out, int64_
       return check_launch("npamd_rms_norm");
     }
   }
-  rms_norm_block_kernel<DT><<<M, 256, 0, st>>>(x, ldx, w, out, ldo, H, eps);
+  launch(rms_norm_block_kernel<DT>, M, 256, 0, st, x, ldx, w, out, ldo, H, eps);
   return check_launch("npamd_rms_norm");
 }
 
@@ -279,7 +279,7 @@ int launch_vq_embedding(const int64_t* ids, int64_t n_ids, const uint16_t* idx, 
     const DieGrid rows((n_ids + tg.tokens - 1) / tg.tokens, n_ids * groups * 16, kAuxDieBytes);
     const dim3 grid(rows.blocks, (unsigned)tg.segments);
 #define NPAMD_VQ_EMB(PERM, VPT)                                                                                      \
-  vq_embedding_vl8_kernel<OUT, PERM, VPT><<<grid, tg.threads, 0, st>>>(ids, n_ids, idx, vocab, groups, cb, (uint32_t)nc - 1u, \
+  launch(vq_embedding_vl8_kernel<OUT, PERM, VPT>, grid, tg.threads, 0, st, ids, n_ids, idx, vocab, groups, cb, (uint32_t)nc - 1u, \
                                                                 inv_perm, scale, scaled, out, tg.lanes, tg.tokens, rows.per_die)
     if (inv_perm) {
       if (tg.vpt == 2) NPAMD_VQ_EMB(true, 2);
@@ -291,7 +291,7 @@ int launch_vq_embedding(const int64_t* ids, int64_t n_ids, const uint16_t* idx, 
 #undef NPAMD_VQ_EMB
   } else {
     const int64_t n = n_ids * groups * vl;
-    vq_embedding_generic_kernel<OUT><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(
+    launch(vq_embedding_generic_kernel<OUT>, (unsigned)((n + 255) / 256), 256, 0, st,
         ids, n_ids, idx, vocab, groups, vl, cb, (uint32_t)nc - 1u, inv_perm, scale, scaled, out);
   }
   return check_launch("npamd_vq_embedding");
@@ -405,14 +405,14 @@ int launch_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
     const DieGrid rows((n_ids + tg.tokens - 1) / tg.tokens, n_ids * dim * 2, kAuxDieBytes);
     const dim3 grid(rows.blocks, (unsigned)tg.segments);
 #define NPAMD_Q4_EMB(VPT)                                                                                            \
-  q4_embedding_kernel<OUT, VPT><<<grid, tg.threads, 0, st>>>(ids, n_ids, w_pack, scale, zp, group_size / 8, vocab, dim,     \
+  launch(q4_embedding_kernel<OUT, VPT>, grid, tg.threads, 0, st, ids, n_ids, w_pack, scale, zp, group_size / 8, vocab, dim,     \
                                                       padding_idx, embed_scale, scaled, out, tg.lanes, tg.tokens, rows.per_die)
     if (tg.vpt == 2) NPAMD_Q4_EMB(2);
     else NPAMD_Q4_EMB(1);
 #undef NPAMD_Q4_EMB
   } else {
     const int64_t n = n_ids * dim;
-    q_embedding_generic_kernel<OUT><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(
+    launch(q_embedding_generic_kernel<OUT>, (unsigned)((n + 255) / 256), 256, 0, st,
         ids, n_ids, w_pack, scale, zp, nbits, group_size, vocab, dim, padding_idx, embed_scale, scaled, out);
   }
   return check_launch("npamd_q_embedding");
@@ -476,9 +476,9 @@ extern "C" int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* p
     const dim3 grid(segments, (unsigned)(M - m0 < 65535 ? M - m0 : 65535));
     const uint16_t* xm = xs + (int64_t)m0 * ldx;
     uint16_t* om = os + (int64_t)m0 * ldo;
-    if (!perm) gather_columns_kernel<false, false><<<grid, 256, 0, st>>>(xm, ldx, perm, om, ldo, K, vec);
-    else if (K <= kGatherRowMax) gather_columns_kernel<true, true><<<grid, 256, (K * 2 + 15) & ~15, st>>>(xm, ldx, perm, om, ldo, K, vec);
-    else gather_columns_kernel<true, false><<<grid, 256, 0, st>>>(xm, ldx, perm, om, ldo, K, vec);
+    if (!perm) launch(gather_columns_kernel<false, false>, grid, 256, 0, st, xm, ldx, perm, om, ldo, K, vec);
+    else if (K <= kGatherRowMax) launch(gather_columns_kernel<true, true>, grid, 256, (K * 2 + 15) & ~15, st, xm, ldx, perm, om, ldo, K, vec);
+    else launch(gather_columns_kernel<true, false>, grid, 256, 0, st, xm, ldx, perm, om, ldo, K, vec);
   }
   return check_launch("npamd_gather_columns");
 }

@@ -152,9 +152,9 @@ __global__ void __launch_bounds__(256) coded_gemv_kernel(const CodedArgs a) {
 template <int ACT>
 static int launch_coded(const CodedArgs& a, hipStream_t st, const char* what) {
   const unsigned rows = (unsigned)((a.N + 3) / 4);
-  if (a.M == 1) coded_gemv_kernel<ACT, 1><<<dim3(rows, 1), 256, 0, st>>>(a);
-  else if (a.M <= 4) coded_gemv_kernel<ACT, 4><<<dim3(rows, 1), 256, 0, st>>>(a);
-  else coded_gemv_kernel<ACT, 8><<<dim3(rows, (unsigned)((a.M + 7) / 8)), 256, 0, st>>>(a);
+  if (a.M == 1) launch(coded_gemv_kernel<ACT, 1>, dim3(rows, 1), 256, 0, st, a);
+  else if (a.M <= 4) launch(coded_gemv_kernel<ACT, 4>, dim3(rows, 1), 256, 0, st, a);
+  else launch(coded_gemv_kernel<ACT, 8>, dim3(rows, (unsigned)((a.M + 7) / 8)), 256, 0, st, a);
   return check_launch(what);
 }
 

@@ -242,7 +242,7 @@ int launch_dense_tile(DenseShape s, hipStream_t st) {
   const hipError_t e = enable_dynamic_lds(latch, reinterpret_cast<const void*>(&dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES>), T::kLds);
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "npamd_dense_gemm: cannot reserve %d bytes of LDS: %s", T::kLds, hipGetErrorString(e));
-  dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES><<<(unsigned)blocks, T::kThreads, T::kLds, st>>>(s);
+  launch(dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES>, (unsigned)blocks, T::kThreads, T::kLds, st, s);
   return check_launch("npamd_dense_gemm");
 }
 

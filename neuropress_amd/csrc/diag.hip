@@ -96,9 +96,9 @@ extern "C" int npamd_diag_mfma(const void* operands, int blocks, int mfmas_per_w
   NPAMD_REQUIRE(act_dtype == NPAMD_F16 || act_dtype == NPAMD_BF16, "npamd_diag_mfma: f16 or bf16");
   const int rounds = (mfmas_per_wave + 11) / 12;
   if (act_dtype == NPAMD_BF16)
-    diag_mfma_kernel<NPAMD_BF16><<<blocks, 256, 0, (hipStream_t)stream>>>((const u32x4*)operands, (float*)sink16, rounds);
+    launch(diag_mfma_kernel<NPAMD_BF16>, blocks, 256, 0, (hipStream_t)stream, (const u32x4*)operands, (float*)sink16, rounds);
   else
-    diag_mfma_kernel<NPAMD_F16><<<blocks, 256, 0, (hipStream_t)stream>>>((const u32x4*)operands, (float*)sink16, rounds);
+    launch(diag_mfma_kernel<NPAMD_F16>, blocks, 256, 0, (hipStream_t)stream, (const u32x4*)operands, (float*)sink16, rounds);
   return check_launch("npamd_diag_mfma");
 }
 
@@ -106,7 +106,7 @@ extern "C" int npamd_diag_stream_read(const void* src, int64_t n_bytes, void* si
   NPAMD_REQUIRE(src && sink16 && n_bytes >= 16 && n_bytes % 16 == 0,
                 "npamd_diag_stream_read: need a non-null buffer of a multiple of 16 bytes");
   const int64_t n16 = n_bytes / 16;
-  diag_stream_read_kernel<<<(unsigned)((n16 + 255) / 256), 256, 0, (hipStream_t)stream>>>(
+  launch(diag_stream_read_kernel, (unsigned)((n16 + 255) / 256), 256, 0, (hipStream_t)stream,
       (const u32x4*)src, (u32x4*)sink16, n16);
   return check_launch("npamd_diag_stream_read");
 }
@@ -120,7 +120,7 @@ extern "C" int npamd_diag_gather(const void* idx_u16, int64_t n_indices, const v
   const int64_t n8 = n_indices / 8;
   hipStream_t st = (hipStream_t)stream;
   if (!from_lds) {
-    diag_gather_global_kernel<<<(unsigned)((n8 + 255) / 256), 256, 0, st>>>(
+    launch(diag_gather_global_kernel, (unsigned)((n8 + 255) / 256), 256, 0, st,
         (const u32x4*)idx_u16, (const u32x4*)table16, (uint32_t)table_entries - 1u, (u32x4*)sink16, n8);
     return check_launch("npamd_diag_gather");
   }
@@ -133,7 +133,7 @@ extern "C" int npamd_diag_gather(const void* idx_u16, int64_t n_indices, const v
   }
   const int blocks = 512;
   const int64_t per_block = (n8 + blocks - 1) / blocks;
-  diag_gather_lds_kernel<<<blocks, 1024, lds, st>>>((const u32x4*)idx_u16, (const u32x4*)table16,
+  launch(diag_gather_lds_kernel, blocks, 1024, lds, st, (const u32x4*)idx_u16, (const u32x4*)table16,
                                                     table_entries, (u32x4*)sink16, n8, per_block);
   return check_launch("npamd_diag_gather");
 }

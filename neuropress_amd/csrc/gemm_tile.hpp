@@ -526,10 +526,10 @@ int launch_tile_gemm_mw_cb(const GemmShape& s, const typename Provider::Args& pa
       enable_dynamic_lds(latch, reinterpret_cast<const void*>(&tile_gemm_kernel<ACT, Provider, MW, CB_LDS>), lds);
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds, hipGetErrorString(e));
-  tile_gemm_kernel<ACT, Provider, MW, CB_LDS><<<grid, 512, lds, st>>>(s, pargs);
+  launch(tile_gemm_kernel<ACT, Provider, MW, CB_LDS>, grid, 512, lds, st, s, pargs);
   if (s.splits > 1) {
     const int64_t quads = (int64_t)s.M * ((s.N + 3) / 4);
-    splitk_reduce_kernel<ACT><<<(unsigned)((quads + 255) / 256), 256, 0, st>>>(s.partials, s.splits, s.M, s.N,
+    launch(splitk_reduce_kernel<ACT>, (unsigned)((quads + 255) / 256), 256, 0, st, s.partials, s.splits, s.M, s.N,
                                                                              s.bias, s.y, s.ldy);
   }
   return check_launch(what);

@@ -578,10 +578,10 @@ int launch_tile2_mw(const GemmShape& s, const typename Prod::Args& a, const T2Pa
   const hipError_t e = enable_dynamic_lds(latch, reinterpret_cast<const void*>(&tile2_gemm_kernel<ACT, MW, Prod>), lds);
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds, hipGetErrorString(e));
-  tile2_gemm_kernel<ACT, MW, Prod><<<grid, 512, lds, st>>>(s, a, pair);
+  launch(tile2_gemm_kernel<ACT, MW, Prod>, grid, 512, lds, st, s, a, pair);
   if (s.splits > 2) {
     const int64_t quads = (int64_t)s.M * ((s.N + 3) / 4);
-    splitk_reduce_kernel<ACT><<<(unsigned)((quads + 255) / 256), 256, 0, st>>>(s.partials, s.splits, s.M, s.N,
+    launch(splitk_reduce_kernel<ACT>, (unsigned)((quads + 255) / 256), 256, 0, st, s.partials, s.splits, s.M, s.N,
                                                                              s.bias, s.y, s.ldy);
   }
   return check_launch(what);

@@ -377,7 +377,7 @@ int launch_fused_gemv_r(GemvShape s, const typename Provider::Args& pargs, const
       return fail(NPAMD_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds, hipGetErrorString(e));
   }
   last_gemv_staged() = XS ? 1 : 0;
-  fused_gemv_kernel<ACT, Provider, R, CB_LDS, X_LDS, MT, H, XS><<<blocks, plan.waves * 64, lds, st>>>(s, pargs);
+  launch(fused_gemv_kernel<ACT, Provider, R, CB_LDS, X_LDS, MT, H, XS>, blocks, plan.waves * 64, lds, st, s, pargs);
   return check_launch(what);
 }
 
@@ -547,9 +547,9 @@ template <int ACT, class Elem>
 int launch_generic_gemv(const void* x, int64_t ldx, const float* bias, void* y, int64_t ldy,
                         int M, int N, int K, const Elem& elem, hipStream_t st, const char* what) {
   const unsigned rows = (unsigned)((N + 3) / 4);
-  if (M == 1) generic_rows_kernel<ACT, Elem, 1><<<dim3(rows, 1), 256, 0, st>>>(x, ldx, bias, y, ldy, M, N, K, elem);
-  else if (M <= 4) generic_rows_kernel<ACT, Elem, 4><<<dim3(rows, 1), 256, 0, st>>>(x, ldx, bias, y, ldy, M, N, K, elem);
-  else generic_rows_kernel<ACT, Elem, 16><<<dim3(rows, (unsigned)((M + 15) / 16)), 256, 0, st>>>(x, ldx, bias, y, ldy, M, N, K, elem);
+  if (M == 1) launch(generic_rows_kernel<ACT, Elem, 1>, dim3(rows, 1), 256, 0, st, x, ldx, bias, y, ldy, M, N, K, elem);
+  else if (M <= 4) launch(generic_rows_kernel<ACT, Elem, 4>, dim3(rows, 1), 256, 0, st, x, ldx, bias, y, ldy, M, N, K, elem);
+  else launch(generic_rows_kernel<ACT, Elem, 16>, dim3(rows, (unsigned)((M + 15) / 16)), 256, 0, st, x, ldx, bias, y, ldy, M, N, K, elem);
   return check_launch(what);
 }
 

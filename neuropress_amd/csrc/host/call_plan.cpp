@@ -3,9 +3,9 @@
 //
 // What bounds a decode step of small layers is the time to issue its launches, not the kernels: through
 // Python argument checks and ctypes a call took 12-19 us of host time against 3-9 us of kernel.  Through a plan it
-// takes 4.5-5 us, 2.8 of them the HIP launch itself and 1.0 the output's allocation (us per eager call, before / now:
-// 2048 x 640 with a 256-row codebook 14.6 / 4.5, the nine calls of a block with hidden size 2048 128 / 44, residual VQ
-// 4096 x 4096 18.1 / 8.6 and int4 14336 x 4096 12.3 / 8.3, which are then bound by their kernels).  A plan
+// takes 3.2-4 us, 2.4 of them the HIP launch itself and 0.8 the output's allocation (us per eager call, before / now:
+// 2048 x 640 with a 256-row codebook 15.1 / 3.5, the nine calls of a block with hidden size 2048 130 / 35, residual VQ
+// 4096 x 4096 18.1 / 8.6 and int4 14336 x 4096 12.6 / 8.3, which are then bound by their kernels).  A plan
 // keeps the entry point's constant arguments (addresses, sizes, the kernel that serves a token count) and does
 // per call only what depends on the call: check that nothing it was built from has changed, allocate the output,
 // pass the addresses on.
@@ -24,6 +24,7 @@
 #include <c10/core/GradMode.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <deque>
 #include <unordered_map>
@@ -51,7 +52,7 @@ struct Guard {
   PyObject* dict = nullptr;  // borrowed for the module's own __dict__, owned otherwise
   bool wrappers = false;     // entries that instrumentation replaces: the plan's own calls step aside for them, no more
   uint64_t tag = 0;
-  std::vector<std::pair<PyObject*, PyObject*>> entries;  // owned
+  std::vector<std::pair<PyObject*, PyObject*>> entries;  // owned; a null value: the key has to be absent
 };
 
 uint64_t dict_tag(PyObject* dict) {
@@ -113,6 +114,12 @@ struct Plan {
   bool guarded;
   Guard self;  // entries of the module's own __dict__
   std::vector<Guard>* guards;
+  // What `module(x)` may go straight to the plan under: the class whose forward the plan stands for (null: not at all),
+  // and that torch's own call of a module would do nothing but call that forward.
+  PyTypeObject* direct_type;
+  Guard direct_self;                   // entries of the module's own __dict__
+  std::vector<Guard>* direct_guards;   // of its class and of torch.nn.Module
+  std::vector<PyObject*>* hooks;       // dictionaries of hooks, all of which have to be empty
   std::vector<PyObject*>* held;
   std::vector<Source>* sources;
   std::deque<Template>* templates;
@@ -352,6 +359,17 @@ PyObject* run(Plan* p, PyObject* xo) {
   }
 }
 
+// What torch.nn.Module.__call__ looks at before it calls forward: hooks of the module and of all modules, a compiled
+// call, a replaced forward, a trace being recorded.
+bool direct(Plan* p, PyObject* module) {
+  if (Py_TYPE(module) != p->direct_type || !holds(p->direct_self, *_PyObject_GetDictPtr(module))) return false;
+  for (Guard& g : *p->direct_guards)
+    if (!holds(g, g.dict)) return false;
+  for (PyObject* d : *p->hooks)
+    if (PyDict_GET_SIZE(d) != 0) return false;
+  return !torch::jit::tracer::isTracing();
+}
+
 // plan(module, x)
 PyObject* plan_call(PyObject* self, PyObject* const* args, size_t nargsf, PyObject* kwnames) {
   Plan* p = reinterpret_cast<Plan*>(self);
@@ -391,6 +409,10 @@ PyObject* plan_new(PyTypeObject* type, PyObject* args, PyObject*) {
   new (&p->self) Guard();
   p->names = names;
   p->guards = new std::vector<Guard>();
+  p->direct_type = nullptr;
+  new (&p->direct_self) Guard();
+  p->direct_guards = new std::vector<Guard>();
+  p->hooks = new std::vector<PyObject*>();
   p->held = new std::vector<PyObject*>();
   p->sources = new std::vector<Source>();
   p->templates = new std::deque<Template>();
@@ -400,19 +422,23 @@ PyObject* plan_new(PyTypeObject* type, PyObject* args, PyObject*) {
 
 int plan_traverse(PyObject* self, visitproc visit, void* arg) {
   Plan* p = reinterpret_cast<Plan*>(self);
-  for (auto& e : p->self.entries) {
-    Py_VISIT(e.first);
-    Py_VISIT(e.second);
-  }
-  Py_VISIT(p->names);
-  for (PyObject* o : *p->held) Py_VISIT(o);
-  for (Guard& g : *p->guards) {
-    Py_VISIT(g.dict);
-    for (auto& e : g.entries) {
+  for (Guard* g : {&p->self, &p->direct_self})
+    for (auto& e : g->entries) {
       Py_VISIT(e.first);
       Py_VISIT(e.second);
     }
-  }
+  Py_VISIT(p->direct_type);
+  for (PyObject* o : *p->hooks) Py_VISIT(o);
+  Py_VISIT(p->names);
+  for (PyObject* o : *p->held) Py_VISIT(o);
+  for (std::vector<Guard>* list : {p->guards, p->direct_guards})
+    for (Guard& g : *list) {
+      Py_VISIT(g.dict);
+      for (auto& e : g.entries) {
+        Py_VISIT(e.first);
+        Py_VISIT(e.second);
+      }
+    }
   return 0;
 }
 
@@ -422,6 +448,12 @@ int plan_clear(PyObject* self) {
   clear_guard(p->self, false);
   for (Guard& g : *p->guards) clear_guard(g, true);
   p->guards->clear();
+  clear_guard(p->direct_self, false);
+  for (Guard& g : *p->direct_guards) clear_guard(g, true);
+  p->direct_guards->clear();
+  Py_CLEAR(p->direct_type);
+  for (PyObject* o : *p->hooks) Py_DECREF(o);
+  p->hooks->clear();
   Py_CLEAR(p->names);
   for (PyObject* o : *p->held) Py_DECREF(o);
   p->held->clear();
@@ -433,7 +465,10 @@ void plan_dealloc(PyObject* self) {
   plan_clear(self);
   Plan* p = reinterpret_cast<Plan*>(self);
   p->self.~Guard();
+  p->direct_self.~Guard();
   delete p->guards;
+  delete p->direct_guards;
+  delete p->hooks;
   delete p->held;
   delete p->sources;
   delete p->templates;
@@ -449,10 +484,23 @@ bool fill_guard(Guard& g, PyObject* entries) {
     return false;
   }
   while (PyDict_Next(entries, &at, &key, &value)) {
+    if (value == Py_Ellipsis) value = nullptr;  // the key has to be absent
     Py_INCREF(key);
-    Py_INCREF(value);
+    Py_XINCREF(value);
     g.entries.emplace_back(key, value);
   }
+  return true;
+}
+
+bool make_guard(Guard& g, PyObject* where, PyObject* entries) {
+  PyObject* dict = PyType_Check(where) ? reinterpret_cast<PyTypeObject*>(where)->tp_dict : where;
+  if (!PyDict_Check(dict)) {
+    PyErr_SetString(PyExc_TypeError, "a guard takes a dict or a class");
+    return false;
+  }
+  if (!fill_guard(g, entries)) return false;
+  Py_INCREF(dict);
+  g.dict = dict;
   return true;
 }
 
@@ -461,15 +509,8 @@ PyObject* plan_guard(PyObject* self, PyObject* args) {
   PyObject *where, *entries;
   int wrappers;
   if (!PyArg_ParseTuple(args, "OOp", &where, &entries, &wrappers)) return nullptr;
-  PyObject* dict = PyType_Check(where) ? reinterpret_cast<PyTypeObject*>(where)->tp_dict : where;
-  if (!PyDict_Check(dict)) {
-    PyErr_SetString(PyExc_TypeError, "guard() takes a dict or a class");
-    return nullptr;
-  }
   Guard g;
-  if (!fill_guard(g, entries)) return nullptr;
-  Py_INCREF(dict);
-  g.dict = dict;
+  if (!make_guard(g, where, entries)) return nullptr;
   g.wrappers = wrappers != 0;
   reinterpret_cast<Plan*>(self)->guards->push_back(std::move(g));
   Py_RETURN_NONE;
@@ -481,6 +522,33 @@ PyObject* plan_guard_module(PyObject* self, PyObject* entries) {
   Plan* p = reinterpret_cast<Plan*>(self);
   if (!fill_guard(p->self, entries)) return nullptr;
   p->guarded = true;
+  Py_RETURN_NONE;
+}
+
+// direct(class, {attribute: expected} of the module, ((dict_or_class, {key: expected}), ...), (dict of hooks, ...))
+PyObject* plan_direct(PyObject* self, PyObject* args) {
+  Plan* p = reinterpret_cast<Plan*>(self);
+  PyObject *type, *own, *guards, *hooks;
+  if (p->direct_type || !PyArg_ParseTuple(args, "O!OO!O!", &PyType_Type, &type, &own, &PyTuple_Type, &guards, &PyTuple_Type, &hooks))
+    return nullptr;
+  if (!fill_guard(p->direct_self, own)) return nullptr;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(guards); ++i) {
+    PyObject *where, *entries;
+    Guard g;
+    if (!PyArg_ParseTuple(PyTuple_GET_ITEM(guards, i), "OO", &where, &entries) || !make_guard(g, where, entries)) return nullptr;
+    p->direct_guards->push_back(std::move(g));
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(hooks); ++i) {
+    PyObject* d = PyTuple_GET_ITEM(hooks, i);
+    if (!PyDict_Check(d)) {
+      PyErr_SetString(PyExc_TypeError, "direct(): hooks are dictionaries");
+      return nullptr;
+    }
+    Py_INCREF(d);
+    p->hooks->push_back(d);
+  }
+  Py_INCREF(type);
+  p->direct_type = reinterpret_cast<PyTypeObject*>(type);
   Py_RETURN_NONE;
 }
 
@@ -572,6 +640,7 @@ PyObject* plan_reduce(PyObject*, PyObject*) { return Py_BuildValue("(O())", Py_T
 PyMethodDef plan_methods[] = {
     {"guard", plan_guard, METH_VARARGS, "guard(dict_or_class, {key: expected}, wrappers)"},
     {"guard_module", plan_guard_module, METH_O, "guard_module({attribute: expected})"},
+    {"direct", plan_direct, METH_VARARGS, "direct(class, own, guards, hooks): when module(x) may go straight to the plan"},
     {"source", plan_source, METH_O, "source(tensor or None)"},
     {"hold", plan_hold, METH_O, "hold(object)"},
     {"template", plan_template, METH_VARARGS, "template(kind, n, k, k_in, args, f, out, perm, bias, own, keep) -> number"},
@@ -590,6 +659,63 @@ PyMemberDef plan_members[] = {
 
 PyTypeObject plan_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+// `__call__` of the module classes that have plans: module(x) goes to the plan when torch's call of the module would
+// only find the way to a forward that asks it (two Python frames and the checks in them: 4.7 -> 4.1 us per call),
+// and is torch.nn.Module.__call__ otherwise.
+struct ModuleCall {
+  PyObject_HEAD
+  vectorcallfunc call;
+};
+
+PyTypeObject module_call_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+PyTypeObject* g_module_class = nullptr;  // torch.nn.Module
+PyObject *g_plan_key = nullptr, *g_call_key = nullptr;
+
+PyObject* module_call(PyObject*, PyObject* const* args, size_t nargsf, PyObject* kwnames) {
+  if (PyVectorcall_NARGS(nargsf) == 2 && !kwnames) {
+    PyObject** dict = _PyObject_GetDictPtr(args[0]);
+    PyObject* plan = dict && *dict ? PyDict_GetItemWithError(*dict, g_plan_key) : nullptr;
+    if (plan && Py_TYPE(plan) == &plan_type) {
+      Plan* p = reinterpret_cast<Plan*>(plan);
+      if (p->guarded && p->direct_type && direct(p, args[0]) && !stale(p, args[0]) && !wrapped(p)) {
+        Py_INCREF(plan);  // the module may drop it meanwhile
+        PyObject* y = run(p, args[1]);
+        Py_DECREF(plan);
+        if (y != Py_None) return y;
+        Py_DECREF(y);
+      }
+    } else if (!plan && PyErr_Occurred()) {
+      return nullptr;
+    }
+  }
+  PyObject* call = g_module_class ? PyDict_GetItemWithError(g_module_class->tp_dict, g_call_key) : nullptr;
+  if (!call) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "torch.nn.Module has no __call__");
+    return nullptr;
+  }
+  return PyObject_Vectorcall(call, args, nargsf, kwnames);
+}
+
+PyObject* module_call_get(PyObject* self, PyObject* obj, PyObject*) {
+  if (obj && obj != Py_None) return PyMethod_New(self, obj);
+  Py_INCREF(self);
+  return self;
+}
+
+// set_module_class(torch.nn.Module, call): `call` is what Python code sees as ModuleCall.__call__ -- compilers that trace
+// Python source go through it -- while calls from the interpreter arrive in module_call.
+PyObject* set_module_class(PyObject*, PyObject* args) {
+  PyObject *type, *call;
+  if (!PyArg_ParseTuple(args, "O!O", &PyType_Type, &type, &call) ||
+      PyDict_SetItem(module_call_type.tp_dict, g_call_key, call) < 0)
+    return nullptr;
+  PyType_Modified(&module_call_type);
+  Py_INCREF(type);
+  Py_XDECREF(reinterpret_cast<PyObject*>(g_module_class));
+  g_module_class = reinterpret_cast<PyTypeObject*>(type);
+  Py_RETURN_NONE;
+}
+
 PyObject* set_workspaces(PyObject*, PyObject* args) {
   PyObject *dict, *drop;
   if (!PyArg_ParseTuple(args, "O!O", &PyDict_Type, &dict, &drop)) return nullptr;
@@ -603,6 +729,7 @@ PyObject* set_workspaces(PyObject*, PyObject* args) {
 }
 
 PyMethodDef module_methods[] = {
+    {"set_module_class", set_module_class, METH_VARARGS, "set_module_class(torch.nn.Module, its call in Python)"},
     {"set_workspaces", set_workspaces, METH_VARARGS, "set_workspaces(dict, drop): the slice-list GEMV's scratch buffers"},
     {nullptr, nullptr, 0, nullptr},
 };
@@ -629,5 +756,19 @@ PyMODINIT_FUNC PyInit_npamd_host(void) {
   if (!m) return nullptr;
   Py_INCREF(&plan_type);
   if (PyModule_AddObject(m, "CallPlan", reinterpret_cast<PyObject*>(&plan_type)) < 0) return nullptr;
+  g_plan_key = PyUnicode_InternFromString("_plan");
+  g_call_key = PyUnicode_InternFromString("__call__");
+  module_call_type.tp_name = "npamd_host.ModuleCall";
+  module_call_type.tp_basicsize = sizeof(ModuleCall);
+  module_call_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL | Py_TPFLAGS_METHOD_DESCRIPTOR;
+  module_call_type.tp_doc = "module(x), straight to the module's plan where nothing stands between";
+  module_call_type.tp_call = PyVectorcall_Call;
+  module_call_type.tp_vectorcall_offset = offsetof(ModuleCall, call);
+  module_call_type.tp_descr_get = module_call_get;
+  if (!g_plan_key || !g_call_key || PyType_Ready(&module_call_type) < 0) return nullptr;
+  ModuleCall* call = PyObject_New(ModuleCall, &module_call_type);
+  if (!call) return nullptr;
+  call->call = module_call;
+  if (PyModule_AddObject(m, "module_call", reinterpret_cast<PyObject*>(call)) < 0) return nullptr;
   return m;
 }

@@ -531,8 +531,8 @@ static int launch_q4_rowwise_rw(const Q4RowArgs& a, hipStream_t st, const char* 
   const int rows_per_block = R * W;
   const int blocks = (a.N + rows_per_block - 1) / rows_per_block;
   const int lds = M * a.passes * (4 * 64 * 16 + 64 * 4 * 2);
-  if (a.zp) q4_rowwise_gemv_kernel<ACT, M, R, true, W><<<blocks, W * 64, lds, st>>>(a);
-  else q4_rowwise_gemv_kernel<ACT, M, R, false, W><<<blocks, W * 64, lds, st>>>(a);
+  if (a.zp) launch(q4_rowwise_gemv_kernel<ACT, M, R, true, W>, blocks, W * 64, lds, st, a);
+  else launch(q4_rowwise_gemv_kernel<ACT, M, R, false, W>, blocks, W * 64, lds, st, a);
   return check_launch(what);
 }
 
@@ -604,8 +604,8 @@ static int launch_q4_stream(const QCall& c, const Q4StreamGeom& geo) {
   a.gs_shift = log2i(c.gs / 32);
   const int lds = geo.passes * 128 * kQ4StreamXStride + geo.iterations * geo.row_lanes * geo.passes * 4;
   const dim3 grid(geo.blocks), block(geo.waves * 64);
-  if (a.zp) q4_stream_gemv_kernel<ACT, true><<<grid, block, lds, c.st>>>(a, geo);
-  else q4_stream_gemv_kernel<ACT, false><<<grid, block, lds, c.st>>>(a, geo);
+  if (a.zp) launch(q4_stream_gemv_kernel<ACT, true>, grid, block, lds, c.st, a, geo);
+  else launch(q4_stream_gemv_kernel<ACT, false>, grid, block, lds, c.st, a, geo);
   return check_launch(c.what);
 }
 
@@ -729,11 +729,11 @@ extern "C" int npamd_q_dequant(const uint8_t* w_pack, const void* scale_f16, con
 #define NPAMD_Q4_LAUNCH(OUT)                                                                              \
   do {                                                                                                    \
     if (zero_point_f16)                                                                                   \
-      q4_dequant_kernel<OUT, true><<<grid.blocks, 256, 0, st>>>(                                               \
+      launch(q4_dequant_kernel<OUT, true>, grid.blocks, 256, 0, st,                                                \
           (const uint32_t*)w_pack, (const uint16_t*)scale_f16, (const uint16_t*)zero_point_f16, n_words,  \
           K / 8, K / group_size, group_size / 8, grid.per_die, out);                                                    \
     else                                                                                                  \
-      q4_dequant_kernel<OUT, false><<<grid.blocks, 256, 0, st>>>(                                              \
+      launch(q4_dequant_kernel<OUT, false>, grid.blocks, 256, 0, st,                                               \
           (const uint32_t*)w_pack, (const uint16_t*)scale_f16, nullptr, n_words, K / 8, K / group_size,   \
           group_size / 8, grid.per_die, out);                                                                           \
   } while (0)
@@ -746,7 +746,7 @@ extern "C" int npamd_q_dequant(const uint8_t* w_pack, const void* scale_f16, con
     const int64_t n_octets = total / 8;
     const DieGrid grid((n_octets + 255) / 256, total * (out_dtype == NPAMD_F32 ? 4 : 2));
 #define NPAMD_QN_LAUNCH(NB, OUT)                                                                       \
-  qn_dequant_kernel<NB, OUT><<<grid.blocks, 256, 0, st>>>(w_pack, (const uint16_t*)scale_f16,               \
+  launch(qn_dequant_kernel<NB, OUT>, grid.blocks, 256, 0, st, w_pack, (const uint16_t*)scale_f16,               \
                                                      (const uint16_t*)zero_point_f16, n_octets, K / 8, \
                                                      K / group_size, group_size / 8, grid.per_die, out)
 #define NPAMD_QN_OUT(NB)                                         \
@@ -763,7 +763,7 @@ extern "C" int npamd_q_dequant(const uint8_t* w_pack, const void* scale_f16, con
   } else {
     const unsigned blocks = (unsigned)((total + 255) / 256);
 #define NPAMD_QG_LAUNCH(OUT)                                                                   \
-  q_dequant_generic_kernel<OUT><<<blocks, 256, 0, st>>>(w_pack, (const uint16_t*)scale_f16,    \
+  launch(q_dequant_generic_kernel<OUT>, blocks, 256, 0, st, w_pack, (const uint16_t*)scale_f16,    \
                                                         (const uint16_t*)zero_point_f16, total, \
                                                         K, nbits, group_size, out)
     if (out_dtype == NPAMD_F16) NPAMD_QG_LAUNCH(NPAMD_F16);

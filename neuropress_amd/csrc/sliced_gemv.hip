@@ -401,7 +401,7 @@ int launch_sliced_tokens_p(const SlicedArgs& a, int n_workgroups, hipStream_t st
   const hipError_t e = enable_dynamic_lds(latch, reinterpret_cast<const void*>(&sliced_gemv_kernel<ACT, M, PERM>), kLdsBytes);
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, kLdsBytes, hipGetErrorString(e));
-  sliced_gemv_kernel<ACT, M, PERM><<<n_workgroups, kSlicedTasks, kLdsBytes, st>>>(a);
+  launch(sliced_gemv_kernel<ACT, M, PERM>, n_workgroups, kSlicedTasks, kLdsBytes, st, a);
   return check_launch(what);
 }
 
@@ -472,7 +472,7 @@ int launch_sliced(const npamd_sliced_header& h, const uint8_t* blob, const void*
     if (rc != NPAMD_OK) return rc;
   }
   if (!a.fused_finish)
-    sliced_reduce_kernel<ACT><<<dim3((h.n + 15) / 16, M), 256, 0, st>>>(workspace, h.n_partials, h.n, bias, y, ldy);
+    launch(sliced_reduce_kernel<ACT>, dim3((h.n + 15) / 16, M), 256, 0, st, workspace, h.n_partials, h.n, bias, y, ldy);
   return check_launch(what);
 }
 
@@ -583,7 +583,7 @@ extern "C" int npamd_vq_gemv_sliced_static(const void* x, int64_t ldx, const int
     workspace = scratch_of_device[device];
     if (scratch_suspect[device]) {
       constexpr int n16 = NPAMD_SLICED_STATIC_WORKSPACE_BYTES / 16;
-      scratch_zero_kernel<<<(n16 + 255) / 256, 256, 0, (hipStream_t)stream>>>((u32x4*)workspace, n16);
+      launch(scratch_zero_kernel, (n16 + 255) / 256, 256, 0, (hipStream_t)stream, (u32x4*)workspace, n16);
       const int zrc = check_launch(what);
       if (zrc != NPAMD_OK) return zrc;
       scratch_suspect[device] = false;

@@ -221,7 +221,7 @@ static int launch_vq_dequant(const uint8_t* packed, int64_t n_bytes, int bits, c
     const DieGrid grid((n_vectors + per_block - 1) / per_block, bytes);
     const bool b16 = bits == 16 && (reinterpret_cast<uintptr_t>(packed) % 2) == 0;
 #define NPAMD_VQ_LDS(B, V) \
-  vq_dequant_lds_kernel<B, OUT, V><<<grid.blocks, 1024, lds, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, per_block, grid.per_die)
+  launch(vq_dequant_lds_kernel<B, OUT, V>, grid.blocks, 1024, lds, st, packed, n_bytes, bits, c, nc, out, n_vectors, per_block, grid.per_die)
     if (vl == 8) {
       if (b16) NPAMD_VQ_LDS(16, 8);
       else NPAMD_VQ_LDS(0, 8);
@@ -235,22 +235,22 @@ static int launch_vq_dequant(const uint8_t* packed, int64_t n_bytes, int bits, c
   if (vl == 8 && cb_aligned && out_aligned) {
     const u32x4* c = reinterpret_cast<const u32x4*>(cb);
     if (bits == 16 && (reinterpret_cast<uintptr_t>(packed) % 2) == 0)
-      vq_dequant_vl8_kernel<16, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
+      launch(vq_dequant_vl8_kernel<16, OUT>, grid.blocks, 256, 0, st, packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
     else if (bits == 8)
-      vq_dequant_vl8_kernel<8, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
+      launch(vq_dequant_vl8_kernel<8, OUT>, grid.blocks, 256, 0, st, packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
     else
-      vq_dequant_vl8_kernel<0, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
+      launch(vq_dequant_vl8_kernel<0, OUT>, grid.blocks, 256, 0, st, packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
   } else if (vl == 4 && (reinterpret_cast<uintptr_t>(cb) % 8) == 0 && out_aligned) {
     const u32x2* c = reinterpret_cast<const u32x2*>(cb);
     const DieGrid grid(((n_vectors + 1) / 2 + 255) / 256, bytes);  // two vectors per thread
     if (bits == 16 && (reinterpret_cast<uintptr_t>(packed) % 2) == 0)
-      vq_dequant_vl4_kernel<16, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
+      launch(vq_dequant_vl4_kernel<16, OUT>, grid.blocks, 256, 0, st, packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
     else if (bits == 8)
-      vq_dequant_vl4_kernel<8, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
+      launch(vq_dequant_vl4_kernel<8, OUT>, grid.blocks, 256, 0, st, packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
     else
-      vq_dequant_vl4_kernel<0, OUT><<<grid.blocks, 256, 0, st>>>(packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
+      launch(vq_dequant_vl4_kernel<0, OUT>, grid.blocks, 256, 0, st, packed, n_bytes, bits, c, nc, out, n_vectors, grid.per_die);
   } else {
-    vq_dequant_generic_kernel<OUT><<<blocks, 256, 0, st>>>(
+    launch(vq_dequant_generic_kernel<OUT>, blocks, 256, 0, st,
         packed, n_bytes, bits, reinterpret_cast<const uint16_t*>(cb), nc, out, n_vectors, vl);
   }
   return check_launch("npamd_vq_dequant");
@@ -312,7 +312,7 @@ extern "C" int npamd_vq_widen_u16(const uint8_t* packed, int64_t n_bytes, int bi
   if (n_indices == 0) return NPAMD_OK;
   NPAMD_REQUIRE(packed && out, "npamd_vq_widen_u16: null pointer");
   const unsigned blocks = (unsigned)((n_indices + 255) / 256);
-  vq_widen_u16_kernel<<<blocks, 256, 0, (hipStream_t)stream>>>(packed, n_bytes, bits, n_indices, out);
+  launch(vq_widen_u16_kernel, blocks, 256, 0, (hipStream_t)stream, packed, n_bytes, bits, n_indices, out);
   return check_launch("npamd_vq_widen_u16");
 }
 
@@ -327,7 +327,7 @@ extern "C" int npamd_vq_lut_gather(const float* lut, const uint8_t* packed, int6
   if (M == 0 || N == 0) return NPAMD_OK;
   NPAMD_REQUIRE(lut && packed && y, "%s: null pointer", what);
   const dim3 grid((unsigned)((N + 3) / 4), (unsigned)M);
-  vq_lut_gather_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(lut, packed, n_bytes, bits, y, N, groups, nc);
+  launch(vq_lut_gather_kernel, grid, 256, 0, (hipStream_t)stream, lut, packed, n_bytes, bits, y, N, groups, nc);
   return check_launch(what);
 }
 
@@ -357,7 +357,7 @@ extern "C" int npamd_rvq_dequant(const uint8_t* packed_main, int64_t n_bytes_mai
     const bool m16 = bits_main == 16 && (reinterpret_cast<uintptr_t>(packed_main) % 2) == 0;
     const bool r8 = bits_res == 8;
 #define NPAMD_RVQ8_LAUNCH(BM, BR, OUT)                                                               \
-  rvq_dequant_vl8_kernel<BM, BR, OUT><<<grid, 256, 0, st>>>(                                         \
+  launch(rvq_dequant_vl8_kernel<BM, BR, OUT>, grid, 256, 0, st,                                          \
       packed_main, n_bytes_main, bits_main, packed_res, n_bytes_res, bits_res, (const u32x4*)cb_main_f16, \
       (uint32_t)nc_main, (const u32x4*)cb_res_f16, (uint32_t)nc_res, (const uint16_t*)row_scale_f16,  \
       (const uint16_t*)row_bias_f16, N, (int)groups, rows.per_die, out)
@@ -378,7 +378,7 @@ extern "C" int npamd_rvq_dequant(const uint8_t* packed_main, int64_t n_bytes_mai
     return check_launch("npamd_rvq_dequant");
   }
 #define NPAMD_RVQ_LAUNCH(OUT)                                                                   \
-  rvq_dequant_kernel<OUT><<<blocks, 256, 0, st>>>(                                              \
+  launch(rvq_dequant_kernel<OUT>, blocks, 256, 0, st,                                               \
       packed_main, n_bytes_main, bits_main, packed_res, n_bytes_res, bits_res,                  \
       (const uint16_t*)cb_main_f16, (uint32_t)nc_main, (const uint16_t*)cb_res_f16,             \
       (uint32_t)nc_res, (const uint16_t*)row_scale_f16, \

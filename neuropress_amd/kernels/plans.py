@@ -9,8 +9,11 @@ read, and the wrapper functions of ``kernels`` are what they were; otherwise it 
 from __future__ import annotations
 
 import torch
+import torch.nn.modules.module as nn_module
 
 from .. import _lib
+
+_TORCH_CALL = torch.nn.Module.__call__
 
 (SLICED, VQ_GEMV, VQ_GEMV_PERM, VQ_TILE, VQ_DENSE, RVQ_GEMV, RVQ_TILE, RVQ_DENSE,
  Q_GEMV, Q_TILE, Q_DENSE, RMS_NORM, VQ_EMBEDDING, Q_EMBEDDING) = range(14)  # fmt: skip
@@ -47,7 +50,35 @@ def make(module, attributes, thresholds=None, names=(), holders=(), sources=()):
     plan.guard(kernels.SlicedCallPlan, {"run": kernels.SLICED_RUN}, True)
     for t in sources:
         plan.source(t)
+    _call_directly(plan, module)
     return plan
+
+
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+
+
+def _call_directly(plan, module) -> None:
+    """Let ``module(x)`` go to the plan without ``torch.nn.Module.__call__`` and ``forward`` in between.
+
+    For the classes that declare their ``forward`` to do nothing but ask the plan first (``_planned_forward``), and
+    only while that call would find nothing else to do: no hooks, no compiled call, neither function replaced."""
+    cls, call = type(module), _lib.host().module_call
+    if vars(cls).get("_planned_forward") is None:
+        return
+    if "__call__" not in vars(cls):
+        cls.__call__ = call
+    if vars(cls)["__call__"] is not call:
+        return
+    every = tuple(getattr(nn_module, "_global" + name) for name in _HOOKS)
+    own = {name: module.__dict__.get(name) for name in _HOOKS}
+    if any(hooks is None for hooks in own.values()):
+        return
+    plan.direct(
+        cls,
+        {**own, "forward": ..., "_compiled_call_impl": ...},
+        ((cls, {"forward": cls._planned_forward, "__call__": call}), (torch.nn.Module, {"__call__": _TORCH_CALL})),
+        (*own.values(), *every),
+    )
 
 
 def template(plan, kind, n, k, args, dtype, *, f=0.0, k_in=None, perm=None, bias=None, own=False):

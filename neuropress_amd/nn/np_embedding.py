@@ -165,6 +165,8 @@ class NPEmbedding(nn.Module):
                 return y
         return self._forward(x)
 
+    _planned_forward = forward  # module(x) may go straight to the plan (kernels/plans.py)
+
     def _planned(self, ids: torch.Tensor):
         """Let a plan issue this lookup, whatever the number of ids; None where it cannot."""
         from ..kernels import plans

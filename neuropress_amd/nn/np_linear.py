@@ -300,6 +300,8 @@ class NPLinear(nn.Module):
         # default / compile: the torch-op specification of the layer.
         return self._forward_compile(x)
 
+    _planned_forward = forward  # module(x) may go straight to the plan (kernels/plans.py)
+
     def _forward_compile(self, x: torch.Tensor) -> torch.Tensor:
         return _q_dequant_linear(
             x, self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point,

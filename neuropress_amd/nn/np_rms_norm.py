@@ -45,6 +45,8 @@ class NPRMSNorm(nn.Module):
                 return y
         return self._forward(x)
 
+    _planned_forward = forward  # module(x) may go straight to the plan (kernels/plans.py)
+
     def _planned(self, x: torch.Tensor, w: torch.Tensor):
         """Let a plan issue this norm, whatever the number of rows; None where it cannot."""
         from ..kernels import plans

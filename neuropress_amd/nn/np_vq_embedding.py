@@ -104,6 +104,8 @@ class NPVQEmbedding(nn.Module):
                 return y
         return self._forward(input_ids)
 
+    _planned_forward = forward  # module(x) may go straight to the plan (kernels/plans.py)
+
     def _planned(self, ids: torch.Tensor, perm: torch.Tensor | None):
         """Let a plan issue this lookup, whatever the number of ids; None where it cannot."""
         from ..kernels import plans

@@ -717,6 +717,8 @@ class NPVQLinear(nn.Module):
                 return y
         return self._forward(x)
 
+    _planned_forward = forward  # module(x) may go straight to the plan (kernels/plans.py)
+
     def _forward(self, x: torch.Tensor) -> torch.Tensor:
         m = x.numel() // self.in_features
         band = self._band(x, m)

@@ -103,3 +103,36 @@ def test_planned_norm_and_lookups(gpu):
             first = emb(ids)
             assert first.shape == (*shape, 256) and torch.equal(emb._plan(emb, ids), first)
             assert emb._plan(emb, ids.int()) is None and torch.equal(emb(ids.int()), first)
+
+
+@pytest.mark.parametrize("kind", ["vq8", "q4"])
+def test_module_call_takes_the_long_way_when_something_stands_between(gpu, kind, monkeypatch):
+    """``module(x)`` skips torch's module call only while that would do nothing but call the class's own forward."""
+    layer = _layer(kind, gpu, torch.float16)
+    x = torch.randn(1, layer.in_features, generator=cases.gen(1)).half().to(gpu)
+    first = layer(x)
+    assert torch.equal(layer(x), first) and type(layer).__call__ is not torch.nn.Module.__call__
+    seen = []
+    for register in (layer.register_forward_pre_hook, layer.register_forward_hook,
+                     torch.nn.modules.module.register_module_forward_hook):  # fmt: skip
+        handle = register(lambda *args: seen.append(1))
+        assert torch.equal(layer(x), first) and len(seen) == 1
+        handle.remove()
+        assert torch.equal(layer(x), first) and len(seen) == 1
+        seen.clear()
+    own = layer.forward
+    layer.forward = lambda t: own(t) + 1
+    assert torch.equal(layer(x), first + 1)
+    del layer.forward
+    monkeypatch.setattr(type(layer), "forward", lambda self, t: type(self)._planned_forward(self, t) + 2)
+    assert torch.equal(layer(x), first + 2)
+    monkeypatch.undo()
+    torch_call = torch.nn.Module.__call__
+    monkeypatch.setattr(torch.nn.Module, "__call__", lambda self, *a, **k: seen.append(1) or torch_call(self, *a, **k))
+    assert torch.equal(layer(x), first) and len(seen) == 1
+    monkeypatch.undo()
+    assert torch.equal(layer(x), first) and len(seen) == 1
+    copied = copy.deepcopy(layer)
+    assert torch.equal(copied(x), copied(x))
+    with pytest.raises(TypeError):
+        layer()
