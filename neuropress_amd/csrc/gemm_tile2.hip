@@ -579,11 +579,7 @@ int launch_tile2_mw(const GemmShape& s, const typename Prod::Args& a, const T2Pa
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds, hipGetErrorString(e));
   launch(tile2_gemm_kernel<ACT, MW, Prod>, grid, 512, lds, st, s, a, pair);
-  if (s.splits > 2) {
-    const int64_t quads = (int64_t)s.M * ((s.N + 3) / 4);
-    launch(splitk_reduce_kernel<ACT>, (unsigned)((quads + 255) / 256), 256, 0, st, s.partials, s.splits, s.M, s.N,
-                                                                             s.bias, s.y, s.ldy);
-  }
+  if (s.splits > 2) launch_splitk_reduce<ACT>(s.partials, s.splits, s.M, s.N, s.bias, s.y, s.ldy, st);
   return check_launch(what);
 }
 
