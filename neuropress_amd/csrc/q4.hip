@@ -31,20 +31,28 @@ q_dequant_generic_kernel(const uint8_t* __restrict__ w_pack, const uint16_t* __r
   store_from_f32<OUT>(out, e, d * f16_bits_to_f32(scale[sidx]));
 }
 
+// The group of octet i of a weight: rows are whole numbers of groups, so the rows drop out, and one division is left, a
+// shift where a group is a power of two octets.  (With a 64-bit division by the row's octets in front of it, arithmetic
+// was what small decodes waited for.)
+struct GroupOf {
+  uint32_t octets;
+  int shift;  // -1: not a power of two
+  explicit GroupOf(int octets_) : octets((uint32_t)octets_), shift((octets_ & (octets_ - 1)) == 0 ? __builtin_ctz((unsigned)octets_) : -1) {}
+  __device__ __forceinline__ int64_t operator()(int64_t i) const { return shift >= 0 ? i >> shift : i / octets; }
+};
+
 // Decode, 4-bit (symmetric, or ASYM with per-group zero points): one thread per dword of
 // nibbles = 8 weights, one 16-byte (32-byte for f32) store.  group_size % 8 == 0 so the 8
 // share a scale.
 template <int OUT, bool ASYM>
 __global__ void __launch_bounds__(256)
 q4_dequant_kernel(const uint32_t* __restrict__ w_pack, const uint16_t* __restrict__ scale,
-                  const uint16_t* __restrict__ zero_point, int64_t n_words, int words_per_row,
-                  int groups_per_row, int words_per_group, unsigned per_die, void* __restrict__ out) {
+                  const uint16_t* __restrict__ zero_point, int64_t n_words, GroupOf group, unsigned per_die,
+                  void* __restrict__ out) {
 #pragma clang fp contract(off)
   const int64_t i = die_block(blockIdx.x, per_die) * 256 + threadIdx.x;
   if (i >= n_words) return;
-  const int64_t n = i / words_per_row;
-  const int wr = (int)(i - n * words_per_row);
-  const int64_t sidx = n * groups_per_row + wr / words_per_group;
+  const int64_t sidx = group(i);
   const float sc = f16_bits_to_f32(scale[sidx]);
   const float zp = ASYM ? f16_bits_to_f32(zero_point[sidx]) : 8.0f;
   const uint32_t w = w_pack[i];
@@ -76,14 +84,12 @@ q4_dequant_kernel(const uint32_t* __restrict__ w_pack, const uint16_t* __restric
 template <int NBITS, int OUT>
 __global__ void __launch_bounds__(256)
 qn_dequant_kernel(const uint8_t* __restrict__ w_pack, const uint16_t* __restrict__ scale,
-                  const uint16_t* __restrict__ zero_point, int64_t n_octets, int octets_per_row,
-                  int groups_per_row, int octets_per_group, unsigned per_die, void* __restrict__ out) {
+                  const uint16_t* __restrict__ zero_point, int64_t n_octets, GroupOf group, unsigned per_die,
+                  void* __restrict__ out) {
 #pragma clang fp contract(off)
   const int64_t i = die_block(blockIdx.x, per_die) * 256 + threadIdx.x;
   if (i >= n_octets) return;
-  const int64_t n = i / octets_per_row;
-  const int o = (int)(i - n * octets_per_row);
-  const int64_t sidx = n * groups_per_row + o / octets_per_group;
+  const int64_t sidx = group(i);
   const float sc = f16_bits_to_f32(scale[sidx]);
   const float zp = zero_point ? f16_bits_to_f32(zero_point[sidx]) : (float)(1 << (NBITS - 1));
   uint64_t bits;
@@ -731,11 +737,11 @@ extern "C" int npamd_q_dequant(const uint8_t* w_pack, const void* scale_f16, con
     if (zero_point_f16)                                                                                   \
       launch(q4_dequant_kernel<OUT, true>, grid.blocks, 256, 0, st,                                                \
           (const uint32_t*)w_pack, (const uint16_t*)scale_f16, (const uint16_t*)zero_point_f16, n_words,  \
-          K / 8, K / group_size, group_size / 8, grid.per_die, out);                                                    \
+          GroupOf(group_size / 8), grid.per_die, out);                                                    \
     else                                                                                                  \
       launch(q4_dequant_kernel<OUT, false>, grid.blocks, 256, 0, st,                                               \
-          (const uint32_t*)w_pack, (const uint16_t*)scale_f16, nullptr, n_words, K / 8, K / group_size,   \
-          group_size / 8, grid.per_die, out);                                                                           \
+          (const uint32_t*)w_pack, (const uint16_t*)scale_f16, nullptr, n_words,                          \
+          GroupOf(group_size / 8), grid.per_die, out);                                                                          \
   } while (0)
     if (out_dtype == NPAMD_F16) NPAMD_Q4_LAUNCH(NPAMD_F16);
     else if (out_dtype == NPAMD_BF16) NPAMD_Q4_LAUNCH(NPAMD_BF16);
@@ -747,8 +753,8 @@ extern "C" int npamd_q_dequant(const uint8_t* w_pack, const void* scale_f16, con
     const DieGrid grid((n_octets + 255) / 256, total * (out_dtype == NPAMD_F32 ? 4 : 2));
 #define NPAMD_QN_LAUNCH(NB, OUT)                                                                       \
   launch(qn_dequant_kernel<NB, OUT>, grid.blocks, 256, 0, st, w_pack, (const uint16_t*)scale_f16,               \
-                                                     (const uint16_t*)zero_point_f16, n_octets, K / 8, \
-                                                     K / group_size, group_size / 8, grid.per_die, out)
+                                                     (const uint16_t*)zero_point_f16, n_octets,        \
+                                                     GroupOf(group_size / 8), grid.per_die, out)
 #define NPAMD_QN_OUT(NB)                                         \
   do {                                                           \
     if (out_dtype == NPAMD_F16) NPAMD_QN_LAUNCH(NB, NPAMD_F16);  \
