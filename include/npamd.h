@@ -404,9 +404,13 @@ int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* 
  * Dense product of the decode + GEMM band: y[m, n] = sum_k x[m, k] w[n, k] (+ bias[n]), f32 accumulate, on a weight a
  * *_dequant entry point has written (the reference calls F.linear there, neuropress/nn/np_vq_linear.py:1148).
  * x, w, y: act_dtype (NPAMD_F16 or NPAMD_BF16); K a multiple of 64; x and w 16-byte aligned, ldx and ldw multiples of 8.
+ * workspace: optional, npamd_dense_gemm_workspace_bytes of them, contents irrelevant; with less, K is not split over blocks.
  */
 int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
-                     int M, int N, int K, int act_dtype, void* stream);
+                     int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Bytes of workspace npamd_dense_gemm can use for this shape (0: none).  Host-only arithmetic. */
+int64_t npamd_dense_gemm_workspace_bytes(int M, int N, int K);
 
 /* 1 where npamd_dense_gemm is the better choice for this shape against a library GEMM.  Host-only arithmetic. */
 int npamd_dense_gemm_preferred(int M, int N, int K);

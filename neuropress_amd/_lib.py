@@ -59,7 +59,8 @@ SIGNATURES: dict[str, list] = {
     "npamd_vq_embedding": [_vp, _i64, _vp, _i64, _int, _vp, _int, _int, _vp, ctypes.c_float, _vp, _int, _vp],
     "npamd_q_embedding": [_vp, _i64, _vp, _vp, _vp, _int, _int, _i64, _int, _i64, ctypes.c_float, _vp, _int, _vp],
     "npamd_q_gemm_tile": _Q_LINEAR[:-1] + _WS + [_vp],
-    "npamd_dense_gemm": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _int, _int, _int, _int, _vp],
+    "npamd_dense_gemm": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _int, _int, _int, _int, _vp, _i64, _vp],
+    "npamd_dense_gemm_workspace_bytes": [_int, _int, _int],
     "npamd_dense_gemm_preferred": [_int, _int, _int],
     "npamd_gather_columns": [_vp, _i64, _vp, _vp, _i64, _int, _int, _vp],
     "npamd_diag_reload_tuning": [],
@@ -69,7 +70,7 @@ SIGNATURES: dict[str, list] = {
     "npamd_diag_mfma": [_vp, _int, _int, _int, _vp, _vp],
 }
 
-_RESTYPES = {"npamd_vq_sliced_workspace_bytes": _i64, "npamd_gemm_tile_workspace_bytes": _i64,
+_RESTYPES = {"npamd_vq_sliced_workspace_bytes": _i64, "npamd_gemm_tile_workspace_bytes": _i64, "npamd_dense_gemm_workspace_bytes": _i64,
              "npamd_diag_reload_tuning": None}
 SLICED_HEADER_BYTES = 128
 SLICED_STATIC_WORKSPACE_BYTES = 4 * 1024 * 1024

@@ -67,6 +67,7 @@ static Tuning read_tuning() {
   t.q4_rowwise_bf16 = env_int("NPAMD_Q4_ROWWISE_BF16", 0);
   t.q4_stream = env_int("NPAMD_Q4_STREAM", 1);
   t.dense_tile = env_int("NPAMD_DENSE_TILE", 0);
+  t.dense_splits = env_int("NPAMD_DENSE_SPLITS", 0);
   return t;
 }
 

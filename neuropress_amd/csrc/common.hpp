@@ -56,6 +56,7 @@ struct Tuning {
   int gemv_lds_cb, tile_lds_cb, gemv_lds_x, gemv_r, gemv_spw, gemv_parts, gemv_xstage, tile_splits, tile_mw, tile_wide;
   int q4_rows, q4_rowwise, q4_rowwise_bf16, q4_stream;
   int dense_tile;  // NPAMD_DENSE_TILE: 1 .. forces a tile of the dense product (wherever it applies), -1 switches it off
+  int dense_splits;  // NPAMD_DENSE_SPLITS: parts of K of the dense product, as far as its limits allow (0: planned)
 };
 const Tuning& tuning();
 

@@ -7,6 +7,11 @@
 // (group g takes every KG-th 64-k step): a small tile then has 8 waves and up to 128 KiB of operands on their way,
 // and the groups' sums meet in LDS, in group order, without a second kernel or a workspace.
 //
+// Long reductions over few output tiles (47 tokens on 384 x 8320: 12 tiles of 32 x 64) leave most of the chip idle
+// all the same, here as in the library.  There K is split over blocks too (`splits` parts of equal length, give or take
+// a step): every block stores its f32 tile to the workspace and splitk_reduce_kernel adds the parts in their order.
+// The parts of a column tile stay on the die that decoded its rows.
+//
 // Both operand tiles are loaded straight into LDS (global_load_lds_dwordx4; rows of 128 bytes, 16-byte piece p of
 // row r in slot p ^ ((r >> 1) & 7), so that a read of 32 consecutive rows touches every bank group twice), a ring of
 // kStages steps per group; one in-order counter tracks a wave's loads and the waits are written by hand.  A wave
@@ -42,7 +47,8 @@ struct DenseShape {
   void* y;
   int64_t ldx, ldw, ldy;
   int M, N, steps;   // steps = K / 64
-  int row_tiles, col_tiles, tiles_per_die;
+  int row_tiles, col_tiles, splits, units_per_die;  // unit: a part of K of one tile
+  float* partials;   // splits > 1: [splits][M][N]
 };
 
 template <int WGM, int WGN, int MT, int KG, int STAGES>
@@ -69,10 +75,12 @@ __global__ void __launch_bounds__((DenseTile<WGM, WGN, MT, KG, STAGES>::kThreads
 dense_gemm_kernel(const DenseShape s) {
   using T = DenseTile<WGM, WGN, MT, KG, STAGES>;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  // blockIdx.x % 8 names the die; a die takes an eighth of the tiles, counted down the columns
-  const int tile = (blockIdx.x & 7) * s.tiles_per_die + (blockIdx.x >> 3);
-  const int ct = tile / s.row_tiles, rt = tile % s.row_tiles;
+  // blockIdx.x % 8 names the die; a die takes an eighth of the units, counted down the columns
+  const int unit = (blockIdx.x & 7) * s.units_per_die + (blockIdx.x >> 3);
+  const int rt = unit % s.row_tiles, part = unit / s.row_tiles % s.splits, ct = unit / s.row_tiles / s.splits;
   if (ct >= s.col_tiles) return;
+  const int step0 = (int)((int64_t)s.steps * part / s.splits);
+  const int steps = (int)((int64_t)s.steps * (part + 1) / s.splits) - step0;  // of this part
   const int m0 = rt * T::kBM, n0 = ct * T::kBN;
 
   const int lane = threadIdx.x & 63;
@@ -81,10 +89,10 @@ dense_gemm_kernel(const DenseShape s) {
   const int wm = wave % WGM, wn = wave / WGM;
   const int c = lane & 31, h = lane >> 5;
 
-  const int steps_g = (s.steps - g + KG - 1) / KG;  // this group's steps: g, g + KG, ...
-  const int base = s.steps / KG;                    // steps every group has
-  const uint8_t* const xb = reinterpret_cast<const uint8_t*>(s.x) + (int64_t)m0 * s.ldx * 2;
-  const uint8_t* const wb = reinterpret_cast<const uint8_t*>(s.w) + (int64_t)n0 * s.ldw * 2;
+  const int steps_g = (steps - g + KG - 1) / KG;  // this group's steps: g, g + KG, ... of the part
+  const int base = steps / KG;                    // steps every group has
+  const uint8_t* const xb = reinterpret_cast<const uint8_t*>(s.x) + (int64_t)m0 * s.ldx * 2 + (int64_t)step0 * 128;
+  const uint8_t* const wb = reinterpret_cast<const uint8_t*>(s.w) + (int64_t)n0 * s.ldw * 2 + (int64_t)step0 * 128;
   uint32_t voff[T::kLoadsX + T::kLoadsW];
 #pragma unroll
   for (int i = 0; i < T::kLoadsX + T::kLoadsW; ++i) {
@@ -189,7 +197,7 @@ dense_gemm_kernel(const DenseShape s) {
     compute(std::false_type{}, slot, 0);
     next_slot();
   }
-  if (KG > 1 && s.steps % KG) {
+  if (KG > 1 && steps % KG) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     block_sync_lds();
     if (base < steps_g) compute(std::false_type{}, slot, 0);
@@ -226,6 +234,23 @@ dense_gemm_kernel(const DenseShape s) {
           }
     }
   }
+  if (s.splits > 1) {
+    // D[m = 8 (i / 4) + 4 h + i % 4][n = c] of each 32 x 32 tile
+    float* const mine = s.partials + (size_t)part * s.M * s.N;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int n = n0 + wn * 64 + t * 32 + c;
+      if (n >= s.N) continue;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int m = m0 + wm * 32 * MT + mt * 32 + 8 * (i / 4) + 4 * h + (i % 4);
+          if (m < s.M) mine[(size_t)m * s.N + n] = acc[mt][t][i];
+        }
+    }
+    return;
+  }
   store_wave_tile<ACT, MT, 2>(acc, lds + T::kRedBytes + wave * (32 * MT * 128), lane, s.y, s.ldy, m0 + wm * 32 * MT, n0 + wn * 64,
                               s.M, s.N, s.bias);
 }
@@ -235,14 +260,15 @@ int launch_dense_tile(DenseShape s, hipStream_t st) {
   using T = DenseTile<WGM, WGN, MT, KG, STAGES>;
   s.row_tiles = (s.M + T::kBM - 1) / T::kBM;
   s.col_tiles = (s.N + T::kBN - 1) / T::kBN;
-  const int64_t tiles = (int64_t)s.col_tiles * s.row_tiles, blocks = (tiles + 7) / 8 * 8;
-  s.tiles_per_die = (int)(blocks / 8);
+  const int64_t units = (int64_t)s.col_tiles * s.row_tiles * s.splits, blocks = (units + 7) / 8 * 8;
+  s.units_per_die = (int)(blocks / 8);
   if (blocks > 0x7FFFFFFF) return fail(NPAMD_ERR_UNSUPPORTED, "npamd_dense_gemm: too many tiles");
   static LdsLatch latch;
   const hipError_t e = enable_dynamic_lds(latch, reinterpret_cast<const void*>(&dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES>), T::kLds);
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "npamd_dense_gemm: cannot reserve %d bytes of LDS: %s", T::kLds, hipGetErrorString(e));
   launch(dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES>, (unsigned)blocks, T::kThreads, T::kLds, st, s);
+  if (s.splits > 1) launch_splitk_reduce<ACT>(s.partials, s.splits, s.M, s.N, s.bias, s.y, s.ldy, st);
   return check_launch("npamd_dense_gemm");
 }
 
@@ -277,22 +303,37 @@ int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
   }
 }
 
-// The tile of least estimate, and the estimate.
-int plan_dense_tile(int M, int N, int K, float* us) {
-  int best = 0;
-  float best_us = 1e30f;
+constexpr int kDenseMaxSplits = 16;
+constexpr int kDenseMinSplitSteps = 4;  // 64-k steps of a part
+// What a split adds: the reduction kernel and the gap in front of it, and its bytes, us and us per MB.
+constexpr float kSplitFixed = 4.5f, kSplitPerMb = 0.45f;
+
+struct DensePlan {
+  int tile, splits;
+  float us;
+};
+
+// The tile and split of least estimate.
+DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits) {
+  DensePlan best{0, 1, 1e30f};
+  const int steps = K / 64;
+  const int forced = tuning().dense_splits, most = max_splits < steps ? max_splits : steps;
+  const int forced_splits = forced < most ? forced : most;
   for (int i = 0; i < kDenseTiles; ++i) {
+    if (forced_tile > 0 && forced_tile <= kDenseTiles && i != forced_tile - 1) continue;
     const DenseCost& c = kDenseCost[i];
     const double tiles = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-    const double rounds = ceil(ceil(tiles / 8) / 32), steps = K / 64;
-    const double walk = rounds * ceil(steps / c.groups) * c.per_step, load = tiles * steps * (c.bm + c.bn) * 128e-6 * c.per_mb;
-    const float t = (float)(c.fixed + rounds * c.per_round + sqrt(walk * walk + load * load));
-    if (t < best_us) {
-      best_us = t;
-      best = i;
+    const double load = tiles * steps * (c.bm + c.bn) * 128e-6 * c.per_mb;
+    for (int splits = 1; splits <= max_splits; ++splits) {
+      if (forced_splits > 0 && splits != forced_splits) continue;
+      if (forced_splits <= 0 && splits > 1 && (steps / splits < kDenseMinSplitSteps || tiles * splits > 512)) break;
+      const double rounds = ceil(ceil(tiles * splits / 8) / 32);
+      const double walk = rounds * ceil(ceil((double)steps / splits) / c.groups) * c.per_step;
+      float t = (float)(c.fixed + rounds * c.per_round + sqrt(walk * walk + load * load));
+      if (splits > 1) t += kSplitFixed + kSplitPerMb * (float)(1e-6 * splits * M * N * 4);
+      if (t < best.us) best = {i, splits, t};
     }
   }
-  if (us) *us = best_us;
   return best;
 }
 
@@ -301,8 +342,14 @@ int plan_dense_tile(int M, int N, int K, float* us) {
 
 using namespace npamd;
 
+extern "C" int64_t npamd_dense_gemm_workspace_bytes(int M, int N, int K) {
+  if (M < 1 || N < 1 || K < 64) return 0;
+  const DensePlan p = plan_dense(M, N, K, tuning().dense_tile, kDenseMaxSplits);
+  return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
+}
+
 extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
-                                int M, int N, int K, int act_dtype, void* stream) {
+                                int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
   const char* what = "npamd_dense_gemm";
   NPAMD_REQUIRE(act_dtype == NPAMD_F16 || act_dtype == NPAMD_BF16, "%s: f16 or bf16 only", what);
   NPAMD_REQUIRE(M >= 0 && N >= 0 && K >= 64 && K % 64 == 0, "%s: bad shape M=%d N=%d K=%d (K has to be a multiple of 64)", what, M, N, K);
@@ -310,27 +357,34 @@ extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64
   if (M == 0 || N == 0) return NPAMD_OK;
   NPAMD_REQUIRE(x && w && y && (((uintptr_t)x | (uintptr_t)w) & 15) == 0, "%s: null or unaligned pointer", what);
   NPAMD_REQUIRE(ldx < (1 << 22) && ldw < (1 << 22), "%s: row stride too large", what);
-  const DenseShape s{x, w, bias, y, ldx, ldw, ldy, M, N, K / 64, 0, 0, 0};
   hipStream_t st = (hipStream_t)stream;
-  const int forced = tuning().dense_tile;
-  const int tile = forced > 0 && forced <= kDenseTiles ? forced - 1 : plan_dense_tile(M, N, K, nullptr);
+  const int64_t room = workspace && ((uintptr_t)workspace & 3) == 0 ? workspace_bytes / ((int64_t)M * N * 4) : 1;
+  DensePlan p = plan_dense(M, N, K, tuning().dense_tile, kDenseMaxSplits);
+  if (p.splits > room) p = plan_dense(M, N, K, tuning().dense_tile, 1);  // too little workspace: unsplit
+  const DenseShape s{x, w, bias, y, ldx, ldw, ldy, M, N, K / 64, 0, 0, p.splits, 0, (float*)workspace};
+  const int tile = p.tile;
   return act_dtype == NPAMD_BF16 ? launch_dense<NPAMD_BF16>(s, tile, st) : launch_dense<NPAMD_F16>(s, tile, st);
 }
 
 // Where this kernel is the better one against the library's product: its estimate against what the library reaches
-// (5 us + 0.85 PFLOP/s; 1.3 once 256 x 256 tiles cover 180 compute units; this kernel's estimates are some 15 % high
-// there) -- or against 16 us, which is what issuing a library product costs the host, so that below it no eager call
-// gains from a faster kernel.  Measured, library / this kernel, us: 171 x 256 x 640
-// 14.6 / 4.8, 77 x 3003 x 2240 13.4 / 8.8, 100 x 14336 x 512 9.7 / 6.7, 384 x 4096 x 4096 23.0 / 20.3, 250 x 11008 x 2048
-// 21.5 / 17.3, 2500 x 3000 x 1024 26.2 / 20.3, 1024 x 4096 x 4096 37.2 / 34.5; but 384 x 14336 x 4096 55.5 / 58.1,
-// 700 x 6000 x 6016 56.8 / 64.8, 4096^3 93 / 124: products of more than 40 GFLOP go to the library.
+// (5 us + 0.85 PFLOP/s; 1.3 once 256 x 256 tiles cover 180 compute units; 1.5 us more per 1024 of K past 4096, which it
+// walks in few tiles) -- or against 25 us: a library product takes 18.3-19 us per eager call whatever its size and
+// 33 us go by between two calls of decode + library product, whatever the GPU does meanwhile (2048 x 4096 with int4 weights,
+// 600 tokens: 35.8 us per call; with this kernel 25).
+// This kernel's estimates are some 15 % high at the larger shapes.  Measured, library / this kernel, us:
+// 171 x 256 x 640 14.6 / 4.8, 77 x 3003 x 2240 13.4 / 8.8, 100 x 14336 x 512 9.7 / 6.7,
+// 384 x 4096 x 4096 23.0 / 20.3, 250 x 11008 x 2048 21.5 / 17.3, 2500 x 3000 x 1024 26.2 / 20.3, 1024 x 4096 x 4096
+// 37.2 / 34.5; but 384 x 14336 x 4096 55.5 / 58.1, 700 x 6000 x 6016 56.8 / 64.8, 4096^3 93 / 124: products of more than
+// 40 GFLOP go to the library.  Long K, split over blocks: 47 x 384 x 8320 19.0 / 8.8 (16.3 unsplit), 945 x 512 x 14336
+// 38.4 / 26.2, 230 x 3152 x 7296 27.3 / 22.2, 460 x 2432 x 7936 36.1 / 29.4, 460 x 4096 x 14336 (54 GFLOP) 72 / 60, but
+// 945 x 4096 x 14336 110 / 108: from K = 8192 the line is 60 GFLOP.
 extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {
   if (M < 1 || N < 1 || K < 64 || K % 64) return 0;
   const int forced = tuning().dense_tile;
   if (forced) return forced > 0;
   const double gflop = 2e-9 * M * N * K;
-  float us = 0.f;
-  plan_dense_tile(M, N, K, &us);
+  const float us = plan_dense(M, N, K, 0, kDenseMaxSplits).us;
   const double big_tiles = ceil(M / 256.0) * ceil(N / 256.0), rate = big_tiles >= 180 ? 1.3 : 0.85;
-  return gflop <= 40.0 && us <= fmax(16.0, 1.15 * (5.0 + gflop / rate)) ? 1 : 0;
+  const double library = 5.0 + gflop / rate + fmax(0.0, (K - 4096) / 1024.0) * 1.5;
+  return gflop <= (K >= 8192 ? 60.0 : 40.0) && us <= fmax(25.0, 1.15 * library) ? 1 : 0;
 }

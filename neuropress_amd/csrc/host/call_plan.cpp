@@ -210,9 +210,11 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
                            w.data_ptr(), code, st);
     if (rc != NPAMD_OK) return false;
     if (t.own) {
+      at::Tensor parts;
+      if (r.ws > 0) parts = empty({r.ws / 4}, at::kFloat, device);
       at::Tensor y = empty(sizes, t.out, device);
       if (npamd_dense_gemm(x.const_data_ptr(), ldx, w.data_ptr(), t.k, t.bias.defined() ? t.bias.const_data_ptr<float>() : nullptr,
-                           y.data_ptr(), t.n, (int)m, (int)t.n, (int)t.k, code, st) != NPAMD_OK)
+                           y.data_ptr(), t.n, (int)m, (int)t.n, (int)t.k, code, r.ws > 0 ? parts.data_ptr() : nullptr, r.ws, st) != NPAMD_OK)
         return false;
       *out = std::move(y);
       return true;

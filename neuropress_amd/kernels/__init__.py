@@ -867,8 +867,10 @@ def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = N
     w = w.contiguous()
     y = torch.empty((m, n), device=x.device, dtype=x.dtype)
     b32 = _bias_f32(bias)
+    need = _lib.load().npamd_dense_gemm_workspace_bytes(m, n, k)
+    ws = torch.empty(need // 4, device=x.device, dtype=torch.float32) if need > 0 else None
     _lib.call("npamd_dense_gemm", x.data_ptr(), x.stride(0), w.data_ptr(), k, _ptr(b32), y.data_ptr(), n, m, n, k,
-              _DT[x.dtype], _stream(x))  # fmt: skip
+              _DT[x.dtype], _ptr(ws), need, _stream(x))  # fmt: skip
     return y
 
 

@@ -93,3 +93,8 @@ def template(plan, kind, n, k, args, dtype, *, f=0.0, k_in=None, perm=None, bias
 def tile_scratch(m: int, n: int, k: int) -> int:
     """Bytes of scratch a tile GEMM of this shape can use."""
     return max(0, int(_lib.load().npamd_gemm_tile_workspace_bytes(m, n, k))) // 4 * 4
+
+
+def product_scratch(m: int, n: int, k: int) -> int:
+    """Bytes of scratch the package's own dense product of this shape can use, next to the decoded weight."""
+    return int(_lib.load().npamd_dense_gemm_workspace_bytes(m, n, k))

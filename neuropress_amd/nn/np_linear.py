@@ -421,7 +421,8 @@ class NPLinear(nn.Module):
             args = (self.u8_blob, self.scale, self.zero_point, self._bias_f32(), 0, 0, self.nbits, self.group_size, code)
             bias = self._bias_as(x.dtype) if band == "dense" else self._bias_f32() if band == "product" else None
             number = plan.names[band, x.dtype] = plans.template(plan, kind, n, k, args, x.dtype, bias=bias, own=band == "product")
-        plan.route(code, m, number, plans.tile_scratch(m, n, k) if band == "tile" else 0)
+        scratch = {"tile": plans.tile_scratch, "product": plans.product_scratch}.get(band)
+        plan.route(code, m, number, scratch(m, n, k) if scratch else 0)
         self._plan = plan
         return None if plan.wrapped() else plan.run(x)
 

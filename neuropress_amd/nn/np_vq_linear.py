@@ -820,7 +820,8 @@ class NPVQLinear(nn.Module):
             for tokens in range(1, min(limit, _SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)) + 1):
                 plan.route(code, tokens, number, sl.workspace_bytes(tokens))
         else:
-            plan.route(code, m, number, plans.tile_scratch(m, self.out_features, self._kernel_k()) if tile else 0)
+            scratch = plans.tile_scratch if tile else plans.product_scratch if kind == "product" else None
+            plan.route(code, m, number, scratch(m, self.out_features, self._kernel_k()) if scratch else 0)
 
     def _template(self, plan, dtype: torch.dtype, kind: str) -> int:
         from ..kernels import plans

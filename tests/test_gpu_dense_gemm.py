@@ -45,6 +45,27 @@ def test_dense_gemm_tiles(gpu, dense_tile, tile, act):
     assert torch.equal(kernels.dense_linear(xs, w), kernels.dense_linear(xs.contiguous(), w))
 
 
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tile,splits", [(1, 2), (1, 16), (2, 9), (3, 3), (4, 8), (5, 7), (6, 2)])
+def test_dense_gemm_parts_of_k(gpu, dense_tile, monkeypatch, tile, splits, act):
+    """K in parts over blocks: parts of unequal length, of fewer steps than a ring is deep or a block has groups of
+    waves, columns the reduction reads four at a time and not."""
+    from neuropress_amd import _lib, kernels
+
+    monkeypatch.setenv("NPAMD_DENSE_SPLITS", str(splits))
+    dense_tile(tile)
+    for m, n, k in ((1, 1, 128), (33, 65, 576), (65, 130, 1088), (129, 260, 1600), (70, 257, 2112)):
+        assert _lib.load().npamd_dense_gemm_workspace_bytes(m, n, k) == min(splits, k // 64) * m * n * 4
+        g = cases.gen(m + n + k)
+        x = torch.randn(m, k, generator=g).to(act)
+        w = (torch.randn(n, k, generator=g) * 0.05).to(act)
+        bias = torch.randn(n, generator=g)
+        y = kernels.dense_linear(x.to(gpu), w.to(gpu), bias.to(gpu)).float().cpu()
+        ref = x.double() @ w.double().T + bias.double()
+        tol = 2.0 ** (-10 if act == torch.float16 else -7)  # the rounding of the output, and f32 sums
+        assert bool(((y - ref).abs() <= tol * ref.abs() + 1e-4).all()), (tile, splits, m, n, k, float((y - ref).abs().max()))
+
+
 def test_dense_gemm_refuses_what_it_does_not_take(gpu):
     from neuropress_amd import kernels
 
