@@ -138,8 +138,11 @@ def tensor_version(t) -> int:
 
 
 # Layers of fewer weights than this decode in 4-8 us, and the dense product that follows is the faster kernel: they
-# leave the tile GEMM earlier (tile_band_ok).  Long reductions of fewer weights than the second leave it past 256 tokens.
+# leave the tile GEMM earlier (tile_band_ok).  Long reductions of fewer weights than the last leave it past 256 tokens, and
+# so do those of at least _MID_LAYER_K features on layers of at least the second.
 _SMALL_LAYER_WEIGHTS: int = 8_000_000
+_MID_LAYER_WEIGHTS: int = 12_000_000
+_MID_LAYER_K: int = 6144
 _LARGE_LAYER_WEIGHTS: int = 1 << 25
 
 
@@ -154,7 +157,9 @@ def tile_band_ok(
 
     Measured, us, tile GEMM / decode + dense product: 3008 x 2240 with a 4096-row codebook 13.7 / 14.1 at 33 tokens,
     14.4 / 14.2 at 64, 17.5 / 15.2 at 128, with int4 weights 15.8 / 13.1 at 33; 6144 x 1024 int4 13.9 / 10.9 at 33;
-    2048 x 8192 int4 29.6 / 30.2 at 256, 39.3 / 35.4 at 384; 4096 x 14336 int4 68 / 104 at 384."""
+    2048 x 8192 int4 29.6 / 30.2 at 256, 39.3 / 35.4 at 384; 4096 x 14336 int4 68 / 104 at 384.  At 230 tokens: 2432 x 7936
+    int4 29.0 / 31.2, with a 256-row codebook 25.1 / 35.8, residual VQ 31.9 / 40.1; 4096 x 6144 30.5 / 34.3, 28.2 / 34.2,
+    35.9 / 40.7; 4096 x 4096 26.1 / 24.6, 26.7 / 25, 28.8 / 28.6."""
     blocks = -(-n // 64) * -(-m // 384)
     if blocks >= min_fraction * cus:
         return True
@@ -163,4 +168,6 @@ def tile_band_ok(
         return False
     if n * k < _SMALL_LAYER_WEIGHTS and m > small_max_tokens:
         return False
-    return m <= split_max_tokens or (k >= long_k and (n * k >= _LARGE_LAYER_WEIGHTS or m <= 256))
+    if m <= split_max_tokens or (k >= _MID_LAYER_K and n * k >= _MID_LAYER_WEIGHTS and m <= 256):
+        return True
+    return k >= long_k and (n * k >= _LARGE_LAYER_WEIGHTS or m <= 256)

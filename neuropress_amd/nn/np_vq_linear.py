@@ -45,7 +45,9 @@ from ..transforms.vq_packing import (
     TieredIndexPacking,
     ZeroEscapePacking,
 )
-from .backends import Backend, VQBackend, is_hip_backend_available, tensor_version, tile_band_ok
+from .backends import (
+    _MID_LAYER_K, _MID_LAYER_WEIGHTS, _SMALL_LAYER_WEIGHTS, Backend, VQBackend, is_hip_backend_available, tensor_version, tile_band_ok,
+)  # fmt: skip
 
 log = logging.getLogger(__name__)
 
@@ -117,18 +119,18 @@ _TILE_MAX_TOKENS: int = _env_int(
 
 # Layers whose codebook LDS does not hold (more than 4096 rows of eight) run the 128-column tile GEMM,
 # which splits the reduction by itself and stays ahead of decode + GEMM up to a token count that goes
-# with the layer's weights (us at 64 / 128 / 256 / 384 tokens, tile against decode + GEMM): 14336 x 4096
-# 42 / 46 / 59 / 70 against 58 / 65 / 75 / 87, 4096 x 14336 44 / 50 / 63 / 80 against 68 / 70 / 85 / 103;
-# 4096 x 4096 23 / 28 / 34 / 42 against 26 / 26 / 30 / 35, 8192 x 2048 22 / 29 / 35 / 46 against 23 / 25 / 30 / 33,
-# 2048 x 8192 27 / 28 / 35 / 44 against 32 / 32 / 33 / 38; 3008 x 2240 15 / 19 / 26 / 31 against 15 / 16 / 18 / 21;
-# 1024 x 4096 15 / 19 / 24 / 28 against 15 / 16 / 17 / 18, 2048 x 2048 13 / 15 / 22 / 28 against 12 / 12 / 13 / 15.
+# with the layer's weights and with K (us at 96 / 144 / 230 / 384 tokens, tile against decode + dense product):
+# 4096 x 14336 44 / 50 / 57 / 73 against 66 / 81 / 78 / 97; 3152 x 7296 26 / 31 / 36 / 47 against 45 / 42 / 46 / 53,
+# 2048 x 10752 24 / 30 / 34 / 43 against 33 / 35 / 38 / 46; 1024 x 8192 16 / 21 / 23 / 29 against 20 / 22 / 24 / 27;
+# 4096 x 4096 24 / 27 / 29 / 37 against 27 / 26 / 30 / 35, 2048 x 4096 16 / 21 / 23 / 28 against 19 / 20 / 22 / 24; and at
+# 64 / 128 / 256 tokens 8192 x 2048 22 / 29 / 35 against 23 / 25 / 30, 3008 x 2240 15 / 19 / 26 against 15 / 16 / 18,
+# 1024 x 4096 15 / 19 / 24 against 15 / 16 / 17, 2048 x 2048 13 / 15 / 22 against 12 / 12 / 13.
 _TILE_WIDE_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_TILE_WIDE_MAX_TOKENS",), 384)
-_TILE_WIDE_MIN_WEIGHTS: int = 1 << 25  # below: 80 tokens, on long reductions 160
-_TILE_WIDE_SMALL_WEIGHTS: int = 1 << 24  # below: 64 tokens
+_TILE_WIDE_MIN_WEIGHTS: int = 1 << 25  # below: 384 tokens only with _MID_LAYER_K features on _MID_LAYER_WEIGHTS
 _TILE_WIDE_TINY_WEIGHTS: int = 5_000_000  # below: 32 tokens, where the GEMV ends
-_TILE_WIDE_MID_MAX_TOKENS: int = 80
-_TILE_WIDE_LONG_MAX_TOKENS: int = 160
-_TILE_WIDE_SMALL_MAX_TOKENS: int = 64
+_TILE_WIDE_LONG_MAX_TOKENS: int = 256  # _SMALL_LAYER_WEIGHTS and K of _TILE_SPLIT_LONG_K
+_TILE_WIDE_MID_MAX_TOKENS: int = 128  # _SMALL_LAYER_WEIGHTS and K of 4096
+_TILE_WIDE_SMALL_MAX_TOKENS: int = 64  # all others
 
 # The tile GEMM gives each workgroup 64 output columns (and up to 384 rows).  When
 # that grid covers less than this fraction of the compute units the kernel splits
@@ -171,7 +173,7 @@ _PLAN_ATTRIBUTES = ("backend", "proxy", "residual_proxy", "out_features", "in_fe
                     "bias", "column_perm", "packed_residual", "row_scale", "row_bias")  # fmt: skip
 _PLAN_THRESHOLDS = ("_FUSED_MAX_TOKENS", "_FUSED_WIDE_MAX_TOKENS", "_FUSED_WIDE_MAX_ACTIVATIONS", "_SLICED_MAX_TOKENS",
                     "_SLICED_MIN_CENTROIDS", "_SLICED_MIN_INDICES", "_LUT_MAX_TOKENS", "_TILE_MAX_TOKENS", "_TILE_WIDE_MAX_TOKENS",
-                    "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_SMALL_WEIGHTS", "_TILE_WIDE_TINY_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS",
+                    "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_TINY_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS",
                     "_TILE_WIDE_LONG_MAX_TOKENS", "_TILE_WIDE_SMALL_MAX_TOKENS", "_TILE_SMALL_LAYER_MAX_TOKENS",
                     "_TILE_MIN_GRID_FRACTION", "_TILE_SPLIT_MAX_TOKENS", "_TILE_SPLIT_LONG_K", "_tile_failed")  # fmt: skip
 
@@ -1100,11 +1102,13 @@ class NPVQLinear(nn.Module):
         """Upper end of the tile-decode GEMM band for this layer."""
         if _TILE_MAX_TOKENS > 0 and self._wide_tile_layer():
             weights = self.in_features * self.out_features
+            k = self.in_features
             if weights >= _TILE_WIDE_MIN_WEIGHTS:
                 return max(_TILE_MAX_TOKENS, _TILE_WIDE_MAX_TOKENS)
-            if weights >= _TILE_WIDE_SMALL_WEIGHTS:
-                long = self.in_features >= _TILE_SPLIT_LONG_K
-                return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS if long else _TILE_WIDE_MID_MAX_TOKENS)
+            if weights >= _MID_LAYER_WEIGHTS and k >= _MID_LAYER_K:
+                return _TILE_WIDE_MAX_TOKENS
+            if weights >= _SMALL_LAYER_WEIGHTS and k >= 4096:
+                return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS if k >= _TILE_SPLIT_LONG_K else _TILE_WIDE_MID_MAX_TOKENS)
             if weights < _TILE_WIDE_TINY_WEIGHTS and _TILE_MIN_GRID_FRACTION > 0:
                 return min(_TILE_WIDE_MAX_TOKENS, _GEMV_KERNEL_MAX_TOKENS)
             return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_SMALL_MAX_TOKENS)
