@@ -371,7 +371,8 @@ extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64
 // walks in few tiles) -- or against 25 us: a library product takes 18.3-19 us per eager call whatever its size and
 // 33 us go by between two calls of decode + library product, whatever the GPU does meanwhile (2048 x 4096 with int4 weights,
 // 600 tokens: 35.8 us per call; with this kernel 25).
-// This kernel's estimates are some 15 % high at the larger shapes.  Measured, library / this kernel, us:
+// This kernel's estimates are some 15 % high at the larger shapes, not where K is short and 64 such tiles already make
+// the library quick (1.2 PFLOP/s: 945 x 8192 x 2048 30.9 / 32.3 us, 8192 x 2048 VQ layers at 600 tokens 39 / 42).  Measured, library / this kernel, us:
 // 171 x 256 x 640 14.6 / 4.8, 77 x 3003 x 2240 13.4 / 8.8, 100 x 14336 x 512 9.7 / 6.7,
 // 384 x 4096 x 4096 23.0 / 20.3, 250 x 11008 x 2048 21.5 / 17.3, 2500 x 3000 x 1024 26.2 / 20.3, 1024 x 4096 x 4096
 // 37.2 / 34.5; but 384 x 14336 x 4096 55.5 / 58.1, 700 x 6000 x 6016 56.8 / 64.8, 4096^3 93 / 124: products of more than
@@ -384,7 +385,9 @@ extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {
   if (forced) return forced > 0;
   const double gflop = 2e-9 * M * N * K;
   const float us = plan_dense(M, N, K, 0, kDenseMaxSplits).us;
-  const double big_tiles = ceil(M / 256.0) * ceil(N / 256.0), rate = big_tiles >= 180 ? 1.3 : 0.85;
+  const double big_tiles = ceil(M / 256.0) * ceil(N / 256.0);
+  const bool wide = big_tiles >= 64 && K < 4096;
+  const double rate = big_tiles >= 180 ? 1.3 : wide ? 1.2 : 0.85, margin = wide ? 1.0 : 1.15;
   const double library = 5.0 + gflop / rate + fmax(0.0, (K - 4096) / 1024.0) * 1.5;
-  return gflop <= (K >= 8192 ? 60.0 : 40.0) && us <= fmax(25.0, 1.15 * library) ? 1 : 0;
+  return gflop <= (K >= 8192 ? 60.0 : 40.0) && us <= fmax(25.0, margin * library) ? 1 : 0;
 }

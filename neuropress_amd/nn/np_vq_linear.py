@@ -128,7 +128,7 @@ _TILE_MAX_TOKENS: int = _env_int(
 _TILE_WIDE_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_TILE_WIDE_MAX_TOKENS",), 384)
 _TILE_WIDE_MIN_WEIGHTS: int = 1 << 25  # below: 384 tokens only with _MID_LAYER_K features on _MID_LAYER_WEIGHTS
 _TILE_WIDE_TINY_WEIGHTS: int = 5_000_000  # below: 32 tokens, where the GEMV ends
-_TILE_WIDE_LONG_MAX_TOKENS: int = 256  # _SMALL_LAYER_WEIGHTS and K of _TILE_SPLIT_LONG_K
+_TILE_WIDE_LONG_MAX_TOKENS: int = 256  # _MID_LAYER_WEIGHTS and K of 4096, or _SMALL_LAYER_WEIGHTS and K of _TILE_SPLIT_LONG_K
 _TILE_WIDE_MID_MAX_TOKENS: int = 128  # _SMALL_LAYER_WEIGHTS and K of 4096
 _TILE_WIDE_SMALL_MAX_TOKENS: int = 64  # all others
 
@@ -1105,8 +1105,8 @@ class NPVQLinear(nn.Module):
             k = self.in_features
             if weights >= _TILE_WIDE_MIN_WEIGHTS:
                 return max(_TILE_MAX_TOKENS, _TILE_WIDE_MAX_TOKENS)
-            if weights >= _MID_LAYER_WEIGHTS and k >= _MID_LAYER_K:
-                return _TILE_WIDE_MAX_TOKENS
+            if weights >= _MID_LAYER_WEIGHTS and k >= 4096:
+                return _TILE_WIDE_MAX_TOKENS if k >= _MID_LAYER_K else min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS)
             if weights >= _SMALL_LAYER_WEIGHTS and k >= 4096:
                 return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS if k >= _TILE_SPLIT_LONG_K else _TILE_WIDE_MID_MAX_TOKENS)
             if weights < _TILE_WIDE_TINY_WEIGHTS and _TILE_MIN_GRID_FRACTION > 0:
