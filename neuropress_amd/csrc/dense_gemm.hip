@@ -288,6 +288,7 @@ constexpr DenseCost kDenseCost[] = {
     {128, 128, 1, 0.00f, 0.388f, 0.047f, 3.68f}, // 8 waves
     {128, 128, 1, 0.00f, 0.375f, 0.045f, 4.55f}, // 4 waves
     {256, 128, 1, 0.00f, 0.622f, 0.053f, 4.39f}, // 8 waves
+    {192, 128, 1, 0.00f, 0.515f, 0.040f, 4.20f}, // 4 waves of 96 x 64: fewest LDS reads per MFMA
 };
 constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]);
 
@@ -299,7 +300,8 @@ int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
     case 2: return launch_dense_tile<ACT, 2, 2, 1, 2, 3>(s, st);
     case 3: return launch_dense_tile<ACT, 4, 2, 1, 1, 5>(s, st);
     case 4: return launch_dense_tile<ACT, 2, 2, 2, 1, 5>(s, st);
-    default: return launch_dense_tile<ACT, 4, 2, 2, 1, 3>(s, st);
+    case 5: return launch_dense_tile<ACT, 4, 2, 2, 1, 3>(s, st);
+    default: return launch_dense_tile<ACT, 2, 2, 3, 1, 4>(s, st);
   }
 }
 
@@ -371,10 +373,11 @@ extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64
 // walks in few tiles) -- or against 25 us: a library product takes 18.3-19 us per eager call whatever its size and
 // 33 us go by between two calls of decode + library product, whatever the GPU does meanwhile (2048 x 4096 with int4 weights,
 // 600 tokens: 35.8 us per call; with this kernel 25).
-// This kernel's estimates are some 15 % high at the larger shapes, not where K is short and 64 such tiles already make
-// the library quick (1.2 PFLOP/s: 945 x 8192 x 2048 30.9 / 32.3 us, 8192 x 2048 VQ layers at 600 tokens 39 / 42).  Measured, library / this kernel, us:
+// This kernel's estimates are some 15 % high at the larger shapes; where 64 such tiles make the library quicker
+// (1.05 PFLOP/s, on short K 1.2: 288 x 14336 x 4096 39.4 / 43.8 us, 945 x 8192 x 2048 30.9 / 32.3) the margin is smaller.
+// Measured, library / this kernel, us:
 // 171 x 256 x 640 14.6 / 4.8, 77 x 3003 x 2240 13.4 / 8.8, 100 x 14336 x 512 9.7 / 6.7,
-// 384 x 4096 x 4096 23.0 / 20.3, 250 x 11008 x 2048 21.5 / 17.3, 2500 x 3000 x 1024 26.2 / 20.3, 1024 x 4096 x 4096
+// 384 x 4096 x 4096 23.0 / 20.3, 384 x 11008 x 2048 25.3 / 24.5, 250 x 11008 x 2048 21.5 / 17.3, 2500 x 3000 x 1024 26.2 / 20.3, 1024 x 4096 x 4096
 // 37.2 / 34.5; but 384 x 14336 x 4096 55.5 / 58.1, 700 x 6000 x 6016 56.8 / 64.8, 4096^3 93 / 124: products of more than
 // 40 GFLOP go to the library.  Long K, split over blocks: 47 x 384 x 8320 19.0 / 8.8 (16.3 unsplit), 945 x 512 x 14336
 // 38.4 / 26.2, 230 x 3152 x 7296 27.3 / 22.2, 460 x 2432 x 7936 36.1 / 29.4, 460 x 4096 x 14336 (54 GFLOP) 72 / 60, but
@@ -386,8 +389,8 @@ extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {
   const double gflop = 2e-9 * M * N * K;
   const float us = plan_dense(M, N, K, 0, kDenseMaxSplits).us;
   const double big_tiles = ceil(M / 256.0) * ceil(N / 256.0);
-  const bool wide = big_tiles >= 64 && K < 4096;
-  const double rate = big_tiles >= 180 ? 1.3 : wide ? 1.2 : 0.85, margin = wide ? 1.0 : 1.15;
+  const bool many = big_tiles >= 64, shallow = many && K < 4096;
+  const double rate = big_tiles >= 180 ? 1.3 : shallow ? 1.2 : many ? 1.05 : 0.85, margin = shallow ? 1.0 : many ? 1.1 : 1.15;
   const double library = 5.0 + gflop / rate + fmax(0.0, (K - 4096) / 1024.0) * 1.5;
   return gflop <= (K >= 8192 ? 60.0 : 40.0) && us <= fmax(25.0, margin * library) ? 1 : 0;
 }

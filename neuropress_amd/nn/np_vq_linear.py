@@ -127,6 +127,10 @@ _TILE_MAX_TOKENS: int = _env_int(
 # 1024 x 4096 15 / 19 / 24 against 15 / 16 / 17, 2048 x 2048 13 / 15 / 22 against 12 / 12 / 13.
 _TILE_WIDE_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_TILE_WIDE_MAX_TOKENS",), 384)
 _TILE_WIDE_MIN_WEIGHTS: int = 1 << 25  # below: 384 tokens only with _MID_LAYER_K features on _MID_LAYER_WEIGHTS
+# Column blocks that nearly fill the GPU by themselves (K in two or three parts): 256 tokens.  At 200 tokens, tile / decode +
+# product: 11008 x 2048 31.6 / 35.1, 10000 x 3072 40.7 / 46.5, 14336 x 2048 35.3 / 39.8; 8192 x 2048 33 / 27.
+_TILE_WIDE_BROAD_WEIGHTS: int = 1 << 24
+_TILE_WIDE_BROAD_FEATURES: int = 9216
 _TILE_WIDE_TINY_WEIGHTS: int = 5_000_000  # below: 32 tokens, where the GEMV ends
 _TILE_WIDE_LONG_MAX_TOKENS: int = 256  # _MID_LAYER_WEIGHTS and K of 4096, or _SMALL_LAYER_WEIGHTS and K of _TILE_SPLIT_LONG_K
 _TILE_WIDE_MID_MAX_TOKENS: int = 128  # _SMALL_LAYER_WEIGHTS and K of 4096
@@ -173,7 +177,8 @@ _PLAN_ATTRIBUTES = ("backend", "proxy", "residual_proxy", "out_features", "in_fe
                     "bias", "column_perm", "packed_residual", "row_scale", "row_bias")  # fmt: skip
 _PLAN_THRESHOLDS = ("_FUSED_MAX_TOKENS", "_FUSED_WIDE_MAX_TOKENS", "_FUSED_WIDE_MAX_ACTIVATIONS", "_SLICED_MAX_TOKENS",
                     "_SLICED_MIN_CENTROIDS", "_SLICED_MIN_INDICES", "_LUT_MAX_TOKENS", "_TILE_MAX_TOKENS", "_TILE_WIDE_MAX_TOKENS",
-                    "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_TINY_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS",
+                    "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_BROAD_WEIGHTS", "_TILE_WIDE_BROAD_FEATURES",
+                    "_TILE_WIDE_TINY_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS",
                     "_TILE_WIDE_LONG_MAX_TOKENS", "_TILE_WIDE_SMALL_MAX_TOKENS", "_TILE_SMALL_LAYER_MAX_TOKENS",
                     "_TILE_MIN_GRID_FRACTION", "_TILE_SPLIT_MAX_TOKENS", "_TILE_SPLIT_LONG_K", "_tile_failed")  # fmt: skip
 
@@ -1107,6 +1112,8 @@ class NPVQLinear(nn.Module):
                 return max(_TILE_MAX_TOKENS, _TILE_WIDE_MAX_TOKENS)
             if weights >= _MID_LAYER_WEIGHTS and k >= 4096:
                 return _TILE_WIDE_MAX_TOKENS if k >= _MID_LAYER_K else min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS)
+            if weights >= _TILE_WIDE_BROAD_WEIGHTS and self.out_features >= _TILE_WIDE_BROAD_FEATURES:
+                return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS)
             if weights >= _SMALL_LAYER_WEIGHTS and k >= 4096:
                 return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS if k >= _TILE_SPLIT_LONG_K else _TILE_WIDE_MID_MAX_TOKENS)
             if weights < _TILE_WIDE_TINY_WEIGHTS and _TILE_MIN_GRID_FRACTION > 0:

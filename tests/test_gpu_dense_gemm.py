@@ -23,13 +23,13 @@ def dense_tile(monkeypatch):
 
 
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
 def test_dense_gemm_tiles(gpu, dense_tile, tile, act):
     from neuropress_amd import kernels
 
     dense_tile(tile)
     for m, n, k in ((1, 1, 64), (31, 63, 128), (33, 65, 192), (64, 128, 256), (65, 129, 320), (127, 200, 448), (129, 257, 704),
-                    (256, 130, 576), (300, 500, 1088), (520, 40, 64)):  # fmt: skip
+                    (256, 130, 576), (300, 500, 1088), (520, 40, 64), (193, 129, 320)):  # fmt: skip
         g = cases.gen(m + n + k)
         x = torch.randn(m, k, generator=g).to(act)
         w = (torch.randn(n, k, generator=g) * 0.05).to(act)
@@ -46,7 +46,7 @@ def test_dense_gemm_tiles(gpu, dense_tile, tile, act):
 
 
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("tile,splits", [(1, 2), (1, 16), (2, 9), (3, 3), (4, 8), (5, 7), (6, 2)])
+@pytest.mark.parametrize("tile,splits", [(1, 2), (1, 16), (2, 9), (3, 3), (4, 8), (5, 7), (6, 2), (7, 3)])
 def test_dense_gemm_parts_of_k(gpu, dense_tile, monkeypatch, tile, splits, act):
     """K in parts over blocks: parts of unequal length, of fewer steps than a ring is deep or a block has groups of
     waves, columns the reduction reads four at a time and not."""
