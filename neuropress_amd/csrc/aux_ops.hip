@@ -423,40 +423,65 @@ int launch_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
 // whole number of 64-column chunks, 16-bit elements:
 //   out[m, k] = x[m, perm ? perm[k] : k] for k < K, 0 for K <= k < ldo.
 //
-// Bound by the launch at the token counts of a decode step and by HBM beyond.  A block takes 2048
-// output columns of one row.  With a permutation it first copies the whole row into LDS (one
-// contiguous read) and gathers there with 2-byte reads: through the vector memory path an element
-// gather costs a lane one cycle and a cache line each.  77 x 2184 with a permutation: 2.3 us where
-// torch's gather takes 4.2; 4096 x 3456: see the table of cases in the design notes.
+// Bound by the launch at the token counts of a decode step and by HBM beyond.  With a permutation a block first
+// copies whole rows into LDS (one contiguous read) and gathers there with 2-byte reads: through the vector memory path
+// an element gather costs a lane one cycle and a cache line each (77 x 2184: 2.3 us where torch's gather takes 4.2).
+// Few rows: a block takes 2048 output columns of one, and a row is copied once per block.  Where the rows alone fill the
+// GPU a block takes all columns (the copy is made once), from 1024 rows on of two rows at a time, which share the reads
+// of the permutation.  A row copied by every block of 2048 columns / once, us: 300 x 13968 20.2 / 8.0, 600 x 4096
+// 7.6 / 4.3, 1200 x 13968 65.0 / 23.5, 4096 x 3456 39.3 / 11.4, 4096 x 14336 195.6 / 54.4 (4.3 TB/s).
 // ---------------------------------------------------------------------------
-constexpr int kGatherRowMax = 32768;  // elements of a row held in LDS (64 KiB)
-template <bool PERM, bool LDS>
+constexpr int kGatherRowMax = 32768;  // elements of the rows held in LDS (64 KiB)
+constexpr int kGatherWholeRows = 256, kGatherPairRows = 1024;
+template <bool PERM, bool LDS, int ROWS>
 __global__ void __launch_bounds__(256)
 gather_columns_kernel(const uint16_t* __restrict__ x, int64_t ldx, const int32_t* __restrict__ perm,
-                      uint16_t* __restrict__ out, int64_t ldo, int K, bool vec) {
+                      uint16_t* __restrict__ out, int64_t ldo, int M, int K, bool vec, bool perm_vec) {
   extern __shared__ __attribute__((aligned(16))) uint16_t row_lds[];
-  const uint16_t* xr = x + (int64_t)blockIdx.y * ldx;
+  const int row0 = blockIdx.y * ROWS;
+  const int stride = (K + 7) & ~7;  // elements between the rows in LDS
+  const uint16_t* xr[ROWS];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) xr[r] = x + (int64_t)min(row0 + r, M - 1) * ldx;
   if constexpr (PERM && LDS) {
     const int whole = vec ? K >> 3 : 0;
-    for (int i = threadIdx.x; i < whole; i += 256)
-      reinterpret_cast<u32x4*>(row_lds)[i] = reinterpret_cast<const u32x4*>(xr)[i];
-    for (int i = whole * 8 + threadIdx.x; i < K; i += 256) row_lds[i] = xr[i];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      uint16_t* const mine = row_lds + r * stride;
+#pragma unroll 4
+      for (int i = threadIdx.x; i < whole; i += 256)
+        reinterpret_cast<u32x4*>(mine)[i] = reinterpret_cast<const u32x4*>(xr[r])[i];
+      for (int i = whole * 8 + threadIdx.x; i < K; i += 256) mine[i] = xr[r][i];
+      xr[r] = mine;
+    }
     __syncthreads();
-    xr = row_lds;
   }
-  const int k0 = (blockIdx.x * 256 + threadIdx.x) * 8;
-  if (k0 >= ldo) return;
-  uint16_t v[8];
+  for (int64_t c0 = (int64_t)(blockIdx.x * 256 + threadIdx.x) * 8; c0 < ldo; c0 += (int64_t)gridDim.x * 2048) {
+    const int k0 = (int)c0;
+    int at[8];
+    if (PERM && perm_vec && k0 + 8 <= K) {
+      const u32x4 lo = *reinterpret_cast<const u32x4*>(perm + k0), hi = *reinterpret_cast<const u32x4*>(perm + k0 + 4);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int k = k0 + e;
-    v[e] = 0;
-    if (k < K) v[e] = xr[PERM ? perm[k] : k];
+      for (int e = 0; e < 4; ++e) {
+        at[e] = (int)lo[e];
+        at[4 + e] = (int)hi[e];
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) at[e] = k0 + e < K ? (PERM ? perm[k0 + e] : k0 + e) : -1;
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      if (row0 + r >= M) break;
+      uint16_t v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = at[e] >= 0 ? xr[r][at[e]] : (uint16_t)0;
+      u32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (uint32_t)v[2 * e] | ((uint32_t)v[2 * e + 1] << 16);
+      *reinterpret_cast<u32x4*>(out + (int64_t)(row0 + r) * ldo + k0) = o;
+    }
   }
-  u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = (uint32_t)v[2 * e] | ((uint32_t)v[2 * e + 1] << 16);
-  *reinterpret_cast<u32x4*>(out + (int64_t)blockIdx.y * ldo + k0) = o;
 }
 
 }  // namespace
@@ -472,13 +497,18 @@ extern "C" int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* p
   auto xs = (const uint16_t*)x;
   auto os = (uint16_t*)out;
   const unsigned segments = (unsigned)((ldo + 2047) / 2048);
-  for (int m0 = 0; m0 < M; m0 += 65535) {
-    const dim3 grid(segments, (unsigned)(M - m0 < 65535 ? M - m0 : 65535));
+  const bool lds = perm && K <= kGatherRowMax, pair = lds && M >= kGatherPairRows && 2 * ((K + 7) & ~7) <= kGatherRowMax;
+  const int lds_bytes = ((K + 7) & ~7) * 2;
+  const bool pv = aligned16(perm);
+  for (int m0 = 0; m0 < M; m0 += 65534) {
+    const int rows = M - m0 < 65534 ? M - m0 : 65534;
+    const dim3 grid(lds && M >= kGatherWholeRows ? 1 : segments, (unsigned)(pair ? (rows + 1) / 2 : rows));
     const uint16_t* xm = xs + (int64_t)m0 * ldx;
     uint16_t* om = os + (int64_t)m0 * ldo;
-    if (!perm) launch(gather_columns_kernel<false, false>, grid, 256, 0, st, xm, ldx, perm, om, ldo, K, vec);
-    else if (K <= kGatherRowMax) launch(gather_columns_kernel<true, true>, grid, 256, (K * 2 + 15) & ~15, st, xm, ldx, perm, om, ldo, K, vec);
-    else launch(gather_columns_kernel<true, false>, grid, 256, 0, st, xm, ldx, perm, om, ldo, K, vec);
+    if (!perm) launch(gather_columns_kernel<false, false, 1>, grid, 256, 0, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);
+    else if (pair) launch(gather_columns_kernel<true, true, 2>, grid, 256, 2 * lds_bytes, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);
+    else if (lds) launch(gather_columns_kernel<true, true, 1>, grid, 256, lds_bytes, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);
+    else launch(gather_columns_kernel<true, false, 1>, grid, 256, 0, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);
   }
   return check_launch("npamd_gather_columns");
 }

@@ -26,6 +26,21 @@ def test_gather_columns(gpu, k, width):
             assert torch.equal(out[:, :k], x if p is None else x[:, p]) and not out[:, k:].any()
 
 
+@pytest.mark.parametrize("rows", [255, 256, 1023, 1025])
+@pytest.mark.parametrize("k", [40, 2056, 5003, 16384, 16392, 32768])
+def test_gather_columns_of_many_rows(gpu, k, rows):
+    """Whole rows per block, and two rows per block where LDS holds them: an odd last row, rows around the LDS limits."""
+    from neuropress_amd import kernels
+
+    g = torch.Generator(device=gpu).manual_seed(k)
+    x = torch.randint(-30000, 30000, (rows, k), generator=g, device=gpu, dtype=torch.int16).view(torch.half)
+    big = torch.zeros(k + 4, dtype=torch.int32, device=gpu)
+    big[1 : k + 1] = torch.randperm(k, generator=g, device=gpu)
+    for perm in (big[1 : k + 1].clone(), big[1 : k + 1]):  # 16-byte aligned, and not
+        out = kernels.gather_columns(x, perm, (k + 63) // 64 * 64)
+        assert torch.equal(out[:, :k].view(torch.int16), x.view(torch.int16)[:, perm.long()]) and not out[:, k:].any()
+
+
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("n,k,nc,vl,perm", [(70, 8, 16, 8, False), (130, 200, 1000, 8, True), (257, 1000, 4096, 4, False),
                                             (64, 2184, 65536, 8, True), (96, 1544, 300, 8, False)])  # fmt: skip
