@@ -324,15 +324,17 @@ DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits) {
   for (int i = 0; i < kDenseTiles; ++i) {
     if (forced_tile > 0 && forced_tile <= kDenseTiles && i != forced_tile - 1) continue;
     const DenseCost& c = kDenseCost[i];
-    const double tiles = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-    const double load = tiles * steps * (c.bm + c.bn) * 128e-6 * c.per_mb;
+    const int64_t tiles = (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const float load = (float)tiles * steps * (c.bm + c.bn) * 128e-6f * c.per_mb;
     for (int splits = 1; splits <= max_splits; ++splits) {
       if (forced_splits > 0 && splits != forced_splits) continue;
-      if (forced_splits <= 0 && splits > 1 && (steps / splits < kDenseMinSplitSteps || tiles * splits > 512)) break;
-      const double rounds = ceil(ceil(tiles * splits / 8) / 32);
-      const double walk = rounds * ceil(ceil((double)steps / splits) / c.groups) * c.per_step;
-      float t = (float)(c.fixed + rounds * c.per_round + sqrt(walk * walk + load * load));
-      if (splits > 1) t += kSplitFixed + kSplitPerMb * (float)(1e-6 * splits * M * N * 4);
+      if (forced_splits <= 0 && splits > 1 && (steps < kDenseMinSplitSteps * splits || tiles * splits > 512)) break;
+      const int64_t rounds = ((tiles * splits + 7) / 8 + 31) / 32;
+      const int part = (steps + splits - 1) / splits;
+      const float walk = (float)rounds * ((part + c.groups - 1) / c.groups) * c.per_step;
+      float t = c.fixed + (float)rounds * c.per_round + (splits > 1 ? kSplitFixed + kSplitPerMb * (4e-6f * splits * M * N) : 0.f);
+      if (t + fmaxf(walk, load) >= best.us) continue;
+      t += sqrtf(walk * walk + load * load);
       if (t < best.us) best = {i, splits, t};
     }
   }
