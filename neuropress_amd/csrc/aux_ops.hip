@@ -426,13 +426,14 @@ int launch_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
 // Bound by the launch at the token counts of a decode step and by HBM beyond.  With a permutation a block first
 // copies whole rows into LDS (one contiguous read) and gathers there with 2-byte reads: through the vector memory path
 // an element gather costs a lane one cycle and a cache line each (77 x 2184: 2.3 us where torch's gather takes 4.2).
-// Few rows: a block takes 2048 output columns of one, and a row is copied once per block.  Where the rows alone fill the
-// GPU a block takes all columns (the copy is made once), from 1024 rows on of two rows at a time, which share the reads
-// of the permutation.  A row copied by every block of 2048 columns / once, us: 300 x 13968 20.2 / 8.0, 600 x 4096
+// Few rows: a block takes 2048 output columns of one, and a row is copied once per block.  Past kGatherBlocks blocks of
+// those a row has only as many as make up that number, which stride over its columns (220 x 13968 10.4 -> 5.8 us), one
+// from 1024 rows on, of two rows at a time then, which share the reads of the permutation.  A row copied by every
+// block of 2048 columns / like this, us: 300 x 13968 20.2 / 7.0, 600 x 4096
 // 7.6 / 4.3, 1200 x 13968 65.0 / 23.5, 4096 x 3456 39.3 / 11.4, 4096 x 14336 195.6 / 54.4 (4.3 TB/s).
 // ---------------------------------------------------------------------------
 constexpr int kGatherRowMax = 32768;  // elements of the rows held in LDS (64 KiB)
-constexpr int kGatherWholeRows = 256, kGatherPairRows = 1024;
+constexpr int kGatherBlocks = 1024, kGatherPairRows = 1024;
 template <bool PERM, bool LDS, int ROWS>
 __global__ void __launch_bounds__(256)
 gather_columns_kernel(const uint16_t* __restrict__ x, int64_t ldx, const int32_t* __restrict__ perm,
@@ -502,7 +503,8 @@ extern "C" int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* p
   const bool pv = aligned16(perm);
   for (int m0 = 0; m0 < M; m0 += 65534) {
     const int rows = M - m0 < 65534 ? M - m0 : 65534;
-    const dim3 grid(lds && M >= kGatherWholeRows ? 1 : segments, (unsigned)(pair ? (rows + 1) / 2 : rows));
+    const unsigned per_row = lds ? (unsigned)(M < kGatherBlocks ? kGatherBlocks / M : 1) : segments;
+    const dim3 grid(per_row < segments ? per_row : segments, (unsigned)(pair ? (rows + 1) / 2 : rows));
     const uint16_t* xm = xs + (int64_t)m0 * ldx;
     uint16_t* om = os + (int64_t)m0 * ldo;
     if (!perm) launch(gather_columns_kernel<false, false, 1>, grid, 256, 0, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);

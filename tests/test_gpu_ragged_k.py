@@ -26,7 +26,7 @@ def test_gather_columns(gpu, k, width):
             assert torch.equal(out[:, :k], x if p is None else x[:, p]) and not out[:, k:].any()
 
 
-@pytest.mark.parametrize("rows", [255, 256, 1023, 1025])
+@pytest.mark.parametrize("rows", [255, 400, 600, 1023, 1025])
 @pytest.mark.parametrize("k", [40, 2056, 5003, 16384, 16392, 32768])
 def test_gather_columns_of_many_rows(gpu, k, rows):
     """Whole rows per block, and two rows per block where LDS holds them: an odd last row, rows around the LDS limits."""
