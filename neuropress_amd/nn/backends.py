@@ -148,12 +148,13 @@ _LARGE_LAYER_WEIGHTS: int = 1 << 25
 
 def tile_band_ok(
     m: int, n: int, k: int, cus: int, min_fraction: float, split_max_tokens: int, long_k: int,
-    small_max_tokens: int = 1 << 30,
+    small_max_tokens: int = 1 << 30, half_ok: bool = False,
 ) -> bool:
     """Whether the tile-decode GEMM has enough workgroups for ``m`` tokens on an
     ``n x k`` layer.  Mirrors the kernel's own plan: without a split when the
     (64 columns x up to 384 rows) grid covers ``min_fraction`` of ``cus`` compute
-    units; otherwise up to 16 reduction splits of at least 512 input features.
+    units; otherwise up to 16 reduction splits of at least 512 input features.  *half_ok*: a grid of more than half
+    the compute units, too large to split, will do.
 
     Measured, us, tile GEMM / decode + dense product: 3008 x 2240 with a 4096-row codebook 13.7 / 14.1 at 33 tokens,
     14.4 / 14.2 at 64, 17.5 / 15.2 at 128, with int4 weights 15.8 / 13.1 at 33; 6144 x 1024 int4 13.9 / 10.9 at 33;
@@ -161,7 +162,7 @@ def tile_band_ok(
     int4 29.0 / 31.2, with a 256-row codebook 25.1 / 35.8, residual VQ 31.9 / 40.1; 4096 x 6144 30.5 / 34.3, 28.2 / 34.2,
     35.9 / 40.7; 4096 x 4096 26.1 / 24.6, 26.7 / 25, 28.8 / 28.6."""
     blocks = -(-n // 64) * -(-m // 384)
-    if blocks >= min_fraction * cus:
+    if blocks >= min_fraction * cus or (half_ok and 2 * blocks > cus):
         return True
     splits = max(1, min(cus // blocks, k // 512, 16))
     if splits * blocks < min_fraction * cus:

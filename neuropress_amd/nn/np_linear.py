@@ -54,6 +54,11 @@ _Q_TILE_WIDE_MIN_FEATURES: int = 8192
 _Q_TILE_MIN_GRID_FRACTION: float = 0.7
 _Q_TILE_SPLIT_MAX_TOKENS: int = 144
 _Q_TILE_SPLIT_LONG_K: int = 8192
+# Grids of more than half the compute units that are too large to split (8193 to 11456 output features): the fused GEMM
+# from this K on, below it up to 256 tokens without zero points.  Decode + GEMM / fused, us at 36 / 100 / 256 / 384 tokens:
+# 11008 x 4096 40 / 42 / 51 / 61 against 26 / 29 / 39 / 52, 8320 x 12288 93 / 108 / 132 / 151 against 48 / 56 / 81 / 114; 10240 x 2048
+# 20 / 22 / 27 / 31 against 17 / 20 / 25 / 34, with zero points 20 / 22 / 27 / 32 against 22 / 23 / 29 / 39.
+_Q_TILE_HALF_GRID_K: int = 4096
 _Q_FUSED_MAX_TOKENS: int = 16
 # 17..32 tokens: the GEMV reuses every dequantized operand for two 16-token tiles, and each
 # workgroup reads all of x from L2, so it beats the fused GEMM while x is small.  Measured
@@ -156,7 +161,8 @@ def _q_dequant_linear(
 # What the choice of a kernel reads besides the buffers: a call plan is valid while these are unchanged.
 _PLAN_ATTRIBUTES = ("backend", "out_features", "in_features", "group_size", "nbits", "zero_point", "bias")
 _PLAN_THRESHOLDS = ("_Q_TILE_MAX_TOKENS", "_Q_TILE_LONG_K_MAX_TOKENS", "_Q_TILE_WIDE_MAX_TOKENS", "_Q_TILE_WIDE_MIN_FEATURES",
-                    "_Q_TILE_MIN_GRID_FRACTION", "_Q_TILE_SPLIT_MAX_TOKENS", "_Q_TILE_SPLIT_LONG_K", "_Q_FUSED_MAX_TOKENS",
+                    "_Q_TILE_MIN_GRID_FRACTION", "_Q_TILE_SPLIT_MAX_TOKENS", "_Q_TILE_SPLIT_LONG_K", "_Q_TILE_HALF_GRID_K",
+                    "_Q_FUSED_MAX_TOKENS",
                     "_Q_FUSED_WIDE_MAX_TOKENS", "_Q_FUSED_WIDE_MAX_ACTIVATIONS")  # fmt: skip
 
 
@@ -325,6 +331,7 @@ class NPLinear(nn.Module):
         return tile_band_ok(
             m, self.out_features, self.in_features, cus,
             _Q_TILE_MIN_GRID_FRACTION, _Q_TILE_SPLIT_MAX_TOKENS, _Q_TILE_SPLIT_LONG_K, _Q_FUSED_WIDE_MAX_TOKENS,
+            self.in_features >= _Q_TILE_HALF_GRID_K or (self.zero_point is None and m <= 256),
         )  # fmt: skip
 
     def _gemv_max_tokens(self, m: int) -> int:

@@ -149,6 +149,11 @@ _TILE_MIN_GRID_FRACTION: float = 0.7
 _TILE_SPLIT_MAX_TOKENS: int = 128
 # Small layers (fewer than 8 M weights) decode in 4-8 us and leave the band earlier; residual ones at 32 tokens.
 _TILE_SMALL_LAYER_MAX_TOKENS: int = 64
+# Grids of more than half the compute units that are too large to split (8193 to 11456 output features): the tile GEMM up
+# to 256 tokens, fewer on very long reductions.  Decode + GEMM / tile, us at 36 / 100 / 256 tokens: 11008 x 4096 with a
+# 256-row codebook 44 / 46 / 53 against 18 / 20 / 36, with 4096 rows 38 / 40 / 50 against 21 / 24 / 43, residual 43 / 45 / 55
+# against 34 / 39 / 51; 8320 x 12288 with 256 rows 69 / 76 / 105 against 43 / 53 / 109, residual 121 / 127 / 152 against 83 / 107 / 164.
+_TILE_HALF_GRID_MAX_ACTIVATIONS: int = 5 << 19  # tokens x K
 _TILE_SPLIT_LONG_K: int = 8192  # from this many input features on, _TILE_MAX_TOKENS applies
 # Layers of at least this many indices time their slice-list GEMV against the fused one when the
 # lists are built (NPVQLinear._sliced_token_limit).
@@ -180,7 +185,8 @@ _PLAN_THRESHOLDS = ("_FUSED_MAX_TOKENS", "_FUSED_WIDE_MAX_TOKENS", "_FUSED_WIDE_
                     "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_BROAD_WEIGHTS", "_TILE_WIDE_BROAD_FEATURES",
                     "_TILE_WIDE_TINY_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS",
                     "_TILE_WIDE_LONG_MAX_TOKENS", "_TILE_WIDE_SMALL_MAX_TOKENS", "_TILE_SMALL_LAYER_MAX_TOKENS",
-                    "_TILE_MIN_GRID_FRACTION", "_TILE_SPLIT_MAX_TOKENS", "_TILE_SPLIT_LONG_K", "_tile_failed")  # fmt: skip
+                    "_TILE_MIN_GRID_FRACTION", "_TILE_SPLIT_MAX_TOKENS", "_TILE_SPLIT_LONG_K",
+                    "_TILE_HALF_GRID_MAX_ACTIVATIONS", "_tile_failed")  # fmt: skip
 
 # Latched once the tile GEMM fails with fallback allowed, so later calls go
 # straight to decode + GEMM (reference: np_vq_linear.py:91-93).
@@ -1139,6 +1145,7 @@ class NPVQLinear(nn.Module):
             m, self.out_features, self._kernel_k(), cus,
             _TILE_MIN_GRID_FRACTION, _TILE_SPLIT_MAX_TOKENS, _TILE_SPLIT_LONG_K,
             32 if self.is_residual else _TILE_SMALL_LAYER_MAX_TOKENS,
+            m <= 256 and m * self._kernel_k() <= _TILE_HALF_GRID_MAX_ACTIVATIONS,
         )  # fmt: skip
 
     # -- torch-op paths ---------------------------------------------------
