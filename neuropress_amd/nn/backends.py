@@ -144,17 +144,22 @@ _SMALL_LAYER_WEIGHTS: int = 8_000_000
 _MID_LAYER_WEIGHTS: int = 12_000_000
 _MID_LAYER_K: int = 6144
 _LARGE_LAYER_WEIGHTS: int = 1 << 25
+# Decode + GEMM / tile, us at 36 / 128 tokens: 5632 x 2048 with a 256-row codebook 14.0 / 15.9 against 11.5 / 14.7, residual 17.1 / 18.9
+# against 16.9 / 21.6, int4 14.0 / 16.3 against 15.8 / 19.4; 5632 x 4096 int4 22.3 / 25.7 against 20.4 / 23.3, with zero points
+# 22.4 / 25.7 against 24.9 / 27.7; 5504 x 8192 int4 41.6 / 48.3 against 29.5 / 36.3, 256-row codebook 43.4 / 50.2 against 20.7 / 27.1.
+_TIGHT_GRID_FRACTION: float = 0.66
 
 
 def tile_band_ok(
     m: int, n: int, k: int, cus: int, min_fraction: float, split_max_tokens: int, long_k: int,
-    small_max_tokens: int = 1 << 30, half_ok: bool = False,
+    small_max_tokens: int = 1 << 30, half_ok: bool = False, tight_k: int = 1 << 30,
 ) -> bool:
     """Whether the tile-decode GEMM has enough workgroups for ``m`` tokens on an
     ``n x k`` layer.  Mirrors the kernel's own plan: without a split when the
     (64 columns x up to 384 rows) grid covers ``min_fraction`` of ``cus`` compute
     units; otherwise up to 16 reduction splits of at least 512 input features.  *half_ok*: a grid of more than half
-    the compute units, too large to split, will do.
+    the compute units, too large to split, will do.  From *tight_k* input features on 0.66 of them will do for a split
+    grid (86 to 89 column blocks, in two parts).
 
     Measured, us, tile GEMM / decode + dense product: 3008 x 2240 with a 4096-row codebook 13.7 / 14.1 at 33 tokens,
     14.4 / 14.2 at 64, 17.5 / 15.2 at 128, with int4 weights 15.8 / 13.1 at 33; 6144 x 1024 int4 13.9 / 10.9 at 33;
@@ -165,7 +170,7 @@ def tile_band_ok(
     if blocks >= min_fraction * cus or (half_ok and 2 * blocks > cus):
         return True
     splits = max(1, min(cus // blocks, k // 512, 16))
-    if splits * blocks < min_fraction * cus:
+    if splits * blocks < min_fraction * cus and not (splits > 1 and k >= tight_k and splits * blocks >= _TIGHT_GRID_FRACTION * cus):
         return False
     if n * k < _SMALL_LAYER_WEIGHTS and m > small_max_tokens:
         return False

@@ -332,6 +332,7 @@ class NPLinear(nn.Module):
             m, self.out_features, self.in_features, cus,
             _Q_TILE_MIN_GRID_FRACTION, _Q_TILE_SPLIT_MAX_TOKENS, _Q_TILE_SPLIT_LONG_K, _Q_FUSED_WIDE_MAX_TOKENS,
             self.in_features >= _Q_TILE_HALF_GRID_K or (self.zero_point is None and m <= 256),
+            4096 if self.zero_point is None else 6144,
         )  # fmt: skip
 
     def _gemv_max_tokens(self, m: int) -> int:

@@ -1145,7 +1145,7 @@ class NPVQLinear(nn.Module):
             m, self.out_features, self._kernel_k(), cus,
             _TILE_MIN_GRID_FRACTION, _TILE_SPLIT_MAX_TOKENS, _TILE_SPLIT_LONG_K,
             32 if self.is_residual else _TILE_SMALL_LAYER_MAX_TOKENS,
-            m <= 256 and m * self._kernel_k() <= _TILE_HALF_GRID_MAX_ACTIVATIONS,
+            m <= 256 and m * self._kernel_k() <= _TILE_HALF_GRID_MAX_ACTIVATIONS, 4096 if self.is_residual else 2048,
         )  # fmt: skip
 
     # -- torch-op paths ---------------------------------------------------
