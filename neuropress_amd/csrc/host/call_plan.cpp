@@ -314,18 +314,19 @@ bool stale(Plan* p, PyObject* module) {
   return false;
 }
 
-// Whether x is a stack of contiguous rows at one distance (the last tokens of a batch of prompts, say).
+// Whether x is a stack of contiguous rows at one distance (the last tokens of a batch of prompts, say).  Expanded inputs
+// are not: their rows lie at distance 0, or at several.
 bool rows_at_one_stride(const at::Tensor& x, int64_t* ldx) {
-  const int64_t dims = x.dim();
   if (x.stride(-1) != 1) return false;
-  int64_t row = 0, next = 0;  // distance of two rows; stride the next dimension outwards must have
-  for (int64_t d = dims - 2; d >= 0; --d) {
+  bool found = false;
+  int64_t row = x.size(-1), next = 0;  // distance of two rows; stride the next dimension outwards must have
+  for (int64_t d = x.dim() - 2; d >= 0; --d) {
     if (x.size(d) == 1) continue;
-    if (row == 0) row = x.stride(d);
+    if (!found) row = x.stride(d);
     else if (x.stride(d) != next) return false;
+    found = true;
     next = x.stride(d) * x.size(d);
   }
-  if (row == 0) row = x.size(-1);
   *ldx = row;
   return row >= x.size(-1);
 }
@@ -730,7 +731,20 @@ PyObject* set_workspaces(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
+// row_distance(x): elements between the rows of x that a plan would hand to a kernel, or None where it declines.
+PyObject* row_distance(PyObject*, PyObject* xo) {
+  if (!THPVariable_Check(xo) || THPVariable_Unpack(xo).dim() < 1) {
+    PyErr_SetString(PyExc_TypeError, "row_distance() takes a tensor of one dimension or more");
+    return nullptr;
+  }
+  const at::Tensor& x = THPVariable_Unpack(xo);
+  int64_t ldx = x.size(-1);
+  if (!x.is_contiguous() && !rows_at_one_stride(x, &ldx)) Py_RETURN_NONE;
+  return PyLong_FromLongLong(ldx);
+}
+
 PyMethodDef module_methods[] = {
+    {"row_distance", row_distance, METH_O, "row_distance(x): elements between the rows a plan would read, or None"},
     {"set_module_class", set_module_class, METH_VARARGS, "set_module_class(torch.nn.Module, its call in Python)"},
     {"set_workspaces", set_workspaces, METH_VARARGS, "set_workspaces(dict, drop): the slice-list GEMV's scratch buffers"},
     {nullptr, nullptr, 0, nullptr},

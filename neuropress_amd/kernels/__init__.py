@@ -86,9 +86,16 @@ def _bias_f32(bias: torch.Tensor | None) -> torch.Tensor | None:
 def _x2d(x: torch.Tensor, what: str) -> torch.Tensor:
     if x.dim() != 2:
         raise RuntimeError(f"{what}: x must be 2-D [M, K]")
-    if x.stride(1) != 1:
-        x = x.contiguous()
-    return x
+    return _rows(x)
+
+
+def _rows(x: torch.Tensor) -> torch.Tensor:
+    """2-D *x* as the kernels read it: contiguous rows at one distance of at least their length.  Expanded and
+    overlapping rows (distance below the length) are copied."""
+    if x.stride(1) == 1 and x.stride(0) >= x.shape[1]:
+        return x
+    # a copy, or a view with the row distance spelt out: a single row is contiguous at any distance
+    return x.contiguous().view(-1).view(x.shape)
 
 
 def _tile_workspace(entry: str, m: int, n: int, k: int, device) -> tuple[int | None, int]:
@@ -901,8 +908,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
         raise RuntimeError(f"{what}: weight must be 1-D [H] matching x.size(1)")
     if x.dtype != weight.dtype:
         raise RuntimeError(f"{what}: x and weight must share dtype")
-    if x.stride(1) != 1:
-        x = x.contiguous()
+    x = _rows(x)
     weight = weight.contiguous()
     out = torch.empty((x.shape[0], x.shape[1]), device=x.device, dtype=x.dtype)
     _lib.call("npamd_rms_norm", x.data_ptr(), x.stride(0), weight.data_ptr(), out.data_ptr(), out.stride(0),

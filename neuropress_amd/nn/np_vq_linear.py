@@ -1072,9 +1072,7 @@ class NPVQLinear(nn.Module):
         perm = self._perm_i32(x.device) if self.column_perm is not None else None
         if x.device != self.packed_indices.device:
             raise RuntimeError(f"NPVQLinear: input on {x.device}, weights on {self.packed_indices.device}")
-        x2d = x.reshape(-1, self.in_features)
-        if x2d.stride(1) != 1:
-            x2d = x2d.contiguous()
+        x2d = kernels._rows(x.reshape(-1, self.in_features))
         try:
             # forward() has checked x's dtype and device; the other tensors come out of this
             # module's caches in the form the kernel reads.

@@ -136,3 +136,32 @@ def test_module_call_takes_the_long_way_when_something_stands_between(gpu, kind,
     assert torch.equal(copied(x), copied(x))
     with pytest.raises(TypeError):
         layer()
+
+
+def _small_bands(monkeypatch):
+    """Every band on small layers: 1-7 tokens sliced, to 32 GEMV, to 64 tile, then decode + product."""
+    monkeypatch.setattr(vqmod, "_SLICED_MIN_INDICES", 1)
+    for module, prefix in ((vqmod, "_TILE"), (qmod, "_Q_TILE")):
+        monkeypatch.setattr(module, prefix + "_MAX_TOKENS", 64)
+        monkeypatch.setattr(module, prefix + "_MIN_GRID_FRACTION", 0.0)
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["vq8", "vq8-perm", "vq16", "vq16-perm", "rvq", "q4", "norm"])
+def test_expanded_inputs_equal_their_copies(gpu, kind, act, monkeypatch):
+    """One row for a whole batch, one row per beam, one prompt for every beam: rows at distance 0 or at several, on the
+    first call and on the planned ones."""
+    from neuropress_amd.nn.np_rms_norm import NPRMSNorm
+
+    _small_bands(monkeypatch)
+    k = 512
+    layer = NPRMSNorm(torch.rand(k, generator=cases.gen(1)).to(act), 1e-5).to(gpu) if kind == "norm" else _layer(kind, gpu, act)
+    for rows in (3, 9, 20, 65):  # times two: every band
+        base = torch.randn(rows, k, generator=cases.gen(rows)).to(act).to(gpu)
+        for x in (base[:1].expand(2 * rows, k), base[:, None].expand(rows, 2, k), base[None].expand(2, rows, k),
+                  base[0].expand(1, k), base[0].expand(2, rows, k)):  # fmt: skip
+            for call in range(2):
+                y, ref = layer(x), layer(x.clone(memory_format=torch.contiguous_format))
+                assert y.shape == ref.shape
+                # the dense products may sum in another order
+                assert torch.equal(y, ref) if rows < 65 else torch.allclose(y, ref, rtol=2e-2, atol=2e-2), (rows, x.stride(), call)
