@@ -306,6 +306,7 @@ int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
 }
 
 constexpr int kDenseMaxSplits = 16;
+constexpr int64_t kDenseStrideMax = 1 << 22;  // elements between rows: offsets into a tile (256 rows) have 32 bits
 constexpr int kDenseMinSplitSteps = 4;  // 64-k steps of a part
 // What a split adds: the reduction kernel and the gap in front of it, and its bytes, us and us per MB.
 constexpr float kSplitFixed = 4.5f, kSplitPerMb = 0.45f;
@@ -360,7 +361,7 @@ extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64
   NPAMD_REQUIRE(ldx >= K && ldw >= K && ldy >= N && ldx % 8 == 0 && ldw % 8 == 0, "%s: bad row stride", what);
   if (M == 0 || N == 0) return NPAMD_OK;
   NPAMD_REQUIRE(x && w && y && (((uintptr_t)x | (uintptr_t)w) & 15) == 0, "%s: null or unaligned pointer", what);
-  NPAMD_REQUIRE(ldx < (1 << 22) && ldw < (1 << 22), "%s: row stride too large", what);
+  NPAMD_REQUIRE(ldx < kDenseStrideMax && ldw < kDenseStrideMax, "%s: row stride too large", what);
   hipStream_t st = (hipStream_t)stream;
   const int64_t room = workspace && ((uintptr_t)workspace & 3) == 0 ? workspace_bytes / ((int64_t)M * N * 4) : 1;
   DensePlan p = plan_dense(M, N, K, tuning().dense_tile, kDenseMaxSplits);
@@ -385,7 +386,7 @@ extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64
 // 38.4 / 26.2, 230 x 3152 x 7296 27.3 / 22.2, 460 x 2432 x 7936 36.1 / 29.4, 460 x 4096 x 14336 (54 GFLOP) 72 / 60, but
 // 945 x 4096 x 14336 110 / 108: from K = 8192 the line is 60 GFLOP.
 extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {
-  if (M < 1 || N < 1 || K < 64 || K % 64) return 0;
+  if (M < 1 || N < 1 || K < 64 || K % 64 || K >= kDenseStrideMax) return 0;
   const int forced = tuning().dense_tile;
   if (forced) return forced > 0;
   const double gflop = 2e-9 * M * N * K;

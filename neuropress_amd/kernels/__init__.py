@@ -867,8 +867,8 @@ def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = N
     x = _x2d(x, what)
     if x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype or w.dim() != 2 or w.shape[1] != x.shape[1]:
         raise RuntimeError(f"{what}: x and w must be float16 or bfloat16 [M, K] and [N, K]")
-    if x.stride(0) % 8 or x.data_ptr() % 16:
-        x = x.contiguous()
+    if x.stride(0) % 8 or x.data_ptr() % 16 or x.stride(0) >= 1 << 22:
+        x = torch.clone(x, memory_format=torch.contiguous_format)  # .contiguous() keeps dense rows at any address
     m, k = x.shape
     n = w.shape[0]
     w = w.contiguous()

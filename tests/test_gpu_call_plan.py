@@ -165,3 +165,15 @@ def test_expanded_inputs_equal_their_copies(gpu, kind, act, monkeypatch):
                 assert y.shape == ref.shape
                 # the dense products may sum in another order
                 assert torch.equal(y, ref) if rows < 65 else torch.allclose(y, ref, rtol=2e-2, atol=2e-2), (rows, x.stride(), call)
+
+
+@pytest.mark.parametrize("kind", ["vq8", "vq8-perm", "rvq", "q4"])
+def test_inputs_at_odd_addresses(gpu, kind, monkeypatch):
+    """Dense rows that do not start at a 16-byte boundary (a slice of a flat buffer), in every band."""
+    _small_bands(monkeypatch)
+    layer, k = _layer(kind, gpu, torch.float16), 512
+    for m in (20, 40, 130) if kind == "vq8-perm" else (2, 20, 40, 130):  # the GEMV that gathers columns refuses them
+        x = torch.randn(m * k + 1, generator=cases.gen(m)).half().to(gpu)[1:].view(m, k)
+        ref = layer(x.clone())
+        for call in range(2):
+            assert torch.allclose(layer(x), ref, rtol=2e-2, atol=2e-2), (m, call)

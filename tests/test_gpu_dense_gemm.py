@@ -66,6 +66,20 @@ def test_dense_gemm_parts_of_k(gpu, dense_tile, monkeypatch, tile, splits, act):
         assert bool(((y - ref).abs() <= tol * ref.abs() + 1e-4).all()), (tile, splits, m, n, k, float((y - ref).abs().max()))
 
 
+def test_dense_linear_copies_rows_the_kernel_does_not_take(gpu):
+    """Dense rows at an odd address, one row at an odd distance, rows far apart: each equals the product of the copy."""
+    from neuropress_amd import kernels
+
+    m, n, k = 40, 96, 128
+    w = (torch.randn(n, k, generator=cases.gen(3)) * 0.05).half().to(gpu)
+    flat = torch.randn(m * (k + 1) + 1, generator=cases.gen(4)).half().to(gpu)
+    far = torch.zeros(2, (1 << 22) + 8, dtype=torch.half, device=gpu)
+    far[:, :k] = flat[: 2 * k].view(2, k)
+    for x in (flat[1 : 1 + m * k].view(m, k), flat[: m * (k + 1)].view(m, k + 1)[:1, :k], far[:, :k]):
+        assert torch.equal(kernels.dense_linear(x, w), kernels.dense_linear(x.clone(memory_format=torch.contiguous_format), w))
+    assert not kernels.dense_preferred(1, 1, 1 << 22)
+
+
 def test_dense_gemm_refuses_what_it_does_not_take(gpu):
     from neuropress_amd import kernels
 
