@@ -174,7 +174,7 @@ class NPEmbedding(nn.Module):
         blob, scale, zp = self.u8_blob, self.scale, self.zero_point
         dtype, dim = self.out_dtype or scale.dtype, self.embedding_dim
         if ids.dtype != torch.int64 or ids.device != blob.device or dtype not in plans.DTYPE_CODES or blob.dim() != 2 or (
-            scale.dtype != torch.float16 or (zp is not None and zp.dtype != torch.float16)
+            blob.dtype != torch.uint8 or scale.dtype != torch.float16 or (zp is not None and zp.dtype != torch.float16)
             or blob.shape[1] * 8 != dim * self.nbits or scale.numel() * self.group_size != blob.shape[0] * dim
             or torch.cuda.is_current_stream_capturing()
         ):  # fmt: skip

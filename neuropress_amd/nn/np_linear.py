@@ -411,7 +411,8 @@ class NPLinear(nn.Module):
         if m < 1 or x.dtype not in plans.DTYPE_CODES or x.device != self.u8_blob.device or (
             self.u8_blob.dtype != torch.uint8 or self.scale.dtype != torch.float16
             or tuple(self.u8_blob.shape) != (n, k * self.nbits // 8) or self.scale.numel() * self.group_size != n * k
-            or (self.zero_point is not None and self.zero_point.numel() != self.scale.numel())
+            or (self.zero_point is not None
+                and (self.zero_point.numel() != self.scale.numel() or self.zero_point.dtype != torch.float16))
         ):  # fmt: skip
             return None
         plan = self._plan

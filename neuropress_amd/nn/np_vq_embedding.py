@@ -113,7 +113,7 @@ class NPVQEmbedding(nn.Module):
         table, cb = self.all_indices, self.proxy.centroids
         dtype = self.out_dtype or torch.float16
         if ids.dtype != torch.int64 or ids.device != table.device or dtype not in plans.DTYPE_CODES or table.dim() != 2 or (
-            cb.dtype != torch.float16 or table.shape[1] * cb.shape[1] != self.embedding_dim
+            cb.dtype != torch.float16 or table.dtype != torch.int16 or table.shape[1] * cb.shape[1] != self.embedding_dim
             or torch.cuda.is_current_stream_capturing()
         ):  # fmt: skip
             return None

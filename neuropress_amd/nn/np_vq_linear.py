@@ -794,7 +794,7 @@ class NPVQLinear(nn.Module):
         if plan is not None and band == "sliced" and (band, x.dtype) in plan.names:
             return kernels.SlicedCallPlan(plan).run(x)  # the wrapper functions have been replaced
         if m < 1 or band == "torch" or (band == "tile" and _tile_failed) or x.dtype not in plans.DTYPE_CODES or (
-            x.device != self.packed_indices.device or self.packed_indices.dtype != torch.uint8
+            x.device != self.packed_indices.device or not self._kernel_types(band)
         ):  # fmt: skip
             return None
         if plan is None:
@@ -804,6 +804,16 @@ class NPVQLinear(nn.Module):
         self._add_route(plan, x.dtype, m, band)
         self._plan = plan
         return None if plan.wrapped() else plan.run(x)
+
+    def _kernel_types(self, band: str) -> bool:
+        """Whether the buffers have the types the kernels of *band* read them as.  ``model.to(dtype)`` casts codebooks and
+        row tensors; the bands of plain layers that look rows up in a copy of x's type take any codebook."""
+        if self.packed_indices.dtype != torch.uint8:
+            return False
+        if not self.is_residual:
+            return band != "dense" or self.proxy.centroids.dtype == torch.float16
+        f16 = (self.proxy.centroids, self._res_centroids(), self.row_scale, self.row_bias)
+        return self._res_stream().dtype == torch.uint8 and all(t is None or t.dtype == torch.float16 for t in f16)
 
     def _new_plan(self):
         from ..kernels import plans

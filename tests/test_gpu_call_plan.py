@@ -177,3 +177,24 @@ def test_inputs_at_odd_addresses(gpu, kind, monkeypatch):
         ref = layer(x.clone())
         for call in range(2):
             assert torch.allclose(layer(x), ref, rtol=2e-2, atol=2e-2), (m, call)
+
+
+@pytest.mark.parametrize("cast", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["vq8", "vq16", "rvq"])
+def test_cast_codebooks(gpu, kind, cast, monkeypatch):
+    """``model.to(dtype)`` on a lowered model casts the codebooks: the bands that look rows up in a copy of the
+    activations' type serve them, the decodes read fp16 and say so."""
+    _small_bands(monkeypatch)
+    layer, k = _layer(kind, gpu, torch.float16), 512
+    xs = {m: torch.randn(m, k, generator=cases.gen(m)).half().to(gpu) for m in (2, 20, 40, 130)}
+    before = {m: layer(x) for m, x in xs.items()}
+    for module in (layer, layer.proxy, layer.residual_proxy):
+        if module is not None:
+            module.to(cast)
+    for m, x in xs.items():
+        for call in range(2):
+            if kind == "rvq" or m == 130:
+                with pytest.raises(RuntimeError, match="must be float16"):
+                    layer(x)
+            else:
+                assert torch.allclose(layer(x), before[m], rtol=2e-2, atol=2e-2), (m, call)
