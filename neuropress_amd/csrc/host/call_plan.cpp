@@ -196,7 +196,7 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
 
   if (t.kind == kVqDense || t.kind == kRvqDense || t.kind == kQDense) {
     const int code = dtype_code(t.out);
-    if (t.own && (ldx % 8 || ((uintptr_t)x.const_data_ptr() & 15) || (x_in.requires_grad() && c10::GradMode::is_enabled()))) return false;
+    if (t.own && (ldx % 8 || ((uintptr_t)x.const_data_ptr() & 15))) return false;
     at::Tensor w = empty({t.n, t.k}, t.out, device);
     int rc;
     if (t.kind == kVqDense)
@@ -331,9 +331,14 @@ bool rows_at_one_stride(const at::Tensor& x, int64_t* ldx) {
   return row >= x.size(-1);
 }
 
+// Whether torch records what is done to x.  The kernels' outputs carry no gradient: no plan issues such a call, and the
+// module decides between its kernels and torch's own operations.
+bool tracked(const at::Tensor& x) { return x.requires_grad() && c10::GradMode::is_enabled(); }
+
 PyObject* run(Plan* p, PyObject* xo) {
   if (!THPVariable_CheckExact(xo)) Py_RETURN_NONE;
   const at::Tensor& x = THPVariable_Unpack(xo);
+  if (tracked(x)) Py_RETURN_NONE;
   const int code = dtype_code(x.scalar_type());
   const int64_t dims = x.dim();
   if (code < 0 || dims < 1 || !x.is_cuda() || x.get_device() != p->device) Py_RETURN_NONE;
@@ -743,7 +748,16 @@ PyObject* row_distance(PyObject*, PyObject* xo) {
   return PyLong_FromLongLong(ldx);
 }
 
+PyObject* tracked_tensor(PyObject*, PyObject* xo) {
+  if (!THPVariable_Check(xo)) {
+    PyErr_SetString(PyExc_TypeError, "tracked() takes a tensor");
+    return nullptr;
+  }
+  return PyBool_FromLong(tracked(THPVariable_Unpack(xo)));
+}
+
 PyMethodDef module_methods[] = {
+    {"tracked", tracked_tensor, METH_O, "tracked(x): whether torch records what is done to x, so that no plan issues the call"},
     {"row_distance", row_distance, METH_O, "row_distance(x): elements between the rows a plan would read, or None"},
     {"set_module_class", set_module_class, METH_VARARGS, "set_module_class(torch.nn.Module, its call in Python)"},
     {"set_workspaces", set_workspaces, METH_VARARGS, "set_workspaces(dict, drop): the slice-list GEMV's scratch buffers"},

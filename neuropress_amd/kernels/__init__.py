@@ -854,6 +854,12 @@ def warn_kernel_fallback(kernel: str, fallback: str, exc: BaseException) -> None
 # ---------------------------------------------------------------------------
 
 
+def tracked(x: torch.Tensor) -> bool:
+    """Whether torch records what is done to *x* (a gradient is asked for): the kernels' outputs carry none, so such calls go
+    through torch's own operations wherever the library's product is the one to take."""
+    return _lib.host().tracked(x)
+
+
 def dense_preferred(m: int, n: int, k: int) -> bool:
     """Whether :func:`dense_linear` is the better choice for this shape against ``F.linear``."""
     return bool(_lib.load().npamd_dense_gemm_preferred(int(m), int(n), int(k)))

@@ -152,14 +152,16 @@ _TIGHT_GRID_FRACTION: float = 0.66
 
 def tile_band_ok(
     m: int, n: int, k: int, cus: int, min_fraction: float, split_max_tokens: int, long_k: int,
-    small_max_tokens: int = 1 << 30, half_ok: bool = False, tight_k: int = 1 << 30,
+    small_max_tokens: int = 1 << 30, half_ok: bool = False, tight_k: int = 1 << 30, library: bool = False,
 ) -> bool:
     """Whether the tile-decode GEMM has enough workgroups for ``m`` tokens on an
     ``n x k`` layer.  Mirrors the kernel's own plan: without a split when the
     (64 columns x up to 384 rows) grid covers ``min_fraction`` of ``cus`` compute
     units; otherwise up to 16 reduction splits of at least 512 input features.  *half_ok*: a grid of more than half
     the compute units, too large to split, will do.  From *tight_k* input features on 0.66 of them will do for a split
-    grid (86 to 89 column blocks, in two parts).
+    grid (86 to 89 column blocks, in two parts).  *library*: against decode + the library's product, the alternative of
+    calls that torch has to follow, as measured with int4 weights: 4096 x 4096 24-31 us against 37-45 from 128 to 256
+    tokens; 1024 x 4096 (not enough workgroups even when split) 17-19 against 16-20.
 
     Measured, us, tile GEMM / decode + dense product: 3008 x 2240 with a 4096-row codebook 13.7 / 14.1 at 33 tokens,
     14.4 / 14.2 at 64, 17.5 / 15.2 at 128, with int4 weights 15.8 / 13.1 at 33; 6144 x 1024 int4 13.9 / 10.9 at 33;
@@ -170,6 +172,8 @@ def tile_band_ok(
     if blocks >= min_fraction * cus or (half_ok and 2 * blocks > cus):
         return True
     splits = max(1, min(cus // blocks, k // 512, 16))
+    if library:
+        return splits * blocks >= min_fraction * cus and (m <= split_max_tokens or k >= long_k)
     if splits * blocks < min_fraction * cus and not (splits > 1 and k >= tight_k and splits * blocks >= _TIGHT_GRID_FRACTION * cus):
         return False
     if n * k < _SMALL_LAYER_WEIGHTS and m > small_max_tokens:

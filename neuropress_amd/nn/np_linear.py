@@ -53,6 +53,10 @@ _Q_TILE_WIDE_MIN_FEATURES: int = 8192
 # 8192 x 2048 24 vs 21 at 128; 1024 x 4096 (not enough workgroups even when split) 17 vs 14 us at 64.
 _Q_TILE_MIN_GRID_FRACTION: float = 0.7
 _Q_TILE_SPLIT_MAX_TOKENS: int = 144
+# The same against decode + the library's product, which calls that record a gradient take: 4096 x 4096 24-31 vs 37-45 us
+# from 128 to 256 tokens, 39-41 vs 39-40 us at 320-384.  Where it serves a call, gradients flow: the line is part of
+# what the module does and stays where it is.
+_Q_TILE_SPLIT_LIBRARY_MAX_TOKENS: int = 256
 _Q_TILE_SPLIT_LONG_K: int = 8192
 # Grids of more than half the compute units that are too large to split (8193 to 11456 output features): the fused GEMM
 # from this K on, below it up to 256 tokens without zero points.  Decode + GEMM / fused, us at 36 / 100 / 256 / 384 tokens:
@@ -323,11 +327,14 @@ class NPLinear(nn.Module):
             self._derived["mfma_layer"] = ok
         return ok
 
-    def _tile_grid_fills_gpu(self, x: torch.Tensor, m: int) -> bool:
+    def _tile_grid_fills_gpu(self, x: torch.Tensor, m: int, tracked: bool = False) -> bool:
         cus = self._derived.get("cus")
         if cus is None:
             cus = torch.cuda.get_device_properties(x.device).multi_processor_count
             self._derived["cus"] = cus
+        if tracked:
+            return tile_band_ok(m, self.out_features, self.in_features, cus, _Q_TILE_MIN_GRID_FRACTION,
+                                _Q_TILE_SPLIT_LIBRARY_MAX_TOKENS, _Q_TILE_SPLIT_LONG_K, library=True)  # fmt: skip
         return tile_band_ok(
             m, self.out_features, self.in_features, cus,
             _Q_TILE_MIN_GRID_FRACTION, _Q_TILE_SPLIT_MAX_TOKENS, _Q_TILE_SPLIT_LONG_K, _Q_FUSED_WIDE_MAX_TOKENS,
@@ -361,8 +368,9 @@ class NPLinear(nn.Module):
 
         m = x.numel() // self.in_features
         try:
-            band = self._band(x, m)
-            if not torch.cuda.is_current_stream_capturing():
+            tracked = kernels.tracked(x)
+            band = self._band(x, m, tracked)
+            if not tracked and not torch.cuda.is_current_stream_capturing():
                 y = self._planned(x, m, band)
                 if y is not None:
                     return y
@@ -377,7 +385,7 @@ class NPLinear(nn.Module):
                 raise
             kernels.warn_kernel_fallback("q_linear", "torch dequant + matmul", exc)
             return self._forward_compile(x)
-        if self._own_product(m, x.dtype) and not (x.requires_grad and torch.is_grad_enabled()):
+        if self._own_product(m, x.dtype) and not tracked:
             return kernels.dense_linear(x.reshape(-1, self.in_features), w, self._bias_f32()).reshape(*x.shape[:-1], self.out_features)
         return F.linear(x, w, self._bias_as(x.dtype))
 
@@ -387,8 +395,9 @@ class NPLinear(nn.Module):
 
         return dtype in (torch.float16, torch.bfloat16) and kernels.dense_preferred(m, self.out_features, self.in_features)
 
-    def _band(self, x: torch.Tensor, m: int) -> str:
-        """Which kernel serves a call of *m* tokens: ``fused`` (GEMV), ``tile`` (fused GEMM) or ``dense`` (decode + GEMM)."""
+    def _band(self, x: torch.Tensor, m: int, tracked: bool = False) -> str:
+        """Which kernel serves a call of *m* tokens: ``fused`` (GEMV), ``tile`` (fused GEMM) or ``dense`` (decode + GEMM).
+        *tracked* (``kernels.tracked(x)``): the dense product is the library's, and so are the limits against it."""
         # Layers the MFMA kernels do not take (1 / 2 / 8 bits, odd group sizes) would run an
         # element-wise kernel, slower at every token count than decoding once and calling the
         # dense GEMM (14336 x 4096, 8 bits: 99 us against 57 us at one token, 452 against 57 at 16).
@@ -401,7 +410,7 @@ class NPLinear(nn.Module):
             limit = max(limit, _Q_TILE_LONG_K_MAX_TOKENS)
         if limit > 0 and max(self.in_features, self.out_features) >= _Q_TILE_WIDE_MIN_FEATURES:
             limit = max(limit, _Q_TILE_WIDE_MAX_TOKENS)
-        return "tile" if m <= limit and self._tile_grid_fills_gpu(x, m) else "dense"
+        return "tile" if m <= limit and self._tile_grid_fills_gpu(x, m, tracked) else "dense"
 
     def _planned(self, x: torch.Tensor, m: int, band: str):
         """Add this call to the layer's plan and let the plan issue it; None where it cannot."""

@@ -135,6 +135,11 @@ _TILE_WIDE_TINY_WEIGHTS: int = 5_000_000  # below: 32 tokens, where the GEMV end
 _TILE_WIDE_LONG_MAX_TOKENS: int = 256  # _MID_LAYER_WEIGHTS and K of 4096, or _SMALL_LAYER_WEIGHTS and K of _TILE_SPLIT_LONG_K
 _TILE_WIDE_MID_MAX_TOKENS: int = 128  # _SMALL_LAYER_WEIGHTS and K of 4096
 _TILE_WIDE_SMALL_MAX_TOKENS: int = 64  # all others
+# Against decode + the library's product, which calls that record a gradient take: layers of _TILE_WIDE_BROAD_WEIGHTS, half
+# of it below (us at 128 / 256 / 384 tokens, tile against decode + library product: 6144 x 4096 32 / 41 / 56 against 47 / 61 / 55,
+# 8192 x 2048 28 / 34 / 46 against 34 / 40 / 38; 1024 x 4096 18 / 24 / 29 against 20 / 21 / 22).  Where that product
+# serves a call, gradients flow: the line is part of what the module does and stays where it is.
+_TILE_WIDE_LIBRARY_MAX_TOKENS: int = 256
 
 # The tile GEMM gives each workgroup 64 output columns (and up to 384 rows).  When
 # that grid covers less than this fraction of the compute units the kernel splits
@@ -733,9 +738,12 @@ class NPVQLinear(nn.Module):
     _planned_forward = forward  # module(x) may go straight to the plan (kernels/plans.py)
 
     def _forward(self, x: torch.Tensor) -> torch.Tensor:
+        from .. import kernels
+
         m = x.numel() // self.in_features
-        band = self._band(x, m)
-        if x.is_cuda and not torch.cuda.is_current_stream_capturing():
+        tracked = x.is_cuda and self.backend in _FUSED_BACKENDS and kernels.tracked(x)
+        band = self._band(x, m, tracked)
+        if x.is_cuda and not tracked and not torch.cuda.is_current_stream_capturing():
             y = self._planned(x, m, band)
             if y is not None:
                 return y
@@ -759,9 +767,12 @@ class NPVQLinear(nn.Module):
             return self._forward_compile(x)
         return self._forward_default(x)
 
-    def _band(self, x: torch.Tensor, m: int) -> str:
+    def _band(self, x: torch.Tensor, m: int, tracked: bool = False) -> str:
         """Which kernel serves a call of *m* tokens: ``sliced``, ``gemv_perm`` (the GEMV that gathers x's columns),
-        ``fused`` (the backend's GEMV), ``tile``, ``dense`` (decode + GEMM) or ``torch``."""
+        ``fused`` (the backend's GEMV), ``tile``, ``dense`` (decode + GEMM) or ``torch``.
+
+        *tracked* (``kernels.tracked(x)``): the dense product is the library's, columns are gathered by torch and none
+        are padded; the limits are those against that.  What it serves carries gradients, the other kernels do not."""
         if self.backend not in _FUSED_BACKENDS:
             return "torch"
         if x.dtype not in (torch.float16, torch.bfloat16):
@@ -770,13 +781,13 @@ class NPVQLinear(nn.Module):
             return "sliced"
         if self.column_perm is not None and self._perm_fusable(x, m):
             return "gemv_perm"
-        if x.is_cuda and not self._mfma_layer():
+        if x.is_cuda and (not self._mfma_layer() or (tracked and self._kernel_k() != self.in_features)):
             # Shapes without an MFMA kernel (vector lengths other than 8 and 4, K not a
             # multiple of 64): the element-wise GEMV is slower than decoding once and calling
             # the dense GEMM at every token count (14336 x 4096: 99 us against 57 us at one token).
             return "dense"
         if m > self._gemv_max_tokens(m):
-            if self.backend != VQBackend.CUDA_LUT and m <= self._tile_max_tokens() and self._tile_band_ok(x, m):
+            if self.backend != VQBackend.CUDA_LUT and m <= self._tile_max_tokens(tracked) and self._tile_band_ok(x, m, tracked):
                 return "tile"
             return "dense"
         return "fused"
@@ -1117,13 +1128,16 @@ class NPVQLinear(nn.Module):
             and self.proxy.num_centroids * self.vector_len * 2 > 65536
         )
 
-    def _tile_max_tokens(self) -> int:
+    def _tile_max_tokens(self, tracked: bool = False) -> int:
         """Upper end of the tile-decode GEMM band for this layer."""
         if _TILE_MAX_TOKENS > 0 and self._wide_tile_layer():
             weights = self.in_features * self.out_features
             k = self.in_features
             if weights >= _TILE_WIDE_MIN_WEIGHTS:
                 return max(_TILE_MAX_TOKENS, _TILE_WIDE_MAX_TOKENS)
+            if tracked:
+                broad = weights >= _TILE_WIDE_BROAD_WEIGHTS
+                return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LIBRARY_MAX_TOKENS if broad else _TILE_WIDE_LIBRARY_MAX_TOKENS // 2)
             if weights >= _MID_LAYER_WEIGHTS and k >= 4096:
                 return _TILE_WIDE_MAX_TOKENS if k >= _MID_LAYER_K else min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS)
             if weights >= _TILE_WIDE_BROAD_WEIGHTS and self.out_features >= _TILE_WIDE_BROAD_FEATURES:
@@ -1135,7 +1149,7 @@ class NPVQLinear(nn.Module):
             return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_SMALL_MAX_TOKENS)
         return _TILE_MAX_TOKENS
 
-    def _tile_band_ok(self, x: torch.Tensor, m: int) -> bool:
+    def _tile_band_ok(self, x: torch.Tensor, m: int, tracked: bool = False) -> bool:
         """True when the tile GEMM's grid (64 columns x up to 384 rows per workgroup,
         times the reduction splits the kernel adds for layers with few output
         features) covers at least ``_TILE_MIN_GRID_FRACTION`` of the compute units."""
@@ -1149,6 +1163,9 @@ class NPVQLinear(nn.Module):
         if cus is None:
             cus = torch.cuda.get_device_properties(x.device).multi_processor_count
             self._derived["cus"] = cus
+        if tracked:
+            return tile_band_ok(m, self.out_features, self.in_features, cus, _TILE_MIN_GRID_FRACTION, _TILE_SPLIT_MAX_TOKENS,
+                                _TILE_SPLIT_LONG_K, library=True)  # fmt: skip
         return tile_band_ok(
             m, self.out_features, self._kernel_k(), cus,
             _TILE_MIN_GRID_FRACTION, _TILE_SPLIT_MAX_TOKENS, _TILE_SPLIT_LONG_K,
@@ -1205,7 +1222,7 @@ class NPVQLinear(nn.Module):
         from .. import kernels
 
         try:
-            own = self._own_product(x.numel() // self.in_features, x.dtype) and not (x.requires_grad and torch.is_grad_enabled())
+            own = self._own_product(x.numel() // self.in_features, x.dtype) and not kernels.tracked(x)
             if self.is_residual:
                 w = kernels.rvq_dequant(
                     self.packed_indices, self.bits, self._res_stream(), self._res_bits(),

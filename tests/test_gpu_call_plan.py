@@ -198,3 +198,69 @@ def test_cast_codebooks(gpu, kind, cast, monkeypatch):
                     layer(x)
             else:
                 assert torch.allclose(layer(x), before[m], rtol=2e-2, atol=2e-2), (m, call)
+
+
+@pytest.fixture
+def dense_tile(monkeypatch):
+    from neuropress_amd import _lib
+
+    def force(tile):
+        monkeypatch.setenv("NPAMD_DENSE_TILE", str(tile))
+        _lib.load().npamd_diag_reload_tuning()
+
+    yield force
+    monkeypatch.delenv("NPAMD_DENSE_TILE", raising=False)
+    _lib.load().npamd_diag_reload_tuning()
+
+
+def _dense_cases():
+    # name, format, n, k, tokens: calls the library's product serves when a gradient is asked for
+    return [
+        ("own product", "vq8", 96, 512, 130), ("own product", "q4", 96, 512, 130), ("own product", "rvq", 96, 512, 130),
+        ("library product", "vq8-perm", 96, 512, 130), ("own product", "vq8-perm", 96, 512, 130), ("odd K, gemv", "vq8", 96, 200, 3), ("odd K, tile", "vq8-perm", 96, 200, 40),
+        ("half grid", "vq8", 8320, 512, 100), ("half grid", "q4", 8320, 512, 100), ("half grid", "rvq", 8320, 512, 100),
+        ("tight grid", "vq8", 5504, 2048, 40), ("tight grid", "q4", 5504, 4096, 40), ("long K", "vq8", 2048, 6144, 200),
+        ("wide tile", "vq16", 3072, 4096, 200),
+    ]  # fmt: skip
+
+
+def _weight_layer(kind, n, k, gpu):
+    """A layer and its dense weight in float64."""
+    g = cases.gen(n + k)
+    if kind == "q4":
+        Q = cases.q4_layer(5, n, k)
+        layer = NPLinear(Q["blob"], Q["scale"], n, k, 32, 4, "sym", "cuda").to(gpu)
+        return layer, (Q["codes"].double() - 8) * Q["scale"].double().reshape(n, -1).repeat_interleave(32, 1)
+    if kind == "rvq":
+        R = cases.rvq_layer(6, n, k, nc_main=4096, zipf=False)
+        proxies = VQProxy(R["cbm"]).to(gpu), VQProxy(R["cbr"]).to(gpu)
+        layer = NPVQLinear(proxies[0], R["pm"], R["bm"], n, k, 8, "cuda_wmma", residual_proxy=proxies[1], packed_residual=R["pr"],
+                           row_scale=R["scale"], row_bias=R["wbias"]).to(gpu)  # fmt: skip
+        w = ((R["cbm"][R["im"]] + R["cbr"][R["ir"]]).reshape(n, k) * R["scale"][:, None] + R["wbias"][:, None]).double()
+        return layer, w
+    nc, bits = {"vq8": (256, 8), "vq16": (20000, 16)}[kind.split("-")[0]]
+    V = cases.vq_layer(7, n, k, nc, bits=bits, std=0.05)
+    perm = torch.randperm(k, generator=g) if kind.endswith("perm") else None
+    layer = NPVQLinear(VQProxy(V["cb"]).to(gpu), V["packed"], bits, n, k, 8, "cuda_wmma", column_perm=perm).to(gpu)
+    w = V["cb"][V["idx"]].reshape(n, k).double()
+    return layer, w if perm is None else torch.zeros_like(w).index_copy_(1, perm, w)  # y = x[:, perm] @ w.T
+
+
+@pytest.mark.parametrize("name,kind,n,k,m", _dense_cases())
+def test_gradients_where_the_library_product_had_them(gpu, dense_tile, name, kind, n, k, m):
+    if name == "library product":
+        dense_tile(-1)  # never the package's own
+    layer, w = _weight_layer(kind, n, k, gpu)
+    x = torch.randn(m, k, generator=cases.gen(m)).half().to(gpu)
+    dy = torch.randn(m, n, generator=cases.gen(m + 1)).half()
+    ref = (dy.double() @ w).float()
+    for call in range(2):  # without a plan, and with one the call below has made
+        leaf = x.clone().requires_grad_()
+        y = layer(leaf)
+        assert y.requires_grad
+        y.backward(dy.to(gpu))
+        err = (leaf.grad.float().cpu() - ref).norm() / ref.norm()
+        assert float(err) < 4e-3, (call, float(err))  # the rounding of dy @ w to fp16, of w in fp16
+        with torch.no_grad():
+            assert torch.allclose(layer(leaf), y, rtol=2e-2, atol=2e-2) and not layer(leaf).requires_grad
+        assert not layer(x).requires_grad
