@@ -22,6 +22,7 @@
 #include <ATen/ops/index_select.h>
 #include <ATen/ops/linear.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -331,9 +332,18 @@ bool rows_at_one_stride(const at::Tensor& x, int64_t* ldx) {
   return row >= x.size(-1);
 }
 
-// Whether torch records what is done to x.  The kernels' outputs carry no gradient: no plan issues such a call, and the
+// Whether torch follows what is done to x: it records a gradient or a trace, x carries a tangent, is a wrapper (vmap, grad
+// and jvp of torch.func; a tensor without storage of its own or one that is read negated) or not strided, or a dispatch
+// mode looks on.  The kernels read addresses and their outputs carry nothing: no plan issues such a call, and the
 // module decides between its kernels and torch's own operations.
-bool tracked(const at::Tensor& x) { return x.requires_grad() && c10::GradMode::is_enabled(); }
+bool tracked(const at::Tensor& x) {
+  constexpr c10::DispatchKeySet own = c10::autograd_dispatch_keyset | c10::autocast_dispatch_keyset |
+                                      c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView);
+  const c10::DispatchKeySet keys = x.key_set() - own;
+  if (keys != c10::DispatchKeySet(c10::DispatchKey::CUDA) && keys != c10::DispatchKeySet(c10::DispatchKey::CPU)) return true;
+  return (x.requires_grad() && c10::GradMode::is_enabled()) || x._fw_grad(0).defined() || torch::jit::tracer::isTracing() ||
+         c10::impl::TorchDispatchModeTLS::any_modes_set();
+}
 
 PyObject* run(Plan* p, PyObject* xo) {
   if (!THPVariable_CheckExact(xo)) Py_RETURN_NONE;
@@ -757,7 +767,7 @@ PyObject* tracked_tensor(PyObject*, PyObject* xo) {
 }
 
 PyMethodDef module_methods[] = {
-    {"tracked", tracked_tensor, METH_O, "tracked(x): whether torch records what is done to x, so that no plan issues the call"},
+    {"tracked", tracked_tensor, METH_O, "tracked(x): whether torch follows what is done to x, so that no plan issues the call"},
     {"row_distance", row_distance, METH_O, "row_distance(x): elements between the rows a plan would read, or None"},
     {"set_module_class", set_module_class, METH_VARARGS, "set_module_class(torch.nn.Module, its call in Python)"},
     {"set_workspaces", set_workspaces, METH_VARARGS, "set_workspaces(dict, drop): the slice-list GEMV's scratch buffers"},

@@ -264,3 +264,30 @@ def test_gradients_where_the_library_product_had_them(gpu, dense_tile, name, kin
         with torch.no_grad():
             assert torch.allclose(layer(leaf), y, rtol=2e-2, atol=2e-2) and not layer(leaf).requires_grad
         assert not layer(x).requires_grad
+
+
+@pytest.mark.parametrize("name,kind,n,k,m", _dense_cases()[:10])
+def test_forward_mode_and_vmap_where_the_library_product_had_them(gpu, dense_tile, name, kind, n, k, m):
+    import torch.autograd.forward_ad as fwad
+    from torch.utils.flop_counter import FlopCounterMode
+
+    if name == "library product":
+        dense_tile(-1)  # never the package's own
+
+    layer, w = _weight_layer(kind, n, k, gpu)
+    x, t = (torch.randn(2, m, k, generator=cases.gen(m + i)).half().to(gpu) for i in range(2))
+    tangent, primal = ((v.cpu().double() @ w.T).float() for v in (t, x))
+
+    def close(a, ref):
+        assert float((a.float().cpu() - ref).norm() / ref.norm()) < 4e-3
+
+    for call in range(2):
+        with fwad.dual_level():
+            out = fwad.unpack_dual(layer(fwad.make_dual(x[0], t[0])))
+            assert out.tangent is not None
+            close(out.tangent, tangent[0])
+        close(torch.func.vmap(layer)(x), primal)
+        with FlopCounterMode(display=False) as flops:
+            layer(x[0])
+        assert flops.get_total_flops() == 2 * m * n * k
+        close(layer(x[0]), primal[0])  # makes the plan the second pass meets

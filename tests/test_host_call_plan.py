@@ -35,3 +35,32 @@ def test_rows_read_in_place_are_the_rows_of_x(size, stride):
         assert ldx is None
     else:
         assert ldx >= x.shape[-1] and rows == [r * ldx for r in range(len(rows))]
+
+
+def test_tracked_tensors():
+    """Calls that torch follows are not for a plan: it would drop what is followed, or read a tensor without storage."""
+    import torch.autograd.forward_ad as fwad
+    from torch.utils.flop_counter import FlopCounterMode
+
+    tracked = _lib.host().tracked
+    x = torch.randn(3, 8)
+    assert not tracked(x) and not tracked(x[1:, ::2]) and not tracked(x.half())
+    with torch.inference_mode():
+        assert not tracked(x) and not tracked(torch.ones(2))
+    assert not tracked(torch.nn.Parameter(x, requires_grad=False))
+    leaf = x.clone().requires_grad_()
+    assert tracked(leaf) and tracked(leaf * 2)
+    with torch.no_grad():
+        assert not tracked(leaf)
+    with fwad.dual_level():
+        assert tracked(fwad.make_dual(x, x)) and not tracked(x)
+    assert not tracked(x)
+    seen = []
+    torch.func.vmap(lambda t: seen.append(tracked(t)) or t)(x)
+    torch.func.grad(lambda t: seen.append(tracked(t)) or t.sum())(x)
+    torch.func.jvp(lambda t: seen.append(tracked(t)) or t, (x,), (x,))
+    torch.jit.trace(lambda t: seen.append(tracked(t)) or t + 1, (x,), check_trace=False)
+    with FlopCounterMode(display=False):
+        seen.append(tracked(x))
+    seen += [tracked(torch._neg_view(x)), tracked(x.to_sparse()), tracked(x.to_mkldnn())]
+    assert seen == [True] * len(seen)
