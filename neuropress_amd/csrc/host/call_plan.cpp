@@ -24,6 +24,7 @@
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -345,7 +346,7 @@ bool tracked(const at::Tensor& x) {
          c10::impl::TorchDispatchModeTLS::any_modes_set();
 }
 
-PyObject* run(Plan* p, PyObject* xo) {
+PyObject* issue_planned(Plan* p, PyObject* xo) {
   if (!THPVariable_CheckExact(xo)) Py_RETURN_NONE;
   const at::Tensor& x = THPVariable_Unpack(xo);
   if (tracked(x)) Py_RETURN_NONE;
@@ -367,14 +368,24 @@ PyObject* run(Plan* p, PyObject* xo) {
   const Route route = it->second;
   const Template& t = (*p->templates)[(size_t)route.tmpl];
   if (t.k_in != k) Py_RETURN_NONE;
+  at::Tensor y;
+  if (!issue(t, route, x, m, ldx, p->device, &y)) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(y));
+}
+
+// Runs fn; a C++ exception becomes the Python one torch makes of it (torch.OutOfMemoryError for an allocation that failed).
+template <class Fn>
+PyObject* translated(Fn&& fn) {
   try {
-    at::Tensor y;
-    if (!issue(t, route, x, m, ldx, p->device, &y)) Py_RETURN_NONE;
-    return THPVariable_Wrap(std::move(y));
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return fn();
+  } catch (...) {
+    torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
+}
+
+PyObject* run(Plan* p, PyObject* xo) {
+  return translated([&] { return issue_planned(p, xo); });
 }
 
 // What torch.nn.Module.__call__ looks at before it calls forward: hooks of the module and of all modules, a compiled
@@ -395,8 +406,10 @@ PyObject* plan_call(PyObject* self, PyObject* const* args, size_t nargsf, PyObje
     PyErr_SetString(PyExc_TypeError, "CallPlan(module, x)");
     return nullptr;
   }
-  if (!p->guarded || stale(p, args[0]) || wrapped(p)) Py_RETURN_NONE;
-  return run(p, args[1]);
+  return translated([&]() -> PyObject* {
+    if (!p->guarded || stale(p, args[0]) || wrapped(p)) Py_RETURN_NONE;
+    return issue_planned(p, args[1]);
+  });
 }
 
 void clear_guard(Guard& g, bool owns_dict) {
@@ -577,9 +590,11 @@ PyObject* plan_source(PyObject* self, PyObject* t) {
     PyErr_SetString(PyExc_TypeError, "source() takes a tensor");
     return nullptr;
   }
-  const at::Tensor& v = THPVariable_Unpack(t);
-  reinterpret_cast<Plan*>(self)->sources->push_back({v, v.const_data_ptr(), version_of(v)});
-  Py_RETURN_NONE;
+  return translated([&]() -> PyObject* {
+    const at::Tensor& v = THPVariable_Unpack(t);
+    reinterpret_cast<Plan*>(self)->sources->push_back({v, v.const_data_ptr(), version_of(v)});
+    Py_RETURN_NONE;
+  });
 }
 
 // hold(object): something the template's addresses point into that is not a tensor
@@ -645,7 +660,7 @@ PyObject* plan_route(PyObject* self, PyObject* args) {
 
 PyObject* plan_stale(PyObject* self, PyObject* module) {
   Plan* p = reinterpret_cast<Plan*>(self);
-  return PyBool_FromLong(!p->guarded || stale(p, module));
+  return translated([&] { return PyBool_FromLong(!p->guarded || stale(p, module)); });
 }
 
 PyObject* plan_wrapped(PyObject* self, PyObject*) { return PyBool_FromLong(wrapped(reinterpret_cast<Plan*>(self))); }
@@ -695,13 +710,14 @@ PyObject* module_call(PyObject*, PyObject* const* args, size_t nargsf, PyObject*
     PyObject* plan = dict && *dict ? PyDict_GetItemWithError(*dict, g_plan_key) : nullptr;
     if (plan && Py_TYPE(plan) == &plan_type) {
       Plan* p = reinterpret_cast<Plan*>(plan);
-      if (p->guarded && p->direct_type && direct(p, args[0]) && !stale(p, args[0]) && !wrapped(p)) {
-        Py_INCREF(plan);  // the module may drop it meanwhile
-        PyObject* y = run(p, args[1]);
-        Py_DECREF(plan);
-        if (y != Py_None) return y;
-        Py_DECREF(y);
-      }
+      Py_INCREF(plan);  // the module may drop it meanwhile
+      PyObject* y = translated([&]() -> PyObject* {
+        if (!p->guarded || !p->direct_type || !direct(p, args[0]) || stale(p, args[0]) || wrapped(p)) Py_RETURN_NONE;
+        return issue_planned(p, args[1]);
+      });
+      Py_DECREF(plan);
+      if (y != Py_None) return y;
+      Py_DECREF(y);
     } else if (!plan && PyErr_Occurred()) {
       return nullptr;
     }
@@ -752,10 +768,12 @@ PyObject* row_distance(PyObject*, PyObject* xo) {
     PyErr_SetString(PyExc_TypeError, "row_distance() takes a tensor of one dimension or more");
     return nullptr;
   }
-  const at::Tensor& x = THPVariable_Unpack(xo);
-  int64_t ldx = x.size(-1);
-  if (!x.is_contiguous() && !rows_at_one_stride(x, &ldx)) Py_RETURN_NONE;
-  return PyLong_FromLongLong(ldx);
+  return translated([&]() -> PyObject* {
+    const at::Tensor& x = THPVariable_Unpack(xo);
+    int64_t ldx = x.size(-1);
+    if (!x.is_contiguous() && !rows_at_one_stride(x, &ldx)) Py_RETURN_NONE;
+    return PyLong_FromLongLong(ldx);
+  });
 }
 
 PyObject* tracked_tensor(PyObject*, PyObject* xo) {
@@ -763,7 +781,7 @@ PyObject* tracked_tensor(PyObject*, PyObject* xo) {
     PyErr_SetString(PyExc_TypeError, "tracked() takes a tensor");
     return nullptr;
   }
-  return PyBool_FromLong(tracked(THPVariable_Unpack(xo)));
+  return translated([&] { return PyBool_FromLong(tracked(THPVariable_Unpack(xo))); });
 }
 
 PyMethodDef module_methods[] = {

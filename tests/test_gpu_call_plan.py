@@ -291,3 +291,28 @@ def test_forward_mode_and_vmap_where_the_library_product_had_them(gpu, dense_til
             layer(x[0])
         assert flops.get_total_flops() == 2 * m * n * k
         close(layer(x[0]), primal[0])  # makes the plan the second pass meets
+
+
+def test_out_of_memory_keeps_its_type(gpu):
+    """Callers catch torch.OutOfMemoryError to retry with less: an allocation that fails inside a plan raises it too."""
+    from neuropress_amd.nn.np_embedding import NPEmbedding
+
+    k = 8192
+    blob = torch.zeros(16, k // 2, dtype=torch.uint8, device=gpu)
+    emb = NPEmbedding(blob, torch.ones(16 * k // 32, dtype=torch.half, device=gpu), 16, k, 32, 4, "sym", "cuda").to(gpu)
+    emb(torch.zeros(4, dtype=torch.int64, device=gpu))
+    ids = torch.zeros(1, dtype=torch.int64, device=gpu).expand(1 << 26).contiguous()  # an output of 1 TiB
+    for call in range(2):
+        with pytest.raises(torch.OutOfMemoryError):
+            emb(ids)
+
+
+@pytest.mark.parametrize("kind", ["vq8", "q4"])
+def test_sparse_inputs_are_refused_by_python(gpu, kind):
+    """A tensor whose layout queries throw is the module's to refuse, with a plan and without."""
+    layer = _layer(kind, gpu, torch.float16)
+    x = torch.zeros(1, layer.in_features, dtype=torch.half, device=gpu)
+    for call in range(2):
+        with pytest.raises(RuntimeError):
+            layer(x.to_sparse_csr())
+        layer(x)

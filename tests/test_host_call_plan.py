@@ -64,3 +64,9 @@ def test_tracked_tensors():
         seen.append(tracked(x))
     seen += [tracked(torch._neg_view(x)), tracked(x.to_sparse()), tracked(x.to_mkldnn())]
     assert seen == [True] * len(seen)
+
+
+def test_exceptions_of_torch_reach_python():
+    """A query that throws (a sparse row-compressed tensor has no strides) raises; nothing unwinds through the interpreter."""
+    with pytest.raises(RuntimeError):
+        _lib.host().row_distance(torch.ones(2, 3).to_sparse_csr())
