@@ -395,7 +395,7 @@ int npamd_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
  * Activations as the MFMA kernels read them, 16-bit elements: out[m, k] = x[m, perm[k]] (x[m, k] with perm
  * NULL) for k < K and zero for K <= k < ldo, so that a row holds a whole number of 64-column chunks.  The
  * reference gathers x[..., column_perm] with a torch kernel (neuropress/nn/np_vq_linear.py:1027-1028).
- * perm: K int32 column numbers, each < K.  ldo: a multiple of 8; out 16-byte aligned.
+ * perm: K int32 column numbers; zero where one is negative or not below K.  ldo: a multiple of 8; out 16-byte aligned.
  */
 int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* out, int64_t ldo, int M, int K,
                          void* stream);

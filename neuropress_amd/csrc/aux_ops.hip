@@ -421,7 +421,7 @@ int launch_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
 // ---------------------------------------------------------------------------
 // Activations as the MFMA kernels read them: columns permuted and / or rows padded with zeros to a
 // whole number of 64-column chunks, 16-bit elements:
-//   out[m, k] = x[m, perm ? perm[k] : k] for k < K, 0 for K <= k < ldo.
+//   out[m, k] = x[m, perm ? perm[k] : k] for k < K, 0 for K <= k < ldo and for column numbers that x does not have.
 //
 // Bound by the launch at the token counts of a decode step and by HBM beyond.  With a permutation a block first
 // copies whole rows into LDS (one contiguous read) and gathers there with 2-byte reads: through the vector memory path
@@ -476,7 +476,7 @@ gather_columns_kernel(const uint16_t* __restrict__ x, int64_t ldx, const int32_t
       if (row0 + r >= M) break;
       uint16_t v[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = at[e] >= 0 ? xr[r][at[e]] : (uint16_t)0;
+      for (int e = 0; e < 8; ++e) v[e] = (unsigned)at[e] < (unsigned)K ? xr[r][at[e]] : (uint16_t)0;
       u32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = (uint32_t)v[2 * e] | ((uint32_t)v[2 * e + 1] << 16);

@@ -865,7 +865,7 @@ class NPVQLinear(nn.Module):
         packed, proxy = self.packed_indices.reshape(-1), self.proxy
         perm = None
         if self.column_perm is not None and kind not in ("sliced", "gemv_perm"):
-            perm = self.column_perm if dtype == torch.float32 else self._perm_i32(packed.device)
+            perm = self._perm_i64(packed.device) if dtype == torch.float32 else self._perm_i32(packed.device)
         if kind == "sliced":
             sl, _ = self._derived_hit("sliced", self.packed_indices)
             i32 = None if self.column_perm is None else self._perm_i32(packed.device)
@@ -937,7 +937,10 @@ class NPVQLinear(nn.Module):
         self._kernel_stream()
         self._bias_f32()
         if self.column_perm is not None:
-            self._perm_i32(self.packed_indices.device)
+            try:
+                self._perm_i32(self.packed_indices.device)
+            except (IndexError, RuntimeError):  # e.g. materialised and not loaded yet: a call says so
+                pass
         for dtype in (torch.float16, torch.bfloat16):
             self.proxy.centroids_as(dtype)
         if self.is_residual:
@@ -1029,11 +1032,24 @@ class NPVQLinear(nn.Module):
         return sl if m <= limit else None
 
     def _perm_i32(self, device: torch.device) -> torch.Tensor:
-        """``column_perm`` as the int32 device tensor the kernels read (cached)."""
-        return self._derive(
-            "perm_i32", self.column_perm,
-            lambda: self.column_perm.to(device=device, dtype=torch.int32).contiguous(),
-        )  # fmt: skip
+        """``column_perm`` as the int32 device tensor the kernels read (cached): in range, negative entries wrapped as
+        torch's indexing does.  The check waits for the device, once per buffer contents."""
+
+        def build() -> torch.Tensor:
+            perm, k = self.column_perm.to(device), self.in_features
+            if tuple(perm.shape) != (k,):
+                raise RuntimeError(f"NPVQLinear: column_perm must hold in_features={k} entries, got {tuple(perm.shape)}")
+            if perm.is_cuda and torch.cuda.is_current_stream_capturing():
+                perm = perm.clamp(-k, k - 1)  # not to be looked at here: nothing the kernels could read past x with
+            elif bool(((perm < -k) | (perm >= k)).any()):
+                raise IndexError(f"NPVQLinear: column_perm has entries out of range for in_features={k}")
+            return torch.where(perm < 0, perm + k, perm).to(torch.int32).contiguous()
+
+        return self._derive("perm_i32", self.column_perm, build)
+
+    def _perm_i64(self, device: torch.device) -> torch.Tensor:
+        """The same for torch's gather of 32-bit activations inside a call plan, which wraps nothing."""
+        return self._derive("perm_i64", self.column_perm, lambda: self._perm_i32(device).to(torch.int64))
 
     def _gemv_max_tokens(self, m: int) -> int:
         """End of band (a) for a call of *m* tokens: the fused limit, or 32 while x stays small."""

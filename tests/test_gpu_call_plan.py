@@ -316,3 +316,26 @@ def test_sparse_inputs_are_refused_by_python(gpu, kind):
         with pytest.raises(RuntimeError):
             layer(x.to_sparse_csr())
         layer(x)
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.float32])
+@pytest.mark.parametrize("kind", ["vq8-perm", "vq16-perm"])
+def test_column_permutations_with_negative_entries_and_past_the_end(gpu, kind, act, monkeypatch):
+    """As torch's indexing reads them, in every band: counted from the end, and reported."""
+    _small_bands(monkeypatch)
+    layer, k = _layer(kind, gpu, torch.float16), 512
+    perm = layer.column_perm.clone()
+    xs = {m: torch.randn(m, k, generator=cases.gen(m)).to(act).to(gpu) for m in (2, 20, 40, 130)}
+    ref = {m: layer(x) for m, x in xs.items()}
+    layer.column_perm[::3] -= k
+    for m, x in xs.items():
+        assert torch.equal(layer(x), ref[m]) and torch.equal(layer(x), ref[m]), m
+    layer.column_perm[5] = k
+    for x in xs.values():
+        for call in range(2):
+            with pytest.raises(IndexError, match="out of range"):
+                layer(x)
+    layer.prepare()  # says nothing: the buffer may be about to be loaded
+    layer.column_perm.copy_(perm)
+    for m, x in xs.items():
+        assert torch.equal(layer(x), ref[m]), m

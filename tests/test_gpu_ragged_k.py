@@ -41,6 +41,18 @@ def test_gather_columns_of_many_rows(gpu, k, rows):
         assert torch.equal(out[:, :k].view(torch.int16), x.view(torch.int16)[:, perm.long()]) and not out[:, k:].any()
 
 
+@pytest.mark.parametrize("rows,k", [(3, 40), (1025, 40), (3, 33000)])
+def test_gather_columns_reads_only_columns_that_exist(gpu, rows, k):
+    from neuropress_amd import kernels
+
+    x = torch.randn(rows, k, generator=cases.gen(k)).half().to(gpu)
+    perm = torch.arange(k, dtype=torch.int32)
+    perm[[0, 9, 17, 30, k - 1]] = torch.tensor([k, -1, -(2**31), 2**31 - 1, k + 8], dtype=torch.int32)
+    out = kernels.gather_columns(x, perm.to(gpu), (k + 7) // 8 * 8)
+    there = ((perm >= 0) & (perm < k)).to(gpu)
+    assert torch.equal(out[:, :k][:, there], x[:, there]) and not out[:, :k][:, ~there].any()
+
+
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("n,k,nc,vl,perm", [(70, 8, 16, 8, False), (130, 200, 1000, 8, True), (257, 1000, 4096, 4, False),
                                             (64, 2184, 65536, 8, True), (96, 1544, 300, 8, False)])  # fmt: skip

@@ -512,3 +512,20 @@ def test_modules_built_under_inference_mode_keep_their_caches_working():
     wq = ((Q["codes"].float() - 8).reshape(32, 2, 32) * Q["scale"].float().reshape(32, 2, 1)).reshape(32, 64)
     assert torch.allclose(yq, Q["x"] @ wq.T + Q["bias"], atol=1e-3)
     assert tensor_version(torch.zeros(2)) == 0
+
+
+def test_column_permutation_is_checked_before_a_kernel_reads_it():
+    """Negative entries count from the end as in torch's indexing; entries past the end and other lengths are errors."""
+    proxy = VQProxy(torch.zeros(16, 8))
+    packed = torch.zeros(4 * 8, dtype=torch.uint8)
+    perm = torch.randperm(64)
+    layer = NPVQLinear(proxy, packed, 8, 4, 64, 8, "cuda_wmma", column_perm=torch.where(perm % 3 == 0, perm - 64, perm))
+    cpu = torch.device("cpu")
+    assert torch.equal(layer._perm_i32(cpu), perm.int()) and torch.equal(layer._perm_i64(cpu), perm)
+    for entry in (64, -65, 2**40):
+        layer.column_perm[7] = entry
+        with pytest.raises(IndexError, match="out of range"):
+            layer._perm_i32(cpu)
+    layer.column_perm = perm[:63]
+    with pytest.raises(RuntimeError, match="must hold in_features=64"):
+        layer._perm_i32(cpu)
