@@ -652,8 +652,8 @@ class NPVQLinear(nn.Module):
     def is_residual(self) -> bool:
         return self.residual_proxy is not None or self.row_scale is not None or self.row_bias is not None
 
-    def _derive(self, name: str, source: torch.Tensor, build):
-        """``build()`` cached under *name* until *source* moves, is replaced or is written to.
+    def _derive(self, name: str, source: torch.Tensor, build, *more: torch.Tensor):
+        """``build()`` cached under *name* until *source* (or one of *more*) moves, is replaced or is written to.
 
         Every tensor derived from a buffer (a widened index stream, the slice lists, the fp32
         bias, the int32 permutation) is keyed on the buffer's device, address and version
@@ -662,6 +662,8 @@ class NPVQLinear(nn.Module):
         private pool and holds data only after a replay, so a later eager call must make its own.
         """
         key = (source.device, source.data_ptr(), tensor_version(source))
+        for t in more:
+            key += (t.data_ptr(), tensor_version(t))
         hit = self._derived.get(name)
         if hit is not None and hit[0] == key:
             return hit[1]
@@ -695,8 +697,9 @@ class NPVQLinear(nn.Module):
         64-column chunks, are widened to a 16-bit stream once per
         device so they take the vectorised index loads (precedent: the
         reference re-lays index streams out at construction, np_vq_linear.py:644-696).
-        Rows of the latter are padded to :meth:`_kernel_k` columns by repeating their last index:
-        the activations are zero there.
+        Rows of the latter are padded to :meth:`_kernel_k` columns with the index of a codebook row of finite
+        values: the activations are zero there, and zero times an infinity is not (a codebook none of whose rows is
+        finite can turn an infinite output into NaN).
         """
         pad = (self._kernel_k() - self.in_features) // self.vector_len
         if (self.bits in _FAST_BITS or self.bits > 16) and pad == 0:
@@ -707,10 +710,12 @@ class NPVQLinear(nn.Module):
             wide = kernels.widen_indices_u16(self.packed_indices, self.n_vectors, self.bits)
             if pad:
                 rows = wide.view(torch.int16).reshape(self.out_features, -1)
-                wide = torch.cat([rows, rows[:, -1:].expand(-1, pad)], 1).reshape(-1).view(torch.uint8)
+                finite = torch.isfinite(self.proxy.centroids.to(torch.float16)).all(1).to(torch.uint8)
+                filler = finite.argmax().to(torch.int16)  # bits of the unsigned index
+                wide = torch.cat([rows, filler.expand(self.out_features, pad)], 1).reshape(-1).view(torch.uint8)
             return wide
 
-        return self._derive("wide", self.packed_indices, widen), 16
+        return self._derive("wide", self.packed_indices, widen, *((self.proxy.centroids,) if pad else ())), 16
 
     def _kernel_k(self) -> int:
         """Columns the MFMA kernels contract: K, rounded up to whole 64-column chunks where the layer is otherwise

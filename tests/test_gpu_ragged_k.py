@@ -84,3 +84,28 @@ def test_ragged_k_runs_the_fused_bands(gpu, n, k, nc, vl, perm, act, monkeypatch
             y2 = layer(xs.to(gpu)[:, :k]).float().cpu()
             assert bool(((y2 - ref).abs() <= 1e-2 + 1e-2 * ref.abs()).all()), m
     assert used == [(1, "vq_linear"), (3, "vq_linear"), (17, "vq_linear"), (40, "vq_gemm_tile"), (100, "vq_gemm_tile")]
+
+
+@pytest.mark.parametrize("nc,bad", [(1000, (0, 1, 999)), (65536, (0, 65535)), (40000, tuple(range(39000)))])
+def test_infinities_in_the_codebook_stay_what_they_are(gpu, nc, bad, monkeypatch):
+    """Padded columns multiply zeros with a finite codebook row, so that an infinite output does not turn into NaN."""
+    monkeypatch.setattr(vqmod, "_TILE_MIN_GRID_FRACTION", 0.0)
+    monkeypatch.setattr(vqmod, "_TILE_WIDE_SMALL_MAX_TOKENS", 128)
+    monkeypatch.setattr(vqmod, "_TILE_WIDE_TINY_WEIGHTS", 0)
+    n, k = 70, 200
+    L = cases.vq_layer(nc, n, k, nc, bits=16, std=0.05)
+    idx = torch.randint(max(bad) + 1 if len(bad) > 3 else 2, nc - 1, (n, k // 8), generator=cases.gen(1))
+    idx[0, -1], idx[3, 2], idx[69, -1] = bad[0], bad[-1], bad[1]
+    L["cb"][list(bad), 3] = float("inf")
+    layer = NPVQLinear(VQProxy(torch.zeros_like(L["cb"])).to(gpu), vqmod.IndexPacking.pack(idx.reshape(-1), 16), 16, n, k, 8, "cuda_wmma").to(gpu)
+    layer(torch.zeros(3, k, dtype=torch.half, device=gpu))
+    layer.proxy.centroids.copy_(L["cb"])  # written in place: another row may be the finite one
+    w = L["cb"][idx].reshape(n, k).float()
+    for m in (3, 40, 400):
+        x = torch.randn(m, k, generator=cases.gen(m)).half()
+        ref = torch.nn.functional.linear(x.float(), w)
+        for call in range(2):
+            y = layer(x.to(gpu)).float().cpu()
+            assert torch.equal(y[:, [0, 3, 69]], ref[:, [0, 3, 69]]) and bool(torch.isinf(ref[:, [0, 3, 69]]).all()), (m, call)
+            fine = torch.isfinite(ref)
+            assert bool(((y - ref)[fine].abs() <= 1e-2 + 1e-2 * ref[fine].abs()).all()), (m, call)
