@@ -25,10 +25,11 @@ def make(module, attributes, thresholds=None, names=(), holders=(), sources=()):
     """An empty plan for *module*, or None where it cannot have one (a tensor off the module's GPU, or with gaps).
 
     *attributes*: names in the module's ``__dict__`` the dispatch reads; *thresholds* / *names*: the globals of the
-    module's file it reads; *holders*: further modules whose buffers are used (shared codebooks); *sources*: the
+    module's file it reads (next to the band lines of ``nn.backends``); *holders*: further modules whose buffers are used (shared codebooks); *sources*: the
     buffers themselves.
     """
     from .. import kernels
+    from ..nn import backends
 
     device = None
     for t in sources:
@@ -46,6 +47,7 @@ def make(module, attributes, thresholds=None, names=(), holders=(), sources=()):
         plan.guard(holder._buffers, dict(holder._buffers), False)
     if names:
         plan.guard(thresholds, {name: thresholds[name] for name in names}, False)
+        plan.guard(backends.__dict__, {name: getattr(backends, name) for name in backends.BAND_LINES}, False)
     plan.guard(kernels.__dict__, kernels.WRAPPERS, True)
     plan.guard(kernels.SlicedCallPlan, {"run": kernels.SLICED_RUN}, True)
     for t in sources:

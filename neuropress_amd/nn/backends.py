@@ -148,6 +148,8 @@ _LARGE_LAYER_WEIGHTS: int = 1 << 25
 # against 16.9 / 21.6, int4 14.0 / 16.3 against 15.8 / 19.4; 5632 x 4096 int4 22.3 / 25.7 against 20.4 / 23.3, with zero points
 # 22.4 / 25.7 against 24.9 / 27.7; 5504 x 8192 int4 41.6 / 48.3 against 29.5 / 36.3, 256-row codebook 43.4 / 50.2 against 20.7 / 27.1.
 _TIGHT_GRID_FRACTION: float = 0.66
+# What a call plan's choice of a kernel read here (it is valid while these are unchanged).
+BAND_LINES = ("_SMALL_LAYER_WEIGHTS", "_MID_LAYER_WEIGHTS", "_MID_LAYER_K", "_LARGE_LAYER_WEIGHTS", "_TIGHT_GRID_FRACTION")
 
 
 def tile_band_ok(

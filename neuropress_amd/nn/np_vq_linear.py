@@ -45,9 +45,8 @@ from ..transforms.vq_packing import (
     TieredIndexPacking,
     ZeroEscapePacking,
 )
-from .backends import (
-    _MID_LAYER_K, _MID_LAYER_WEIGHTS, _SMALL_LAYER_WEIGHTS, Backend, VQBackend, is_hip_backend_available, tensor_version, tile_band_ok,
-)  # fmt: skip
+from . import backends
+from .backends import Backend, VQBackend, is_hip_backend_available, tensor_version, tile_band_ok
 
 log = logging.getLogger(__name__)
 
@@ -1159,11 +1158,11 @@ class NPVQLinear(nn.Module):
             if tracked:
                 broad = weights >= _TILE_WIDE_BROAD_WEIGHTS
                 return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LIBRARY_MAX_TOKENS if broad else _TILE_WIDE_LIBRARY_MAX_TOKENS // 2)
-            if weights >= _MID_LAYER_WEIGHTS and k >= 4096:
-                return _TILE_WIDE_MAX_TOKENS if k >= _MID_LAYER_K else min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS)
+            if weights >= backends._MID_LAYER_WEIGHTS and k >= 4096:
+                return _TILE_WIDE_MAX_TOKENS if k >= backends._MID_LAYER_K else min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS)
             if weights >= _TILE_WIDE_BROAD_WEIGHTS and self.out_features >= _TILE_WIDE_BROAD_FEATURES:
                 return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS)
-            if weights >= _SMALL_LAYER_WEIGHTS and k >= 4096:
+            if weights >= backends._SMALL_LAYER_WEIGHTS and k >= 4096:
                 return min(_TILE_WIDE_MAX_TOKENS, _TILE_WIDE_LONG_MAX_TOKENS if k >= _TILE_SPLIT_LONG_K else _TILE_WIDE_MID_MAX_TOKENS)
             if weights < _TILE_WIDE_TINY_WEIGHTS and _TILE_MIN_GRID_FRACTION > 0:
                 return min(_TILE_WIDE_MAX_TOKENS, _GEMV_KERNEL_MAX_TOKENS)

@@ -339,3 +339,22 @@ def test_column_permutations_with_negative_entries_and_past_the_end(gpu, kind, a
     layer.column_perm.copy_(perm)
     for m, x in xs.items():
         assert torch.equal(layer(x), ref[m]), m
+
+
+@pytest.mark.parametrize("kind", ["vq8", "rvq", "q4"])
+def test_plans_follow_the_band_lines(gpu, kind, monkeypatch):
+    """Every line the choice between the bands reads: a plan made under another value is stale."""
+    from neuropress_amd.nn import backends
+
+    layer = _layer(kind, gpu, torch.float16)
+    x = torch.randn(40, 512, generator=cases.gen(1)).half().to(gpu)
+    module = qmod if kind == "q4" else vqmod
+    for owner, name in [(backends, n) for n in backends.BAND_LINES] + [(module, n) for n in module._PLAN_THRESHOLDS]:
+        y = layer(x)
+        plan = layer._plan
+        assert not plan.stale(layer)
+        with monkeypatch.context() as mp:
+            value = getattr(owner, name)
+            mp.setattr(owner, name, dict(value) if isinstance(value, dict) else not value if isinstance(value, bool) else value * 1.0)
+            assert plan.stale(layer) and plan(layer, x) is None, name
+        assert torch.equal(layer(x), y)
