@@ -18,6 +18,7 @@
 #include <Python.h>
 #include <structmember.h>
 
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/index_select.h>
 #include <ATen/ops/linear.h>
@@ -334,8 +335,8 @@ bool rows_at_one_stride(const at::Tensor& x, int64_t* ldx) {
 }
 
 // Whether torch follows what is done to x: it records a gradient or a trace, x carries a tangent, is a wrapper (vmap, grad
-// and jvp of torch.func; a tensor without storage of its own or one that is read negated) or not strided, or a dispatch
-// mode looks on.  The kernels read addresses and their outputs carry nothing: no plan issues such a call, and the
+// and jvp of torch.func; a tensor without storage of its own or one that is read negated) or not strided, a dispatch
+// mode looks on, or autocast gives the library's product another type than x's.  The kernels read addresses and their outputs carry nothing: no plan issues such a call, and the
 // module decides between its kernels and torch's own operations.
 bool tracked(const at::Tensor& x) {
   constexpr c10::DispatchKeySet own = c10::autograd_dispatch_keyset | c10::autocast_dispatch_keyset |
@@ -343,7 +344,9 @@ bool tracked(const at::Tensor& x) {
   const c10::DispatchKeySet keys = x.key_set() - own;
   if (keys != c10::DispatchKeySet(c10::DispatchKey::CUDA) && keys != c10::DispatchKeySet(c10::DispatchKey::CPU)) return true;
   return (x.requires_grad() && c10::GradMode::is_enabled()) || x._fw_grad(0).defined() || torch::jit::tracer::isTracing() ||
-         c10::impl::TorchDispatchModeTLS::any_modes_set();
+         c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+         (at::isReducedFloatingType(x.scalar_type()) && at::autocast::is_autocast_enabled(x.device().type()) &&
+          at::autocast::get_autocast_dtype(x.device().type()) != x.scalar_type());
 }
 
 PyObject* issue_planned(Plan* p, PyObject* xo) {

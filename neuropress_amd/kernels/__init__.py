@@ -856,7 +856,7 @@ def warn_kernel_fallback(kernel: str, fallback: str, exc: BaseException) -> None
 
 def tracked(x: torch.Tensor) -> bool:
     """Whether torch follows what is done to *x* (a gradient or a trace is recorded, *x* carries a tangent or is a wrapper of
-    ``torch.func``, a dispatch mode looks on): the kernels' outputs carry nothing of that, so such calls go through
+    ``torch.func``, a dispatch mode looks on, autocast gives products another type than *x*'s): the kernels' outputs carry nothing of that, so such calls go through
     torch's own operations wherever the library's product is the one to take."""
     return _lib.host().tracked(x)
 

@@ -358,3 +358,17 @@ def test_plans_follow_the_band_lines(gpu, kind, monkeypatch):
             mp.setattr(owner, name, dict(value) if isinstance(value, dict) else not value if isinstance(value, bool) else value * 1.0)
             assert plan.stale(layer) and plan(layer, x) is None, name
         assert torch.equal(layer(x), y)
+
+
+@pytest.mark.parametrize("kind", ["vq8", "vq8-perm", "rvq", "q4"])
+def test_autocast_decides_the_type_of_the_dense_bands(gpu, kind):
+    layer = _layer(kind, gpu, torch.float16)
+    x = torch.randn(130, 512, generator=cases.gen(1)).half().to(gpu)
+    ref = layer(x)
+    for call in range(2):
+        for dtype in (torch.float16, torch.bfloat16):
+            with torch.autocast("cuda", dtype=dtype):
+                y = layer(x)
+                assert y.dtype == dtype and torch.allclose(y.float(), ref.float(), rtol=2e-2, atol=5e-2)
+                assert layer(x[:4]).dtype == torch.float16  # the fused kernels answer in x's type
+                assert layer(x.float()).dtype == dtype

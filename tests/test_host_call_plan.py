@@ -55,6 +55,9 @@ def test_tracked_tensors():
     with fwad.dual_level():
         assert tracked(fwad.make_dual(x, x)) and not tracked(x)
     assert not tracked(x)
+    for dtype in (torch.bfloat16, torch.float16):
+        with torch.autocast("cpu", dtype=dtype):
+            assert tracked(x.half()) == (dtype != torch.half) and not tracked(x) and not tracked(x.long())
     seen = []
     torch.func.vmap(lambda t: seen.append(tracked(t)) or t)(x)
     torch.func.grad(lambda t: seen.append(tracked(t)) or t.sum())(x)
