@@ -1002,5 +1002,5 @@ def q_embedding(
 WRAPPERS = {
     fn.__name__: fn
     for fn in (vq_linear_sliced_checked, vq_linear, vq_gemm_tile, vq_dequant, rvq_linear, rvq_dequant, q_linear, q_gemm_tile,
-               q_dequant, rms_norm, vq_embedding, q_embedding)
+               q_dequant, rms_norm, vq_embedding, q_embedding, dense_linear, gather_columns)
 }  # fmt: skip

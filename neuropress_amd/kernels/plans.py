@@ -14,6 +14,7 @@ import torch.nn.modules.module as nn_module
 from .. import _lib
 
 _TORCH_CALL = torch.nn.Module.__call__
+_TORCH_LINEAR = torch.nn.functional.linear
 
 (SLICED, VQ_GEMV, VQ_GEMV_PERM, VQ_TILE, VQ_DENSE, RVQ_GEMV, RVQ_TILE, RVQ_DENSE,
  Q_GEMV, Q_TILE, Q_DENSE, RMS_NORM, VQ_EMBEDDING, Q_EMBEDDING) = range(14)  # fmt: skip
@@ -49,6 +50,7 @@ def make(module, attributes, thresholds=None, names=(), holders=(), sources=()):
         plan.guard(thresholds, {name: thresholds[name] for name in names}, False)
         plan.guard(backends.__dict__, {name: getattr(backends, name) for name in backends.BAND_LINES}, False)
     plan.guard(kernels.__dict__, kernels.WRAPPERS, True)
+    plan.guard(torch.nn.functional.__dict__, {"linear": _TORCH_LINEAR}, True)
     plan.guard(kernels.SlicedCallPlan, {"run": kernels.SLICED_RUN}, True)
     for t in sources:
         plan.source(t)

@@ -372,3 +372,21 @@ def test_autocast_decides_the_type_of_the_dense_bands(gpu, kind):
                 assert y.dtype == dtype and torch.allclose(y.float(), ref.float(), rtol=2e-2, atol=5e-2)
                 assert layer(x[:4]).dtype == torch.float16  # the fused kernels answer in x's type
                 assert layer(x.float()).dtype == dtype
+
+
+@pytest.mark.parametrize("kind", ["vq8", "rvq", "q4"])
+def test_replaced_products_are_called(gpu, dense_tile, kind, monkeypatch):
+    """The product of the dense band, the package's own and the library's: instrumentation put in its place sees every call."""
+    from neuropress_amd import kernels
+
+    layer = _layer(kind, gpu, torch.float16)
+    x = torch.randn(130, 512, generator=cases.gen(1)).half().to(gpu)
+    for tile, owner, name in ((0, kernels, "dense_linear"), (-1, torch.nn.functional, "linear")):
+        dense_tile(tile)
+        layer._plan = None
+        ref = layer(x)
+        real, seen = getattr(owner, name), []
+        with monkeypatch.context() as mp:
+            mp.setattr(owner, name, lambda *a, **k: seen.append(1) or real(*a, **k))
+            assert torch.equal(layer(x), ref) and torch.equal(layer(x), ref) and len(seen) == 2
+        assert torch.equal(layer(x), ref) and len(seen) == 2
