@@ -696,7 +696,7 @@ class NPVQLinear(nn.Module):
         64-column chunks, are widened to a 16-bit stream once per
         device so they take the vectorised index loads (precedent: the
         reference re-lays index streams out at construction, np_vq_linear.py:644-696).
-        Rows of the latter are padded to :meth:`_kernel_k` columns with the index of a codebook row of finite
+        Rows of the latter are padded to :meth:`_kernel_k` columns with the index of the codebook row of the smallest
         values: the activations are zero there, and zero times an infinity is not (a codebook none of whose rows is
         finite can turn an infinite output into NaN).
         """
@@ -709,8 +709,9 @@ class NPVQLinear(nn.Module):
             wide = kernels.widen_indices_u16(self.packed_indices, self.n_vectors, self.bits)
             if pad:
                 rows = wide.view(torch.int16).reshape(self.out_features, -1)
-                finite = torch.isfinite(self.proxy.centroids.to(torch.float16)).all(1).to(torch.uint8)
-                filler = finite.argmax().to(torch.int16)  # bits of the unsigned index
+                # bits of a value without its sign: infinities and NaN are the largest
+                size = self.proxy.centroids.to(torch.float16).view(torch.int16) & 0x7FFF
+                filler = size.amax(1).argmin().to(torch.int16)  # bits of the unsigned index
                 wide = torch.cat([rows, filler.expand(self.out_features, pad)], 1).reshape(-1).view(torch.uint8)
             return wide
 
@@ -1043,11 +1044,14 @@ class NPVQLinear(nn.Module):
             perm, k = self.column_perm.to(device), self.in_features
             if tuple(perm.shape) != (k,):
                 raise RuntimeError(f"NPVQLinear: column_perm must hold in_features={k} entries, got {tuple(perm.shape)}")
+            low, high = -k, k - 1
             if perm.is_cuda and torch.cuda.is_current_stream_capturing():
-                perm = perm.clamp(-k, k - 1)  # not to be looked at here: nothing the kernels could read past x with
-            elif bool(((perm < -k) | (perm >= k)).any()):
+                perm = perm.clamp(low, high)  # not to be looked at here: nothing the kernels could read past x with
+            elif k:
+                low, high = torch.stack(torch.aminmax(perm)).tolist()
+            if low < -k or high >= k:
                 raise IndexError(f"NPVQLinear: column_perm has entries out of range for in_features={k}")
-            return torch.where(perm < 0, perm + k, perm).to(torch.int32).contiguous()
+            return (perm if low >= 0 else torch.where(perm < 0, perm + k, perm)).to(torch.int32).contiguous()
 
         return self._derive("perm_i32", self.column_perm, build)
 

@@ -247,7 +247,8 @@ def _weight_layer(kind, n, k, gpu):
 
 
 @pytest.mark.parametrize("name,kind,n,k,m", _dense_cases())
-def test_gradients_where_the_library_product_had_them(gpu, dense_tile, name, kind, n, k, m):
+def test_gradients_where_the_library_product_had_them(gpu, dense_tile, name, kind, n, k, m, monkeypatch):
+    monkeypatch.setattr(vqmod, "_SLICED_MAX_TOKENS", 0)  # no slice lists to build and time
     if name == "library product":
         dense_tile(-1)  # never the package's own
     layer, w = _weight_layer(kind, n, k, gpu)
