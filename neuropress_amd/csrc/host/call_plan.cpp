@@ -22,6 +22,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/index_select.h>
 #include <ATen/ops/linear.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -29,6 +30,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
+#include <algorithm>
 #include <deque>
 #include <unordered_map>
 #include <vector>
@@ -127,6 +129,10 @@ struct Plan {
   std::vector<Source>* sources;
   std::deque<Template>* templates;
   std::unordered_map<int64_t, Route>* routes;  // key: dtype code << 32 | tokens
+  // Streams on which the plan and its templates were made -- and, just before, the tensors derived for them (a bias in the
+  // activations' type, a widened index stream) -- and the other streams that have waited for those.
+  std::vector<hipStream_t>* made;
+  std::vector<hipStream_t>* ordered;
 };
 
 PyObject* g_workspaces = nullptr;       // {(device, stream): zero-filled scratch of the slice-list GEMV}
@@ -177,10 +183,51 @@ using U8 = const uint8_t*;
 using F32 = const float*;
 using I32 = const int32_t*;
 
+hipStream_t current_stream(int device) { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream(); }
+
+bool contains(const std::vector<hipStream_t>& streams, hipStream_t st) {
+  return std::find(streams.begin(), streams.end(), st) != streams.end();
+}
+
+void made_on(Plan* p, hipStream_t st) {
+  if (contains(*p->made, st)) return;
+  p->made->push_back(st);
+  p->ordered->clear();
+}
+
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus status;
+  if (hipStreamIsCapturing(st, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;  // the legacy stream while another one is
+}
+
+// A call on a stream the plan was not made on: let that stream wait, once, for what was made on the others.  Not inside a
+// capture or for a stream inside one (captures start on an idle GPU, and an event would tie the streams together).  False:
+// could not be arranged.
+bool order_after_making(Plan* p, hipStream_t st) {
+  if (contains(*p->ordered, st) || capturing(st)) return true;
+  const c10::DeviceGuard guard(c10::Device(c10::kCUDA, (c10::DeviceIndex)p->device));
+  for (hipStream_t from : *p->made) {
+    if (from == st || capturing(from)) continue;
+    hipEvent_t done = nullptr;
+    const bool ok = hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess && hipEventRecord(done, from) == hipSuccess &&
+                    hipStreamWaitEvent(st, done, 0) == hipSuccess;
+    if (done) (void)hipEventDestroy(done);  // freed once it has happened
+    if (!ok) {
+      (void)hipGetLastError();
+      return false;
+    }
+  }
+  if (p->ordered->size() >= 64) p->ordered->clear();  // bounded, however many streams a program makes
+  p->ordered->push_back(st);
+  return true;
+}
+
 // Launches template t on x ([m, k], row stride ldx); the output in *out.  False: not issued, or it failed.
-bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m, int64_t ldx, int device, at::Tensor* out) {
+bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m, int64_t ldx, int device, hipStream_t st,
+           at::Tensor* out) {
   const std::vector<int64_t>& a = t.a;
-  hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
   c10::SmallVector<int64_t, 6> sizes(x_in.sizes().begin(), x_in.sizes().end());
   at::Tensor x = x_in;
   if (t.perm.defined() && t.perm.scalar_type() == at::kLong) {
@@ -371,8 +418,10 @@ PyObject* issue_planned(Plan* p, PyObject* xo) {
   const Route route = it->second;
   const Template& t = (*p->templates)[(size_t)route.tmpl];
   if (t.k_in != k) Py_RETURN_NONE;
+  hipStream_t st = current_stream(p->device);
+  if ((p->made->size() != 1 || p->made->front() != st) && !order_after_making(p, st)) Py_RETURN_NONE;
   at::Tensor y;
-  if (!issue(t, route, x, m, ldx, p->device, &y)) Py_RETURN_NONE;
+  if (!issue(t, route, x, m, ldx, p->device, st, &y)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
 }
 
@@ -392,14 +441,14 @@ PyObject* run(Plan* p, PyObject* xo) {
 }
 
 // What torch.nn.Module.__call__ looks at before it calls forward: hooks of the module and of all modules, a compiled
-// call, a replaced forward, a trace being recorded.
+// call, a replaced forward (and a trace being recorded, for which tracked() sends the call the long way).
 bool direct(Plan* p, PyObject* module) {
   if (Py_TYPE(module) != p->direct_type || !holds(p->direct_self, *_PyObject_GetDictPtr(module))) return false;
   for (Guard& g : *p->direct_guards)
     if (!holds(g, g.dict)) return false;
   for (PyObject* d : *p->hooks)
     if (PyDict_GET_SIZE(d) != 0) return false;
-  return !torch::jit::tracer::isTracing();
+  return true;
 }
 
 // plan(module, x)
@@ -451,6 +500,8 @@ PyObject* plan_new(PyTypeObject* type, PyObject* args, PyObject*) {
   p->sources = new std::vector<Source>();
   p->templates = new std::deque<Template>();
   p->routes = new std::unordered_map<int64_t, Route>();
+  p->made = new std::vector<hipStream_t>();
+  p->ordered = new std::vector<hipStream_t>();
   return reinterpret_cast<PyObject*>(p);
 }
 
@@ -507,6 +558,8 @@ void plan_dealloc(PyObject* self) {
   delete p->sources;
   delete p->templates;
   delete p->routes;
+  delete p->made;
+  delete p->ordered;
   Py_TYPE(self)->tp_free(self);
 }
 
@@ -595,7 +648,9 @@ PyObject* plan_source(PyObject* self, PyObject* t) {
   }
   return translated([&]() -> PyObject* {
     const at::Tensor& v = THPVariable_Unpack(t);
-    reinterpret_cast<Plan*>(self)->sources->push_back({v, v.const_data_ptr(), version_of(v)});
+    Plan* p = reinterpret_cast<Plan*>(self);
+    p->sources->push_back({v, v.const_data_ptr(), version_of(v)});
+    made_on(p, current_stream(p->device));  // as are the derived tensors that a module prepares when it reaches the GPU
     Py_RETURN_NONE;
   });
 }
@@ -642,8 +697,11 @@ PyObject* plan_template(PyObject* self, PyObject* args) {
     PyObject* v = PyTuple_GET_ITEM(keep, i);
     if (v != Py_None && THPVariable_Check(v)) t.keep.push_back(THPVariable_Unpack(v));
   }
-  p->templates->push_back(std::move(t));
-  return PyLong_FromSize_t(p->templates->size() - 1);
+  return translated([&] {
+    made_on(p, current_stream(p->device));
+    p->templates->push_back(std::move(t));
+    return PyLong_FromSize_t(p->templates->size() - 1);
+  });
 }
 
 // route(dtype_code, tokens (0: any number), template, scratch_bytes)
