@@ -200,8 +200,9 @@ __device__ __forceinline__ void store_embedding8(void* out, int64_t at, const ui
 }
 
 // VL = 8: a block takes one token's columns (blockIdx.y: VPT vectors of eight per thread; short rows share a
-// block), so no thread divides 64-bit numbers; a thread's VPT table indices are asked for together, then its codebook rows.  Bound by the
-// output stream and, with a codebook larger than L1, by the row lookups.  An eighth of the tokens to each die: whoever
+// block), so no thread divides 64-bit numbers; a thread's VPT table indices are asked for together, then its codebook rows.  Bound, with a
+// codebook larger than L1, by the L2's requests and the chain id -> index row -> codebook row (4096 tokens x 4096, 65536
+// rows: 15.5-17 us, 11 of them the requests; waves wait 71 % of their time), else by the output stream.  An eighth of the tokens to each die: whoever
 // reads the rows next (a norm deals them the same way) finds them in its own L2.
 template <int OUT, bool PERM, int VPT>
 __global__ void __launch_bounds__(256)

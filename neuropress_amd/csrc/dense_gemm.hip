@@ -16,7 +16,9 @@
 // row r in slot p ^ ((r >> 1) & 7), so that a read of 32 consecutive rows touches every bank group twice), a ring of
 // kStages steps per group; one in-order counter tracks a wave's loads and the waits are written by hand.  A wave
 // computes 32 MT x 64 of the tile (MFMA 32x32x16), reading the operands of a k group while it multiplies the one
-// before.  The row tiles of a column tile go to one die (workgroups go to the eight dies in turn), so that a die's L2
+// before.  At 384 x 4096 x 4096 (21 us) the matrix pipes are busy 40 % of the time of the 192 compute units in use and
+// LDS 32 %; the waves wait 42 % of theirs, for 14 TB/s of lines from the L2s at 389 cycles each, and for each other.
+// The row tiles of a column tile go to one die (workgroups go to the eight dies in turn), so that a die's L2
 // fetches a column tile of W once for all row tiles.
 #include <math.h>
 

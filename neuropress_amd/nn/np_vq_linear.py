@@ -18,8 +18,12 @@ band                  condition                        kernel
 (a) fused GEMV        ``m <= _FUSED_MAX_TOKENS``, or   ``kernels.vq_linear``
                       ``m <= 32`` while x is small
 (b) tile-decode GEMM  ``m <= _TILE_MAX_TOKENS``        ``kernels.vq_gemm_tile``
-(c) decode + GEMM     otherwise                        ``kernels.vq_dequant`` + ``F.linear``
+(c) decode + GEMM     otherwise                        ``kernels.vq_dequant`` + ``kernels.dense_linear`` or ``F.linear``
 ====================  ==============================  ==========================
+
+Only band (c) with ``F.linear`` carries gradients, tangents and the like: calls that ask for them
+(``kernels.tracked``) take it instead of ``dense_linear``, at the token counts where it was the faster one against
+the other bands.
 
 The dispatch rule itself is the reference's (np_vq_linear.py:1014-1058); the
 thresholds are re-derived for one MI355X and stay overridable through the same
