@@ -103,6 +103,7 @@ struct Template {
   at::ScalarType out;
   at::Tensor perm;                  // column permutation applied to x first, or undefined: int32 (16-bit x) or int64
   at::Tensor bias;                  // bias of the dense product, or undefined: float32 for the framework's own
+  at::Tensor leaf;                  // dense kinds: the module's bias itself, which may ask for a gradient
   bool own;                         // dense kinds: the framework's own product, not the library's
   std::vector<at::Tensor> keep;     // what the addresses point into
 };
@@ -247,6 +248,7 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
 
   if (t.kind == kVqDense || t.kind == kRvqDense || t.kind == kQDense) {
     const int code = dtype_code(t.out);
+    if (t.leaf.defined() && t.leaf.requires_grad() && c10::GradMode::is_enabled()) return false;
     if (t.own && (ldx % 8 || ((uintptr_t)x.const_data_ptr() & 15))) return false;
     at::Tensor w = empty({t.n, t.k}, t.out, device);
     int rc;
@@ -663,15 +665,15 @@ PyObject* plan_hold(PyObject* self, PyObject* o) {
   Py_RETURN_NONE;
 }
 
-// template(kind, n, k, k_in, args, f, out_dtype_code, perm or None, bias or None, own, keep) -> number
+// template(kind, n, k, k_in, args, f, out_dtype_code, perm or None, bias or None, leaf or None, own, keep) -> number
 PyObject* plan_template(PyObject* self, PyObject* args) {
   Plan* p = reinterpret_cast<Plan*>(self);
   int kind, out_code, own;
   long long n, k, k_in;
   double f;
-  PyObject *ints, *perm, *bias, *keep;
-  if (!PyArg_ParseTuple(args, "iLLLO!diOOpO!", &kind, &n, &k, &k_in, &PyTuple_Type, &ints, &f, &out_code, &perm, &bias, &own, &PyTuple_Type,
-                        &keep))
+  PyObject *ints, *perm, *bias, *leaf, *keep;
+  if (!PyArg_ParseTuple(args, "iLLLO!diOOOpO!", &kind, &n, &k, &k_in, &PyTuple_Type, &ints, &f, &out_code, &perm, &bias, &leaf, &own,
+                        &PyTuple_Type, &keep))
     return nullptr;
   if (kind < 0 || kind >= kKinds || (int)PyTuple_GET_SIZE(ints) > kArgs[kind]) {
     PyErr_SetString(PyExc_ValueError, "template(): bad kind or argument count");
@@ -694,6 +696,7 @@ PyObject* plan_template(PyObject* self, PyObject* args) {
   t.a.resize((size_t)kArgs[kind], 0);
   if (perm != Py_None) t.perm = THPVariable_Unpack(perm);
   if (bias != Py_None) t.bias = THPVariable_Unpack(bias);
+  if (leaf != Py_None) t.leaf = THPVariable_Unpack(leaf);
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(keep); ++i) {
     PyObject* v = PyTuple_GET_ITEM(keep, i);
     if (v != Py_None && THPVariable_Check(v)) t.keep.push_back(THPVariable_Unpack(v));
@@ -738,7 +741,7 @@ PyMethodDef plan_methods[] = {
     {"direct", plan_direct, METH_VARARGS, "direct(class, own, guards, hooks): when module(x) may go straight to the plan"},
     {"source", plan_source, METH_O, "source(tensor or None)"},
     {"hold", plan_hold, METH_O, "hold(object)"},
-    {"template", plan_template, METH_VARARGS, "template(kind, n, k, k_in, args, f, out, perm, bias, own, keep) -> number"},
+    {"template", plan_template, METH_VARARGS, "template(kind, n, k, k_in, args, f, out, perm, bias, leaf, own, keep) -> number"},
     {"route", plan_route, METH_VARARGS, "route(dtype, tokens, template, scratch_bytes)"},
     {"stale", plan_stale, METH_O, "stale(module): whether anything the plan was built from has changed"},
     {"wrapped", plan_wrapped, METH_NOARGS, "wrapped(): whether a wrapper function has been replaced"},

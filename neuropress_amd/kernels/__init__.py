@@ -854,11 +854,11 @@ def warn_kernel_fallback(kernel: str, fallback: str, exc: BaseException) -> None
 # ---------------------------------------------------------------------------
 
 
-def tracked(x: torch.Tensor) -> bool:
-    """Whether torch follows what is done to *x* (a gradient or a trace is recorded, *x* carries a tangent or is a wrapper of
+def tracked(x: torch.Tensor, bias: torch.Tensor | None = None) -> bool:
+    """Whether torch follows what is done to *x* or to a layer's *bias* (a gradient or a trace is recorded, *x* carries a tangent or is a wrapper of
     ``torch.func``, a dispatch mode looks on, autocast gives products another type than *x*'s): the kernels' outputs carry nothing of that, so such calls go through
     torch's own operations wherever the library's product is the one to take."""
-    return _lib.host().tracked(x)
+    return _lib.host().tracked(x) or (bias is not None and bias.requires_grad and torch.is_grad_enabled())
 
 
 def dense_preferred(m: int, n: int, k: int) -> bool:

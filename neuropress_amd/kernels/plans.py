@@ -85,13 +85,14 @@ def _call_directly(plan, module) -> None:
     )
 
 
-def template(plan, kind, n, k, args, dtype, *, f=0.0, k_in=None, perm=None, bias=None, own=False):
+def template(plan, kind, n, k, args, dtype, *, f=0.0, k_in=None, perm=None, bias=None, leaf=None, own=False):
     """Template number of one call shape.  *args*: its constant arguments, tensors standing for their addresses (the
     plan keeps them alive); *dtype*: of the output; *perm*: columns of x to gather first; *k_in*: columns of x where the
-    kernel contracts more (rows padded with zeros); *own*: the dense product is the package's own (*bias* in float32)."""
+    kernel contracts more (rows padded with zeros); *own*: the dense product is the package's own (*bias* in float32); *leaf*: the
+    module's bias itself, for dense products: the plan declines while it asks for a gradient."""
     ints = tuple(a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args)
     keep = tuple(a for a in args if isinstance(a, torch.Tensor))
-    return plan.template(kind, n, k, k if k_in is None else k_in, ints, f, DTYPE_CODES[dtype], perm, bias, own, keep)
+    return plan.template(kind, n, k, k if k_in is None else k_in, ints, f, DTYPE_CODES[dtype], perm, bias, leaf, own, keep)
 
 
 def tile_scratch(m: int, n: int, k: int) -> int:

@@ -368,7 +368,7 @@ class NPLinear(nn.Module):
 
         m = x.numel() // self.in_features
         try:
-            tracked = kernels.tracked(x)
+            tracked = kernels.tracked(x, self.bias)
             band = self._band(x, m, tracked)
             if not tracked and not torch.cuda.is_current_stream_capturing():
                 y = self._planned(x, m, band)
@@ -438,7 +438,7 @@ class NPLinear(nn.Module):
             kind = {"fused": plans.Q_GEMV, "tile": plans.Q_TILE}.get(band, plans.Q_DENSE)
             args = (self.u8_blob, self.scale, self.zero_point, self._bias_f32(), 0, 0, self.nbits, self.group_size, code)
             bias = self._bias_as(x.dtype) if band == "dense" else self._bias_f32() if band == "product" else None
-            number = plan.names[band, x.dtype] = plans.template(plan, kind, n, k, args, x.dtype, bias=bias, own=band == "product")
+            number = plan.names[band, x.dtype] = plans.template(plan, kind, n, k, args, x.dtype, bias=bias, leaf=self.bias, own=band == "product")
         scratch = {"tile": plans.tile_scratch, "product": plans.product_scratch}.get(band)
         plan.route(code, m, number, scratch(m, n, k) if scratch else 0)
         self._plan = plan

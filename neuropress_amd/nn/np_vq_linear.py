@@ -750,7 +750,7 @@ class NPVQLinear(nn.Module):
         from .. import kernels
 
         m = x.numel() // self.in_features
-        tracked = x.is_cuda and self.backend in _FUSED_BACKENDS and kernels.tracked(x)
+        tracked = x.is_cuda and self.backend in _FUSED_BACKENDS and kernels.tracked(x, self.bias)
         band = self._band(x, m, tracked)
         if x.is_cuda and not tracked and not torch.cuda.is_current_stream_capturing():
             y = self._planned(x, m, band)
@@ -889,7 +889,7 @@ class NPVQLinear(nn.Module):
             if kind in ("dense", "product"):
                 own = kind == "product"
                 bias = self._bias_f32() if own else self._bias_as(dtype)
-                return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=bias, own=own)
+                return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=bias, leaf=self.bias, own=own)
             kind_code = plans.RVQ_TILE if kind == "tile" else plans.RVQ_GEMV
             return plans.template(plan, kind_code, n, k, (*args, self._bias_f32(), code), dtype, perm=perm)
         stream, bits = self._kernel_stream()
@@ -901,7 +901,7 @@ class NPVQLinear(nn.Module):
             if width == k and self._kernel_k() != k:
                 stream, bits = packed, self.bits
             args = (stream, stream.numel(), bits, proxy.centroids, proxy.num_centroids, vl, n * (width // vl))
-            return plans.template(plan, plans.VQ_DENSE, n, width, args, dtype, k_in=k, perm=perm, bias=bias, own=own)
+            return plans.template(plan, plans.VQ_DENSE, n, width, args, dtype, k_in=k, perm=perm, bias=bias, leaf=self.bias, own=own)
         args = (stream, stream.numel(), bits, proxy.centroids_as(dtype), code, proxy.num_centroids, vl, self._bias_f32(), code)
         if kind == "gemv_perm":
             return plans.template(plan, plans.VQ_GEMV_PERM, n, k, (*args, self._perm_i32(stream.device)), dtype)
@@ -1250,7 +1250,7 @@ class NPVQLinear(nn.Module):
         from .. import kernels
 
         try:
-            own = self._own_product(x.numel() // self.in_features, x.dtype) and not kernels.tracked(x)
+            own = self._own_product(x.numel() // self.in_features, x.dtype) and not kernels.tracked(x, self.bias)
             if self.is_residual:
                 w = kernels.rvq_dequant(
                     self.packed_indices, self.bits, self._res_stream(), self._res_bits(),

@@ -391,3 +391,24 @@ def test_replaced_products_are_called(gpu, dense_tile, kind, monkeypatch):
             mp.setattr(owner, name, lambda *a, **k: seen.append(1) or real(*a, **k))
             assert torch.equal(layer(x), ref) and torch.equal(layer(x), ref) and len(seen) == 2
         assert torch.equal(layer(x), ref) and len(seen) == 2
+
+
+@pytest.mark.parametrize("tile", [0, -1])
+@pytest.mark.parametrize("kind", ["vq8", "vq8-perm", "q4"])
+def test_bias_gradients_where_the_library_product_had_them(gpu, dense_tile, kind, tile):
+    """A bias that is trained on its own: the input asks for no gradient."""
+    dense_tile(tile)
+    layer = _layer(kind, gpu, torch.float16)
+    x = torch.randn(130, 512, generator=cases.gen(1)).half().to(gpu)
+    dy = torch.randn(130, 96, generator=cases.gen(2)).half().to(gpu)
+    for call in range(2):
+        layer(x)  # without a gradient asked for: a plan
+        layer.bias.requires_grad_()
+        y = layer(x)
+        assert y.requires_grad
+        (grad,) = torch.autograd.grad(y, layer.bias, dy)
+        assert torch.allclose(grad.float(), dy.float().sum(0), rtol=1e-2, atol=2e-2)
+        with torch.no_grad():
+            assert not layer(x).requires_grad
+        layer.bias.requires_grad_(False)
+        assert not layer(x).requires_grad
