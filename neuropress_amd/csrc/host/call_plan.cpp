@@ -229,6 +229,7 @@ bool order_after_making(Plan* p, hipStream_t st) {
 // Launches template t on x ([m, k], row stride ldx); the output in *out.  False: not issued, or it failed.
 bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m, int64_t ldx, int device, hipStream_t st,
            at::Tensor* out) {
+  if (t.leaf.defined() && t.leaf.requires_grad() && c10::GradMode::is_enabled()) return false;
   const std::vector<int64_t>& a = t.a;
   c10::SmallVector<int64_t, 6> sizes(x_in.sizes().begin(), x_in.sizes().end());
   at::Tensor x = x_in;
@@ -248,7 +249,6 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
 
   if (t.kind == kVqDense || t.kind == kRvqDense || t.kind == kQDense) {
     const int code = dtype_code(t.out);
-    if (t.leaf.defined() && t.leaf.requires_grad() && c10::GradMode::is_enabled()) return false;
     if (t.own && (ldx % 8 || ((uintptr_t)x.const_data_ptr() & 15))) return false;
     at::Tensor w = empty({t.n, t.k}, t.out, device);
     int rc;

@@ -714,7 +714,7 @@ class NPVQLinear(nn.Module):
             if pad:
                 rows = wide.view(torch.int16).reshape(self.out_features, -1)
                 # bits of a value without its sign: infinities and NaN are the largest
-                size = self.proxy.centroids.to(torch.float16).view(torch.int16) & 0x7FFF
+                size = self.proxy.centroids.to(wide.device, torch.float16).view(torch.int16) & 0x7FFF
                 filler = size.amax(1).argmin().to(torch.int16)  # bits of the unsigned index
                 wide = torch.cat([rows, filler.expand(self.out_features, pad)], 1).reshape(-1).view(torch.uint8)
             return wide

@@ -109,3 +109,14 @@ def test_infinities_in_the_codebook_stay_what_they_are(gpu, nc, bad, monkeypatch
             assert torch.equal(y[:, [0, 3, 69]], ref[:, [0, 3, 69]]) and bool(torch.isinf(ref[:, [0, 3, 69]]).all()), (m, call)
             fine = torch.isfinite(ref)
             assert bool(((y - ref)[fine].abs() <= 1e-2 + 1e-2 * ref[fine].abs()).all()), (m, call)
+
+
+def test_layers_prepare_before_their_codebook_arrives(gpu):
+    L = cases.vq_layer(3, 70, 200, 1000, std=0.05)
+    proxy = VQProxy(L["cb"])
+    layer = NPVQLinear(proxy, L["packed"], L["bits"], 70, 200, 8, "cuda_wmma").to(gpu)
+    layer.prepare()
+    proxy.to(gpu)
+    x = torch.randn(3, 200, generator=cases.gen(1)).half()
+    ref = torch.nn.functional.linear(x.float(), L["cb"][L["idx"]].reshape(70, 200).float())
+    assert torch.allclose(layer(x.to(gpu)).float().cpu(), ref, rtol=1e-2, atol=1e-2)
