@@ -130,6 +130,24 @@ int npamd_vq_gemm_tile(const void* x, int64_t ldx, const uint8_t* packed, int64_
                        const float* bias, void* y, int64_t ldy, int M, int N, int K,
                        int act_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/*
+ * Slice GEMM, M <= 32: the same contraction for 16-bit indices into a codebook of 4097 to 65536 rows of eight, kept in
+ * the activation dtype (K a multiple of 64, 16-byte aligned buffers, a stream of less than 4 GiB, the workspace below; any
+ * other request is npamd_vq_gemm_tile's).  Codebook slices of up to 8192 rows lie in the compute units' LDS and every index is walked once
+ * per slice; the slices' partial sums (f32) go through `workspace`, npamd_vq_slice_workspace_bytes(M, N, K, nc) bytes of
+ * 16-byte aligned device memory whose contents are irrelevant before and after, and are added in a fixed order: results
+ * are the same from run to run.  It has no counterpart in the reference.
+ * npamd_vq_slice_estimate_ns: about how long a call takes, whatever the indices (0: not a shape it takes).  The kernels that look
+ * rows up in memory are slower where indices are spread evenly, and faster where they crowd into few rows.
+ * Both questions are host-only arithmetic.
+ */
+int npamd_vq_slice_gemm(const void* x, int64_t ldx, const uint8_t* packed, int64_t n_bytes, int bits,
+                        const void* codebook, int codebook_dtype, int nc, int vl, const float* bias, void* y,
+                        int64_t ldy, int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes,
+                        void* stream);
+int64_t npamd_vq_slice_workspace_bytes(int M, int N, int K, int nc);
+int npamd_vq_slice_estimate_ns(int M, int N, int K, int nc);
+
 /* Bytes of workspace the *_gemm_tile entry points can use for this shape (0: K is not split). */
 int64_t npamd_gemm_tile_workspace_bytes(int M, int N, int K);
 

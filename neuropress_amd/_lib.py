@@ -36,6 +36,9 @@ SIGNATURES: dict[str, list] = {
     "npamd_vq_gemv_perm_supported": [_int] * 6,
     "npamd_vq_gemm_tile": _VQ_LINEAR[:-1] + _WS + [_vp],
     "npamd_gemm_tile_workspace_bytes": [_int, _int, _int],
+    "npamd_vq_slice_gemm": _VQ_LINEAR[:-1] + _WS + [_vp],
+    "npamd_vq_slice_workspace_bytes": [_int, _int, _int, _int],
+    "npamd_vq_slice_estimate_ns": [_int, _int, _int, _int],
     "npamd_vq_widen_u16": [_vp, _i64, _int, _i64, _vp, _vp],
     "npamd_vq_lut_gather": [_vp, _vp, _i64, _int, _vp, _int, _int, _int, _int, _vp],
     "npamd_vq_sliced_build": [_vp, _i64, _int, _int, _int, _int, _int, _int, _vp, _i64,
@@ -71,6 +74,7 @@ SIGNATURES: dict[str, list] = {
 }
 
 _RESTYPES = {"npamd_vq_sliced_workspace_bytes": _i64, "npamd_gemm_tile_workspace_bytes": _i64, "npamd_dense_gemm_workspace_bytes": _i64,
+             "npamd_vq_slice_workspace_bytes": _i64,
              "npamd_diag_reload_tuning": None}
 SLICED_HEADER_BYTES = 128
 SLICED_STATIC_WORKSPACE_BYTES = 4 * 1024 * 1024

@@ -62,6 +62,8 @@ static Tuning read_tuning() {
   t.tile_splits = env_int("NPAMD_TILE_SPLITS", 0);
   t.tile_mw = env_int("NPAMD_TILE_MW", 0);
   t.tile_wide = env_int("NPAMD_TILE_WIDE", 1);
+  t.slice_tiles = env_int("NPAMD_SLICE_TILES", 0);
+  t.slice_parts = env_int("NPAMD_SLICE_PARTS", 0);
   t.q4_rows = env_int("NPAMD_Q4_ROWS", 0);
   t.q4_rowwise = env_int("NPAMD_Q4_ROWWISE", 1);
   t.q4_rowwise_bf16 = env_int("NPAMD_Q4_ROWWISE_BF16", 0);

@@ -46,11 +46,12 @@ enum Kind : int {
   kRvqGemv, kRvqTile, kRvqDense,
   kQGemv, kQTile, kQDense,
   kRmsNorm, kVqEmbedding, kQEmbedding,
+  kVqSlice,
   kKinds,
 };
 
 // Constant arguments each kind takes, in the order of its entry point (see issue()).
-constexpr int kArgs[kKinds] = {7, 9, 10, 9, 7, 15, 15, 13, 9, 9, 9, 2, 8, 8};
+constexpr int kArgs[kKinds] = {7, 9, 10, 9, 7, 15, 15, 13, 9, 9, 9, 2, 8, 8, 9};
 
 // A dictionary some of whose entries the plan was built from.  CPython stamps a dictionary with a new tag on every
 // change, so an unchanged tag means unchanged entries; after a change the entries themselves are compared.
@@ -312,6 +313,10 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
     case kVqTile:
       rc = npamd_vq_gemm_tile(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
                               ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], ws, ws_bytes, st);
+      break;
+    case kVqSlice:
+      rc = npamd_vq_slice_gemm(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
+                               ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], ws, ws_bytes, st);
       break;
     case kRvqGemv:
       rc = npamd_rvq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]), (int)a[7],

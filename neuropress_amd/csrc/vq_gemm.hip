@@ -1,5 +1,6 @@
-// C-ABI entry points of the tile-decode MFMA GEMM (plain and residual VQ).
+// C-ABI entry points of the tile-decode MFMA GEMM (plain and residual VQ) and of the slice GEMM.
 #include "gemm_tile2.hpp"
+#include "slice_gemm.hpp"
 #include "vq_call.hpp"
 
 using namespace npamd;
@@ -94,6 +95,33 @@ extern "C" int npamd_vq_gemm_tile(const void* x, int64_t ldx, const uint8_t* pac
   c.ws = workspace;
   c.ws_bytes = workspace_bytes;
   return run(c);
+}
+
+extern "C" int npamd_vq_slice_gemm(const void* x, int64_t ldx, const uint8_t* packed, int64_t n_bytes, int bits,
+                                   const void* codebook, int codebook_dtype, int nc, int vl, const float* bias, void* y,
+                                   int64_t ldy, int M, int N, int K, int act_dtype, void* workspace,
+                                   int64_t workspace_bytes, void* stream) {
+  VqCall c{x, ldx, packed, n_bytes, bits, codebook, codebook_dtype, nc, vl,
+               nullptr, 0, 0, nullptr, 0, nullptr, nullptr,
+               bias, y, ldy, M, N, K, act_dtype, (hipStream_t)stream, "npamd_vq_slice_gemm"};
+  const int rc = validate(c, 0);
+  if (rc < 0) return rc;
+  if (rc == 1) return NPAMD_OK;
+  c.ws = workspace;
+  c.ws_bytes = workspace_bytes;
+  const bool takes = fast_ok(c) && c.bits == 16 && c.vl == 8 && c.cb_dtype == c.act && slice_takes(c.M, c.N, c.K, c.nc) && workspace &&
+                     aligned(workspace, 16) && workspace_bytes >= slice_workspace_bytes(c.M, c.N, c.K / 64, c.nc);
+  if (!takes) return run(c);
+  const GemmShape s{c.x, c.ldx, c.bias, c.y, c.ldy, c.M, c.N, c.K, c.K / 64, 0};
+  return launch_slice(c.act, s, c.packed, c.cb, c.nc, c.st, c.what, workspace);
+}
+
+extern "C" int64_t npamd_vq_slice_workspace_bytes(int M, int N, int K, int nc) {
+  return slice_takes(M, N, K, nc) ? slice_workspace_bytes(M, N, K / 64, nc) : 0;
+}
+
+extern "C" int npamd_vq_slice_estimate_ns(int M, int N, int K, int nc) {
+  return slice_takes(M, N, K, nc) ? (int)slice_estimate_ns(M, N, K / 64, nc) : 0;
 }
 
 extern "C" int npamd_rvq_gemm_tile(const void* x, int64_t ldx,

@@ -651,6 +651,39 @@ def vq_gemm_tile(
 # ---------------------------------------------------------------------------
 
 
+def vq_slice_gemm(
+    x: torch.Tensor,
+    packed_indices: torch.Tensor,
+    centroids: torch.Tensor,
+    out_features: int,
+    bias: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """``x @ W.T (+ bias)`` for up to 32 tokens and 16-bit indices into a codebook of 4097 to 65536 rows of eight in x's
+    dtype, whose slices the kernel keeps in LDS (``npamd_vq_slice_gemm``)."""
+    what = "vq_slice_gemm"
+    _check_device(what, x, packed_indices, centroids, bias)
+    x = _x2d(x, what)
+    if x.dtype not in (torch.float16, torch.bfloat16) or centroids.dtype != x.dtype:
+        raise RuntimeError(f"{what}: x must be float16 or bfloat16, and centroids of the same dtype")
+    packed = _packed_u8(packed_indices, what)
+    cb = _centroids_f16(centroids, what)
+    (m, k), n, nc = x.shape, int(out_features), cb.shape[0]
+    y = torch.empty((m, n), device=x.device, dtype=x.dtype)
+    b32 = _bias_f32(bias)
+    need = int(_lib.load().npamd_vq_slice_workspace_bytes(m, n, k, nc))
+    ws = torch.empty(max(need, 16) // 4, device=x.device, dtype=torch.float32)
+    _lib.call(
+        "npamd_vq_slice_gemm", x.data_ptr(), x.stride(0), packed.data_ptr(), packed.numel(), 16, cb.data_ptr(), _DT[cb.dtype],
+        nc, cb.shape[1], _ptr(b32), y.data_ptr(), y.stride(0), m, n, k, _DT[x.dtype], ws.data_ptr(), need, _stream(x),
+    )  # fmt: skip
+    return y
+
+
+def slice_gemm_us(m: int, n: int, k: int, num_centroids: int) -> float:
+    """About how many microseconds :func:`vq_slice_gemm` takes, whatever the indices; 0 for shapes it does not take."""
+    return _lib.load().npamd_vq_slice_estimate_ns(int(m), int(n), int(k), int(num_centroids)) / 1e3
+
+
 def _f16_or_none(t: torch.Tensor | None, what: str) -> torch.Tensor | None:
     if t is None:
         return None
@@ -1001,6 +1034,6 @@ def q_embedding(
 # plans step aside, so that the replacement is called.
 WRAPPERS = {
     fn.__name__: fn
-    for fn in (vq_linear_sliced_checked, vq_linear, vq_gemm_tile, vq_dequant, rvq_linear, rvq_dequant, q_linear, q_gemm_tile,
+    for fn in (vq_linear_sliced_checked, vq_linear, vq_gemm_tile, vq_slice_gemm, vq_dequant, rvq_linear, rvq_dequant, q_linear, q_gemm_tile,
                q_dequant, rms_norm, vq_embedding, q_embedding, dense_linear, gather_columns)
 }  # fmt: skip

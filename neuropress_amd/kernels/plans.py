@@ -17,7 +17,7 @@ _TORCH_CALL = torch.nn.Module.__call__
 _TORCH_LINEAR = torch.nn.functional.linear
 
 (SLICED, VQ_GEMV, VQ_GEMV_PERM, VQ_TILE, VQ_DENSE, RVQ_GEMV, RVQ_TILE, RVQ_DENSE,
- Q_GEMV, Q_TILE, Q_DENSE, RMS_NORM, VQ_EMBEDDING, Q_EMBEDDING) = range(14)  # fmt: skip
+ Q_GEMV, Q_TILE, Q_DENSE, RMS_NORM, VQ_EMBEDDING, Q_EMBEDDING, VQ_SLICE) = range(15)  # fmt: skip
 
 DTYPE_CODES = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32, torch.int64: 3}
 
@@ -98,6 +98,11 @@ def template(plan, kind, n, k, args, dtype, *, f=0.0, k_in=None, perm=None, bias
 def tile_scratch(m: int, n: int, k: int) -> int:
     """Bytes of scratch a tile GEMM of this shape can use."""
     return max(0, int(_lib.load().npamd_gemm_tile_workspace_bytes(m, n, k))) // 4 * 4
+
+
+def slice_scratch(m: int, n: int, k: int, num_centroids: int) -> int:
+    """Bytes of scratch a slice GEMM of this shape needs."""
+    return int(_lib.load().npamd_vq_slice_workspace_bytes(m, n, k, num_centroids))
 
 
 def product_scratch(m: int, n: int, k: int) -> int:

@@ -104,6 +104,15 @@ _GEMV_KERNEL_MAX_TOKENS: int = 32  # what the GEMV entry points accept (NPAMD_GE
 _SLICED_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_SLICED_MAX_TOKENS",), 7)
 _SLICED_MIN_CENTROIDS: int = 4097
 _SLICED_MIN_INDICES: int = _env_int(("NEUROPRESS_VQ_SLICED_MIN_INDICES",), 1 << 20)
+# The slice GEMM (kernels.vq_slice_gemm) for the same layers: whole 8192-row slices of the codebook in LDS, up to 32 tokens at
+# once.  Its time does not depend on the indices, that of the kernels that look rows up in memory does: which one is
+# faster is asked of the times taken when the slice lists were made.  Slice GEMM / fused GEMV or tile GEMM, us at 3 / 16 / 32
+# tokens: 4096 x 14336 with 65536 rows 26 / 28 / 39 against 36 / 39 / 41, with 16384 14.6 / 16.6 / 20.6 against 33.7 / 36.9 / 38.5,
+# 14336 x 4096 with 8192 rows 13.1 / 14.9 / 18.6 against 29.5 / 33.4 / 34.3; 4096 x 4096 with 65536 rows 12.8 / 15 / 20.5 against
+# 12 / 13 / 14, with 8192 8.2 / 8.9 / 11.2 against 10.4 / 11.3 / 12.3.
+_SLICE_GEMM_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_SLICE_GEMM_MAX_TOKENS",), 32)
+_SLICE_GEMM_GATHER_US: float = 3.0  # of a column permutation, which the slice lists and some fused GEMVs apply themselves
+
 # Whether a module that reaches a GPU through .to() / .cuda() / load_state_dict() builds the tensors
 # its kernels derive from the buffers there and then (slice lists: a host round trip per layer).
 _PREPARE_ON_MOVE: bool = _env_int(("NEUROPRESS_VQ_PREPARE_ON_MOVE",), 1) != 0
@@ -189,7 +198,7 @@ _FUSED_BACKENDS = frozenset({VQBackend.CUDA_WMMA, VQBackend.CUDA_LUT, VQBackend.
 _PLAN_ATTRIBUTES = ("backend", "proxy", "residual_proxy", "out_features", "in_features", "vector_len", "bits", "residual_bits",
                     "bias", "column_perm", "packed_residual", "row_scale", "row_bias")  # fmt: skip
 _PLAN_THRESHOLDS = ("_FUSED_MAX_TOKENS", "_FUSED_WIDE_MAX_TOKENS", "_FUSED_WIDE_MAX_ACTIVATIONS", "_SLICED_MAX_TOKENS",
-                    "_SLICED_MIN_CENTROIDS", "_SLICED_MIN_INDICES", "_LUT_MAX_TOKENS", "_TILE_MAX_TOKENS", "_TILE_WIDE_MAX_TOKENS",
+                    "_SLICED_MIN_CENTROIDS", "_SLICED_MIN_INDICES", "_SLICE_GEMM_MAX_TOKENS", "_SLICE_GEMM_GATHER_US", "_LUT_MAX_TOKENS", "_TILE_MAX_TOKENS", "_TILE_WIDE_MAX_TOKENS",
                     "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_BROAD_WEIGHTS", "_TILE_WIDE_BROAD_FEATURES",
                     "_TILE_WIDE_TINY_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS",
                     "_TILE_WIDE_LONG_MAX_TOKENS", "_TILE_WIDE_SMALL_MAX_TOKENS", "_TILE_SMALL_LAYER_MAX_TOKENS",
@@ -766,6 +775,8 @@ class NPVQLinear(nn.Module):
             return self._forward_dequant_gemm(x)
         if band == "tile":
             return self._forward_tile_gemm(x)
+        if band == "slice":
+            return self._forward_slice_gemm(x)
         if self.backend == VQBackend.CUDA_LUT:
             return self._forward_cuda_lut(x)
         if self.backend == VQBackend.CUDA_WMMA or self.backend in _CODED_BACKENDS:
@@ -778,7 +789,7 @@ class NPVQLinear(nn.Module):
 
     def _band(self, x: torch.Tensor, m: int, tracked: bool = False) -> str:
         """Which kernel serves a call of *m* tokens: ``sliced``, ``gemv_perm`` (the GEMV that gathers x's columns),
-        ``fused`` (the backend's GEMV), ``tile``, ``dense`` (decode + GEMM) or ``torch``.
+        ``fused`` (the backend's GEMV), ``slice`` (the slice GEMM), ``tile``, ``dense`` (decode + GEMM) or ``torch``.
 
         *tracked* (``kernels.tracked(x)``): the dense product is the library's, columns are gathered by torch and none
         are padded; the limits are those against that.  What it serves carries gradients, the other kernels do not."""
@@ -786,7 +797,10 @@ class NPVQLinear(nn.Module):
             return "torch"
         if x.dtype not in (torch.float16, torch.bfloat16):
             return "dense"  # fp32 activations: decode + GEMM
-        if m <= min(_SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)) and x.is_cuda and self._sliced_for(m) is not None:
+        sliced = m <= min(_SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)) and x.is_cuda and self._sliced_for(m) is not None
+        if x.is_cuda and not tracked and self._slice_gemm_wins(m):
+            return "slice"
+        if sliced:
             return "sliced"
         if self.column_perm is not None and self._perm_fusable(x, m):
             return "gemv_perm"
@@ -859,9 +873,14 @@ class NPVQLinear(nn.Module):
             number = plan.names[kind, dtype] = self._template(plan, dtype, kind)
         code = plans.DTYPE_CODES[dtype]
         if band == "sliced":
-            sl, limit = self._derived_hit("sliced", self.packed_indices)
-            for tokens in range(1, min(limit, _SLICED_MAX_TOKENS, _fused_max_tokens(self.backend)) + 1):
+            sl, limit, _ = self._derived_hit("sliced", self.packed_indices)
+            most = min(limit, _SLICED_MAX_TOKENS, _fused_max_tokens(self.backend))
+            if self._slice_gemm_wins(most):  # from some token count on: those below this one are the lists'
+                most = m
+            for tokens in range(1, most + 1):
                 plan.route(code, tokens, number, sl.workspace_bytes(tokens))
+        elif band == "slice":
+            plan.route(code, m, number, plans.slice_scratch(m, self.out_features, self._kernel_k(), self.proxy.num_centroids))
         else:
             scratch = plans.tile_scratch if tile else plans.product_scratch if kind == "product" else None
             plan.route(code, m, number, scratch(m, self.out_features, self._kernel_k()) if scratch else 0)
@@ -876,7 +895,7 @@ class NPVQLinear(nn.Module):
         if self.column_perm is not None and kind not in ("sliced", "gemv_perm"):
             perm = self._perm_i64(packed.device) if dtype == torch.float32 else self._perm_i32(packed.device)
         if kind == "sliced":
-            sl, _ = self._derived_hit("sliced", self.packed_indices)
+            sl, _, _ = self._derived_hit("sliced", self.packed_indices)
             i32 = None if self.column_perm is None else self._perm_i32(packed.device)
             plan.hold(sl)  # the plan passes the address of its header
             args = (i32, sl.header_ptr, sl.blob, proxy.centroids_as(dtype), code, self._bias_f32(), code)
@@ -905,7 +924,7 @@ class NPVQLinear(nn.Module):
         args = (stream, stream.numel(), bits, proxy.centroids_as(dtype), code, proxy.num_centroids, vl, self._bias_f32(), code)
         if kind == "gemv_perm":
             return plans.template(plan, plans.VQ_GEMV_PERM, n, k, (*args, self._perm_i32(stream.device)), dtype)
-        kind_code = plans.VQ_TILE if kind == "tile" else plans.VQ_GEMV
+        kind_code = {"tile": plans.VQ_TILE, "slice": plans.VQ_SLICE}.get(kind, plans.VQ_GEMV)
         return plans.template(plan, kind_code, n, self._kernel_k(), args, dtype, k_in=k, perm=perm)
 
     # -- slice-list GEMV ---------------------------------------------------
@@ -959,7 +978,7 @@ class NPVQLinear(nn.Module):
             self._plan = self._new_plan()  # still without routes: every call adds its own
 
     def _build_sliced(self):
-        """(slice lists, most tokens for which they beat the fused GEMV on this layer)."""
+        """(slice lists, most tokens for which they beat the fused GEMV on this layer, the times that say so)."""
         from .. import kernels
 
         sl = kernels.vq_slice_indices(
@@ -967,10 +986,11 @@ class NPVQLinear(nn.Module):
             self.vector_len, self.proxy.num_centroids,
         )  # fmt: skip
         kernels.sliced_workspace(sl.blob.device, sl.workspace_bytes(_SLICED_MAX_TOKENS))
-        return sl, self._sliced_token_limit(sl)
+        return sl, *self._sliced_token_limit(sl)
 
-    def _sliced_token_limit(self, sl) -> int:
-        """Most tokens for which this layer's slice-list GEMV beats its fused GEMV.
+    def _sliced_token_limit(self, sl) -> tuple[int, tuple]:
+        """Most tokens for which this layer's slice-list GEMV beats its fused GEMV, and what was timed: (tokens, us of
+        the slice lists, us of the fused GEMV), up to the first token count at which the lists lose.
 
         With indices spread evenly over the codebook the slice lists win up to
         ``_SLICED_MAX_TOKENS`` by a wide margin.  A skewed index distribution (one codebook
@@ -980,7 +1000,7 @@ class NPVQLinear(nn.Module):
         layer of the size the path is meant for is timed here, once, when its lists are
         built (by ``prepare_sliced``, never by ``forward``)."""
         if self.n_vectors < _SLICED_TUNE_MIN_INDICES:
-            return _SLICED_MAX_TOKENS
+            return _SLICED_MAX_TOKENS, ()
         dev = sl.blob.device
         from .. import kernels
 
@@ -1007,9 +1027,9 @@ class NPVQLinear(nn.Module):
                 t1.record()
                 t1.synchronize()
             torch.cuda.current_stream(dev).wait_stream(side)
-            return t0.elapsed_time(t1)
+            return t0.elapsed_time(t1) * 1e3 / 24
 
-        limit = 0
+        limit, times = 0, []
         try:
             for m in (1, 2, 4, _SLICED_MAX_TOKENS):
                 if m > _SLICED_MAX_TOKENS:
@@ -1019,13 +1039,14 @@ class NPVQLinear(nn.Module):
                 t_sliced = timed(lambda: kernels.vq_linear_sliced(x, sl, cb, workspace=ws))
                 xf = kernels.gather_columns(x, None, self._kernel_k()) if self._kernel_k() != self.in_features else x
                 t_fused = timed(lambda: kernels.vq_linear(xf, stream, cb, bits, self.vector_len, None, self.out_features))
+                times.append((m, t_sliced, t_fused))
                 if t_sliced >= t_fused:
                     break
                 limit = m
         except RuntimeError:
             # e.g. another thread of the process is capturing a graph: keep the measured default
-            return _SLICED_MAX_TOKENS
-        return limit
+            return _SLICED_MAX_TOKENS, ()
+        return limit, tuple(times)
 
     def _sliced_for(self, m: int):
         """The slice lists when they exist for the buffer as it is now and win at *m* tokens, else None.
@@ -1037,8 +1058,38 @@ class NPVQLinear(nn.Module):
             if self._sliced_eligible():
                 _warn_unprepared_once()
             return None
-        sl, limit = hit
+        sl, limit, _ = hit
         return sl if m <= limit else None
+
+    def _slice_gemm_wins(self, m: int) -> bool:
+        """Whether the slice GEMM is the fastest kernel for *m* tokens: its estimate against what was timed on this layer's
+        own indices, the slice lists (between two timed token counts: on the line through them) or, past them, the fused GEMV
+        at the most tokens it was timed with (it does not get faster, and the tile GEMM of 17 to 32 tokens is level with
+        it).  Layers that were not timed -- lists never built, or fewer than 2^20 indices -- do not take it."""
+        if m > _SLICE_GEMM_MAX_TOKENS or self.proxy.num_centroids <= 4096:
+            return False
+        hit = self._derived_hit("sliced", self.packed_indices)
+        if hit is None or not hit[2] or m <= min(hit[1], 1) or self.bits > 16 or self.backend == VQBackend.CUDA_LUT or _FUSED_MAX_TOKENS <= 0:
+            return False
+        cached = self._derived.get("slice_gemm")
+        if cached is None or cached[0] is not hit:
+            cached = self._derived["slice_gemm"] = (hit, {})
+        wins = cached[1].get(m)
+        if wins is None:
+            from .. import kernels
+
+            us = kernels.slice_gemm_us(m, self.out_features, self._kernel_k(), self.proxy.num_centroids)
+            us += _SLICE_GEMM_GATHER_US if us and self.column_perm is not None else 0.0
+            _, limit, times = hit
+            if m <= limit:
+                (m0, t0), (m1, t1) = next(
+                    ((a[0], a[1]), (b[0], b[1])) for a, b in zip((times[0], *times), times) if b[0] >= m or b is times[-1]
+                )  # fmt: skip
+                other = t1 if m1 == m0 else t0 + (t1 - t0) * (m - m0) / (m1 - m0)
+            else:
+                other = times[-1][2]
+            wins = cached[1][m] = 0 < us < other
+        return wins
 
     def _perm_i32(self, device: torch.device) -> torch.Tensor:
         """``column_perm`` as the int32 device tensor the kernels read (cached): in range, negative entries wrapped as
@@ -1296,6 +1347,21 @@ class NPVQLinear(nn.Module):
             _tile_failed = True
             return self._forward_dequant_gemm(x)
         return y
+
+    def _forward_slice_gemm(self, x: torch.Tensor) -> torch.Tensor:
+        """Up to 32 tokens on large layers with codebooks of more than 4096 rows (:meth:`_slice_gemm_wins`)."""
+        from .. import kernels
+
+        *leading, _ = x.shape
+        x2d = x.reshape(-1, self.in_features)
+        if self._kernel_k() != self.in_features:
+            x2d = kernels.gather_columns(x2d, None, self._kernel_k())
+        try:
+            y = kernels.vq_slice_gemm(x2d, self._kernel_stream()[0], self.proxy.centroids_as(x.dtype), self.out_features, self._bias_f32())
+        except RuntimeError as exc:
+            self._fallback("vq_slice_gemm", "decode + GEMM", exc)
+            return self._forward_dequant_gemm(x)
+        return y.reshape(*leading, self.out_features)
 
     def _res_stream(self) -> torch.Tensor:
         if self.packed_residual is not None:
