@@ -11,13 +11,19 @@ namespace {
 // of 2048 tokens x 4096: 20.1 us in turn, 16.7 in eighths; of 4096 tokens 27.6 either way, and the norm alone 11.8 / 13.1).
 constexpr int64_t kAuxDieBytes = (int64_t)24 << 20;
 
-// How the lookups split a token's row of `vectors` pieces of eight values: pieces per thread (vpt), blocks per row
-// (segments), and threads per row and block (lanes).  Short rows share a block of up to 256 threads.
+// How the lookups split a token's row of `vectors` pieces of eight values: pieces per thread (vpt, at most `most`), blocks
+// per row (segments), and threads per row and block (lanes).  Short rows share a block of up to 256 threads.  A thread with
+// one piece has the shortest chain, which is all that few tokens take (1 / 2 pieces, us: VQ lookup of 64 tokens x 4096 2.49 /
+// 2.83, of 256 2.82 / 3.05); many tokens wait for fewer rounds of waves with several (int4 lookup of 4096 tokens x 4096 with
+// 1 / 2 / 4 / 8 pieces 13.3 / 11.4 / 10.6 / 9.8, of 3000 10.0 / 8.7 / 7.6 / 7.7, of 2048 7.0 / 6.3 / 6.5 / 6.7; the VQ lookup, bound by
+// the L2, 15.6 / 15.3 / 15.9 / 15.5).
 struct TokenGrid {
   int vpt, segments;
   unsigned lanes, tokens, threads;
-  TokenGrid(int vectors, int64_t n_ids) {
-    vpt = vectors > 256 && n_ids >= 64 ? 2 : 1;
+  TokenGrid(int vectors, int64_t n_ids, int most) {
+    const int64_t pieces = n_ids * vectors;
+    vpt = vectors <= 256 || pieces < 200000 ? 1 : pieces < 1300000 ? 2 : pieces < 1900000 ? 4 : 8;
+    if (vpt > most) vpt = most;
     segments = (vectors + 256 * vpt - 1) / (256 * vpt);
     const unsigned need = (unsigned)((vectors + segments * vpt - 1) / (segments * vpt));
     lanes = need <= 128 ? need : (need + 63) / 64 * 64;
@@ -276,7 +282,7 @@ int launch_vq_embedding(const int64_t* ids, int64_t n_ids, const uint16_t* idx, 
                         hipStream_t st) {
   const bool scaled = scale != 1.0f;
   if (vl == 8 && aligned16(cb) && aligned16(out) && n_ids <= 0x7FFFFFF0 && groups <= 256 * 65535) {
-    const TokenGrid tg(groups, n_ids);
+    const TokenGrid tg(groups, n_ids, 2);
     const DieGrid rows((n_ids + tg.tokens - 1) / tg.tokens, n_ids * groups * 16, kAuxDieBytes);
     const dim3 grid(rows.blocks, (unsigned)tg.segments);
 #define NPAMD_VQ_EMB(PERM, VPT)                                                                                      \
@@ -317,59 +323,81 @@ __device__ __forceinline__ void store_q_embedding(void* out, int64_t at, float v
   else store_from_f32<OUT>(out, at, f16_bits_to_f32(h) * embed_scale);
 }
 
+// Eight 4-bit codes without a zero point -> eight fp16 values (q - 8) * s, natural order: byte i of the codes (elements 2 i and
+// 2 i + 1) under both halves of a pair, whose exponents read it as (1024 + q, 64 + q); the product of a 4-bit and an
+// 11-bit number is rounded once, as the f32 form rounds it.
+__device__ __forceinline__ void q4_values8(uint32_t codes, uint32_t s2, uint32_t (&h)[4]) {
+#pragma clang fp contract(off)
+  const uint32_t spread[4] = {__builtin_amdgcn_perm(0u, codes, 0x0c000c00u), __builtin_amdgcn_perm(0u, codes, 0x0c010c01u),
+                              __builtin_amdgcn_perm(0u, codes, 0x0c020c02u), __builtin_amdgcn_perm(0u, codes, 0x0c030c03u)};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t pair = (spread[i] & 0x00F0000Fu) | 0x54006400u;
+    const f16x2 q = __builtin_bit_cast(f16x2, pair) - __builtin_bit_cast(f16x2, 0x54806408u);
+    h[i] = __builtin_bit_cast(uint32_t, q * __builtin_bit_cast(f16x2, s2));
+  }
+}
+
 // 4-bit codes, group size a multiple of 8: eight elements (one 32-bit load of codes) at a time, VPT of them per thread;
-// blocks and dies as for the VQ lookup.
-template <int OUT, int VPT>
+// blocks and dies as for the VQ lookup.  Was bound by its vector instructions (19 per element, 92 % of all issue slots at 4096
+// tokens x 4096: 11.6 us): converted two at a time in fp16 where there is no zero point, and the group found by a shift where
+// its size allows (group_shift; -1: by a division), 14.0 -> 9.8 us with the pieces per thread of TokenGrid (3.4 TB/s written).
+template <int OUT, int VPT, bool ZP>
 __global__ void __launch_bounds__(256)
 q4_embedding_kernel(const int64_t* __restrict__ ids, int64_t n_ids, const uint8_t* __restrict__ w_pack,
-                    const uint16_t* __restrict__ scale, const uint16_t* __restrict__ zp, int octets_per_group,
-                    int64_t vocab, int dim, int64_t padding_idx, float embed_scale, bool scaled,
+                    const uint16_t* __restrict__ scale, const uint16_t* __restrict__ zp, int octets_per_group, int group_shift,
+                    int groups, int64_t vocab, int dim, int64_t padding_idx, float embed_scale, bool scaled,
                     void* __restrict__ out, unsigned lanes, unsigned tokens, unsigned per_die) {
   int64_t t;
   int col;
   if (!token_of_thread(lanes, tokens, per_die, &t, &col) || t >= n_ids) return;
-  const int per_row = dim >> 3, groups = per_row / octets_per_group;
+  const int per_row = dim >> 3;
   const int64_t raw = ids[t];
   const int64_t tok = raw < 0 ? 0 : (raw >= vocab ? vocab - 1 : raw);
-  const uint32_t* wrow = reinterpret_cast<const uint32_t*>(w_pack + tok * (dim >> 1));
+  const uint32_t* const wrow = reinterpret_cast<const uint32_t*>(w_pack + tok * (dim >> 1));
+  const uint16_t* const srow = scale + tok * groups;
+  const uint16_t* const zrow = ZP ? zp + tok * groups : nullptr;
   const bool pad = raw == padding_idx;
-  uint32_t codes[VPT];
-  float s[VPT], z[VPT];
+  uint32_t codes[VPT], s[VPT], z[VPT];
   const int step = (int)lanes, o0 = blockIdx.y * step * VPT + col;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {  // columns past the end repeat the last one and are not stored
     const int o = min(o0 + step * j, per_row - 1);
-    const int64_t grp = tok * groups + o / octets_per_group;
+    const int grp = group_shift >= 0 ? o >> group_shift : o / octets_per_group;
     codes[j] = wrow[o];
-    s[j] = f16_bits_to_f32(scale[grp]);
-    z[j] = zp ? f16_bits_to_f32(zp[grp]) : 8.0f;
+    s[j] = srow[grp];
+    if constexpr (ZP) z[j] = zrow[grp];
   }
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     if (o0 + step * j >= per_row) return;
     const int64_t i = t * per_row + o0 + step * j;
-    if constexpr (OUT == NPAMD_F32) {
+    uint32_t h[4];
+    if constexpr (ZP) {
+      const float sf = f16_bits_to_f32(s[j]), zf = f16_bits_to_f32(z[j]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float q = (float)((codes[j] >> (4 * e)) & 0xFu);
-        store_q_embedding<OUT>(out, i * 8 + e, pad ? 0.f : (q - z[j]) * s[j], embed_scale, scaled);
+      for (int e = 0; e < 4; ++e) {
+        const float lo = (float)((codes[j] >> (8 * e)) & 0xFu), hi = (float)((codes[j] >> (8 * e + 4)) & 0xFu);
+        h[e] = pack2<NPAMD_F16>((lo - zf) * sf, (hi - zf) * sf);
       }
     } else {
-      // eight 16-bit results leave as one 16-byte store; same roundings as store_q_embedding
-      uint32_t r[8];
+      q4_values8(codes[j], s[j] * 0x10001u, h);
+    }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float q = (float)((codes[j] >> (4 * e)) & 0xFu);
-        const uint32_t h = f32_to_f16_bits(pad ? 0.f : (q - z[j]) * s[j]);
-        if constexpr (OUT == NPAMD_F16) {
-          r[e] = scaled ? f32_to_f16_bits(f16_bits_to_f32(h) * embed_scale) : h;
-        } else {
-          const uint32_t b = f32_to_bf16_bits(f16_bits_to_f32(h));
-          r[e] = scaled ? f32_to_bf16_bits(bf16_bits_to_f32(b) * embed_scale) : b;
-        }
+    for (int e = 0; e < 4; ++e) h[e] = pad ? 0u : h[e];
+    if constexpr (OUT == NPAMD_F32) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        store_q_embedding<OUT>(out, i * 8 + e, f16_bits_to_f32(e % 2 ? h[e / 2] >> 16 : h[e / 2] & 0xFFFFu), embed_scale, scaled);
+    } else {
+      // eight 16-bit results leave as one 16-byte store; same roundings as store_q_embedding
+      u32x4 r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        r[e] = OUT == NPAMD_F16 ? h[e] : f16x2_to_bf16x2(h[e]);
+        if (scaled) r[e] = pack2<OUT>(act_bits_to_f32<OUT>(r[e] & 0xFFFFu) * embed_scale, act_bits_to_f32<OUT>(r[e] >> 16) * embed_scale);
       }
-      *reinterpret_cast<u32x4*>((uint16_t*)out + i * 8) =
-          u32x4{r[0] | (r[1] << 16), r[2] | (r[3] << 16), r[4] | (r[5] << 16), r[6] | (r[7] << 16)};
+      *reinterpret_cast<u32x4*>((uint16_t*)out + i * 8) = r;
     }
   }
 }
@@ -402,14 +430,22 @@ int launch_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
   const bool scaled = embed_scale != 1.0f;
   if (nbits == 4 && group_size % 8 == 0 && dim % 8 == 0 && (reinterpret_cast<uintptr_t>(w_pack) & 3) == 0 &&
       aligned16(out) && n_ids <= 0x7FFFFFF0) {
-    const TokenGrid tg(dim / 8, n_ids);
+    const TokenGrid tg(dim / 8, n_ids, zp ? 2 : 8);
     const DieGrid rows((n_ids + tg.tokens - 1) / tg.tokens, n_ids * dim * 2, kAuxDieBytes);
     const dim3 grid(rows.blocks, (unsigned)tg.segments);
-#define NPAMD_Q4_EMB(VPT)                                                                                            \
-  launch(q4_embedding_kernel<OUT, VPT>, grid, tg.threads, 0, st, ids, n_ids, w_pack, scale, zp, group_size / 8, vocab, dim,     \
-                                                      padding_idx, embed_scale, scaled, out, tg.lanes, tg.tokens, rows.per_die)
-    if (tg.vpt == 2) NPAMD_Q4_EMB(2);
-    else NPAMD_Q4_EMB(1);
+    const int octets = group_size / 8, shift = (octets & (octets - 1)) == 0 ? __builtin_ctz((unsigned)octets) : -1;
+#define NPAMD_Q4_EMB(VPT, ZP)                                                                                            \
+  launch(q4_embedding_kernel<OUT, VPT, ZP>, grid, tg.threads, 0, st, ids, n_ids, w_pack, scale, zp, octets, shift, dim / group_size, \
+         vocab, dim, padding_idx, embed_scale, scaled, out, tg.lanes, tg.tokens, rows.per_die)
+    if (zp) {
+      if (tg.vpt == 2) NPAMD_Q4_EMB(2, true);
+      else NPAMD_Q4_EMB(1, true);
+    } else {
+      if (tg.vpt == 8) NPAMD_Q4_EMB(8, false);
+      else if (tg.vpt == 4) NPAMD_Q4_EMB(4, false);
+      else if (tg.vpt == 2) NPAMD_Q4_EMB(2, false);
+      else NPAMD_Q4_EMB(1, false);
+    }
 #undef NPAMD_Q4_EMB
   } else {
     const int64_t n = n_ids * dim;

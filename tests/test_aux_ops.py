@@ -192,6 +192,24 @@ def test_q_embedding_kernel_is_bit_exact(gpu, oracle_lib, out_dtype, nbits, grou
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n_ids,dim,group_size", [(70, 4096, 32), (400, 4096, 128), (2600, 4104, 24), (3800, 4096, 32)])
+def test_q4_embedding_of_many_tokens_is_bit_exact(gpu, out_dtype, n_ids, dim, group_size):
+    """One to eight pieces of a row per thread, groups found by a shift and by a division; scales of either sign, zero and
+    below the smallest normal number, which the conversion in fp16 has to round as the f32 form does."""
+    from neuropress_amd import kernels
+
+    vocab = 300
+    codes, blob, scale, _ = _q_table(n_ids, vocab, dim, 4, group_size, False)
+    scale[::3] *= -1
+    scale[1::7] = torch.tensor([3.1e-7, 0.0, -5.2e-6], dtype=torch.float16).repeat(len(scale))[: len(scale[1::7])]
+    ids = torch.randint(0, vocab, (n_ids,), generator=_gen(8))
+    out = kernels.q_embedding(ids.to(gpu), blob.to(gpu), scale.to(gpu), 4, group_size, None, 7, 1.0, out_dtype)
+    want = _torch_q_embedding(ids, codes, scale, None, 4, group_size, 7, 1.0, out_dtype)
+    assert torch.equal(out.cpu().view(torch.int16), want.reshape(n_ids, dim).view(torch.int16))
+
+
+@pytest.mark.gpu
 def test_embedding_wrappers_reject_bad_input(gpu):
     from neuropress_amd import kernels
 
