@@ -118,6 +118,25 @@ def test_rvq_dequant_bit_exact(gpu, oracle_lib, dtype, with_affine):
     _bits_equal(out, ref)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,k,nc,bits,affine", [(1030, 8200, 4096, 12, True), (8300, 1016, 3000, 12, False), (2050, 4096, 1500, 16, True)])
+def test_rvq_dequant_with_both_tables_in_lds_bit_exact(gpu, oracle_lib, dtype, n, k, nc, bits, affine):
+    """Layers of at least 2^20 vectors with a main table of 16 to 64 KiB: rows longer and shorter than a block's 1024
+    vectors and not a multiple of 64, a ragged last run, 12-bit and 16-bit indices.  Checked bit for bit against the oracle."""
+    from neuropress_amd import kernels
+    from neuropress_amd.transforms.vq_packing import IndexPacking
+
+    L = cases.rvq_layer(n + nc, n, k, nc_main=nc, zipf=False)
+    pm = L["pm"] if L["bm"] == bits else IndexPacking.pack(L["im"], bits)
+    sc, wb = (L["scale"], L["wbias"]) if affine else (None, None)
+    args = (None if t is None else orc.to_bits(t) for t in (sc, wb))
+    ref = oracle_lib.rvq_decode(pm.numpy(), bits, L["pr"].numpy(), 8, orc.to_bits(L["cbm"]), orc.to_bits(L["cbr"]), *args, n, k,
+                                orc.torch_dtype_code(dtype))
+    out = kernels.rvq_dequant(pm.to(gpu), bits, L["pr"].to(gpu), 8, L["cbm"].to(gpu), L["cbr"].to(gpu),
+                              None if sc is None else sc.to(gpu), None if wb is None else wb.to(gpu), n, k, dtype)
+    _bits_equal(out, ref)
+
+
 @pytest.mark.parametrize("nbits,gs", [(4, 32), (4, 128), (8, 32), (2, 16), (1, 8), (4, 24)])
 @pytest.mark.parametrize("asym", [False, True])
 @pytest.mark.parametrize("dtype", DTYPES)
