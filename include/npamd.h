@@ -62,6 +62,15 @@ int npamd_vq_dequant(const uint8_t* packed, int64_t n_bytes, int bits,
                      int64_t n_vectors, void* out, int out_dtype, void* stream);
 
 /*
+ * npamd_vq_dequant and npamd_gather_columns (below) of the activations x [M, K] that the product on the decoded weight will
+ * read, in one launch where both are short: with fewer than 1024 rows, vector length 8 and 8 / 12 / 16-bit indices.  Any other
+ * request is the two calls, one after the other.  16-bit activations.
+ */
+int npamd_vq_dequant_gather(const uint8_t* packed, int64_t n_bytes, int bits, const void* codebook_f16, int nc, int vl,
+                            int64_t n_vectors, void* out, int out_dtype, const void* x, int64_t ldx, const int32_t* perm,
+                            void* x_out, int64_t ldo, int M, int K, void* stream);
+
+/*
  * Fused decode GEMV, M <= NPAMD_GEMV_MAX_M:
  *   y[m, n] = sum_k x[m, k] * codebook[idx(n, k/VL), k%VL] (+ bias[n]), f32 accumulate.
  * Replaces vq_linear (neuropress/kernels/vq_linear.cu:344-424) and the GEMV

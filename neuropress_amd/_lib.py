@@ -31,6 +31,7 @@ _RVQ_LINEAR = [_vp, _i64, _vp, _i64, _int, _vp, _i64, _int, _vp, _int, _vp, _int
 _Q_LINEAR = [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _int, _int, _int, _int, _int, _int, _vp]
 SIGNATURES: dict[str, list] = {
     "npamd_vq_dequant": [_vp, _i64, _int, _vp, _int, _int, _i64, _vp, _int, _vp],
+    "npamd_vq_dequant_gather": [_vp, _i64, _int, _vp, _int, _int, _i64, _vp, _int, _vp, _i64, _vp, _vp, _i64, _int, _int, _vp],
     "npamd_vq_gemv": _VQ_LINEAR,
     "npamd_vq_gemv_perm": _VQ_LINEAR[:2] + [_vp] + _VQ_LINEAR[2:],
     "npamd_vq_gemv_perm_supported": [_int] * 6,

@@ -2,6 +2,7 @@
 // embedding lookups of VQ- and int-quantized tables.  All three are bound by
 // HBM traffic (or, at one token, by the launch); none of them has matrix work.
 #include "common.hpp"
+#include "gather_columns.hpp"
 
 using namespace npamd;
 
@@ -455,71 +456,13 @@ int launch_q_embedding(const int64_t* ids, int64_t n_ids, const uint8_t* w_pack,
   return check_launch("npamd_q_embedding");
 }
 
-// ---------------------------------------------------------------------------
-// Activations as the MFMA kernels read them: columns permuted and / or rows padded with zeros to a
-// whole number of 64-column chunks, 16-bit elements:
-//   out[m, k] = x[m, perm ? perm[k] : k] for k < K, 0 for K <= k < ldo and for column numbers that x does not have.
-//
-// Bound by the launch at the token counts of a decode step and by HBM beyond.  With a permutation a block first
-// copies whole rows into LDS (one contiguous read) and gathers there with 2-byte reads: through the vector memory path
-// an element gather costs a lane one cycle and a cache line each (77 x 2184: 2.3 us where torch's gather takes 4.2).
-// Few rows: a block takes 2048 output columns of one, and a row is copied once per block.  Past kGatherBlocks blocks of
-// those a row has only as many as make up that number, which stride over its columns (220 x 13968 10.4 -> 5.8 us), one
-// from 1024 rows on, of two rows at a time then, which share the reads of the permutation.  A row copied by every
-// block of 2048 columns / like this, us: 300 x 13968 20.2 / 7.0, 600 x 4096
-// 7.6 / 4.3, 1200 x 13968 65.0 / 23.5, 4096 x 3456 39.3 / 11.4, 4096 x 14336 195.6 / 54.4 (4.3 TB/s).
-// ---------------------------------------------------------------------------
-constexpr int kGatherRowMax = 32768;  // elements of the rows held in LDS (64 KiB)
-constexpr int kGatherBlocks = 1024, kGatherPairRows = 1024;
+// The gather of gather_columns.hpp, one block's share per block.
 template <bool PERM, bool LDS, int ROWS>
 __global__ void __launch_bounds__(256)
 gather_columns_kernel(const uint16_t* __restrict__ x, int64_t ldx, const int32_t* __restrict__ perm,
                       uint16_t* __restrict__ out, int64_t ldo, int M, int K, bool vec, bool perm_vec) {
   extern __shared__ __attribute__((aligned(16))) uint16_t row_lds[];
-  const int row0 = blockIdx.y * ROWS;
-  const int stride = (K + 7) & ~7;  // elements between the rows in LDS
-  const uint16_t* xr[ROWS];
-#pragma unroll
-  for (int r = 0; r < ROWS; ++r) xr[r] = x + (int64_t)min(row0 + r, M - 1) * ldx;
-  if constexpr (PERM && LDS) {
-    const int whole = vec ? K >> 3 : 0;
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-      uint16_t* const mine = row_lds + r * stride;
-#pragma unroll 4
-      for (int i = threadIdx.x; i < whole; i += 256)
-        reinterpret_cast<u32x4*>(mine)[i] = reinterpret_cast<const u32x4*>(xr[r])[i];
-      for (int i = whole * 8 + threadIdx.x; i < K; i += 256) mine[i] = xr[r][i];
-      xr[r] = mine;
-    }
-    __syncthreads();
-  }
-  for (int64_t c0 = (int64_t)(blockIdx.x * 256 + threadIdx.x) * 8; c0 < ldo; c0 += (int64_t)gridDim.x * 2048) {
-    const int k0 = (int)c0;
-    int at[8];
-    if (PERM && perm_vec && k0 + 8 <= K) {
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(perm + k0), hi = *reinterpret_cast<const u32x4*>(perm + k0 + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        at[e] = (int)lo[e];
-        at[4 + e] = (int)hi[e];
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) at[e] = k0 + e < K ? (PERM ? perm[k0 + e] : k0 + e) : -1;
-    }
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-      if (row0 + r >= M) break;
-      uint16_t v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (unsigned)at[e] < (unsigned)K ? xr[r][at[e]] : (uint16_t)0;
-      u32x4 o;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = (uint32_t)v[2 * e] | ((uint32_t)v[2 * e + 1] << 16);
-      *reinterpret_cast<u32x4*>(out + (int64_t)(row0 + r) * ldo + k0) = o;
-    }
-  }
+  gather_columns_block<PERM, LDS, ROWS>(x, ldx, perm, out, ldo, M, K, vec, perm_vec, blockIdx.x, gridDim.x, blockIdx.y, row_lds);
 }
 
 }  // namespace
@@ -534,20 +477,18 @@ extern "C" int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* p
   const bool vec = aligned16(x) && ldx % 8 == 0;
   auto xs = (const uint16_t*)x;
   auto os = (uint16_t*)out;
-  const unsigned segments = (unsigned)((ldo + 2047) / 2048);
-  const bool lds = perm && K <= kGatherRowMax, pair = lds && M >= kGatherPairRows && 2 * ((K + 7) & ~7) <= kGatherRowMax;
-  const int lds_bytes = ((K + 7) & ~7) * 2;
   const bool pv = aligned16(perm);
   for (int m0 = 0; m0 < M; m0 += 65534) {
     const int rows = M - m0 < 65534 ? M - m0 : 65534;
-    const unsigned per_row = lds ? (unsigned)(M < kGatherBlocks ? kGatherBlocks / M : 1) : segments;
-    const dim3 grid(per_row < segments ? per_row : segments, (unsigned)(pair ? (rows + 1) / 2 : rows));
+    GatherPlan plan(perm != nullptr, ldo, M, K);
+    const dim3 grid(plan.segments, (unsigned)(plan.pair ? (rows + 1) / 2 : rows));
     const uint16_t* xm = xs + (int64_t)m0 * ldx;
     uint16_t* om = os + (int64_t)m0 * ldo;
-    if (!perm) launch(gather_columns_kernel<false, false, 1>, grid, 256, 0, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);
-    else if (pair) launch(gather_columns_kernel<true, true, 2>, grid, 256, 2 * lds_bytes, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);
-    else if (lds) launch(gather_columns_kernel<true, true, 1>, grid, 256, lds_bytes, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);
-    else launch(gather_columns_kernel<true, false, 1>, grid, 256, 0, st, xm, ldx, perm, om, ldo, rows, K, vec, pv);
+    const auto go = [&](auto kernel) { launch(kernel, grid, 256, plan.lds_bytes, st, xm, ldx, perm, om, ldo, rows, K, vec, pv); };
+    if (!perm) go(gather_columns_kernel<false, false, 1>);
+    else if (plan.pair) go(gather_columns_kernel<true, true, 2>);
+    else if (plan.lds) go(gather_columns_kernel<true, true, 1>);
+    else go(gather_columns_kernel<true, false, 1>);
   }
   return check_launch("npamd_gather_columns");
 }

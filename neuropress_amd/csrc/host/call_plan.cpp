@@ -234,13 +234,16 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   const std::vector<int64_t>& a = t.a;
   c10::SmallVector<int64_t, 6> sizes(x_in.sizes().begin(), x_in.sizes().end());
   at::Tensor x = x_in;
+  const int64_t ldx_in = ldx;
+  bool with_gather = false;
   if (t.perm.defined() && t.perm.scalar_type() == at::kLong) {
     x = at::index_select(x_in, -1, t.perm);
     ldx = t.k;
   } else if (t.perm.defined() || t.k_in != t.k) {
     sizes.back() = t.k;
     x = empty(sizes, x_in.scalar_type(), device);
-    if (npamd_gather_columns(x_in.const_data_ptr(), ldx, t.perm.defined() ? t.perm.const_data_ptr<int32_t>() : nullptr, x.data_ptr(),
+    with_gather = t.kind == kVqDense && t.own;  // its decode gathers them too
+    if (!with_gather && npamd_gather_columns(x_in.const_data_ptr(), ldx, t.perm.defined() ? t.perm.const_data_ptr<int32_t>() : nullptr, x.data_ptr(),
                              t.k, (int)m, (int)t.k_in, st) != NPAMD_OK)
       return false;
     ldx = t.k;
@@ -253,7 +256,11 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
     if (t.own && (ldx % 8 || ((uintptr_t)x.const_data_ptr() & 15))) return false;
     at::Tensor w = empty({t.n, t.k}, t.out, device);
     int rc;
-    if (t.kind == kVqDense)
+    if (with_gather)
+      rc = npamd_vq_dequant_gather(ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], a[6], w.data_ptr(), code,
+                                   x_in.const_data_ptr(), ldx_in, t.perm.defined() ? t.perm.const_data_ptr<int32_t>() : nullptr,
+                                   x.data_ptr(), t.k, (int)m, (int)t.k_in, st);
+    else if (t.kind == kVqDense)
       rc = npamd_vq_dequant(ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], a[6], w.data_ptr(), code, st);
     else if (t.kind == kRvqDense)
       rc = npamd_rvq_dequant(ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]), (int)a[7],

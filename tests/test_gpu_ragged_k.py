@@ -120,3 +120,29 @@ def test_layers_prepare_before_their_codebook_arrives(gpu):
     x = torch.randn(3, 200, generator=cases.gen(1)).half()
     ref = torch.nn.functional.linear(x.float(), L["cb"][L["idx"]].reshape(70, 200).float())
     assert torch.allclose(layer(x.to(gpu)).float().cpu(), ref, rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits,nc", [(8, 200), (12, 900), (16, 65536)])
+@pytest.mark.parametrize("m,k,perm", [(1, 72, True), (77, 2184, True), (1023, 456, False), (300, 5000, True), (5, 8200, False), (1030, 264, True)])
+def test_decode_and_gather_in_one_launch(gpu, dtype, bits, nc, m, k, perm):
+    """What the one launch writes is what the decode and the gather write one after the other: rows shorter and longer than a
+    block's 2048 columns, one and many, rows at a distance, the most rows it takes and more (the two calls), a weight of a
+    ragged number of vectors."""
+    from neuropress_amd import _lib, kernels
+    from neuropress_amd.transforms.vq_packing import IndexPacking
+
+    n, width = 37, (k + 63) // 64 * 64
+    g = torch.Generator().manual_seed(m + k + bits)
+    packed = IndexPacking.pack(torch.randint(0, nc, (n * width // 8,), generator=g), bits).to(gpu)
+    cb = torch.randn(nc, 8, generator=g).half().to(gpu)
+    x = torch.randn(m, k + 8, generator=g).to(dtype).to(gpu)[:, :k]
+    p = torch.randperm(k, generator=g).int().to(gpu) if perm else None
+    w = torch.full((n, width), 7.0, dtype=dtype, device=gpu)
+    out = torch.full((m, width), 7.0, dtype=dtype, device=gpu)
+    code = _lib.F16 if dtype == torch.float16 else _lib.BF16
+    _lib.call("npamd_vq_dequant_gather", packed.data_ptr(), packed.numel(), bits, cb.data_ptr(), nc, 8, n * width // 8, w.data_ptr(), code,
+              x.data_ptr(), x.stride(0), p.data_ptr() if perm else None, out.data_ptr(), width, m, k,
+              torch.cuda.current_stream().cuda_stream)  # fmt: skip
+    assert torch.equal(w, kernels.vq_dequant(packed, cb, bits, n, width, dtype))
+    assert torch.equal(out, kernels.gather_columns(x, p, width))
