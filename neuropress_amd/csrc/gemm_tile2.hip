@@ -386,13 +386,13 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   block_sync_lds();
 
-  // The word through which the two halves of K meet is looked at a step before the loop ends, so that
-  // the look costs no round trip after it: a stale "not there yet" only means that this half
-  // writes its tile, and the swap that follows decides.
-  unsigned long long* const word = pair.words + (by * gridDim.x + bx);
+  // The halves of K meet through two words per tile.  A step before its loop ends a half swaps the call's number into
+  // the first, so that the swap costs no round trip after it: the one that finds something else there is the first
+  // and will write its tile, the other will wait for that and add it.
+  unsigned long long* const word = pair.words + 2 * (by * gridDim.x + bx);
   unsigned long long early = 0;
-  auto early_look = [&] {
-    if (s.splits == 2 && tid == 0) early = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  auto announce = [&] {
+    if (s.splits == 2 && tid == 0) early = __hip_atomic_exchange(word, pair.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
 
   f32x16 acc[MW][2];
@@ -466,7 +466,7 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
     }
     one_step(0, steps - 2, wslot, 1);
     next_slot();
-    early_look();
+    announce();
     one_step(1, steps - 1, wslot, 0);
   } else {
     // No rows of this pair of waves lie inside M: they still decode their share of the weights.
@@ -495,8 +495,8 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
     unsigned long long* const flag = reinterpret_cast<unsigned long long*>(stage);  // read for the last time two steps ago
     if (tid == 0) flag[0] = early;
     __syncthreads();  // every wave is past its last LDS read
-    bool arrived = flag[0] == pair.call;  // the other half is there already: nothing to write
-    if (!arrived) {
+    finish = flag[0] == pair.call;
+    if (!finish) {
       if (wave_active) {
 #pragma unroll
         for (int mt = 0; mt < MW; ++mt)
@@ -509,13 +509,18 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tile is where the other workgroup will read it
       __syncthreads();
-      if (tid == 0) flag[1] = __hip_atomic_exchange(word, pair.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      arrived = flag[1] == pair.call;  // it came while this half was being written
+      if (tid == 0) __hip_atomic_store(word + 1, pair.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
     }
-    finish = arrived;
-    if (finish) {
-      if (tid == 0) __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for a replay of this call
+    {
+      if (tid == 0) {
+        // The other half is past the swap of its own, so it is running its last steps or writing, and waits for nobody.
+        while (__hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != pair.call) __builtin_amdgcn_s_sleep(4);
+        // for a replay of this call
+        __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(word + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
       if (wave_active) {
         // The other half's tile in one round trip: buffer loads of agent scope (cache policy sc1),
         // which the compiler, unlike atomic loads, leaves in flight together.
@@ -612,7 +617,7 @@ int launch_tile2_prod(GemmShape s, const typename Prods::Args& a, hipStream_t st
   if (s.splits == 2) {
     const int64_t tiles = (int64_t)((s.N + kT2Cols - 1) / kT2Cols) * ((s.M + 128 * mw - 1) / (128 * mw));
     pair.words = (unsigned long long*)workspace;
-    pair.tiles = (float*)((uint8_t*)workspace + ((tiles * 8 + 255) & ~(int64_t)255));
+    pair.tiles = (float*)((uint8_t*)workspace + ((tiles * 16 + 255) & ~(int64_t)255));
     pair.call = next_call_number();
   }
   switch (mw) {
