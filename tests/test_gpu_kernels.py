@@ -119,10 +119,12 @@ def test_rvq_dequant_bit_exact(gpu, oracle_lib, dtype, with_affine):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("n,k,nc,bits,affine", [(1030, 8200, 4096, 12, True), (8300, 1016, 3000, 12, False), (2050, 4096, 1500, 16, True)])
+@pytest.mark.parametrize("n,k,nc,bits,affine", [(1030, 8200, 4096, 12, True), (8300, 1016, 3000, 12, False), (2050, 4096, 1500, 16, True),
+                                                 (3100, 4600, 65536, 16, True)])
 def test_rvq_dequant_with_both_tables_in_lds_bit_exact(gpu, oracle_lib, dtype, n, k, nc, bits, affine):
     """Layers of at least 2^20 vectors with a main table of 16 to 64 KiB: rows longer and shorter than a block's 1024
-    vectors and not a multiple of 64, a ragged last run, 12-bit and 16-bit indices.  Checked bit for bit against the oracle."""
+    vectors and not a multiple of 64, a ragged last run, 12-bit and 16-bit indices; and one whose main table stays in memory,
+    two vectors per thread.  Checked bit for bit against the oracle."""
     from neuropress_amd import kernels
     from neuropress_amd.transforms.vq_packing import IndexPacking
 
