@@ -59,12 +59,12 @@ struct DenseTile {
   static constexpr int kWaves = WGM * WGN;  // of one K group
   static constexpr int kThreads = 64 * kWaves * KG;
   static constexpr int kStageBytes = (kBM + kBN) * 128;
-  static constexpr int kLoadsX = kBM / 8 / kWaves, kLoadsW = kBN / 8 / kWaves;  // per wave and step
+  static constexpr int kPiecesX = kBM / 8, kPiecesW = kBN / 8;  // a load's worth of rows
+  static constexpr int kLoadsX = (kPiecesX + kWaves - 1) / kWaves, kLoadsW = (kPiecesW + kWaves - 1) / kWaves;  // per wave and step
   static constexpr int kRedBytes = (KG - 1) * kBM * kBN * 4;
   static constexpr int kEpBytes = kBM * kBN * 2;
   static constexpr int kRingBytes = KG * STAGES * kStageBytes;
   static constexpr int kLds = kRingBytes > kRedBytes + kEpBytes ? kRingBytes : kRedBytes + kEpBytes;
-  static_assert(kBM / 8 % kWaves == 0 && kBN / 8 % kWaves == 0, "every wave loads whole pieces of one operand at a time");
   // The first operands of a step are read before its barrier where the ring is deep enough for a step to arrive one
   // barrier early with two more on their way (128 x 64 tiles, ring of six: 23.0 -> 20.7 us on 384 x 4096 x 4096; 64 x 128
   // in two groups, ring of three: 19.9 -> 29.3, the loads no longer cover the memory's latency).
@@ -95,11 +95,15 @@ dense_gemm_kernel(const DenseShape s) {
   const int base = steps / KG;                    // steps every group has
   const uint8_t* const xb = reinterpret_cast<const uint8_t*>(s.x) + (int64_t)m0 * s.ldx * 2 + (int64_t)step0 * 128;
   const uint8_t* const wb = reinterpret_cast<const uint8_t*>(s.w) + (int64_t)n0 * s.ldw * 2 + (int64_t)step0 * 128;
+  // The piece of its operand that load i brings.  Where the waves don't divide the pieces, the last is brought more than once.
+  auto piece_of = [&](int i) {
+    return i < T::kLoadsX ? min(wave + T::kWaves * i, T::kPiecesX - 1) : min(wave + T::kWaves * (i - T::kLoadsX), T::kPiecesW - 1);
+  };
   uint32_t voff[T::kLoadsX + T::kLoadsW];
 #pragma unroll
   for (int i = 0; i < T::kLoadsX + T::kLoadsW; ++i) {
     const bool is_x = i < T::kLoadsX;
-    const int r = (wave + T::kWaves * (is_x ? i : i - T::kLoadsX)) * 8 + (lane >> 3);
+    const int r = piece_of(i) * 8 + (lane >> 3);
     const int row = is_x ? min(r, s.M - 1 - m0) : min(r, s.N - 1 - n0);  // rows past the end: a valid row nobody stores
     voff[i] = (uint32_t)((int64_t)row * (is_x ? s.ldx : s.ldw) * 2) + (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
   }
@@ -107,7 +111,7 @@ dense_gemm_kernel(const DenseShape s) {
   auto load = [&](int i, int slot, int it) {
     const bool is_x = i < T::kLoadsX;
     const uint8_t* src = uniform_ptr((is_x ? xb : wb) + (int64_t)(g + KG * it) * 128);
-    const uint32_t piece = (uint32_t)((is_x ? 0 : T::kBM / 8) + wave + T::kWaves * (is_x ? i : i - T::kLoadsX));
+    const uint32_t piece = (uint32_t)((is_x ? 0 : T::kPiecesX) + piece_of(i));
     lds_load16(ring + (uint32_t)(slot * T::kStageBytes) + piece * 1024u, voff[i], src);
   };
 
@@ -291,8 +295,9 @@ constexpr DenseCost kDenseCost[] = {
     {128, 128, 1, 0.00f, 0.375f, 0.045f, 4.55f}, // 4 waves
     {256, 128, 1, 0.00f, 0.622f, 0.053f, 4.39f}, // 8 waves
     {192, 128, 1, 0.00f, 0.515f, 0.040f, 4.20f}, // 4 waves of 96 x 64: fewest LDS reads per MFMA
+    {96, 64, 2, 1.80f, 0.450f, 0.028f, 2.10f},   // 6 waves; only in the place of 64 x 128
 };
-constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]);
+constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]), kDenseTile64x128 = 2, kDenseTile96 = 7;
 
 template <int ACT>
 int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
@@ -303,7 +308,8 @@ int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
     case 3: return launch_dense_tile<ACT, 4, 2, 1, 1, 5>(s, st);
     case 4: return launch_dense_tile<ACT, 2, 2, 2, 1, 5>(s, st);
     case 5: return launch_dense_tile<ACT, 4, 2, 2, 1, 3>(s, st);
-    default: return launch_dense_tile<ACT, 2, 2, 3, 1, 4>(s, st);
+    case 6: return launch_dense_tile<ACT, 2, 2, 3, 1, 4>(s, st);
+    default: return launch_dense_tile<ACT, 3, 1, 1, 2, 4>(s, st);
   }
 }
 
@@ -318,7 +324,10 @@ struct DensePlan {
   float us;
 };
 
-// The tile and split of least estimate.
+// The tile and split of least estimate.  96 x 64 is looked at where 64 x 128 would be taken whole and K is 2048 or more: it
+// loads fewer bytes per compute unit where it fills more of them (384 x 4096: 256 tiles against 192).  384 x 4096 x 4096
+// 23.5 -> 21.6 us; 38 drawn shapes of 65 to 1330 rows where its estimate is lower 1.01 to 1.17 x, geometric mean 1.07.  At
+// K < 2048 0.93 to 1.05 x; against the other tiles, and with K in parts, 0.81 to 1.04 x where the estimates are this close.
 DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits) {
   DensePlan best{0, 1, 1e30f};
   const int steps = K / 64;
@@ -326,10 +335,11 @@ DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits) {
   const int forced_splits = forced < most ? forced : most;
   for (int i = 0; i < kDenseTiles; ++i) {
     if (forced_tile > 0 && forced_tile <= kDenseTiles && i != forced_tile - 1) continue;
+    if (i == kDenseTile96 && !forced_tile && (best.tile != kDenseTile64x128 || best.splits > 1 || steps < 32)) continue;
     const DenseCost& c = kDenseCost[i];
     const int64_t tiles = (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
     const float load = (float)tiles * steps * (c.bm + c.bn) * 128e-6f * c.per_mb;
-    for (int splits = 1; splits <= max_splits; ++splits) {
+    for (int splits = 1; splits <= (i == kDenseTile96 && !forced_tile ? 1 : max_splits); ++splits) {
       if (forced_splits > 0 && splits != forced_splits) continue;
       if (forced_splits <= 0 && splits > 1 && (steps < kDenseMinSplitSteps * splits || tiles * splits > 512)) break;
       const int64_t rounds = ((tiles * splits + 7) / 8 + 31) / 32;

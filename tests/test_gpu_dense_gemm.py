@@ -66,6 +66,30 @@ def test_dense_gemm_parts_of_k(gpu, dense_tile, monkeypatch, tile, splits, act):
         assert bool(((y - ref).abs() <= tol * ref.abs() + 1e-4).all()), (tile, splits, m, n, k, float((y - ref).abs().max()))
 
 
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("splits", [0, 3])
+def test_dense_gemm_96_rows(gpu, dense_tile, monkeypatch, splits, act):
+    """Tiles of 96 x 64, whose three waves share eight pieces of W: the same sums in the same order as 64 x 128's, whole and
+    in parts, around the edges of both; and where the plan takes them by itself."""
+    from neuropress_amd import kernels
+
+    monkeypatch.setenv("NPAMD_DENSE_SPLITS", str(splits))
+    for m, n, k in ((1, 1, 64), (95, 63, 192), (96, 64, 448), (97, 65, 512), (193, 129, 576), (384, 200, 1088), (300, 2560, 2048)):
+        g = cases.gen(m + n + k)
+        x = torch.randn(m, k, generator=g).to(act).to(gpu)
+        w = (torch.randn(n, k, generator=g) * 0.05).to(act).to(gpu)
+        bias = torch.randn(n, generator=g).to(gpu)
+        out = []
+        for tile in (3, 8, 0):
+            dense_tile(tile)
+            out.append(kernels.dense_linear(x, w, bias))
+        ref = x.double() @ w.double().T + bias.double()
+        tol = 2.0 ** (-10 if act == torch.float16 else -7)  # the rounding of the output, and f32 sums
+        assert torch.equal(out[0], out[1]), (m, n, k)
+        for y in out[1:]:
+            assert bool(((y.double() - ref).abs() <= tol * ref.abs() + 1e-4).all()), (m, n, k)
+
+
 def test_dense_linear_copies_rows_the_kernel_does_not_take(gpu):
     """Dense rows at an odd address, one row at an odd distance, rows far apart: each equals the product of the copy."""
     from neuropress_amd import kernels
