@@ -9,6 +9,7 @@
 
 #include "gemm_tile2.hpp"
 #include "gemv.hpp"
+#include "q_gemv.hpp"
 
 namespace npamd {
 
@@ -627,12 +628,25 @@ static bool q4_rowwise_ok(const QCall& c) {
          ptr_aligned(c.scale, 2) && tuning().q4_rowwise != 0;
 }
 
+// Which GEMV calls take q_gemv_kernel (q_gemv.hpp): all but those of few rows whose K fused_gemv_kernel splits over the columns of
+// a tile (up to half the compute units have a 16-row tile; us, fused_gemv / q_gemv: 1024 x 4096 int4 3.8 / 4.4 at one
+// token and 4.6 / 4.7 at 8, 2048 x 8192 with zero points 7.2 / 8.1 at 8; 2880 x 4736 8.6 / 6.0, 512 x 2048 at 16 4.0 / 3.4), and, by
+// what the arguments are, those whose scales are no whole dwords or whose rows of x are too far apart for 32-bit offsets.
+static bool q_gemv_takes_shape(int M, int N, int chunks) {
+  return plan_gemv_parts(M, N, chunks, 0) == 1 || 2 * ((N + 15) / 16) > device_cus_q4();
+}
+static bool q_gemv_takes(const QCall& c) {
+  return q_gemv_takes_shape(c.M, c.N, c.K / 64) && ptr_aligned(c.scale, 4) && (!c.zp || ptr_aligned(c.zp, 4)) &&
+         (int64_t)c.N * (c.K / c.gs) % 2 == 0 && c.ldx < (1 << 26) && c.K < (1 << 24);
+}
+
 template <int ACT, bool ASYM>
 static int q4_fused(const QCall& c, bool gemv) {
   using P = Q4Provider<ACT, ASYM>;
   typename P::Args a{c.w_pack, (const uint16_t*)c.scale, c.K / 64, c.K / c.gs, log2i(c.gs / 32), (const uint16_t*)c.zp};
   if (gemv) {
     GemvShape s{c.x, c.ldx, c.bias, c.y, c.ldy, c.M, c.N, c.K / 64, 0, 0};
+    if (q_gemv_takes(c)) return launch_q_gemv<ACT, 4, ASYM, P>(s, a, device_cus_q4(), c.st, c.what);
     return launch_fused_gemv<ACT, P>(s, a, c.st, c.what);
   }
   GemmShape s{c.x, c.ldx, c.bias, c.y, c.ldy, c.M, c.N, c.K, c.K / 64, 0};
@@ -640,6 +654,7 @@ static int q4_fused(const QCall& c, bool gemv) {
 }
 
 int npamd::q_gemv_plan_stages(int M, int N, int K) {
+  if (q_gemv_takes_shape(M, N, K / 64)) return 1;
   int staged = 0;
   GemvShape s{nullptr, K, nullptr, nullptr, N, M, N, K / 64, 0, 0};
   s.plan_only = &staged;
@@ -655,6 +670,7 @@ static int q8_fused(const QCall& c, bool gemv) {
   typename P::Args a{c.w_pack, (const uint16_t*)c.scale, c.K / 64, c.K / c.gs, log2i(c.gs / 32), (const uint16_t*)c.zp};
   if (gemv) {
     GemvShape s{c.x, c.ldx, c.bias, c.y, c.ldy, c.M, c.N, c.K / 64, 0, 0};
+    if (q_gemv_takes(c)) return launch_q_gemv<ACT, 8, ASYM, P>(s, a, device_cus_q4(), c.st, c.what);
     return launch_fused_gemv<ACT, P>(s, a, c.st, c.what);
   }
   GemmShape s{c.x, c.ldx, c.bias, c.y, c.ldy, c.M, c.N, c.K, c.K / 64, 0};

@@ -327,11 +327,15 @@ class NPLinear(nn.Module):
             self._derived["mfma_layer"] = ok
         return ok
 
-    def _tile_grid_fills_gpu(self, x: torch.Tensor, m: int, tracked: bool = False) -> bool:
+    def _compute_units(self) -> int:
         cus = self._derived.get("cus")
         if cus is None:
-            cus = torch.cuda.get_device_properties(x.device).multi_processor_count
+            cus = torch.cuda.get_device_properties(self.u8_blob.device).multi_processor_count
             self._derived["cus"] = cus
+        return cus
+
+    def _tile_grid_fills_gpu(self, x: torch.Tensor, m: int, tracked: bool = False) -> bool:
+        cus = self._compute_units()
         if tracked:
             return tile_band_ok(m, self.out_features, self.in_features, cus, _Q_TILE_MIN_GRID_FRACTION,
                                 _Q_TILE_SPLIT_LIBRARY_MAX_TOKENS, _Q_TILE_SPLIT_LONG_K, library=True)  # fmt: skip
@@ -342,18 +346,23 @@ class NPLinear(nn.Module):
             4096 if self.zero_point is None else 6144,
         )  # fmt: skip
 
-    def _gemv_max_tokens(self, m: int) -> int:
-        """End of the GEMV band for a call of *m* tokens: 16, or 32 while x stays small."""
+    def _gemv_max_tokens(self, m: int, tracked: bool = False) -> int:
+        """End of the GEMV band for a call of *m* tokens: 16, or 32 while x stays small or the kernel stages it.  *tracked*: as it
+        is against decode + the library's product, which such calls take past it."""
         if _Q_FUSED_MAX_TOKENS < m <= _Q_FUSED_WIDE_MAX_TOKENS:
             cap = _Q_FUSED_WIDE_MAX_ACTIVATIONS.get(self.nbits, 0)
             if self.zero_point is not None and self.nbits == 4:
                 cap = 1 << 30  # the fused GEMM pays for the zero points per tile: GEMV at any K
             if m * self.in_features <= cap:
                 return _Q_FUSED_WIDE_MAX_TOKENS
-            # One row tile per workgroup: the GEMV stages its activations through LDS and stays
-            # ahead of the tile GEMM at any K (int4, GEMV vs tile GEMM at 17 / 24 / 32 tokens:
-            # 4096 x 14336 23.6 / 24.4 / 25.6 vs 29.5-29.9 us, 4096 x 8192 15.2 / 15.0 / 15.6 vs 21.8-22.5 us).
-            if self.nbits == 4:
+            # A GEMV that stages its activations through LDS stays ahead of the tile GEMM at any K (GEMV at 24 / 32 tokens, tile
+            # GEMM at 33, us: 4096 x 14336 int4 19.6 / 21.3, 30.7, int8 24.0 / 24.7, 35; 5888 x 7168 int4 15.7 / 16.6).
+            # Where gradients may flow the line is part of what the module does and stays where it was: int4 layers
+            # of fewer than 1.2 row tiles per compute unit.
+            if tracked:
+                few = -(-self.out_features // 16) * 10 < 12 * self._compute_units()
+                return _Q_FUSED_WIDE_MAX_TOKENS if self.nbits == 4 and few else _Q_FUSED_MAX_TOKENS
+            if self.nbits in (4, 8):
                 from .. import kernels
 
                 if kernels.gemv_stages_activations(m, self.out_features, self.in_features, 0):
@@ -403,7 +412,7 @@ class NPLinear(nn.Module):
         # dense GEMM (14336 x 4096, 8 bits: 99 us against 57 us at one token, 452 against 57 at 16).
         if x.dtype not in (torch.float16, torch.bfloat16) or not self._mfma_layer():
             return "dense"
-        if m <= self._gemv_max_tokens(m):
+        if m <= self._gemv_max_tokens(m, tracked):
             return "fused"
         limit = _Q_TILE_MAX_TOKENS
         if self.in_features >= _Q_TILE_SPLIT_LONG_K:
