@@ -236,6 +236,45 @@ struct RvqProvider {
   }
 };
 
+// (v & mask) | bits in one instruction: an instruction reads one constant from outside the vector registers, and with
+// two of them the compiler takes two.
+__device__ __forceinline__ uint32_t and_or(uint32_t v, uint32_t mask, uint32_t bits) {
+  asm("" : "+v"(bits));
+  return (v & mask) | bits;
+}
+
+// Two weights of the group-affine formats whose products are formed in f32: (q - z) * s, the difference and the product each
+// rounded to f32, then to the activation type.  The fp16 factors are widened by the multiply-add itself (v_fma_mix_f32), with a
+// term that changes nothing: minus zero behind a product (the sign of a zero included), a factor of one in front of the
+// zero point.  The compiler would fold a minus zero it sees into a multiplication with conversions of its own.
+template <int ACT, bool ASYM>
+__device__ __forceinline__ uint32_t scaled_pair(f16x2 q, f16x2 s, float zf) {
+#pragma clang fp contract(off)
+  float lo, hi;
+  if constexpr (ASYM) {
+    float one = 1.0f;
+    asm("" : "+v"(one));
+    lo = __builtin_fmaf((float)q.x, one, -zf) * (float)s.x;
+    hi = __builtin_fmaf((float)q.y, one, -zf) * (float)s.x;
+  } else {
+    float nothing = -0.0f;
+    asm("" : "+v"(nothing));
+    lo = __builtin_fmaf((float)q.x, (float)s.x, nothing);
+    hi = __builtin_fmaf((float)q.y, (float)s.x, nothing);
+  }
+  if constexpr (ACT == NPAMD_F16) {
+    f16x2 h;
+    h.x = (_Float16)lo;
+    h.y = (_Float16)hi;
+    return __builtin_bit_cast(uint32_t, h);
+  } else {
+    bf16x2 b;
+    b.x = (__bf16)lo;
+    b.y = (__bf16)hi;
+    return __builtin_bit_cast(uint32_t, b);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // int4, group size a multiple of 32; symmetric (zero point 8) or, with ASYM, a
 // per-group fp16 zero point.
@@ -319,14 +358,13 @@ struct Q4Provider {
   __device__ __forceinline__ u32x4 dequant8(uint32_t w, uint32_t s2, uint32_t z) const {
 #pragma clang fp contract(off)
     uint32_t o[4];
-    const float sf = f16_bits_to_f32(s2 & 0xFFFFu);
     const float zf = ASYM ? f16_bits_to_f32(z & 0xFFFFu) : 0.f;
     // byte i of w into bytes 0 and 2 (bytes 1 and 3: zero)
     const uint32_t spread[4] = {__builtin_amdgcn_perm(0u, w, 0x0c000c00u), __builtin_amdgcn_perm(0u, w, 0x0c010c01u),
                                 __builtin_amdgcn_perm(0u, w, 0x0c020c02u), __builtin_amdgcn_perm(0u, w, 0x0c030c03u)};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t pair = (spread[i] & 0x00F0000Fu) | 0x54006400u;  // (1024 + q[2i], 64 + q[2i+1])
+      const uint32_t pair = and_or(spread[i], 0x00F0000Fu, 0x54006400u);  // (1024 + q[2i], 64 + q[2i+1])
       if constexpr (ACT == NPAMD_F16 && !ASYM) {
         // minus (1032, 72) -> q - 8 exactly; times the scale: one rounding.
         const f16x2 q = __builtin_bit_cast(f16x2, pair) - __builtin_bit_cast(f16x2, 0x54806408u);
@@ -334,24 +372,7 @@ struct Q4Provider {
       } else {
         // q (ASYM) or q - 8 exactly, in fp16; the rest in f32.
         const f16x2 q = __builtin_bit_cast(f16x2, pair) - __builtin_bit_cast(f16x2, ASYM ? 0x54006400u : 0x54806408u);
-        float lo = (float)q.x, hi = (float)q.y;
-        if constexpr (ASYM) {
-          lo -= zf;
-          hi -= zf;
-        }
-        lo *= sf;
-        hi *= sf;
-        if constexpr (ACT == NPAMD_F16) {
-          f16x2 h;
-          h.x = (_Float16)lo;
-          h.y = (_Float16)hi;
-          o[i] = __builtin_bit_cast(uint32_t, h);
-        } else {
-          bf16x2 b;
-          b.x = (__bf16)lo;
-          b.y = (__bf16)hi;
-          o[i] = __builtin_bit_cast(uint32_t, b);
-        }
+        o[i] = scaled_pair<ACT, ASYM>(q, __builtin_bit_cast(f16x2, s2), zf);
       }
     }
     return u32x4{o[0], o[1], o[2], o[3]};
@@ -434,7 +455,6 @@ struct Q8Provider {
   // Eight bytes (two dwords) -> one operand.
   __device__ __forceinline__ u32x4 dequant8(uint32_t d0, uint32_t d1, uint32_t s2, uint32_t z) const {
 #pragma clang fp contract(off)
-    const float sf = f16_bits_to_f32(s2 & 0xFFFFu);
     const float zf = ASYM ? f16_bits_to_f32(z & 0xFFFFu) : 0.f;
     const uint32_t pairs[4] = {__builtin_amdgcn_perm(0x64646464u, d0, 0x04010400u),   // (1024 + b0, 1024 + b1)
                                __builtin_amdgcn_perm(0x64646464u, d0, 0x04030402u),   // (1024 + b2, 1024 + b3)
@@ -448,24 +468,7 @@ struct Q8Provider {
         o[i] = __builtin_bit_cast(uint32_t, q * __builtin_bit_cast(f16x2, s2));
       } else {
         const f16x2 q = __builtin_bit_cast(f16x2, pairs[i]) - __builtin_bit_cast(f16x2, ASYM ? 0x64006400u : 0x64806480u);
-        float lo = (float)q.x, hi = (float)q.y;
-        if constexpr (ASYM) {
-          lo -= zf;
-          hi -= zf;
-        }
-        lo *= sf;
-        hi *= sf;
-        if constexpr (ACT == NPAMD_F16) {
-          f16x2 h;
-          h.x = (_Float16)lo;
-          h.y = (_Float16)hi;
-          o[i] = __builtin_bit_cast(uint32_t, h);
-        } else {
-          bf16x2 b;
-          b.x = (__bf16)lo;
-          b.y = (__bf16)hi;
-          o[i] = __builtin_bit_cast(uint32_t, b);
-        }
+        o[i] = scaled_pair<ACT, ASYM>(q, __builtin_bit_cast(f16x2, s2), zf);
       }
     }
     return u32x4{o[0], o[1], o[2], o[3]};

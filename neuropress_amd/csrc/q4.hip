@@ -156,13 +156,6 @@ __device__ __forceinline__ float fdot2_act(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), c, false);
 }
 
-// (v & mask) | magic in one instruction; the compiler emits two when both constants are literals.
-__device__ __forceinline__ uint32_t and_or(uint32_t v, uint32_t mask, uint32_t magic) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(magic));
-  return r;
-}
-
 // The row-wise kernel's blocks have W = 4 or 8 waves; a wave owns R consecutive rows.
 
 template <int R>
