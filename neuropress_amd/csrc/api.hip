@@ -102,11 +102,9 @@ static int device_cu_count() {
 bool gemv_lds_codebook_enabled() { return tuning().gemv_lds_cb != 0; }
 bool tile_lds_codebook_enabled() { return tuning().tile_lds_cb != 0; }
 bool gemv_lds_activations_forced() { return tuning().gemv_lds_x != 0; }
-// One row tile per block, us, straight from memory / staged: int4 4096 x 4096 6.6 / 6.6 at 2 tokens,
-// 6.9 / 6.5 at 4, 7.9 / 6.6 at 8, 9.2 / 7.5 at 16, 13.2 / 9.0 at 32; 4096 x 14336 17.5 / 15.7 at 4,
-// 20.5 / 16.2 at 8, 27.5 / 18.9 at 16, 38.7 / 25.4 at 32; 65536-row codebook 4096 x 14336 35.8 / 34.6
-// at 4, 37.8 / 35.4 at 8, 42.4 / 37.6 at 16, 52 / 41 at 32.  With more row tiles per block
-// (14336 x 4096) or the table in LDS it does not pay.
+// One row tile per block, us, straight from memory / staged, 65536-row codebook 4096 x 14336 35.8 / 34.6 at 4 tokens,
+// 37.8 / 35.4 at 8, 42.4 / 37.6 at 16, 52 / 41 at 32; 4096 rows, looked up in LDS, 11.2 / 9.2 at 4, 13.2 / 10.2 at 8,
+// 19.1 / 12.7 at 16.  With more row tiles per block: see launch_fused_gemv.
 int& last_gemv_staged() {
   static thread_local int staged = -1;
   return staged;

@@ -82,11 +82,20 @@ struct GemvStage {
   static constexpr int kRowData = 512 * H;      // bytes of one token's activations in a step
   static constexpr int kBytes = (16 / H) * kRow;  // per token tile
 };
+// Next to a codebook in LDS, which leaves less room, the activations are those of the tokens there are and go straight into
+// LDS, two tokens per instruction: 16-byte piece p of token m in slot p ^ m % 16 of its 512 bytes, the 16 tokens of a
+// read in 16 bank groups.  (From memory lookups and with k parts the copy through registers is level or ahead: 2048 x
+// 2048 at 8 tokens 4.0 / 4.3 us, 4096 x 4096 with 65536 rows 12.5 / 12.3 at 16.)
+struct GemvStageLines {
+  static __host__ __device__ constexpr int bytes(int tokens) { return (tokens + 1) / 2 * 1024; }
+  static __device__ __forceinline__ int slot(int piece, int token) { return piece ^ (token & 15); }
+};
 template <int ACT, class Provider, int R, bool CB_LDS, bool X_LDS, int MT = 1, int H = 1, bool XS = false>
 __global__ void __launch_bounds__((kGemvMaxWaves<R, MT> * 64))
 fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
   static_assert(H == 1 || ((H == 2 || H == 4) && R == 1 && MT == 1), "k parts only with one row tile and one token tile");
-  static_assert(!XS || (R == 1 && !X_LDS), "staged activations: one row tile, x not already in LDS");
+  constexpr bool kStageLines = CB_LDS && Provider::kLdsCodebook;
+  static_assert(!XS || (!X_LDS && (kStageLines ? MT == 1 && H == 1 : R == 1)), "staged activations: the forms there are");
   constexpr int RT = 16 / H;  // weight rows (and tokens) per MFMA tile
   extern __shared__ __attribute__((aligned(16))) float red[];  // [waves][M][16*R] (+ codebook copy)
   Provider prov(pargs);
@@ -209,7 +218,29 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
     for (int r = 0; r < R; ++r) prov.load(raw[r], min(row0 + 16 * r + cr, s.N - 1), kc);
 
     u32x4 xa[MT][8];
-    if constexpr (XS) {
+    if constexpr (XS && kStageLines) {
+      using SL = GemvStageLines;
+      const int stage_bytes = SL::bytes(s.M);
+      uint8_t* const mine = reinterpret_cast<uint8_t*>(red) + s.stage_offset + wave * stage_bytes;
+      const uint32_t mine_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)mine;
+      // Two tokens per instruction straight into LDS, past M and K the last row and chunk again.  The step before has
+      // read its activations out (its products waited for them).  The statement writes m0: see the codebook's copy.
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      for (int at = 0; at < stage_bytes; at += 1024) {
+        const int row = at / 512 + (lane >> 5), piece = SL::slot(lane & 31, row);
+        const uint16_t* src = reinterpret_cast<const uint16_t*>(s.x) + (int64_t)min(row, s.M - 1) * s.ldx +
+                              min(step * 4 + piece / 8, s.chunks - 1) * 64 + piece % 8 * 8;
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(
+                         __builtin_amdgcn_readfirstlane(mine_lds + (uint32_t)at)), "v"(src) : "memory");
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const int row = min(cr, s.M - 1);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        xa[0][j] = *reinterpret_cast<const u32x4*>(mine + row * 512 + SL::slot(q * 8 + j, row) * 16);
+        xa[0][j] = (x_lane[0] && kvalid) ? xa[0][j] : zero4;
+      }
+    } else if constexpr (XS) {
       // LDS operations of a wave complete in order, so the reads below see the stores above
       // them without a barrier; rows past M repeat row M - 1 and are zeroed after the read.
       using SL = GemvStage<H>;
@@ -361,9 +392,16 @@ int launch_fused_gemv_r(GemvShape s, const typename Provider::Args& pargs, const
                             ((X_LDS && s.perm) ? (cb_lds_bytes > x_bytes ? cb_lds_bytes : x_bytes) : cb_lds_bytes);
   if constexpr (XS) {
     s.stage_offset = (lds + 15) & ~15;
-    lds = s.stage_offset + plan.waves * MT * GemvStage<H>::kBytes;
-    if (lds > kGemvLdsPerBlockMax)  // no room for the staging areas: the same kernel without them
+    constexpr bool kStageLines = CB_LDS && Provider::kLdsCodebook;
+    lds = s.stage_offset + plan.waves * (kStageLines ? GemvStageLines::bytes(s.M) : MT * GemvStage<H>::kBytes);
+    if (lds > kGemvLdsPerBlockMax) {  // no room for the staging areas: fewer waves, or the same kernel without them
+      GemvPlan fewer = plan;
+      fewer.steps_per_wave = plan.steps_per_wave + 1;
+      fewer.waves = (s.steps + fewer.steps_per_wave - 1) / fewer.steps_per_wave;
+      if (kStageLines && fewer.waves >= 8)
+        return launch_fused_gemv_r<ACT, Provider, R, CB_LDS, X_LDS, MT, H, true>(s, pargs, fewer, cb_bytes, st, what);
       return launch_fused_gemv_r<ACT, Provider, R, CB_LDS, X_LDS, MT, H, false>(s, pargs, plan, cb_bytes, st, what);
+    }
   }
   if (s.plan_only) {
     *s.plan_only = XS ? 1 : 0;
@@ -415,7 +453,7 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
   if (h > 1 && !s.perm && !gemv_lds_activations_forced()) {
     s.steps = (s.chunks + 4 * h - 1) / (4 * h);
     const GemvPlan plan = plan_gemv_rows(s.N, 16 / h, s.steps);
-    // Staged activations as for whole tiles, except next to a whole codebook in LDS.
+    // Staged activations as for whole tiles, except next to a whole codebook in LDS (2048 x 2048 at 8 tokens 4.0 / 4.3 us).
     const bool staged = gemv_stage_activations(s.M) && !(lds_table && Provider::kLdsCodebook);
     if constexpr (Provider::kLdsResidual || Provider::kLdsCodebook) {
       if (lds_table) {
@@ -493,6 +531,15 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
       return launch_fused_gemv_r<ACT, Provider, 1, false, true>(s, pargs, plan, 0, st, what);
     }
     if (cb_in_lds) {
+      // Staged activations: one row tile from three tokens on, or at any count where a wave walks several steps (K of 8192 and
+      // more); two from nine on; four never.  us straight from memory / staged at 1 / 4 / 8 / 16 tokens: 4096 x 14336
+      // with 4096 rows 9.8 / 9.0, 11.2 / 9.2, 13.2 / 10.2, 19.1 / 12.7; 4096 x 4096 4.9 / 5.1, 5.6 / 5.2, 6.2 / 5.5, 7.6 / 6.4; two
+      // tiles, 5888 x 7168 at 4 / 8 / 12 / 16 7.7 / 8.0, 8.7 / 8.3, 10.0 / 8.7, 11.4 / 9.8, 8944 x 2176 8.2 / 9.1, 8.7 / 9.4, 9.7 / 9.7,
+      // 10.4 / 10.0; four, 14336 x 4096 8.2 / 9.1, 8.7 / 9.4, 9.6 / 10.0, 10.3 / 10.3.
+      if (plan.R == 2 && s.M >= 9 && gemv_stage_activations(s.M))
+        return launch_fused_gemv_r<ACT, Provider, 2, true, false, 1, 1, true>(s, pargs, plan, cb_bytes, st, what);
+      if (plan.R == 1 && gemv_stage_activations(s.steps >= 32 ? 16 : s.M))
+        return launch_fused_gemv_r<ACT, Provider, 1, true, false, 1, 1, true>(s, pargs, plan, cb_bytes, st, what);
       if (plan.R == 4) return launch_fused_gemv_r<ACT, Provider, 4, true>(s, pargs, plan, cb_bytes, st, what);
       if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, true>(s, pargs, plan, cb_bytes, st, what);
       return launch_fused_gemv_r<ACT, Provider, 1, true>(s, pargs, plan, cb_bytes, st, what);
