@@ -180,6 +180,17 @@ struct RvqProvider {
   __device__ __forceinline__ u32x4 operand(const Raw& r) const {
     return combine(idx8_get(r.im, J), idx8_get(r.ir, J), r.s2, r.b2);
   }
+  // Indices change lanes: written to slot `put` of the wave's 2 x 64, read from slot `get`; scale and bias are prepare_row's.
+  __device__ __forceinline__ void turn(Raw& r, u32x4* lds, int put, int get) const {
+    lds[put] = r.im;  // LDS operations of a wave complete in order
+    lds[64 + put] = r.ir;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    r.im = lds[get];
+    r.ir = lds[64 + get];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    r.s2 = s2;
+    r.b2 = b2;
+  }
 
   // As loaded (see VqProvider::PairRaw); the row's scale and bias do not change from step to
   // step, so the producer reads them once (prepare_row) instead of with every pair.

@@ -61,3 +61,34 @@ def test_staged_activations_with_fewer_waves(gpu, staged):
     y = kernels.vq_linear(x, packed, cb, 12, 8, None, n).double()
     # two orders of f32 sums of k products, each rounded to fp16
     assert bool(((y - plain).abs() <= 2.0 ** -10 * plain.abs() + 1e-3).all())
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", ["none", "scale", "both"])
+def test_residual_index_lines(gpu, staged, rows, act):
+    """Residual layers of one row tile per block load their indices four lanes to a row and turn them through LDS: rows and K
+    around the tiles, with the activations straight from memory and staged, against the decoded weight."""
+    from neuropress_amd import kernels
+
+    g = cases.gen(11)
+    cb, cr = ((torch.randn(c, 8, generator=g) * 0.05).half().to(gpu) for c in (5000, 256))
+    for n, k, m in ((3073, 64, 1), (3088, 320, 2), (4099, 2240, 1), (40, 576, 9), (3100, 448, 16), (17, 1088, 31)):
+        idx = torch.randint(0, 5000, (n * k // 8,), generator=g)
+        main = idx.to(torch.int16).view(torch.uint8).to(gpu)
+        res = torch.randint(0, 256, (n * k // 8,), generator=g, dtype=torch.uint8).to(gpu)
+        scale = (torch.rand(n, generator=g) + 0.5).half().to(gpu) if rows != "none" else None
+        bias = (torch.randn(n, generator=g) * 0.01).half().to(gpu) if rows == "both" else None
+        x = torch.randn(m, k, generator=g).to(act).to(gpu)
+        w = cb.cpu()[idx].view(n, k) + cr.cpu()[res.cpu().long()].view(n, k)  # each step rounded to fp16, as the format has it
+        if scale is not None:
+            w = w * scale.cpu()[:, None]
+        if bias is not None:
+            w = w + bias.cpu()[:, None]
+        w = w.to(act).double()
+        ref = x.double().cpu() @ w.T
+        tol = 2.0 ** (-10 if act == torch.float16 else -7)  # the rounding of the output; f32 sums of k products
+        slack = 2.0 ** -22 * (x.double().cpu().abs() @ w.abs().T)
+        for mode in (0, 2):
+            staged(mode)
+            y = kernels.rvq_linear(x, main, 16, res, 8, cb, cr, scale, bias, n).double().cpu()
+            assert bool(((y - ref).abs() <= tol * ref.abs() + slack + 1e-6).all()), (n, k, m, mode)
