@@ -951,7 +951,8 @@ class NPVQLinear(nn.Module):
             return False
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("NPVQLinear.prepare_sliced() copies to the host and back: call it before the capture")
-        self._derive("sliced", self.packed_indices, self._build_sliced)
+        _, limit, _ = self._derive("sliced", self.packed_indices, self._build_sliced)
+        self._slice_gemm_wins(min(limit, _SLICED_MAX_TOKENS))  # what a first call asks, 7 us per layer of it
         self._plan = None  # it may hold routes of the fused GEMV for the token counts the lists serve
         self.prepare()
         return True
