@@ -13,7 +13,7 @@ Dequantisation rule (neuropress/nn/np_linear.py:333-353):
     ``zp = 2**(nbits-1)`` when symmetric
 
 The ``cuda`` backend runs the HIP kernels: a fused dequant GEMV up to 16
-tokens, a fused dequant MFMA GEMM up to ``_Q_TILE_MAX_TOKENS``, and decode +
+tokens (32 where it stages its activations), a fused dequant MFMA GEMM up to ``_Q_TILE_MAX_TOKENS``, and decode +
 dense GEMM above.  bf16 activations are computed natively (the reference casts
 them to fp16 first, np_linear.py:748-749).
 """
@@ -64,11 +64,9 @@ _Q_TILE_SPLIT_LONG_K: int = 8192
 # 20 / 22 / 27 / 31 against 17 / 20 / 25 / 34, with zero points 20 / 22 / 27 / 32 against 22 / 23 / 29 / 39.
 _Q_TILE_HALF_GRID_K: int = 4096
 _Q_FUSED_MAX_TOKENS: int = 16
-# 17..32 tokens: the GEMV reuses every dequantized operand for two 16-token tiles, and each
-# workgroup reads all of x from L2, so it beats the fused GEMM while x is small.  Measured
-# (GEMV vs fused GEMM, 17 / 24 / 32 tokens): int4 14336 x 4096 17.0 / 17.8 / 19.9 vs 26-28 us,
-# 4096 x 14336 25.5 / 29.5 / 33.8 vs 28 us; with zero points 21-24 vs 41-43 us and 29-37 vs 41 us;
-# int8 14336 x 4096 22-25 vs 25-27 us, 4096 x 14336 28-37 vs 26-27 us.
+# 17..32 tokens: the GEMV reuses every dequantized operand for two 16-token tiles and beats the fused GEMM at any K where
+# it stages its activations (us at 24 / 32 tokens against the fused GEMM at 33: int4 14336 x 4096 20.6 / 21.2, 28; 4096 x 14336
+# 19.8 / 21.6, 31; int8 14336 x 4096 22 / 24, 30; 4096 x 14336 24 / 25, 35), elsewhere while x is small:
 _Q_FUSED_WIDE_MAX_TOKENS: int = 32
 _Q_FUSED_WIDE_MAX_ACTIVATIONS = {4: 1 << 18, 8: 1 << 17}  # tokens x in_features, by bit width
 
