@@ -132,7 +132,9 @@ int npamd_gemv_stages_activations(int M, int N, int K, int nc);
  * (whichever finishes second adds the other's tile), more are added by a second
  * kernel; without it, or when it is too small, K is not split.  Contents
  * irrelevant before and after (nobody clears it); two calls that may run at the
- * same time need a workspace each.
+ * same time -- replays of one captured call among them -- need a workspace each.
+ * Calls that share one all the same end, with undefined results: a part waits for
+ * the other's tile no longer than about a second.
  */
 int npamd_vq_gemm_tile(const void* x, int64_t ldx, const uint8_t* packed, int64_t n_bytes,
                        int bits, const void* codebook, int codebook_dtype, int nc, int vl,

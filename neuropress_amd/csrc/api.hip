@@ -62,6 +62,8 @@ static Tuning read_tuning() {
   t.tile_splits = env_int("NPAMD_TILE_SPLITS", 0);
   t.tile_mw = env_int("NPAMD_TILE_MW", 0);
   t.tile_wide = env_int("NPAMD_TILE_WIDE", 1);
+  t.tile_call = env_int("NPAMD_TILE_CALL", 0);
+  t.tile_spins = env_int("NPAMD_TILE_SPINS", 0);
   t.slice_tiles = env_int("NPAMD_SLICE_TILES", 0);
   t.slice_parts = env_int("NPAMD_SLICE_PARTS", 0);
   t.q4_rows = env_int("NPAMD_Q4_ROWS", 0);

@@ -54,6 +54,7 @@ inline void launch(void (*kernel)(P...), dim3 grid, dim3 block, unsigned lds, hi
 // Values of the NPAMD_* tuning environment variables, read once per process.
 struct Tuning {
   int gemv_lds_cb, tile_lds_cb, gemv_lds_x, gemv_r, gemv_spw, gemv_parts, gemv_xstage, tile_splits, tile_mw, tile_wide;
+  int tile_call, tile_spins;  // NPAMD_TILE_CALL, NPAMD_TILE_SPINS: number of every call, length of the wait of K halves (0: their own)
   int slice_tiles, slice_parts;  // NPAMD_SLICE_TILES (1, 2, 4) / _PARTS: row tiles per wave, parts of K of the slice GEMM (0: planned)
   int q4_rows, q4_rowwise, q4_rowwise_bf16, q4_stream;
   int dense_tile;  // NPAMD_DENSE_TILE: 1 .. forces a tile of the dense product (wherever it applies), -1 switches it off

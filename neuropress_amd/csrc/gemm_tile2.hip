@@ -15,7 +15,9 @@ namespace npamd {
 // there need no clearing, because a word only counts while it holds the number of the call that
 // reads it, and 64 pseudo-random bits are never what memory happens to hold (the finishing
 // workgroup stores zero over it, so a graph that replays one call, number included, starts clean).
+// NPAMD_TILE_CALL gives every call that number instead: calls that share a workspace at the same time, as a test makes them.
 static unsigned long long next_call_number() {
+  if (tuning().tile_call > 0) return (unsigned long long)tuning().tile_call;
   static std::atomic<unsigned long long> counter{[] {
     std::random_device rd;
     return ((unsigned long long)rd() << 32) ^ (unsigned long long)rd() ^
@@ -514,8 +516,13 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
     }
     {
       if (tid == 0) {
-        // The other half is past the swap of its own, so it is running its last steps or writing, and waits for nobody.
-        while (__hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != pair.call) __builtin_amdgcn_s_sleep(4);
+        // The other half is past the swap of its own, so it is running its last steps or writing, and waits for nobody:
+        // microseconds at most.  Where another call uses the same workspace at the same time (one captured call replayed on two
+        // streams has its number, too) both halves can find the number and nobody write: the wait ends all the same, and
+        // the sum is what the two calls made of each other.
+        for (unsigned left = pair.spins;
+             left && __hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != pair.call; --left)
+          __builtin_amdgcn_s_sleep(4);
         // for a replay of this call
         __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(word + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -613,12 +620,13 @@ int launch_tile2_prod(GemmShape s, const typename Prods::Args& a, hipStream_t st
   // The kernel's loop ends in two steps of their own behind an even number of others.
   if (s.split_chunks < 3 || s.chunks - (s.splits - 1) * s.split_chunks < 3) return 1;
   s.partials = (float*)workspace;
-  T2Pair pair{nullptr, nullptr, 0ull};
+  T2Pair pair{nullptr, nullptr, 0ull, 0u};
   if (s.splits == 2) {
     const int64_t tiles = (int64_t)((s.N + kT2Cols - 1) / kT2Cols) * ((s.M + 128 * mw - 1) / (128 * mw));
     pair.words = (unsigned long long*)workspace;
     pair.tiles = (float*)((uint8_t*)workspace + ((tiles * 16 + 255) & ~(int64_t)255));
     pair.call = next_call_number();
+    pair.spins = tuning().tile_spins > 0 ? (unsigned)tuning().tile_spins : kT2HandoffSpins;
   }
   switch (mw) {
     case 1: return launch_tile2_mw<ACT, 1, typename Prods::template Of<1>>(s, a, pair, st, what);

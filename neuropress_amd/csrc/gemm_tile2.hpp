@@ -38,7 +38,7 @@
 // x).  The halves meet without a second kernel: a step before its end a workgroup swaps the call's
 // number into the tile's word; the first of a pair to do so stores its f32 tile to the workspace and says so in a
 // second word, the other waits for that, adds the tile to its registers, adds the bias and stores y.  It waits for a
-// workgroup that is running and waits for nobody.  When both stored their tiles, and a swap behind that decided who
+// workgroup that is running and waits for nobody, and the wait is bounded for callers who share a workspace all the same.  When both stored their tiles, and a swap behind that decided who
 // adds, they mostly ended together and wrote twice the bytes (14336 x 4096, 384 tokens 63.3 -> 61.7 us, int4 at 256
 // 42.4 -> 41.3; halves of unequal length gain nothing).  Two addends commute, so the result does not depend on which half
 // was first.  More than two splits (layers
@@ -73,7 +73,11 @@ struct T2Pair {
   unsigned long long* words;  // two per tile, each holding `call`: one half of the tile is about to end in this call; its tile is written
   float* tiles;
   unsigned long long call;    // this call's number, drawn at random: never what memory happens to hold
+  unsigned spins;             // looks at the second word before a half goes on without the other's tile
 };
+// A look sleeps 256 clocks and waits for a load past the L2: half a second and more in all, where a half is never behind
+// the other's swap by more than its last step and its stores.
+constexpr unsigned kT2HandoffSpins = 1u << 20;
 
 // Splits of K for the 128-column kernel: 1 while the block tiles cover most compute units, else as
 // many as fill them, each at least 8 steps long.

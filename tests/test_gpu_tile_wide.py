@@ -234,3 +234,52 @@ def test_wide_tile_gemm_walks_lines_of_codes(gpu, tile_wide, nbits, asym, gs, m,
     for splits in (1, 2):
         tile_wide(2, splits)
         assert torch.equal(kernels.q_gemm_tile(x, blob, sc, nbits, gs, zp), wt[pick]), f"{splits} splits"
+
+
+@pytest.mark.parametrize("kind", ["vq", "q"])
+@pytest.mark.parametrize("m", [17, 200])
+def test_wide_tile_gemm_does_not_wait_for_ever_in_a_shared_workspace(gpu, tile_wide, monkeypatch, kind, m):
+    """The words as another call with the same number leaves them between its own swaps and its end: both halves of every
+    tile find the number, each takes the other for the one that writes, and no tile is written.  The wait is bounded:
+    the call ends, clears the words, and the next one in the same workspace is right."""
+    from neuropress_amd import _lib
+    from neuropress_amd.kernels import plans
+
+    lib = _lib.load()
+    n, k, act = 300, 1024, torch.bfloat16
+    code, stream = plans.DTYPE_CODES[act], torch.cuda.current_stream().cuda_stream
+    y = torch.empty(m, n, dtype=act, device=gpu)
+    if kind == "vq":
+        L = cases.vq_layer(40 + m, n, k, 65536, bits=16, act=act, m=m, std=0.05)
+        x, pk, cb = L["x"].to(gpu), L["packed"].to(gpu), L["cb"].to(act).to(gpu)
+        call = lambda ws: lib.npamd_vq_gemm_tile(x.data_ptr(), k, pk.data_ptr(), pk.numel(), 16, cb.data_ptr(), code, cb.shape[0], 8, None,
+                                                 y.data_ptr(), n, m, n, k, code, ws.data_ptr(), ws.numel(), stream)  # fmt: skip
+    else:
+        Q = cases.q4_layer(40 + m, n, k, act=act, m=m)
+        x, blob, sc = Q["x"].to(gpu), Q["blob"].to(gpu), Q["scale"].to(gpu)
+        call = lambda ws: lib.npamd_q_gemm_tile(x.data_ptr(), k, blob.data_ptr(), sc.data_ptr(), None, None, y.data_ptr(), n, m, n, k,
+                                                4, 32, code, ws.data_ptr(), ws.numel(), stream)  # fmt: skip
+    tile_wide(2, 2)
+    rows = 128 * ((m + 127) // 128)  # one block of rows
+    tiles = (n + 127) // 128
+    head = (tiles * 16 + 255) // 256 * 256
+    ws = torch.full((head + 2 * tiles * rows * 128 * 4,), 0xFF, dtype=torch.uint8, device=gpu)
+    assert lib.npamd_gemm_tile_workspace_bytes(m, n, k) >= ws.numel()
+    assert call(ws) == 0
+    expect = y.clone()
+    words = ws[: tiles * 16].view(torch.int64).view(tiles, 2)
+    assert not words.any()  # K was split in two halves, which met here
+    number = 0x5EED
+    monkeypatch.setenv("NPAMD_TILE_CALL", str(number))
+    monkeypatch.setenv("NPAMD_TILE_SPINS", "64")
+    tile_wide(2, 2)
+    words[:, 0] = number
+    y.zero_()
+    assert call(ws) == 0
+    torch.cuda.synchronize()
+    assert not words.any()
+    monkeypatch.delenv("NPAMD_TILE_CALL")
+    monkeypatch.delenv("NPAMD_TILE_SPINS")
+    tile_wide(2, 2)
+    assert call(ws) == 0
+    assert torch.equal(y, expect)
