@@ -120,6 +120,12 @@ int npamd_vq_fused_supported(int K, int vl, int bits);
  * it is run up to the point of the launch.  Host-only arithmetic. */
 int npamd_gemv_stages_activations(int M, int N, int K, int nc);
 
+/* npamd_q_gemv has two kernels for 4- and 8-bit layers.  Bit 1 (value 2): M tokens on a layer with these scales and zero
+ * points run the one that brings codes, scales and activations through LDS in whole lines (an even count of scales, 4-byte
+ * aligned).  Bit 0: the other one, which serves what is left, would stage its activations for this shape.  The
+ * pointers are looked at, not read.  Host-only arithmetic. */
+int npamd_q_gemv_staging(int M, int N, int K, int nbits, int group_size, const void* scale_f16, const void* zero_point_f16);
+
 /*
  * Tile-decode MFMA GEMM, any M >= 1: same contraction, weight tiles decoded
  * inside the kernel, dense weight never written.

@@ -628,9 +628,11 @@ static bool q4_rowwise_ok(const QCall& c) {
 static bool q_gemv_takes_shape(int M, int N, int chunks) {
   return plan_gemv_parts(M, N, chunks, 0) == 1 || 2 * ((N + 15) / 16) > device_cus_q4();
 }
+static bool q_gemv_takes_layer(int N, int K, int gs, const void* scale, const void* zp) {
+  return ptr_aligned(scale, 4) && (!zp || ptr_aligned(zp, 4)) && (int64_t)N * (K / gs) % 2 == 0 && K < (1 << 24);
+}
 static bool q_gemv_takes(const QCall& c) {
-  return q_gemv_takes_shape(c.M, c.N, c.K / 64) && ptr_aligned(c.scale, 4) && (!c.zp || ptr_aligned(c.zp, 4)) &&
-         (int64_t)c.N * (c.K / c.gs) % 2 == 0 && c.ldx < (1 << 26) && c.K < (1 << 24);
+  return q_gemv_takes_shape(c.M, c.N, c.K / 64) && q_gemv_takes_layer(c.N, c.K, c.gs, c.scale, c.zp) && c.ldx < (1 << 26);
 }
 
 template <int ACT, bool ASYM>
@@ -646,8 +648,7 @@ static int q4_fused(const QCall& c, bool gemv) {
   return launch_tile_gemm<ACT, P>(s, a, c.st, c.what, c.ws, c.ws_bytes);
 }
 
-int npamd::q_gemv_plan_stages(int M, int N, int K) {
-  if (q_gemv_takes_shape(M, N, K / 64)) return 1;
+static int q_fused_gemv_plan_stages(int M, int N, int K) {
   int staged = 0;
   GemvShape s{nullptr, K, nullptr, nullptr, N, M, N, K / 64, 0, 0};
   s.plan_only = &staged;
@@ -655,6 +656,10 @@ int npamd::q_gemv_plan_stages(int M, int N, int K) {
   typename P::Args a{};
   launch_fused_gemv<NPAMD_F16, P>(s, a, nullptr, "plan");
   return staged;
+}
+
+int q_gemv_plan_stages(int M, int N, int K) {
+  return q_gemv_takes_shape(M, N, K / 64) ? 1 : q_fused_gemv_plan_stages(M, N, K);
 }
 
 template <int ACT, bool ASYM>
@@ -794,6 +799,12 @@ extern "C" int npamd_q_fused_supported(int K, int nbits, int group_size) {
                  K % group_size == 0
              ? 1
              : 0;
+}
+
+extern "C" int npamd_q_gemv_staging(int M, int N, int K, int nbits, int group_size, const void* scale_f16, const void* zero_point_f16) {
+  if (M < 1 || M > NPAMD_GEMV_MAX_M || N < 1 || !npamd_q_fused_supported(K, nbits, group_size)) return 0;
+  return (q_fused_gemv_plan_stages(M, N, K) ? 1 : 0) |
+         (q_gemv_takes_shape(M, N, K / 64) && q_gemv_takes_layer(N, K, group_size, scale_f16, zero_point_f16) ? 2 : 0);
 }
 
 extern "C" int npamd_q_gemv(const void* x, int64_t ldx, const uint8_t* w_pack, const void* scale_f16,

@@ -266,6 +266,15 @@ def gemv_stages_activations(m: int, n: int, k: int, num_centroids: int) -> bool:
     return bool(_lib.load().npamd_gemv_stages_activations(int(m), int(n), int(k), int(num_centroids)))
 
 
+def q_gemv_staging(m: int, n: int, k: int, nbits: int, group_size: int, scale: torch.Tensor | None,
+                   zero_point: torch.Tensor | None) -> tuple[bool, bool]:  # fmt: skip
+    """For *m* tokens on a 4- or 8-bit layer with these scales and zero points: whether the GEMV's kernel that reads whole
+    lines takes the call, and whether the one that serves what is left would stage its activations (``npamd_q_gemv_staging``)."""
+    at = [None if t is None else t.data_ptr() for t in (scale, zero_point)]
+    bits = _lib.load().npamd_q_gemv_staging(int(m), int(n), int(k), int(nbits), int(group_size), *at)
+    return bool(bits & 2), bool(bits & 1)
+
+
 def vq_fused_supported(in_features: int, vector_len: int, bits: int) -> bool:
     """Whether the MFMA GEMV / tile GEMM take a VQ layer of this shape (``npamd_vq_fused_supported``).
     Other shapes run an element-wise kernel that decodes the weight once per 16 tokens."""

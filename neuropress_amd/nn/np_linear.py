@@ -13,7 +13,7 @@ Dequantisation rule (neuropress/nn/np_linear.py:333-353):
     ``zp = 2**(nbits-1)`` when symmetric
 
 The ``cuda`` backend runs the HIP kernels: a fused dequant GEMV up to 16
-tokens (32 where it stages its activations), a fused dequant MFMA GEMM up to ``_Q_TILE_MAX_TOKENS``, and decode +
+tokens (32 where it reads whole lines), a fused dequant MFMA GEMM up to ``_Q_TILE_MAX_TOKENS``, and decode +
 dense GEMM above.  bf16 activations are computed natively (the reference casts
 them to fp16 first, np_linear.py:748-749).
 """
@@ -65,10 +65,11 @@ _Q_TILE_SPLIT_LONG_K: int = 8192
 _Q_TILE_HALF_GRID_K: int = 4096
 _Q_FUSED_MAX_TOKENS: int = 16
 # 17..32 tokens: the GEMV reuses every dequantized operand for two 16-token tiles and beats the fused GEMM at any K where
-# it stages its activations (us at 24 / 32 tokens against the fused GEMM at 33: int4 14336 x 4096 20.6 / 21.2, 28; 4096 x 14336
-# 19.8 / 21.6, 31; int8 14336 x 4096 22 / 24, 30; 4096 x 14336 24 / 25, 35), elsewhere while x is small:
+# it reads whole lines (us at 24 / 32 tokens against the fused GEMM at 33: int4 14336 x 4096 20.6 / 21.2, 28; 4096 x 14336
+# 19.8 / 21.6, 31; int8 14336 x 4096 22 / 24, 30; 4096 x 14336 24 / 25, 35), elsewhere while x is small (_gemv_max_tokens):
 _Q_FUSED_WIDE_MAX_TOKENS: int = 32
 _Q_FUSED_WIDE_MAX_ACTIVATIONS = {4: 1 << 18, 8: 1 << 17}  # tokens x in_features, by bit width
+_Q_FUSED_WIDE_INT8_MAX_K: int = 8192
 
 _ALLOW_FALLBACK: bool = os.environ.get("NEUROPRESS_ALLOW_KERNEL_FALLBACK", "").strip() in (
     "1", "true", "yes",
@@ -165,7 +166,7 @@ _PLAN_ATTRIBUTES = ("backend", "out_features", "in_features", "group_size", "nbi
 _PLAN_THRESHOLDS = ("_Q_TILE_MAX_TOKENS", "_Q_TILE_LONG_K_MAX_TOKENS", "_Q_TILE_WIDE_MAX_TOKENS", "_Q_TILE_WIDE_MIN_FEATURES",
                     "_Q_TILE_MIN_GRID_FRACTION", "_Q_TILE_SPLIT_MAX_TOKENS", "_Q_TILE_SPLIT_LONG_K", "_Q_TILE_HALF_GRID_K",
                     "_Q_FUSED_MAX_TOKENS",
-                    "_Q_FUSED_WIDE_MAX_TOKENS", "_Q_FUSED_WIDE_MAX_ACTIVATIONS")  # fmt: skip
+                    "_Q_FUSED_WIDE_MAX_TOKENS", "_Q_FUSED_WIDE_MAX_ACTIVATIONS", "_Q_FUSED_WIDE_INT8_MAX_K")  # fmt: skip
 
 
 class NPLinear(nn.Module):
@@ -345,26 +346,32 @@ class NPLinear(nn.Module):
         )  # fmt: skip
 
     def _gemv_max_tokens(self, m: int, tracked: bool = False) -> int:
-        """End of the GEMV band for a call of *m* tokens: 16, or 32 while x stays small or the kernel stages it.  *tracked*: as it
+        """End of the GEMV band for a call of *m* tokens: 16, or 32 where a GEMV stays ahead of the fused GEMM.  *tracked*: as it
         is against decode + the library's product, which such calls take past it."""
         if _Q_FUSED_MAX_TOKENS < m <= _Q_FUSED_WIDE_MAX_TOKENS:
+            from .. import kernels
+
+            scales = (None, None) if tracked else (self.scale, self.zero_point)  # tracked: storage may be a trace's
+            lines, staged = kernels.q_gemv_staging(m, self.out_features, self.in_features, self.nbits, self.group_size, *scales)
+            # The GEMV that reads whole lines stays ahead of the tile GEMM at any K (GEMV at 24 / 32 tokens, tile GEMM at 33, us:
+            # 4096 x 14336 int4 19.6 / 21.3, 30.7, int8 24.0 / 24.7, 35; 5888 x 7168 int4 15.7 / 16.6).  The other GEMV serves layers
+            # with an odd count of scales or scales that start between two dwords.  Against the tile GEMM, us at 24 tokens:
+            # int4 14336 x 14336 65.8 / 76.3, 4096 x 14336 22.9 / 26.8; int8, whose codes are twice the bytes, where no compute
+            # unit has two row tiles and K is short, or too few have none for the tile GEMM to gain by its parts of K:
+            # 4096 x 8192 17.2 / 19.3, 3584 x 14336 26.4 / 27.6, 1536 x 8192 13.9 / 14.5 and x 10240 16.5 / 14.9, 3072 x 14336
+            # 26.0 / 24.5, 4904 x 8192 29.7 / 24.0, 14336 x 8192 52.8 / 47.5.
+            tiles, cus = -(-self.out_features // 16), self._compute_units()
+            if not tracked and (lines or self.nbits == 4 or (
+                staged and tiles <= cus and (self.in_features <= _Q_FUSED_WIDE_INT8_MAX_K or 5 * tiles >= 4 * cus)
+            )):  # fmt: skip
+                return _Q_FUSED_WIDE_MAX_TOKENS
+            # Calls that record a gradient, where the line is part of what the module does: while x is small, past that
+            # int4 where the other GEMV stages its activations.
             cap = _Q_FUSED_WIDE_MAX_ACTIVATIONS.get(self.nbits, 0)
             if self.zero_point is not None and self.nbits == 4:
                 cap = 1 << 30  # the fused GEMM pays for the zero points per tile: GEMV at any K
-            if m * self.in_features <= cap:
+            if m * self.in_features <= cap or (staged and self.nbits == 4):
                 return _Q_FUSED_WIDE_MAX_TOKENS
-            # A GEMV that stages its activations through LDS stays ahead of the tile GEMM at any K (GEMV at 24 / 32 tokens, tile
-            # GEMM at 33, us: 4096 x 14336 int4 19.6 / 21.3, 30.7, int8 24.0 / 24.7, 35; 5888 x 7168 int4 15.7 / 16.6).
-            # Where gradients may flow the line is part of what the module does and stays where it was: int4 layers
-            # of fewer than 1.2 row tiles per compute unit.
-            if tracked:
-                few = -(-self.out_features // 16) * 10 < 12 * self._compute_units()
-                return _Q_FUSED_WIDE_MAX_TOKENS if self.nbits == 4 and few else _Q_FUSED_MAX_TOKENS
-            if self.nbits in (4, 8):
-                from .. import kernels
-
-                if kernels.gemv_stages_activations(m, self.out_features, self.in_features, 0):
-                    return _Q_FUSED_WIDE_MAX_TOKENS
         return _Q_FUSED_MAX_TOKENS
 
     def _forward_cuda(self, x: torch.Tensor) -> torch.Tensor:

@@ -529,3 +529,30 @@ def test_column_permutation_is_checked_before_a_kernel_reads_it():
     layer.column_perm = perm[:63]
     with pytest.raises(RuntimeError, match="must hold in_features=64"):
         layer._perm_i32(cpu)
+
+
+@pytest.mark.parametrize("nbits", [4, 8])
+@pytest.mark.parametrize("n,k,group,shift", [(4096, 4672, 64, 0), (4097, 4672, 64, 0), (4095, 8256, 64, 0), (4096, 4672, 64, 1),
+                                             (4096, 9216, 64, 1), (3184, 9216, 64, 1), (14336, 9216, 64, 0), (14335, 8256, 64, 0), (14336, 9216, 64, 1)])  # fmt: skip
+def test_group_quantized_layers_past_16_tokens_ask_which_gemv_takes_them(nbits, n, k, group, shift):
+    """17..32 tokens: a layer that the GEMV of whole lines takes stays with it.  An odd count of scales, or scales that start
+    between two dwords, leave the other GEMV, which int8 layers keep only where it is ahead of the tile GEMM: no compute
+    unit with two row tiles, and short K or few without one.  Calls that record a gradient: while x is small, past that int4 where the other
+    GEMV stages its activations, whichever of the two it is."""
+    from neuropress_amd import kernels
+    from neuropress_amd.nn.np_linear import _Q_FUSED_WIDE_MAX_ACTIVATIONS
+
+    storage = torch.ones(n * (k // group) + shift, dtype=torch.float16)
+    layer = NPLinear(torch.empty(n, k * nbits // 8, dtype=torch.uint8), storage[shift:], n, k, group, nbits, "sym", "cuda")
+    layer._derived["cus"] = 256  # what the kernel library takes without a GPU, and the card's
+    assert layer.scale.data_ptr() % 4 == 2 * shift
+    takes = shift == 0 and layer.scale.numel() % 2 == 0
+    m = 32
+    assert m * k > _Q_FUSED_WIDE_MAX_ACTIVATIONS[8]
+    small = m * k <= _Q_FUSED_WIDE_MAX_ACTIVATIONS[nbits]
+    few = -(-n // 16) * 10 < 12 * 256
+    assert kernels.q_gemv_staging(m, n, k, nbits, group, layer.scale, None) == (takes, few)
+    assert layer._gemv_max_tokens(m) == (32 if takes or nbits == 4 or (n <= 4096 and (k <= 8192 or n > 3260)) else 16)
+    assert layer._gemv_max_tokens(m, tracked=True) == (32 if small or (nbits == 4 and few) else 16)
+    assert layer._gemv_max_tokens(16) == 16 and layer._gemv_max_tokens(33) == 16
+    assert kernels.q_gemv_staging(4, 256, 4096, nbits, 32, storage, None)[0] is False  # few rows: K in parts
