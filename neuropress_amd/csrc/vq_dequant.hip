@@ -7,6 +7,7 @@
 // store.  Traffic = index stream + output; the codebook is read from cache.
 #include "common.hpp"
 #include "gather_columns.hpp"
+#include "../../include/npamd_diag.h"
 
 namespace npamd {
 
@@ -405,6 +406,21 @@ extern "C" int npamd_vq_dequant(const uint8_t* packed, int64_t n_bytes, int bits
   return fail(NPAMD_ERR_INVALID, "npamd_vq_dequant: out_dtype must be f16, bf16 or f32");
 }
 
+// The whole launch has the LDS of a block that gathers: K elements where columns are permuted.  Up to 10240 of them eight blocks,
+// all their waves, still fit a compute unit; past that the decoding blocks, which wait for memory, are fewer, and the larger the
+// layer the sooner that costs more than a launch.  us with 60 rows, one launch / two: 8-bit indices 4096 x 10240 17.0 / 19.5,
+// 4096 x 12288 21.7 / 22.4, 4096 x 14336 27.1 / 25.2, 1024 x 16384 12.2 / 13.2, 4096 x 16384 35.2 / 27.8, 11008 x 16384 125.6 / 105.8;
+// 16-bit 4096 x 14336 39.1 / 39.9, 11008 x 12288 134.8 / 134.7, 4096 x 16384 48.6 / 44.8, 11008 x 16384 182.4 / 176.9.
+static bool gather_fits_decode(int bits, int64_t n_vectors, int K, bool perm) {
+  if (!perm || K <= 10240) return true;
+  const int over = K > 12288 ? (K - 12288 + 2047) / 2048 : 0;
+  return K <= 16384 && n_vectors <= ((int64_t)(bits == 16 ? 16 : 8) << 20) >> over;
+}
+
+extern "C" int npamd_diag_gather_fits_decode(int bits, int64_t n_vectors, int K, int permuted) {
+  return gather_fits_decode(bits, n_vectors, K, permuted != 0) ? 1 : 0;
+}
+
 extern "C" int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* out, int64_t ldo, int M, int K, void* stream);
 
 extern "C" int npamd_vq_dequant_gather(const uint8_t* packed, int64_t n_bytes, int bits, const void* codebook_f16, int nc, int vl,
@@ -417,7 +433,7 @@ extern "C" int npamd_vq_dequant_gather(const uint8_t* packed, int64_t n_bytes, i
                     !(table_bytes > 16 * 1024 && table_bytes <= 64 * 1024 && n_vectors >= (1 << 20)) && n_vectors > 0 &&
                     n_vectors <= (int64_t)1 << 30 && nc >= 1 && (n_vectors * bits + 7) / 8 <= n_bytes && packed && codebook_f16 && out &&
                     al(packed, 2) && al(codebook_f16, 16) && al(out, 16) && x && x_out && al(x_out, 16) && M >= 1 &&
-                    M < kGatherPairRows && K >= 1 && K <= 16384 && ldx >= K && ldo >= K && ldo % 8 == 0 && ldo <= 32768;
+                    M < kGatherPairRows && K >= 1 && K <= 16384 && gather_fits_decode(bits, n_vectors, K, perm != nullptr) && ldx >= K && ldo >= K && ldo % 8 == 0 && ldo <= 32768;
   if (!fits) {
     const int rc = npamd_gather_columns(x, ldx, perm, x_out, ldo, M, K, stream);
     return rc != NPAMD_OK ? rc : npamd_vq_dequant(packed, n_bytes, bits, codebook_f16, nc, vl, n_vectors, out, out_dtype, stream);

@@ -556,3 +556,17 @@ def test_group_quantized_layers_past_16_tokens_ask_which_gemv_takes_them(nbits, 
     assert layer._gemv_max_tokens(m, tracked=True) == (32 if small or (nbits == 4 and few) else 16)
     assert layer._gemv_max_tokens(16) == 16 and layer._gemv_max_tokens(33) == 16
     assert kernels.q_gemv_staging(4, 256, 4096, nbits, 32, storage, None)[0] is False  # few rows: K in parts
+
+
+def test_the_gather_joins_the_decode_where_its_rows_in_lds_leave_the_decode_its_waves():
+    """Permuted columns lie in the LDS that every block of the launch has, the decoding ones too: past 10240 columns (eight
+    blocks per compute unit) only layers small enough that the saved launch outweighs a slower decode."""
+    from neuropress_amd import _lib
+
+    fits = _lib.load().npamd_diag_gather_fits_decode
+    assert all(fits(bits, n * k // 8, k, 1) for bits in (8, 12, 16) for n in (64, 3003, 14336) for k in (64, 2184, 10240))
+    assert all(fits(bits, 14336 * k // 8, k, 0) for bits in (8, 12, 16) for k in (10248, 16384))  # no rows in LDS
+    for bits, scale in ((8, 1), (12, 1), (16, 2)):
+        for k, rows in ((10241, 6400), (12288, 5461), (12289, 2730), (14336, 2340), (14337, 1170), (16384, 1024)):
+            assert fits(bits, scale * rows * k // 8, k, 1), (bits, k)
+            assert not fits(bits, scale * (rows + 400) * k // 8, k, 1), (bits, k)
