@@ -877,10 +877,10 @@ class NPVQLinear(nn.Module):
         if band == "sliced":
             sl, limit, _ = self._derived_hit("sliced", self.packed_indices)
             most = min(limit, _SLICED_MAX_TOKENS, _fused_max_tokens(self.backend))
-            if self._slice_gemm_wins(most):  # from some token count on: those below this one are the lists'
-                most = m
+            others = self._slice_gemm_counts()
             for tokens in range(1, most + 1):
-                plan.route(code, tokens, number, sl.workspace_bytes(tokens))
+                if tokens not in others or tokens > _SLICE_GEMM_MAX_TOKENS:
+                    plan.route(code, tokens, number, sl.workspace_bytes(tokens))
         elif band == "slice":
             plan.route(code, m, number, plans.slice_scratch(m, self.out_features, self._kernel_k(), self.proxy.num_centroids))
         else:
@@ -953,8 +953,8 @@ class NPVQLinear(nn.Module):
             return False
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("NPVQLinear.prepare_sliced() copies to the host and back: call it before the capture")
-        _, limit, _ = self._derive("sliced", self.packed_indices, self._build_sliced)
-        self._slice_gemm_wins(min(limit, _SLICED_MAX_TOKENS))  # what a first call asks, 7 us per layer of it
+        self._derive("sliced", self.packed_indices, self._build_sliced)
+        self._slice_gemm_counts()  # a first call asks it
         self._plan = None  # it may hold routes of the fused GEMV for the token counts the lists serve
         self.prepare()
         return True
@@ -1065,34 +1065,40 @@ class NPVQLinear(nn.Module):
         return sl if m <= limit else None
 
     def _slice_gemm_wins(self, m: int) -> bool:
-        """Whether the slice GEMM is the fastest kernel for *m* tokens: its estimate against what was timed on this layer's
+        """Whether the slice GEMM is the fastest kernel for *m* tokens."""
+        return m <= _SLICE_GEMM_MAX_TOKENS and m in self._slice_gemm_counts()
+
+    def _slice_gemm_counts(self) -> frozenset[int]:
+        """The token counts at which the slice GEMM is the fastest kernel: its estimate against what was timed on this layer's
         own indices, the slice lists (between two timed token counts: on the line through them) or, past them, the fused GEMV
         at the most tokens it was timed with (it does not get faster, and the tile GEMM of 17 to 32 tokens is level with
-        it).  Layers that were not timed -- lists never built, or fewer than 2^20 indices -- do not take it."""
-        if m > _SLICE_GEMM_MAX_TOKENS or self.proxy.num_centroids <= 4096:
-            return False
+        it).  One token stays with the lists where they won it.  Layers that were not timed -- lists never built, or fewer
+        than 2^20 indices -- do not take it."""
+        if self.proxy.num_centroids <= 4096 or self.bits > 16 or self.backend == VQBackend.CUDA_LUT or _FUSED_MAX_TOKENS <= 0:
+            return frozenset()
         hit = self._derived_hit("sliced", self.packed_indices)
-        if hit is None or not hit[2] or m <= min(hit[1], 1) or self.bits > 16 or self.backend == VQBackend.CUDA_LUT or _FUSED_MAX_TOKENS <= 0:
-            return False
+        if hit is None or not hit[2]:
+            return frozenset()
         cached = self._derived.get("slice_gemm")
         if cached is None or cached[0] is not hit:
-            cached = self._derived["slice_gemm"] = (hit, {})
-        wins = cached[1].get(m)
-        if wins is None:
-            from .. import kernels
+            counts = frozenset(m for m in range(min(hit[1], 1) + 1, 33) if self._slice_gemm_ahead(m, hit))
+            cached = self._derived["slice_gemm"] = (hit, counts)
+        return cached[1]
 
-            us = kernels.slice_gemm_us(m, self.out_features, self._kernel_k(), self.proxy.num_centroids)
-            us += _SLICE_GEMM_GATHER_US if us and self.column_perm is not None else 0.0
-            _, limit, times = hit
-            if m <= limit:
-                (m0, t0), (m1, t1) = next(
-                    ((a[0], a[1]), (b[0], b[1])) for a, b in zip((times[0], *times), times) if b[0] >= m or b is times[-1]
-                )  # fmt: skip
-                other = t1 if m1 == m0 else t0 + (t1 - t0) * (m - m0) / (m1 - m0)
-            else:
-                other = times[-1][2]
-            wins = cached[1][m] = 0 < us < other
-        return wins
+    def _slice_gemm_ahead(self, m: int, timed) -> bool:
+        from .. import kernels
+
+        us = kernels.slice_gemm_us(m, self.out_features, self._kernel_k(), self.proxy.num_centroids)
+        us += _SLICE_GEMM_GATHER_US if us and self.column_perm is not None else 0.0
+        _, limit, times = timed
+        if m <= limit:
+            (m0, t0), (m1, t1) = next(
+                ((a[0], a[1]), (b[0], b[1])) for a, b in zip((times[0], *times), times) if b[0] >= m or b is times[-1]
+            )  # fmt: skip
+            other = t1 if m1 == m0 else t0 + (t1 - t0) * (m - m0) / (m1 - m0)
+        else:
+            other = times[-1][2]
+        return 0 < us < other
 
     def _perm_i32(self, device: torch.device) -> torch.Tensor:
         """``column_perm`` as the int32 device tensor the kernels read (cached): in range, negative entries wrapped as

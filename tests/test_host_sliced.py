@@ -194,3 +194,39 @@ def test_gemv_sliced_validates_before_touching_the_gpu():
     with pytest.raises(RuntimeError, match="not a slice-list header"):
         call(hdr=ctypes.addressof(bad))
     call(m=0)  # nothing to do: returns before any launch
+
+
+@pytest.mark.parametrize("taken", [set(), {2, 3, 4, 5, 6, 7}, {4, 5}, {2, 7}])
+def test_a_call_of_the_lists_leaves_the_slice_gemm_its_token_counts(monkeypatch, taken):
+    """The first call that the slice lists serve makes routes for all their token counts, and only for theirs: those that the
+    slice GEMM wins need not be the last ones."""
+    from neuropress_amd.nn import NPVQLinear, VQProxy
+    from neuropress_amd.nn import np_vq_linear as vqmod
+
+    n, k = 64, 512
+    L = cases.vq_layer(3, n, k, 8192, bits=16, act=torch.float16, m=1, std=0.05)
+    layer = NPVQLinear(VQProxy(L["cb"]), L["packed"], 16, n, k, 8, "cuda_wmma")
+    packed = layer.packed_indices
+
+    class Lists:
+        def workspace_bytes(self, tokens):
+            return 100 * tokens
+
+    class Plan:
+        def __init__(self):
+            self.names, self.routes = {}, {}
+
+        def route(self, code, tokens, number, scratch):
+            self.routes[tokens] = scratch
+
+    layer._derived["sliced"] = ((packed.device, packed.data_ptr(), packed._version), (Lists(), 7, ((1, 10.0, 20.0),)))
+    monkeypatch.setattr(NPVQLinear, "_template", lambda *a: 0)
+    monkeypatch.setattr(NPVQLinear, "_slice_gemm_ahead", lambda self, m, timed: m in taken)
+    assert {m for m in range(1, 33) if layer._slice_gemm_wins(m)} == taken
+    first = next(m for m in range(1, 8) if m not in taken)
+    plan = Plan()
+    layer._add_route(plan, torch.float16, first, "sliced")
+    assert plan.routes == {m: 100 * m for m in range(1, 8) if m not in taken}
+    monkeypatch.setattr(vqmod, "_SLICE_GEMM_MAX_TOKENS", 0)  # switched off: every count is the lists'
+    layer._add_route(plan, torch.float16, first, "sliced")
+    assert plan.routes == {m: 100 * m for m in range(1, 8)}
