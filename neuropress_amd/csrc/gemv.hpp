@@ -36,8 +36,7 @@ struct GemvShape {
   // Optional gather of the activation columns: the kernel contracts x[m, perm[k]] with W[n, k].
   // Only with the X_LDS variant (every block first copies the permuted rows of x into LDS).
   const int32_t* perm = nullptr;
-  int stage_offset = 0;  // XS kernels: byte offset of the waves' activation staging areas in LDS
-  int turn_offset = 0, turn_bytes = 0;  // kernels that load index lines: where in LDS the waves turn them, bytes per wave
+  int stage_offset = 0;  // byte offset of the waves' own areas in LDS: XS kernels stage activations there, kernels that load index lines turn them
   // Planning only: when set, the launcher writes here whether the kernel it chose stages its
   // activations (1 / 0) and launches nothing.
   int* plan_only = nullptr;
@@ -96,6 +95,9 @@ struct GemvStageLines {
 // spend 64 cycles instead of 16 on a load whose lanes are 16 rows; the rows' scales and biases are read once.
 // 4096 x 4096 with 65536 + 256 rows, Zipf indices, us at 1 / 2 / 24 / 32 tokens: 8.8 / 8.7 / 11.0 / 11.8 before, 8.1 / 8.1 / 10.8 / 11.3;
 // uniform 13.2 / 12.9 at one; 4096 x 14336 20.2 / 19.2.
+// With staged activations the lines are turned in the wave's staging area, between the reads of one step's activations and the
+// stores of the next's.
+constexpr int kGemvTurnBytes = 2048;
 template <class Provider, int R, bool CB_LDS, int H>
 constexpr bool gemv_loads_lines = Provider::kLdsResidual && CB_LDS && R == 1 && H == 1;
 template <int ACT, class Provider, int R, bool CB_LDS, bool X_LDS, int MT = 1, int H = 1, bool XS = false>
@@ -226,7 +228,8 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
     typename Provider::Raw raw[R];
     if constexpr (kLines) {
       prov.load(raw[0], min(row0 + (lane >> 2), s.N - 1), min(step * 4 + (lane & 3), s.chunks - 1));
-      u32x4* const turn = reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(red) + s.turn_offset + wave * s.turn_bytes);
+      constexpr int kTurn = XS ? MT * GemvStage<H>::kBytes : kGemvTurnBytes;
+      u32x4* const turn = reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(red) + s.stage_offset + wave * kTurn);
       prov.turn(raw[0], turn, lane ^ (lane >> 4), (4 * c + q) ^ (c >> 2));
     } else {
 #pragma unroll
@@ -419,15 +422,9 @@ int launch_fused_gemv_r(GemvShape s, const typename Provider::Args& pargs, const
       return launch_fused_gemv_r<ACT, Provider, R, CB_LDS, X_LDS, MT, H, false>(s, pargs, plan, cb_bytes, st, what);
     }
   }
-  if constexpr (gemv_loads_lines<Provider, R, CB_LDS, H>) {
-    if constexpr (XS) {  // in the wave's own staging area, between the reads of one step's activations and the stores of the next's
-      s.turn_offset = s.stage_offset;
-      s.turn_bytes = MT * GemvStage<H>::kBytes;
-    } else {
-      s.turn_offset = (lds + 15) & ~15;
-      s.turn_bytes = 2048;
-      lds = s.turn_offset + plan.waves * s.turn_bytes;
-    }
+  if constexpr (gemv_loads_lines<Provider, R, CB_LDS, H> && !XS) {
+    s.stage_offset = (lds + 15) & ~15;
+    lds = s.stage_offset + plan.waves * kGemvTurnBytes;
   }
   if (s.plan_only) {
     *s.plan_only = XS ? 1 : 0;

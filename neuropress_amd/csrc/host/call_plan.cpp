@@ -3,10 +3,13 @@
 //
 // What bounds a decode step of small layers is the time to issue its launches, not the kernels: through
 // Python argument checks and ctypes a call took 12-19 us of host time against 3-9 us of kernel.  Through a plan it
-// takes 3.6-4.5 us, 2.4 of them the HIP launch itself and 0.8 the output's allocation (us per eager call, before / now:
-// 2048 x 640 with a 256-row codebook 15.1 / 4.4, the nine calls of a block with hidden size 2048 132 / 43 -- both go with the
-// process, 3.6-4.5 and 37-44 have been seen --, residual VQ 4096 x 4096 18.1 / 8.6 and int4 14336 x 4096 12.6 / 8.2, which
-// are then bound by their kernels).  The looks at what torch follows (tracked) are 0.03 of it.  A plan
+// takes 3.4 us in a stream of calls, 2.4 of them the HIP launch itself and 0.5 the output's allocation (us per eager call, before / now:
+// 2048 x 640 with a 256-row codebook 15.1 / 3.5, the nine calls of a block with hidden size 2048 132 / 36).  In other processes
+// the same calls take 4.3 and 44: the first 75 or so launches behind a synchronisation then cost 6 to 12 us each, inside the
+// runtime.  A bare loop over the launch shows it as well; what selects it is which CPU the scheduler gives the runtime's own
+// thread, busy with the commands of the time before while this one launches (moved by hand, each process goes from one state
+// to the other, whatever this file does).  (Residual VQ 4096 x 4096 18.1 / 8.2 and int4 14336 x 4096 12.6 / 8.2
+// are bound by their kernels.)  The looks at what torch follows (tracked) are 0.03 of it.  A plan
 // keeps the entry point's constant arguments (addresses, sizes, the kernel that serves a token count) and does
 // per call only what depends on the call: check that nothing it was built from has changed, allocate the output,
 // pass the addresses on.
