@@ -121,3 +121,98 @@ def test_module_takes_the_slice_gemm_where_it_was_timed_faster(gpu, monkeypatch,
         torch.testing.assert_close(layer(x).float(), ref, rtol=2e-3, atol=5e-3)
     layer._derived["sliced"] = (key, (None, 0, ((1, 1.0, 1.0),)))
     assert not layer._slice_gemm_wins(12)
+
+
+def _timed_module(gpu, n, k, nc, act, perm=False, bias=False, seed=5):
+    """A lowered layer as if both GEMVs had been timed at a millisecond, so that the slice GEMM serves up to 32 tokens; and its
+    weight as torch multiplies it (columns of x in their own order), in float32."""
+    from neuropress_amd import AutoKernelLowering
+    from neuropress_amd.qweights import VQWeight, attach_quantized_weight
+
+    L = cases.vq_layer(seed + n + k, n, k, nc, act=act, m=1, bias=True, std=0.05)
+    order = torch.randperm(k, generator=cases.gen(seed)) if perm else None
+    weight = VQWeight.from_indices(L["idx"], L["cb"], n, k, column_permutation=order)
+    linear = attach_quantized_weight(torch.nn.Linear(k, n, bias=False, device="meta"), weight)
+    if bias:
+        linear.bias = torch.nn.Parameter(L["bias"], requires_grad=False)
+    model = torch.nn.Sequential(linear)
+    AutoKernelLowering().apply(model)
+    layer = model.to(gpu)[0]
+    packed = layer.packed_indices
+    layer._derived["sliced"] = ((packed.device, packed.data_ptr(), packed._version), (None, 0, ((1, 1e3, 1e3),)))
+    layer._plan = None
+    w = kernels.vq_dequant(packed, L["cb"].to(gpu), layer.bits, n, k, act).float()
+    if order is not None:
+        w = w[:, torch.argsort(order).to(gpu)]
+    return layer, w, L["bias"].to(gpu).float() if bias else torch.zeros(n, device=gpu)
+
+
+def _near(y, x, w, b, act):
+    """Sums are f32 and the output is rounded once: half an ulp of it, and 2^-20 of the products' absolute values."""
+    ref = x.double() @ w.double().t() + b.double()
+    tol = 2.0 ** (-11 if act == torch.float16 else -8) * ref.abs() + 2.0 ** -20 * (x.double().abs() @ w.double().abs().t()) + 1e-6
+    return bool(((y.double() - ref).abs() <= 1.01 * tol).all())
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("k,perm,bias", [(1000, False, True), (1000, True, False), (584, False, False), (1024, True, True)])
+def test_module_slice_band_eager_planned_captured_and_on_two_streams(gpu, act, k, perm, bias):
+    """K that is no whole number of 64-column chunks (rows padded with zeros), columns permuted, a bias: the module's first
+    call, the calls its plan issues, a captured call replayed between eager work, and calls on two streams at once, each with
+    a workspace of its own."""
+    n, nc, m = 300, 9000, 12
+    layer, w, b = _timed_module(gpu, n, k, nc, act, perm, bias)
+    xs = [torch.randn(m, k, generator=cases.gen(i)).to(act).to(gpu) for i in range(4)]
+    assert layer._band(xs[0], m) == "slice"
+    eager = [layer(x) for x in xs]
+    assert layer._plan is not None
+    for x, y in zip(xs, eager):
+        assert _near(y, x, w, b, act)
+        assert torch.equal(layer(x), y)
+    static, s = xs[0].clone(), torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        layer(static)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            out = layer(static)
+    for i in (1, 2, 3, 0):
+        static.copy_(xs[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[i]), f"replay on input {i}"
+        assert torch.equal(layer(xs[i]), eager[i])
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    got = []
+    for turn in range(8):
+        for j, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got.append((2 * j + turn % 2, layer(xs[2 * j + turn % 2])))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, eager[i]) for i, y in got)
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+def test_module_with_real_lists_takes_the_slice_gemm(gpu, act):
+    """A layer large enough for slice lists, prepared and timed as a program prepares it: one token goes to the lists, sixteen to
+    the slice GEMM (16 against 37 us for lookups in memory on a layer of this size), and every count to the kernel of its
+    band whichever count came first."""
+    from neuropress_amd.nn import NPVQLinear, VQProxy
+
+    n, k, nc = 8192, 4096, 16384
+    L = cases.vq_layer(11, n, k, nc, bits=16, act=act, m=1, std=0.05)
+    layer = NPVQLinear(VQProxy(L["cb"]).to(gpu), L["packed"].to(gpu), 16, n, k, 8, "cuda_wmma").to(gpu)
+    assert layer.prepare_sliced()
+    counts = layer._slice_gemm_counts()
+    assert 16 in counts and 1 not in counts
+    w = kernels.vq_dequant(layer.packed_indices, L["cb"].to(gpu), 16, n, k, act).float()
+    b = torch.zeros(n, device=gpu)
+    for m in (1, 16, 2, 3, 7, 32, 5, 1):
+        x = torch.randn(m, k, generator=cases.gen(m)).to(act).to(gpu)
+        assert (layer._band(x, m) == "slice") == (m in counts)
+        first = layer(x)
+        assert _near(first, x, w, b, act), m
+        if m in counts:  # partial sums in a fixed order, and nothing but this kernel gives these bits
+            assert torch.equal(first, kernels.vq_slice_gemm(x, layer.packed_indices, layer.proxy.centroids_as(act), n))
+        assert torch.equal(layer(x), first)
