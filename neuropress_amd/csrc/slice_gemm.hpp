@@ -13,7 +13,8 @@
 // (through the module 36.9 / 24.4), 14336 x 4096 39 / 32, 8192 x 8192 43 / 28; with 16384 rows 37 / 16.6, 37 / 16.6 and 41 / 17;
 // with 8192 rows 34 / 14.8, 34 / 14.9 and 37 / 13.2.  Where it goes at 4096 x 14336 with 65536 rows (kernel 21.5): 8.5 for the
 // launch, the fill and the end, 0.93 per super-step of 256 rows -- LDS reads 0.6 of it, the rest mostly waiting for
-// activations and indices -- and 6 for the reduction.  What did not pay: checks for infinities on the way to LDS
+// activations and indices -- and the reduction, 6 of the 27.5 and 3 of the 24.4.  LDS is active in 84 % of the walk's cycles
+// (50 % of the launch), matrix pipes 30 % and vector instructions 32 % of the launch.  What did not pay: checks for infinities on the way to LDS
 // (0.15 per super-step; now only where a sum shows one), sixteen waves of half the registers, all activations read behind
 // one barrier (a third of the time in waits), eight row tiles per wave, a reduction by four waves per row.
 //

@@ -17,8 +17,9 @@ band                  condition                        kernel
 ====================  ==============================  ==========================
 (a) fused GEMV        ``m <= _FUSED_MAX_TOKENS``, or   ``kernels.vq_linear``
                       ``m <= 32`` while x is small
-    slice GEMM        2 to 32 tokens of large tables,  ``kernels.vq_slice_gemm``
-                      where timed lists say so
+    slice GEMM        up to 32 tokens of large tables, ``kernels.vq_slice_gemm``
+                      where timed lists say so (one
+                      token: only where they lost)
 (b) tile-decode GEMM  ``m <= _TILE_MAX_TOKENS``        ``kernels.vq_gemm_tile``
 (c) decode + GEMM     otherwise                        ``kernels.vq_dequant`` + ``kernels.dense_linear`` or ``F.linear``
 ====================  ==============================  ==========================
