@@ -146,3 +146,26 @@ def test_decode_and_gather_in_one_launch(gpu, dtype, bits, nc, m, k, perm):
               torch.cuda.current_stream().cuda_stream)  # fmt: skip
     assert torch.equal(w, kernels.vq_dequant(packed, cb, bits, n, width, dtype))
     assert torch.equal(out, kernels.gather_columns(x, p, width))
+
+
+@pytest.mark.parametrize("bits,nc,n", [(8, 200, 1024), (8, 200, 1025), (16, 65536, 2048), (16, 65536, 2049)])
+@pytest.mark.parametrize("k", [16384, 16380])
+def test_decode_and_gather_on_both_sides_of_the_line_for_long_rows(gpu, bits, nc, n, k):
+    """The longest rows the one launch takes, layers up to its line and one row past it (the two calls): the same bytes."""
+    from neuropress_amd import _lib, kernels
+    from neuropress_amd.transforms.vq_packing import IndexPacking
+
+    m, width = 5, 16384
+    assert _lib.load().npamd_diag_gather_fits_decode(bits, n * width // 8, k, 1) == (n in (1024, 2048))
+    g = torch.Generator().manual_seed(n + k)
+    packed = IndexPacking.pack(torch.randint(0, nc, (n * width // 8,), generator=g), bits).to(gpu)
+    cb = torch.randn(nc, 8, generator=g).half().to(gpu)
+    x = torch.randn(m, k, generator=g).half().to(gpu)
+    p = torch.randperm(k, generator=g).int().to(gpu)
+    w = torch.full((n, width), 7.0, dtype=torch.half, device=gpu)
+    out = torch.full((m, width), 7.0, dtype=torch.half, device=gpu)
+    _lib.call("npamd_vq_dequant_gather", packed.data_ptr(), packed.numel(), bits, cb.data_ptr(), nc, 8, n * width // 8, w.data_ptr(),
+              _lib.F16, x.data_ptr(), x.stride(0), p.data_ptr(), out.data_ptr(), width, m, k,
+              torch.cuda.current_stream().cuda_stream)  # fmt: skip
+    assert torch.equal(w, kernels.vq_dequant(packed, cb, bits, n, width, torch.half))
+    assert torch.equal(out, kernels.gather_columns(x, p, width))
