@@ -140,7 +140,8 @@ int npamd_q_gemv_staging(int M, int N, int K, int nbits, int group_size, const v
  * irrelevant before and after (nobody clears it); two calls that may run at the
  * same time -- replays of one captured call among them -- need a workspace each.
  * Calls that share one all the same end, with undefined results: a part waits for
- * the other's tile no longer than about a second.
+ * the other's tile no longer than about a second.  Replays that did may leave words
+ * that the next replay of the same captured call takes for its own; no other call does.
  */
 int npamd_vq_gemm_tile(const void* x, int64_t ldx, const uint8_t* packed, int64_t n_bytes,
                        int bits, const void* codebook, int codebook_dtype, int nc, int vl,
