@@ -84,6 +84,23 @@ int npamd_vq_gemv(const void* x, int64_t ldx, const uint8_t* packed, int64_t n_b
                   int act_dtype, void* stream);
 
 /*
+ * The same for any number of tokens, 32 to a workgroup, each of which decodes the weights again: for layers so small
+ * that one launch of it is over before decode + product would be (npamd_gemv_blocks_preferred).  Rows of x may end inside the
+ * index rows' last 64 columns: k_in columns, a multiple of 8 with K - 64 < k_in <= K; what lies past them counts as zero, in x
+ * and in the weights (the indices there are fillers).  Only shapes and alignments that the MFMA kernels take
+ * (npamd_vq_fused_supported, residual streams of 8 bits next to 8 / 12 / 16, or 16 next to 16); others are NPAMD_ERR_UNSUPPORTED.
+ */
+int npamd_vq_gemv_blocks(const void* x, int64_t ldx, int k_in, const uint8_t* packed, int64_t n_bytes,
+                         int bits, const void* codebook, int codebook_dtype, int nc, int vl,
+                         const float* bias, void* y, int64_t ldy, int M, int N, int K,
+                         int act_dtype, void* stream);
+
+/* Whether the *_gemv_blocks entry point is the better choice for more than 16 tokens against decode + dense product and the tile GEMM.
+ * kind: 0 VQ with a codebook of table_rows rows of eight, 1 residual VQ (rows of the main codebook), 4 / 8 bits per weight (table_rows
+ * ignored).  gathered: the columns of x have to be gathered first, which npamd_vq_dequant_gather does next to the decode.  Host-only arithmetic. */
+int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int table_rows, int gathered);
+
+/*
  * The same GEMV with the reference's column permutation folded in:
  *   y[m, n] = sum_k x[m, column_perm[k]] * W[n, k] (+ bias[n]),
  * i.e. vq_linear applied to x[..., column_perm] (neuropress/nn/np_vq_linear.py:1027-1028)
@@ -343,6 +360,15 @@ int npamd_rvq_gemv(const void* x, int64_t ldx,
                    const float* bias, void* y, int64_t ldy, int M, int N, int K,
                    int act_dtype, void* stream);
 
+/* npamd_rvq_gemv for any number of tokens and ragged rows of x: see npamd_vq_gemv_blocks. */
+int npamd_rvq_gemv_blocks(const void* x, int64_t ldx, int k_in,
+                          const uint8_t* packed_main, int64_t n_bytes_main, int bits_main,
+                          const uint8_t* packed_res, int64_t n_bytes_res, int bits_res,
+                          const void* cb_main_f16, int nc_main, const void* cb_res_f16, int nc_res,
+                          const void* row_scale_f16, const void* row_bias_f16, int vl,
+                          const float* bias, void* y, int64_t ldy, int M, int N, int K,
+                          int act_dtype, void* stream);
+
 int npamd_rvq_gemm_tile(const void* x, int64_t ldx,
                         const uint8_t* packed_main, int64_t n_bytes_main, int bits_main,
                         const uint8_t* packed_res, int64_t n_bytes_res, int bits_res,
@@ -381,6 +407,11 @@ int npamd_q_fused_supported(int K, int nbits, int group_size);
 int npamd_q_gemv(const void* x, int64_t ldx, const uint8_t* w_pack, const void* scale_f16,
                  const void* zero_point_f16, const float* bias, void* y, int64_t ldy,
                  int M, int N, int K, int nbits, int group_size, int act_dtype, void* stream);
+
+/* npamd_q_gemv for any number of tokens, 4 and 8 bits: see npamd_vq_gemv_blocks. */
+int npamd_q_gemv_blocks(const void* x, int64_t ldx, const uint8_t* w_pack, const void* scale_f16,
+                        const void* zero_point_f16, const float* bias, void* y, int64_t ldy,
+                        int M, int N, int K, int nbits, int group_size, int act_dtype, void* stream);
 
 /*
  * Fused dequant MFMA GEMM, any M.  The reference has no kernel of its own here

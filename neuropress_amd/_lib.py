@@ -33,6 +33,7 @@ SIGNATURES: dict[str, list] = {
     "npamd_vq_dequant": [_vp, _i64, _int, _vp, _int, _int, _i64, _vp, _int, _vp],
     "npamd_vq_dequant_gather": [_vp, _i64, _int, _vp, _int, _int, _i64, _vp, _int, _vp, _i64, _vp, _vp, _i64, _int, _int, _vp],
     "npamd_vq_gemv": _VQ_LINEAR,
+    "npamd_vq_gemv_blocks": _VQ_LINEAR[:2] + [_int] + _VQ_LINEAR[2:],
     "npamd_vq_gemv_perm": _VQ_LINEAR[:2] + [_vp] + _VQ_LINEAR[2:],
     "npamd_vq_gemv_perm_supported": [_int] * 6,
     "npamd_vq_gemm_tile": _VQ_LINEAR[:-1] + _WS + [_vp],
@@ -57,9 +58,11 @@ SIGNATURES: dict[str, list] = {
     "npamd_rvq_dequant": [_vp, _i64, _int, _vp, _i64, _int, _vp, _int, _vp, _int, _vp, _vp, _int,
                           _int, _int, _vp, _int, _vp],  # fmt: skip
     "npamd_rvq_gemv": _RVQ_LINEAR,
+    "npamd_rvq_gemv_blocks": _RVQ_LINEAR[:2] + [_int] + _RVQ_LINEAR[2:],
     "npamd_rvq_gemm_tile": _RVQ_LINEAR[:-1] + _WS + [_vp],
     "npamd_q_dequant": [_vp, _vp, _vp, _int, _int, _int, _int, _vp, _int, _vp],
     "npamd_q_gemv": _Q_LINEAR,
+    "npamd_q_gemv_blocks": _Q_LINEAR,
     "npamd_rms_norm": [_vp, _i64, _vp, _vp, _i64, _int, _int, ctypes.c_float, _int, _vp],
     "npamd_vq_embedding": [_vp, _i64, _vp, _i64, _int, _vp, _int, _int, _vp, ctypes.c_float, _vp, _int, _vp],
     "npamd_q_embedding": [_vp, _i64, _vp, _vp, _vp, _int, _int, _i64, _int, _i64, ctypes.c_float, _vp, _int, _vp],
@@ -67,6 +70,7 @@ SIGNATURES: dict[str, list] = {
     "npamd_dense_gemm": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _int, _int, _int, _int, _vp, _i64, _vp],
     "npamd_dense_gemm_workspace_bytes": [_int, _int, _int],
     "npamd_dense_gemm_preferred": [_int, _int, _int],
+    "npamd_gemv_blocks_preferred": [_int] * 6,
     "npamd_gather_columns": [_vp, _i64, _vp, _vp, _i64, _int, _int, _vp],
     "npamd_diag_reload_tuning": [],
     "npamd_diag_last_gemv_staged": [],

@@ -117,7 +117,28 @@ bool gemv_stage_activations(int M) {
   return mode >= 2 || (mode == 1 && M >= 3);
 }
 
-GemvPlan plan_gemv(int N, int chunks, int max_r, int max_waves_cap) {
+// Whether the blocks of 17 and more tokens look a table that LDS could hold up in memory: where their lookups are few, the copy
+// is what a block waits for, and a table of more than 32 KiB next to 16 KiB of activations per wave leaves room for six waves.
+// fp16, 64 tokens, table in LDS / in memory, us: 256 rows 512 x 512 4.7 / 4.0, 8192 x 512 6.4 / 6.0, 1024 x 1024 4.8 / 4.7, but at 512
+// tokens 1024 x 1024 (8192 lookups per compute unit) 6.9 / 9.2 and 2048 x 2048 (whose blocks have 4096) 5.7 / 5.7; 4096 rows 512 x 2048
+// 7.3 / 5.4, 2048 x 2048 10.0 / 7.0, 1024 x 4096 9.6 / 8.1, at 128 tokens 9.1 / 12.5 and 9.8 / 10.3.
+bool gemv_wide_looks_up_in_memory(int M, int row_tiles, int chunks, int cb_bytes) {
+  const int cus = device_cu_count();
+  const int64_t block = (int64_t)16 * chunks * 8, fullest = (row_tiles + cus - 1) / cus * block;
+  return fullest <= 4096 && (block <= 2048 || (cb_bytes > 32 * 1024 && M > 24));
+}
+
+// Row tiles of a block with staged activations next to the table: two where one leaves compute units a second round of blocks
+// (us with one / two / four, 24 tokens: 14336 x 4096 21.6 / 13.7 / 15.6 with 256 rows, 23.4 / 14.7 / 16.0 with 4096; 128 tokens: 2048 x
+// 2048 9.7 / 6.5 / 11.1, 4096 x 1024 9.5 / 6.9 / 9.8; 256 tokens 1024 x 4096 13.1 / 8.4 / 16.5).  Large tables past 24 tokens leave room for
+// six waves: four row tiles, activations from memory, on large grids (14336 x 4096 at 32 tokens 32.9 / 20.4 / 18.4).
+int gemv_wide_row_tiles(int M, int row_tiles, int cb_bytes) {
+  const int cus = device_cu_count();
+  if (cb_bytes > 32 * 1024 && M > 24 && row_tiles * 10 >= cus * 24) return 4;
+  return row_tiles > cus ? 2 : 1;
+}
+
+GemvPlan plan_gemv(int N, int chunks, int max_r, int max_waves_cap, bool exact) {
   const int steps = (chunks + 3) / 4;
   const int tiles = (N + 15) / 16;
   const int64_t jobs = (int64_t)tiles * steps;
@@ -131,7 +152,7 @@ GemvPlan plan_gemv(int N, int chunks, int max_r, int max_waves_cap) {
   // and one copy of the codebook in LDS.  The largest R that leaves blocks for at least 0.6 of
   // the compute units wins at every token count, measured on N = 2048 ... 28672.
   p.R = (tiles * 10 >= cus * 24) ? 4 : (tiles * 10 >= cus * 12) ? 2 : 1;
-  if (p.R > max_r) p.R = max_r;
+  if (p.R > max_r || exact) p.R = max_r;
   int spw = (jpw + p.R - 1) / p.R;
   const int r_env = tuning().gemv_r;
   if (r_env == 1 || r_env == 2 || r_env == 4) p.R = r_env;

@@ -383,6 +383,50 @@ extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64
   return act_dtype == NPAMD_BF16 ? launch_dense<NPAMD_BF16>(s, tile, st) : launch_dense<NPAMD_F16>(s, tile, st);
 }
 
+// Whether a call of more than 16 tokens goes to the GEMV with a block per 32 tokens (npamd_*_gemv_blocks) rather than to decode +
+// product or the tile GEMM.  Up to a round or two of its blocks it is one short launch in the place of two that follow each
+// other; past that every block of tokens decodes its weights again.  All three are estimated.  kind: 0 VQ, 1 residual VQ, 4 and 8 bits
+// per weight.  The GEMV's figures are fitted to layers of 512 to 8192 rows and K of 512 to 14336 at 33 to 512 tokens (within 10 %, residual
+// VQ as with indices that are all as frequent).  us, before / blocks, at 64 and 256 tokens: int4 512 x 512 6.9 / 4.0 and 6.9 / 4.1,
+// 1024 x 4096 11.8 / 6.4 and 13.3 / 9.5, 3072 x 3072 14.8 / 8.2; 256 rows 1024 x 1024 7.9 / 4.7 and 8.0 / 5.7, 2048 x 2048 10.4 / 5.7 and 11.1 / 11.2;
+// 4096 rows 1024 x 1024 8.1 / 4.7 and 8.1 / 6.6; 65536 rows 512 x 512 7.0 / 4.2 and 7.1 / 4.8, 1024 x 4096 13.2 / 10.0 and 16.5 / 24.8.
+namespace npamd {
+static float gemv_blocks_us(int kind, int table_rows, int M, int N, int K) {
+  constexpr int cus = 256;
+  const int tokens = (M + kGemvTokens - 1) / kGemvTokens, rows = (N + 15) / 16, tiles = rows * tokens;
+  const int steps = (K + 255) / 256, chunks = (K + 63) / 64, load = (tiles + cus - 1) / cus;
+  auto per = [](int a, int b) { return (a + b - 1) / b; };
+  if (kind == 4) return 2.6f + 0.18f * load * steps + 0.7f * load;
+  if (kind == 8) return load <= 1 ? 3.3f + 0.24f * steps : 1.8f + per((rows + 1) / 2 * tokens, cus) * (3.4f + 0.25f * steps);
+  const int table = table_rows * 16;
+  if (kind == 0 && table <= kGemvLdsCodebookMax && !gemv_wide_looks_up_in_memory(M, tiles, chunks, table)) {
+    const int R = gemv_wide_row_tiles(M, tiles, table);
+    const int waves = R < 4 && table > 32 * 1024 ? 6 : 8, spw = per(steps, waves), rounds = per(per(rows, R) * tokens, cus);
+    return 1.8f + rounds * (R == 1 ? 1.4f + 2.1f * spw : R == 2 ? 2.7f + 2.0f * spw : 8.5f + 3.0f * spw);
+  }
+  const float lookups = 2.0f * K;  // of a block
+  const float served = table_rows <= 2048 ? 1100e3f : 275e3f;  // by the L1s; by the L2s
+  return (kind == 1 ? 4.1f : 3.3f) + load * lookups / 2400.f + tiles * lookups / served;
+}
+}  // namespace npamd
+
+extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int table_rows, int gathered) {
+  if (M <= 16 || N < 1 || K < 64 || K % 64) return 0;
+  const float gather = gathered ? 3.0f + M * (float)K * 4 / 4.4e6f : 0.f;
+  const float blocks = gemv_blocks_us(kind, table_rows, M, N, K) + gather;
+  const float weights = (float)N * K;
+  const bool gathers = kind < 4 && table_rows > 2048;
+  const float decode = 2.0f + fmaxf(gathers ? weights / 8 / 236e3f : 0.f, weights * 2 / 4.4e6f);
+  const float product = fmaxf(6.8f, decode + plan_dense(M, N, K, 0, kDenseMaxSplits).us);
+  if (blocks * 1.03f >= product) return 0;
+  const int columns = (N + 63) / 64 * ((M + 383) / 384), chunks = K / 64;
+  int splits = columns * 10 < 256 * 7 ? 256 / columns : 1;
+  splits = splits > chunks / 8 ? chunks / 8 : splits;
+  splits = splits > 16 ? 16 : splits < 1 ? 1 : splits;
+  const float tile = gather + (kind == 0 && table_rows <= 4096 ? 0.9f : kind >= 4 ? 1.05f : 1.15f) * (7.8f + 0.25f * chunks / splits + (splits > 1 ? 2.5f : 0.f));
+  return blocks * 1.03f < tile ? 1 : 0;
+}
+
 // Where this kernel is the better one against the library's product: its estimate against what the library reaches
 // (5 us + 0.85 PFLOP/s; 1.3 once 256 x 256 tiles cover 180 compute units; 1.5 us more per 1024 of K past 4096, which it
 // walks in few tiles) -- or against 25 us: a library product takes 18.3-19 us per eager call whatever its size and

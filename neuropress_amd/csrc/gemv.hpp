@@ -36,11 +36,26 @@ struct GemvShape {
   // Optional gather of the activation columns: the kernel contracts x[m, perm[k]] with W[n, k].
   // Only with the X_LDS variant (every block first copies the permuted rows of x into LDS).
   const int32_t* perm = nullptr;
+  // 16-byte pieces of a row of x: fewer than 8 * chunks where its columns end inside the last chunk (0: they do not).  What lies
+  // past them counts as zero, the weights there (filler rows of the index stream) too.
+  int pieces = 0;
   int stage_offset = 0;  // byte offset of the waves' own areas in LDS: XS kernels stage activations there, kernels that load index lines turn them
   // Planning only: when set, the launcher writes here whether the kernel it chose stages its
   // activations (1 / 0) and launches nothing.
   int* plan_only = nullptr;
 };
+
+// Tokens of one block.  More of them (npamd_*_gemv_blocks) are blocks of their own, along y, each of which decodes its weights: on a
+// small layer the grid of one launch then fills the compute units that the rows alone leave empty, and the call is over in
+// the time that decode + product spend on being two launches (npamd_gemv_blocks_preferred has the figures).
+constexpr int kGemvTokens = 32;
+__device__ __forceinline__ GemvShape gemv_token_block(GemvShape s) {
+  const int m0 = blockIdx.y * kGemvTokens;
+  s.M = min(s.M - m0, kGemvTokens);
+  s.x = reinterpret_cast<const uint16_t*>(s.x) + (int64_t)m0 * s.ldx;
+  s.y = reinterpret_cast<uint16_t*>(s.y) + (int64_t)m0 * s.ldy;
+  return s;
+}
 
 // Largest M * K (elements) whose activations the GEMV stages in LDS (32 KiB; the unpermuted
 // copy shares its place with the codebook of up to 64 KiB).
@@ -102,10 +117,11 @@ template <class Provider, int R, bool CB_LDS, int H>
 constexpr bool gemv_loads_lines = Provider::kLdsResidual && CB_LDS && R == 1 && H == 1;
 template <int ACT, class Provider, int R, bool CB_LDS, bool X_LDS, int MT = 1, int H = 1, bool XS = false>
 __global__ void __launch_bounds__((kGemvMaxWaves<R, MT> * 64))
-fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
+fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
+  const GemvShape s = gemv_token_block(all);
   static_assert(H == 1 || ((H == 2 || H == 4) && R == 1 && MT == 1), "k parts only with one row tile and one token tile");
   constexpr bool kStageLines = CB_LDS && Provider::kLdsCodebook;
-  static_assert(!XS || (!X_LDS && (kStageLines ? MT == 1 && H == 1 : R == 1)), "staged activations: the forms there are");
+  static_assert(!XS || (!X_LDS && (kStageLines ? H == 1 : R == 1)), "staged activations: the forms there are");
   constexpr bool kLines = gemv_loads_lines<Provider, R, CB_LDS, H>;
   constexpr int RT = 16 / H;  // weight rows (and tokens) per MFMA tile
   extern __shared__ __attribute__((aligned(16))) float red[];  // [waves][M][16*R] (+ codebook copy)
@@ -137,8 +153,9 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
     for (int i = threadIdx.x; i < items; i += blockDim.x) {
       const int m = i / k8s;
       const int k8 = i - m * k8s;
-      *reinterpret_cast<u32x4*>(xraw + (int64_t)i * 8) =
-          *reinterpret_cast<const u32x4*>(xg + (int64_t)m * s.ldx + k8 * 8);
+      u32x4 v = *reinterpret_cast<const u32x4*>(xg + (int64_t)m * s.ldx + min(k8, s.pieces - 1) * 8);
+      if (k8 >= s.pieces) v = u32x4{0, 0, 0, 0};
+      *reinterpret_cast<u32x4*>(xraw + (int64_t)i * 8) = v;
     }
     if (s.perm) {
       __syncthreads();
@@ -146,18 +163,56 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
         const int m = i / k8s;
         const int k8 = i - m * k8s;
         const uint16_t* xr = xraw + (int64_t)m * K;
-        const u32x4 p0 = *reinterpret_cast<const u32x4*>(s.perm + k8 * 8);
-        const u32x4 p1 = *reinterpret_cast<const u32x4*>(s.perm + k8 * 8 + 4);
+        const u32x4 p0 = *reinterpret_cast<const u32x4*>(s.perm + min(k8, s.pieces - 1) * 8);
+        const u32x4 p1 = *reinterpret_cast<const u32x4*>(s.perm + min(k8, s.pieces - 1) * 8 + 4);
         u32x4 v;
         v.x = (uint32_t)xr[p0.x] | ((uint32_t)xr[p0.y] << 16);
         v.y = (uint32_t)xr[p0.z] | ((uint32_t)xr[p0.w] << 16);
         v.z = (uint32_t)xr[p1.x] | ((uint32_t)xr[p1.y] << 16);
         v.w = (uint32_t)xr[p1.z] | ((uint32_t)xr[p1.w] << 16);
+        if (k8 >= s.pieces) v = u32x4{0, 0, 0, 0};
         *reinterpret_cast<u32x4*>(xs + (int64_t)i * 8) = v;
       }
       if constexpr (CB_LDS) __syncthreads();  // the codebook overwrites the unpermuted copy
     }
     x_lds = xs;
+  }
+  const int c = lane & 15;
+  const int q = lane >> 4;
+  const int cr = c & (RT - 1), part = c / RT;  // H = 1: cr = c, part = 0
+  const int row0 = blockIdx.x * (RT * R);
+  const int step_begin = wave * s.steps_per_wave;
+  const int step_end = min(step_begin + s.steps_per_wave, s.steps);
+  typename Provider::Raw raw[R];
+  auto load_packed = [&](int step) {
+    if constexpr (kLines) {
+      prov.load(raw[0], min(row0 + (lane >> 2), s.N - 1), min(step * 4 + (lane & 3), s.chunks - 1));
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) prov.load(raw[r], min(row0 + 16 * r + cr, s.N - 1), min((step * 4 + q) * H + part, s.chunks - 1));
+    }
+  };
+  // Two tokens per instruction straight into LDS, past M and K the last row and piece again.
+  auto stage_lines = [&](int step) {
+    using SL = GemvStageLines;
+    const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)red + (uint32_t)(s.stage_offset + wave * SL::bytes(s.M));
+    for (int at = 0; at < SL::bytes(s.M); at += 1024) {
+      const int row = at / 512 + (lane >> 5), piece = SL::slot(lane & 31, row);
+      const uint16_t* src = reinterpret_cast<const uint16_t*>(s.x) + (int64_t)min(row, s.M - 1) * s.ldx + min(step * 32 + piece, s.pieces - 1) * 8;
+      // The statement writes m0: see the codebook's copy.
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(
+                       __builtin_amdgcn_readfirstlane(mine + (uint32_t)at)), "v"(src) : "memory");
+    }
+  };
+  // Next to a table in LDS, activations staged: the first step's packed bytes and activations are asked for in front of the
+  // table, whose copy waits for all of them at once.  Both at 17 and more tokens, us before / now (24 tokens): 512 x 2048 with 256 rows
+  // 6.0 / 4.8, 1024 x 4096 9.5 / 6.4, 14336 x 4096 15.6 / 13.7 with 256 rows and 16.0 / 14.7 with 4096.
+  constexpr bool kFirstAhead = XS && kStageLines && (R == 1 || MT == 2);  // two row tiles within 128 registers: no room
+  if constexpr (kFirstAhead) {
+    if (step_begin < step_end) {
+      load_packed(step_begin);
+      stage_lines(step_begin);
+    }
   }
   if constexpr (CB_LDS) {
     // Four requests per thread in flight: a block of few waves (short K) would otherwise copy
@@ -178,7 +233,6 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
         const uint32_t voff = (uint32_t)(chunk * 64 + lane) * 16u;
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(src) : "memory");
       }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     } else
     for (int base = threadIdx.x; base < n16; base += (int)blockDim.x * kBatch) {
       u32x4 t[kBatch];
@@ -189,13 +243,10 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
       for (int j = 0; j < kBatch; ++j)
         if (base + j * (int)blockDim.x < n16) cb_lds[base + j * (int)blockDim.x] = t[j];
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     prov.use_codebook(cb_lds);
   }
   if constexpr (CB_LDS || X_LDS) __syncthreads();
-  const int c = lane & 15;
-  const int q = lane >> 4;
-  const int cr = c & (RT - 1), part = c / RT;  // H = 1: cr = c, part = 0
-  const int row0 = blockIdx.x * (RT * R);
 
   f32x4 acc[R][MT];
 #pragma unroll
@@ -203,8 +254,6 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int step_begin = wave * s.steps_per_wave;
-  const int step_end = min(step_begin + s.steps_per_wave, s.steps);
   // Loads are branch-free: out-of-range lanes read a clamped (valid) address and
   // their operand is zeroed afterwards, so all gathers of a step are in flight
   // together instead of each sitting behind its own branch and wait.
@@ -222,42 +271,37 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
 
   for (int step = step_begin; step < step_end; ++step) {
     const int kc_raw = (step * 4 + q) * H + part;
+    // Whether piece j of the chunk lies in front of the end of K, in kernels that take rows of x which end inside a chunk.
+    constexpr bool kShortRows = XS || X_LDS;
     const bool kvalid = kc_raw < s.chunks;
+    auto there = [&](int j) { return kShortRows ? kc_raw * 8 + j < s.pieces : kvalid; };
     const int kc = min(kc_raw, s.chunks - 1);
 
-    typename Provider::Raw raw[R];
+    if (!kFirstAhead || step != step_begin) load_packed(step);
     if constexpr (kLines) {
-      prov.load(raw[0], min(row0 + (lane >> 2), s.N - 1), min(step * 4 + (lane & 3), s.chunks - 1));
       constexpr int kTurn = XS ? MT * GemvStage<H>::kBytes : kGemvTurnBytes;
       u32x4* const turn = reinterpret_cast<u32x4*>(reinterpret_cast<uint8_t*>(red) + s.stage_offset + wave * kTurn);
       prov.turn(raw[0], turn, lane ^ (lane >> 4), (4 * c + q) ^ (c >> 2));
-    } else {
-#pragma unroll
-      for (int r = 0; r < R; ++r) prov.load(raw[r], min(row0 + 16 * r + cr, s.N - 1), kc);
     }
 
     u32x4 xa[MT][8];
     if constexpr (XS && kStageLines) {
       using SL = GemvStageLines;
-      const int stage_bytes = SL::bytes(s.M);
-      uint8_t* const mine = reinterpret_cast<uint8_t*>(red) + s.stage_offset + wave * stage_bytes;
-      const uint32_t mine_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)mine;
-      // Two tokens per instruction straight into LDS, past M and K the last row and chunk again.  The step before has
-      // read its activations out (its products waited for them).  The statement writes m0: see the codebook's copy.
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      for (int at = 0; at < stage_bytes; at += 1024) {
-        const int row = at / 512 + (lane >> 5), piece = SL::slot(lane & 31, row);
-        const uint16_t* src = reinterpret_cast<const uint16_t*>(s.x) + (int64_t)min(row, s.M - 1) * s.ldx +
-                              min(step * 4 + piece / 8, s.chunks - 1) * 64 + piece % 8 * 8;
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(
-                         __builtin_amdgcn_readfirstlane(mine_lds + (uint32_t)at)), "v"(src) : "memory");
+      const uint8_t* const mine = reinterpret_cast<const uint8_t*>(red) + s.stage_offset + wave * SL::bytes(s.M);
+      if (!kFirstAhead || step != step_begin) {
+        // The step before has read its activations out (its products waited for them).
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        stage_lines(step);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      const int row = min(cr, s.M - 1);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        xa[0][j] = *reinterpret_cast<const u32x4*>(mine + row * 512 + SL::slot(q * 8 + j, row) * 16);
-        xa[0][j] = (x_lane[0] && kvalid) ? xa[0][j] : zero4;
+      for (int t = 0; t < MT; ++t) {
+        const int row = min(16 * t + cr, s.M - 1);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          xa[t][j] = *reinterpret_cast<const u32x4*>(mine + row * 512 + SL::slot(q * 8 + j, row) * 16);
+          xa[t][j] = (x_lane[t] && there(j)) ? xa[t][j] : zero4;
+        }
       }
     } else if constexpr (XS) {
       // LDS operations of a wave complete in order, so the reads below see the stores above
@@ -272,9 +316,8 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
           const int flat = i * 1024 + lane * 16;
           const int row = min(RT * t + flat / SL::kRowData, s.M - 1);
           const int off = flat % SL::kRowData;
-          const int kcp = min(step * 4 * H + off / 128, s.chunks - 1);
-          tmp[t * 8 + i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(s.x) + (int64_t)row * s.ldx +
-                                                           (int64_t)kcp * 64 + (off % 128) / 2);
+          const int piece = min(step * 32 * H + off / 16, s.pieces - 1);
+          tmp[t * 8 + i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(s.x) + (int64_t)row * s.ldx + piece * 8);
         }
 #pragma unroll
       for (int t = 0; t < MT; ++t)
@@ -290,7 +333,7 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           xa[t][j] = *reinterpret_cast<const u32x4*>(mine + (RT * t + cr) * SL::kRow + (q * H + part) * SL::kChunk + j * 16);
-          xa[t][j] = (x_lane[t] && kvalid) ? xa[t][j] : zero4;
+          xa[t][j] = (x_lane[t] && there(j)) ? xa[t][j] : zero4;
         }
     } else {
 #pragma unroll
@@ -317,11 +360,11 @@ fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
       b[r][6] = prov.template operand<6>(raw[r]);
       b[r][7] = prov.template operand<7>(raw[r]);
     }
-    if (s.chunks % (4 * H)) {  // uniform: only shapes with a ragged last step pay for the select
+    if (s.chunks % (4 * H) || (kShortRows && s.pieces % 8)) {  // uniform: only shapes with a ragged last step pay for the select
 #pragma unroll
       for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) b[r][j] = kvalid ? b[r][j] : zero4;
+        for (int j = 0; j < 8; ++j) b[r][j] = there(j) ? b[r][j] : zero4;
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -371,8 +414,11 @@ struct GemvPlan {
 };
 
 // max_r: most row tiles per block the caller wants (4, or 2 for lookups served by L2);
-// max_waves_cap: most waves per block its kernel variant is built for.
-GemvPlan plan_gemv(int N, int chunks, int max_r = 4, int max_waves_cap = 16);
+// max_waves_cap: most waves per block its kernel variant is built for.  exact: max_r row tiles, whatever the grid.
+GemvPlan plan_gemv(int N, int chunks, int max_r = 4, int max_waves_cap = 16, bool exact = false);
+// 17 tokens and more, tables LDS can hold.  row_tiles: 16-row tiles of all blocks of 32 tokens.
+bool gemv_wide_looks_up_in_memory(int M, int row_tiles, int chunks, int cb_bytes);
+int gemv_wide_row_tiles(int M, int row_tiles, int cb_bytes);  // per block, with staged activations
 // k parts per MFMA tile (1, 2 or 4) for M tokens on an N-row layer: more than one only where
 // whole 16-row tiles would leave most compute units without a block.  NPAMD_GEMV_PARTS overrides.
 // lds_rows: rows of the table every block copies into LDS first (0: none).
@@ -400,24 +446,32 @@ bool gemv_lds_activations_forced();  // NPAMD_GEMV_LDS_X=1: stage x in LDS also 
 template <int ACT, class Provider, int R, bool CB_LDS, bool X_LDS = false, int MT = 1, int H = 1, bool XS = false>
 int launch_fused_gemv_r(GemvShape s, const typename Provider::Args& pargs, const GemvPlan& plan,
                         int cb_bytes, hipStream_t st, const char* what) {
+  if (!XS && !X_LDS && s.pieces < s.chunks * 8)
+    return fail(NPAMD_ERR_UNSUPPORTED, "%s: rows of x that end inside a chunk need a kernel that stages them", what);
   s.steps_per_wave = plan.steps_per_wave;
+  const int M = s.M < kGemvTokens ? s.M : kGemvTokens;  // of a block
   const int blocks = (s.N + 16 / H * R - 1) / (16 / H * R);
-  const int red_bytes = ((plan.waves * s.M * 16 * R + 3) & ~3) * (int)sizeof(float);
-  const int x_bytes = X_LDS ? s.M * s.chunks * 64 * 2 : 0;
+  const int red_bytes = ((plan.waves * M * 16 * R + 3) & ~3) * (int)sizeof(float);
+  const int x_bytes = X_LDS ? M * s.chunks * 64 * 2 : 0;
   const int cb_lds_bytes = CB_LDS ? cb_bytes : 0;
   int lds = (CB_LDS && !X_LDS)
                       ? (red_bytes > cb_lds_bytes ? red_bytes : cb_lds_bytes)
                       : red_bytes + x_bytes +
                             ((X_LDS && s.perm) ? (cb_lds_bytes > x_bytes ? cb_lds_bytes : x_bytes) : cb_lds_bytes);
   if constexpr (XS) {
-    s.stage_offset = (lds + 15) & ~15;
     constexpr bool kStageLines = CB_LDS && Provider::kLdsCodebook;
-    lds = s.stage_offset + plan.waves * (kStageLines ? GemvStageLines::bytes(s.M) : MT * GemvStage<H>::kBytes);
+    if (kStageLines) {  // the reduction buffer, needed after the last step, lies over both
+      s.stage_offset = (cb_lds_bytes + 15) & ~15;
+      lds = max(red_bytes, s.stage_offset + plan.waves * GemvStageLines::bytes(M));
+    } else {
+      s.stage_offset = (lds + 15) & ~15;
+      lds = s.stage_offset + plan.waves * MT * GemvStage<H>::kBytes;
+    }
     if (lds > kGemvLdsPerBlockMax) {  // no room for the staging areas: fewer waves, or the same kernel without them
       GemvPlan fewer = plan;
       fewer.steps_per_wave = plan.steps_per_wave + 1;
       fewer.waves = (s.steps + fewer.steps_per_wave - 1) / fewer.steps_per_wave;
-      if (kStageLines && fewer.waves >= 8)
+      if (s.pieces < s.chunks * 8 || (kStageLines && fewer.waves >= (MT == 2 ? 5 : 8)))
         return launch_fused_gemv_r<ACT, Provider, R, CB_LDS, X_LDS, MT, H, true>(s, pargs, fewer, cb_bytes, st, what);
       return launch_fused_gemv_r<ACT, Provider, R, CB_LDS, X_LDS, MT, H, false>(s, pargs, plan, cb_bytes, st, what);
     }
@@ -438,7 +492,7 @@ int launch_fused_gemv_r(GemvShape s, const typename Provider::Args& pargs, const
       return fail(NPAMD_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds, hipGetErrorString(e));
   }
   last_gemv_staged() = XS ? 1 : 0;
-  launch(fused_gemv_kernel<ACT, Provider, R, CB_LDS, X_LDS, MT, H, XS>, blocks, plan.waves * 64, lds, st, s, pargs);
+  launch(fused_gemv_kernel<ACT, Provider, R, CB_LDS, X_LDS, MT, H, XS>, dim3(blocks, (s.M + kGemvTokens - 1) / kGemvTokens), plan.waves * 64, lds, st, s, pargs);
   return check_launch(what);
 }
 
@@ -452,6 +506,10 @@ template <int ACT, class Provider>
 int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStream_t st,
                       const char* what, int cb_bytes = 0) {
   s.steps = (s.chunks + 3) / 4;
+  if (s.pieces == 0) s.pieces = s.chunks * 8;
+  // Rows of x that end inside the last chunk: the kernels that stage activations, and those that copy x, look where they end.
+  const bool short_rows = s.pieces < s.chunks * 8;
+  auto stages = [&](int tokens) { return short_rows || gemv_stage_activations(tokens); };
   // Layers of few rows, few tokens: 16 / H rows x H parts of k per tile (see the kernel).
   bool lds_table = false;
   if constexpr (Provider::kLdsResidual)
@@ -460,6 +518,9 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
     lds_table = cb_bytes > 0 && cb_bytes <= kGemvLdsCodebookMax && gemv_lds_codebook_enabled();
   int h = plan_gemv_parts(s.M, s.N, s.chunks, lds_table ? cb_bytes / 16 : 0);
   bool whole_codebook_in_lds = lds_table && Provider::kLdsCodebook;
+  const int row_tiles = (s.N + 15) / 16 * ((s.M + kGemvTokens - 1) / kGemvTokens);  // of all blocks of tokens
+  if (whole_codebook_in_lds && s.M > 16 && !s.perm && gemv_wide_looks_up_in_memory(s.M, row_tiles, s.chunks, cb_bytes))
+    lds_table = whole_codebook_in_lds = false;
   if (whole_codebook_in_lds && s.M <= 16 && !s.perm && !gemv_lds_activations_forced()) {
     // A block that has few lookups to make does them in memory rather than copy the table first:
     // with as many parts as the layer admits when nothing is copied, up to 2048 lookups per
@@ -473,11 +534,12 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
       lds_table = whole_codebook_in_lds = false;
     }
   }
+  if (short_rows && whole_codebook_in_lds) h = 1;
   if (h > 1 && !s.perm && !gemv_lds_activations_forced()) {
     s.steps = (s.chunks + 4 * h - 1) / (4 * h);
     const GemvPlan plan = plan_gemv_rows(s.N, 16 / h, s.steps);
     // Staged activations as for whole tiles, except next to a whole codebook in LDS (2048 x 2048 at 8 tokens 4.0 / 4.3 us).
-    const bool staged = gemv_stage_activations(s.M) && !(lds_table && Provider::kLdsCodebook);
+    const bool staged = stages(s.M) && !(lds_table && Provider::kLdsCodebook);
     if constexpr (Provider::kLdsResidual || Provider::kLdsCodebook) {
       if (lds_table) {
         if constexpr (Provider::kLdsResidual) {
@@ -499,15 +561,15 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
     // looks up in memory.
     if (cb_bytes > 0 && cb_bytes <= kGemvLdsResidualMax && gemv_lds_codebook_enabled()) {
       if (s.M > 16) {
-        const GemvPlan plan = plan_gemv(s.N, s.chunks, gemv_stage_activations(s.M) ? 1 : 2, 8);  // as for plain VQ below
+        const GemvPlan plan = plan_gemv(s.N, s.chunks, stages(s.M) ? 1 : 2, 8);  // as for plain VQ below
         if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, true, false, 2>(s, pargs, plan, cb_bytes, st, what);
-        if (gemv_stage_activations(s.M))
+        if (stages(s.M))
           return launch_fused_gemv_r<ACT, Provider, 1, true, false, 2, 1, true>(s, pargs, plan, cb_bytes, st, what);
         return launch_fused_gemv_r<ACT, Provider, 1, true, false, 2>(s, pargs, plan, cb_bytes, st, what);
       }
-      const GemvPlan plan = plan_gemv(s.N, s.chunks, 2);
+      const GemvPlan plan = plan_gemv(s.N, s.chunks, short_rows ? 1 : 2);
       if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, true>(s, pargs, plan, cb_bytes, st, what);
-      if (gemv_stage_activations(s.M))
+      if (stages(s.M))
         return launch_fused_gemv_r<ACT, Provider, 1, true, false, 1, 1, true>(s, pargs, plan, cb_bytes, st, what);
       return launch_fused_gemv_r<ACT, Provider, 1, true>(s, pargs, plan, cb_bytes, st, what);
     }
@@ -525,10 +587,16 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
     // 74.8 / 77.7, 8192 x 8192 47.0 / 50.3 -> 45.3 / 46.8); at 16 tokens and below it depends on
     // the layer (6144 x 4096 20.5 -> 21.45 at 16), so there the plan stands.
     const bool memory_lookups = Provider::kGathers && !cb_in_lds;
-    const GemvPlan plan = plan_gemv(s.N, s.chunks, memory_lookups ? (gemv_stage_activations(s.M) ? 1 : 2) : 4, 8);
+    const int tiles = cb_in_lds && stages(s.M) ? gemv_wide_row_tiles(s.M, row_tiles, cb_bytes) : 0;
+    const int most = short_rows && tiles == 4 ? 2 : tiles;
+    const GemvPlan plan = plan_gemv(16 * row_tiles, s.chunks, most ? most : memory_lookups ? (stages(s.M) ? 1 : 2) : 4, 8, most == 2);
     if constexpr (Provider::kLdsCodebook) {
       if (cb_in_lds) {
         if (plan.R == 4) return launch_fused_gemv_r<ACT, Provider, 4, true, false, 2>(s, pargs, plan, cb_bytes, st, what);
+        if (plan.R == 2 && stages(s.M))
+          return launch_fused_gemv_r<ACT, Provider, 2, true, false, 2, 1, true>(s, pargs, plan, cb_bytes, st, what);
+        if (stages(s.M))
+          return launch_fused_gemv_r<ACT, Provider, 1, true, false, 2, 1, true>(s, pargs, plan, cb_bytes, st, what);
         if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, true, false, 2>(s, pargs, plan, cb_bytes, st, what);
         return launch_fused_gemv_r<ACT, Provider, 1, true, false, 2>(s, pargs, plan, cb_bytes, st, what);
       }
@@ -536,11 +604,11 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
     if constexpr (!Provider::kGathers)
       if (plan.R == 4) return launch_fused_gemv_r<ACT, Provider, 4, false, false, 2>(s, pargs, plan, 0, st, what);
     if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, false, false, 2>(s, pargs, plan, 0, st, what);
-    if (gemv_stage_activations(s.M))
+    if (stages(s.M))
       return launch_fused_gemv_r<ACT, Provider, 1, false, false, 2, 1, true>(s, pargs, plan, 0, st, what);
     return launch_fused_gemv_r<ACT, Provider, 1, false, false, 2>(s, pargs, plan, 0, st, what);
   }
-  const GemvPlan plan = plan_gemv(s.N, s.chunks, (Provider::kGathers && !cb_in_lds) ? 2 : 4);
+  const GemvPlan plan = plan_gemv(s.N, s.chunks, short_rows && !s.perm ? (cb_in_lds ? 2 : 1) : (Provider::kGathers && !cb_in_lds) ? 2 : 4);
   if constexpr (Provider::kLdsCodebook) {
     const bool x_fits = (int64_t)s.M * s.chunks * 64 <= kGemvLdsActivationsMax;
     if (s.perm || (x_fits && gemv_lds_activations_forced())) {  // with a permutation the caller has checked the size
@@ -559,9 +627,9 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
       // with 4096 rows 9.8 / 9.0, 11.2 / 9.2, 13.2 / 10.2, 19.1 / 12.7; 4096 x 4096 4.9 / 5.1, 5.6 / 5.2, 6.2 / 5.5, 7.6 / 6.4; two
       // tiles, 5888 x 7168 at 4 / 8 / 12 / 16 7.7 / 8.0, 8.7 / 8.3, 10.0 / 8.7, 11.4 / 9.8, 8944 x 2176 8.2 / 9.1, 8.7 / 9.4, 9.7 / 9.7,
       // 10.4 / 10.0; four, 14336 x 4096 8.2 / 9.1, 8.7 / 9.4, 9.6 / 10.0, 10.3 / 10.3.
-      if (plan.R == 2 && s.M >= 9 && gemv_stage_activations(s.M))
+      if (plan.R == 2 && (short_rows || (s.M >= 9 && stages(s.M))))
         return launch_fused_gemv_r<ACT, Provider, 2, true, false, 1, 1, true>(s, pargs, plan, cb_bytes, st, what);
-      if (plan.R == 1 && gemv_stage_activations(s.steps >= 32 ? 16 : s.M))
+      if (plan.R == 1 && stages(s.steps >= 32 ? 16 : s.M))
         return launch_fused_gemv_r<ACT, Provider, 1, true, false, 1, 1, true>(s, pargs, plan, cb_bytes, st, what);
       if (plan.R == 4) return launch_fused_gemv_r<ACT, Provider, 4, true>(s, pargs, plan, cb_bytes, st, what);
       if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, true>(s, pargs, plan, cb_bytes, st, what);
@@ -570,7 +638,7 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
   }
   if (plan.R == 4) return launch_fused_gemv_r<ACT, Provider, 4, false>(s, pargs, plan, 0, st, what);
   if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, false>(s, pargs, plan, 0, st, what);
-  if (gemv_stage_activations(s.M))
+  if (stages(s.M))
     return launch_fused_gemv_r<ACT, Provider, 1, false, false, 1, 1, true>(s, pargs, plan, 0, st, what);
   return launch_fused_gemv_r<ACT, Provider, 1, false>(s, pargs, plan, 0, st, what);
 }

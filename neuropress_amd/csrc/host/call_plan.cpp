@@ -242,7 +242,7 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   if (t.perm.defined() && t.perm.scalar_type() == at::kLong) {
     x = at::index_select(x_in, -1, t.perm);
     ldx = t.k;
-  } else if (t.perm.defined() || t.k_in != t.k) {
+  } else if (t.perm.defined() || (t.k_in != t.k && t.kind != kVqGemv && t.kind != kRvqGemv)) {
     sizes.back() = t.k;
     x = empty(sizes, x_in.scalar_type(), device);
     with_gather = t.kind == kVqDense && t.own;  // its decode gathers them too
@@ -301,6 +301,7 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   const void* xp = x.const_data_ptr();
   void* yp = y.data_ptr();
   const int M = (int)m, N = (int)t.n, K = (int)t.k;
+  const int x_columns = t.perm.defined() ? K : (int)t.k_in;  // the gather pads what it copies
   int rc = NPAMD_ERR_INVALID;
   switch (t.kind) {
     case kSliced:
@@ -313,8 +314,12 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
       }
       break;
     case kVqGemv:
-      rc = npamd_vq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
-                         ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
+      if (M > NPAMD_GEMV_MAX_M || x_columns != K)
+        rc = npamd_vq_gemv_blocks(xp, ldx, x_columns, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
+                                  ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
+      else
+        rc = npamd_vq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
+                           ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
       break;
     case kVqGemvPerm:
       rc = npamd_vq_gemv_perm(xp, ldx, ptr<I32>(a[9]), ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4],
@@ -329,9 +334,14 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
                                ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], ws, ws_bytes, st);
       break;
     case kRvqGemv:
-      rc = npamd_rvq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]), (int)a[7],
-                          ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12], ptr<F32>(a[13]), yp,
-                          t.n, M, N, K, (int)a[14], st);
+      if (M > NPAMD_GEMV_MAX_M || x_columns != K)
+        rc = npamd_rvq_gemv_blocks(xp, ldx, x_columns, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]),
+                                   (int)a[7], ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12],
+                                   ptr<F32>(a[13]), yp, t.n, M, N, K, (int)a[14], st);
+      else
+        rc = npamd_rvq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]), (int)a[7],
+                            ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12], ptr<F32>(a[13]), yp,
+                            t.n, M, N, K, (int)a[14], st);
       break;
     case kRvqTile:
       rc = npamd_rvq_gemm_tile(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]),
@@ -339,7 +349,7 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
                                ptr<F32>(a[13]), yp, t.n, M, N, K, (int)a[14], ws, ws_bytes, st);
       break;
     case kQGemv:
-      rc = npamd_q_gemv(xp, ldx, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), ptr<F32>(a[3]), yp, t.n, M, N, K,
+      rc = (M > NPAMD_GEMV_MAX_M ? npamd_q_gemv_blocks : npamd_q_gemv)(xp, ldx, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), ptr<F32>(a[3]), yp, t.n, M, N, K,
                         (int)a[6], (int)a[7], (int)a[8], st);
       break;
     case kQTile:

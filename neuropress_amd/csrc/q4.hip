@@ -712,17 +712,19 @@ static int q_dispatch(const QCall& c, bool gemv) {
   return launch_generic_gemm<ACT>(c.x, c.ldx, c.bias, c.y, c.ldy, c.M, c.N, c.K, e, c.st, c.what);
 }
 
-static int q_run(const QCall& c, bool gemv) {
+static int q_run(const QCall& c, bool gemv, bool any_m = false) {
   const int rc = validate_q(c.what, c.N, c.K, c.nbits, c.gs);
   if (rc) return rc;
   NPAMD_REQUIRE(c.act == NPAMD_F16 || c.act == NPAMD_BF16,
                 "%s: activations must be f16 or bf16 (got dtype code %d)", c.what, c.act);
   NPAMD_REQUIRE(c.M >= 0, "%s: negative M", c.what);
-  NPAMD_REQUIRE(!gemv || c.M <= NPAMD_GEMV_MAX_M, "%s: M=%d exceeds the fused limit %d", c.what, c.M,
+  NPAMD_REQUIRE(!gemv || any_m || c.M <= NPAMD_GEMV_MAX_M, "%s: M=%d exceeds the fused limit %d", c.what, c.M,
                 NPAMD_GEMV_MAX_M);
   NPAMD_REQUIRE(c.ldx >= c.K && c.ldy >= c.N, "%s: row stride smaller than the row", c.what);
   if (c.M == 0 || c.N == 0) return NPAMD_OK;
   NPAMD_REQUIRE(c.x && c.y && (c.K == 0 || (c.w_pack && c.scale)), "%s: null pointer", c.what);
+  if (any_m && (!q_fast_ok(c) || (c.M + kGemvTokens - 1) / kGemvTokens > 65535))
+    return fail(NPAMD_ERR_UNSUPPORTED, "%s: needs a shape and alignment of the MFMA kernels", c.what);
   return c.act == NPAMD_BF16 ? q_dispatch<NPAMD_BF16>(c, gemv) : q_dispatch<NPAMD_F16>(c, gemv);
 }
 
@@ -814,6 +816,15 @@ extern "C" int npamd_q_gemv(const void* x, int64_t ldx, const uint8_t* w_pack, c
   const QCall c{x, ldx, w_pack, scale_f16, zero_point_f16, bias, y, ldy, M, N, K, nbits, group_size,
                 act_dtype, (hipStream_t)stream, "npamd_q_gemv"};
   return q_run(c, true);
+}
+
+extern "C" int npamd_q_gemv_blocks(const void* x, int64_t ldx, const uint8_t* w_pack, const void* scale_f16,
+                                   const void* zero_point_f16, const float* bias, void* y, int64_t ldy,
+                                   int M, int N, int K, int nbits, int group_size, int act_dtype,
+                                   void* stream) {
+  const QCall c{x, ldx, w_pack, scale_f16, zero_point_f16, bias, y, ldy, M, N, K, nbits, group_size,
+                act_dtype, (hipStream_t)stream, "npamd_q_gemv_blocks"};
+  return q_run(c, true, true);
 }
 
 extern "C" int npamd_q_gemm_tile(const void* x, int64_t ldx, const uint8_t* w_pack,

@@ -51,7 +51,8 @@ struct QGemvLds {
 // XI: load instructions for a step's activations: up to 2 XI tokens.
 template <int ACT, int NBITS, bool ASYM, class Provider, int R, int XI>
 __global__ void __launch_bounds__(512)
-q_gemv_kernel(const GemvShape s, const typename Provider::Args a) {
+q_gemv_kernel(const GemvShape all, const typename Provider::Args a) {
+  const GemvShape s = gemv_token_block(all);
   using L = QGemvLds<NBITS, ASYM, R, XI>;
   constexpr int MT = XI > 8 ? 2 : 1;
   constexpr int kSlots = L::kRow / 16, kRowsPerLoad = 64 / kSlots, kCodeLoads = L::kCodes / 1024;
@@ -228,7 +229,7 @@ int launch_q_gemv_rx(GemvShape s, const typename Provider::Args& a, int blocks_p
   if (tuning().gemv_spw > 0) s.steps_per_wave = max(tuning().gemv_spw, (s.steps + L::kMaxWaves - 1) / L::kMaxWaves);
   const int waves = (s.steps + s.steps_per_wave - 1) / s.steps_per_wave;
   const int blocks = (s.N + 16 * R - 1) / (16 * R);
-  const int stage = waves * L::kWave, red = waves * s.M * 16 * R * 4;
+  const int stage = waves * L::kWave, red = waves * (s.M < kGemvTokens ? s.M : kGemvTokens) * 16 * R * 4;
   const int lds = stage > red ? stage : red;
   if (lds > 64 * 1024) {
     static LdsLatch latch;  // per instantiation
@@ -237,7 +238,7 @@ int launch_q_gemv_rx(GemvShape s, const typename Provider::Args& a, int blocks_p
     if (e != hipSuccess) return fail(NPAMD_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds, hipGetErrorString(e));
   }
   last_gemv_staged() = 1;
-  launch(q_gemv_kernel<ACT, NBITS, ASYM, Provider, R, XI>, blocks, waves * 64, lds, st, s, a);
+  launch(q_gemv_kernel<ACT, NBITS, ASYM, Provider, R, XI>, dim3(blocks, (s.M + kGemvTokens - 1) / kGemvTokens), waves * 64, lds, st, s, a);
   return check_launch(what);
 }
 
@@ -256,9 +257,20 @@ int launch_q_gemv_r(const GemvShape& s, const typename Provider::Args& a, int bl
 template <int ACT, int NBITS, bool ASYM, class Provider>
 int launch_q_gemv(GemvShape s, const typename Provider::Args& a, int cus, hipStream_t st, const char* what) {
   s.steps = (s.chunks + 3) / 4;
-  const int tiles = (s.N + 15) / 16, pairs = (tiles + 1) / 2;
+  const int token_blocks = (s.M + kGemvTokens - 1) / kGemvTokens;
+  const int tiles = (s.N + 15) / 16 * token_blocks, pairs = ((s.N + 15) / 16 + 1) / 2 * token_blocks;
   const int load1 = (tiles + cus - 1) / cus, load2 = (pairs + cus - 1) / cus;  // blocks of the fullest compute unit
   int R = s.M > 2 && s.steps >= 8 && load1 > 1 && 2 * load2 * 8 <= load1 * 9 ? 2 : 1;
+  // More than 32 tokens: a block's activations take 16 KiB of LDS per wave whatever its row tiles.  Two where that saves a round of
+  // blocks: int8 at 64 tokens, one / two, 4096 x 1024 6.9 / 5.4, 3072 x 3072 10.4 / 8.2; int4, two blocks of one tile to a compute unit,
+  // 3072 x 3072 at 96 11.1 / 14.8, 4096 x 1024 at 128 8.3 / 9.1, 2048 x 2048 at 256 11.6 / 12.1.
+  if (token_blocks > 1) {
+    const int waves = s.steps < 4 ? s.steps : 4;
+    const int fit1 = kGemvLdsPerBlockMax / (waves * QGemvLds<NBITS, ASYM, 1, 16>::kWave);
+    const int fit2 = kGemvLdsPerBlockMax / (waves * QGemvLds<NBITS, ASYM, 2, 16>::kWave);
+    const int rounds1 = (load1 + fit1 - 1) / fit1, rounds2 = (load2 + fit2 - 1) / fit2;
+    R = rounds2 < rounds1 || (R == 2 && rounds2 == rounds1) ? 2 : 1;
+  }
   if (tuning().gemv_r > 0) R = tuning().gemv_r > 1 ? 2 : 1;
   if (R == 2) return launch_q_gemv_r<ACT, NBITS, ASYM, Provider, 2>(s, a, load2, st, what);
   return launch_q_gemv_r<ACT, NBITS, ASYM, Provider, 1>(s, a, load1, st, what);

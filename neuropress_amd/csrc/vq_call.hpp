@@ -19,6 +19,7 @@ struct VqCall {
   const char* what;
   void* ws = nullptr;      // tile GEMM only: f32 scratch for split-K partial tiles (may stay null)
   int64_t ws_bytes = 0;
+  int k_in = 0;  // columns of x where the index rows are padded to K with filler rows (0: K)
   const int32_t* perm = nullptr;  // fused GEMV only: contract x[m, perm[k]] with W[n, k]
 };
 
@@ -34,7 +35,7 @@ inline int validate(const VqCall& c, int max_m) {
   NPAMD_REQUIRE(c.M >= 0 && c.N >= 0 && c.K >= 0, "%s: negative dimension", c.what);
   NPAMD_REQUIRE(max_m <= 0 || c.M <= max_m, "%s: M=%d exceeds the fused limit %d", c.what, c.M, max_m);
   NPAMD_REQUIRE(c.K % c.vl == 0, "%s: K=%d not divisible by VL=%d", c.what, c.K, c.vl);
-  NPAMD_REQUIRE(c.ldx >= c.K && c.ldy >= c.N, "%s: row stride smaller than the row", c.what);
+  NPAMD_REQUIRE(c.ldx >= (c.k_in ? c.k_in : c.K) && c.ldy >= c.N, "%s: row stride smaller than the row", c.what);
   const int64_t n_idx = (int64_t)c.N * (c.K / c.vl);
   NPAMD_REQUIRE((n_idx * c.bits + 7) / 8 <= c.n_bytes, "%s: packed buffer too short", c.what);
   if (c.packed_r) {

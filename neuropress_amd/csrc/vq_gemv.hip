@@ -5,18 +5,27 @@ using namespace npamd;
 
 namespace {
 
+// Past 16 tokens layers whose table LDS can hold stage their activations too, but do not stay ahead of the tile GEMM at any K, which is what
+// callers of npamd_gemv_stages_activations ask for: the answer is no.
+bool table_fits(int M, int table_bytes) { return M > 16 && table_bytes > 0 && table_bytes <= kGemvLdsCodebookMax; }
+int staged_answer(int rc, int M, int table_bytes) {
+  if (table_fits(M, table_bytes)) last_gemv_staged() = 0;
+  return rc;
+}
+
 template <int ACT, int BITS, int VL>
 int run_vq(const VqCall& c, const GemvShape& s) {
+  const int table = VL == 8 ? c.nc * 16 : c.nc % 2 == 0 ? c.nc * 8 : 0;
   if constexpr (ACT == NPAMD_BF16) {
     if (c.cb_dtype == NPAMD_F16) {
       using P = VqProvider<ACT, BITS, true, VL>;
       typename P::Args a{c.packed, (const u32x4*)c.cb, (uint32_t)c.nc - 1u, s.chunks};
-      return launch_fused_gemv<ACT, P>(s, a, c.st, c.what, (VL == 8 ? c.nc * 16 : (c.nc % 2 == 0 ? c.nc * 8 : 0)));
+      return staged_answer(launch_fused_gemv<ACT, P>(s, a, c.st, c.what, table), c.M, table);
     }
   }
   using P = VqProvider<ACT, BITS, false, VL>;
   typename P::Args a{c.packed, (const u32x4*)c.cb, (uint32_t)c.nc - 1u, s.chunks};
-  return launch_fused_gemv<ACT, P>(s, a, c.st, c.what, (VL == 8 ? c.nc * 16 : (c.nc % 2 == 0 ? c.nc * 8 : 0)));
+  return staged_answer(launch_fused_gemv<ACT, P>(s, a, c.st, c.what, table), c.M, table);
 }
 
 }  // namespace
@@ -28,7 +37,7 @@ int npamd::vq_gemv_plan_stages(int M, int N, int K, int nc) {
   using P = VqProvider<NPAMD_F16, 16, false, 8>;  // the choice depends on the table's size, not on the index width
   typename P::Args a{};
   launch_fused_gemv<NPAMD_F16, P>(s, a, nullptr, "plan", nc * 16);
-  return staged;
+  return table_fits(M, nc * 16) ? 0 : staged;
 }
 
 namespace {
@@ -60,6 +69,7 @@ int run_rvq(const VqCall& c, const GemvShape& s) {
 template <int ACT>
 int dispatch(const VqCall& c) {
   GemvShape s{c.x, c.ldx, c.bias, c.y, c.ldy, c.M, c.N, c.K / 64, 0, 0};
+  s.pieces = (c.k_in ? c.k_in : c.K) / 8;
   if (c.perm) {
     // The gather is done while x is copied to LDS, which only the MFMA kernel for plain VQ does.
     if (!(fast_ok(c) && !c.packed_r && c.M <= 16 && (int64_t)c.M * c.K <= kGemvLdsActivationsMax && aligned(c.perm, 16)))
@@ -77,6 +87,24 @@ int dispatch(const VqCall& c) {
     if (res_ok && c.bits == 8 && c.bits_r == 8) return run_rvq<ACT, 8, 8>(c, s);
   }
   return launch_generic_gemv<ACT>(c.x, c.ldx, c.bias, c.y, c.ldy, c.M, c.N, c.K, make_elem(c), c.st, c.what);
+}
+
+bool takes(const VqCall& c) {
+  const bool res_ok = !c.packed_r || (aligned(c.packed_r, 16) && aligned(c.cb_r, 16) &&
+                                      ((c.bits == 16 && (c.bits_r == 8 || c.bits_r == 16)) || (c.bits_r == 8 && (c.bits == 12 || c.bits == 8))));
+  return fast_ok(c) && res_ok;
+}
+
+// Any number of tokens, 32 to a block, and rows of x that end inside the last 64 columns; only what the MFMA kernel takes.
+int run_blocks(VqCall c, int k_in) {
+  NPAMD_REQUIRE(k_in > 0 && k_in % 8 == 0 && k_in <= c.K && c.K - k_in < 64, "%s: x of %d columns against index rows of %d", c.what, k_in, c.K);
+  c.k_in = k_in;
+  const int rc = validate(c, 0);
+  if (rc < 0) return rc;
+  if (rc == 1) return NPAMD_OK;
+  if (!takes(c) || (c.M + kGemvTokens - 1) / kGemvTokens > 65535)
+    return fail(NPAMD_ERR_UNSUPPORTED, "%s: needs a shape and alignment of the MFMA kernels", c.what);
+  return c.act == NPAMD_BF16 ? dispatch<NPAMD_BF16>(c) : dispatch<NPAMD_F16>(c);
 }
 
 int run(const VqCall& c) {
@@ -110,6 +138,16 @@ extern "C" int npamd_vq_gemv_perm(const void* x, int64_t ldx, const int32_t* col
   return run(c);
 }
 
+extern "C" int npamd_vq_gemv_blocks(const void* x, int64_t ldx, int k_in, const uint8_t* packed, int64_t n_bytes,
+                                    int bits, const void* codebook, int codebook_dtype, int nc, int vl,
+                                    const float* bias, void* y, int64_t ldy, int M, int N, int K,
+                                    int act_dtype, void* stream) {
+  VqCall c{x, ldx, packed, n_bytes, bits, codebook, codebook_dtype, nc, vl,
+               nullptr, 0, 0, nullptr, 0, nullptr, nullptr,
+               bias, y, ldy, M, N, K, act_dtype, (hipStream_t)stream, "npamd_vq_gemv_blocks"};
+  return run_blocks(c, k_in);
+}
+
 extern "C" int npamd_vq_fused_supported(int K, int vl, int bits) {
   const bool bits_ok = bits == 4 || bits == 8 || bits == 12 || bits == 16;
   return (vl == 8 || vl == 4) && bits_ok && K > 0 && K % 64 == 0 ? 1 : 0;
@@ -134,4 +172,18 @@ extern "C" int npamd_rvq_gemv(const void* x, int64_t ldx,
                packed_res, n_bytes_res, bits_res, cb_res_f16, nc_res, row_scale_f16, row_bias_f16,
                bias, y, ldy, M, N, K, act_dtype, (hipStream_t)stream, "npamd_rvq_gemv"};
   return run(c);
+}
+
+extern "C" int npamd_rvq_gemv_blocks(const void* x, int64_t ldx, int k_in,
+                                     const uint8_t* packed_main, int64_t n_bytes_main, int bits_main,
+                                     const uint8_t* packed_res, int64_t n_bytes_res, int bits_res,
+                                     const void* cb_main_f16, int nc_main, const void* cb_res_f16, int nc_res,
+                                     const void* row_scale_f16, const void* row_bias_f16, int vl,
+                                     const float* bias, void* y, int64_t ldy, int M, int N, int K,
+                                     int act_dtype, void* stream) {
+  if (!packed_res) return fail(NPAMD_ERR_INVALID, "npamd_rvq_gemv_blocks: residual stream is null");
+  VqCall c{x, ldx, packed_main, n_bytes_main, bits_main, cb_main_f16, NPAMD_F16, nc_main, vl,
+               packed_res, n_bytes_res, bits_res, cb_res_f16, nc_res, row_scale_f16, row_bias_f16,
+               bias, y, ldy, M, N, K, act_dtype, (hipStream_t)stream, "npamd_rvq_gemv_blocks"};
+  return run_blocks(c, k_in);
 }

@@ -98,6 +98,13 @@ def _rows(x: torch.Tensor) -> torch.Tensor:
     return x.contiguous().view(-1).view(x.shape)
 
 
+def _aligned_rows(x: torch.Tensor) -> torch.Tensor:
+    """2-D *x* with rows that start at 16-byte addresses, copied where they do not."""
+    if x.stride(0) % 8 or x.data_ptr() % 16:
+        x = torch.clone(x, memory_format=torch.contiguous_format)  # .contiguous() keeps dense rows at any address
+    return x
+
+
 def _tile_workspace(entry: str, m: int, n: int, k: int, device) -> tuple[int | None, int]:
     """Scratch for the tile GEMM's split-K (layers with few output features); (None, 0) for the
     other entry points and for shapes the library does not split.  Allocated per call from
@@ -187,9 +194,10 @@ def _vq_fused(
     out_features: int | None,
     bias: torch.Tensor | None,
     column_perm: torch.Tensor | None = None,
+    width: int | None = None,
 ) -> torch.Tensor:
     _check_device(entry, x, packed_indices, centroids, bias)
-    x = _x2d(x, entry)
+    x = _x2d(x, entry) if width is None else _aligned_rows(_x2d(x, entry))
     if x.dtype not in (torch.float16, torch.bfloat16):
         raise RuntimeError(f"{entry}: x must be float16 or bfloat16, got {x.dtype}")
     packed = _packed_u8(packed_indices, entry)
@@ -197,6 +205,8 @@ def _vq_fused(
     if cb.dtype not in (torch.float16, x.dtype):
         raise RuntimeError(f"{entry}: centroids must be float16 or x's dtype")
     m, k = x.shape
+    perm = () if width is None else (k,)
+    k = width or k
     vl = cb.shape[1]
     if k % vl:
         raise RuntimeError(f"{entry}: K={k} not divisible by VL={vl}")
@@ -211,7 +221,6 @@ def _vq_fused(
     b32 = _bias_f32(bias)
     ws, ws_bytes = _tile_workspace(entry, m, out_features, k, x.device)
     extra = (_ptr(ws), ws_bytes) if entry.endswith("_gemm_tile") else ()
-    perm = ()
     if column_perm is not None:
         if column_perm.dtype != torch.int32 or column_perm.numel() != k or not column_perm.is_contiguous():
             raise RuntimeError(f"{entry}: column_perm must be a contiguous int32 tensor of K={k} entries")
@@ -248,6 +257,20 @@ def vq_linear(
         return _vq_fused("npamd_vq_gemv_perm", x, packed_indices, centroids, bits, out_features, bias,
                          column_perm)  # fmt: skip
     return _vq_fused("npamd_vq_gemv", x, packed_indices, centroids, bits, out_features, bias)
+
+
+def vq_linear_blocks(x: torch.Tensor, packed_indices: torch.Tensor, centroids: torch.Tensor, bits: int, out_features: int,
+                     bias: torch.Tensor | None = None, *, width: int) -> torch.Tensor:  # fmt: skip
+    """The fused GEMV for any number of tokens, 32 to a workgroup (``npamd_vq_gemv_blocks``), where :func:`gemv_blocks_preferred` says so.
+    *width*: columns of the index rows, a multiple of 64, of which *x* may lack up to 56 (multiples of 8)."""
+    return _vq_fused("npamd_vq_gemv_blocks", x, packed_indices, centroids, bits, out_features, bias, width=int(width))
+
+
+def gemv_blocks_preferred(m: int, n: int, k: int, kind: int, table_rows: int = 0, gathered: bool = False) -> bool:
+    """Whether the GEMV with a workgroup per 32 tokens is the better choice for more than 16 of them (``npamd_gemv_blocks_preferred``):
+    *kind* 0 for a VQ layer with a codebook of *table_rows* rows of eight, 1 for a residual one, else bits per weight; *gathered*: the columns of x
+    are gathered first, which decode + product do along with the decode."""
+    return bool(_lib.load().npamd_gemv_blocks_preferred(int(m), int(n), int(k), int(kind), int(table_rows), int(gathered)))
 
 
 def vq_linear_perm_supported(m: int, n: int, k: int, num_centroids: int, vector_len: int, bits: int) -> bool:
@@ -647,11 +670,15 @@ def vq_gemm_tile(
     bits: int,
     out_features: int,
     bias: torch.Tensor | None = None,
+    width: int | None = None,
 ) -> torch.Tensor:
     """``x @ W.T (+ bias)`` with W decoded tile by tile inside an MFMA GEMM.
 
-    Signature of the reference's ``vq_gemm_triton`` (neuropress/kernels/vq_triton.py:119-126).
+    Signature of the reference's ``vq_gemm_triton`` (neuropress/kernels/vq_triton.py:119-126), and *width*: the kernel of
+    :func:`vq_linear_blocks` instead, where :func:`gemv_blocks_preferred` says so.
     """
+    if width is not None:
+        return vq_linear_blocks(x, packed_indices, centroids, bits, out_features, bias, width=width)
     return _vq_fused("npamd_vq_gemm_tile", x, packed_indices, centroids, bits, out_features, bias)
 
 
@@ -743,8 +770,10 @@ def rvq_linear(
     out_features: int,
     bias: torch.Tensor | None = None,
     tile: bool | None = None,
+    width: int | None = None,
 ) -> torch.Tensor:
-    """Fused residual-VQ linear; ``tile=None`` picks GEMV for ``M <= 32`` else the tile GEMM."""
+    """Fused residual-VQ linear; ``tile=None`` picks GEMV for ``M <= 32`` else the tile GEMM.  *width*: any number of tokens through
+    the GEMV, index rows of that many columns (see :func:`vq_linear_blocks`)."""
     what = "rvq_linear"
     _check_device(what, x, packed_main, packed_res, centroids_main, centroids_res)
     x = _x2d(x, what)
@@ -761,11 +790,14 @@ def rvq_linear(
     y = torch.empty((m, out_features), device=x.device, dtype=x.dtype)
     b32 = _bias_f32(bias)
     entry = "npamd_rvq_gemm_tile" if tile else "npamd_rvq_gemv"
+    columns = ()
+    if width is not None:
+        entry, tile, x, columns, k = "npamd_rvq_gemv_blocks", False, _aligned_rows(x), (k,), int(width)
     ws, ws_bytes = _tile_workspace(entry, m, out_features, k, x.device)
     extra = (_ptr(ws), ws_bytes) if tile else ()
     _lib.call(
         entry,
-        x.data_ptr(), x.stride(0), pm.data_ptr(), pm.numel(), int(bits_main), pr.data_ptr(),
+        x.data_ptr(), x.stride(0), *columns, pm.data_ptr(), pm.numel(), int(bits_main), pr.data_ptr(),
         pr.numel(), int(bits_res), cm.data_ptr(), cm.shape[0], cr.data_ptr(), cr.shape[0],
         _ptr(sc), _ptr(rb), cm.shape[1], _ptr(b32), y.data_ptr(), y.stride(0), m, out_features, k,
         _DT[x.dtype], *extra, _stream(x),
@@ -829,6 +861,8 @@ def _q_fused(entry, x, w_pack, scale, nbits, group_size, zero_point, bias):
         raise RuntimeError(f"{entry}: x has K={x.shape[-1]}, the packed weight has K={k}")
     lead = x.shape[:-1]
     x2 = _x2d(x.reshape(-1, k), entry)
+    if entry.endswith("_blocks"):
+        x2 = _aligned_rows(x2)
     m = x2.shape[0]
     y = torch.empty((m, n), device=x.device, dtype=x.dtype)
     b32 = _bias_f32(bias)
@@ -859,9 +893,14 @@ def q_linear(
     return _q_fused(entry, x, w_pack, scale, nbits, group_size, zero_point, bias)
 
 
-def q_gemm_tile(x, w_pack, scale, nbits, group_size, zero_point=None, bias=None) -> torch.Tensor:
-    """Fused dequant MFMA GEMM at any M."""
-    return _q_fused("npamd_q_gemm_tile", x, w_pack, scale, nbits, group_size, zero_point, bias)
+def q_linear_blocks(x, w_pack, scale, nbits, group_size, zero_point=None, bias=None) -> torch.Tensor:
+    """The fused GEMV for any number of tokens, 4 or 8 bits (``npamd_q_gemv_blocks``), where :func:`gemv_blocks_preferred` says so."""
+    return _q_fused("npamd_q_gemv_blocks", x, w_pack, scale, nbits, group_size, zero_point, bias)
+
+
+def q_gemm_tile(x, w_pack, scale, nbits, group_size, zero_point=None, bias=None, blocks=False) -> torch.Tensor:
+    """Fused dequant MFMA GEMM at any M; *blocks*: the kernel of :func:`q_linear_blocks` instead."""
+    return _q_fused("npamd_q_gemv_blocks" if blocks else "npamd_q_gemm_tile", x, w_pack, scale, nbits, group_size, zero_point, bias)
 
 
 # ---------------------------------------------------------------------------
@@ -1043,6 +1082,7 @@ def q_embedding(
 # plans step aside, so that the replacement is called.
 WRAPPERS = {
     fn.__name__: fn
-    for fn in (vq_linear_sliced_checked, vq_linear, vq_gemm_tile, vq_slice_gemm, vq_dequant, rvq_linear, rvq_dequant, q_linear, q_gemm_tile,
+    for fn in (vq_linear_sliced_checked, vq_linear, vq_linear_blocks, vq_gemm_tile, vq_slice_gemm, vq_dequant, rvq_linear, rvq_dequant, q_linear,
+               q_linear_blocks, q_gemm_tile,
                q_dequant, rms_norm, vq_embedding, q_embedding, dense_linear, gather_columns)
 }  # fmt: skip

@@ -27,6 +27,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import _lib
 from ..qweights import ScalarQScheme, ScalarQWeight, is_scalar_qweight
 from ..t2n.packing import BitPacking
 from .backends import Backend, LinearBackend, is_hip_backend_available, tensor_version, tile_band_ok
@@ -37,6 +38,8 @@ log = logging.getLogger(__name__)
 # Measured on one MI355X (14336 x 4096, group 32): fused GEMM 35-40 us up to 128
 # tokens and 56 us at 256 against 56-64 / 80 us for decode + GEMM; 83-84 vs 78-84 us at
 # 320-384, 158 vs 93 us at 512.
+# Most tokens of the GEMV with a workgroup per 32 tokens, which serves small layers past the GEMV's own (kernels.gemv_blocks_preferred).
+_Q_BLOCKS_MAX_TOKENS: int = int(os.environ.get("NEUROPRESS_Q_BLOCKS_MAX_TOKENS", "65536"))
 _Q_TILE_MAX_TOKENS: int = int(os.environ.get("NEUROPRESS_Q_TILE_MAX_TOKENS", "256"))
 # Long reductions (K >= _Q_TILE_SPLIT_LONG_K), where the dense GEMM is slow, keep the fused
 # GEMM up to this many tokens: 4096 x 14336 80 vs 105-109 us at 320-384, 148 vs 120 us at 512.
@@ -165,7 +168,7 @@ def _q_dequant_linear(
 _PLAN_ATTRIBUTES = ("backend", "out_features", "in_features", "group_size", "nbits", "zero_point", "bias")
 _PLAN_THRESHOLDS = ("_Q_TILE_MAX_TOKENS", "_Q_TILE_LONG_K_MAX_TOKENS", "_Q_TILE_WIDE_MAX_TOKENS", "_Q_TILE_WIDE_MIN_FEATURES",
                     "_Q_TILE_MIN_GRID_FRACTION", "_Q_TILE_SPLIT_MAX_TOKENS", "_Q_TILE_SPLIT_LONG_K", "_Q_TILE_HALF_GRID_K",
-                    "_Q_FUSED_MAX_TOKENS",
+                    "_Q_FUSED_MAX_TOKENS", "_Q_BLOCKS_MAX_TOKENS",
                     "_Q_FUSED_WIDE_MAX_TOKENS", "_Q_FUSED_WIDE_MAX_ACTIVATIONS", "_Q_FUSED_WIDE_INT8_MAX_K")  # fmt: skip
 
 
@@ -389,8 +392,9 @@ class NPLinear(nn.Module):
                 if y is not None:
                     return y
             if band != "dense":
-                fn = kernels.q_linear if band == "fused" else kernels.q_gemm_tile
-                return fn(x, self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point, self._bias_f32())
+                fn = {"fused": kernels.q_linear, "blocks": kernels.q_linear_blocks}.get(band, kernels.q_gemm_tile)
+                more = {"blocks": True} if band == "tile" and not tracked and self._blocks_win(m) else {}
+                return fn(x, self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point, self._bias_f32(), **more)
             w = kernels.q_dequant(
                 self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point, x.dtype
             )
@@ -410,7 +414,7 @@ class NPLinear(nn.Module):
         return dtype in (torch.float16, torch.bfloat16) and kernels.dense_preferred(m, self.out_features, self.in_features)
 
     def _band(self, x: torch.Tensor, m: int, tracked: bool = False) -> str:
-        """Which kernel serves a call of *m* tokens: ``fused`` (GEMV), ``tile`` (fused GEMM) or ``dense`` (decode + GEMM).
+        """Which kernel serves a call of *m* tokens: ``fused`` (GEMV), ``blocks`` (GEMV, a workgroup per 32 tokens), ``tile`` (fused GEMM) or ``dense`` (decode + GEMM).
         *tracked* (``kernels.tracked(x)``): the dense product is the library's, and so are the limits against it."""
         # Layers the MFMA kernels do not take (1 / 2 / 8 bits, odd group sizes) would run an
         # element-wise kernel, slower at every token count than decoding once and calling the
@@ -424,7 +428,21 @@ class NPLinear(nn.Module):
             limit = max(limit, _Q_TILE_LONG_K_MAX_TOKENS)
         if limit > 0 and max(self.in_features, self.out_features) >= _Q_TILE_WIDE_MIN_FEATURES:
             limit = max(limit, _Q_TILE_WIDE_MAX_TOKENS)
-        return "tile" if m <= limit and self._tile_grid_fills_gpu(x, m, tracked) else "dense"
+        if m <= limit and self._tile_grid_fills_gpu(x, m, tracked):
+            return "tile"
+        return "blocks" if not tracked and self._blocks_win(m) else "dense"
+
+    def _blocks_win(self, m: int) -> bool:
+        """Whether the GEMV with a workgroup per 32 tokens is ahead of the fused GEMM and of decode + GEMM (NPVQLinear._blocks_win)."""
+        from .. import kernels
+
+        if not 16 < m <= _Q_BLOCKS_MAX_TOKENS or self.out_features < 256 or min(_Q_FUSED_MAX_TOKENS, _Q_TILE_MAX_TOKENS) <= 0:
+            return False
+
+        lines, _ = kernels.q_gemv_staging(
+            _lib.GEMV_MAX_M, self.out_features, self.in_features, self.nbits, self.group_size, self.scale, self.zero_point
+        )
+        return lines and kernels.gemv_blocks_preferred(m, self.out_features, self.in_features, self.nbits)
 
     def _planned(self, x: torch.Tensor, m: int, band: str):
         """Add this call to the layer's plan and let the plan issue it; None where it cannot."""
@@ -445,11 +463,13 @@ class NPLinear(nn.Module):
             if plan is None:
                 return None
         code = plans.DTYPE_CODES[x.dtype]
+        if band == "tile" and self._blocks_win(m):
+            band = "blocks"
         if band == "dense" and self._own_product(m, x.dtype):
             band = "product"
         number = plan.names.get((band, x.dtype))
         if number is None:
-            kind = {"fused": plans.Q_GEMV, "tile": plans.Q_TILE}.get(band, plans.Q_DENSE)
+            kind = {"fused": plans.Q_GEMV, "blocks": plans.Q_GEMV, "tile": plans.Q_TILE}.get(band, plans.Q_DENSE)
             args = (self.u8_blob, self.scale, self.zero_point, self._bias_f32(), 0, 0, self.nbits, self.group_size, code)
             bias = self._bias_as(x.dtype) if band == "dense" else self._bias_f32() if band == "product" else None
             number = plan.names[band, x.dtype] = plans.template(plan, kind, n, k, args, x.dtype, bias=bias, leaf=self.bias, own=band == "product")

@@ -123,6 +123,8 @@ _PREPARE_ON_MOVE: bool = _env_int(("NEUROPRESS_VQ_PREPARE_ON_MOVE",), 1) != 0
 # cuda_lut layers: 0 = always decode + GEMM, the reference's default routing.
 _LUT_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_LUT_MAX_TOKENS",), 0)
 
+# Most tokens of the GEMV with a workgroup per 32 tokens, which serves small layers past 16 of them (kernels.gemv_blocks_preferred).
+_BLOCKS_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_BLOCKS_MAX_TOKENS",), 1 << 16)
 # Upper end of the tile-decode GEMM band.  NEUROPRESS_VQ_TRITON_MAX_TOKENS is the
 # reference's name for the same knob and is honoured too.  0 disables the band.
 # Measured on one MI355X (14336 x 4096 layer): the tile GEMM beats decode + GEMM
@@ -201,7 +203,7 @@ _FUSED_BACKENDS = frozenset({VQBackend.CUDA_WMMA, VQBackend.CUDA_LUT, VQBackend.
 _PLAN_ATTRIBUTES = ("backend", "proxy", "residual_proxy", "out_features", "in_features", "vector_len", "bits", "residual_bits",
                     "bias", "column_perm", "packed_residual", "row_scale", "row_bias")  # fmt: skip
 _PLAN_THRESHOLDS = ("_FUSED_MAX_TOKENS", "_FUSED_WIDE_MAX_TOKENS", "_FUSED_WIDE_MAX_ACTIVATIONS", "_SLICED_MAX_TOKENS",
-                    "_SLICED_MIN_CENTROIDS", "_SLICED_MIN_INDICES", "_SLICE_GEMM_MAX_TOKENS", "_SLICE_GEMM_GATHER_US", "_LUT_MAX_TOKENS", "_TILE_MAX_TOKENS", "_TILE_WIDE_MAX_TOKENS",
+                    "_SLICED_MIN_CENTROIDS", "_SLICED_MIN_INDICES", "_SLICE_GEMM_MAX_TOKENS", "_SLICE_GEMM_GATHER_US", "_LUT_MAX_TOKENS", "_BLOCKS_MAX_TOKENS", "_TILE_MAX_TOKENS", "_TILE_WIDE_MAX_TOKENS",
                     "_TILE_WIDE_MIN_WEIGHTS", "_TILE_WIDE_BROAD_WEIGHTS", "_TILE_WIDE_BROAD_FEATURES",
                     "_TILE_WIDE_TINY_WEIGHTS", "_TILE_WIDE_MID_MAX_TOKENS",
                     "_TILE_WIDE_LONG_MAX_TOKENS", "_TILE_WIDE_SMALL_MAX_TOKENS", "_TILE_SMALL_LAYER_MAX_TOKENS",
@@ -780,6 +782,8 @@ class NPVQLinear(nn.Module):
             return self._forward_tile_gemm(x)
         if band == "slice":
             return self._forward_slice_gemm(x)
+        if band == "blocks":
+            return self._fused(x, tile=False, blocks=True)
         if self.backend == VQBackend.CUDA_LUT:
             return self._forward_cuda_lut(x)
         if self.backend == VQBackend.CUDA_WMMA or self.backend in _CODED_BACKENDS:
@@ -792,7 +796,7 @@ class NPVQLinear(nn.Module):
 
     def _band(self, x: torch.Tensor, m: int, tracked: bool = False) -> str:
         """Which kernel serves a call of *m* tokens: ``sliced``, ``gemv_perm`` (the GEMV that gathers x's columns),
-        ``fused`` (the backend's GEMV), ``slice`` (the slice GEMM), ``tile``, ``dense`` (decode + GEMM) or ``torch``.
+        ``fused`` (the backend's GEMV), ``blocks`` (it with a workgroup per 32 tokens), ``slice`` (the slice GEMM), ``tile``, ``dense`` (decode + GEMM) or ``torch``.
 
         *tracked* (``kernels.tracked(x)``): the dense product is the library's, columns are gathered by torch and none
         are padded; the limits are those against that.  What it serves carries gradients, the other kernels do not."""
@@ -815,7 +819,7 @@ class NPVQLinear(nn.Module):
         if m > self._gemv_max_tokens(m):
             if self.backend != VQBackend.CUDA_LUT and m <= self._tile_max_tokens(tracked) and self._tile_band_ok(x, m, tracked):
                 return "tile"
-            return "dense"
+            return "blocks" if x.is_cuda and not tracked and self._blocks_win(m) else "dense"
         return "fused"
 
     # -- call plan ---------------------------------------------------------
@@ -870,6 +874,8 @@ class NPVQLinear(nn.Module):
         from ..kernels import plans
 
         tile = band == "tile" or (band == "fused" and m > _GEMV_KERNEL_MAX_TOKENS)
+        if band == "tile" and self._blocks_win(m):
+            tile, band = False, "blocks"
         kind = "tile" if tile else "product" if band == "dense" and self._own_product(m, dtype) else band
         number = plan.names.get((kind, dtype))
         if number is None:
@@ -913,7 +919,8 @@ class NPVQLinear(nn.Module):
                 bias = self._bias_f32() if own else self._bias_as(dtype)
                 return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=bias, leaf=self.bias, own=own)
             kind_code = plans.RVQ_TILE if kind == "tile" else plans.RVQ_GEMV
-            return plans.template(plan, kind_code, n, k, (*args, self._bias_f32(), code), dtype, perm=perm)
+            leaf = self.bias if kind == "blocks" else None  # in the place of the dense product
+            return plans.template(plan, kind_code, n, k, (*args, self._bias_f32(), code), dtype, perm=perm, leaf=leaf)
         stream, bits = self._kernel_stream()
         stream = stream.reshape(-1)
         if kind in ("dense", "product"):
@@ -928,7 +935,8 @@ class NPVQLinear(nn.Module):
         if kind == "gemv_perm":
             return plans.template(plan, plans.VQ_GEMV_PERM, n, k, (*args, self._perm_i32(stream.device)), dtype)
         kind_code = {"tile": plans.VQ_TILE, "slice": plans.VQ_SLICE}.get(kind, plans.VQ_GEMV)
-        return plans.template(plan, kind_code, n, self._kernel_k(), args, dtype, k_in=k, perm=perm)
+        leaf = self.bias if kind == "blocks" else None  # in the place of the dense product
+        return plans.template(plan, kind_code, n, self._kernel_k(), args, dtype, k_in=k, perm=perm, leaf=leaf)
 
     # -- slice-list GEMV ---------------------------------------------------
 
@@ -1133,6 +1141,21 @@ class NPVQLinear(nn.Module):
             if self._gemv_stages_activations(m) and not self._tile_ahead_from_17():
                 return 32
         return limit
+
+    def _blocks_win(self, m: int) -> bool:
+        """Whether the GEMV with a workgroup per 32 tokens is ahead of the tile GEMM and of decode + GEMM.  It takes their place on
+        layers of 256 output features and more: what smaller ones do, heads and probes, they do through the products
+        that callers put their own in the place of."""
+        if not 16 < m <= _BLOCKS_MAX_TOKENS or self.out_features < 256 or min(_FUSED_MAX_TOKENS, _TILE_MAX_TOKENS) <= 0 or self.backend == VQBackend.CUDA_LUT:
+            return False
+        if self.vector_len != 8 or self.proxy.centroids.dtype != torch.float16 or not self._mfma_layer() or (
+            self.is_residual and (self.bits, self._res_bits()) not in ((16, 8), (16, 16), (12, 8), (8, 8))
+        ):  # fmt: skip
+            return False
+        from .. import kernels
+
+        return kernels.gemv_blocks_preferred(m, self.out_features, self._kernel_k(), int(self.is_residual), self.proxy.num_centroids,
+                                             self.column_perm is not None)  # fmt: skip
 
     def _tile_ahead_from_17(self) -> bool:
         """Large layers with at least twice as many output as input features and a codebook kept in memory: the
@@ -1390,22 +1413,26 @@ class NPVQLinear(nn.Module):
             "zero_cb", self.packed_indices, lambda: torch.zeros((1, self.vector_len), dtype=torch.float16, device=dev)
         )
 
-    def _fused(self, x: torch.Tensor, tile: bool, perm: torch.Tensor | None = None) -> torch.Tensor:
+    def _fused(self, x: torch.Tensor, tile: bool, perm: torch.Tensor | None = None, blocks: bool = False) -> torch.Tensor:
         from .. import kernels
 
         *leading, _ = x.shape
         x2d = x.reshape(-1, self.in_features)
+        width = self._kernel_k() if blocks or (tile and self._blocks_win(x2d.shape[0])) else None
         if self.is_residual:
             y = kernels.rvq_linear(
                 x2d, self.packed_indices, self.bits, self._res_stream(), self._res_bits(),
                 self.proxy.centroids, self._res_centroids(), self.row_scale, self.row_bias,
-                self.out_features, self._bias_f32(), tile=tile,
+                self.out_features, self._bias_f32(), tile=tile, width=width,
             )  # fmt: skip
         else:
             stream, bits = self._kernel_stream()
+            cb = self.proxy.centroids_as(x.dtype)
+            if width is not None:
+                fn = kernels.vq_gemm_tile if tile else kernels.vq_linear_blocks
+                return fn(x2d, stream, cb, bits, self.out_features, self._bias_f32(), width=width).reshape(*leading, self.out_features)
             if self._kernel_k() != self.in_features:
                 x2d = kernels.gather_columns(x2d, None, self._kernel_k())
-            cb = self.proxy.centroids_as(x.dtype)
             fn = kernels.vq_gemm_tile if tile else kernels.vq_linear
             if tile:
                 y = fn(x2d, stream, cb, bits, self.out_features, self._bias_f32())

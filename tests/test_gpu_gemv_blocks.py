@@ -1,0 +1,134 @@
+"""The fused GEMVs with a workgroup per 32 tokens: token counts around the blocks' edges, tables in LDS (one and two row tiles, large and
+small) and in memory, K of one chunk up to several steps per wave, rows of x that end inside the last chunk, rows at a
+stride; against the decoded weight in float64.  And the calls that lowered layers send there."""
+
+import pytest
+import torch
+
+import neuropress_amd.nn.np_linear as qmod
+import neuropress_amd.nn.np_vq_linear as vqmod
+from neuropress_amd.nn import NPLinear, NPVQLinear, VQProxy
+from neuropress_amd.transforms.vq_packing import IndexPacking
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+TOKENS = (17, 32, 33, 63, 64, 65, 130)
+
+
+def _check(y, x, w, bias=None):
+    """One rounding of the output, and f32 sums of K products in some order."""
+    x, w = x.double(), w.double()
+    ref, size = x @ w.T, x.abs() @ w.abs().T
+    if bias is not None:
+        ref, size = ref + bias.double(), size + bias.double().abs()
+    bound = ref.abs() * (2.0**-10 if y.dtype == torch.float16 else 2.0**-7) + size * w.shape[1] * 2.0**-24 + 2.0**-24
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+def _rows(m, k, act, gpu, g):
+    return torch.randn(m, k + 24, generator=g).to(act).to(gpu)[:, :k]
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("nc,bits", [(16, 4), (256, 8), (1000, 16), (4096, 12), (65536, 16)])
+def test_vq(gpu, nc, bits, act):
+    from neuropress_amd import kernels
+
+    g = cases.gen(nc)
+    cb = (torch.randn(nc, 8, generator=g) * 0.05).to(act).to(gpu)
+    for n, k, short in ((259, 64, 0), (256, 2112, 8), (1030, 1088, 56), (2064, 2048, 0), (300, 4224, 24), (4112, 576, 40)):
+        idx = torch.randint(0, nc, (n, k // 8), generator=g)
+        packed = IndexPacking.pack(idx.reshape(-1), bits).to(gpu)
+        w = cb[idx.to(gpu)].reshape(n, k)[:, : k - short]
+        bias = torch.randn(n, generator=g).to(gpu)
+        for m in TOKENS + ((1, 3, 9, 16, 300) if short else (300,)):
+            x = _rows(m, k - short, act, gpu, g)
+            _check(kernels.vq_linear_blocks(x, packed, cb, bits, n, bias, width=k), x, w, bias)
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("nc,ncr", [(65536, 256), (4096, 256), (65536, 65536)])
+def test_residual(gpu, nc, ncr, act):
+    from neuropress_amd import kernels
+
+    for n, k, short in ((259, 64, 0), (256, 2112, 8), (1030, 1088, 56), (2064, 2048, 0), (6000, 576, 16)):
+        L = cases.rvq_layer(n, n, k, nc, ncr, zipf=False)
+        pm, pr, cm, cr, sc, rb = (L[name].to(gpu) for name in ("pm", "pr", "cbm", "cbr", "scale", "wbias"))
+        w = kernels.rvq_dequant(pm, L["bm"], pr, L["br"], cm, cr, sc, rb, n, k, act)[:, : k - short]
+        g = cases.gen(n)
+        for m in TOKENS + ((1, 2, 5, 16) if short else ()):
+            x = _rows(m, k - short, act, gpu, g)
+            _check(kernels.rvq_linear(x, pm, L["bm"], pr, L["br"], cm, cr, sc, rb, n, width=k), x, w)
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits,zero_point", [(4, False), (4, True), (8, False), (8, True)])
+def test_group_quantized(gpu, bits, zero_point, act):
+    from neuropress_amd import kernels
+
+    for n, k, group in ((258, 64, 32), (256, 2112, 64), (1030, 1024, 128), (2064, 512, 32), (4112, 320, 64), (257, 192, 64)):
+        L = cases.q4_layer(n + k, n, k, nbits=bits, gs=group, asym=zero_point)
+        blob, sc, zp = (None if L[name] is None else L[name].to(gpu) for name in ("blob", "scale", "zp"))
+        w = kernels.q_dequant(blob, sc, bits, group, zp, act)
+        g = cases.gen(n)
+        for m in TOKENS + (300,):
+            x = _rows(m, k, act, gpu, g)
+            _check(kernels.q_linear_blocks(x, blob, sc, bits, group, zp), x, w)
+
+
+def test_what_the_entries_refuse(gpu):
+    from neuropress_amd import kernels
+
+    cb = torch.zeros(256, 8, dtype=torch.half, device=gpu)
+    packed = torch.zeros(256 * 16, dtype=torch.uint8, device=gpu)
+    x = torch.zeros(40, 128, dtype=torch.half, device=gpu)
+    for columns, width in ((64, 128), (124, 128), (128, 120)):  # a whole chunk missing, no whole piece, no whole chunk
+        with pytest.raises(RuntimeError):
+            kernels.vq_linear_blocks(x[:, :columns].contiguous(), packed, cb, 8, 256, width=width)
+    with pytest.raises(RuntimeError):
+        kernels.vq_linear(x, packed, cb, 8, 8, None, 256)  # more than 32 tokens
+
+
+def _layers(gpu, n, k, perm):
+    L = cases.vq_layer(n + k, n, k, 1000, bias=True)
+    cp = torch.randperm(k, generator=cases.gen(k)) if perm else None
+    yield vqmod, "_BLOCKS_MAX_TOKENS", lambda: NPVQLinear(
+        VQProxy(L["cb"]).to(gpu), L["packed"], L["bits"], n, k, 8, "cuda_wmma", bias=L["bias"].float(), column_perm=cp).to(gpu)  # fmt: skip
+    if not perm:
+        Q = cases.q4_layer(n + k, n, k, bias=True)
+        yield qmod, "_Q_BLOCKS_MAX_TOKENS", lambda: NPLinear(
+            Q["blob"], Q["scale"], n, k, 32, 4, "sym", "cuda", bias=Q["bias"].float()).to(gpu)  # fmt: skip
+        R = cases.rvq_layer(n + k, n, k)
+        yield vqmod, "_BLOCKS_MAX_TOKENS", lambda: NPVQLinear(
+            VQProxy(R["cbm"]).to(gpu), R["pm"], R["bm"], n, k, 8, "cuda_wmma", residual_proxy=VQProxy(R["cbr"]).to(gpu),
+            packed_residual=R["pr"], residual_bits=R["br"], row_scale=R["scale"], row_bias=R["wbias"]).to(gpu)  # fmt: skip
+
+
+@pytest.mark.parametrize("perm", [False, True])
+def test_layers_against_the_other_bands(gpu, perm, monkeypatch):
+    """Layers that take the blocks, on the first call, the planned one, with rows at odd addresses and under capture, against the same
+    layers without them; a bias that asks for a gradient keeps it."""
+    for module, name, make in _layers(gpu, 512, 2048, perm):
+        layer = make()
+        for m in (40, 100):
+            base = torch.randn(m, 2048 + 3, generator=cases.gen(m)).half().to(gpu)
+            x = base[:, :2048].contiguous()
+            assert layer._blocks_win(m) and layer._band(x, m) in ("blocks", "tile") and layer._band(x, m, True) != "blocks"
+            first, again, strided = layer(x), layer(x), layer(base[:, :2048])
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                captured = layer(x)
+            for _ in range(3):
+                captured.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(captured, first)
+            assert torch.equal(first, again) and torch.equal(first, strided)
+            with monkeypatch.context() as mp:
+                mp.setattr(module, name, 0)
+                assert layer._band(x, m) not in ("blocks", "fused")
+                other = layer(x)
+            assert torch.allclose(first.float(), other.float(), rtol=2e-3, atol=2e-3)  # two orders of the same f32 sums, each rounded once
+        if getattr(layer, "bias", None) is not None and layer._band(x, m) == "blocks":
+            layer.bias.requires_grad_()
+            assert layer(x).requires_grad
