@@ -476,6 +476,10 @@ int npamd_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* 
 int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
                      int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same for K a multiple of 8.  Workspace: as npamd_dense_gemm_workspace_bytes says for K rounded up to 64. */
+int npamd_dense_gemm_ragged(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
+                            int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Bytes of workspace npamd_dense_gemm can use for this shape (0: none).  Host-only arithmetic. */
 int64_t npamd_dense_gemm_workspace_bytes(int M, int N, int K);
 

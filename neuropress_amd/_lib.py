@@ -68,6 +68,7 @@ SIGNATURES: dict[str, list] = {
     "npamd_q_embedding": [_vp, _i64, _vp, _vp, _vp, _int, _int, _i64, _int, _i64, ctypes.c_float, _vp, _int, _vp],
     "npamd_q_gemm_tile": _Q_LINEAR[:-1] + _WS + [_vp],
     "npamd_dense_gemm": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _int, _int, _int, _int, _vp, _i64, _vp],
+    "npamd_dense_gemm_ragged": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _int, _int, _int, _int, _vp, _i64, _vp],
     "npamd_dense_gemm_workspace_bytes": [_int, _int, _int],
     "npamd_dense_gemm_preferred": [_int, _int, _int],
     "npamd_gemv_blocks_preferred": [_int] * 6,

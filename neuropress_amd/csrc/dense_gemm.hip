@@ -18,6 +18,8 @@
 // computes 32 MT x 64 of the tile (MFMA 32x32x16), reading the operands of a k group while it multiplies the one
 // before.  At 384 x 4096 x 4096 (21 us) the matrix pipes are busy 40 % of the time of the 192 compute units in use and
 // LDS 32 %; the waves wait 42 % of theirs, for 14 TB/s of lines from the L2s at 389 cycles each, and for each other.
+// Rows that end inside a step (SHORT) are read where they lie: residual VQ 1157 x 272 at 471 tokens 21.7 -> 9.1 us per call (the library's product
+// before), VQ 1920 x 288 at 1590 tokens 13.1 -> 10.8 (x copied to rows of whole steps).
 // The row tiles of a column tile go to one die (workgroups go to the eight dies in turn), so that a die's L2
 // fetches a column tile of W once for all row tiles.
 #include <math.h>
@@ -51,6 +53,7 @@ struct DenseShape {
   int M, N, steps;   // steps = K / 64
   int row_tiles, col_tiles, splits, units_per_die;  // unit: a part of K of one tile
   float* partials;   // splits > 1: [splits][M][N]
+  int pieces;        // 16-byte pieces of a row: K / 8
 };
 
 template <int WGM, int WGN, int MT, int KG, int STAGES>
@@ -72,7 +75,9 @@ struct DenseTile {
   static_assert(kLds <= kLdsPerBlockMax, "the block's tiles do not fit LDS");
 };
 
-template <int ACT, int WGM, int WGN, int MT, int KG, int STAGES>
+// SHORT: rows end inside the last step.  Loads past their end bring the last piece again, and the operands there are zeroed
+// as they are used, in the one step that has any.
+template <int ACT, int WGM, int WGN, int MT, int KG, int STAGES, bool SHORT = false>
 __global__ void __launch_bounds__((DenseTile<WGM, WGN, MT, KG, STAGES>::kThreads))
 dense_gemm_kernel(const DenseShape s) {
   using T = DenseTile<WGM, WGN, MT, KG, STAGES>;
@@ -93,8 +98,9 @@ dense_gemm_kernel(const DenseShape s) {
 
   const int steps_g = (steps - g + KG - 1) / KG;  // this group's steps: g, g + KG, ... of the part
   const int base = steps / KG;                    // steps every group has
-  const uint8_t* const xb = reinterpret_cast<const uint8_t*>(s.x) + (int64_t)m0 * s.ldx * 2 + (int64_t)step0 * 128;
-  const uint8_t* const wb = reinterpret_cast<const uint8_t*>(s.w) + (int64_t)n0 * s.ldw * 2 + (int64_t)step0 * 128;
+  const int64_t part_at = SHORT ? 0 : (int64_t)step0 * 128;
+  const uint8_t* const xb = reinterpret_cast<const uint8_t*>(s.x) + (int64_t)m0 * s.ldx * 2 + part_at;
+  const uint8_t* const wb = reinterpret_cast<const uint8_t*>(s.w) + (int64_t)n0 * s.ldw * 2 + part_at;
   // The piece of its operand that load i brings.  Where the waves don't divide the pieces, the last is brought more than once.
   auto piece_of = [&](int i) {
     return i < T::kLoadsX ? min(wave + T::kWaves * i, T::kPiecesX - 1) : min(wave + T::kWaves * (i - T::kLoadsX), T::kPiecesW - 1);
@@ -105,13 +111,19 @@ dense_gemm_kernel(const DenseShape s) {
     const bool is_x = i < T::kLoadsX;
     const int r = piece_of(i) * 8 + (lane >> 3);
     const int row = is_x ? min(r, s.M - 1 - m0) : min(r, s.N - 1 - n0);  // rows past the end: a valid row nobody stores
-    voff[i] = (uint32_t)((int64_t)row * (is_x ? s.ldx : s.ldw) * 2) + (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
+    voff[i] = (uint32_t)((int64_t)row * (is_x ? s.ldx : s.ldw) * 2) + (SHORT ? 0u : (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16));
   }
   const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + (uint32_t)(g * STAGES * T::kStageBytes);
   auto load = [&](int i, int slot, int it) {
     const bool is_x = i < T::kLoadsX;
-    const uint8_t* src = uniform_ptr((is_x ? xb : wb) + (int64_t)(g + KG * it) * 128);
     const uint32_t piece = (uint32_t)((is_x ? 0 : T::kPiecesX) + piece_of(i));
+    if constexpr (SHORT) {
+      const int p = (lane & 7) ^ ((piece_of(i) * 4 + (lane >> 4)) & 7);  // of the step, as above
+      const uint32_t at = voff[i] + (uint32_t)min((step0 + g + KG * it) * 8 + p, s.pieces - 1) * 16u;
+      lds_load16(ring + (uint32_t)(slot * T::kStageBytes) + piece * 1024u, at, uniform_ptr(is_x ? xb : wb));
+      return;
+    }
+    const uint8_t* src = uniform_ptr((is_x ? xb : wb) + (int64_t)(g + KG * it) * 128);
     lds_load16(ring + (uint32_t)(slot * T::kStageBytes) + piece * 1024u, voff[i], src);
   };
 
@@ -146,8 +158,9 @@ dense_gemm_kernel(const DenseShape s) {
 
   // One step out of ring slot `slot`: the operands of k group j + 1 are read in front of the MFMAs of group j, those of
   // the next step's first group in front of the last MFMAs (its pieces have arrived one barrier early), and with
-  // LOADS the pieces of step `ahead` are requested behind them, into the slot of the step before this one.
-  auto compute = [&](auto loads, int slot, int ahead) {
+  // LOADS the pieces of step `ahead` are requested behind them, into the slot of the step before this one.  `there`: pieces of the step
+  // in front of the rows' end (SHORT).
+  auto compute = [&](auto loads, int slot, int ahead, int there) {
     constexpr bool LOADS = decltype(loads)::value;
     const uint8_t* const stage = ring_p + slot * T::kStageBytes;
     const uint8_t* const next = ring_p + (slot == STAGES - 1 ? 0 : slot + 1) * T::kStageBytes;
@@ -157,6 +170,13 @@ dense_gemm_kernel(const DenseShape s) {
     for (int j = 0; j < 4; ++j) {
       if (j < 3) read_ops((j + 1) & 1, stage, j + 1);
       else if (T::kAhead) read_ops(0, next, 0);  // behind the last step: nothing anybody uses
+      if constexpr (SHORT && !LOADS) {  // the last step is never one that requests another
+        const bool dead = 4 * h + j >= there;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) bo[j & 1][t] = dead ? u32x4{0, 0, 0, 0} : bo[j & 1][t];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) ao[j & 1][mt] = dead ? u32x4{0, 0, 0, 0} : ao[j & 1][mt];
+      }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -178,6 +198,7 @@ dense_gemm_kernel(const DenseShape s) {
     else if (young == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   };
+  auto pieces_there = [&](int it) { return s.pieces - (step0 + g + KG * it) * 8; };
   int slot = 0;
   auto next_slot = [&] { slot = slot == STAGES - 1 ? 0 : slot + 1; };
   int it = 0;
@@ -190,7 +211,7 @@ dense_gemm_kernel(const DenseShape s) {
   for (; it < base - (STAGES - 1); ++it) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2 - T::kAhead) * kLoads) : "memory");
     block_sync_lds();  // everybody's pieces have arrived, and nobody reads the slot of the step before any more
-    compute(std::true_type{}, slot, it + STAGES - 1);
+    compute(std::true_type{}, slot, it + STAGES - 1, 8);
     next_slot();
   }
   for (; it < base; ++it) {
@@ -200,13 +221,13 @@ dense_gemm_kernel(const DenseShape s) {
 #pragma unroll
       for (int i = 0; i < kLoads; ++i) load(i, slot == 0 ? STAGES - 1 : slot - 1, it + STAGES - 1);
     }
-    compute(std::false_type{}, slot, 0);
+    compute(std::false_type{}, slot, 0, pieces_there(it));
     next_slot();
   }
   if (KG > 1 && steps % KG) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     block_sync_lds();
-    if (base < steps_g) compute(std::false_type{}, slot, 0);
+    if (base < steps_g) compute(std::false_type{}, slot, 0, pieces_there(base));
   }
 
   // The groups' sums meet in group 0, in group order.
@@ -269,11 +290,13 @@ int launch_dense_tile(DenseShape s, hipStream_t st) {
   const int64_t units = (int64_t)s.col_tiles * s.row_tiles * s.splits, blocks = (units + 7) / 8 * 8;
   s.units_per_die = (int)(blocks / 8);
   if (blocks > 0x7FFFFFFF) return fail(NPAMD_ERR_UNSUPPORTED, "npamd_dense_gemm: too many tiles");
-  static LdsLatch latch;
-  const hipError_t e = enable_dynamic_lds(latch, reinterpret_cast<const void*>(&dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES>), T::kLds);
+  static LdsLatch latches[2];
+  const bool ends_inside = s.pieces % 8 != 0;
+  const auto kernel = ends_inside ? dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES, true> : dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES, false>;
+  const hipError_t e = enable_dynamic_lds(latches[ends_inside], reinterpret_cast<const void*>(kernel), T::kLds);
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "npamd_dense_gemm: cannot reserve %d bytes of LDS: %s", T::kLds, hipGetErrorString(e));
-  launch(dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES>, (unsigned)blocks, T::kThreads, T::kLds, st, s);
+  launch(kernel, (unsigned)blocks, T::kThreads, T::kLds, st, s);
   if (s.splits > 1) launch_splitk_reduce<ACT>(s.partials, s.splits, s.M, s.N, s.bias, s.y, s.ldy, st);
   return check_launch("npamd_dense_gemm");
 }
@@ -365,22 +388,36 @@ extern "C" int64_t npamd_dense_gemm_workspace_bytes(int M, int N, int K) {
   return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
 }
 
-extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
-                                int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
-  const char* what = "npamd_dense_gemm";
+static int dense_gemm(const char* what, const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
+                      int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
   NPAMD_REQUIRE(act_dtype == NPAMD_F16 || act_dtype == NPAMD_BF16, "%s: f16 or bf16 only", what);
-  NPAMD_REQUIRE(M >= 0 && N >= 0 && K >= 64 && K % 64 == 0, "%s: bad shape M=%d N=%d K=%d (K has to be a multiple of 64)", what, M, N, K);
   NPAMD_REQUIRE(ldx >= K && ldw >= K && ldy >= N && ldx % 8 == 0 && ldw % 8 == 0, "%s: bad row stride", what);
   if (M == 0 || N == 0) return NPAMD_OK;
   NPAMD_REQUIRE(x && w && y && (((uintptr_t)x | (uintptr_t)w) & 15) == 0, "%s: null or unaligned pointer", what);
   NPAMD_REQUIRE(ldx < kDenseStrideMax && ldw < kDenseStrideMax, "%s: row stride too large", what);
   hipStream_t st = (hipStream_t)stream;
   const int64_t room = workspace && ((uintptr_t)workspace & 3) == 0 ? workspace_bytes / ((int64_t)M * N * 4) : 1;
-  DensePlan p = plan_dense(M, N, K, tuning().dense_tile, kDenseMaxSplits);
-  if (p.splits > room) p = plan_dense(M, N, K, tuning().dense_tile, 1);  // too little workspace: unsplit
-  const DenseShape s{x, w, bias, y, ldx, ldw, ldy, M, N, K / 64, 0, 0, p.splits, 0, (float*)workspace};
+  const int width = (K + 63) / 64 * 64;
+  DensePlan p = plan_dense(M, N, width, tuning().dense_tile, kDenseMaxSplits);
+  if (p.splits > room) p = plan_dense(M, N, width, tuning().dense_tile, 1);  // too little workspace: unsplit
+  const DenseShape s{x, w, bias, y, ldx, ldw, ldy, M, N, width / 64, 0, 0, p.splits, 0, (float*)workspace, K / 8};
   const int tile = p.tile;
   return act_dtype == NPAMD_BF16 ? launch_dense<NPAMD_BF16>(s, tile, st) : launch_dense<NPAMD_F16>(s, tile, st);
+}
+
+extern "C" int npamd_dense_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
+                                int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* what = "npamd_dense_gemm";
+  NPAMD_REQUIRE(M >= 0 && N >= 0 && K >= 64 && K % 64 == 0, "%s: bad shape M=%d N=%d K=%d (K has to be a multiple of 64)", what, M, N, K);
+  return dense_gemm(what, x, ldx, w, ldw, bias, y, ldy, M, N, K, act_dtype, workspace, workspace_bytes, stream);
+}
+
+// Rows of x and w that end inside a 64-k step, K a multiple of 8: neither is copied to whole steps first.
+extern "C" int npamd_dense_gemm_ragged(const void* x, int64_t ldx, const void* w, int64_t ldw, const float* bias, void* y, int64_t ldy,
+                                       int M, int N, int K, int act_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* what = "npamd_dense_gemm_ragged";
+  NPAMD_REQUIRE(M >= 0 && N >= 0 && K >= 8 && K % 8 == 0, "%s: bad shape M=%d N=%d K=%d (K has to be a multiple of 8)", what, M, N, K);
+  return dense_gemm(what, x, ldx, w, ldw, bias, y, ldy, M, N, K, act_dtype, workspace, workspace_bytes, stream);
 }
 
 // Whether a call of more than 16 tokens goes to the GEMV with a block per 32 tokens (npamd_*_gemv_blocks) rather than to decode +

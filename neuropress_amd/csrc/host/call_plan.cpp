@@ -239,10 +239,13 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   at::Tensor x = x_in;
   const int64_t ldx_in = ldx;
   bool with_gather = false;
+  // The GEMVs take rows that end inside the last 64 columns, as long as they are whole 16 bytes and start at such addresses.
+  const bool short_rows = (t.kind == kVqGemv || t.kind == kRvqGemv) && !t.perm.defined() && t.k_in != t.k && t.k_in % 8 == 0 && ldx % 8 == 0 &&
+                          ((uintptr_t)x_in.const_data_ptr() & 15) == 0;
   if (t.perm.defined() && t.perm.scalar_type() == at::kLong) {
     x = at::index_select(x_in, -1, t.perm);
     ldx = t.k;
-  } else if (t.perm.defined() || (t.k_in != t.k && t.kind != kVqGemv && t.kind != kRvqGemv)) {
+  } else if (t.perm.defined() || (t.k_in != t.k && !short_rows)) {
     sizes.back() = t.k;
     x = empty(sizes, x_in.scalar_type(), device);
     with_gather = t.kind == kVqDense && t.own;  // its decode gathers them too
@@ -277,7 +280,7 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
       at::Tensor parts;
       if (r.ws > 0) parts = empty({r.ws / 4}, at::kFloat, device);
       at::Tensor y = empty(sizes, t.out, device);
-      if (npamd_dense_gemm(x.const_data_ptr(), ldx, w.data_ptr(), t.k, t.bias.defined() ? t.bias.const_data_ptr<float>() : nullptr,
+      if ((t.k % 64 ? npamd_dense_gemm_ragged : npamd_dense_gemm)(x.const_data_ptr(), ldx, w.data_ptr(), t.k, t.bias.defined() ? t.bias.const_data_ptr<float>() : nullptr,
                            y.data_ptr(), t.n, (int)m, (int)t.n, (int)t.k, code, r.ws > 0 ? parts.data_ptr() : nullptr, r.ws, st) != NPAMD_OK)
         return false;
       *out = std::move(y);
@@ -301,7 +304,7 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   const void* xp = x.const_data_ptr();
   void* yp = y.data_ptr();
   const int M = (int)m, N = (int)t.n, K = (int)t.k;
-  const int x_columns = t.perm.defined() ? K : (int)t.k_in;  // the gather pads what it copies
+  const int x_columns = short_rows ? (int)t.k_in : K;  // the gather pads what it copies
   int rc = NPAMD_ERR_INVALID;
   switch (t.kind) {
     case kSliced:

@@ -947,9 +947,9 @@ def dense_preferred(m: int, n: int, k: int) -> bool:
     return bool(_lib.load().npamd_dense_gemm_preferred(int(m), int(n), int(k)))
 
 
-def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
-    """``x @ w.T (+ bias)`` of a 2-D fp16 / bf16 *x* with a decoded weight of its dtype, K a multiple of 64
-    (``npamd_dense_gemm``): the product of the decode + GEMM band where :func:`dense_preferred` says so."""
+def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, ragged: bool = False) -> torch.Tensor:
+    """``x @ w.T (+ bias)`` of a 2-D fp16 / bf16 *x* with a decoded weight of its dtype, K a multiple of 64 or, *ragged*, of 8
+    (``npamd_dense_gemm``, ``npamd_dense_gemm_ragged``): the product of the decode + GEMM band where :func:`dense_preferred` says so."""
     what = "dense_linear"
     _check_device(what, x, w, bias)
     x = _x2d(x, what)
@@ -962,9 +962,9 @@ def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = N
     w = w.contiguous()
     y = torch.empty((m, n), device=x.device, dtype=x.dtype)
     b32 = _bias_f32(bias)
-    need = _lib.load().npamd_dense_gemm_workspace_bytes(m, n, k)
+    need = _lib.load().npamd_dense_gemm_workspace_bytes(m, n, -(-k // 64) * 64)
     ws = torch.empty(need // 4, device=x.device, dtype=torch.float32) if need > 0 else None
-    _lib.call("npamd_dense_gemm", x.data_ptr(), x.stride(0), w.data_ptr(), k, _ptr(b32), y.data_ptr(), n, m, n, k,
+    _lib.call("npamd_dense_gemm_ragged" if ragged else "npamd_dense_gemm", x.data_ptr(), x.stride(0), w.data_ptr(), k, _ptr(b32), y.data_ptr(), n, m, n, k,
               _DT[x.dtype], _ptr(ws), need, _stream(x))  # fmt: skip
     return y
 

@@ -735,11 +735,29 @@ class NPVQLinear(nn.Module):
 
         return self._derive("wide", self.packed_indices, widen, *((self.proxy.centroids,) if pad else ())), 16
 
+    def _kernel_res_stream(self) -> tuple[torch.Tensor, int]:
+        """The residual stream next to :meth:`_kernel_stream`: 8 or 16 bits wide and padded where that is padded."""
+        pad = (self._kernel_k() - self.in_features) // self.vector_len
+        stream, bits = self._res_stream(), self._res_bits()
+        if pad == 0:
+            return stream, bits
+        from .. import kernels
+
+        def widen() -> torch.Tensor:
+            wide = stream if bits == 8 else kernels.widen_indices_u16(stream, self.n_vectors, bits)
+            size = 1 if bits == 8 else 2  # bytes
+            rows = wide.reshape(-1)[: self.n_vectors * size].reshape(self.out_features, -1)
+            return torch.nn.functional.pad(rows, (0, pad * size)).reshape(-1)
+
+        return self._derive("wide_res", stream, widen), 8 if bits == 8 else 16
+
     def _kernel_k(self) -> int:
         """Columns the MFMA kernels contract: K, rounded up to whole 64-column chunks where the layer is otherwise
-        of a form they take (vector length 8 or 4, at most 16 bits per index, no residual stream)."""
+        of a form they take (vector length 8, or 4 without a residual stream, at most 16 bits per index)."""
         k = self.in_features
-        if k % 64 == 0 or self.vector_len not in (4, 8) or self.bits > 16 or self.is_residual or self.n_vectors == 0:
+        if k % 64 == 0 or self.vector_len not in (4, 8) or self.bits > 16 or self.n_vectors == 0:
+            return k
+        if self.is_residual and (self.vector_len != 8 or self._res_bits() > 16):
             return k
         return k + 64 - k % 64
 
@@ -910,9 +928,11 @@ class NPVQLinear(nn.Module):
             args = (i32, sl.header_ptr, sl.blob, proxy.centroids_as(dtype), code, self._bias_f32(), code)
             return plans.template(plan, plans.SLICED, n, k, args, dtype)
         if self.is_residual:
-            res = self._res_stream().reshape(-1)
-            cr = self._res_centroids()
-            args = (packed, packed.numel(), self.bits, res, res.numel(), self._res_bits(), proxy.centroids, proxy.num_centroids,
+            dense = kind in ("dense", "product")
+            (main, bits), (res, res_bits) = ((packed, self.bits), (self._res_stream(), self._res_bits())) if dense else (
+                self._kernel_stream(), self._kernel_res_stream())  # fmt: skip
+            main, res, cr = main.reshape(-1), res.reshape(-1), self._res_centroids()
+            args = (main, main.numel(), bits, res, res.numel(), res_bits, proxy.centroids, proxy.num_centroids,
                     cr, cr.shape[0], self.row_scale, self.row_bias, vl)  # fmt: skip
             if kind in ("dense", "product"):
                 own = kind == "product"
@@ -920,13 +940,14 @@ class NPVQLinear(nn.Module):
                 return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=bias, leaf=self.bias, own=own)
             kind_code = plans.RVQ_TILE if kind == "tile" else plans.RVQ_GEMV
             leaf = self.bias if kind == "blocks" else None  # in the place of the dense product
-            return plans.template(plan, kind_code, n, k, (*args, self._bias_f32(), code), dtype, perm=perm, leaf=leaf)
+            return plans.template(plan, kind_code, n, self._kernel_k(), (*args, self._bias_f32(), code), dtype, k_in=k, perm=perm, leaf=leaf)
         stream, bits = self._kernel_stream()
         stream = stream.reshape(-1)
         if kind in ("dense", "product"):
             own = kind == "product"
             bias = self._bias_f32() if own else self._bias_as(dtype)
-            width = self._kernel_k() if own else k  # the library's product takes any K: no padding
+            # The library's product takes any K; the package's own any whole 16 bytes, but what a permutation copies is padded.
+            width = self._kernel_k() if own and (perm is not None or k % 8) else k
             if width == k and self._kernel_k() != k:
                 stream, bits = packed, self.bits
             args = (stream, stream.numel(), bits, proxy.centroids, proxy.num_centroids, vl, n * (width // vl))
@@ -985,6 +1006,7 @@ class NPVQLinear(nn.Module):
             self.proxy.centroids_as(dtype)
         if self.is_residual:
             self._res_stream()
+            self._kernel_res_stream()
             self._res_centroids()
         if self.backend in _FUSED_BACKENDS and (self._plan is None or self._plan.stale(self)):
             self._plan = self._new_plan()  # still without routes: every call adds its own
@@ -1149,7 +1171,8 @@ class NPVQLinear(nn.Module):
         if not 16 < m <= _BLOCKS_MAX_TOKENS or self.out_features < 256 or min(_FUSED_MAX_TOKENS, _TILE_MAX_TOKENS) <= 0 or self.backend == VQBackend.CUDA_LUT:
             return False
         if self.vector_len != 8 or self.proxy.centroids.dtype != torch.float16 or not self._mfma_layer() or (
-            self.is_residual and (self.bits, self._res_bits()) not in ((16, 8), (16, 16), (12, 8), (8, 8))
+            self.is_residual and self._kernel_k() == self.in_features
+            and (self.bits if self.bits in _FAST_BITS else 16, self._res_bits()) not in ((16, 8), (16, 16), (12, 8), (8, 8))
         ):  # fmt: skip
             return False
         from .. import kernels
@@ -1267,8 +1290,8 @@ class NPVQLinear(nn.Module):
         features) covers at least ``_TILE_MIN_GRID_FRACTION`` of the compute units."""
         if not x.is_cuda:
             return True
-        if not self._mfma_layer():
-            return False  # the tile entry point would run its element-wise fallback
+        if not self._mfma_layer() or (self.is_residual and self._kernel_k() != self.in_features):
+            return False  # the tile entry point would run its element-wise fallback, or ask for padded columns
         if self._wide_tile_layer():
             return True  # the 128-column kernel fills the GPU by splitting the reduction; its band is a token count
         cus = self._derived.get("cus")
@@ -1341,7 +1364,7 @@ class NPVQLinear(nn.Module):
                     self.proxy.centroids, self._res_centroids(), self.row_scale, self.row_bias,
                     self.out_features, self.in_features, x.dtype,
                 )  # fmt: skip
-            elif own and self._kernel_k() != self.in_features:
+            elif own and self.in_features % 8:
                 stream, bits = self._kernel_stream()
                 w = kernels.vq_dequant(stream, self.proxy.centroids, bits, self.out_features, self._kernel_k(), x.dtype)
             else:
@@ -1353,7 +1376,8 @@ class NPVQLinear(nn.Module):
                 x2d = x.reshape(-1, self.in_features)
                 if w.shape[1] != self.in_features:
                     x2d = kernels.gather_columns(x2d, None, w.shape[1])
-                return kernels.dense_linear(x2d, w, self._bias_f32()).reshape(*x.shape[:-1], self.out_features)
+                more = {"ragged": True} if w.shape[1] % 64 else {}
+                return kernels.dense_linear(x2d, w, self._bias_f32(), **more).reshape(*x.shape[:-1], self.out_features)
         except RuntimeError as exc:
             self._fallback("vq_dequant", "the gather path", exc)
             return self._forward_compile(x)
@@ -1418,10 +1442,12 @@ class NPVQLinear(nn.Module):
 
         *leading, _ = x.shape
         x2d = x.reshape(-1, self.in_features)
-        width = self._kernel_k() if blocks or (tile and self._blocks_win(x2d.shape[0])) else None
+        short = self.is_residual and self._kernel_k() != self.in_features
+        width = self._kernel_k() if blocks or short or (tile and self._blocks_win(x2d.shape[0])) else None
         if self.is_residual:
+            (main, bits), (res, res_bits) = self._kernel_stream(), self._kernel_res_stream()
             y = kernels.rvq_linear(
-                x2d, self.packed_indices, self.bits, self._res_stream(), self._res_bits(),
+                x2d, main, bits, res, res_bits,
                 self.proxy.centroids, self._res_centroids(), self.row_scale, self.row_bias,
                 self.out_features, self._bias_f32(), tile=tile, width=width,
             )  # fmt: skip

@@ -1,0 +1,71 @@
+"""Rows that end inside the last 64 columns, read where they lie: the dense product on every tile and with K split over blocks, and
+residual layers of such a K in every band; against float64."""
+
+import pytest
+import torch
+
+from neuropress_amd.nn import NPVQLinear, VQProxy
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def dense(monkeypatch):
+    from neuropress_amd import _lib
+
+    def force(tile, splits):
+        monkeypatch.setenv("NPAMD_DENSE_TILE", str(tile))
+        monkeypatch.setenv("NPAMD_DENSE_SPLITS", str(splits))
+        _lib.load().npamd_diag_reload_tuning()
+
+    yield force
+    monkeypatch.undo()
+    _lib.load().npamd_diag_reload_tuning()
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tile", range(9))
+def test_dense_product(gpu, dense, tile, act):
+    from neuropress_amd import kernels
+
+    for splits in (0, 1, 3) if tile else (0,):
+        dense(tile, splits)
+        for m, n, k in ((1, 3, 8), (33, 70, 56), (130, 257, 72), (300, 130, 584), (77, 301, 2184), (65, 65, 320), (260, 390, 1336)):
+            g = cases.gen(m + k)
+            x = torch.randn(m, k + 40, generator=g).to(act).to(gpu)[:, :k]
+            w = (torch.randn(n, k, generator=g) * 0.05).to(act).to(gpu)
+            w[:, -1] = w[:, -1].abs() + 0.01
+            x[m // 2, -1] = float("inf")  # past the end of K the last pieces come again: they must not count
+            bias = torch.randn(n, generator=g).to(gpu)
+            y = kernels.dense_linear(x, w, bias, ragged=True).double()
+            ref, size = x.double() @ w.double().T + bias.double(), x.double().abs() @ w.double().abs().T + bias.double().abs()
+            assert bool((y[m // 2] == float("inf")).all())
+            rows = torch.arange(m, device=gpu) != m // 2
+            bound = ref.abs() * (2.0**-10 if act == torch.float16 else 2.0**-7) + size * k * 2.0**-24 + 2.0**-24  # a rounding and f32 sums
+            assert bool(((y - ref).abs() <= bound)[rows].all()), (tile, splits, m, n, k)
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k,nc,ncr,perm", [(70, 8, 256, 256, False), (384, 672, 4096, 256, False), (611, 464, 65536, 256, True),
+                                             (1157, 272, 4096, 3000, False), (300, 2184, 1000, 16, True)])  # fmt: skip
+def test_residual_layers(gpu, n, k, nc, ncr, perm, act):
+    L = cases.rvq_layer(n + k, n, k, nc, ncr, zipf=False)
+    cp = torch.randperm(k, generator=cases.gen(k)) if perm else None
+    bias = torch.randn(n, generator=cases.gen(n))
+    layer = NPVQLinear(VQProxy(L["cbm"]).to(gpu), L["pm"], L["bm"], n, k, 8, "cuda_wmma", bias=bias, column_perm=cp,
+                       residual_proxy=VQProxy(L["cbr"]).to(gpu), packed_residual=L["pr"], residual_bits=L["br"],
+                       row_scale=L["scale"], row_bias=L["wbias"]).to(gpu)  # fmt: skip
+    w = (((L["cbm"][L["im"]] + L["cbr"][L["ir"]]).reshape(n, k) * L["scale"][:, None]) + L["wbias"][:, None]).to(act).float()
+    for m in (1, 3, 17, 40, 100, 400, 1100):
+        base = torch.randn(m, k + 3, generator=cases.gen(m)).to(act)
+        x = base[:, :k].contiguous()
+        ref = torch.nn.functional.linear((x if cp is None else x[:, cp]).float(), w, bias)
+        for given in (x.to(gpu), x.to(gpu), base.to(gpu)[:, :k]):  # the first call, the planned one, rows at odd addresses
+            err = (layer(given).float().cpu() - ref).abs()
+            assert bool((err <= 1e-2 + 1e-2 * ref.abs()).all()), (m, float(err.max()))
+        lead = layer(x.to(gpu).reshape(1, m, k))
+        assert lead.shape == (1, m, n)
+        xg = x.to(gpu).requires_grad_()
+        layer(xg).sum().backward()  # followed by torch: the library's product
+        assert torch.isfinite(xg.grad).all()
