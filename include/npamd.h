@@ -85,7 +85,8 @@ int npamd_vq_gemv(const void* x, int64_t ldx, const uint8_t* packed, int64_t n_b
 
 /*
  * The same for any number of tokens, 32 to a workgroup, each of which decodes the weights again: for layers so small
- * that one launch of it is over before decode + product would be (npamd_gemv_blocks_preferred).  Rows of x may end inside the
+ * that one launch of it is over before decode + product would be (npamd_gemv_blocks_preferred).  Past 16 tokens, VL = 8 and a codebook of up
+ * to 4096 rows in the activation dtype may be served by tiles of 32 to 128 tokens x 64 rows instead, on layers of any size.  Rows of x may end inside the
  * index rows' last 64 columns: k_in columns, a multiple of 8 with K - 64 < k_in <= K; what lies past them counts as zero, in x
  * and in the weights (the indices there are fillers).  Only shapes and alignments that the MFMA kernels take
  * (npamd_vq_fused_supported, residual streams of 8 bits next to 8 / 12 / 16, or 16 next to 16); others are NPAMD_ERR_UNSUPPORTED.
@@ -97,8 +98,9 @@ int npamd_vq_gemv_blocks(const void* x, int64_t ldx, int k_in, const uint8_t* pa
 
 /* Whether the *_gemv_blocks entry point is the better choice for more than 16 tokens against decode + dense product and the tile GEMM.
  * kind: 0 VQ with a codebook of table_rows rows of eight, 1 residual VQ (rows of the main codebook), 4 / 8 bits per weight (table_rows
- * ignored).  gathered: the columns of x have to be gathered first, which npamd_vq_dequant_gather does next to the decode.  Host-only arithmetic. */
-int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int table_rows, int gathered);
+ * ignored).  gathered: the columns of x have to be gathered first, which npamd_vq_dequant_gather does next to the decode.  tile: 0 where the
+ * caller would not take the tile GEMM.  Host-only arithmetic. */
+int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int table_rows, int gathered, int tile);
 
 /*
  * The same GEMV with the reference's column permutation folded in:

@@ -71,11 +71,12 @@ SIGNATURES: dict[str, list] = {
     "npamd_dense_gemm_ragged": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _int, _int, _int, _int, _vp, _i64, _vp],
     "npamd_dense_gemm_workspace_bytes": [_int, _int, _int],
     "npamd_dense_gemm_preferred": [_int, _int, _int],
-    "npamd_gemv_blocks_preferred": [_int] * 6,
+    "npamd_gemv_blocks_preferred": [_int] * 7,
     "npamd_gather_columns": [_vp, _i64, _vp, _vp, _i64, _int, _int, _vp],
     "npamd_diag_reload_tuning": [],
     "npamd_diag_last_gemv_staged": [],
     "npamd_diag_gather_fits_decode": [_int, _i64, _int, _int],
+    "npamd_diag_table_tile": [_int] * 4,
     "npamd_diag_stream_read": [_vp, _i64, _vp, _vp],
     "npamd_diag_gather": [_vp, _i64, _vp, _int, _int, _vp, _vp],
     "npamd_diag_mfma": [_vp, _int, _int, _int, _vp, _vp],

@@ -72,6 +72,7 @@ static Tuning read_tuning() {
   t.q4_stream = env_int("NPAMD_Q4_STREAM", 1);
   t.dense_tile = env_int("NPAMD_DENSE_TILE", 0);
   t.dense_splits = env_int("NPAMD_DENSE_SPLITS", 0);
+  t.table_tile = env_int("NPAMD_TABLE_TILE", 0);
   return t;
 }
 

@@ -59,6 +59,7 @@ struct Tuning {
   int q4_rows, q4_rowwise, q4_rowwise_bf16, q4_stream;
   int dense_tile;  // NPAMD_DENSE_TILE: 1 .. forces a tile of the dense product (wherever it applies), -1 switches it off
   int dense_splits;  // NPAMD_DENSE_SPLITS: parts of K of the dense product, as far as its limits allow (0: planned)
+  int table_tile;  // NPAMD_TABLE_TILE: 1 .. forces a tile of the table GEMM (wherever it applies), -1 switches it off
 };
 const Tuning& tuning();
 

@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "gemm_tile.hpp"
+#include "table_gemm.hpp"
 
 namespace npamd {
 
@@ -420,15 +421,22 @@ extern "C" int npamd_dense_gemm_ragged(const void* x, int64_t ldx, const void* w
   return dense_gemm(what, x, ldx, w, ldw, bias, y, ldy, M, N, K, act_dtype, workspace, workspace_bytes, stream);
 }
 
-// Whether a call of more than 16 tokens goes to the GEMV with a block per 32 tokens (npamd_*_gemv_blocks) rather than to decode +
-// product or the tile GEMM.  Up to a round or two of its blocks it is one short launch in the place of two that follow each
+// Whether a call of more than 16 tokens goes to the GEMV with a block per 32 tokens (npamd_*_gemv_blocks), or the table GEMM behind the same
+// entry (table_gemm.hip), rather than to decode + product or the tile GEMM.  Up to a round or two of its blocks it is one short launch in the place of two that follow each
 // other; past that every block of tokens decodes its weights again.  All three are estimated.  kind: 0 VQ, 1 residual VQ, 4 and 8 bits
 // per weight.  The GEMV's figures are fitted to layers of 512 to 8192 rows and K of 512 to 14336 at 33 to 512 tokens (within 10 %, residual
 // VQ as with indices that are all as frequent).  us, before / blocks, at 64 and 256 tokens: int4 512 x 512 6.9 / 4.0 and 6.9 / 4.1,
 // 1024 x 4096 11.8 / 6.4 and 13.3 / 9.5, 3072 x 3072 14.8 / 8.2; 256 rows 1024 x 1024 7.9 / 4.7 and 8.0 / 5.7, 2048 x 2048 10.4 / 5.7 and 11.1 / 11.2;
 // 4096 rows 1024 x 1024 8.1 / 4.7 and 8.1 / 6.6; 65536 rows 512 x 512 7.0 / 4.2 and 7.1 / 4.8, 1024 x 4096 13.2 / 10.0 and 16.5 / 24.8.
 namespace npamd {
-static float gemv_blocks_us(int kind, int table_rows, int M, int N, int K) {
+// What the library's product takes, us (see npamd_dense_gemm_preferred).
+static double library_us(int M, int N, int K) {
+  const double big_tiles = ceil(M / 256.0) * ceil(N / 256.0);
+  const double rate = big_tiles >= 180 ? 1.3 : big_tiles >= 64 ? (K < 4096 ? 1.2 : 1.05) : 0.85;
+  return 5.0 + 2e-9 * M * N * K / rate + fmax(0.0, (K - 4096) / 1024.0) * 1.5;
+}
+
+float gemv_blocks_us(int kind, int table_rows, int M, int N, int K) {
   constexpr int cus = 256;
   const int tokens = (M + kGemvTokens - 1) / kGemvTokens, rows = (N + 15) / 16, tiles = rows * tokens;
   const int steps = (K + 255) / 256, chunks = (K + 63) / 64, load = (tiles + cus - 1) / cus;
@@ -447,21 +455,35 @@ static float gemv_blocks_us(int kind, int table_rows, int M, int N, int K) {
 }
 }  // namespace npamd
 
-extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int table_rows, int gathered) {
+extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int table_rows, int gathered, int tile) {
   if (M <= 16 || N < 1 || K < 64 || K % 64) return 0;
   const float gather = gathered ? 3.0f + M * (float)K * 4 / 4.4e6f : 0.f;
-  const float blocks = gemv_blocks_us(kind, table_rows, M, N, K) + gather;
+  float blocks = gemv_blocks_us(kind, table_rows, M, N, K);
+  const bool in_lds = kind == 0 && table_rows <= 4096;
+  if (in_lds && table_rows > 16) blocks = fminf(blocks, plan_table_gemm(M, N, K, table_rows).us);  // up to 16 rows: indices of 4 bits
+  blocks = 1.03f * (blocks + gather);
   const float weights = (float)N * K;
-  const bool gathers = kind < 4 && table_rows > 2048;
+  const bool gathers = kind < 4 && table_rows > (in_lds ? 4096 : 2048);  // of plain VQ: a large layer's decode keeps such a table in LDS
   const float decode = 2.0f + fmaxf(gathers ? weights / 8 / 236e3f : 0.f, weights * 2 / 4.4e6f);
-  const float product = fmaxf(6.8f, decode + plan_dense(M, N, K, 0, kDenseMaxSplits).us);
-  if (blocks * 1.03f >= product) return 0;
+  // The library's rate here is what it reaches, 1.25 PFLOP/s from 100 of its tiles on; below, with less of a risk in the other direction, as in npamd_dense_gemm_preferred.
+  const bool own = npamd_dense_gemm_preferred(M, N, K), many = ceil(M / 256.0) * ceil(N / 256.0) >= 100;
+  const float library = many ? 5.f + 2e-9f * M * N * K / 1.25f : (float)library_us(M, N, K);
+  const float product = fmaxf(own ? 6.8f : 33.f, decode + (own ? plan_dense(M, N, K, 0, kDenseMaxSplits).us : library));
+  if (blocks >= product) return 0;
+  if (!tile || (in_lds && M > 256)) return 1;  // past 256 tokens such layers have no tile GEMM
   const int columns = (N + 63) / 64 * ((M + 383) / 384), chunks = K / 64;
   int splits = columns * 10 < 256 * 7 ? 256 / columns : 1;
   splits = splits > chunks / 8 ? chunks / 8 : splits;
   splits = splits > 16 ? 16 : splits < 1 ? 1 : splits;
-  const float tile = gather + (kind == 0 && table_rows <= 4096 ? 0.9f : kind >= 4 ? 1.05f : 1.15f) * (7.8f + 0.25f * chunks / splits + (splits > 1 ? 2.5f : 0.f));
-  return blocks * 1.03f < tile ? 1 : 0;
+  if (in_lds) {
+    // us of a step at 64 / 128 / 192 / 256 tokens: 0.23, 0.27, 0.45, 0.53, with 4096 rows a fifth more
+    const int rounds = (columns * splits + 255) / 256;
+    const float step = (M <= 128 ? 0.19f + 0.0006f * M : 0.30f + 0.0009f * M) * (1.f + 0.2f * table_rows / 4096);
+    const float us = gather + 3.3f + rounds * step * ((chunks + splits - 1) / splits) + (splits > 1 ? kSplitFixed + kSplitPerMb * (4e-6f * splits * M * N) : 0.f);
+    return blocks < us ? 1 : 0;
+  }
+  const float us = gather + (kind >= 4 ? 1.05f : 1.15f) * (7.8f + 0.25f * chunks / splits + (splits > 1 ? 2.5f : 0.f));
+  return blocks < us ? 1 : 0;
 }
 
 // Where this kernel is the better one against the library's product: its estimate against what the library reaches
@@ -484,9 +506,7 @@ extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {
   if (forced) return forced > 0;
   const double gflop = 2e-9 * M * N * K;
   const float us = plan_dense(M, N, K, 0, kDenseMaxSplits).us;
-  const double big_tiles = ceil(M / 256.0) * ceil(N / 256.0);
-  const bool many = big_tiles >= 64, shallow = many && K < 4096;
-  const double rate = big_tiles >= 180 ? 1.3 : shallow ? 1.2 : many ? 1.05 : 0.85, margin = shallow ? 1.0 : many ? 1.1 : 1.15;
-  const double library = 5.0 + gflop / rate + fmax(0.0, (K - 4096) / 1024.0) * 1.5;
-  return gflop <= (K >= 8192 ? 60.0 : 40.0) && us <= fmax(25.0, margin * library) ? 1 : 0;
+  const bool many = ceil(M / 256.0) * ceil(N / 256.0) >= 64, shallow = many && K < 4096;
+  const double margin = shallow ? 1.0 : many ? 1.1 : 1.15;
+  return gflop <= (K >= 8192 ? 60.0 : 40.0) && us <= fmax(25.0, margin * library_us(M, N, K)) ? 1 : 0;
 }

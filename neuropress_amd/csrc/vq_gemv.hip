@@ -1,4 +1,5 @@
 // C-ABI entry points of the fused decode GEMV (plain and residual VQ).
+#include "table_gemm.hpp"
 #include "vq_call.hpp"
 
 using namespace npamd;
@@ -95,7 +96,7 @@ bool takes(const VqCall& c) {
   return fast_ok(c) && res_ok;
 }
 
-// Any number of tokens, 32 to a block, and rows of x that end inside the last 64 columns; only what the MFMA kernel takes.
+// Any number of tokens, 32 to a block or, where that is the better one, as tiles of the table GEMM, and rows of x that end inside the last 64 columns; only what the MFMA kernel takes.
 int run_blocks(VqCall c, int k_in) {
   NPAMD_REQUIRE(k_in > 0 && k_in % 8 == 0 && k_in <= c.K && c.K - k_in < 64, "%s: x of %d columns against index rows of %d", c.what, k_in, c.K);
   c.k_in = k_in;
@@ -104,6 +105,8 @@ int run_blocks(VqCall c, int k_in) {
   if (rc == 1) return NPAMD_OK;
   if (!takes(c) || (c.M + kGemvTokens - 1) / kGemvTokens > 65535)
     return fail(NPAMD_ERR_UNSUPPORTED, "%s: needs a shape and alignment of the MFMA kernels", c.what);
+  const int taken = launch_table_gemm(c, 0.95f * gemv_blocks_us(0, c.nc, c.M, c.N, c.K));  // estimates: the GEMV where they are level
+  if (taken != 1) return taken;
   return c.act == NPAMD_BF16 ? dispatch<NPAMD_BF16>(c) : dispatch<NPAMD_F16>(c);
 }
 

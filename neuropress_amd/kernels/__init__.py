@@ -266,11 +266,11 @@ def vq_linear_blocks(x: torch.Tensor, packed_indices: torch.Tensor, centroids: t
     return _vq_fused("npamd_vq_gemv_blocks", x, packed_indices, centroids, bits, out_features, bias, width=int(width))
 
 
-def gemv_blocks_preferred(m: int, n: int, k: int, kind: int, table_rows: int = 0, gathered: bool = False) -> bool:
+def gemv_blocks_preferred(m: int, n: int, k: int, kind: int, table_rows: int = 0, gathered: bool = False, tile: bool = True) -> bool:
     """Whether the GEMV with a workgroup per 32 tokens is the better choice for more than 16 of them (``npamd_gemv_blocks_preferred``):
     *kind* 0 for a VQ layer with a codebook of *table_rows* rows of eight, 1 for a residual one, else bits per weight; *gathered*: the columns of x
-    are gathered first, which decode + product do along with the decode."""
-    return bool(_lib.load().npamd_gemv_blocks_preferred(int(m), int(n), int(k), int(kind), int(table_rows), int(gathered)))
+    are gathered first, which decode + product do along with the decode; *tile* False: the tile GEMM is no alternative."""
+    return bool(_lib.load().npamd_gemv_blocks_preferred(int(m), int(n), int(k), int(kind), int(table_rows), int(gathered), int(tile)))
 
 
 def vq_linear_perm_supported(m: int, n: int, k: int, num_centroids: int, vector_len: int, bits: int) -> bool:

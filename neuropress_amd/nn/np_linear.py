@@ -430,10 +430,10 @@ class NPLinear(nn.Module):
             limit = max(limit, _Q_TILE_WIDE_MAX_TOKENS)
         if m <= limit and self._tile_grid_fills_gpu(x, m, tracked):
             return "tile"
-        return "blocks" if not tracked and self._blocks_win(m) else "dense"
+        return "blocks" if not tracked and self._blocks_win(m, tile=False) else "dense"
 
-    def _blocks_win(self, m: int) -> bool:
-        """Whether the GEMV with a workgroup per 32 tokens is ahead of the fused GEMM and of decode + GEMM (NPVQLinear._blocks_win)."""
+    def _blocks_win(self, m: int, tile: bool = True) -> bool:
+        """Whether the GEMV with a workgroup per 32 tokens is ahead of the fused GEMM (*tile*) and of decode + GEMM (NPVQLinear._blocks_win)."""
         from .. import kernels
 
         if not 16 < m <= _Q_BLOCKS_MAX_TOKENS or self.out_features < 256 or min(_Q_FUSED_MAX_TOKENS, _Q_TILE_MAX_TOKENS) <= 0:
@@ -442,7 +442,7 @@ class NPLinear(nn.Module):
         lines, _ = kernels.q_gemv_staging(
             _lib.GEMV_MAX_M, self.out_features, self.in_features, self.nbits, self.group_size, self.scale, self.zero_point
         )
-        return lines and kernels.gemv_blocks_preferred(m, self.out_features, self.in_features, self.nbits)
+        return lines and kernels.gemv_blocks_preferred(m, self.out_features, self.in_features, self.nbits, tile=tile)
 
     def _planned(self, x: torch.Tensor, m: int, band: str):
         """Add this call to the layer's plan and let the plan issue it; None where it cannot."""

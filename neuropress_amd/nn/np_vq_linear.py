@@ -837,7 +837,7 @@ class NPVQLinear(nn.Module):
         if m > self._gemv_max_tokens(m):
             if self.backend != VQBackend.CUDA_LUT and m <= self._tile_max_tokens(tracked) and self._tile_band_ok(x, m, tracked):
                 return "tile"
-            return "blocks" if x.is_cuda and not tracked and self._blocks_win(m) else "dense"
+            return "blocks" if x.is_cuda and not tracked and self._blocks_win(m, tile=False) else "dense"
         return "fused"
 
     # -- call plan ---------------------------------------------------------
@@ -1164,8 +1164,9 @@ class NPVQLinear(nn.Module):
                 return 32
         return limit
 
-    def _blocks_win(self, m: int) -> bool:
-        """Whether the GEMV with a workgroup per 32 tokens is ahead of the tile GEMM and of decode + GEMM.  It takes their place on
+    def _blocks_win(self, m: int, tile: bool = True) -> bool:
+        """Whether the GEMV with a workgroup per 32 tokens (or the table GEMM behind the same entry) is ahead of
+        the tile GEMM (*tile*) and of decode + GEMM.  It takes their place on
         layers of 256 output features and more: what smaller ones do, heads and probes, they do through the products
         that callers put their own in the place of."""
         if not 16 < m <= _BLOCKS_MAX_TOKENS or self.out_features < 256 or min(_FUSED_MAX_TOKENS, _TILE_MAX_TOKENS) <= 0 or self.backend == VQBackend.CUDA_LUT:
@@ -1178,7 +1179,7 @@ class NPVQLinear(nn.Module):
         from .. import kernels
 
         return kernels.gemv_blocks_preferred(m, self.out_features, self._kernel_k(), int(self.is_residual), self.proxy.num_centroids,
-                                             self.column_perm is not None)  # fmt: skip
+                                             self.column_perm is not None, tile)  # fmt: skip
 
     def _tile_ahead_from_17(self) -> bool:
         """Large layers with at least twice as many output as input features and a codebook kept in memory: the

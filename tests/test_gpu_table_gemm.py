@@ -1,0 +1,63 @@
+"""The table GEMM, in which the blocks entry ends past a few dozen tokens: every tile at its edges -- token counts around whole tiles, rows of
+8, 12 and 16 bits, tables from one row to 4096, K of one step up to several turns per wave, an odd number of them, rows of x
+that end inside the last -- against the decoded weight in float64."""
+
+import pytest
+import torch
+
+from neuropress_amd.transforms.vq_packing import IndexPacking
+from tests import cases
+
+TILES = ((32, 8), (64, 8), (64, 4), (96, 4), (128, 4))  # rows, waves
+
+
+def test_every_tile_is_the_best_somewhere():
+    from neuropress_amd import _lib
+
+    plan = _lib.load().npamd_diag_table_tile
+    found = {plan(m, n, k, rows) for m in (32, 64, 256, 384, 512) for n in (512, 4096, 8192) for k in (256, 4096) for rows in (256, 4096)}
+    assert found == set(range(len(TILES)))
+    for m, n, k, rows in ((16, 512, 512, 256), (64, 512, 500, 256), (64, 512, 512, 4097), (64, 0, 512, 256), (64, 512, 0, 256)):
+        assert plan(m, n, k, rows) == -1
+
+
+@pytest.fixture(params=range(1, len(TILES) + 1))
+def forced(request, monkeypatch):
+    from neuropress_amd import _lib
+
+    lib = _lib.load()
+    with monkeypatch.context() as mp:
+        mp.setenv("NPAMD_TABLE_TILE", str(request.param))
+        lib.npamd_diag_reload_tuning()
+        yield TILES[request.param - 1][0]
+    lib.npamd_diag_reload_tuning()
+
+
+@pytest.mark.gpu
+def test_tiles(gpu, forced):
+    from neuropress_amd import kernels
+
+    rows = forced
+    shapes = ((259, 64, 0), (64, 128, 56), (300, 192, 0), (256, 2112, 8), (65, 1088, 40), (130, 4096 + 64, 24))
+    for act in (torch.float16, torch.bfloat16):
+        for nc, bits in ((1, 8), (200, 8), (1000, 16), (4096, 12), (4096, 16)):
+            g = cases.gen(nc + bits)
+            cb = (torch.randn(nc, 8, generator=g) * 0.05).to(act).to(gpu)
+            for n, k, short in shapes:
+                idx = torch.randint(0, nc, (n, k // 8), generator=g)
+                packed = IndexPacking.pack(idx.reshape(-1), bits).to(gpu)
+                w = cb[idx.to(gpu)].reshape(n, k)[:, : k - short].double()
+                bias = torch.randn(n, generator=g).to(gpu) if n % 2 else None
+                for m in (17, rows - 1, rows, rows + 1, 2 * rows + 33):
+                    x = torch.full((m, k + 16), float("nan"), dtype=act)
+                    x[:, : k - short] = torch.randn(m, k - short, generator=g).to(act)  # what lies behind a row counts for nothing
+                    x = x.to(gpu)[:, : k - short]
+                    y = kernels.vq_linear_blocks(x, packed, cb, bits, n, bias, width=k).double()
+                    xd = x.double()
+                    ref, size = xd @ w.T, xd.abs() @ w.abs().T
+                    if bias is not None:
+                        ref, size = ref + bias.double(), size + bias.double().abs()
+                    # one rounding of the output, and f32 sums of K products in some order
+                    bound = ref.abs() * (2.0**-10 if act == torch.float16 else 2.0**-7) + size * k * 2.0**-24 + 2.0**-24
+                    assert bool(((y - ref).abs() <= bound).all())
+
