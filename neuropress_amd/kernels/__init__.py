@@ -261,7 +261,7 @@ def vq_linear(
 
 def vq_linear_blocks(x: torch.Tensor, packed_indices: torch.Tensor, centroids: torch.Tensor, bits: int, out_features: int,
                      bias: torch.Tensor | None = None, *, width: int) -> torch.Tensor:  # fmt: skip
-    """The fused GEMV for any number of tokens, 32 to a workgroup (``npamd_vq_gemv_blocks``), where :func:`gemv_blocks_preferred` says so.
+    """The fused GEMV for any number of tokens, 32 to a workgroup, or the table GEMM (``npamd_vq_gemv_blocks``), where :func:`gemv_blocks_preferred` says so.
     *width*: columns of the index rows, a multiple of 64, of which *x* may lack up to 56 (multiples of 8)."""
     return _vq_fused("npamd_vq_gemv_blocks", x, packed_indices, centroids, bits, out_features, bias, width=int(width))
 

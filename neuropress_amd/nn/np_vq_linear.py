@@ -21,6 +21,10 @@ band                  condition                        kernel
                       where timed lists say so (one
                       token: only where they lost)
 (b) tile-decode GEMM  ``m <= _TILE_MAX_TOKENS``        ``kernels.vq_gemm_tile``
+    table GEMM        past 16 tokens where its         ``kernels.vq_linear_blocks``
+                      estimate is the least (up to
+                      4096 rows; small layers: a GEMV
+                      with a workgroup per 32 tokens)
 (c) decode + GEMM     otherwise                        ``kernels.vq_dequant`` + ``kernels.dense_linear`` or ``F.linear``
 ====================  ==============================  ==========================
 
@@ -123,7 +127,8 @@ _PREPARE_ON_MOVE: bool = _env_int(("NEUROPRESS_VQ_PREPARE_ON_MOVE",), 1) != 0
 # cuda_lut layers: 0 = always decode + GEMM, the reference's default routing.
 _LUT_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_LUT_MAX_TOKENS",), 0)
 
-# Most tokens of the GEMV with a workgroup per 32 tokens, which serves small layers past 16 of them (kernels.gemv_blocks_preferred).
+# Most tokens of the GEMV with a workgroup per 32 tokens, which serves small layers past 16 of them, and of the table GEMM behind the same
+# entry point, which serves layers of any size with a codebook of up to 4096 rows (kernels.gemv_blocks_preferred).
 _BLOCKS_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_BLOCKS_MAX_TOKENS",), 1 << 16)
 # Upper end of the tile-decode GEMM band.  NEUROPRESS_VQ_TRITON_MAX_TOKENS is the
 # reference's name for the same knob and is honoured too.  0 disables the band.
