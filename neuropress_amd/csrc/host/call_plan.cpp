@@ -304,7 +304,8 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   const void* xp = x.const_data_ptr();
   void* yp = y.data_ptr();
   const int M = (int)m, N = (int)t.n, K = (int)t.k;
-  const int x_columns = short_rows ? (int)t.k_in : K;  // the gather pads what it copies
+  // What lies past a row's end counts for nothing: residual rows have no filler whose product with a padded zero is sure to be one.
+  const int x_columns = short_rows || t.kind == kRvqGemv ? (int)t.k_in : K;
   int rc = NPAMD_ERR_INVALID;
   switch (t.kind) {
     case kSliced:

@@ -896,7 +896,8 @@ class NPVQLinear(nn.Module):
     def _add_route(self, plan, dtype: torch.dtype, m: int, band: str) -> None:
         from ..kernels import plans
 
-        tile = band == "tile" or (band == "fused" and m > _GEMV_KERNEL_MAX_TOKENS)
+        short = self.is_residual and self._kernel_k() != self.in_features  # the tile GEMM would multiply what pads their rows
+        tile = band == "tile" or (band == "fused" and m > _GEMV_KERNEL_MAX_TOKENS and not short)
         if band == "tile" and self._blocks_win(m):
             tile, band = False, "blocks"
         kind = "tile" if tile else "product" if band == "dense" and self._own_product(m, dtype) else band

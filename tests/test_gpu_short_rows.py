@@ -4,7 +4,9 @@ residual layers of such a K in every band; against float64."""
 import pytest
 import torch
 
+import neuropress_amd.nn.np_vq_linear as vqmod
 from neuropress_amd.nn import NPVQLinear, VQProxy
+from neuropress_amd.transforms.vq_packing import IndexPacking
 from tests import cases
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +71,27 @@ def test_residual_layers(gpu, n, k, nc, ncr, perm, act):
         xg = x.to(gpu).requires_grad_()
         layer(xg).sum().backward()  # followed by torch: the library's product
         assert torch.isfinite(xg.grad).all()
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("perm", [False, True])
+def test_unused_rows_of_a_residual_codebook_count_for_nothing(gpu, perm, bad, monkeypatch):
+    """Row 0 of the residual codebook is not finite and no index names it (what a cluster without members leaves behind): rows of x read where
+    they lie, copied for a permutation or from odd addresses, and past 32 tokens with the GEMV's band raised."""
+    monkeypatch.setattr(vqmod, "_FUSED_MAX_TOKENS", 64)
+    n, k, bias = 96, 200, torch.randn(96, generator=cases.gen(1))
+    L = cases.rvq_layer(5, n, k, 4096, 256, zipf=False)
+    ir = L["ir"].clamp(min=1)
+    L["cbr"][0] = bad
+    cp = torch.randperm(k, generator=cases.gen(k)) if perm else None
+    layer = NPVQLinear(VQProxy(L["cbm"]).to(gpu), L["pm"], L["bm"], n, k, 8, "cuda_wmma", bias=bias, column_perm=cp,
+                       residual_proxy=VQProxy(L["cbr"]).to(gpu), packed_residual=IndexPacking.pack(ir, L["br"]), residual_bits=L["br"],
+                       row_scale=L["scale"], row_bias=L["wbias"]).to(gpu)  # fmt: skip
+    w = ((L["cbm"][L["im"]] + L["cbr"][ir]).reshape(n, k) * L["scale"][:, None] + L["wbias"][:, None]).float()
+    for m in (1, 5, 20, 40):
+        base = torch.randn(m, k + 3, generator=cases.gen(m)).half()
+        x = base[:, :k].contiguous()
+        ref = torch.nn.functional.linear((x if cp is None else x[:, cp]).float(), w, bias)
+        for given in (x.to(gpu), x.to(gpu), base.to(gpu)[:, :k], base.to(gpu)[:, :k]):  # the first call, the planned one, rows at odd addresses
+            err = (layer(given).float().cpu() - ref).abs()
+            assert bool((err <= 1e-2 + 1e-2 * ref.abs()).all()), (m, float(err.max()))
