@@ -933,6 +933,8 @@ class NPVQLinear(nn.Module):
             plan.hold(sl)  # the plan passes the address of its header
             args = (i32, sl.header_ptr, sl.blob, proxy.centroids_as(dtype), code, self._bias_f32(), code)
             return plans.template(plan, plans.SLICED, n, k, args, dtype)
+        # In the place of the dense product, which carries the bias's gradient: past the GEMV's band, and for all calls of ragged rows that ask for one.
+        leaf = self.bias if kind == "blocks" or self._kernel_k() != k else None
         if self.is_residual:
             dense = kind in ("dense", "product")
             (main, bits), (res, res_bits) = ((packed, self.bits), (self._res_stream(), self._res_bits())) if dense else (
@@ -945,7 +947,6 @@ class NPVQLinear(nn.Module):
                 bias = self._bias_f32() if own else self._bias_as(dtype)
                 return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=bias, leaf=self.bias, own=own)
             kind_code = plans.RVQ_TILE if kind == "tile" else plans.RVQ_GEMV
-            leaf = self.bias if kind == "blocks" else None  # in the place of the dense product
             return plans.template(plan, kind_code, n, self._kernel_k(), (*args, self._bias_f32(), code), dtype, k_in=k, perm=perm, leaf=leaf)
         stream, bits = self._kernel_stream()
         stream = stream.reshape(-1)
@@ -962,7 +963,6 @@ class NPVQLinear(nn.Module):
         if kind == "gemv_perm":
             return plans.template(plan, plans.VQ_GEMV_PERM, n, k, (*args, self._perm_i32(stream.device)), dtype)
         kind_code = {"tile": plans.VQ_TILE, "slice": plans.VQ_SLICE}.get(kind, plans.VQ_GEMV)
-        leaf = self.bias if kind == "blocks" else None  # in the place of the dense product
         return plans.template(plan, kind_code, n, self._kernel_k(), args, dtype, k_in=k, perm=perm, leaf=leaf)
 
     # -- slice-list GEMV ---------------------------------------------------

@@ -95,3 +95,27 @@ def test_unused_rows_of_a_residual_codebook_count_for_nothing(gpu, perm, bad, mo
         for given in (x.to(gpu), x.to(gpu), base.to(gpu)[:, :k], base.to(gpu)[:, :k]):  # the first call, the planned one, rows at odd addresses
             err = (layer(given).float().cpu() - ref).abs()
             assert bool((err <= 1e-2 + 1e-2 * ref.abs()).all()), (m, float(err.max()))
+
+
+@pytest.mark.parametrize("k,nc,ncr,tokens", [(200, 65536, 0, (3, 24)), (200, 4096, 256, (3, 24)), (204, 1000, 0, (3, 24)), (2184, 65536, 0, (40,))])
+def test_a_planned_call_keeps_the_gradient_of_the_bias(gpu, k, nc, ncr, tokens, monkeypatch):
+    """A layer planned where no gradient was asked for, and called again where the bias asks for one: as without a plan, the library's
+    product, which carries it.  Vector length 8 and 4, residual layers, the GEMV's band and the tile GEMM's."""
+    monkeypatch.setattr(vqmod, "_TILE_MIN_GRID_FRACTION", 0.0)
+    n, vl = 96, 4 if k % 8 else 8
+    L = cases.rvq_layer(5, n, k, nc, ncr, zipf=False) if ncr else cases.vq_layer(n, n, k, nc, vl=vl)
+    more = dict(residual_proxy=VQProxy(L["cbr"]).to(gpu), packed_residual=L["pr"], residual_bits=L["br"], row_scale=L["scale"],
+                row_bias=L["wbias"]) if ncr else {}  # fmt: skip
+    cb, packed, bits = (L["cbm"], L["pm"], L["bm"]) if ncr else (L["cb"], L["packed"], L["bits"])
+    layer = NPVQLinear(VQProxy(cb).to(gpu), packed, bits, n, k, vl, "cuda_wmma", bias=torch.zeros(n), **more).to(gpu)
+    layer.bias.requires_grad_()
+    for m in tokens:
+        x = torch.randn(m, k, generator=cases.gen(3)).half().to(gpu)
+        with torch.no_grad():
+            y = layer(x)
+            assert torch.equal(layer(x), y) and not y.requires_grad
+        y = layer(x)
+        assert y.requires_grad
+        y.float().sum().backward()
+        assert torch.equal(layer.bias.grad, torch.full_like(layer.bias, m))
+        layer.bias.grad = None
