@@ -50,11 +50,12 @@ enum Kind : int {
   kQGemv, kQTile, kQDense,
   kRmsNorm, kVqEmbedding, kQEmbedding,
   kVqSlice,
+  kVqBlocks, kRvqBlocks, kQBlocks,  // the *_gemv_blocks entry points: any number of tokens, rows of x that end inside the last 64 columns
   kKinds,
 };
 
 // Constant arguments each kind takes, in the order of its entry point (see issue()).
-constexpr int kArgs[kKinds] = {7, 9, 10, 9, 7, 15, 15, 13, 9, 9, 9, 2, 8, 8, 9};
+constexpr int kArgs[kKinds] = {7, 9, 10, 9, 7, 15, 15, 13, 9, 9, 9, 2, 8, 8, 9, 9, 15, 9};
 
 // A dictionary some of whose entries the plan was built from.  CPython stamps a dictionary with a new tag on every
 // change, so an unchanged tag means unchanged entries; after a change the entries themselves are compared.
@@ -239,13 +240,12 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   at::Tensor x = x_in;
   const int64_t ldx_in = ldx;
   bool with_gather = false;
-  // The GEMVs take rows that end inside the last 64 columns, as long as they are whole 16 bytes and start at such addresses.
-  const bool short_rows = (t.kind == kVqGemv || t.kind == kRvqGemv) && !t.perm.defined() && t.k_in != t.k && t.k_in % 8 == 0 && ldx % 8 == 0 &&
-                          ((uintptr_t)x_in.const_data_ptr() & 15) == 0;
+  const bool blocks = t.kind == kVqBlocks || t.kind == kRvqBlocks || t.kind == kQBlocks;
+  const bool readable = ldx % 8 == 0 && ((uintptr_t)x_in.const_data_ptr() & 15) == 0;  // 16 bytes at a time, where it lies
   if (t.perm.defined() && t.perm.scalar_type() == at::kLong) {
     x = at::index_select(x_in, -1, t.perm);
     ldx = t.k;
-  } else if (t.perm.defined() || (t.k_in != t.k && !short_rows)) {
+  } else if (t.perm.defined() || (t.k_in != t.k && !(blocks && readable))) {
     sizes.back() = t.k;
     x = empty(sizes, x_in.scalar_type(), device);
     with_gather = t.kind == kVqDense && t.own;  // its decode gathers them too
@@ -304,8 +304,8 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   const void* xp = x.const_data_ptr();
   void* yp = y.data_ptr();
   const int M = (int)m, N = (int)t.n, K = (int)t.k;
-  // What lies past a row's end counts for nothing: residual rows have no filler whose product with a padded zero is sure to be one.
-  const int x_columns = short_rows || t.kind == kRvqGemv ? (int)t.k_in : K;
+  // Also of a padded copy: residual rows have no filler whose product with a padded zero is sure to be one.
+  const int x_columns = (int)t.k_in;
   int rc = NPAMD_ERR_INVALID;
   switch (t.kind) {
     case kSliced:
@@ -318,12 +318,12 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
       }
       break;
     case kVqGemv:
-      if (M > NPAMD_GEMV_MAX_M || x_columns != K)
-        rc = npamd_vq_gemv_blocks(xp, ldx, x_columns, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
-                                  ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
-      else
-        rc = npamd_vq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
-                           ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
+      rc = npamd_vq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
+                         ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
+      break;
+    case kVqBlocks:
+      rc = npamd_vq_gemv_blocks(xp, ldx, x_columns, ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4], (int)a[5], (int)a[6],
+                                ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], st);
       break;
     case kVqGemvPerm:
       rc = npamd_vq_gemv_perm(xp, ldx, ptr<I32>(a[9]), ptr<U8>(a[0]), a[1], (int)a[2], ptr<void*>(a[3]), (int)a[4],
@@ -338,14 +338,14 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
                                ptr<F32>(a[7]), yp, t.n, M, N, K, (int)a[8], ws, ws_bytes, st);
       break;
     case kRvqGemv:
-      if (M > NPAMD_GEMV_MAX_M || x_columns != K)
-        rc = npamd_rvq_gemv_blocks(xp, ldx, x_columns, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]),
-                                   (int)a[7], ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12],
-                                   ptr<F32>(a[13]), yp, t.n, M, N, K, (int)a[14], st);
-      else
-        rc = npamd_rvq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]), (int)a[7],
-                            ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12], ptr<F32>(a[13]), yp,
-                            t.n, M, N, K, (int)a[14], st);
+      rc = npamd_rvq_gemv(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]), (int)a[7],
+                          ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12], ptr<F32>(a[13]), yp,
+                          t.n, M, N, K, (int)a[14], st);
+      break;
+    case kRvqBlocks:
+      rc = npamd_rvq_gemv_blocks(xp, ldx, x_columns, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]),
+                                 (int)a[7], ptr<void*>(a[8]), (int)a[9], ptr<void*>(a[10]), ptr<void*>(a[11]), (int)a[12],
+                                 ptr<F32>(a[13]), yp, t.n, M, N, K, (int)a[14], st);
       break;
     case kRvqTile:
       rc = npamd_rvq_gemm_tile(xp, ldx, ptr<U8>(a[0]), a[1], (int)a[2], ptr<U8>(a[3]), a[4], (int)a[5], ptr<void*>(a[6]),
@@ -353,8 +353,12 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
                                ptr<F32>(a[13]), yp, t.n, M, N, K, (int)a[14], ws, ws_bytes, st);
       break;
     case kQGemv:
-      rc = (M > NPAMD_GEMV_MAX_M ? npamd_q_gemv_blocks : npamd_q_gemv)(xp, ldx, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), ptr<F32>(a[3]), yp, t.n, M, N, K,
+      rc = npamd_q_gemv(xp, ldx, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), ptr<F32>(a[3]), yp, t.n, M, N, K,
                         (int)a[6], (int)a[7], (int)a[8], st);
+      break;
+    case kQBlocks:
+      rc = npamd_q_gemv_blocks(xp, ldx, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), ptr<F32>(a[3]), yp, t.n, M, N, K,
+                               (int)a[6], (int)a[7], (int)a[8], st);
       break;
     case kQTile:
       rc = npamd_q_gemm_tile(xp, ldx, ptr<U8>(a[0]), ptr<void*>(a[1]), ptr<void*>(a[2]), ptr<F32>(a[3]), yp, t.n, M, N, K,

@@ -1086,3 +1086,8 @@ WRAPPERS = {
                q_linear_blocks, q_gemm_tile,
                q_dequant, rms_norm, vq_embedding, q_embedding, dense_linear, gather_columns)
 }  # fmt: skip
+
+
+def replaced(*names: str) -> bool:
+    """Whether one of the functions *names* of ``WRAPPERS`` is another than this module's own."""
+    return any(globals()[name] is not WRAPPERS[name] for name in names)

@@ -17,7 +17,7 @@ _TORCH_CALL = torch.nn.Module.__call__
 _TORCH_LINEAR = torch.nn.functional.linear
 
 (SLICED, VQ_GEMV, VQ_GEMV_PERM, VQ_TILE, VQ_DENSE, RVQ_GEMV, RVQ_TILE, RVQ_DENSE,
- Q_GEMV, Q_TILE, Q_DENSE, RMS_NORM, VQ_EMBEDDING, Q_EMBEDDING, VQ_SLICE) = range(15)  # fmt: skip
+ Q_GEMV, Q_TILE, Q_DENSE, RMS_NORM, VQ_EMBEDDING, Q_EMBEDDING, VQ_SLICE, VQ_BLOCKS, RVQ_BLOCKS, Q_BLOCKS) = range(18)  # fmt: skip
 
 DTYPE_CODES = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32, torch.int64: 3}
 

@@ -469,7 +469,7 @@ class NPLinear(nn.Module):
             band = "product"
         number = plan.names.get((band, x.dtype))
         if number is None:
-            kind = {"fused": plans.Q_GEMV, "blocks": plans.Q_GEMV, "tile": plans.Q_TILE}.get(band, plans.Q_DENSE)
+            kind = {"fused": plans.Q_GEMV, "blocks": plans.Q_BLOCKS, "tile": plans.Q_TILE}.get(band, plans.Q_DENSE)
             args = (self.u8_blob, self.scale, self.zero_point, self._bias_f32(), 0, 0, self.nbits, self.group_size, code)
             bias = self._bias_as(x.dtype) if band == "dense" else self._bias_f32() if band == "product" else None
             number = plan.names[band, x.dtype] = plans.template(plan, kind, n, k, args, x.dtype, bias=bias, leaf=self.bias, own=band == "product")

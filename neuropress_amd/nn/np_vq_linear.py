@@ -741,7 +741,8 @@ class NPVQLinear(nn.Module):
         return self._derive("wide", self.packed_indices, widen, *((self.proxy.centroids,) if pad else ())), 16
 
     def _kernel_res_stream(self) -> tuple[torch.Tensor, int]:
-        """The residual stream next to :meth:`_kernel_stream`: 8 or 16 bits wide and padded where that is padded."""
+        """The residual stream next to :meth:`_kernel_stream`: 8 or 16 bits wide and padded where that is padded, with index 0: no row
+        is sure to be finite together with the main one and the row's scale, so nothing may multiply the padding."""
         pad = (self._kernel_k() - self.in_features) // self.vector_len
         stream, bits = self._res_stream(), self._res_bits()
         if pad == 0:
@@ -793,6 +794,8 @@ class NPVQLinear(nn.Module):
             y = self._planned(x, m, band)
             if y is not None:
                 return y
+        if band == "blocks" and kernels.replaced("vq_linear"):
+            band = self._band(x, m, tracked, blocks=False)  # what it takes the place of
         if band == "sliced":
             return self._forward_sliced(x, self._sliced_for(m))  # applies column_perm inside the kernel
         if band == "gemv_perm":
@@ -817,12 +820,14 @@ class NPVQLinear(nn.Module):
             return self._forward_compile(x)
         return self._forward_default(x)
 
-    def _band(self, x: torch.Tensor, m: int, tracked: bool = False) -> str:
+    def _band(self, x: torch.Tensor, m: int, tracked: bool = False, blocks: bool = True) -> str:
         """Which kernel serves a call of *m* tokens: ``sliced``, ``gemv_perm`` (the GEMV that gathers x's columns),
-        ``fused`` (the backend's GEMV), ``blocks`` (it with a workgroup per 32 tokens), ``slice`` (the slice GEMM), ``tile``, ``dense`` (decode + GEMM) or ``torch``.
+        ``fused`` (the backend's GEMV), ``blocks`` (it with a workgroup per 32 tokens and for rows of x that end inside the last 64
+        columns, or the table GEMM), ``slice`` (the slice GEMM), ``tile``, ``dense`` (decode + GEMM) or ``torch``.
 
         *tracked* (``kernels.tracked(x)``): the dense product is the library's, columns are gathered by torch and none
-        are padded; the limits are those against that.  What it serves carries gradients, the other kernels do not."""
+        are padded; the limits are those against that.  What it serves carries gradients, the other kernels do not.
+        *blocks* False: what ``blocks`` takes the place of."""
         if self.backend not in _FUSED_BACKENDS:
             return "torch"
         if x.dtype not in (torch.float16, torch.bfloat16):
@@ -834,7 +839,8 @@ class NPVQLinear(nn.Module):
             return "sliced"
         if self.column_perm is not None and self._perm_fusable(x, m):
             return "gemv_perm"
-        if x.is_cuda and (not self._mfma_layer() or (tracked and self._kernel_k() != self.in_features)):
+        ragged = self._kernel_k() != self.in_features
+        if x.is_cuda and (not self._mfma_layer() or (ragged and (tracked or (self.is_residual and not blocks)))):
             # Shapes without an MFMA kernel (vector lengths other than 8 and 4, K not a
             # multiple of 64): the element-wise GEMV is slower than decoding once and calling
             # the dense GEMM at every token count (14336 x 4096: 99 us against 57 us at one token).
@@ -842,8 +848,12 @@ class NPVQLinear(nn.Module):
         if m > self._gemv_max_tokens(m):
             if self.backend != VQBackend.CUDA_LUT and m <= self._tile_max_tokens(tracked) and self._tile_band_ok(x, m, tracked):
                 return "tile"
-            return "blocks" if x.is_cuda and not tracked and self._blocks_win(m, tile=False) else "dense"
-        return "fused"
+            return "blocks" if blocks and x.is_cuda and not tracked and self._blocks_win(m, tile=False) else "dense"
+        # Ragged rows, where they are whole 16 bytes, are read where they lie.  Those that a permutation copies are padded on the way: the GEMV on
+        # whole chunks is ahead (us per call, read as ragged rows / padded: 8000 x 4104 with 256 rows 7.9 / 7.4 at one token, 8.1 / 7.8 at 4).
+        # Residual rows are never padded, see _kernel_res_stream, nor given to the tile GEMM (past 32 tokens, a raised band).
+        short = ragged and (self.is_residual or (self.in_features % 8 == 0 and self.column_perm is None and m <= _GEMV_KERNEL_MAX_TOKENS))
+        return "blocks" if blocks and x.is_cuda and short else "fused"
 
     # -- call plan ---------------------------------------------------------
 
@@ -896,8 +906,7 @@ class NPVQLinear(nn.Module):
     def _add_route(self, plan, dtype: torch.dtype, m: int, band: str) -> None:
         from ..kernels import plans
 
-        short = self.is_residual and self._kernel_k() != self.in_features  # the tile GEMM would multiply what pads their rows
-        tile = band == "tile" or (band == "fused" and m > _GEMV_KERNEL_MAX_TOKENS and not short)
+        tile = band == "tile" or (band == "fused" and m > _GEMV_KERNEL_MAX_TOKENS)
         if band == "tile" and self._blocks_win(m):
             tile, band = False, "blocks"
         kind = "tile" if tile else "product" if band == "dense" and self._own_product(m, dtype) else band
@@ -946,7 +955,7 @@ class NPVQLinear(nn.Module):
                 own = kind == "product"
                 bias = self._bias_f32() if own else self._bias_as(dtype)
                 return plans.template(plan, plans.RVQ_DENSE, n, k, args, dtype, perm=perm, bias=bias, leaf=self.bias, own=own)
-            kind_code = plans.RVQ_TILE if kind == "tile" else plans.RVQ_GEMV
+            kind_code = {"tile": plans.RVQ_TILE, "blocks": plans.RVQ_BLOCKS}.get(kind, plans.RVQ_GEMV)
             return plans.template(plan, kind_code, n, self._kernel_k(), (*args, self._bias_f32(), code), dtype, k_in=k, perm=perm, leaf=leaf)
         stream, bits = self._kernel_stream()
         stream = stream.reshape(-1)
@@ -962,7 +971,7 @@ class NPVQLinear(nn.Module):
         args = (stream, stream.numel(), bits, proxy.centroids_as(dtype), code, proxy.num_centroids, vl, self._bias_f32(), code)
         if kind == "gemv_perm":
             return plans.template(plan, plans.VQ_GEMV_PERM, n, k, (*args, self._perm_i32(stream.device)), dtype)
-        kind_code = {"tile": plans.VQ_TILE, "slice": plans.VQ_SLICE}.get(kind, plans.VQ_GEMV)
+        kind_code = {"tile": plans.VQ_TILE, "slice": plans.VQ_SLICE, "blocks": plans.VQ_BLOCKS}.get(kind, plans.VQ_GEMV)
         return plans.template(plan, kind_code, n, self._kernel_k(), args, dtype, k_in=k, perm=perm, leaf=leaf)
 
     # -- slice-list GEMV ---------------------------------------------------
@@ -1449,8 +1458,7 @@ class NPVQLinear(nn.Module):
 
         *leading, _ = x.shape
         x2d = x.reshape(-1, self.in_features)
-        short = self.is_residual and self._kernel_k() != self.in_features
-        width = self._kernel_k() if blocks or short or (tile and self._blocks_win(x2d.shape[0])) else None
+        width = self._kernel_k() if blocks or (tile and self._blocks_win(x2d.shape[0])) else None
         if self.is_residual:
             (main, bits), (res, res_bits) = self._kernel_stream(), self._kernel_res_stream()
             y = kernels.rvq_linear(

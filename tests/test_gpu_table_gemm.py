@@ -61,3 +61,29 @@ def test_tiles(gpu, forced):
                     bound = ref.abs() * (2.0**-10 if act == torch.float16 else 2.0**-7) + size * k * 2.0**-24 + 2.0**-24
                     assert bool(((y - ref).abs() <= bound).all())
 
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,nc", [(4096, 12544, 256), (1100, 2040, 4096)])
+def test_17_to_32_tokens_run_one_kernel_on_every_way(gpu, n, k, nc):
+    """Long or ragged rows, where the blocks entry serves as few tokens as the GEMV: planned, first, with rows at odd addresses and captured calls give the
+    same bits, those of the entry itself."""
+    from neuropress_amd import kernels
+    from neuropress_amd.nn import NPVQLinear, VQProxy
+
+    L = cases.vq_layer(n, n, k, nc)
+    layer = NPVQLinear(VQProxy(L["cb"]).to(gpu), L["packed"], L["bits"], n, k, 8, "cuda_wmma").to(gpu)
+    for m in (24, 32):
+        base = torch.randn(m, k + 3, generator=cases.gen(m)).half().to(gpu)
+        x = base[:, :k].contiguous()
+        stream, bits = layer._kernel_stream()
+        expect = kernels.vq_linear_blocks(x, stream, layer.proxy.centroids, bits, n, width=layer._kernel_k())
+        for given in (x, x, base[:, :k], base[:, :k]):
+            assert torch.equal(layer(given), expect)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = layer(x)
+        for _ in range(3):
+            captured.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(captured, expect)
