@@ -670,15 +670,11 @@ def vq_gemm_tile(
     bits: int,
     out_features: int,
     bias: torch.Tensor | None = None,
-    width: int | None = None,
 ) -> torch.Tensor:
     """``x @ W.T (+ bias)`` with W decoded tile by tile inside an MFMA GEMM.
 
-    Signature of the reference's ``vq_gemm_triton`` (neuropress/kernels/vq_triton.py:119-126), and *width*: the kernel of
-    :func:`vq_linear_blocks` instead, where :func:`gemv_blocks_preferred` says so.
+    Signature of the reference's ``vq_gemm_triton`` (neuropress/kernels/vq_triton.py:119-126).
     """
-    if width is not None:
-        return vq_linear_blocks(x, packed_indices, centroids, bits, out_features, bias, width=width)
     return _vq_fused("npamd_vq_gemm_tile", x, packed_indices, centroids, bits, out_features, bias)
 
 
@@ -772,8 +768,13 @@ def rvq_linear(
     tile: bool | None = None,
     width: int | None = None,
 ) -> torch.Tensor:
-    """Fused residual-VQ linear; ``tile=None`` picks GEMV for ``M <= 32`` else the tile GEMM.  *width*: any number of tokens through
-    the GEMV, index rows of that many columns (see :func:`vq_linear_blocks`)."""
+    """Fused residual-VQ linear; ``tile=None`` picks GEMV for ``M <= 32`` else the tile GEMM.  *width*: :func:`rvq_linear_blocks`."""
+    return _rvq_linear(x, packed_main, bits_main, packed_res, bits_res, centroids_main, centroids_res, row_scale, row_bias,
+                       out_features, bias, tile, width)  # fmt: skip
+
+
+def _rvq_linear(x, packed_main, bits_main, packed_res, bits_res, centroids_main, centroids_res, row_scale, row_bias,
+                out_features, bias, tile, width) -> torch.Tensor:  # fmt: skip
     what = "rvq_linear"
     _check_device(what, x, packed_main, packed_res, centroids_main, centroids_res)
     x = _x2d(x, what)
@@ -803,6 +804,26 @@ def rvq_linear(
         _DT[x.dtype], *extra, _stream(x),
     )  # fmt: skip
     return y
+
+
+def rvq_linear_blocks(
+    x: torch.Tensor,
+    packed_main: torch.Tensor,
+    bits_main: int,
+    packed_res: torch.Tensor,
+    bits_res: int,
+    centroids_main: torch.Tensor,
+    centroids_res: torch.Tensor,
+    row_scale: torch.Tensor | None,
+    row_bias: torch.Tensor | None,
+    out_features: int,
+    bias: torch.Tensor | None = None,
+    *,
+    width: int,
+) -> torch.Tensor:
+    """The residual GEMV for any number of tokens and rows of x that end inside the last 64 columns (see :func:`vq_linear_blocks`)."""
+    return _rvq_linear(x, packed_main, bits_main, packed_res, bits_res, centroids_main, centroids_res, row_scale, row_bias,
+                       out_features, bias, False, width)  # fmt: skip
 
 
 # ---------------------------------------------------------------------------
@@ -898,9 +919,9 @@ def q_linear_blocks(x, w_pack, scale, nbits, group_size, zero_point=None, bias=N
     return _q_fused("npamd_q_gemv_blocks", x, w_pack, scale, nbits, group_size, zero_point, bias)
 
 
-def q_gemm_tile(x, w_pack, scale, nbits, group_size, zero_point=None, bias=None, blocks=False) -> torch.Tensor:
-    """Fused dequant MFMA GEMM at any M; *blocks*: the kernel of :func:`q_linear_blocks` instead."""
-    return _q_fused("npamd_q_gemv_blocks" if blocks else "npamd_q_gemm_tile", x, w_pack, scale, nbits, group_size, zero_point, bias)
+def q_gemm_tile(x, w_pack, scale, nbits, group_size, zero_point=None, bias=None) -> torch.Tensor:
+    """Fused dequant MFMA GEMM at any M."""
+    return _q_fused("npamd_q_gemm_tile", x, w_pack, scale, nbits, group_size, zero_point, bias)
 
 
 # ---------------------------------------------------------------------------
@@ -1082,7 +1103,7 @@ def q_embedding(
 # plans step aside, so that the replacement is called.
 WRAPPERS = {
     fn.__name__: fn
-    for fn in (vq_linear_sliced_checked, vq_linear, vq_linear_blocks, vq_gemm_tile, vq_slice_gemm, vq_dequant, rvq_linear, rvq_dequant, q_linear,
+    for fn in (vq_linear_sliced_checked, vq_linear, vq_linear_blocks, vq_gemm_tile, vq_slice_gemm, vq_dequant, rvq_linear, rvq_linear_blocks, rvq_dequant, q_linear,
                q_linear_blocks, q_gemm_tile,
                q_dequant, rms_norm, vq_embedding, q_embedding, dense_linear, gather_columns)
 }  # fmt: skip

@@ -391,10 +391,11 @@ class NPLinear(nn.Module):
                 y = self._planned(x, m, band)
                 if y is not None:
                     return y
+            if band == "blocks" and kernels.replaced("q_gemm_tile", "q_dequant", "dense_linear"):
+                band = self._band(x, m, tracked, blocks=False)  # whose function a caller has put another in the place of
             if band != "dense":
                 fn = {"fused": kernels.q_linear, "blocks": kernels.q_linear_blocks}.get(band, kernels.q_gemm_tile)
-                more = {"blocks": True} if band == "tile" and not tracked and self._blocks_win(m) else {}
-                return fn(x, self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point, self._bias_f32(), **more)
+                return fn(x, self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point, self._bias_f32())
             w = kernels.q_dequant(
                 self.u8_blob, self.scale, self.nbits, self.group_size, self.zero_point, x.dtype
             )
@@ -413,9 +414,10 @@ class NPLinear(nn.Module):
 
         return dtype in (torch.float16, torch.bfloat16) and kernels.dense_preferred(m, self.out_features, self.in_features)
 
-    def _band(self, x: torch.Tensor, m: int, tracked: bool = False) -> str:
+    def _band(self, x: torch.Tensor, m: int, tracked: bool = False, blocks: bool = True) -> str:
         """Which kernel serves a call of *m* tokens: ``fused`` (GEMV), ``blocks`` (GEMV, a workgroup per 32 tokens), ``tile`` (fused GEMM) or ``dense`` (decode + GEMM).
-        *tracked* (``kernels.tracked(x)``): the dense product is the library's, and so are the limits against it."""
+        *tracked* (``kernels.tracked(x)``): the dense product is the library's, and so are the limits against it.  *blocks* False: what ``blocks``
+        takes the place of."""
         # Layers the MFMA kernels do not take (1 / 2 / 8 bits, odd group sizes) would run an
         # element-wise kernel, slower at every token count than decoding once and calling the
         # dense GEMM (14336 x 4096, 8 bits: 99 us against 57 us at one token, 452 against 57 at 16).
@@ -428,9 +430,10 @@ class NPLinear(nn.Module):
             limit = max(limit, _Q_TILE_LONG_K_MAX_TOKENS)
         if limit > 0 and max(self.in_features, self.out_features) >= _Q_TILE_WIDE_MIN_FEATURES:
             limit = max(limit, _Q_TILE_WIDE_MAX_TOKENS)
-        if m <= limit and self._tile_grid_fills_gpu(x, m, tracked):
-            return "tile"
-        return "blocks" if not tracked and self._blocks_win(m, tile=False) else "dense"
+        tile = m <= limit and self._tile_grid_fills_gpu(x, m, tracked)
+        if blocks and not tracked and self._blocks_win(m, tile):
+            return "blocks"
+        return "tile" if tile else "dense"
 
     def _blocks_win(self, m: int, tile: bool = True) -> bool:
         """Whether the GEMV with a workgroup per 32 tokens is ahead of the fused GEMM (*tile*) and of decode + GEMM (NPVQLinear._blocks_win)."""
@@ -463,8 +466,6 @@ class NPLinear(nn.Module):
             if plan is None:
                 return None
         code = plans.DTYPE_CODES[x.dtype]
-        if band == "tile" and self._blocks_win(m):
-            band = "blocks"
         if band == "dense" and self._own_product(m, x.dtype):
             band = "product"
         number = plan.names.get((band, x.dtype))

@@ -794,8 +794,8 @@ class NPVQLinear(nn.Module):
             y = self._planned(x, m, band)
             if y is not None:
                 return y
-        if band == "blocks" and kernels.replaced("vq_linear"):
-            band = self._band(x, m, tracked, blocks=False)  # what it takes the place of
+        if band == "blocks" and kernels.replaced("vq_linear", "vq_gemm_tile", "vq_dequant", "rvq_linear", "rvq_dequant", "dense_linear"):
+            band = self._band(x, m, tracked, blocks=False)  # whose function a caller has put another in the place of
         if band == "sliced":
             return self._forward_sliced(x, self._sliced_for(m))  # applies column_perm inside the kernel
         if band == "gemv_perm":
@@ -809,7 +809,7 @@ class NPVQLinear(nn.Module):
         if band == "slice":
             return self._forward_slice_gemm(x)
         if band == "blocks":
-            return self._fused(x, tile=False, blocks=True)
+            return self._forward_blocks(x)
         if self.backend == VQBackend.CUDA_LUT:
             return self._forward_cuda_lut(x)
         if self.backend == VQBackend.CUDA_WMMA or self.backend in _CODED_BACKENDS:
@@ -846,9 +846,10 @@ class NPVQLinear(nn.Module):
             # the dense GEMM at every token count (14336 x 4096: 99 us against 57 us at one token).
             return "dense"
         if m > self._gemv_max_tokens(m):
-            if self.backend != VQBackend.CUDA_LUT and m <= self._tile_max_tokens(tracked) and self._tile_band_ok(x, m, tracked):
-                return "tile"
-            return "blocks" if blocks and x.is_cuda and not tracked and self._blocks_win(m, tile=False) else "dense"
+            tile = self.backend != VQBackend.CUDA_LUT and m <= self._tile_max_tokens(tracked) and self._tile_band_ok(x, m, tracked)
+            if blocks and x.is_cuda and not tracked and self._blocks_win(m, tile):
+                return "blocks"
+            return "tile" if tile else "dense"
         # Ragged rows, where they are whole 16 bytes, are read where they lie.  Those that a permutation copies are padded on the way: the GEMV on
         # whole chunks is ahead (us per call, read as ragged rows / padded: 8000 x 4104 with 256 rows 7.9 / 7.4 at one token, 8.1 / 7.8 at 4).
         # Residual rows are never padded, see _kernel_res_stream, nor given to the tile GEMM (past 32 tokens, a raised band).
@@ -907,8 +908,6 @@ class NPVQLinear(nn.Module):
         from ..kernels import plans
 
         tile = band == "tile" or (band == "fused" and m > _GEMV_KERNEL_MAX_TOKENS)
-        if band == "tile" and self._blocks_win(m):
-            tile, band = False, "blocks"
         kind = "tile" if tile else "product" if band == "dense" and self._own_product(m, dtype) else band
         number = plan.names.get((kind, dtype))
         if number is None:
@@ -1374,13 +1373,16 @@ class NPVQLinear(nn.Module):
 
         try:
             own = self._own_product(x.numel() // self.in_features, x.dtype) and not kernels.tracked(x, self.bias)
+            # Ragged rows as they are only where nothing has taken the place of the product: one that has is given whole 64-column chunks.
+            padded = self._kernel_k() != self.in_features and (self.in_features % 8 or kernels.replaced("dense_linear"))
+            own = own and not (padded and self.is_residual)
             if self.is_residual:
                 w = kernels.rvq_dequant(
                     self.packed_indices, self.bits, self._res_stream(), self._res_bits(),
                     self.proxy.centroids, self._res_centroids(), self.row_scale, self.row_bias,
                     self.out_features, self.in_features, x.dtype,
                 )  # fmt: skip
-            elif own and self.in_features % 8:
+            elif own and padded:
                 stream, bits = self._kernel_stream()
                 w = kernels.vq_dequant(stream, self.proxy.centroids, bits, self.out_features, self._kernel_k(), x.dtype)
             else:
@@ -1453,27 +1455,42 @@ class NPVQLinear(nn.Module):
             "zero_cb", self.packed_indices, lambda: torch.zeros((1, self.vector_len), dtype=torch.float16, device=dev)
         )
 
-    def _fused(self, x: torch.Tensor, tile: bool, perm: torch.Tensor | None = None, blocks: bool = False) -> torch.Tensor:
+    def _forward_blocks(self, x: torch.Tensor) -> torch.Tensor:
+        """Any number of tokens and rows that end inside the last 64 columns: the GEMV with a workgroup per 32 tokens, or the table GEMM."""
+        from .. import kernels
+
+        x2d, width = x.reshape(-1, self.in_features), self._kernel_k()
+        main, bits = self._kernel_stream()
+        try:
+            if self.is_residual:
+                y = kernels.rvq_linear_blocks(
+                    x2d, main, bits, *self._kernel_res_stream(), self.proxy.centroids, self._res_centroids(), self.row_scale,
+                    self.row_bias, self.out_features, self._bias_f32(), width=width,
+                )  # fmt: skip
+            else:
+                y = kernels.vq_linear_blocks(x2d, main, self.proxy.centroids_as(x.dtype), bits, self.out_features, self._bias_f32(), width=width)
+        except RuntimeError as exc:
+            self._fallback("rvq_linear_blocks" if self.is_residual else "vq_linear_blocks", "decode + GEMM", exc)
+            return self._forward_dequant_gemm(x)
+        return y.reshape(*x.shape[:-1], self.out_features)
+
+    def _fused(self, x: torch.Tensor, tile: bool, perm: torch.Tensor | None = None) -> torch.Tensor:
         from .. import kernels
 
         *leading, _ = x.shape
         x2d = x.reshape(-1, self.in_features)
-        width = self._kernel_k() if blocks or (tile and self._blocks_win(x2d.shape[0])) else None
         if self.is_residual:
             (main, bits), (res, res_bits) = self._kernel_stream(), self._kernel_res_stream()
             y = kernels.rvq_linear(
                 x2d, main, bits, res, res_bits,
                 self.proxy.centroids, self._res_centroids(), self.row_scale, self.row_bias,
-                self.out_features, self._bias_f32(), tile=tile, width=width,
+                self.out_features, self._bias_f32(), tile=tile,
             )  # fmt: skip
         else:
             stream, bits = self._kernel_stream()
-            cb = self.proxy.centroids_as(x.dtype)
-            if width is not None:
-                fn = kernels.vq_gemm_tile if tile else kernels.vq_linear_blocks
-                return fn(x2d, stream, cb, bits, self.out_features, self._bias_f32(), width=width).reshape(*leading, self.out_features)
             if self._kernel_k() != self.in_features:
                 x2d = kernels.gather_columns(x2d, None, self._kernel_k())
+            cb = self.proxy.centroids_as(x.dtype)
             fn = kernels.vq_gemm_tile if tile else kernels.vq_linear
             if tile:
                 y = fn(x2d, stream, cb, bits, self.out_features, self._bias_f32())

@@ -132,3 +132,90 @@ def test_layers_against_the_other_bands(gpu, perm, monkeypatch):
         if getattr(layer, "bias", None) is not None and layer._band(x, m) == "blocks":
             layer.bias.requires_grad_()
             assert layer(x).requires_grad
+
+
+def test_replaced_wrappers_get_the_arguments_they_document(gpu, monkeypatch):
+    """A caller's function in the place of one that the blocks entries now and then stand in for is called with the arguments it has always
+    had, and undone again the layer is what it was."""
+    from neuropress_amd import kernels
+
+    monkeypatch.setattr(vqmod, "_TILE_MIN_GRID_FRACTION", 0.0)  # the tile GEMM's band without the blocks
+    monkeypatch.setattr(qmod, "_Q_TILE_MIN_GRID_FRACTION", 0.0)
+    seen = []
+
+    def spy(name, real):
+        def vq_gemm_tile(x, packed_indices, centroids, bits, out_features, bias=None):
+            seen.append(name)
+            return real(x, packed_indices, centroids, bits, out_features, bias)
+
+        def q_gemm_tile(x, w_pack, scale, nbits, group_size, zero_point=None, bias=None):
+            seen.append(name)
+            return real(x, w_pack, scale, nbits, group_size, zero_point, bias)
+
+        def rvq_linear(x, packed_main, bits_main, packed_res, bits_res, centroids_main, centroids_res, row_scale, row_bias, out_features,
+                       bias=None, tile=None):  # fmt: skip
+            seen.append(name)
+            return real(x, packed_main, bits_main, packed_res, bits_res, centroids_main, centroids_res, row_scale, row_bias, out_features,
+                        bias, tile=tile)  # fmt: skip
+
+        def dense_linear(x, w, bias=None):
+            seen.append(name)
+            return real(x, w, bias)
+
+        def rvq_dequant(*args):
+            seen.append(name)
+            return real(*args)
+
+        return {f.__name__: f for f in (vq_gemm_tile, q_gemm_tile, rvq_linear, dense_linear, rvq_dequant)}[name]
+
+    n, k = 1024, 4096
+    L = cases.vq_layer(1, n, k, 4096)
+    plain = NPVQLinear(VQProxy(L["cb"]).to(gpu), L["packed"], L["bits"], n, k, 8, "cuda_wmma").to(gpu)
+    R = cases.rvq_layer(1, n, k, 4096, 256, zipf=False)
+    res = NPVQLinear(VQProxy(R["cbm"]).to(gpu), R["pm"], R["bm"], n, k, 8, "cuda_wmma", residual_proxy=VQProxy(R["cbr"]).to(gpu),
+                     packed_residual=R["pr"], residual_bits=R["br"], row_scale=R["scale"], row_bias=R["wbias"]).to(gpu)  # fmt: skip
+    Q = cases.q4_layer(1, n, k)
+    q = NPLinear(Q["blob"], Q["scale"], n, k, 32, 4, "sym", "cuda").to(gpu)
+    S = cases.vq_layer(2, n, 2184, 65536)
+    ragged = NPVQLinear(VQProxy(S["cb"]).to(gpu), S["packed"], S["bits"], n, 2184, 8, "cuda_wmma").to(gpu)
+    T = cases.rvq_layer(2, n, 2184, 4096, 256, zipf=False)
+    ragged_res = NPVQLinear(VQProxy(T["cbm"]).to(gpu), T["pm"], T["bm"], n, 2184, 8, "cuda_wmma", residual_proxy=VQProxy(T["cbr"]).to(gpu),
+                            packed_residual=T["pr"], residual_bits=T["br"], row_scale=T["scale"], row_bias=T["wbias"]).to(gpu)  # fmt: skip
+    for layer, name, m, kk in ((plain, "vq_gemm_tile", 40, k), (q, "q_gemm_tile", 40, k), (res, "rvq_linear", 40, k), (res, "rvq_linear", 24, k),
+                               (ragged, "dense_linear", 600, 2184), (ragged_res, "rvq_dequant", 24, 2184), (ragged_res, "rvq_dequant", 600, 2184)):  # fmt: skip
+        x = torch.randn(m, kk, generator=cases.gen(m)).half().to(gpu)
+        before = layer(x)
+        seen.clear()
+        with monkeypatch.context() as mp:
+            mp.setattr(kernels, name, spy(name, getattr(kernels, name)))
+            during = layer(x)
+        assert seen == [name], (name, m, kk)
+        assert torch.allclose(before.float(), during.float(), rtol=2e-3, atol=2e-3), name
+        assert torch.equal(layer(x), before), name
+
+
+def test_a_blocks_entry_that_fails_leaves_the_tile_gemm_alone(gpu, monkeypatch):
+    """Where fallbacks are allowed: the call goes to decode + product, other layers keep the tile GEMM."""
+    from neuropress_amd import kernels
+
+    monkeypatch.setattr(vqmod, "_ALLOW_FALLBACK", True)
+    monkeypatch.setattr(vqmod, "_tile_failed", False)
+    monkeypatch.setattr(kernels, "_warned_fallbacks", set())
+
+    def fails(*args, **more):
+        raise RuntimeError("no such kernel")
+
+    n, k = 1024, 4096
+    for residual, kk, m in ((False, k, 40), (True, k, 40), (True, 2184, 3)):
+        L = cases.rvq_layer(1, n, kk, 4096, 256, zipf=False) if residual else cases.vq_layer(1, n, kk, 4096)
+        cb, packed, bits = (L["cbm"], L["pm"], L["bm"]) if residual else (L["cb"], L["packed"], L["bits"])
+        more = dict(residual_proxy=VQProxy(L["cbr"]).to(gpu), packed_residual=L["pr"], residual_bits=L["br"], row_scale=L["scale"],
+                    row_bias=L["wbias"]) if residual else {}  # fmt: skip
+        layer = NPVQLinear(VQProxy(cb).to(gpu), packed, bits, n, kk, 8, "cuda_wmma", **more).to(gpu)
+        x = torch.randn(m, kk, generator=cases.gen(m)).half().to(gpu)
+        assert layer._band(x, m) == "blocks"
+        before = layer(x)
+        with monkeypatch.context() as mp:
+            mp.setattr(kernels, "rvq_linear_blocks" if residual else "vq_linear_blocks", fails)
+            assert torch.allclose(layer(x).float(), before.float(), rtol=2e-3, atol=2e-3)
+        assert not vqmod._tile_failed and torch.equal(layer(x), before)
