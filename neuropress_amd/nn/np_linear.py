@@ -441,7 +441,8 @@ class NPLinear(nn.Module):
 
         if not 16 < m <= _Q_BLOCKS_MAX_TOKENS or self.out_features < 256 or min(_Q_FUSED_MAX_TOKENS, _Q_TILE_MAX_TOKENS) <= 0:
             return False
-
+        if self.u8_blob.data_ptr() % 16:
+            return False  # a slice of a larger buffer, say: the entry refuses it, the kernels it takes the place of serve it
         lines, _ = kernels.q_gemv_staging(
             _lib.GEMV_MAX_M, self.out_features, self.in_features, self.nbits, self.group_size, self.scale, self.zero_point
         )

@@ -840,7 +840,7 @@ class NPVQLinear(nn.Module):
         if self.column_perm is not None and self._perm_fusable(x, m):
             return "gemv_perm"
         ragged = self._kernel_k() != self.in_features
-        if x.is_cuda and (not self._mfma_layer() or (ragged and (tracked or (self.is_residual and not blocks)))):
+        if x.is_cuda and (not self._mfma_layer() or (ragged and (tracked or (self.is_residual and not (blocks and self._blocks_read()))))):
             # Shapes without an MFMA kernel (vector lengths other than 8 and 4, K not a
             # multiple of 64): the element-wise GEMV is slower than decoding once and calling
             # the dense GEMM at every token count (14336 x 4096: 99 us against 57 us at one token).
@@ -854,7 +854,7 @@ class NPVQLinear(nn.Module):
         # whole chunks is ahead (us per call, read as ragged rows / padded: 8000 x 4104 with 256 rows 7.9 / 7.4 at one token, 8.1 / 7.8 at 4).
         # Residual rows are never padded, see _kernel_res_stream, nor given to the tile GEMM (past 32 tokens, a raised band).
         short = ragged and (self.is_residual or (self.in_features % 8 == 0 and self.column_perm is None and m <= _GEMV_KERNEL_MAX_TOKENS))
-        return "blocks" if blocks and x.is_cuda and short else "fused"
+        return "blocks" if blocks and x.is_cuda and short and self._blocks_read() else "fused"
 
     # -- call plan ---------------------------------------------------------
 
@@ -1190,10 +1190,20 @@ class NPVQLinear(nn.Module):
             and (self.bits if self.bits in _FAST_BITS else 16, self._res_bits()) not in ((16, 8), (16, 16), (12, 8), (8, 8))
         ):  # fmt: skip
             return False
+        if not self._blocks_read():
+            return False
         from .. import kernels
 
         return kernels.gemv_blocks_preferred(m, self.out_features, self._kernel_k(), int(self.is_residual), self.proxy.num_centroids,
                                              self.column_perm is not None, tile)  # fmt: skip
+
+    def _blocks_read(self) -> bool:
+        """Whether the buffers start at 16-byte addresses (not slices of larger ones, say): the blocks entries refuse others, the kernels
+        they take the place of serve them."""
+        buffers = [self.packed_indices, self.proxy.centroids]
+        if self.is_residual:
+            buffers += [self._res_stream(), self._res_centroids()]
+        return all(t.data_ptr() % 16 == 0 for t in buffers)
 
     def _tile_ahead_from_17(self) -> bool:
         """Large layers with at least twice as many output as input features and a codebook kept in memory: the

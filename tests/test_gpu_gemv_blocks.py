@@ -219,3 +219,51 @@ def test_a_blocks_entry_that_fails_leaves_the_tile_gemm_alone(gpu, monkeypatch):
             mp.setattr(kernels, "rvq_linear_blocks" if residual else "vq_linear_blocks", fails)
             assert torch.allclose(layer(x).float(), before.float(), rtol=2e-3, atol=2e-3)
         assert not vqmod._tile_failed and torch.equal(layer(x), before)
+
+
+def _at_odd_addresses(t):
+    """The same values in a contiguous tensor that starts 4 bytes behind a 16-byte address."""
+    flat = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)
+    out = flat[4 // t.element_size():][: t.numel()].view(t.shape)
+    out.copy_(t)
+    return out
+
+
+@pytest.mark.parametrize("odd", ["packed", "codebook", "residual"])
+def test_vq_weights_at_any_address(gpu, odd):
+    """Buffers that start between two 16-byte addresses, at every band, planned or not."""
+    for n, k, residual in ((512, 2048, False), (512, 2048, True), (512, 2040, False), (512, 2040, True)):
+        if odd == "residual" and not residual:
+            continue
+        move = lambda t, name: _at_odd_addresses(t.to(gpu)) if odd == name else t.to(gpu)
+        if residual:
+            L = cases.rvq_layer(n + k, n, k, 4096, 256, zipf=False)
+            w = ((L["cbm"][L["im"]] + L["cbr"][L["ir"]]).reshape(n, k) * L["scale"][:, None] + L["wbias"][:, None]).float()
+            layer = NPVQLinear(VQProxy(move(L["cbm"], "codebook")), move(L["pm"], "packed"), L["bm"], n, k, 8, "cuda_wmma",
+                               residual_proxy=VQProxy(move(L["cbr"], "residual")), packed_residual=move(L["pr"], "residual"),
+                               residual_bits=L["br"], row_scale=L["scale"].to(gpu), row_bias=L["wbias"].to(gpu))  # fmt: skip
+        else:
+            L = cases.vq_layer(n + k, n, k, 1000)
+            w = L["cb"][L["idx"]].reshape(n, k).float()
+            layer = NPVQLinear(VQProxy(move(L["cb"], "codebook")), move(L["packed"], "packed"), L["bits"], n, k, 8, "cuda_wmma")
+        for m in (1, 20, 40, 100, 300):
+            x = torch.randn(m, k, generator=cases.gen(m)).half()
+            ref = x.float() @ w.T
+            for _ in range(2):
+                err = (layer(x.to(gpu)).float().cpu() - ref).abs()
+                assert bool((err <= 1e-2 + 1e-2 * ref.abs()).all()), (k, residual, m, float(err.max()))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_group_quantized_weights_at_any_address(gpu, bits):
+    n, k = 512, 2048
+    Q = cases.q4_layer(n + k, n, k, nbits=bits)
+    layer = NPLinear(_at_odd_addresses(Q["blob"].to(gpu)), Q["scale"].to(gpu), n, k, 32, bits, "sym", "cuda")
+    assert layer.u8_blob.data_ptr() % 16
+    w = ((Q["codes"].float() - (1 << (bits - 1))).reshape(n, k // 32, 32) * Q["scale"].float().reshape(n, k // 32, 1)).reshape(n, k).half().float()
+    for m in (1, 20, 40, 100, 300):
+        x = torch.randn(m, k, generator=cases.gen(m)).half()
+        ref = x.float() @ w.T
+        for _ in range(2):
+            err = (layer(x.to(gpu)).float().cpu() - ref).abs()
+            assert bool((err <= 1e-2 + 1e-2 * ref.abs()).all()), (m, float(err.max()))
