@@ -241,11 +241,12 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   const int64_t ldx_in = ldx;
   bool with_gather = false;
   const bool blocks = t.kind == kVqBlocks || t.kind == kRvqBlocks || t.kind == kQBlocks;
-  const bool readable = ldx % 8 == 0 && ((uintptr_t)x_in.const_data_ptr() & 15) == 0;  // 16 bytes at a time, where it lies
+  // The package's product and the blocks entries read 16 bytes at a time: rows that do not start at such addresses are copied first.
+  const bool copied = (blocks || t.own) && (ldx % 8 || ((uintptr_t)x_in.const_data_ptr() & 15));
   if (t.perm.defined() && t.perm.scalar_type() == at::kLong) {
     x = at::index_select(x_in, -1, t.perm);
     ldx = t.k;
-  } else if (t.perm.defined() || (t.k_in != t.k && !(blocks && readable))) {
+  } else if (t.perm.defined() || copied || (t.k_in != t.k && !blocks)) {
     sizes.back() = t.k;
     x = empty(sizes, x_in.scalar_type(), device);
     with_gather = t.kind == kVqDense && t.own;  // its decode gathers them too
@@ -259,7 +260,6 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
 
   if (t.kind == kVqDense || t.kind == kRvqDense || t.kind == kQDense) {
     const int code = dtype_code(t.out);
-    if (t.own && (ldx % 8 || ((uintptr_t)x.const_data_ptr() & 15))) return false;
     at::Tensor w = empty({t.n, t.k}, t.out, device);
     int rc;
     if (with_gather)

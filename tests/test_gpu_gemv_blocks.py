@@ -267,3 +267,28 @@ def test_group_quantized_weights_at_any_address(gpu, bits):
         for _ in range(2):
             err = (layer(x.to(gpu)).float().cpu() - ref).abs()
             assert bool((err <= 1e-2 + 1e-2 * ref.abs()).all()), (m, float(err.max()))
+
+
+@pytest.mark.parametrize("form,n,k,m,band", [("vq", 1157, 680, 471, "dense"), ("rvq", 1157, 680, 471, "dense"), ("vq", 1024, 4096, 600, "dense"),
+                                             ("table", 512, 2048, 100, "blocks"), ("rvq", 512, 2048, 40, "blocks"), ("rvq", 512, 680, 3, "blocks"),
+                                             ("q", 512, 2048, 40, "blocks"), ("q", 1024, 4096, 900, "dense")])  # fmt: skip
+def test_rows_at_odd_addresses_stay_with_the_plan(gpu, form, n, k, m, band):
+    """The package's product and the blocks entries read whole 16 bytes: a planned call copies rows at other addresses or distances first."""
+    if form == "q":
+        L = cases.q4_layer(n, n, k)
+        layer = NPLinear(L["blob"], L["scale"], n, k, 32, 4, "sym", "cuda").to(gpu)
+    elif form == "rvq":
+        L = cases.rvq_layer(n, n, k, 4096, 256, zipf=False)
+        layer = NPVQLinear(VQProxy(L["cbm"]).to(gpu), L["pm"], L["bm"], n, k, 8, "cuda_wmma", residual_proxy=VQProxy(L["cbr"]).to(gpu),
+                           packed_residual=L["pr"], residual_bits=L["br"], row_scale=L["scale"], row_bias=L["wbias"]).to(gpu)  # fmt: skip
+    else:
+        L = cases.vq_layer(n, n, k, 4096 if form == "table" else 65536)
+        layer = NPVQLinear(VQProxy(L["cb"]).to(gpu), L["packed"], L["bits"], n, k, 8, "cuda_wmma").to(gpu)
+    base = torch.randn(m, k + 3, generator=cases.gen(m)).half().to(gpu)
+    x = base[:, :k]
+    assert layer._band(x, m) == band and (band == "blocks" or layer._own_product(m, x.dtype))
+    expect = layer(x.contiguous())
+    shifted = torch.empty(m * k + 1, dtype=x.dtype, device=gpu)[1:].view(m, k).copy_(x)
+    for given in (x, shifted):  # at an odd distance, from an odd address
+        planned = layer._plan.run(given)
+        assert planned is not None and torch.equal(planned, expect) and torch.equal(layer(given), expect)
