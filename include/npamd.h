@@ -43,6 +43,10 @@ extern "C" {
  * element-wise kernels take further passes over the weight instead). */
 #define NPAMD_GEMV_MAX_M 32
 
+/* The dense product refuses rows this many elements apart or more (offsets into a tile of up to 256 rows have 32 bits), and the
+ * *_gemv_blocks entry points do not give them to tiles. */
+#define NPAMD_TILE_MAX_STRIDE (1 << 22)
+
 /* Library ABI version (bumped on any signature change). */
 int npamd_version(void);
 

@@ -16,6 +16,7 @@ HOST_PATH = LIB_PATH.with_name("npamd_host.so")
 
 F16, BF16, F32 = 0, 1, 2
 GEMV_MAX_M = 32
+TILE_MAX_STRIDE = 1 << 22
 ABI_VERSION = 3
 
 _vp = ctypes.c_void_p

@@ -338,7 +338,7 @@ int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
 }
 
 constexpr int kDenseMaxSplits = 16;
-constexpr int64_t kDenseStrideMax = 1 << 22;  // elements between rows: offsets into a tile (256 rows) have 32 bits
+constexpr int64_t kDenseStrideMax = NPAMD_TILE_MAX_STRIDE;
 constexpr int kDenseMinSplitSteps = 4;  // 64-k steps of a part
 // What a split adds: the reduction kernel and the gap in front of it, and its bytes, us and us per MB.
 constexpr float kSplitFixed = 4.5f, kSplitPerMb = 0.45f;

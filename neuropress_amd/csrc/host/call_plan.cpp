@@ -241,8 +241,8 @@ bool issue(const Template& t, const Route& r, const at::Tensor& x_in, int64_t m,
   const int64_t ldx_in = ldx;
   bool with_gather = false;
   const bool blocks = t.kind == kVqBlocks || t.kind == kRvqBlocks || t.kind == kQBlocks;
-  // The package's product and the blocks entries read 16 bytes at a time: rows that do not start at such addresses are copied first.
-  const bool copied = (blocks || t.own) && (ldx % 8 || ((uintptr_t)x_in.const_data_ptr() & 15));
+  // The package's product and the blocks entries read 16 bytes at a time: rows that do not start at such addresses, or lie too far apart, are copied first.
+  const bool copied = (blocks || t.own) && (ldx % 8 || ldx >= NPAMD_TILE_MAX_STRIDE || ((uintptr_t)x_in.const_data_ptr() & 15));
   if (t.perm.defined() && t.perm.scalar_type() == at::kLong) {
     x = at::index_select(x_in, -1, t.perm);
     ldx = t.k;

@@ -354,7 +354,8 @@ int launch_table(const VqCall& c, int tile) {
 // compute unit take `pair` times as long as one.  The figures are those of 16-bit indices, which take the most LDS.
 TablePlan plan_table_gemm(int M, int N, int K, int nc) {
   TablePlan best{-1, 1e30f};
-  if (M <= 16 || N < 1 || K < 64 || K % 64 || K > kTableMaxK || nc < 1 || nc * 16 > kTileLdsCodebookMax) return best;
+  const int forced = tuning().table_tile, twos = (K / 64 + 1) / 2;
+  if (forced < 0 || M <= 16 || N < 1 || K < 64 || K % 64 || K > kTableMaxK || nc < 1 || nc * 16 > kTileLdsCodebookMax) return best;
   constexpr struct { float fixed, round, step, crowded, table, pair; } kCost[kTableTiles] = {
       {2.85f, 1.11f, 0.468f, 0.226f, 3.3f, 1.66f},
       {2.10f, 2.51f, 0.679f, 0.309f, 3.2f, 1.5f},
@@ -362,7 +363,6 @@ TablePlan plan_table_gemm(int M, int N, int K, int nc) {
       {1.70f, 3.28f, 0.592f, 0.105f, 3.1f, 1.5f},
       {1.62f, 3.95f, 0.727f, 0.190f, 3.3f, 1.5f},
   };
-  const int forced = tuning().table_tile, twos = (K / 64 + 1) / 2;
   for (int i = 0; i < kTableTiles; ++i) {
     if (table_lds(i, 16, nc) > kLdsPerBlockMax || (forced > 0 && i != forced - 1)) continue;
     const auto& t = kTableTile[i];
@@ -377,10 +377,9 @@ TablePlan plan_table_gemm(int M, int N, int K, int nc) {
 }
 
 int launch_table_gemm(const VqCall& c, float other_us) {
-  const int forced = tuning().table_tile;
-  if (forced < 0 || c.packed_r || c.vl != 8 || c.cb_dtype != c.act || c.ldx >= (1 << 22) || (c.bits != 8 && c.bits != 12 && c.bits != 16)) return 1;
+  if (c.packed_r || c.vl != 8 || c.cb_dtype != c.act || c.ldx >= NPAMD_TILE_MAX_STRIDE || (c.bits != 8 && c.bits != 12 && c.bits != 16)) return 1;
   const TablePlan p = plan_table_gemm(c.M, c.N, c.K, c.nc);
-  if (p.tile < 0 || (!forced && p.us >= other_us)) return 1;
+  if (p.tile < 0 || (tuning().table_tile == 0 && p.us >= other_us)) return 1;
   return c.act == NPAMD_BF16 ? launch_table<NPAMD_BF16>(c, p.tile) : launch_table<NPAMD_F16>(c, p.tile);
 }
 

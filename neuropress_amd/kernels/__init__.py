@@ -99,8 +99,8 @@ def _rows(x: torch.Tensor) -> torch.Tensor:
 
 
 def _aligned_rows(x: torch.Tensor) -> torch.Tensor:
-    """2-D *x* with rows that start at 16-byte addresses, copied where they do not."""
-    if x.stride(0) % 8 or x.data_ptr() % 16:
+    """2-D *x* with rows that start at 16-byte addresses and not too far apart for the tile kernels, copied where they do not."""
+    if x.stride(0) % 8 or x.data_ptr() % 16 or x.stride(0) >= _lib.TILE_MAX_STRIDE:
         x = torch.clone(x, memory_format=torch.contiguous_format)  # .contiguous() keeps dense rows at any address
     return x
 
@@ -976,8 +976,7 @@ def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = N
     x = _x2d(x, what)
     if x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype or w.dim() != 2 or w.shape[1] != x.shape[1]:
         raise RuntimeError(f"{what}: x and w must be float16 or bfloat16 [M, K] and [N, K]")
-    if x.stride(0) % 8 or x.data_ptr() % 16 or x.stride(0) >= 1 << 22:
-        x = torch.clone(x, memory_format=torch.contiguous_format)  # .contiguous() keeps dense rows at any address
+    x = _aligned_rows(x)
     m, k = x.shape
     n = w.shape[0]
     w = w.contiguous()

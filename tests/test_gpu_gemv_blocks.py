@@ -292,3 +292,20 @@ def test_rows_at_odd_addresses_stay_with_the_plan(gpu, form, n, k, m, band):
     for given in (x, shifted):  # at an odd distance, from an odd address
         planned = layer._plan.run(given)
         assert planned is not None and torch.equal(planned, expect) and torch.equal(layer(given), expect)
+
+
+def test_rows_too_far_apart_for_tiles_are_copied(gpu):
+    """A layer routed to the table GEMM keeps it: its rows' offsets have 32 bits, the GEMV in its place would decode the weight per 32 tokens."""
+    n, k, m, apart = 4096, 2048, 100, 1 << 22
+    L = cases.vq_layer(n, n, k, 4096)
+    layer = NPVQLinear(VQProxy(L["cb"]).to(gpu), L["packed"], L["bits"], n, k, 8, "cuda_wmma").to(gpu)
+    far = torch.empty(m * apart, dtype=torch.half, device=gpu).view(m, apart)[:, :k].copy_(torch.randn(m, k, generator=cases.gen(m)))
+    expect = layer(far.contiguous())
+    planned = layer._plan.run(far)
+    assert layer._band(far, m) == "blocks" and planned is not None and torch.equal(planned, expect)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):  # not by the plan
+        captured = layer(far)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(captured, expect)

@@ -21,6 +21,21 @@ def test_every_tile_is_the_best_somewhere():
         assert plan(m, n, k, rows) == -1
 
 
+def test_switched_off_it_is_not_what_the_band_line_counts_on(monkeypatch):
+    """The line that sends calls to the blocks entry and the entry itself ask the same plan."""
+    from neuropress_amd import _lib
+
+    lib = _lib.load()
+    large = ((384, 14336, 14336, 4096), (256, 9856, 12544, 256), (1024, 4096, 4096, 1000))
+    assert all(lib.npamd_gemv_blocks_preferred(m, n, k, 0, rows, 0, 1) == 1 for m, n, k, rows in large)
+    with monkeypatch.context() as mp:
+        mp.setenv("NPAMD_TABLE_TILE", "-1")
+        lib.npamd_diag_reload_tuning()
+        off = [(lib.npamd_gemv_blocks_preferred(m, n, k, 0, rows, 0, 1), lib.npamd_diag_table_tile(m, n, k, rows)) for m, n, k, rows in large]
+    lib.npamd_diag_reload_tuning()
+    assert off == [(0, -1)] * len(large)
+
+
 @pytest.fixture(params=range(1, len(TILES) + 1))
 def forced(request, monkeypatch):
     from neuropress_amd import _lib
