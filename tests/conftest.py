@@ -32,3 +32,12 @@ def gpu():
 
     _lib.load()  # raises RuntimeError: a GPU box without the kernel library is an error
     return torch.device("cuda:0")
+
+
+@pytest.fixture(autouse=True)
+def _tuning_ends_with_the_test():
+    """The library reads the NPAMD_* variables once: what a test set of them is read again behind its monkeypatch, so that no later test runs with it."""
+    yield
+    lib = getattr(sys.modules.get("neuropress_amd._lib"), "_lib", None)
+    if lib is not None:
+        lib.npamd_diag_reload_tuning()
