@@ -49,13 +49,6 @@ struct GemvShape {
 // small layer the grid of one launch then fills the compute units that the rows alone leave empty, and the call is over in
 // the time that decode + product spend on being two launches (npamd_gemv_blocks_preferred has the figures).
 constexpr int kGemvTokens = 32;
-__device__ __forceinline__ GemvShape gemv_token_block(GemvShape s) {
-  const int m0 = blockIdx.y * kGemvTokens;
-  s.M = min(s.M - m0, kGemvTokens);
-  s.x = reinterpret_cast<const uint16_t*>(s.x) + (int64_t)m0 * s.ldx;
-  s.y = reinterpret_cast<uint16_t*>(s.y) + (int64_t)m0 * s.ldy;
-  return s;
-}
 
 // Largest M * K (elements) whose activations the GEMV stages in LDS (32 KiB; the unpermuted
 // copy shares its place with the codebook of up to 64 KiB).
@@ -115,12 +108,17 @@ struct GemvStageLines {
 constexpr int kGemvTurnBytes = 2048;
 template <class Provider, int R, bool CB_LDS, int H>
 constexpr bool gemv_loads_lines = Provider::kLdsResidual && CB_LDS && R == 1 && H == 1;
-template <int ACT, class Provider, int R, bool CB_LDS, bool X_LDS, int MT = 1, int H = 1, bool XS = false>
+// SHORT (XS kernels): rows of x end inside the last chunk.  A kernel of its own, as what it does for that -- masks per 16-byte piece in the place of one
+// per chunk -- costs whole rows 1 to 3 % (us: 14336 x 4096 with 65536 rows, Zipf, at 32 tokens 28.5 / 27.9, residual 4096 x 14336 at 24 27.5 / 27.3).
+template <int ACT, class Provider, int R, bool CB_LDS, bool X_LDS, int MT = 1, int H = 1, bool XS = false, bool SHORT = false>
 __global__ void __launch_bounds__((kGemvMaxWaves<R, MT> * 64))
-fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
-  const GemvShape s = gemv_token_block(all);
+fused_gemv_kernel(const GemvShape s, const typename Provider::Args pargs) {
+  // This block's tokens: M of them from m0 on.  Up to 16 are one block, whose kernels do nothing for it; shifted pointers, worked out in front of
+  // everything else, cost every call (8192 x 8192 with 65536 rows, Zipf, at 9 tokens 20.8 / 20.0 us, 3003 x 2176 at 4 7.7 / 7.4).
+  const int m0 = MT == 1 ? 0 : blockIdx.y * kGemvTokens, M = MT == 1 ? s.M : min(s.M - m0, kGemvTokens);
   static_assert(H == 1 || ((H == 2 || H == 4) && R == 1 && MT == 1), "k parts only with one row tile and one token tile");
   constexpr bool kStageLines = CB_LDS && Provider::kLdsCodebook;
+  static_assert(!SHORT || XS, "rows that end inside a chunk: the kernels that stage activations");
   static_assert(!XS || (!X_LDS && (kStageLines ? H == 1 : R == 1)), "staged activations: the forms there are");
   constexpr bool kLines = gemv_loads_lines<Provider, R, CB_LDS, H>;
   constexpr int RT = 16 / H;  // weight rows (and tokens) per MFMA tile
@@ -132,7 +130,7 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
   // LDS after the reduction buffer (16-byte aligned): the codebook copy, then the copy of x.
   // While x is being permuted its unpermuted copy lies where the codebook goes afterwards, so
   // the region in front of x is max(codebook, x) bytes.
-  const int red_floats = (n_waves * s.M * 16 * R + 3) & ~3;
+  const int red_floats = (n_waves * M * 16 * R + 3) & ~3;
   // Without a copy of x the reduction buffer, needed only after the loop, lies over the codebook.
   constexpr bool kRedOverCodebook = CB_LDS && !X_LDS;
   uint8_t* const lds0 = reinterpret_cast<uint8_t*>(red) + (kRedOverCodebook ? 0 : red_floats * (int)sizeof(float));
@@ -145,17 +143,16 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
     // cheaper from LDS than through the vector memory path, and every block needs all of them.
     const int K = s.chunks * 64;
     const int k8s = s.chunks * 8;  // 8-element pieces per row
-    const int items = s.M * k8s;
-    const int x_bytes = s.M * K * 2;
+    const int items = M * k8s;
+    const int x_bytes = M * K * 2;
     uint16_t* const xs = reinterpret_cast<uint16_t*>(lds0 + (s.perm ? max(cb_lds_bytes, x_bytes) : cb_lds_bytes));
     uint16_t* const xraw = s.perm ? reinterpret_cast<uint16_t*>(lds0) : xs;
     const uint16_t* xg = reinterpret_cast<const uint16_t*>(s.x);
     for (int i = threadIdx.x; i < items; i += blockDim.x) {
       const int m = i / k8s;
       const int k8 = i - m * k8s;
-      u32x4 v = *reinterpret_cast<const u32x4*>(xg + (int64_t)m * s.ldx + min(k8, s.pieces - 1) * 8);
-      if (k8 >= s.pieces) v = u32x4{0, 0, 0, 0};
-      *reinterpret_cast<u32x4*>(xraw + (int64_t)i * 8) = v;
+      *reinterpret_cast<u32x4*>(xraw + (int64_t)i * 8) =
+          *reinterpret_cast<const u32x4*>(xg + (int64_t)m * s.ldx + k8 * 8);
     }
     if (s.perm) {
       __syncthreads();
@@ -163,14 +160,13 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
         const int m = i / k8s;
         const int k8 = i - m * k8s;
         const uint16_t* xr = xraw + (int64_t)m * K;
-        const u32x4 p0 = *reinterpret_cast<const u32x4*>(s.perm + min(k8, s.pieces - 1) * 8);
-        const u32x4 p1 = *reinterpret_cast<const u32x4*>(s.perm + min(k8, s.pieces - 1) * 8 + 4);
+        const u32x4 p0 = *reinterpret_cast<const u32x4*>(s.perm + k8 * 8);
+        const u32x4 p1 = *reinterpret_cast<const u32x4*>(s.perm + k8 * 8 + 4);
         u32x4 v;
         v.x = (uint32_t)xr[p0.x] | ((uint32_t)xr[p0.y] << 16);
         v.y = (uint32_t)xr[p0.z] | ((uint32_t)xr[p0.w] << 16);
         v.z = (uint32_t)xr[p1.x] | ((uint32_t)xr[p1.y] << 16);
         v.w = (uint32_t)xr[p1.z] | ((uint32_t)xr[p1.w] << 16);
-        if (k8 >= s.pieces) v = u32x4{0, 0, 0, 0};
         *reinterpret_cast<u32x4*>(xs + (int64_t)i * 8) = v;
       }
       if constexpr (CB_LDS) __syncthreads();  // the codebook overwrites the unpermuted copy
@@ -195,10 +191,10 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
   // Two tokens per instruction straight into LDS, past M and K the last row and piece again.
   auto stage_lines = [&](int step) {
     using SL = GemvStageLines;
-    const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)red + (uint32_t)(s.stage_offset + wave * SL::bytes(s.M));
-    for (int at = 0; at < SL::bytes(s.M); at += 1024) {
+    const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)red + (uint32_t)(s.stage_offset + wave * SL::bytes(M));
+    for (int at = 0; at < SL::bytes(M); at += 1024) {
       const int row = at / 512 + (lane >> 5), piece = SL::slot(lane & 31, row);
-      const uint16_t* src = reinterpret_cast<const uint16_t*>(s.x) + (int64_t)min(row, s.M - 1) * s.ldx + min(step * 32 + piece, s.pieces - 1) * 8;
+      const uint16_t* src = reinterpret_cast<const uint16_t*>(s.x) + (int64_t)(m0 + min(row, M - 1)) * s.ldx + min(step * 32 + piece, s.pieces - 1) * 8;
       // The statement writes m0: see the codebook's copy.
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(
                        __builtin_amdgcn_readfirstlane(mine + (uint32_t)at)), "v"(src) : "memory");
@@ -206,8 +202,9 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
   };
   // Next to a table in LDS, activations staged: the first step's packed bytes and activations are asked for in front of the
   // table, whose copy waits for all of them at once.  Both at 17 and more tokens, us before / now (24 tokens): 512 x 2048 with 256 rows
-  // 6.0 / 4.8, 1024 x 4096 9.5 / 6.4, 14336 x 4096 15.6 / 13.7 with 256 rows and 16.0 / 14.7 with 4096.
-  constexpr bool kFirstAhead = XS && kStageLines && (R == 1 || MT == 2);  // two row tiles within 128 registers: no room
+  // 6.0 / 4.8, 1024 x 4096 9.5 / 6.4.  Up to 16 tokens the branch in the loop costs more than it saves (us with / without: 4096 x 14336 with 4096
+  // rows at 8 tokens 11.9 / 10.9, with 256 rows at one 8.6 / 8.1).
+  constexpr bool kFirstAhead = XS && kStageLines && MT == 2;
   if constexpr (kFirstAhead) {
     if (step_begin < step_end) {
       load_packed(step_begin);
@@ -261,20 +258,19 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
   bool x_lane[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const int x_row = min(16 * t + cr, s.M - 1);
+    const int x_row = min(16 * t + cr, M - 1);
     xrow[t] = X_LDS ? x_lds + (int64_t)x_row * (s.chunks * 64)
-                    : reinterpret_cast<const uint16_t*>(s.x) + (int64_t)x_row * s.ldx;
-    x_lane[t] = 16 * t + cr < s.M;
+                    : reinterpret_cast<const uint16_t*>(s.x) + (int64_t)(m0 + x_row) * s.ldx;
+    x_lane[t] = 16 * t + cr < M;
   }
   const u32x4 zero4{0, 0, 0, 0};
   if constexpr (kLines) prov.prepare_row(min(row0 + c, s.N - 1));
 
   for (int step = step_begin; step < step_end; ++step) {
     const int kc_raw = (step * 4 + q) * H + part;
-    // Whether piece j of the chunk lies in front of the end of K, in kernels that take rows of x which end inside a chunk.
-    constexpr bool kShortRows = XS || X_LDS;
     const bool kvalid = kc_raw < s.chunks;
-    auto there = [&](int j) { return kShortRows ? kc_raw * 8 + j < s.pieces : kvalid; };
+    const int left = s.pieces - kc_raw * 8;  // pieces of the chunk in front of the end of K (SHORT)
+    auto there = [&](int j) { return SHORT ? j < left : kvalid; };
     const int kc = min(kc_raw, s.chunks - 1);
 
     if (!kFirstAhead || step != step_begin) load_packed(step);
@@ -287,7 +283,7 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
     u32x4 xa[MT][8];
     if constexpr (XS && kStageLines) {
       using SL = GemvStageLines;
-      const uint8_t* const mine = reinterpret_cast<const uint8_t*>(red) + s.stage_offset + wave * SL::bytes(s.M);
+      const uint8_t* const mine = reinterpret_cast<const uint8_t*>(red) + s.stage_offset + wave * SL::bytes(M);
       if (!kFirstAhead || step != step_begin) {
         // The step before has read its activations out (its products waited for them).
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -296,7 +292,7 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
       }
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
-        const int row = min(16 * t + cr, s.M - 1);
+        const int row = min(16 * t + cr, M - 1);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           xa[t][j] = *reinterpret_cast<const u32x4*>(mine + row * 512 + SL::slot(q * 8 + j, row) * 16);
@@ -314,10 +310,10 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {  // 1 KiB per instruction of the tile's RT x kRowData bytes
           const int flat = i * 1024 + lane * 16;
-          const int row = min(RT * t + flat / SL::kRowData, s.M - 1);
+          const int row = min(RT * t + flat / SL::kRowData, M - 1);
           const int off = flat % SL::kRowData;
           const int piece = min(step * 32 * H + off / 16, s.pieces - 1);
-          tmp[t * 8 + i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(s.x) + (int64_t)row * s.ldx + piece * 8);
+          tmp[t * 8 + i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(s.x) + (int64_t)(m0 + row) * s.ldx + piece * 8);
         }
 #pragma unroll
       for (int t = 0; t < MT; ++t)
@@ -360,7 +356,7 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
       b[r][6] = prov.template operand<6>(raw[r]);
       b[r][7] = prov.template operand<7>(raw[r]);
     }
-    if (s.chunks % (4 * H) || (kShortRows && s.pieces % 8)) {  // uniform: only shapes with a ragged last step pay for the select
+    if (s.chunks % (4 * H) || (SHORT && s.pieces % 8)) {  // uniform: only shapes with a ragged last step pay for the select
 #pragma unroll
       for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -387,20 +383,20 @@ fused_gemv_kernel(const GemvShape all, const typename Provider::Args pargs) {
       for (int i = 0; i < 4; ++i) {
         const int mp = 4 * q + i;
         const int m = 16 * t + (mp & (RT - 1));
-        if (m < s.M && mp / RT == part)
-          red[((int64_t)(wave * H + part) * s.M + m) * cols + r * 16 + cr] = acc[r][t][i];
+        if (m < M && mp / RT == part)
+          red[((int64_t)(wave * H + part) * M + m) * cols + r * 16 + cr] = acc[r][t][i];
       }
   }
   __syncthreads();
-  for (int o = threadIdx.x; o < s.M * cols; o += blockDim.x) {
+  for (int o = threadIdx.x; o < M * cols; o += blockDim.x) {
     const int m = o / cols;
     const int col = o - m * cols;
     const int n = row0 + col;
     if (n >= s.N) continue;
     float v = 0.f;
-    for (int w = 0; w < n_waves * H; ++w) v += red[((int64_t)w * s.M + m) * cols + col];
+    for (int w = 0; w < n_waves * H; ++w) v += red[((int64_t)w * M + m) * cols + col];
     if (s.bias) v += s.bias[n];
-    store_from_f32<ACT>(s.y, (int64_t)m * s.ldy + n, v);
+    store_from_f32<ACT>(s.y, (int64_t)(m0 + m) * s.ldy + n, v);
   }
 }
 
@@ -446,7 +442,7 @@ bool gemv_lds_activations_forced();  // NPAMD_GEMV_LDS_X=1: stage x in LDS also 
 template <int ACT, class Provider, int R, bool CB_LDS, bool X_LDS = false, int MT = 1, int H = 1, bool XS = false>
 int launch_fused_gemv_r(GemvShape s, const typename Provider::Args& pargs, const GemvPlan& plan,
                         int cb_bytes, hipStream_t st, const char* what) {
-  if (!XS && !X_LDS && s.pieces < s.chunks * 8)
+  if (!(XS && Provider::kGathers) && s.pieces < s.chunks * 8)
     return fail(NPAMD_ERR_UNSUPPORTED, "%s: rows of x that end inside a chunk need a kernel that stages them", what);
   s.steps_per_wave = plan.steps_per_wave;
   const int M = s.M < kGemvTokens ? s.M : kGemvTokens;  // of a block
@@ -484,15 +480,18 @@ int launch_fused_gemv_r(GemvShape s, const typename Provider::Args& pargs, const
     *s.plan_only = XS ? 1 : 0;
     return 0;
   }
+  auto* kernel = fused_gemv_kernel<ACT, Provider, R, CB_LDS, X_LDS, MT, H, XS>;
+  const bool short_rows = s.pieces < s.chunks * 8;
+  if constexpr (XS && Provider::kGathers)
+    if (short_rows) kernel = fused_gemv_kernel<ACT, Provider, R, CB_LDS, X_LDS, MT, H, XS, true>;
   if (lds > 64 * 1024) {
-    static LdsLatch latch;  // per instantiation
-    const hipError_t e = enable_dynamic_lds(
-        latch, reinterpret_cast<const void*>(&fused_gemv_kernel<ACT, Provider, R, CB_LDS, X_LDS, MT, H, XS>), lds);
+    static LdsLatch latches[2];  // per instantiation
+    const hipError_t e = enable_dynamic_lds(latches[short_rows], reinterpret_cast<const void*>(kernel), lds);
     if (e != hipSuccess)
       return fail(NPAMD_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, lds, hipGetErrorString(e));
   }
   last_gemv_staged() = XS ? 1 : 0;
-  launch(fused_gemv_kernel<ACT, Provider, R, CB_LDS, X_LDS, MT, H, XS>, dim3(blocks, (s.M + kGemvTokens - 1) / kGemvTokens), plan.waves * 64, lds, st, s, pargs);
+  launch(kernel, dim3(blocks, (s.M + kGemvTokens - 1) / kGemvTokens), plan.waves * 64, lds, st, s, pargs);
   return check_launch(what);
 }
 
@@ -507,7 +506,7 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
                       const char* what, int cb_bytes = 0) {
   s.steps = (s.chunks + 3) / 4;
   if (s.pieces == 0) s.pieces = s.chunks * 8;
-  // Rows of x that end inside the last chunk: the kernels that stage activations, and those that copy x, look where they end.
+  // Rows of x that end inside the last chunk: the kernels that stage activations look where they end.
   const bool short_rows = s.pieces < s.chunks * 8;
   auto stages = [&](int tokens) { return short_rows || gemv_stage_activations(tokens); };
   // Layers of few rows, few tokens: 16 / H rows x H parts of k per tile (see the kernel).
@@ -535,7 +534,7 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
     }
   }
   if (short_rows && whole_codebook_in_lds) h = 1;
-  if (h > 1 && !s.perm && !gemv_lds_activations_forced()) {
+  if (h > 1 && !s.perm && (short_rows || !gemv_lds_activations_forced())) {
     s.steps = (s.chunks + 4 * h - 1) / (4 * h);
     const GemvPlan plan = plan_gemv_rows(s.N, 16 / h, s.steps);
     // Staged activations as for whole tiles, except next to a whole codebook in LDS (2048 x 2048 at 8 tokens 4.0 / 4.3 us).
@@ -611,7 +610,7 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
   const GemvPlan plan = plan_gemv(s.N, s.chunks, short_rows && !s.perm ? (cb_in_lds ? 2 : 1) : (Provider::kGathers && !cb_in_lds) ? 2 : 4);
   if constexpr (Provider::kLdsCodebook) {
     const bool x_fits = (int64_t)s.M * s.chunks * 64 <= kGemvLdsActivationsMax;
-    if (s.perm || (x_fits && gemv_lds_activations_forced())) {  // with a permutation the caller has checked the size
+    if (s.perm || (x_fits && !short_rows && gemv_lds_activations_forced())) {  // with a permutation the caller has checked the size
       if (cb_in_lds) {
         if (plan.R == 4) return launch_fused_gemv_r<ACT, Provider, 4, true, true>(s, pargs, plan, cb_bytes, st, what);
         if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, true, true>(s, pargs, plan, cb_bytes, st, what);

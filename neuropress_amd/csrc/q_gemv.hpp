@@ -48,13 +48,24 @@ struct QGemvLds {
   static constexpr int kMaxWaves = kGemvLdsPerBlockMax / kWave < 8 ? kGemvLdsPerBlockMax / kWave : 8;
 };
 
+// The 32 tokens of a block, one behind the other along y; up to 16 are one block.
+template <int MT>
+__device__ __forceinline__ GemvShape q_gemv_tokens(GemvShape s) {
+  if constexpr (MT == 1) return s;
+  const int m0 = blockIdx.y * kGemvTokens;
+  s.M = min(s.M - m0, kGemvTokens);
+  s.x = reinterpret_cast<const uint16_t*>(s.x) + (int64_t)m0 * s.ldx;
+  s.y = reinterpret_cast<uint16_t*>(s.y) + (int64_t)m0 * s.ldy;
+  return s;
+}
+
 // XI: load instructions for a step's activations: up to 2 XI tokens.
 template <int ACT, int NBITS, bool ASYM, class Provider, int R, int XI>
 __global__ void __launch_bounds__(512)
 q_gemv_kernel(const GemvShape all, const typename Provider::Args a) {
-  const GemvShape s = gemv_token_block(all);
-  using L = QGemvLds<NBITS, ASYM, R, XI>;
   constexpr int MT = XI > 8 ? 2 : 1;
+  const GemvShape s = q_gemv_tokens<MT>(all);
+  using L = QGemvLds<NBITS, ASYM, R, XI>;
   constexpr int kSlots = L::kRow / 16, kRowsPerLoad = 64 / kSlots, kCodeLoads = L::kCodes / 1024;
   extern __shared__ __attribute__((aligned(16))) uint8_t q_lds[];
   const Provider prov(a);
