@@ -137,11 +137,13 @@ int npamd_vq_fused_supported(int K, int vl, int bits);
 
 /* 1 when a fused GEMV call of M tokens on an N x K layer runs the kernel that stages every step's
  * activations through LDS: npamd_vq_gemv on a layer with a codebook of `nc` rows of eight (nc > 0),
- * or npamd_q_gemv (nc = 0).  Such a call stays ahead of the tile GEMM up to the GEMV's 32 tokens
- * whatever K is, which is what the callers' band thresholds ask (the reference fixes its own
- * thresholds per backend, neuropress/nn/np_vq_linear.py:73-98).  The answer is the launcher's own:
- * it is run up to the point of the launch.  Host-only arithmetic. */
+ * or npamd_q_gemv (nc = 0).  The answer is the launcher's own: it is run up to the point of the launch.  Host-only arithmetic. */
 int npamd_gemv_stages_activations(int M, int N, int K, int nc);
+
+/* 1 when such a call stays ahead of the tile GEMM up to the GEMV's 32 tokens whatever K is, which is what the callers' band
+ * thresholds ask (the reference fixes its own thresholds per backend, neuropress/nn/np_vq_linear.py:73-98): it stages its
+ * activations, and past 16 tokens its table is not one that LDS could hold.  Host-only arithmetic. */
+int npamd_gemv_ahead_of_tile(int M, int N, int K, int nc);
 
 /* npamd_q_gemv has two kernels for 4- and 8-bit layers.  Bit 1 (value 2): M tokens on a layer with these scales and zero
  * points run the one that brings codes, scales and activations through LDS in whole lines (an even count of scales, 4-byte

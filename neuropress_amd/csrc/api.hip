@@ -262,6 +262,13 @@ extern "C" int npamd_gemv_stages_activations(int M, int N, int K, int nc) {
   return nc ? npamd::vq_gemv_plan_stages(M, N, K, nc) : npamd::q_gemv_plan_stages(M, N, K);
 }
 
+// Next to a table in LDS staging keeps the GEMV ahead at 17 and 24 tokens, not to 32: 4096 x 14336 with 4096 rows 15.4 / 17.8 / 24.3 us against
+// 21.6 / 21.8 / 21.9 of the tile GEMM, 2048 x 14336 at 24 16.0 against 16.8; the blocks entries' line (npamd_gemv_blocks_preferred) tells them apart.
+extern "C" int npamd_gemv_ahead_of_tile(int M, int N, int K, int nc) {
+  const bool table_in_lds = M > 16 && nc > 0 && nc <= npamd::kGemvLdsCodebookMax / 16;
+  return table_in_lds ? 0 : npamd_gemv_stages_activations(M, N, K, nc);
+}
+
 extern "C" int npamd_diag_last_gemv_staged(void) { return npamd::last_gemv_staged(); }
 
 extern "C" void npamd_diag_reload_tuning(void) { npamd::tuning_table() = npamd::read_tuning(); }

@@ -6,14 +6,6 @@ using namespace npamd;
 
 namespace {
 
-// Past 16 tokens layers whose table LDS can hold stage their activations too, but do not stay ahead of the tile GEMM at any K, which is what
-// callers of npamd_gemv_stages_activations ask for: the answer is no.
-bool table_fits(int M, int table_bytes) { return M > 16 && table_bytes > 0 && table_bytes <= kGemvLdsCodebookMax; }
-int staged_answer(int rc, int M, int table_bytes) {
-  if (table_fits(M, table_bytes)) last_gemv_staged() = 0;
-  return rc;
-}
-
 template <int ACT, int BITS, int VL>
 int run_vq(const VqCall& c, const GemvShape& s) {
   const int table = VL == 8 ? c.nc * 16 : c.nc % 2 == 0 ? c.nc * 8 : 0;
@@ -21,12 +13,12 @@ int run_vq(const VqCall& c, const GemvShape& s) {
     if (c.cb_dtype == NPAMD_F16) {
       using P = VqProvider<ACT, BITS, true, VL>;
       typename P::Args a{c.packed, (const u32x4*)c.cb, (uint32_t)c.nc - 1u, s.chunks};
-      return staged_answer(launch_fused_gemv<ACT, P>(s, a, c.st, c.what, table), c.M, table);
+      return launch_fused_gemv<ACT, P>(s, a, c.st, c.what, table);
     }
   }
   using P = VqProvider<ACT, BITS, false, VL>;
   typename P::Args a{c.packed, (const u32x4*)c.cb, (uint32_t)c.nc - 1u, s.chunks};
-  return staged_answer(launch_fused_gemv<ACT, P>(s, a, c.st, c.what, table), c.M, table);
+  return launch_fused_gemv<ACT, P>(s, a, c.st, c.what, table);
 }
 
 }  // namespace
@@ -38,7 +30,7 @@ int npamd::vq_gemv_plan_stages(int M, int N, int K, int nc) {
   using P = VqProvider<NPAMD_F16, 16, false, 8>;  // the choice depends on the table's size, not on the index width
   typename P::Args a{};
   launch_fused_gemv<NPAMD_F16, P>(s, a, nullptr, "plan", nc * 16);
-  return table_fits(M, nc * 16) ? 0 : staged;
+  return staged;
 }
 
 namespace {

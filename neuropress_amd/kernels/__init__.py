@@ -283,10 +283,10 @@ def vq_linear_perm_supported(m: int, n: int, k: int, num_centroids: int, vector_
 
 def gemv_stages_activations(m: int, n: int, k: int, num_centroids: int) -> bool:
     """Whether a fused GEMV call of *m* tokens on an ``n x k`` layer runs the kernel that stages its
-    activations through LDS (``npamd_gemv_stages_activations``): then the GEMV stays ahead of the
+    activations through LDS and looks no rows up there (``npamd_gemv_ahead_of_tile``): then the GEMV stays ahead of the
     tile GEMM up to its 32 tokens at any ``k``.  *num_centroids*: rows of the layer's codebook of
     eight-element vectors, 0 for a group-quantized layer."""
-    return bool(_lib.load().npamd_gemv_stages_activations(int(m), int(n), int(k), int(num_centroids)))
+    return bool(_lib.load().npamd_gemv_ahead_of_tile(int(m), int(n), int(k), int(num_centroids)))
 
 
 def q_gemv_staging(m: int, n: int, k: int, nbits: int, group_size: int, scale: torch.Tensor | None,

@@ -36,6 +36,22 @@ def test_switched_off_it_is_not_what_the_band_line_counts_on(monkeypatch):
     assert off == [(0, -1)] * len(large)
 
 
+def test_staging_and_the_band_are_two_questions(monkeypatch):
+    """Past 16 tokens layers whose table LDS holds stage their activations, and do not stay ahead of the tile GEMM at any K for it."""
+    from neuropress_amd import _lib, kernels
+
+    lib = _lib.load()
+    for m, n, k, nc, stages, ahead in ((24, 4096, 4096, 4096, 1, 0), (32, 2048, 8192, 256, 1, 0), (24, 4096, 4096, 65536, 1, 1), (2, 14336, 4096, 65536, 0, 0),
+                                       (16, 4096, 4096, 4096, 1, 1), (24, 4096, 4096, 0, 1, 1)):
+        asked = lib.npamd_gemv_stages_activations(m, n, k, nc), lib.npamd_gemv_ahead_of_tile(m, n, k, nc)
+        assert asked == (stages, ahead), (m, n, k, nc, asked)
+        assert kernels.gemv_stages_activations(m, n, k, nc) == bool(ahead)
+    with monkeypatch.context() as mp:
+        mp.setenv("NPAMD_GEMV_XSTAGE", "0")
+        lib.npamd_diag_reload_tuning()
+        assert lib.npamd_gemv_stages_activations(24, 4096, 4096, 4096) == 0
+
+
 @pytest.fixture(params=range(1, len(TILES) + 1))
 def forced(request, monkeypatch):
     from neuropress_amd import _lib
