@@ -38,6 +38,9 @@ extern "C" {
  * npamd_diag_table_tile: the tile of the table GEMM (csrc/table_gemm.hip) with the least estimate for M tokens of an N x K layer whose
  *   codebook has `rows` rows, -1 where it takes no such call.  Host-only.
  *
+ * npamd_diag_last_table_tile: the tile that the calling thread's last npamd_vq_gemv_blocks call ran, -1 where that went to the GEMV (and
+ *   before the first).
+ *
  * npamd_diag_reload_tuning: the NPAMD_* tuning environment variables are read once, at the first
  *   launch; this reads them again.  For tests and tuning runs only: it must not run while
  *   another thread launches.
@@ -46,6 +49,7 @@ void npamd_diag_reload_tuning(void);
 int npamd_diag_last_gemv_staged(void);
 int npamd_diag_gather_fits_decode(int bits, int64_t n_vectors, int K, int permuted);
 int npamd_diag_table_tile(int M, int N, int K, int rows);
+int npamd_diag_last_table_tile(void);
 int npamd_diag_stream_read(const void* src, int64_t n_bytes, void* sink16, void* stream);
 int npamd_diag_gather(const void* idx_u16, int64_t n_indices, const void* table16,
                       int table_entries, int from_lds, void* sink16, void* stream);

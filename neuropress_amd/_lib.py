@@ -79,6 +79,7 @@ SIGNATURES: dict[str, list] = {
     "npamd_diag_last_gemv_staged": [],
     "npamd_diag_gather_fits_decode": [_int, _i64, _int, _int],
     "npamd_diag_table_tile": [_int] * 4,
+    "npamd_diag_last_table_tile": [],
     "npamd_diag_stream_read": [_vp, _i64, _vp, _vp],
     "npamd_diag_gather": [_vp, _i64, _vp, _int, _int, _vp, _vp],
     "npamd_diag_mfma": [_vp, _int, _int, _int, _vp, _vp],

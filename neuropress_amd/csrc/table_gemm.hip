@@ -376,13 +376,21 @@ TablePlan plan_table_gemm(int M, int N, int K, int nc) {
   return best;
 }
 
+static int& last_table_tile() {
+  static thread_local int tile = -1;
+  return tile;
+}
+
 int launch_table_gemm(const VqCall& c, float other_us) {
+  last_table_tile() = -1;
   if (c.packed_r || c.vl != 8 || c.cb_dtype != c.act || c.ldx >= NPAMD_TILE_MAX_STRIDE || (c.bits != 8 && c.bits != 12 && c.bits != 16)) return 1;
   const TablePlan p = plan_table_gemm(c.M, c.N, c.K, c.nc);
   if (p.tile < 0 || (tuning().table_tile == 0 && p.us >= other_us)) return 1;
+  last_table_tile() = p.tile;
   return c.act == NPAMD_BF16 ? launch_table<NPAMD_BF16>(c, p.tile) : launch_table<NPAMD_F16>(c, p.tile);
 }
 
 }  // namespace npamd
 
+extern "C" int npamd_diag_last_table_tile(void) { return npamd::last_table_tile(); }
 extern "C" int npamd_diag_table_tile(int M, int N, int K, int rows) { return npamd::plan_table_gemm(M, N, K, rows).tile; }

@@ -47,6 +47,30 @@ def test_vq(gpu, nc, bits, act):
 
 
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("nc,bits", [(256, 8), (4096, 12)])
+def test_two_row_tiles_next_to_a_table_walk_several_steps(gpu, nc, bits, act, monkeypatch):
+    """More row tiles than compute units and long rows, which the table GEMM takes unless it is off: each wave stages its activations again
+    for every step."""
+    from neuropress_amd import _lib, kernels
+
+    lib = _lib.load()
+    monkeypatch.setenv("NPAMD_TABLE_TILE", "-1")
+    lib.npamd_diag_reload_tuning()
+    g = cases.gen(nc)
+    cb = (torch.randn(nc, 8, generator=g) * 0.05).to(act).to(gpu)
+    for n, k, short in ((4112, 4096, 0), (4130, 8512, 24)):
+        idx = torch.randint(0, nc, (n, k // 8), generator=g)
+        packed = IndexPacking.pack(idx.reshape(-1), bits).to(gpu)
+        w = cb[idx.to(gpu)].reshape(n, k)[:, : k - short]
+        bias = torch.randn(n, generator=g).to(gpu)
+        for m in (17, 24, 32):
+            x = _rows(m, k - short, act, gpu, g)
+            y = kernels.vq_linear_blocks(x, packed, cb, bits, n, bias, width=k)
+            assert (lib.npamd_diag_last_table_tile(), lib.npamd_diag_last_gemv_staged()) == (-1, 1)
+            _check(y, x, w, bias)
+
+
+@pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("nc,ncr", [(65536, 256), (4096, 256), (65536, 65536)])
 def test_residual(gpu, nc, ncr, act):
     from neuropress_amd import kernels

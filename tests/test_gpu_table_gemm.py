@@ -66,7 +66,7 @@ def forced(request, monkeypatch):
 
 @pytest.mark.gpu
 def test_tiles(gpu, forced):
-    from neuropress_amd import kernels
+    from neuropress_amd import _lib, kernels
 
     rows = forced
     shapes = ((259, 64, 0), (64, 128, 56), (300, 192, 0), (256, 2112, 8), (65, 1088, 40), (130, 4096 + 64, 24))
@@ -84,6 +84,7 @@ def test_tiles(gpu, forced):
                     x[:, : k - short] = torch.randn(m, k - short, generator=g).to(act)  # what lies behind a row counts for nothing
                     x = x.to(gpu)[:, : k - short]
                     y = kernels.vq_linear_blocks(x, packed, cb, bits, n, bias, width=k).double()
+                    assert TILES[_lib.load().npamd_diag_last_table_tile()][0] == rows  # not the GEMV, which would be as right
                     xd = x.double()
                     ref, size = xd @ w.T, xd.abs() @ w.abs().T
                     if bias is not None:
