@@ -509,6 +509,11 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
   // Rows of x that end inside the last chunk: the kernels that stage activations look where they end.
   const bool short_rows = s.pieces < s.chunks * 8;
   auto stages = [&](int tokens) { return short_rows || gemv_stage_activations(tokens); };
+  // There are none of those with more than two row tiles per block next to a table in LDS and one elsewhere, whatever NPAMD_GEMV_R asks for.
+  auto staged_rows = [&](GemvPlan p, int most) {
+    if (short_rows && p.R > most) p.R = most;
+    return p;
+  };
   // Layers of few rows, few tokens: 16 / H rows x H parts of k per tile (see the kernel).
   bool lds_table = false;
   if constexpr (Provider::kLdsResidual)
@@ -560,13 +565,13 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
     // looks up in memory.
     if (cb_bytes > 0 && cb_bytes <= kGemvLdsResidualMax && gemv_lds_codebook_enabled()) {
       if (s.M > 16) {
-        const GemvPlan plan = plan_gemv(s.N, s.chunks, stages(s.M) ? 1 : 2, 8);  // as for plain VQ below
+        const GemvPlan plan = staged_rows(plan_gemv(s.N, s.chunks, stages(s.M) ? 1 : 2, 8), 1);  // as for plain VQ below
         if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, true, false, 2>(s, pargs, plan, cb_bytes, st, what);
         if (stages(s.M))
           return launch_fused_gemv_r<ACT, Provider, 1, true, false, 2, 1, true>(s, pargs, plan, cb_bytes, st, what);
         return launch_fused_gemv_r<ACT, Provider, 1, true, false, 2>(s, pargs, plan, cb_bytes, st, what);
       }
-      const GemvPlan plan = plan_gemv(s.N, s.chunks, short_rows ? 1 : 2);
+      const GemvPlan plan = staged_rows(plan_gemv(s.N, s.chunks, short_rows ? 1 : 2), 1);
       if (plan.R == 2) return launch_fused_gemv_r<ACT, Provider, 2, true>(s, pargs, plan, cb_bytes, st, what);
       if (stages(s.M))
         return launch_fused_gemv_r<ACT, Provider, 1, true, false, 1, 1, true>(s, pargs, plan, cb_bytes, st, what);
@@ -588,7 +593,7 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
     const bool memory_lookups = Provider::kGathers && !cb_in_lds;
     const int tiles = cb_in_lds && stages(s.M) ? gemv_wide_row_tiles(s.M, row_tiles, cb_bytes) : 0;
     const int most = short_rows && tiles == 4 ? 2 : tiles;
-    const GemvPlan plan = plan_gemv(16 * row_tiles, s.chunks, most ? most : memory_lookups ? (stages(s.M) ? 1 : 2) : 4, 8, most == 2);
+    const GemvPlan plan = staged_rows(plan_gemv(16 * row_tiles, s.chunks, most ? most : memory_lookups ? (stages(s.M) ? 1 : 2) : 4, 8, most == 2), cb_in_lds ? 2 : 1);
     if constexpr (Provider::kLdsCodebook) {
       if (cb_in_lds) {
         if (plan.R == 4) return launch_fused_gemv_r<ACT, Provider, 4, true, false, 2>(s, pargs, plan, cb_bytes, st, what);
@@ -607,7 +612,7 @@ int launch_fused_gemv(GemvShape s, const typename Provider::Args& pargs, hipStre
       return launch_fused_gemv_r<ACT, Provider, 1, false, false, 2, 1, true>(s, pargs, plan, 0, st, what);
     return launch_fused_gemv_r<ACT, Provider, 1, false, false, 2>(s, pargs, plan, 0, st, what);
   }
-  const GemvPlan plan = plan_gemv(s.N, s.chunks, short_rows && !s.perm ? (cb_in_lds ? 2 : 1) : (Provider::kGathers && !cb_in_lds) ? 2 : 4);
+  const GemvPlan plan = staged_rows(plan_gemv(s.N, s.chunks, short_rows && !s.perm ? (cb_in_lds ? 2 : 1) : (Provider::kGathers && !cb_in_lds) ? 2 : 4), cb_in_lds ? 2 : 1);
   if constexpr (Provider::kLdsCodebook) {
     const bool x_fits = (int64_t)s.M * s.chunks * 64 <= kGemvLdsActivationsMax;
     if (s.perm || (x_fits && !short_rows && gemv_lds_activations_forced())) {  // with a permutation the caller has checked the size

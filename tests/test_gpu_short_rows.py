@@ -119,3 +119,34 @@ def test_a_planned_call_keeps_the_gradient_of_the_bias(gpu, k, nc, ncr, tokens, 
         y.float().sum().backward()
         assert torch.equal(layer.bias.grad, torch.full_like(layer.bias, m))
         layer.bias.grad = None
+
+
+@pytest.mark.parametrize("rows", [1, 2, 4])
+def test_row_tiles_asked_for(gpu, monkeypatch, rows):
+    """NPAMD_GEMV_R asks for more row tiles per block than the kernels that look where a row ends have: such layers run with what those have."""
+    from neuropress_amd import _lib, kernels
+
+    monkeypatch.setenv("NPAMD_GEMV_R", str(rows))
+    _lib.load().npamd_diag_reload_tuning()
+    n, k, width = 200, 552, 576
+    for nc, bits in ((256, 8), (4096, 12), (65536, 16)):
+        g = cases.gen(nc + rows)
+        cb = (torch.randn(nc, 8, generator=g) * 0.05).half().to(gpu)
+        idx = torch.randint(0, nc, (n, width // 8), generator=g)
+        packed, w = IndexPacking.pack(idx.reshape(-1), bits).to(gpu), cb[idx.to(gpu)].reshape(n, width)[:, :k]
+        for m in (1, 5, 16, 29, 70):
+            x = torch.randn(m, k, generator=g).half().to(gpu)
+            _close(kernels.vq_linear_blocks(x, packed, cb, bits, n, width=width), x, w)
+    for ncr in (256, 65536):
+        L = cases.rvq_layer(ncr + rows, n, width, 65536, ncr, zipf=False)
+        pm, pr, cm, cr, sc, rb = (L[name].to(gpu) for name in ("pm", "pr", "cbm", "cbr", "scale", "wbias"))
+        w = kernels.rvq_dequant(pm, L["bm"], pr, L["br"], cm, cr, sc, rb, n, width, torch.float16)[:, :k]
+        for m in (1, 5, 16, 29, 70):
+            x = torch.randn(m, k, generator=cases.gen(m)).half().to(gpu)
+            _close(kernels.rvq_linear_blocks(x, pm, L["bm"], pr, L["br"], cm, cr, sc, rb, n, width=width), x, w)
+
+
+def _close(y, x, w):
+    """One rounding of the output and f32 sums of K products in some order."""
+    ref, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    assert bool(((y.double() - ref).abs() <= ref.abs() * 2.0**-10 + size * w.shape[1] * 2.0**-24 + 2.0**-24).all())
