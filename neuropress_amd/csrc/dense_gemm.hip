@@ -453,6 +453,20 @@ float gemv_blocks_us(int kind, int table_rows, int M, int N, int K) {
   const float served = table_rows <= 2048 ? 1100e3f : 275e3f;  // by the L1s; by the L2s
   return (kind == 1 ? 4.1f : 3.3f) + load * lookups / 2400.f + tiles * lookups / served;
 }
+
+// What the figures of gemv_blocks_us, which the line against the tile GEMM was drawn with, leave out on rows of more than some 4096 columns:
+// a step of a wave takes longer where most compute units have a block, and a block's lookups in a large codebook, which no L2 has
+// yet, one after the other take their time however few blocks there are.  Decode + product / blocks, us: int8 1102 x 6656 at 358 tokens 24.4 / 28.5 (21.6 by
+// those figures, 28.2 by these), 691 x 6272 at 614 21.6 / 25.3, 377 x 8064 at 500 20.4 / 16.8, 820 x 7936 at 262 20.1 / 15.9; int4 1276 x 6400 at 362
+// 23.2 / 25.3, 265 x 5632 at 1082 20.2 / 21.5, 1658 x 5120 at 169 20.3 / 15.5, 404 x 7296 at 441 18.0 / 15.9; 65536 rows 491 x 6272 at 100
+// 14.3 / 16.6, 373 x 7296 at 62 14.6 / 20.1, 1308 x 4096 at 81 18.1 / 13.8; residual 679 x 7168 at 53 17.1 / 19.2, 1871 x 3968 at 35 20.2 / 14.7.
+static float gemv_blocks_long_rows_us(int kind, int table_rows, int M, int N, int K) {
+  const float us = gemv_blocks_us(kind, table_rows, M, N, K);
+  const int tokens = (M + kGemvTokens - 1) / kGemvTokens, rows = (N + 15) / 16, steps = (K + 255) / 256, load = (rows * tokens + 255) / 256;
+  if (kind == 4) return us + (steps > 16 ? 0.02f * load * steps : 0.f);
+  if (kind == 8) return load <= 1 ? us : fmaxf(us, 1.8f + ((rows + 1) / 2 * tokens + 255) / 256 * (1.5f + 0.45f * steps));
+  return table_rows > 16384 ? fmaxf(us, (kind == 1 ? 4.1f : 3.3f) + 2.0f * K / 960.f) : us;
+}
 }  // namespace npamd
 
 extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int table_rows, int gathered, int tile) {
@@ -469,6 +483,7 @@ extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int ta
   const bool own = npamd_dense_gemm_preferred(M, N, K), many = ceil(M / 256.0) * ceil(N / 256.0) >= 100;
   const float library = many ? 5.f + 2e-9f * M * N * K / 1.25f : (float)library_us(M, N, K);
   const float product = fmaxf(own ? 6.8f : 33.f, decode + (own ? plan_dense(M, N, K, 0, kDenseMaxSplits).us : library));
+  if (!tile && !in_lds) return 1.03f * (gemv_blocks_long_rows_us(kind, table_rows, M, N, K) + gather) < product ? 1 : 0;
   if (blocks >= product) return 0;
   if (!tile || (in_lds && M > 256)) return 1;  // past 256 tokens such layers have no tile GEMM
   const int columns = (N + 63) / 64 * ((M + 383) / 384), chunks = K / 64;
