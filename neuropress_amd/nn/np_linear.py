@@ -34,12 +34,12 @@ from .backends import Backend, LinearBackend, is_hip_backend_available, tensor_v
 
 log = logging.getLogger(__name__)
 
+# Most tokens of the GEMV with a workgroup per 32 tokens, which serves small layers past the GEMV's own (kernels.gemv_blocks_preferred).
+_Q_BLOCKS_MAX_TOKENS: int = int(os.environ.get("NEUROPRESS_Q_BLOCKS_MAX_TOKENS", "65536"))
 # Upper end of the fused-GEMM band for the int4 path; above it decode + GEMM.
 # Measured on one MI355X (14336 x 4096, group 32): fused GEMM 35-40 us up to 128
 # tokens and 56 us at 256 against 56-64 / 80 us for decode + GEMM; 83-84 vs 78-84 us at
 # 320-384, 158 vs 93 us at 512.
-# Most tokens of the GEMV with a workgroup per 32 tokens, which serves small layers past the GEMV's own (kernels.gemv_blocks_preferred).
-_Q_BLOCKS_MAX_TOKENS: int = int(os.environ.get("NEUROPRESS_Q_BLOCKS_MAX_TOKENS", "65536"))
 _Q_TILE_MAX_TOKENS: int = int(os.environ.get("NEUROPRESS_Q_TILE_MAX_TOKENS", "256"))
 # Long reductions (K >= _Q_TILE_SPLIT_LONG_K), where the dense GEMM is slow, keep the fused
 # GEMM up to this many tokens: 4096 x 14336 80 vs 105-109 us at 320-384, 148 vs 120 us at 512.
@@ -436,17 +436,22 @@ class NPLinear(nn.Module):
         return "tile" if tile else "dense"
 
     def _blocks_win(self, m: int, tile: bool = True) -> bool:
-        """Whether the GEMV with a workgroup per 32 tokens is ahead of the fused GEMM (*tile*) and of decode + GEMM (NPVQLinear._blocks_win)."""
+        """Whether the GEMV with a workgroup per 32 tokens is ahead of the fused GEMM (*tile*) and of decode + GEMM.  Layers of fewer than
+        256 output features, the least that the estimates were checked on, keep those (NPVQLinear._blocks_win), though most would gain: decode +
+        GEMM / this, int4, us at 64 tokens 64 x 512 7.8 / 4.2, 200 x 4096 11.8 / 6.6, at 1024 tokens 128 x 8192 14.2 / 21.1."""
         from .. import kernels
 
         if not 16 < m <= _Q_BLOCKS_MAX_TOKENS or self.out_features < 256 or min(_Q_FUSED_MAX_TOKENS, _Q_TILE_MAX_TOKENS) <= 0:
+            return False
+        # By sizes first: every token count a layer meets asks, and most of them get their answer there.
+        if not kernels.gemv_blocks_preferred(m, self.out_features, self.in_features, self.nbits, tile=tile):
             return False
         if self.u8_blob.data_ptr() % 16:
             return False  # a slice of a larger buffer, say: the entry refuses it, the kernels it takes the place of serve it
         lines, _ = kernels.q_gemv_staging(
             _lib.GEMV_MAX_M, self.out_features, self.in_features, self.nbits, self.group_size, self.scale, self.zero_point
         )
-        return lines and kernels.gemv_blocks_preferred(m, self.out_features, self.in_features, self.nbits, tile=tile)
+        return lines
 
     def _planned(self, x: torch.Tensor, m: int, band: str):
         """Add this call to the layer's plan and let the plan issue it; None where it cannot."""

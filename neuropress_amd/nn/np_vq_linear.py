@@ -1180,9 +1180,10 @@ class NPVQLinear(nn.Module):
 
     def _blocks_win(self, m: int, tile: bool = True) -> bool:
         """Whether the GEMV with a workgroup per 32 tokens (or the table GEMM behind the same entry) is ahead of
-        the tile GEMM (*tile*) and of decode + GEMM.  It takes their place on
-        layers of 256 output features and more: what smaller ones do, heads and probes, they do through the products
-        that callers put their own in the place of."""
+        the tile GEMM (*tile*) and of decode + GEMM.  Layers of fewer than 256 output features, the least that
+        the estimates were checked on, keep those.  Many would gain, those with long rows or a large codebook lose: decode +
+        GEMM / this, us at 64 tokens, 4096 rows 128 x 1024 7.9 / 4.9, 200 x 4096 11.8 / 9.4, 128 x 8192 11.8 / 15.9, 65536 rows
+        128 x 1024 8.1 / 5.4, 64 x 4096 11.7 / 14.4, 128 x 8192 12.3 / 23.0, residual 128 x 2048 10.5 / 9.6, 200 x 4096 12.7 / 16.0."""
         if not 16 < m <= _BLOCKS_MAX_TOKENS or self.out_features < 256 or min(_FUSED_MAX_TOKENS, _TILE_MAX_TOKENS) <= 0 or self.backend == VQBackend.CUDA_LUT:
             return False
         if self.vector_len != 8 or self.proxy.centroids.dtype != torch.float16 or not self._mfma_layer() or (
@@ -1190,12 +1191,10 @@ class NPVQLinear(nn.Module):
             and (self.bits if self.bits in _FAST_BITS else 16, self._res_bits()) not in ((16, 8), (16, 16), (12, 8), (8, 8))
         ):  # fmt: skip
             return False
-        if not self._blocks_read():
-            return False
         from .. import kernels
 
         return kernels.gemv_blocks_preferred(m, self.out_features, self._kernel_k(), int(self.is_residual), self.proxy.num_centroids,
-                                             self.column_perm is not None, tile)  # fmt: skip
+                                             self.column_perm is not None, tile) and self._blocks_read()  # fmt: skip
 
     def _blocks_read(self) -> bool:
         """Whether the buffers start at 16-byte addresses (not slices of larger ones, say): the blocks entries refuse others, the kernels
