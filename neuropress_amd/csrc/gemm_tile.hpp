@@ -428,6 +428,10 @@ tile_gemm_kernel(const GemmShape s, const typename Provider::Args pargs) {
         for (int i = kPieceOfGroup[j]; i < kPieceOfGroup[j + 1]; ++i) fetch_piece(i, fbuf, src);
       }
       if (kIssueAtEnd && j == 3) {
+        // Behind the MFMAs, whose operands are what was read last of this buffer: scheduled in front of them, as nothing else forbids, the
+        // transfers overwrote rows whose reads were still on their way (7494 x 13568 with 4096 rows at 163 tokens: some of rows 64 to 79
+        // and 96 to 127 wrong in 28 of 30 calls).  Us: 14336 x 4096 at 256 tokens 51.8 -> 52.2, 4096 x 14336 55.2 -> 56.5.
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < kPiecesW; ++i) fetch_piece(i, fbuf, src);
       }

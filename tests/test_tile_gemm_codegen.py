@@ -174,3 +174,31 @@ def test_the_gemv_leaves_m0_to_its_codebook_copy(assembly_gemv):
                 transfers += 1
         with_copy += transfers > 0
     assert with_copy >= 20  # the variants that keep a table in LDS
+
+
+def test_transfers_into_the_buffer_just_read_follow_its_products(assembly):
+    """With two x tiles in LDS the transfers of tile step + 2 go into the buffer of tile `step`, whose last reads the step's last products
+    wait for: every one of those products comes in front of them, and nothing is read between."""
+    lines = assembly
+    starts = [i for i, ln in enumerate(lines) if re.match(r"^_ZN5npamd16tile_gemm_kernel\S*: ;", ln)]
+    checked = 0
+    for i in starts:
+        name = lines[i].split(":")[0]
+        m = re.search(r"ELi(\d)ELb([01])EEEvNS_9GemmShape", name)
+        tiles = int(m.group(1))
+        if not (tiles == 3 or (tiles == 2 and m.group(2) == "1" and "VqProvider" in name and "RvqProvider" not in name)):
+            continue
+        end = next(j for j in range(i, len(lines)) if lines[j].startswith(".Lfunc_end"))
+        ops = [op.group(1) for op in (re.match(r"\s+(ds_\w+|v_mfma\w+|global_load_lds\w+|s_barrier)", ln) for ln in lines[i:end]) if op]
+        first, last = (f(k for k, op in enumerate(ops) if op.startswith("v_mfma")) for f in (min, max))
+        runs = 0
+        for k in range(first, last + 1):
+            if ops[k].startswith("global_load_lds") and not ops[k - 1].startswith("global_load_lds"):
+                products = 0
+                while ops[k - 1 - products].startswith("v_mfma"):
+                    products += 1
+                assert products >= 2 * tiles, (name, ops[k - 8 : k + 2])
+                runs += 1
+        assert runs >= 2, name
+        checked += 1
+    assert checked >= 30
