@@ -92,9 +92,9 @@ _FUSED_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_FUSED_MAX_TOKENS",), 16)
 # 17..32 tokens: the GEMV reuses every decoded operand for two 16-token tiles.  Each of its
 # workgroups reads all of x from L2, so it wins while x is small (tokens x in_features at most
 # _FUSED_WIDE_MAX_ACTIVATIONS).  Measured, GEMV vs tile GEMM at 17 / 24 / 32 tokens, bf16:
-# 14336 x 4096, 4096-row codebook 12.9 / 14.6 / 16.2 vs 27 us, 65536-row 42 / 44 / 47 vs 46-50 us;
-# 4096 x 4096 8.7 / 9.8 / 11.1 vs 16 us; 4096 x 14336 22.4 / 26.4 / 31.2 vs 28 us.  Residual
-# layers 35-41 vs 70 us (14336 x 4096) and 41-50 vs 74 us (4096 x 14336): GEMV at any length.
+# 14336 x 4096, 4096-row codebook 15.7 / 16.7 / 15.1 vs 22 us, 65536-row 39.2 / 40.2 / 41.6 vs 39 us;
+# 4096 x 4096 7.1 / 7.6 / 9.6 vs 12.7 us; 4096 x 14336 15.7 / 17.3 / 24.0 vs 22.4 / 22.8 / 23.5 us.  Residual
+# layers 31-32 vs 32 us (14336 x 4096): GEMV at any length.
 _FUSED_WIDE_MAX_TOKENS: int = _env_int(("NEUROPRESS_VQ_FUSED_WIDE_MAX_TOKENS",), 32)
 _FUSED_WIDE_MAX_ACTIVATIONS: int = 1 << 18
 _GEMV_KERNEL_MAX_TOKENS: int = 32  # what the GEMV entry points accept (NPAMD_GEMV_MAX_M)

@@ -232,8 +232,8 @@ def test_cfg3_through_the_module_in_band_c(gpu, m, monkeypatch):
 
 
 def test_the_staging_predicate_names_the_kernel_the_launcher_takes(gpu):
-    """npamd_gemv_stages_activations decides how far the modules keep the fused GEMV ahead of the tile
-    GEMM; it restates the launcher's choice, so every shape class is launched once and asked about."""
+    """npamd_gemv_stages_activations, behind npamd_gemv_ahead_of_tile, which decides how far the modules keep the fused GEMV
+    ahead of the tile GEMM, restates the launcher's choice, so every shape class is launched once and asked about."""
     from neuropress_amd import _lib, kernels
 
     lib = _lib.load()
