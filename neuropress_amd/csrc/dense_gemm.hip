@@ -27,23 +27,12 @@
 #include <type_traits>
 
 #include "gemm_tile.hpp"
+#include "lds_transfer.hpp"
 #include "table_gemm.hpp"
 
 namespace npamd {
 
 namespace {
-
-__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-}
-// Lane l's 16 bytes land at dst + 16 l; dst is uniform over the wave.  The statement writes m0, which an asm
-// statement cannot declare as clobbered: sound while the compiler keeps nothing of its own in m0 in this kernel.
-__device__ __forceinline__ void lds_load16(uint32_t dst, uint32_t voff, const void* base) {
-  dst = __builtin_amdgcn_readfirstlane(dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(base) : "memory");
-}
 
 struct DenseShape {
   const void* x;
@@ -424,8 +413,9 @@ extern "C" int npamd_dense_gemm_ragged(const void* x, int64_t ldx, const void* w
 // Whether a call of more than 16 tokens goes to the GEMV with a block per 32 tokens (npamd_*_gemv_blocks), or the table GEMM behind the same
 // entry (table_gemm.hip), rather than to decode + product or the tile GEMM.  Up to a round or two of its blocks it is one short launch in the place of two that follow each
 // other; past that every block of tokens decodes its weights again.  All three are estimated.  kind: 0 VQ, 1 residual VQ, 4 and 8 bits
-// per weight.  The GEMV's figures are fitted to layers of 512 to 8192 rows and K of 512 to 14336 at 33 to 512 tokens (within 10 %, residual
-// VQ as with indices that are all as frequent).  us, before / blocks, at 64 and 256 tokens: int4 512 x 512 6.9 / 4.0 and 6.9 / 4.1,
+// per weight.  The GEMV's figures are fitted to layers of 512 to 8192 rows and K of 512 to 14336 at 33 to 512 tokens (within 10 %, on long rows up
+// to a third low, see gemv_blocks_long_rows_us; residual VQ as with indices that are all as frequent).  What the line sends there, 162 drawn calls past the
+// GEMV's own band: decode + product or tile GEMM / blocks 0.89 to 2.4 x, 1.24 to 1.66 x in the mean of each format and table.  us, before / blocks, at 64 and 256 tokens: int4 512 x 512 6.9 / 4.0 and 6.9 / 4.1,
 // 1024 x 4096 11.8 / 6.4 and 13.3 / 9.5, 3072 x 3072 14.8 / 8.2; 256 rows 1024 x 1024 7.9 / 4.7 and 8.0 / 5.7, 2048 x 2048 10.4 / 5.7 and 11.1 / 11.2;
 // 4096 rows 1024 x 1024 8.1 / 4.7 and 8.1 / 6.6; 65536 rows 512 x 512 7.0 / 4.2 and 7.1 / 4.8, 1024 x 4096 13.2 / 10.0 and 16.5 / 24.8.
 namespace npamd {

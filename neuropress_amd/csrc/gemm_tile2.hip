@@ -1,5 +1,6 @@
 // The 128-column tile-decode GEMM (see gemm_tile2.hpp): kernel, weight-tile producers and launchers.
 #include "gemm_tile2.hpp"
+#include "lds_transfer.hpp"
 
 #include <stdlib.h>
 
@@ -42,24 +43,6 @@ __device__ __forceinline__ void store4_sc1(float* p, const f32x4& v0, const f32x
 
 // Cache policy bits of a raw buffer load: bit 4 is sc1 (agent scope).
 constexpr int kAuxSc1 = 16;
-
-// A pointer that is the same in every lane, said so to the compiler (an "s" operand has to live in scalar registers).
-__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-}
-// Loads that write LDS directly: lane l's 16 (4) bytes land at dst + 16 l (4 l); dst is uniform
-// over the wave.  The statements write m0, which the compiler does not let an asm statement declare
-// as clobbered; that is sound as long as the compiler keeps nothing of its own in m0 in these kernels.
-__device__ __forceinline__ void lds_load16(uint32_t dst, uint32_t voff, const void* base) {
-  dst = __builtin_amdgcn_readfirstlane(dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(base) : "memory");
-}
-__device__ __forceinline__ void lds_load4(uint32_t dst, uint32_t voff, const void* base) {
-  dst = __builtin_amdgcn_readfirstlane(dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(voff), "s"(base) : "memory");
-}
 
 // The block's walk over K: step t contracts chunk (t + rot) mod steps of the block's range (column
 // blocks start at different chunks, which spreads the traffic over the L2 channels); steps past the

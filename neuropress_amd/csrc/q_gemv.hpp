@@ -17,19 +17,10 @@
 #pragma once
 
 #include "gemv.hpp"
+#include "lds_transfer.hpp"
 
 namespace npamd {
 
-// Lane l's 16 (4) bytes land at dst + 16 l (4 l); dst is uniform over the wave.  The statements write m0, which an asm statement
-// cannot declare as clobbered: sound while the compiler keeps nothing of its own in m0 in this kernel.
-__device__ __forceinline__ void q_gemv_load16(uint32_t dst, uint32_t voff, const void* base) {
-  dst = __builtin_amdgcn_readfirstlane(dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(base) : "memory");
-}
-__device__ __forceinline__ void q_gemv_load4(uint32_t dst, uint32_t voff, const void* base) {
-  dst = __builtin_amdgcn_readfirstlane(dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(voff), "s"(base) : "memory");
-}
 template <int N>
 __device__ __forceinline__ void q_gemv_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -107,7 +98,7 @@ q_gemv_kernel(const GemvShape all, const typename Provider::Args a) {
 #pragma unroll
       for (int i = 0; i < XI; ++i) {
         const int p = step * 32 + (xpiece ^ ((2 * i + (lane >> 5)) & 15));  // 16-byte piece of the row
-        q_gemv_load16(mine_lds + (uint32_t)(i * 1024), xoff[i] + (uint32_t)(min(p, s.chunks * 8 - 1) * 16), s.x);
+        lds_load16(mine_lds + (uint32_t)(i * 1024), xoff[i] + (uint32_t)(min(p, s.chunks * 8 - 1) * 16), s.x);
       }
     };
     auto load_item = [&](int r, int step) {
@@ -115,13 +106,13 @@ q_gemv_kernel(const GemvShape all, const typename Provider::Args a) {
 #pragma unroll
       for (int t = 0; t < kCodeLoads; ++t) {
         const int kc = min(step * 4 + wpiece[t] / (kSlots / 4), s.chunks - 1);
-        q_gemv_load16(dst + (uint32_t)(t * 1024),
+        lds_load16(dst + (uint32_t)(t * 1024),
                       woff[r][t] + (uint32_t)(kc * (NBITS * 8) + wpiece[t] % (kSlots / 4) * 16), wbase);
       }
       const int kc = min(step * 4 + (lane & 3), s.chunks - 1);
       const uint32_t at = ((srow[r] + (uint32_t)((2 * kc) >> a.gs_shift_chunks)) * 2u) & ~3u;
-      q_gemv_load4(dst + (uint32_t)L::kCodes, at, a.scale + scale0);
-      if constexpr (ASYM) q_gemv_load4(dst + (uint32_t)(L::kCodes + 256), at, a.zp + scale0);
+      lds_load4(dst + (uint32_t)L::kCodes, at, a.scale + scale0);
+      if constexpr (ASYM) lds_load4(dst + (uint32_t)(L::kCodes + 256), at, a.zp + scale0);
     };
 
     load_x(step_begin);

@@ -12,7 +12,7 @@
 // A step: its operands of x go into registers at once, which frees their place for the next step's while the MFMAs run; behind
 // the MFMAs of a k group the rows of that group in the next step are looked up; the indices of the step after that are read.
 //
-// What bounds it: at 256 x 4096 x 4096 with 256 rows (13 us; start and end 4 of them) the matrix pipes are busy a third of the time, LDS 45 %; a
+// What bounds it: at 256 x 4096 x 4096 with 256 rows (12.3 us; start and end 4 of them) the matrix pipes are busy a third of the time, LDS 45 %; a
 // wave's step is a chain of its x arriving, its LDS reads and its MFMAs, which two waves per SIMD (KG = 8) or larger tiles
 // cover in part.  Tried without gain: two and three places for x, reads a step ahead, copies of the table side by side
 // (fewer bank conflicts), column tiles that start K at different steps, loads between the single MFMAs (14.2 us for 11.9).
@@ -29,26 +29,11 @@
 #include <type_traits>
 
 #include "gemm_tile.hpp"
+#include "lds_transfer.hpp"
 
 namespace npamd {
 
 namespace {
-
-__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-}
-// Lane l's 16 (4) bytes land at dst + 16 l (dst + 4 l); dst is uniform over the wave.  The statements write m0, which an asm
-// statement cannot declare as clobbered: sound while the compiler keeps nothing of its own in m0 in this kernel.
-__device__ __forceinline__ void lds_load16(uint32_t dst, uint32_t voff, const void* base) {
-  dst = __builtin_amdgcn_readfirstlane(dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(base) : "memory");
-}
-__device__ __forceinline__ void lds_load4(uint32_t dst, uint32_t voff, const void* base) {
-  dst = __builtin_amdgcn_readfirstlane(dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(voff), "s"(base) : "memory");
-}
 
 struct TableShape {
   const void* x;
