@@ -1,23 +1,23 @@
 // Dense MFMA GEMM of the decode + GEMM band: y = x @ W^T (+ bias) on a weight that the one-pass decode has just
 // written, f32 accumulate.
 //
-// What bounds the band's small and middle shapes in a library GEMM is not the arithmetic: a few dozen output tiles
-// leave most compute units idle, each walks all of K with little in flight, and the call costs the host more than
-// both kernels together.  Here a block keeps one output tile and splits K over groups of waves inside the block
-// (group g takes every KG-th 64-k step): a small tile then has 8 waves and up to 128 KiB of operands on their way,
-// and the groups' sums meet in LDS, in group order, without a second kernel or a workspace.
+// What bounds the band's small shapes in a library GEMM is not the arithmetic: a few dozen output tiles leave most compute
+// units idle, each walks all of K with little in flight, and the call costs the host more than both kernels together.  Two
+// kernels serve the band here.  The wide tiles (wide_gemm.hpp, 64 x 64 to 256 x 256) have a wave per 16 MT x 16 NT of the tile and one ring of
+// 64-k steps; which of them a shape takes, and whether K is split over blocks, the plan below estimates.  The kernel in this file is for what
+// is left without a tile for every compute unit even at 64 x 64, or is a long chain of steps for few: a block keeps a tile of 32 x 64 and splits K over
+// four waves (wave g takes every fourth 64-k step), 8 KiB of operands per step each on their way three steps deep, and the waves' sums meet in
+// LDS, in their order, without a second kernel or a workspace (47 x 384 x 8320 unsplit 16.3 us, the library's product 19.0; 90 x 609 x 13312 28).
 //
-// Long reductions over few output tiles (47 tokens on 384 x 8320: 12 tiles of 32 x 64) leave most of the chip idle
-// all the same, here as in the library.  There K is split over blocks too (`splits` parts of equal length, give or take
-// a step): every block stores its f32 tile to the workspace and splitk_reduce_kernel adds the parts in their order.
-// The parts of a column tile stay on the die that decoded its rows.
+// Long reductions over few output tiles leave most of the chip idle all the same, here as in the library.  There K is split over blocks
+// too (`splits` parts of equal length, give or take a step): every block stores its f32 tile to the workspace and splitk_reduce_kernel adds
+// the parts in their order.  In this kernel the parts of a column tile stay on the die that decoded its rows.
 //
 // Both operand tiles are loaded straight into LDS (global_load_lds_dwordx4; rows of 128 bytes, 16-byte piece p of
 // row r in slot p ^ ((r >> 1) & 7), so that a read of 32 consecutive rows touches every bank group twice), a ring of
 // kStages steps per group; one in-order counter tracks a wave's loads and the waits are written by hand.  A wave
 // computes 32 MT x 64 of the tile (MFMA 32x32x16), reading the operands of a k group while it multiplies the one
-// before.  At 384 x 4096 x 4096 (21 us) the matrix pipes are busy 40 % of the time of the 192 compute units in use and
-// LDS 32 %; the waves wait 42 % of theirs, for 14 TB/s of lines from the L2s at 389 cycles each, and for each other.
+// before.
 // Rows that end inside a step (SHORT) are read where they lie: residual VQ 1157 x 272 at 471 tokens 21.7 -> 9.1 us per call (the library's product
 // before), VQ 1920 x 288 at 1590 tokens 13.1 -> 10.8 (x copied to rows of whole steps).
 // The row tiles of a column tile go to one die (workgroups go to the eight dies in turn), so that a die's L2
@@ -26,6 +26,7 @@
 
 #include <type_traits>
 
+#include "dense_gemm.hpp"
 #include "gemm_tile.hpp"
 #include "lds_transfer.hpp"
 #include "table_gemm.hpp"
@@ -33,18 +34,6 @@
 namespace npamd {
 
 namespace {
-
-struct DenseShape {
-  const void* x;
-  const void* w;
-  const float* bias;
-  void* y;
-  int64_t ldx, ldw, ldy;
-  int M, N, steps;   // steps = K / 64
-  int row_tiles, col_tiles, splits, units_per_die;  // unit: a part of K of one tile
-  float* partials;   // splits > 1: [splits][M][N]
-  int pieces;        // 16-byte pieces of a row: K / 8
-};
 
 template <int WGM, int WGN, int MT, int KG, int STAGES>
 struct DenseTile {
@@ -58,10 +47,6 @@ struct DenseTile {
   static constexpr int kEpBytes = kBM * kBN * 2;
   static constexpr int kRingBytes = KG * STAGES * kStageBytes;
   static constexpr int kLds = kRingBytes > kRedBytes + kEpBytes ? kRingBytes : kRedBytes + kEpBytes;
-  // The first operands of a step are read before its barrier where the ring is deep enough for a step to arrive one
-  // barrier early with two more on their way (128 x 64 tiles, ring of six: 23.0 -> 20.7 us on 384 x 4096 x 4096; 64 x 128
-  // in two groups, ring of three: 19.9 -> 29.3, the loads no longer cover the memory's latency).
-  static constexpr bool kAhead = STAGES >= 5;
   static_assert(kLds <= kLdsPerBlockMax, "the block's tiles do not fit LDS");
 };
 
@@ -146,20 +131,17 @@ dense_gemm_kernel(const DenseShape s) {
     for (int mt = 0; mt < MT; ++mt) ao[set][mt] = *reinterpret_cast<const u32x4*>(stage + a_off + mt * 4096 + slot_off[j]);
   };
 
-  // One step out of ring slot `slot`: the operands of k group j + 1 are read in front of the MFMAs of group j, those of
-  // the next step's first group in front of the last MFMAs (its pieces have arrived one barrier early), and with
+  // One step out of ring slot `slot`: the operands of k group j + 1 are read in front of the MFMAs of group j, and with
   // LOADS the pieces of step `ahead` are requested behind them, into the slot of the step before this one.  `there`: pieces of the step
   // in front of the rows' end (SHORT).
   auto compute = [&](auto loads, int slot, int ahead, int there) {
     constexpr bool LOADS = decltype(loads)::value;
     const uint8_t* const stage = ring_p + slot * T::kStageBytes;
-    const uint8_t* const next = ring_p + (slot == STAGES - 1 ? 0 : slot + 1) * T::kStageBytes;
     const int into = slot == 0 ? STAGES - 1 : slot - 1;
-    if (!T::kAhead) read_ops(0, stage, 0);
+    read_ops(0, stage, 0);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (j < 3) read_ops((j + 1) & 1, stage, j + 1);
-      else if (T::kAhead) read_ops(0, next, 0);  // behind the last step: nothing anybody uses
       if constexpr (SHORT && !LOADS) {  // the last step is never one that requests another
         const bool dead = 4 * h + j >= there;
 #pragma unroll
@@ -181,7 +163,6 @@ dense_gemm_kernel(const DenseShape s) {
     }
   };
   // The wave's own pieces of a step have arrived when only those of `young` younger steps are still on their way.
-  // With kAhead every barrier stands for two steps: the one that follows and the one whose first operands that one reads.
   auto wait_young = [&](int young) {
     if (young >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * kLoads < 63 ? 3 * kLoads : 63) : "memory");
     else if (young == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoads) : "memory");
@@ -192,20 +173,15 @@ dense_gemm_kernel(const DenseShape s) {
   int slot = 0;
   auto next_slot = [&] { slot = slot == STAGES - 1 ? 0 : slot + 1; };
   int it = 0;
-  if constexpr (T::kAhead) {
-    wait_young(min(steps_g, STAGES - 1) - 1);
-    block_sync_lds();
-    read_ops(0, ring_p, 0);
-  }
   // Steps every group has, while there is something left to request.
   for (; it < base - (STAGES - 1); ++it) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2 - T::kAhead) * kLoads) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * kLoads) : "memory");
     block_sync_lds();  // everybody's pieces have arrived, and nobody reads the slot of the step before any more
     compute(std::true_type{}, slot, it + STAGES - 1, 8);
     next_slot();
   }
   for (; it < base; ++it) {
-    wait_young(base - 1 - T::kAhead - it);
+    wait_young(base - 1 - it);
     block_sync_lds();
     if (it + STAGES - 1 < steps_g) {  // the last step of a group that has one more than the others
 #pragma unroll
@@ -287,49 +263,53 @@ int launch_dense_tile(DenseShape s, hipStream_t st) {
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "npamd_dense_gemm: cannot reserve %d bytes of LDS: %s", T::kLds, hipGetErrorString(e));
   launch(kernel, (unsigned)blocks, T::kThreads, T::kLds, st, s);
-  if (s.splits > 1) launch_splitk_reduce<ACT>(s.partials, s.splits, s.M, s.N, s.bias, s.y, s.ldy, st);
   return check_launch("npamd_dense_gemm");
 }
 
 // The tiles there are and what a launch on each costs, us: fixed + per round of workgroups + hypot(step time, bytes
-// loaded / rate), fitted to 34 shapes of 64 to 4096 rows, 64 to 14336 columns and K of 64 to 14336 (the tile of least
-// estimate is at most 3 % slower than the best of them on every one; the estimates are within 15 % but for the shortest).
-// A round is one tile per compute unit of every die.  What the figures say: a 64-k step of a 64 x 128 tile costs 0.25 us
-// (0.11 of MFMAs, 0.16 to bring 24 KiB at 64 bytes per cycle into LDS), and all of them together load at 22-28 TB/s from the L2s.
+// loaded / rate), fitted to 700 shapes of 17 to 4096 rows, 256 to 14336 columns and K of 256 to 14336, fp16 and bf16 (the tile of least
+// estimate is 0.2 % slower than the best of them in the mean, 13 % at most; each tile is there because without it that is 0.4 to 7 % in the mean or 15 % and
+// more on some shape; estimates are within 4 to 9 %).  A round is one tile per compute unit of every die.  What the figures say: a tile of
+// 256 x 256 takes 0.85 us a 64-k step (2048 cycles of MFMAs, at the 1.8 to 2.0 GHz the chip runs at under them) and 7.7 us to start and end; all
+// of them together load at 14 to 36 TB/s from the L2s.
 struct DenseCost {
   int bm, bn, groups;
   float fixed, per_step, per_mb, per_round;
 };
 constexpr DenseCost kDenseCost[] = {
-    {32, 64, 4, 1.78f, 0.445f, 0.038f, 1.79f},   // 4 waves
-    {64, 64, 2, 1.72f, 0.307f, 0.043f, 2.10f},   // 4 waves
-    {64, 128, 2, 1.48f, 0.499f, 0.036f, 1.97f},  // 8 waves
-    {128, 128, 1, 0.00f, 0.388f, 0.047f, 3.68f}, // 8 waves
-    {128, 128, 1, 0.00f, 0.375f, 0.045f, 4.55f}, // 4 waves
-    {256, 128, 1, 0.00f, 0.622f, 0.053f, 4.39f}, // 8 waves
-    {192, 128, 1, 0.00f, 0.515f, 0.040f, 4.20f}, // 4 waves of 96 x 64: fewest LDS reads per MFMA
-    {96, 64, 2, 1.80f, 0.450f, 0.028f, 2.10f},   // 6 waves; only in the place of 64 x 128
+    {32, 64, 4, 1.438f, 0.420f, 0.040f, 2.328f},   // the kernel above; from here on the wide tiles, numbered as in launch_wide
+    {64, 64, 1, 1.319f, 0.164f, 0.028f, 2.617f},
+    {64, 128, 1, 1.287f, 0.232f, 0.030f, 3.028f},
+    {128, 128, 1, 1.342f, 0.288f, 0.043f, 4.153f},
+    {160, 128, 1, 1.179f, 0.342f, 0.047f, 5.014f},
+    {256, 128, 1, 1.316f, 0.450f, 0.052f, 5.727f},
+    {192, 128, 1, 1.100f, 0.342f, 0.050f, 4.627f},
+    {96, 128, 1, 1.275f, 0.265f, 0.037f, 3.473f},
+    {160, 256, 1, 0.773f, 0.600f, 0.057f, 7.067f},
+    {192, 256, 1, 0.926f, 0.748f, 0.059f, 7.195f},
+    {256, 224, 1, 2.348f, 0.814f, 0.067f, 6.872f},
+    {256, 256, 1, 2.163f, 0.853f, 0.073f, 7.682f},
+    {96, 64, 1, 1.473f, 0.198f, 0.038f, 2.770f},
+    {192, 192, 1, 0.000f, 0.487f, 0.055f, 8.035f},
 };
-constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]), kDenseTile64x128 = 2, kDenseTile96 = 7;
+constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]);
 
 template <int ACT>
 int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
-  switch (tile) {
-    case 0: return launch_dense_tile<ACT, 1, 1, 1, 4, 3>(s, st);
-    case 1: return launch_dense_tile<ACT, 2, 1, 1, 2, 5>(s, st);
-    case 2: return launch_dense_tile<ACT, 2, 2, 1, 2, 3>(s, st);
-    case 3: return launch_dense_tile<ACT, 4, 2, 1, 1, 5>(s, st);
-    case 4: return launch_dense_tile<ACT, 2, 2, 2, 1, 5>(s, st);
-    case 5: return launch_dense_tile<ACT, 4, 2, 2, 1, 3>(s, st);
-    case 6: return launch_dense_tile<ACT, 2, 2, 3, 1, 4>(s, st);
-    default: return launch_dense_tile<ACT, 3, 1, 1, 2, 4>(s, st);
-  }
+  const int rc = tile > 0 ? launch_wide(s, ACT, tile, st) : launch_dense_tile<ACT, 1, 1, 1, 4, 3>(s, st);
+  if (rc != NPAMD_OK || s.splits == 1) return rc;
+  launch_splitk_reduce<ACT>(s.partials, s.splits, s.M, s.N, s.bias, s.y, s.ldy, st);
+  return check_launch("npamd_dense_gemm");
 }
 
 constexpr int kDenseMaxSplits = 16;
 constexpr int64_t kDenseStrideMax = NPAMD_TILE_MAX_STRIDE;
 constexpr int kDenseMinSplitSteps = 4;  // 64-k steps of a part
-// What a split adds: the reduction kernel and the gap in front of it, and its bytes, us and us per MB.
+// What a split of this product adds: the reduction kernel and the gap in front of it, and its bytes, us and us per MB (200 shapes of
+// long K, 2 to 16 parts, within 1.4 us in the median).  A ninth part costs the sum another round trip of loads, some 4 us: by itself the plan takes no more than eight.
+constexpr float kDenseSplitFixed = 3.5f, kDenseSplitPerMb = 0.6f;
+constexpr int kDensePlannedSplits = 8;
+// The same for the tile GEMM's (estimates of npamd_gemv_blocks_preferred).
 constexpr float kSplitFixed = 4.5f, kSplitPerMb = 0.45f;
 
 struct DensePlan {
@@ -337,28 +317,26 @@ struct DensePlan {
   float us;
 };
 
-// The tile and split of least estimate.  96 x 64 is looked at where 64 x 128 would be taken whole and K is 2048 or more: it
-// loads fewer bytes per compute unit where it fills more of them (384 x 4096: 256 tiles against 192).  384 x 4096 x 4096
-// 23.5 -> 21.6 us; 38 drawn shapes of 65 to 1330 rows where its estimate is lower 1.01 to 1.17 x, geometric mean 1.07.  At
-// K < 2048 0.93 to 1.05 x; against the other tiles, and with K in parts, 0.81 to 1.04 x where the estimates are this close.
-DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits) {
+// The tile and split of least estimate.  The wide tiles address their part of the result with 31 bits: with rows of y, or columns, that
+// could lie further apart than that, the other kernel.
+DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits, bool wide = true) {
   DensePlan best{0, 1, 1e30f};
   const int steps = K / 64;
   const int forced = tuning().dense_splits, most = max_splits < steps ? max_splits : steps;
   const int forced_splits = forced < most ? forced : most;
-  for (int i = 0; i < kDenseTiles; ++i) {
-    if (forced_tile > 0 && forced_tile <= kDenseTiles && i != forced_tile - 1) continue;
-    if (i == kDenseTile96 && !forced_tile && (best.tile != kDenseTile64x128 || best.splits > 1 || steps < 32)) continue;
+  const int last = wide && N < kDenseStrideMax ? kDenseTiles : 1;
+  for (int i = 0; i < last; ++i) {
+    if (last > 1 && forced_tile > 0 && forced_tile <= kDenseTiles && i != forced_tile - 1) continue;
     const DenseCost& c = kDenseCost[i];
     const int64_t tiles = (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
     const float load = (float)tiles * steps * (c.bm + c.bn) * 128e-6f * c.per_mb;
-    for (int splits = 1; splits <= (i == kDenseTile96 && !forced_tile ? 1 : max_splits); ++splits) {
+    for (int splits = 1; splits <= max_splits; ++splits) {
       if (forced_splits > 0 && splits != forced_splits) continue;
-      if (forced_splits <= 0 && splits > 1 && (steps < kDenseMinSplitSteps * splits || tiles * splits > 512)) break;
+      if (forced_splits <= 0 && splits > 1 && (splits > kDensePlannedSplits || steps < kDenseMinSplitSteps * splits || tiles * splits > 512)) break;
       const int64_t rounds = ((tiles * splits + 7) / 8 + 31) / 32;
       const int part = (steps + splits - 1) / splits;
       const float walk = (float)rounds * ((part + c.groups - 1) / c.groups) * c.per_step;
-      float t = c.fixed + (float)rounds * c.per_round + (splits > 1 ? kSplitFixed + kSplitPerMb * (4e-6f * splits * M * N) : 0.f);
+      float t = c.fixed + (float)rounds * c.per_round + (splits > 1 ? kDenseSplitFixed + kDenseSplitPerMb * (4e-6f * splits * M * N) : 0.f);
       if (t + fmaxf(walk, load) >= best.us) continue;
       t += sqrtf(walk * walk + load * load);
       if (t < best.us) best = {i, splits, t};
@@ -388,9 +366,10 @@ static int dense_gemm(const char* what, const void* x, int64_t ldx, const void* 
   hipStream_t st = (hipStream_t)stream;
   const int64_t room = workspace && ((uintptr_t)workspace & 3) == 0 ? workspace_bytes / ((int64_t)M * N * 4) : 1;
   const int width = (K + 63) / 64 * 64;
-  DensePlan p = plan_dense(M, N, width, tuning().dense_tile, kDenseMaxSplits);
-  if (p.splits > room) p = plan_dense(M, N, width, tuning().dense_tile, 1);  // too little workspace: unsplit
-  const DenseShape s{x, w, bias, y, ldx, ldw, ldy, M, N, width / 64, 0, 0, p.splits, 0, (float*)workspace, K / 8};
+  const bool wide = ldy < kDenseStrideMax;
+  DensePlan p = plan_dense(M, N, width, tuning().dense_tile, kDenseMaxSplits, wide);
+  if (p.splits > room) p = plan_dense(M, N, width, tuning().dense_tile, 1, wide);  // too little workspace: unsplit
+  const DenseShape s{x, w, bias, y, ldx, ldw, ldy, M, N, width / 64, 0, 0, p.splits, 0, (float*)workspace, K / 8, 0};
   const int tile = p.tile;
   return act_dtype == NPAMD_BF16 ? launch_dense<NPAMD_BF16>(s, tile, st) : launch_dense<NPAMD_F16>(s, tile, st);
 }
@@ -472,7 +451,9 @@ extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int ta
   // The library's rate here is what it reaches, 1.25 PFLOP/s from 100 of its tiles on; below, with less of a risk in the other direction, as in npamd_dense_gemm_preferred.
   const bool own = npamd_dense_gemm_preferred(M, N, K), many = ceil(M / 256.0) * ceil(N / 256.0) >= 100;
   const float library = many ? 5.f + 2e-9f * M * N * K / 1.25f : (float)library_us(M, N, K);
-  const float product = fmaxf(own ? 6.8f : 33.f, decode + (own ? plan_dense(M, N, K, 0, kDenseMaxSplits).us : library));
+  const DensePlan p = plan_dense(M, N, K, 0, kDenseMaxSplits);
+  const float host = own ? (p.splits > 1 ? 10.3f : 6.8f) : 33.f;  // of two or three launches
+  const float product = fmaxf(host, decode + (own ? p.us : library));
   if (!tile && !in_lds) return 1.03f * (gemv_blocks_long_rows_us(kind, table_rows, M, N, K) + gather) < product ? 1 : 0;
   if (blocks >= product) return 0;
   if (!tile || (in_lds && M > 256)) return 1;  // past 256 tokens such layers have no tile GEMM
@@ -491,27 +472,18 @@ extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int ta
   return blocks < us ? 1 : 0;
 }
 
-// Where this kernel is the better one against the library's product: its estimate against what the library reaches
-// (5 us + 0.85 PFLOP/s; 1.3 once 256 x 256 tiles cover 180 compute units; 1.5 us more per 1024 of K past 4096, which it
-// walks in few tiles) -- or against 25 us: a library product takes 18.3-19 us per eager call whatever its size and
-// 33 us go by between two calls of decode + library product, whatever the GPU does meanwhile (2048 x 4096 with int4 weights,
-// 600 tokens: 35.8 us per call; with this kernel 25).
-// This kernel's estimates are some 15 % high at the larger shapes; where 64 such tiles make the library quicker
-// (1.05 PFLOP/s, on short K 1.2: 288 x 14336 x 4096 39.4 / 43.8 us, 945 x 8192 x 2048 30.9 / 32.3) the margin is smaller.
-// Measured, library / this kernel, us:
-// 171 x 256 x 640 14.6 / 4.8, 77 x 3003 x 2240 13.4 / 8.8, 100 x 14336 x 512 9.7 / 6.7,
-// 384 x 4096 x 4096 23.0 / 20.3, 384 x 11008 x 2048 25.3 / 24.5, 250 x 11008 x 2048 21.5 / 17.3, 2500 x 3000 x 1024 26.2 / 20.3, 1024 x 4096 x 4096
-// 37.2 / 34.5; but 384 x 14336 x 4096 55.5 / 58.1, 700 x 6000 x 6016 56.8 / 64.8, 4096^3 93 / 124: products of more than
-// 40 GFLOP go to the library.  Long K, split over blocks: 47 x 384 x 8320 19.0 / 8.8 (16.3 unsplit), 945 x 512 x 14336
-// 38.4 / 26.2, 230 x 3152 x 7296 27.3 / 22.2, 460 x 2432 x 7936 36.1 / 29.4, 460 x 4096 x 14336 (54 GFLOP) 72 / 60, but
-// 945 x 4096 x 14336 110 / 108: from K = 8192 the line is 60 GFLOP.
+// Where this product is the better one against the library's.  That takes 18.3-19 us per eager call whatever its size and 33 us go by between two
+// calls of decode + library product, whatever the GPU does meanwhile; past that its kernels are the slower ones but where its tiles of
+// 256 x 256 fit: M and N whole multiples, and rounds of them on all compute units that are at least 0.85 full.  Of 112 products with such M and N, us, library / this,
+// fp16 and bf16: 4096 x 4096 x 4096 93.4 / 103.6 and 89.7 / 95.5, 2048 x 8192 x 2048 53.0 / 56.6 and 52.7 / 54.2, 3072 x 5120 x 5120 117.9 / 118.2 and
+// 112.6 / 117.8, 4096 x 14336 x 4096 358 / 381 and 347 / 366, 2048 x 14336 x 4096 191.9 / 187.4 and 173.4 / 180.1; less full 4096 x 6144 x 4096 174.5 / 177.6 and
+// 166.3 / 157.8, 2048 x 11008 x 4096 170.3 / 150.0 and 162.0 / 145.6, 4096 x 11008 x 4096 418 / 284 and 412 / 278, 1024 x 4096 x 4096 44.3 / 37.8 and 38.6 / 36.8.  Any
+// other M and N, 300 products of 0.3 to 490 GFLOP: 0.95 to 1.64 x from 25 GFLOP on, 1.2 in the mean (1646 x 13120 x 11136 fp16 690 / 444, 2355 x 3424 x 1792 37.9 / 30.0,
+// 3552 x 8681 x 7616 368 / 330); below, the library's kernel alone 0.5 to 1.5 x, its call 18.3 us and more.
 extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {
   if (M < 1 || N < 1 || K < 64 || K % 64 || K >= kDenseStrideMax) return 0;
   const int forced = tuning().dense_tile;
   if (forced) return forced > 0;
-  const double gflop = 2e-9 * M * N * K;
-  const float us = plan_dense(M, N, K, 0, kDenseMaxSplits).us;
-  const bool many = ceil(M / 256.0) * ceil(N / 256.0) >= 64, shallow = many && K < 4096;
-  const double margin = shallow ? 1.0 : many ? 1.1 : 1.15;
-  return gflop <= (K >= 8192 ? 60.0 : 40.0) && us <= fmax(25.0, margin * library_us(M, N, K)) ? 1 : 0;
+  const int64_t tiles = (int64_t)(M / 256) * (N / 256), rounds = (tiles + 255) / 256;
+  return M % 256 == 0 && N % 256 == 0 && K >= 768 && tiles >= 0.85 * 256 * rounds ? 0 : 1;
 }
