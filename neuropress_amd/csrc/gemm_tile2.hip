@@ -75,6 +75,7 @@ template <int ACT>
 struct T2ProdVq16 {
   using Args = T2Args;
   static constexpr int kWRing = 3;
+  static constexpr bool kMeetsInside = false;  // its lookups need the whole step
   static constexpr int kLoads = 2;
   static constexpr int kQuadLoads = 1;
   static constexpr int kHandoffBatch = 3;  // row tiles of the other half's tile loaded per round trip (registers)
@@ -131,6 +132,7 @@ struct T2ProdVq16 {
     work<3, 0>(step, wslot, rem);
     work<3, 1>(step, wslot, rem);
   }
+  __device__ __forceinline__ void work_behind(int, int, int) const {}
   // Everything but the loads this step issued last (its lookups, and the index quad behind them in
   // the steps that fetch one) has to be there when the next step starts.
   __device__ __forceinline__ void wait_step_end(int step, int rem) const {
@@ -162,6 +164,11 @@ struct T2ProdQ {
   using P = typename std::conditional<NBITS == 4, Q4Provider<ACT, ASYM>, Q8Provider<ACT, ASYM>>::type;
   using Args = typename P::Args;
   static constexpr int kWRing = 2;
+  // Where the waves meet in a step (see the kernel): in front of its last k group where that is the faster way, us, at its end / inside, 14336 x 4096: int4 fp16 at
+  // 48 / 128 / 256 / 512 tokens 25.3 / 30.2 / 42.2 / 67.7 and 25.5 / 29.0 / 40.3 / 65.7, int8 fp16 22.6 / 28.3 / 42.4 / 69.0 and 23.7 / 28.2 / 41.3 / 68.2,
+  // at 384 57.6 and 57.0; 11008 x 4096 int8 bf16 with zero points at 48 / 200 / 384 25.2 / 38.2 / 55.9 and 26.0 / 39.2 / 52.7.  A decode in f32 (bf16, zero
+  // points) fills the time that is won: 14336 x 4096 int4 bf16 at 256 and 512 40.6 / 64.1 and 40.7 / 64.6.
+  static constexpr bool kMeetsInside = (ACT == NPAMD_F16 && !ASYM && (NBITS == 4 || MW > 1)) || (NBITS == 8 && MW == 3);
   static constexpr int kHandoffBatch = 2;
   static constexpr int kStepBytes = NBITS * 8;            // of a column
   static constexpr int kLine = MW == 3 ? 64 : 128;        // beside three row tiles LDS holds half lines
@@ -265,19 +272,29 @@ struct T2ProdQ {
     fetch(1);
   }
   // The last bytes of line l are read in step kSteps l + kSteps - 3; line l + kRing is requested from the step after
-  // on: one step later where a line is several steps (two steps before its first bytes are read), at once where it is one.
+  // on: one step later where a line is several steps (two steps before its first bytes are read), at once where it is one -- there behind the
+  // barrier of a step that the waves meet in, as the reads of the step before end at that barrier.
   static __device__ __forceinline__ bool requests(int step) { return (step + 2) % kSteps == 0; }
   template <int J_, int T>
   __device__ __forceinline__ void work(int step, int wslot, int rem) {
     if (J_ == 1 && T == 0 && rem >= 1) decode<0>(wslot ^ 1);
     if (J_ == 2 && T == 0 && rem >= 1) decode<1>(wslot ^ 1);
-    if (J_ == 2 && T == 1 && rem >= 2 && requests(step)) request((step + 2) / kSteps + 1);
+    constexpr bool kBehind = kSteps == 1 && kMeetsInside;
+    if (J_ == (kBehind ? 3 : 2) && T == (kBehind ? 0 : 1) && rem >= 2 && requests(step)) request((step + 2) / kSteps + 1);
     if (J_ == 3 && T == 1 && rem >= 2) fetch(step + 2);
   }
+  // What comes in front of the step's barrier, and what behind it.
   __device__ __forceinline__ void work_all(int step, int wslot, int rem) {
     work<1, 0>(step, wslot, rem);
     work<2, 0>(step, wslot, rem);
     work<2, 1>(step, wslot, rem);
+    if (!kMeetsInside) last_group(step, wslot, rem);
+  }
+  __device__ __forceinline__ void work_behind(int step, int wslot, int rem) {
+    if (kMeetsInside) last_group(step, wslot, rem);
+  }
+  __device__ __forceinline__ void last_group(int step, int wslot, int rem) {
+    work<3, 0>(step, wslot, rem);
     work<3, 1>(step, wslot, rem);
   }
   // The x pieces of the next step, requested before a line, have to be there; the line has a step more.
@@ -295,6 +312,7 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
   constexpr int kXBufBytes = 128 * MW * kStepK * 2;
   constexpr int kPieces = 2 * MW;  // x-tile load instructions per wave and step (8 rows each): half of the pair's
   constexpr int kWRing = Prod::kWRing;
+  constexpr bool kInside = Prod::kMeetsInside;
   static_assert(2 * kXBufBytes + kWRing * kT2WSlotBytes + Prod::kStageBytes <= kLdsPerBlockMax, "the block's tiles do not fit LDS");
   uint8_t* const xs = lds;                              // [2][BM][128]
   uint8_t* const ws = lds + 2 * kXBufBytes;             // [kWRing][16 KiB]
@@ -402,22 +420,34 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
 #pragma unroll
       for (int mt = 0; mt < MW; ++mt) ao[set][mt] = *reinterpret_cast<const u32x4*>(xa + mt * 32 * 128);
     };
+    // The waves of a block meet once a step: at its end, or (kInside) between its third and its last k group.  Then the last group's MFMAs
+    // run while the first operands of the next step come from LDS, which behind a barrier at the end every wave waits for at once, and
+    // the x tile of step + 2 goes out from there on: its buffer is the step's own, read for the last time in front of the barrier.
     // One step: eight (k group, column tile) slots of MW MFMAs; behind them, one instruction per
     // slot, the wave's x pieces of step + 1 (other buffer), and the producer's work.  `rem`: steps after
     // this one, 2 standing for two or more; the last step has no x tile to fetch and the producers
     // leave out what would serve steps past the end.
     auto one_step = [&](int buf, int step, int wslot, int rem) {
-      read_ops(0, buf, wslot, 0);
+      if (!kInside) read_ops(0, buf, wslot, 0);
       const uint8_t* src = tile_src(step + 1);
+      const int next = wslot == kWRing - 1 ? 0 : wslot + 1;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        if (kInside && j == 3 && rem >= 1) {
+          prod.wait_step_end(step, rem);
+          block_sync_lds();
+          read_ops(0, buf ^ 1, next, 0);
+          src = tile_src(step + 2);
+        }
         if (j < 3) read_ops((j + 1) & 1, buf, wslot, j + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
 #pragma unroll
           for (int mt = 0; mt < MW; ++mt) acc[mt][t] = mfma32<ACT>(ao[j & 1][mt], bo[j & 1][t], acc[mt][t]);
-          if (rem >= 1 && j * 2 + t < kPieces) fetch_piece(j * 2 + t, buf ^ 1, src);
+          if (!kInside && rem >= 1 && j * 2 + t < kPieces) fetch_piece(j * 2 + t, buf ^ 1, src);
+          if (kInside && rem >= 1 && j < 3 && j * 2 + t + 2 < kPieces) fetch_piece(j * 2 + t + 2, buf ^ 1, src);
+          if (kInside && rem >= 2 && j == 3) fetch_piece(t, buf, src);
           if (j == 0 && t == 0) prod.template work<0, 0>(step, wslot, rem);
           if (j == 0 && t == 1) prod.template work<0, 1>(step, wslot, rem);
           if (j == 1 && t == 0) prod.template work<1, 0>(step, wslot, rem);
@@ -429,9 +459,17 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
           __builtin_amdgcn_sched_barrier(0);
         }
       }
-      prod.wait_step_end(step, rem);
-      if (rem >= 1) block_sync_lds();
+      if (!kInside) {
+        prod.wait_step_end(step, rem);
+        if (rem >= 1) block_sync_lds();
+      }
     };
+    if (kInside) {
+      const uint8_t* src = tile_src(1);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) fetch_piece(i, (steps & 1) ^ 1, src);
+      read_ops(0, steps & 1, 0, 0);
+    }
     // Step t reads x buffer (t + steps) % 2, so that the last two steps, which are instantiated
     // apart, and the pairs of the loop in front of them always see buffers 0 and 1 in this order;
     // an odd number of steps starts with a step of its own on buffer 1.
@@ -461,6 +499,7 @@ tile2_gemm_kernel(const GemmShape s, const typename Prod::Args pargs, const T2Pa
       prod.work_all(t, wslot, rem);
       prod.wait_step_end(t, rem);
       block_sync_lds();
+      prod.work_behind(t, wslot, rem);
       wslot = wslot == kWRing - 1 ? 0 : wslot + 1;
     }
   }

@@ -29,7 +29,8 @@
 //            .. + 7, x and W alike.  int4 / int8: the producers' arithmetic between the MFMAs.
 // All loads of a wave complete in order and the waits are written by hand (s_waitcnt vmcnt(n) with
 // the number of younger loads that may stay in flight): everything a wave requests in step t is due
-// at the end of step t + 1 at the latest, in front of the step's only barrier.  The last two steps
+// at the end of step t + 1 at the latest, in front of the step's only barrier.  Producers with a short
+// decode have that barrier in front of the step's last k group (T2ProdQ::kMeetsInside).  The last two steps
 // are instantiated apart: nothing is looked up or fetched for steps past the end.
 //
 // K is split in two (blockIdx.z) when the column blocks alone leave compute units idle:
