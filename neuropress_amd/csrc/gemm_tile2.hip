@@ -164,11 +164,12 @@ struct T2ProdQ {
   using P = typename std::conditional<NBITS == 4, Q4Provider<ACT, ASYM>, Q8Provider<ACT, ASYM>>::type;
   using Args = typename P::Args;
   static constexpr int kWRing = 2;
-  // Where the waves meet in a step (see the kernel): in front of its last k group where that is the faster way, us, at its end / inside, 14336 x 4096: int4 fp16 at
-  // 48 / 128 / 256 / 512 tokens 25.3 / 30.2 / 42.2 / 67.7 and 25.5 / 29.0 / 40.3 / 65.7, int8 fp16 22.6 / 28.3 / 42.4 / 69.0 and 23.7 / 28.2 / 41.3 / 68.2,
-  // at 384 57.6 and 57.0; 11008 x 4096 int8 bf16 with zero points at 48 / 200 / 384 25.2 / 38.2 / 55.9 and 26.0 / 39.2 / 52.7.  A decode in f32 (bf16, zero
-  // points) fills the time that is won: 14336 x 4096 int4 bf16 at 256 and 512 40.6 / 64.1 and 40.7 / 64.6.
-  static constexpr bool kMeetsInside = (ACT == NPAMD_F16 && !ASYM && (NBITS == 4 || MW > 1)) || (NBITS == 8 && MW == 3);
+  // Where the waves meet in a step (see the kernel): in front of its last k group where that is the faster way, us, at its end / inside, 14336 x 4096: fp16 int4 at 200 / 256
+  // / 512 tokens 41.1 / 41.2 / 66.4 and 39.7 / 40.0 / 64.3, int8 41.5 / 42.1 / 69.0 and 40.9 / 41.2 / 67.6; int8 on three row tiles, 300 / 384 tokens, bf16 56.7 / 54.9 and
+  // 55.5 / 54.6, with zero points 60.1 / 62.0 and 58.7 / 61.5, fp16 with zero points 61.6 / 62.2 and 61.4 / 61.9.  One row tile at 48 tokens, where half of the waves only decode,
+  // loses (int4 24.6 and 24.9, int8 23.3 and 24.2; at 128 29.0 and 28.0, 28.9 and 28.8), and a longer decode (bf16, zero points) on two
+  // fills the time that is won: int4 bf16 at 256 / 512 40.2 / 63.2 and 40.2 / 63.8, int8 40.8 / 66.3 and 41.4 / 67.0; int4 on three 53.9 / 54.9 and 53.6 / 55.0.
+  static constexpr bool kMeetsInside = MW == 2 ? ACT == NPAMD_F16 && !ASYM : MW == 3 && NBITS == 8 && (ACT == NPAMD_BF16 || ASYM);
   static constexpr int kHandoffBatch = 2;
   static constexpr int kStepBytes = NBITS * 8;            // of a column
   static constexpr int kLine = MW == 3 ? 64 : 128;        // beside three row tiles LDS holds half lines
@@ -271,16 +272,22 @@ struct T2ProdQ {
     decode<1>(0);
     fetch(1);
   }
-  // The last bytes of line l are read in step kSteps l + kSteps - 3; line l + kRing is requested from the step after
-  // on: one step later where a line is several steps (two steps before its first bytes are read), at once where it is one -- there behind the
-  // barrier of a step that the waves meet in, as the reads of the step before end at that barrier.
-  static __device__ __forceinline__ bool requests(int step) { return (step + 2) % kSteps == 0; }
+  // The last bytes of line l are read at the end of step kSteps l + kSteps - 3 (kLastRead), by both waves of a column tile, and line l + kRing takes
+  // its place: what requests it lies behind a barrier that every wave reaches after that read.  Where the waves meet at a step's end that is the next
+  // step's; where they meet inside, the read is behind that step's barrier, so it is the next step's barrier that counts: lines of several steps go out in front of the barrier of
+  // the step after the next, those of one step behind the barrier of the next.
+  static constexpr bool kBehind = kSteps == 1 && kMeetsInside;
+  static constexpr int kAhead = kSteps > 1 && kMeetsInside ? 1 : 2;
+  static constexpr int kLastRead = kSteps - 3, kRequest = kSteps * (kRing - 1) - kAhead;  // steps, from the first of line l
+  static_assert(kRequest + (kBehind ? 1 : 0) >= kLastRead + (kMeetsInside ? 2 : 1), "a line is overwritten while it may still be read");
+  // A line has to be there behind the barrier of the step that reads its first bytes, two before its first: by then the wave has waited for it.
+  static_assert(kSteps * kRing - 2 >= kRequest + (kSteps > 1 && !kMeetsInside ? 2 : 1), "a line is read before it is there");
+  static __device__ __forceinline__ bool requests(int step) { return (step + kAhead) % kSteps == 0; }
   template <int J_, int T>
   __device__ __forceinline__ void work(int step, int wslot, int rem) {
     if (J_ == 1 && T == 0 && rem >= 1) decode<0>(wslot ^ 1);
     if (J_ == 2 && T == 0 && rem >= 1) decode<1>(wslot ^ 1);
-    constexpr bool kBehind = kSteps == 1 && kMeetsInside;
-    if (J_ == (kBehind ? 3 : 2) && T == (kBehind ? 0 : 1) && rem >= 2 && requests(step)) request((step + 2) / kSteps + 1);
+    if (J_ == (kBehind ? 3 : 2) && T == (kBehind ? 0 : 1) && rem >= 2 && requests(step)) request((step + kAhead) / kSteps + 1);
     if (J_ == 3 && T == 1 && rem >= 2) fetch(step + 2);
   }
   // What comes in front of the step's barrier, and what behind it.
