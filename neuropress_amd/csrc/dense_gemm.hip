@@ -454,11 +454,13 @@ extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int ta
   const DensePlan p = plan_dense(M, N, K, 0, kDenseMaxSplits);
   const float host = own ? (p.splits > 1 ? 10.3f : 6.8f) : 33.f;  // of two or three launches
   // The plan's figures are of products one after the other.  Behind a decode they take a little more: with 0.6 to 0.9 us the line puts every call
-  // of 8 % and more that was measured (tests/test_blocks_line.py) on its side, with the sum of its parts as a third launch more (int8 431 x 8960 at 390 tokens,
-  // product / blocks, 21.0 / 17.4 us, 65536 rows 608 x 4096 at 43 11.7 / 8.8).  Not behind the lookups in memory of a middle-sized table or of shorter
-  // rows, nor behind a decode of codes of four to twelve steps: 65536 rows 320 x 1536 at 422 9.1 / 10.8, 16384 rows 272 x 8448 at 88 13.1 / 16.0, residual 10144 x 384 at 56 7.9 / 9.5, 576 x 1152 at 271 8.9 / 10.3, int8 2960 x 1664 at 97 10.8 / 11.9, int4 592 x 1280 at 776 9.6 / 10.3.
-  const bool no_more = kind >= 4 ? K > 768 && K <= 3072 : !in_lds && (K <= 3072 || (kind == 0 && table_rows <= 16384));
-  const float behind_decode = no_more ? 0.f : p.splits > 1 ? 1.75f : 0.75f;
+  // of 8 % and more that was measured (tests/test_blocks_line.py) on its side, and more with the sum of its parts as a third launch, but for int4 (product / blocks, us:
+  // int8 431 x 8960 at 390 tokens 21.0 / 17.4, 65536 rows 608 x 4096 at 43 11.7 / 8.8; int4 640 x 7552 at 510 19.7 / 23.3).  Not behind the lookups in
+  // memory of a middle-sized table or of shorter rows, nor behind a decode of codes of four to twelve steps (int4: to six): 65536 rows 320 x 1536 at 422
+  // 9.1 / 10.8, 16384 rows 272 x 8448 at 88 13.1 / 16.0, residual 10144 x 384 at 56 7.9 / 9.5, 576 x 1152 at 271 8.9 / 10.3, int8 2960 x 1664 at 97
+  // 10.8 / 11.9, int4 592 x 1280 at 776 9.6 / 10.3.
+  const bool no_more = kind >= 4 ? K > 768 && K <= (kind == 4 ? 1536 : 3072) : !in_lds && (K <= 3072 || (kind == 0 && table_rows <= 16384));
+  const float behind_decode = no_more ? 0.f : p.splits > 1 && kind != 4 ? 1.75f : 0.75f;
   const float product = fmaxf(host, decode + (own ? p.us + behind_decode : library));
   // What the blocks take past their estimate where the product is close: int4 of some steps on compute units that are full, and the second
   // table of a residual layer whose first the L1s serve.  Decode + product / blocks: int4 8192 x 4096 at 160 tokens 35.5 / 42.0 (38.4 by the
