@@ -4,10 +4,12 @@
 // What bounds the band's small shapes in a library GEMM is not the arithmetic: a few dozen output tiles leave most compute
 // units idle, each walks all of K with little in flight, and the call costs the host more than both kernels together.  Two
 // kernels serve the band here.  The wide tiles (wide_gemm.hpp, 64 x 64 to 256 x 256) have a wave per 16 MT x 16 NT of the tile and one ring of
-// 64-k steps; which of them a shape takes, and whether K is split over blocks, the plan below estimates.  The kernel in this file is for what
-// is left without a tile for every compute unit even at 64 x 64, or is a long chain of steps for few: a block keeps a tile of 32 x 64 and splits K over
-// four waves (wave g takes every fourth 64-k step), 8 KiB of operands per step each on their way three steps deep, and the waves' sums meet in
-// LDS, in their order, without a second kernel or a workspace (47 x 384 x 8320 unsplit 16.3 us, the library's product 19.0; 90 x 609 x 13312 28).
+// 64-k steps; which of them a shape takes, and whether K is split over blocks, the plan below estimates.  The kernel in this file splits K over groups of
+// waves inside the block (group g takes every KG-th step), and the groups' sums meet in LDS, in their order, without a second kernel or a workspace.  It has two tiles.
+// 32 x 64 in four groups of a wave is for what is left without a tile for every compute unit even at 64 x 64, or is a long chain of steps for few: 8 KiB of operands per
+// step on their way three steps deep (47 x 384 x 8320 unsplit 16.3 us, the library's product 19.0; 90 x 609 x 13312 28).  64 x 128 in two groups of
+// four waves is for long K over few tiles, next to parts of K over blocks: half as many steps one behind the other as in a part of a wide tile.  Decode + product, us, best of all wide
+// tiles and splits / this: 548 x 320 x 9728 20.0 / 17.6, 444 x 352 x 9856 19.7 / 17.2, 370 x 659 x 12800 28.9 / 26.6, 709 x 501 x 10880 30.7 / 25.3, 1160 x 403 x 10112 35.0 / 32.7.
 //
 // Long reductions over few output tiles leave most of the chip idle all the same, here as in the library.  There K is split over blocks
 // too (`splits` parts of equal length, give or take a step): every block stores its f32 tile to the workspace and splitk_reduce_kernel adds
@@ -15,8 +17,8 @@
 //
 // Both operand tiles are loaded straight into LDS (global_load_lds_dwordx4; rows of 128 bytes, 16-byte piece p of
 // row r in slot p ^ ((r >> 1) & 7), so that a read of 32 consecutive rows touches every bank group twice), a ring of
-// kStages steps per group; one in-order counter tracks a wave's loads and the waits are written by hand.  A wave
-// computes 32 MT x 64 of the tile (MFMA 32x32x16), reading the operands of a k group while it multiplies the one
+// kDenseRing steps per group; one in-order counter tracks a wave's loads and the waits are written by hand.  A wave
+// computes 32 x 64 of the tile (MFMA 32x32x16), reading the operands of a k group while it multiplies the one
 // before.
 // Rows that end inside a step (SHORT) are read where they lie: residual VQ 1157 x 272 at 471 tokens 21.7 -> 9.1 us per call (the library's product
 // before), VQ 1920 x 288 at 1590 tokens 13.1 -> 10.8 (x copied to rows of whole steps).
@@ -35,9 +37,12 @@ namespace npamd {
 
 namespace {
 
-template <int WGM, int WGN, int MT, int KG, int STAGES>
+constexpr int kDenseRing = 3;  // steps of a group of waves in LDS
+
+// WGM x WGN waves of 32 x 64 and KG groups of them, each with a part of the steps.
+template <int WGM, int WGN, int KG>
 struct DenseTile {
-  static constexpr int kBM = 32 * MT * WGM, kBN = 64 * WGN;
+  static constexpr int kBM = 32 * WGM, kBN = 64 * WGN;
   static constexpr int kWaves = WGM * WGN;  // of one K group
   static constexpr int kThreads = 64 * kWaves * KG;
   static constexpr int kStageBytes = (kBM + kBN) * 128;
@@ -45,17 +50,17 @@ struct DenseTile {
   static constexpr int kLoadsX = (kPiecesX + kWaves - 1) / kWaves, kLoadsW = (kPiecesW + kWaves - 1) / kWaves;  // per wave and step
   static constexpr int kRedBytes = (KG - 1) * kBM * kBN * 4;
   static constexpr int kEpBytes = kBM * kBN * 2;
-  static constexpr int kRingBytes = KG * STAGES * kStageBytes;
+  static constexpr int kRingBytes = KG * kDenseRing * kStageBytes;
   static constexpr int kLds = kRingBytes > kRedBytes + kEpBytes ? kRingBytes : kRedBytes + kEpBytes;
   static_assert(kLds <= kLdsPerBlockMax, "the block's tiles do not fit LDS");
 };
 
 // SHORT: rows end inside the last step.  Loads past their end bring the last piece again, and the operands there are zeroed
 // as they are used, in the one step that has any.
-template <int ACT, int WGM, int WGN, int MT, int KG, int STAGES, bool SHORT = false>
-__global__ void __launch_bounds__((DenseTile<WGM, WGN, MT, KG, STAGES>::kThreads))
+template <int ACT, int WGM, int WGN, int KG, bool SHORT>
+__global__ void __launch_bounds__((DenseTile<WGM, WGN, KG>::kThreads))
 dense_gemm_kernel(const DenseShape s) {
-  using T = DenseTile<WGM, WGN, MT, KG, STAGES>;
+  using T = DenseTile<WGM, WGN, KG>;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   // blockIdx.x % 8 names the die; a die takes an eighth of the units, counted down the columns
   const int unit = (blockIdx.x & 7) * s.units_per_die + (blockIdx.x >> 3);
@@ -88,7 +93,7 @@ dense_gemm_kernel(const DenseShape s) {
     const int row = is_x ? min(r, s.M - 1 - m0) : min(r, s.N - 1 - n0);  // rows past the end: a valid row nobody stores
     voff[i] = (uint32_t)((int64_t)row * (is_x ? s.ldx : s.ldw) * 2) + (SHORT ? 0u : (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16));
   }
-  const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + (uint32_t)(g * STAGES * T::kStageBytes);
+  const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + (uint32_t)(g * kDenseRing * T::kStageBytes);
   auto load = [&](int i, int slot, int it) {
     const bool is_x = i < T::kLoadsX;
     const uint32_t piece = (uint32_t)((is_x ? 0 : T::kPiecesX) + piece_of(i));
@@ -102,17 +107,15 @@ dense_gemm_kernel(const DenseShape s) {
     lds_load16(ring + (uint32_t)(slot * T::kStageBytes) + piece * 1024u, voff[i], src);
   };
 
-  f32x16 acc[MT][2];
+  f32x16 acc[1][2];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[mt][t][i] = 0.f;
+    for (int i = 0; i < 16; ++i) acc[0][t][i] = 0.f;
 
   constexpr int kLoads = T::kLoadsX + T::kLoadsW;
 #pragma unroll
-  for (int p = 0; p < STAGES - 1; ++p)
+  for (int p = 0; p < kDenseRing - 1; ++p)
     if (p < steps_g) {
 #pragma unroll
       for (int i = 0; i < kLoads; ++i) load(i, p, p);
@@ -121,14 +124,13 @@ dense_gemm_kernel(const DenseShape s) {
   uint32_t slot_off[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) slot_off[j] = (uint32_t)((((h << 2) | j) ^ ((c >> 1) & 7)) << 4);
-  const uint8_t* const ring_p = lds + g * STAGES * T::kStageBytes;
-  const uint32_t a_off = (uint32_t)((wm * 32 * MT + c) * 128), b_off = (uint32_t)((T::kBM + wn * 64 + c) * 128);
-  u32x4 ao[2][MT], bo[2][2];
+  const uint8_t* const ring_p = lds + g * kDenseRing * T::kStageBytes;
+  const uint32_t a_off = (uint32_t)((wm * 32 + c) * 128), b_off = (uint32_t)((T::kBM + wn * 64 + c) * 128);
+  u32x4 ao[2], bo[2][2];
   auto read_ops = [&](int set, const uint8_t* stage, int j) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) bo[set][t] = *reinterpret_cast<const u32x4*>(stage + b_off + t * 4096 + slot_off[j]);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) ao[set][mt] = *reinterpret_cast<const u32x4*>(stage + a_off + mt * 4096 + slot_off[j]);
+    ao[set] = *reinterpret_cast<const u32x4*>(stage + a_off + slot_off[j]);
   };
 
   // One step out of ring slot `slot`: the operands of k group j + 1 are read in front of the MFMAs of group j, and with
@@ -137,7 +139,7 @@ dense_gemm_kernel(const DenseShape s) {
   auto compute = [&](auto loads, int slot, int ahead, int there) {
     constexpr bool LOADS = decltype(loads)::value;
     const uint8_t* const stage = ring_p + slot * T::kStageBytes;
-    const int into = slot == 0 ? STAGES - 1 : slot - 1;
+    const int into = slot == 0 ? kDenseRing - 1 : slot - 1;
     read_ops(0, stage, 0);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -146,14 +148,12 @@ dense_gemm_kernel(const DenseShape s) {
         const bool dead = 4 * h + j >= there;
 #pragma unroll
         for (int t = 0; t < 2; ++t) bo[j & 1][t] = dead ? u32x4{0, 0, 0, 0} : bo[j & 1][t];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) ao[j & 1][mt] = dead ? u32x4{0, 0, 0, 0} : ao[j & 1][mt];
+        ao[j & 1] = dead ? u32x4{0, 0, 0, 0} : ao[j & 1];
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[mt][t] = mfma32<ACT>(ao[j & 1][mt], bo[j & 1][t], acc[mt][t]);
+        acc[0][t] = mfma32<ACT>(ao[j & 1], bo[j & 1][t], acc[0][t]);
         if constexpr (LOADS) {
 #pragma unroll
           for (int i = (j * 2 + t) * kLoads / 8; i < (j * 2 + t + 1) * kLoads / 8; ++i) load(i, into, ahead);
@@ -162,35 +162,30 @@ dense_gemm_kernel(const DenseShape s) {
       }
     }
   };
-  // The wave's own pieces of a step have arrived when only those of `young` younger steps are still on their way.
-  auto wait_young = [&](int young) {
-    if (young >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * kLoads < 63 ? 3 * kLoads : 63) : "memory");
-    else if (young == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoads) : "memory");
-    else if (young == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  };
   auto pieces_there = [&](int it) { return s.pieces - (step0 + g + KG * it) * 8; };
   int slot = 0;
-  auto next_slot = [&] { slot = slot == STAGES - 1 ? 0 : slot + 1; };
+  auto next_slot = [&] { slot = slot == kDenseRing - 1 ? 0 : slot + 1; };
   int it = 0;
   // Steps every group has, while there is something left to request.
-  for (; it < base - (STAGES - 1); ++it) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * kLoads) : "memory");
+  for (; it < base - (kDenseRing - 1); ++it) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kDenseRing - 2) * kLoads) : "memory");
     block_sync_lds();  // everybody's pieces have arrived, and nobody reads the slot of the step before any more
-    compute(std::true_type{}, slot, it + STAGES - 1, 8);
+    compute(std::true_type{}, slot, it + kDenseRing - 1, 8);
     next_slot();
   }
   for (; it < base; ++it) {
-    wait_young(base - 1 - it);
+    // The step's pieces have arrived when only those of the one behind it are still on their way.
+    if (it == base - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     block_sync_lds();
-    if (it + STAGES - 1 < steps_g) {  // the last step of a group that has one more than the others
+    if (it + kDenseRing - 1 < steps_g) {  // the last step of a group that has one more than the others
 #pragma unroll
-      for (int i = 0; i < kLoads; ++i) load(i, slot == 0 ? STAGES - 1 : slot - 1, it + STAGES - 1);
+      for (int i = 0; i < kLoads; ++i) load(i, slot == 0 ? kDenseRing - 1 : slot - 1, it + kDenseRing - 1);
     }
     compute(std::false_type{}, slot, 0, pieces_there(it));
     next_slot();
   }
-  if (KG > 1 && steps % KG) {
+  if (steps % KG) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     block_sync_lds();
     if (base < steps_g) compute(std::false_type{}, slot, 0, pieces_there(base));
@@ -198,34 +193,28 @@ dense_gemm_kernel(const DenseShape s) {
 
   // The groups' sums meet in group 0, in group order.
   __syncthreads();
-  if constexpr (KG > 1) {
-    if (g > 0) {
-      float* mine = reinterpret_cast<float*>(lds) + ((size_t)(g - 1) * T::kWaves + wave) * (MT * 2 * 1024) + lane * 4;
+  if (g > 0) {
+    float* mine = reinterpret_cast<float*>(lds) + ((size_t)(g - 1) * T::kWaves + wave) * 2048 + lane * 4;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(mine + (t * 4 + q) * 256) =
+            f32x4{acc[0][t][4 * q], acc[0][t][4 * q + 1], acc[0][t][4 * q + 2], acc[0][t][4 * q + 3]};
+  }
+  __syncthreads();
+  if (g > 0) return;
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            *reinterpret_cast<f32x4*>(mine + ((mt * 2 + t) * 4 + q) * 256) =
-                f32x4{acc[mt][t][4 * q], acc[mt][t][4 * q + 1], acc[mt][t][4 * q + 2], acc[mt][t][4 * q + 3]};
-    }
-    __syncthreads();
-    if (g > 0) return;
+  for (int o = 0; o < KG - 1; ++o) {
+    const float* theirs = reinterpret_cast<const float*>(lds) + ((size_t)o * T::kWaves + wave) * 2048 + lane * 4;
 #pragma unroll
-    for (int o = 0; o < KG - 1; ++o) {
-      const float* theirs = reinterpret_cast<const float*>(lds) + ((size_t)o * T::kWaves + wave) * (MT * 2 * 1024) + lane * 4;
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(theirs + (t * 4 + q) * 256);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(theirs + ((mt * 2 + t) * 4 + q) * 256);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[mt][t][4 * q + e] += v[e];
-          }
-    }
+        for (int e = 0; e < 4; ++e) acc[0][t][4 * q + e] += v[e];
+      }
   }
   if (s.splits > 1) {
     // D[m = 8 (i / 4) + 4 h + i % 4][n = c] of each 32 x 32 tile
@@ -235,22 +224,19 @@ dense_gemm_kernel(const DenseShape s) {
       const int n = n0 + wn * 64 + t * 32 + c;
       if (n >= s.N) continue;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int m = m0 + wm * 32 * MT + mt * 32 + 8 * (i / 4) + 4 * h + (i % 4);
-          if (m < s.M) mine[(size_t)m * s.N + n] = acc[mt][t][i];
-        }
+      for (int i = 0; i < 16; ++i) {
+        const int m = m0 + wm * 32 + 8 * (i / 4) + 4 * h + (i % 4);
+        if (m < s.M) mine[(size_t)m * s.N + n] = acc[0][t][i];
+      }
     }
     return;
   }
-  store_wave_tile<ACT, MT, 2>(acc, lds + T::kRedBytes + wave * (32 * MT * 128), lane, s.y, s.ldy, m0 + wm * 32 * MT, n0 + wn * 64,
-                              s.M, s.N, s.bias);
+  store_wave_tile<ACT, 1, 2>(acc, lds + T::kRedBytes + wave * 4096, lane, s.y, s.ldy, m0 + wm * 32, n0 + wn * 64, s.M, s.N, s.bias);
 }
 
-template <int ACT, int WGM, int WGN, int MT, int KG, int STAGES>
+template <int ACT, int WGM, int WGN, int KG>
 int launch_dense_tile(DenseShape s, hipStream_t st) {
-  using T = DenseTile<WGM, WGN, MT, KG, STAGES>;
+  using T = DenseTile<WGM, WGN, KG>;
   s.row_tiles = (s.M + T::kBM - 1) / T::kBM;
   s.col_tiles = (s.N + T::kBN - 1) / T::kBN;
   const int64_t units = (int64_t)s.col_tiles * s.row_tiles * s.splits, blocks = (units + 7) / 8 * 8;
@@ -258,7 +244,7 @@ int launch_dense_tile(DenseShape s, hipStream_t st) {
   if (blocks > 0x7FFFFFFF) return fail(NPAMD_ERR_UNSUPPORTED, "npamd_dense_gemm: too many tiles");
   static LdsLatch latches[2];
   const bool ends_inside = s.pieces % 8 != 0;
-  const auto kernel = ends_inside ? dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES, true> : dense_gemm_kernel<ACT, WGM, WGN, MT, KG, STAGES, false>;
+  const auto kernel = ends_inside ? dense_gemm_kernel<ACT, WGM, WGN, KG, true> : dense_gemm_kernel<ACT, WGM, WGN, KG, false>;
   const hipError_t e = enable_dynamic_lds(latches[ends_inside], reinterpret_cast<const void*>(kernel), T::kLds);
   if (e != hipSuccess)
     return fail(NPAMD_ERR_LAUNCH, "npamd_dense_gemm: cannot reserve %d bytes of LDS: %s", T::kLds, hipGetErrorString(e));
@@ -291,12 +277,15 @@ constexpr DenseCost kDenseCost[] = {
     {256, 256, 1, 2.163f, 0.853f, 0.073f, 7.682f},
     {96, 64, 1, 1.473f, 0.198f, 0.038f, 2.770f},
     {192, 192, 1, 0.000f, 0.487f, 0.055f, 8.035f},
+    {64, 128, 2, 2.600f, 0.440f, 0.020f, 0.000f},  // the kernel above again; where the plan looks at it
 };
-constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]);
+constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]), kDenseTwoGroups = kDenseTiles - 1;
 
 template <int ACT>
 int launch_dense(const DenseShape& s, int tile, hipStream_t st) {
-  const int rc = tile > 0 ? launch_wide(s, ACT, tile, st) : launch_dense_tile<ACT, 1, 1, 1, 4, 3>(s, st);
+  const int rc = tile == 0 ? launch_dense_tile<ACT, 1, 1, 4>(s, st)
+                 : tile == kDenseTwoGroups ? launch_dense_tile<ACT, 2, 2, 2>(s, st)
+                                           : launch_wide(s, ACT, tile, st);
   if (rc != NPAMD_OK || s.splits == 1) return rc;
   launch_splitk_reduce<ACT>(s.partials, s.splits, s.M, s.N, s.bias, s.y, s.ldy, st);
   return check_launch("npamd_dense_gemm");
@@ -317,8 +306,10 @@ struct DensePlan {
   float us;
 };
 
-// The tile and split of least estimate.  The wide tiles address their part of the result with 31 bits: with rows of y, or columns, that
-// could lie further apart than that, the other kernel.
+// The tile and split of least estimate.  64 x 128 in two groups is looked at in parts of one round, on up to 40 tiles of at least 320 rows and K from 5120 on: of 97 such
+// products that it takes, behind a decode, 60 are more than 3 % faster than without it (36 more than 8 %) and 23 slower (9), 4 % in the mean; with more tiles, on fewer rows, or whole,
+// it loses more calls than it gains.  The wide tiles address their part of the result with 31 bits: with rows of y, or columns, that
+// could lie further apart than that, the other kernel's.
 DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits, bool wide = true) {
   DensePlan best{0, 1, 1e30f};
   const int steps = K / 64;
@@ -326,7 +317,8 @@ DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits, bool 
   const int forced_splits = forced < most ? forced : most;
   const int last = wide && N < kDenseStrideMax ? kDenseTiles : 1;
   for (int i = 0; i < last; ++i) {
-    if (last > 1 && forced_tile > 0 && forced_tile <= kDenseTiles && i != forced_tile - 1) continue;
+    const bool forced_one = last > 1 && forced_tile > 0 && forced_tile <= kDenseTiles;
+    if (forced_one && i != forced_tile - 1) continue;
     const DenseCost& c = kDenseCost[i];
     const int64_t tiles = (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
     const float load = (float)tiles * steps * (c.bm + c.bn) * 128e-6f * c.per_mb;
@@ -334,6 +326,7 @@ DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits, bool 
       if (forced_splits > 0 && splits != forced_splits) continue;
       if (forced_splits <= 0 && splits > 1 && (splits > kDensePlannedSplits || steps < kDenseMinSplitSteps * splits || tiles * splits > 512)) break;
       const int64_t rounds = ((tiles * splits + 7) / 8 + 31) / 32;
+      if (i == kDenseTwoGroups && !forced_one && (splits == 1 || rounds > 1 || tiles > 40 || M < 320 || steps < 80)) continue;
       const int part = (steps + splits - 1) / splits;
       const float walk = (float)rounds * ((part + c.groups - 1) / c.groups) * c.per_step;
       float t = c.fixed + (float)rounds * c.per_round + (splits > 1 ? kDenseSplitFixed + kDenseSplitPerMb * (4e-6f * splits * M * N) : 0.f);

@@ -23,7 +23,7 @@ def dense_tile(monkeypatch):
 
 
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6, 7, 15])
 def test_dense_gemm_tiles(gpu, dense_tile, tile, act):
     from neuropress_amd import kernels
 
@@ -46,7 +46,7 @@ def test_dense_gemm_tiles(gpu, dense_tile, tile, act):
 
 
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("tile,splits", [(1, 2), (1, 16), (2, 9), (3, 3), (4, 8), (5, 7), (6, 2), (7, 3)])
+@pytest.mark.parametrize("tile,splits", [(1, 2), (1, 16), (2, 9), (3, 3), (4, 8), (5, 7), (6, 2), (7, 3), (15, 2), (15, 8)])
 def test_dense_gemm_parts_of_k(gpu, dense_tile, monkeypatch, tile, splits, act):
     """K in parts over blocks: parts of unequal length, of fewer steps than a ring is deep or a block has groups of
     waves, columns the reduction reads four at a time and not."""
