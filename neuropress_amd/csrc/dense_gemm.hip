@@ -478,18 +478,24 @@ extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int ta
   return blocks < us ? 1 : 0;
 }
 
-// Where this product is the better one against the library's.  That takes 18.3-19 us per eager call whatever its size and 33 us go by between two
-// calls of decode + library product, whatever the GPU does meanwhile; past that its kernels are the slower ones but where its tiles of
-// 256 x 256 fit: M and N whole multiples, and rounds of them on all compute units that are at least 0.85 full.  Of 112 products with such M and N, us, library / this,
-// fp16 and bf16: 4096 x 4096 x 4096 93.4 / 103.6 and 89.7 / 95.5, 2048 x 8192 x 2048 53.0 / 56.6 and 52.7 / 54.2, 3072 x 5120 x 5120 117.9 / 118.2 and
-// 112.6 / 117.8, 4096 x 14336 x 4096 358 / 381 and 347 / 366, 2048 x 14336 x 4096 191.9 / 187.4 and 173.4 / 180.1; less full 4096 x 6144 x 4096 174.5 / 177.6 and
-// 166.3 / 157.8, 2048 x 11008 x 4096 170.3 / 150.0 and 162.0 / 145.6, 4096 x 11008 x 4096 418 / 284 and 412 / 278, 1024 x 4096 x 4096 44.3 / 37.8 and 38.6 / 36.8.  Any
-// other M and N, 300 products of 0.3 to 490 GFLOP: 0.95 to 1.64 x from 25 GFLOP on, 1.2 in the mean (1646 x 13120 x 11136 fp16 690 / 444, 2355 x 3424 x 1792 37.9 / 30.0,
-// 3552 x 8681 x 7616 368 / 330); below, the library's kernel alone 0.5 to 1.5 x, its call 18.3 us and more.
+// Where this product is the better one against the library's.  That takes 18.3-19 us per eager call whatever its size and 33 us go by between two calls of
+// decode + library product, whatever the GPU does meanwhile: below 64 GFLOP this one.  Past that the library's kernels are ahead where its tiles of 256 x 256, those at the edges
+// counted whole, fill their rounds of all compute units, the more of a product the less they have to.  Of 3728 products of 10 to 5000 GFLOP, K from 64 to 28672, fp16 and bf16, this one's time over the library's
+// (median, quarters): rounds at least 0.98 full, 64 to 300 GFLOP 1.05 (1.03 to 1.06), to 1600 1.08, past that 1.13; 0.9 to 0.98 full, to 300 GFLOP 0.97 (0.87 to 1.04), to
+// 800 1.03 (0.92 to 1.08), to 1600 1.05, past that 1.08; 0.86 to 0.9 full, past 1600 GFLOP 1.11; less full 0.87 to 0.97 (the library is 10 % and more ahead on one in twenty of those, by
+// no size that tells which: 1024 x 9728 x 14336 239 / 299 us, 1024 x 13824 x 13824 479 / 327).  Rounds of exactly seven eighths are level up to 14336 columns and the library's by 7 % past them, unlike their
+// neighbours (4096 x 14336 x 4096 in bf16 331 to 336 / 336 to 341, fp16 348 to 351 / 352; 4096 x 11008 x 4096, 0.896 full, 405 / 262); so are both types.  Where K is short (512 to 768: 0.81 up to
+// 64 GFLOP, 1.05 up to 300) or N no multiple of 8 (0.95 up to 300 GFLOP) the line is at 300.  Library / this, us: 4095 x 4096 x 4096 bf16 92.7 / 97.9, 8000 x 4096 x 14336 590 / 695,
+// 2842 x 64000 x 4992 1265 / 1652, 5000 x 128256 x 2048 1957 / 2282; 4096 x 6144 x 4096 174.5 / 177.6 and bf16 166.3 / 157.8, 1646 x 13120 x 11136 690 / 444.
 extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {
   if (M < 1 || N < 1 || K < 64 || K % 64 || K >= kDenseStrideMax) return 0;
   const int forced = tuning().dense_tile;
   if (forced) return forced > 0;
-  const int64_t tiles = (int64_t)(M / 256) * (N / 256), rounds = (tiles + 255) / 256;
-  return M % 256 == 0 && N % 256 == 0 && K >= 768 && tiles >= 0.85 * 256 * rounds ? 0 : 1;
+  if (N >= kDenseStrideMax) return 0;  // the wide tiles do not take it
+  const double gflop = 2e-9 * M * N * K;
+  const int64_t tiles = (((int64_t)M + 255) / 256) * ((N + 255) / 256), rounds = (tiles + 255) / 256;
+  const double full = tiles / (256.0 * rounds);
+  const bool whole = full >= 0.98 || 8 * tiles == 7 * 256 * rounds;
+  if (gflop < 300) return gflop >= 64 && K >= 768 && N % 8 == 0 && whole ? 0 : 1;
+  return whole || (gflop >= 800 && full >= 0.9) || (gflop >= 1600 && full >= 0.86) ? 0 : 1;
 }

@@ -9,3 +9,16 @@ from neuropress_amd import _lib
 def test_long_k_over_few_tiles(m, n, k, parts):
     """As many parts of K as make one round of 64 x 128 tiles, up to eight: the tile in two groups.  With wide tiles alone 5, 6, 3 and 4 parts, 8 to 15 % slower."""
     assert _lib.load().npamd_dense_gemm_workspace_bytes(m, n, k) == parts * m * n * 4
+
+
+# Products (tokens, rows, columns) that one of the two serves faster, by 3 % and more on both types; the last is one that no wide tile takes.
+LIBRARY = [(4095, 4096, 4096), (4096, 4096, 4096), (4000, 8192, 8192), (3500, 4096, 14336), (8000, 4096, 14336), (2842, 64000, 4992), (14422, 16128, 5760), (32461, 37751, 640),
+           (5000, 128256, 2048), (3500, 32000, 4096), (6144, 14336, 8192), (3000, 28672, 8192), (64, 1 << 22, 64)]  # fmt: skip
+PACKAGE = [(1646, 13120, 11136), (2048, 4096, 4096), (4096, 11008, 4096), (4000, 11008, 4096), (3072, 9728, 12288), (2687, 10983, 7232), (4096, 11008, 1280), (2789, 11008, 1664),
+           (2048, 13824, 13824), (384, 4096, 4096), (777, 1280, 8192)]  # fmt: skip
+
+
+def test_line_to_the_library():
+    preferred = _lib.load().npamd_dense_gemm_preferred
+    assert [p for p in LIBRARY if preferred(*p)] == []
+    assert [p for p in PACKAGE if not preferred(*p)] == []

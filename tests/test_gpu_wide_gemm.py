@@ -1,5 +1,5 @@
 """The wide tiles of the dense product around their edges: rows and columns one off a tile, fewer steps of K than a ring is deep, rows that
-end inside a step, columns that leave as whole pieces and one by one, K in parts whose sums are stored either way; and which calls go to the library."""
+end inside a step, columns that leave as whole pieces and one by one, K in parts whose sums are stored either way."""
 
 import pytest
 import torch
@@ -75,11 +75,3 @@ def test_rows_past_a_product(gpu, tuned):
                                         torch.cuda.current_stream().cuda_stream) == 0  # fmt: skip
             assert torch.allclose(y[:m, :n].float(), x.float() @ w.float().T, rtol=2e-3, atol=2e-3)
             assert bool((y[m:] == 7).all()) and bool((y[:, n:] == 7).all()), (tile, n)
-
-
-def test_line_to_the_library():
-    from neuropress_amd import _lib
-
-    preferred = _lib.load().npamd_dense_gemm_preferred
-    assert not preferred(4096, 4096, 4096) and not preferred(2048, 8192, 2048)  # whole rounds of 256 x 256
-    assert preferred(4095, 4096, 4096) and preferred(4096, 4095, 4096) and preferred(2048, 4096, 4096) and preferred(1646, 13120, 11136)
