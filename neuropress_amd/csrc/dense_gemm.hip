@@ -26,7 +26,9 @@
 // fetches a column tile of W once for all row tiles.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "dense_gemm.hpp"
 #include "gemm_tile.hpp"
@@ -306,33 +308,60 @@ struct DensePlan {
   float us;
 };
 
+template <size_t... I>
+void count_tiles(int M, int N, int64_t* tiles, std::index_sequence<I...>) {
+  ((tiles[I] = (int64_t)((M - 1) / kDenseCost[I].bm + 1) * ((N - 1) / kDenseCost[I].bn + 1)), ...);
+}
+
 // The tile and split of least estimate.  64 x 128 in two groups is looked at in parts of one round, on up to 40 tiles of at least 320 rows and K from 5120 on: of 97 such
 // products that it takes, behind a decode, 60 are more than 3 % faster than without it (36 more than 8 %) and 23 slower (9), 4 % in the mean; with more tiles, on fewer rows, or whole,
 // it loses more calls than it gains.  The wide tiles address their part of the result with 31 bits: with rows of y, or columns, that
 // could lie further apart than that, the other kernel's.
+//
+// Every call of the band is planned, one at a new token count three times: sizes are divided by constants, and the parts of a tile are looked at only while what they cannot go
+// below (their bytes, their share of the walk and the sum) is less than the best so far.  us on the host, all tiles and parts in turn / so: 384 x 4096 x 4096
+// 0.61 / 0.17, 77 x 3003 x 2176 0.83 / 0.16, 64 x 1024 x 4096 0.87 / 0.32, 528 x 336 x 13440 0.94 / 0.56.
 DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits, bool wide = true) {
   DensePlan best{0, 1, 1e30f};
   const int steps = K / 64;
   const int forced = tuning().dense_splits, most = max_splits < steps ? max_splits : steps;
   const int forced_splits = forced < most ? forced : most;
-  const int last = wide && N < kDenseStrideMax ? kDenseTiles : 1;
-  for (int i = 0; i < last; ++i) {
-    const bool forced_one = last > 1 && forced_tile > 0 && forced_tile <= kDenseTiles;
-    if (forced_one && i != forced_tile - 1) continue;
+  wide = wide && N < kDenseStrideMax;
+  const int only = wide && forced_tile > 0 && forced_tile <= kDenseTiles ? forced_tile - 1 : wide ? -1 : 0;
+  int64_t tiles[kDenseTiles];
+  count_tiles(M, N, tiles, std::make_index_sequence<kDenseTiles>{});
+  const bool two_groups = only >= 0 || (tiles[kDenseTwoGroups] <= 40 && M >= 320 && steps >= 80);
+  auto load = [&](int i) { return (float)tiles[i] * steps * (kDenseCost[i].bm + kDenseCost[i].bn) * 128e-6f * kDenseCost[i].per_mb; };
+  auto look = [&](int i, int splits, int part, float bytes, float sum) {
     const DenseCost& c = kDenseCost[i];
-    const int64_t tiles = (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-    const float load = (float)tiles * steps * (c.bm + c.bn) * 128e-6f * c.per_mb;
-    for (int splits = 1; splits <= max_splits; ++splits) {
-      if (forced_splits > 0 && splits != forced_splits) continue;
-      if (forced_splits <= 0 && splits > 1 && (splits > kDensePlannedSplits || steps < kDenseMinSplitSteps * splits || tiles * splits > 512)) break;
-      const int64_t rounds = ((tiles * splits + 7) / 8 + 31) / 32;
-      if (i == kDenseTwoGroups && !forced_one && (splits == 1 || rounds > 1 || tiles > 40 || M < 320 || steps < 80)) continue;
-      const int part = (steps + splits - 1) / splits;
-      const float walk = (float)rounds * ((part + c.groups - 1) / c.groups) * c.per_step;
-      float t = c.fixed + (float)rounds * c.per_round + (splits > 1 ? kDenseSplitFixed + kDenseSplitPerMb * (4e-6f * splits * M * N) : 0.f);
-      if (t + fmaxf(walk, load) >= best.us) continue;
-      t += sqrtf(walk * walk + load * load);
-      if (t < best.us) best = {i, splits, t};
+    const int64_t rounds = ((tiles[i] * splits + 7) / 8 + 31) / 32;
+    if (i == kDenseTwoGroups && only < 0 && (splits == 1 || rounds > 1 || !two_groups)) return;
+    const float walk = (float)rounds * ((part + c.groups - 1) / c.groups) * c.per_step;
+    float t = c.fixed + (float)rounds * c.per_round + sum;
+    if (t + fmaxf(walk, bytes) >= best.us) return;
+    t += sqrtf(walk * walk + bytes * bytes);
+    if (t < best.us) best = {i, splits, t};
+  };
+  const int first = only < 0 ? 0 : only, last = only < 0 ? kDenseTiles : only + 1;
+  if (forced_splits <= 1)
+    for (int i = first; i < last; ++i) look(i, 1, steps, load(i), 0.f);
+  if (forced_splits == 1 || max_splits < 2) return best;
+  const float mb = 4e-6f * M * N;
+  if (forced_splits > 1) {
+    const int part = (steps + forced_splits - 1) / forced_splits;
+    for (int i = first; i < last; ++i) look(i, forced_splits, part, load(i), kDenseSplitFixed + kDenseSplitPerMb * mb * forced_splits);
+    return best;
+  }
+  const int parts = std::min(std::min(max_splits, kDensePlannedSplits), steps / kDenseMinSplitSteps);
+  int part_of[kDensePlannedSplits + 1];
+  for (int splits = 2; splits <= parts; ++splits) part_of[splits] = (steps + splits - 1) / splits;
+  for (int i = first; i < last; ++i) {
+    const DenseCost& c = kDenseCost[i];
+    const float bytes = load(i), least = c.fixed + c.per_round + kDenseSplitFixed + fmaxf(bytes, tiles[i] * steps / (256.f * c.groups) * c.per_step);
+    for (int splits = 2; splits <= parts && tiles[i] * splits <= 512; ++splits) {
+      const float sum = kDenseSplitPerMb * mb * splits;
+      if (least + sum >= best.us) break;
+      look(i, splits, part_of[splits], bytes, kDenseSplitFixed + sum);
     }
   }
   return best;
