@@ -279,7 +279,7 @@ constexpr DenseCost kDenseCost[] = {
     {256, 256, 1, 2.163f, 0.853f, 0.073f, 7.682f},
     {96, 64, 1, 1.473f, 0.198f, 0.038f, 2.770f},
     {192, 192, 1, 0.000f, 0.487f, 0.055f, 8.035f},
-    {64, 128, 2, 2.600f, 0.440f, 0.020f, 0.000f},  // the kernel above again; where the plan looks at it
+    {64, 128, 2, 3.600f, 0.440f, 0.020f, 0.000f},  // the kernel above again; where the plan looks at it
 };
 constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]), kDenseTwoGroups = kDenseTiles - 1;
 
@@ -313,8 +313,8 @@ void count_tiles(int M, int N, int64_t* tiles, std::index_sequence<I...>) {
   ((tiles[I] = (int64_t)((M - 1) / kDenseCost[I].bm + 1) * ((N - 1) / kDenseCost[I].bn + 1)), ...);
 }
 
-// The tile and split of least estimate.  64 x 128 in two groups is looked at in parts of one round, on up to 40 tiles of at least 320 rows and K from 5120 on: of 97 such
-// products that it takes, behind a decode, 60 are more than 3 % faster than without it (36 more than 8 %) and 23 slower (9), 4 % in the mean; with more tiles, on fewer rows, or whole,
+// The tile and split of least estimate.  64 x 128 in two groups is looked at in parts of one round, on up to 40 tiles of at least 320 rows and K from 5120 on: of 74 such
+// products that it takes, behind a decode, 46 are more than 3 % faster than without it (28 more than 8 %) and 17 slower (5), 4.5 % in the mean; with more tiles, on fewer rows, or whole,
 // it loses more calls than it gains.  The wide tiles address their part of the result with 31 bits: with rows of y, or columns, that
 // could lie further apart than that, the other kernel's.
 //
@@ -414,9 +414,9 @@ extern "C" int npamd_dense_gemm_ragged(const void* x, int64_t ldx, const void* w
 // Whether a call of more than 16 tokens goes to the GEMV with a block per 32 tokens (npamd_*_gemv_blocks), or the table GEMM behind the same
 // entry (table_gemm.hip), rather than to decode + product or the tile GEMM.  Up to a round or two of its blocks it is one short launch in the place of two that follow each
 // other; past that every block of tokens decodes its weights again.  All three are estimated.  kind: 0 VQ, 1 residual VQ, 4 and 8 bits
-// per weight.  The GEMV's figures are fitted to layers of 512 to 8192 rows and K of 512 to 14336 at 33 to 512 tokens (within 10 %, on long rows up
-// to a third low, see gemv_blocks_long_rows_us; residual VQ as with indices that are all as frequent).  What the line sends there, 162 drawn calls past the
-// GEMV's own band: decode + product or tile GEMM / blocks 0.89 to 2.4 x, 1.24 to 1.66 x in the mean of each format and table.  us, before / blocks, at 64 and 256 tokens: int4 512 x 512 6.9 / 4.0 and 6.9 / 4.1,
+// per weight.  Codebooks in memory and residual VQ are estimated as with indices that are all as frequent, and with the tables of four layers in turn.  Of 3015 calls
+// near the line, 17 to 4096 tokens, two fifths of them seen by no fit, those that it sends to the slower side lose 0.8 % in the mean of all, 111 of them more than 8 % (the line before this
+// one, with corrections by format and range of K on the decode's side: 3.2 %, 416).  us, before / blocks, at 64 and 256 tokens: int4 512 x 512 6.9 / 4.0 and 6.9 / 4.1,
 // 1024 x 4096 11.8 / 6.4 and 13.3 / 9.5, 3072 x 3072 14.8 / 8.2; 256 rows 1024 x 1024 7.9 / 4.7 and 8.0 / 5.7, 2048 x 2048 10.4 / 5.7 and 11.1 / 11.2;
 // 4096 rows 1024 x 1024 8.1 / 4.7 and 8.1 / 6.6; 65536 rows 512 x 512 7.0 / 4.2 and 7.1 / 4.8, 1024 x 4096 13.2 / 10.0 and 16.5 / 24.8.
 namespace npamd {
@@ -427,36 +427,55 @@ static double library_us(int M, int N, int K) {
   return 5.0 + 2e-9 * M * N * K / rate + fmax(0.0, (K - 4096) / 1024.0) * 1.5;
 }
 
+// The blocks entry, us.  Of int4 / int8, of residual VQ and of tables that LDS does not hold: a start, what a round of the blocks that LDS holds at a time takes, and what its waves do, the
+// longest of them one step behind the other and all of a compute unit's together.  As their launchers choose them (launch_q_gemv; launch_fused_gemv with one
+// staged row tile); fitted to 1758 calls near the line, each format and table apart, K of 128 to 14336: within 4 to 6 % in the median of 725 others, 12 % in nine of ten.
 float gemv_blocks_us(int kind, int table_rows, int M, int N, int K) {
   constexpr int cus = 256;
   const int tokens = (M + kGemvTokens - 1) / kGemvTokens, rows = (N + 15) / 16, tiles = rows * tokens;
   const int steps = (K + 255) / 256, chunks = (K + 63) / 64, load = (tiles + cus - 1) / cus;
   auto per = [](int a, int b) { return (a + b - 1) / b; };
-  if (kind == 4) return 2.6f + 0.18f * load * steps + 0.7f * load;
-  if (kind == 8) return load <= 1 ? 3.3f + 0.24f * steps : 1.8f + per((rows + 1) / 2 * tokens, cus) * (3.4f + 0.25f * steps);
+  if (kind >= 4) {
+    const int item = 512 * kind + 256, load2 = per((rows + 1) / 2 * tokens, cus), four = std::min(steps, 4);  // LDS of a row tile's step; of pairs of row tiles
+    auto held = [&](int waves, int R) { return std::max(1, kGemvLdsPerBlockMax / (waves * (16384 + R * item))); };
+    bool two = steps >= 8 && load > 1 && 16 * load2 <= 9 * load;
+    if (tokens > 1) {
+      const int rounds1 = per(load, held(four, 1)), rounds2 = per(load2, held(four, 2));
+      two = rounds2 < rounds1 || (two && rounds2 == rounds1);
+    }
+    const int R = two ? 2 : 1, blocks = two ? load2 : load;
+    const int spw = per(steps, !two && load <= 1 && 8 * (16384 + item) <= kGemvLdsPerBlockMax ? 8 : 4), waves = per(steps, spw);
+    const int rounds = per(blocks, held(waves, R));
+    if (kind == 4) return 2.63f + 1.11f * rounds + 0.081f * blocks * R + hypotf(0.296f * spw * rounds, 0.212f * blocks * R * steps);
+    return 2.12f + 2.01f * rounds + hypotf(0.563f * spw * rounds, 0.205f * blocks * R * steps);
+  }
   const int table = table_rows * 16;
-  if (kind == 0 && table <= kGemvLdsCodebookMax && !gemv_wide_looks_up_in_memory(M, tiles, chunks, table)) {
+  if (kind == 0 && table <= kGemvLdsCodebookMax) {
+    if (gemv_wide_looks_up_in_memory(M, tiles, chunks, table)) {
+      const float lookups = 2.0f * K, served = table_rows <= 2048 ? 1100e3f : 275e3f;  // of a block; by the L1s, by the L2s
+      return 3.3f + load * lookups / 2400.f + tiles * lookups / served;
+    }
     const int R = gemv_wide_row_tiles(M, tiles, table);
     const int waves = R < 4 && table > 32 * 1024 ? 6 : 8, spw = per(steps, waves), rounds = per(per(rows, R) * tokens, cus);
     return 1.8f + rounds * (R == 1 ? 1.4f + 2.1f * spw : R == 2 ? 2.7f + 2.0f * spw : 8.5f + 3.0f * spw);
   }
-  const float lookups = 2.0f * K;  // of a block
-  const float served = table_rows <= 2048 ? 1100e3f : 275e3f;  // by the L1s; by the L2s
-  return (kind == 1 ? 4.1f : 3.3f) + load * lookups / 2400.f + tiles * lookups / served;
-}
-
-// What the figures of gemv_blocks_us, which the line against the tile GEMM was drawn with, leave out on rows of more than some 4096 columns:
-// a step of a wave takes longer where most compute units have a block, and a block's lookups in a large codebook, which no L2 has
-// yet, one after the other take their time however few blocks there are.  Decode + product / blocks, us: int8 1102 x 6656 at 358 tokens 24.4 / 28.5 (21.6 by
-// those figures, 28.2 by these), 691 x 6272 at 614 21.6 / 25.3, 377 x 8064 at 500 20.4 / 16.8, 820 x 7936 at 262 20.1 / 15.9; int4 1276 x 6400 at 362
-// 23.2 / 25.3, 265 x 5632 at 1082 20.2 / 21.5, 1658 x 5120 at 169 20.3 / 15.5, 404 x 7296 at 441 18.0 / 15.9; 65536 rows 491 x 6272 at 100
-// 14.3 / 16.6, 373 x 7296 at 62 14.6 / 20.1, 1308 x 4096 at 81 18.1 / 13.8; residual 679 x 7168 at 53 17.1 / 19.2, 1871 x 3968 at 35 20.2 / 14.7.
-static float gemv_blocks_long_rows_us(int kind, int table_rows, int M, int N, int K) {
-  const float us = gemv_blocks_us(kind, table_rows, M, N, K);
-  const int tokens = (M + kGemvTokens - 1) / kGemvTokens, rows = (N + 15) / 16, steps = (K + 255) / 256, load = (rows * tokens + 255) / 256;
-  if (kind == 4) return us + (steps > 16 ? 0.02f * load * steps : 0.f);
-  if (kind == 8) return load <= 1 ? us : fmaxf(us, 1.8f + ((rows + 1) / 2 * tokens + 255) / 256 * (1.5f + 0.45f * steps));
-  return table_rows > 16384 ? fmaxf(us, (kind == 1 ? 4.1f : 3.3f) + 2.0f * K / 960.f) : us;
+  // Lookups in memory.
+  int spw = std::max(per((kind == 1 ? rows : tiles) * steps, 16 * cus), per(steps, 8)), waves = 0, lds = 0;
+  for (;; ++spw) {
+    waves = per(steps, spw);
+    const int sums = waves * std::min(M, kGemvTokens) * 64;
+    lds = (kind == 1 ? std::max(sums, 4096) : sums) + waves * 2 * GemvStage<1>::kBytes;
+    if (lds <= kGemvLdsPerBlockMax) break;
+  }
+  const int rounds = per(load, std::max(1, std::min(kGemvLdsPerBlockMax / lds, 32 / waves)));
+  // Tables by who serves them: the L1s (up to 2048 rows, the main table of residual layers), an L2 next to the weights, an L2 that other layers' tables share.
+  struct { float start, round, step, lookups, block; } c =
+      kind == 0 ? table_rows <= 16384 ? decltype(c){2.50f, 0.59f, 0.619f, 0.444f, 0.144f} : decltype(c){3.26f, 0.33f, 0.803f, 0.471f, 0.150f}
+                : table_rows <= 2048    ? decltype(c){2.14f, 1.86f, 0.681f, 0.306f, 0.182f}
+                  : table_rows <= 8192  ? decltype(c){2.47f, 1.46f, 0.476f, 0.395f, 0.191f}
+                  : table_rows <= 16384 ? decltype(c){2.24f, 1.52f, 0.f, 0.586f, 0.265f}
+                                        : decltype(c){3.72f, 1.44f, 0.515f, 0.535f, 0.115f};
+  return c.start + (c.round + c.step * spw) * rounds + c.lookups * load * K / 256 + c.block * load;
 }
 }  // namespace npamd
 
@@ -466,31 +485,24 @@ extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int ta
   float blocks = gemv_blocks_us(kind, table_rows, M, N, K);
   const bool in_lds = kind == 0 && table_rows <= 4096;
   if (in_lds && table_rows > 16) blocks = fminf(blocks, plan_table_gemm(M, N, K, table_rows).us);  // up to 16 rows: indices of 4 bits
-  blocks = 1.03f * (blocks + gather);
-  const float weights = (float)N * K;
-  const bool gathers = kind < 4 && table_rows > (in_lds ? 4096 : 2048);  // of plain VQ: a large layer's decode keeps such a table in LDS
-  const float decode = 2.0f + fmaxf(gathers ? weights / 8 / 236e3f : 0.f, weights * 2 / 4.4e6f);
-  // The library's rate here is what it reaches, 1.25 PFLOP/s from 100 of its tiles on; below, with less of a risk in the other direction, as in npamd_dense_gemm_preferred.
+  // Near the line the blocks' figures are 3 % high at fewer tokens (2483 calls of 17 to 1024 tokens: 0.70 % lost in the mean so, with 1 0.81, with 1.03 1.04), and not past 512.
+  blocks = (M > 512 ? 1.f : 0.97f) * (blocks + gather);
+  // The decode, us: what it takes by itself and per million weights, behind it the product, and what K in parts takes there past the plan's figure (or less).  Fitted to the same calls
+  // as the blocks' figures, 0.1 to 45 million weights: within 3 to 5 % in the median, 10 % in nine of ten.
+  const float weights = 1e-6f * N * K;
+  const float decode = kind == 4 ? 2.4f + 0.26f * weights
+                     : kind == 8 ? 2.45f + 0.33f * weights
+                     : kind == 1 ? 2.8f + (table_rows <= 4096 ? 0.77f : 1.0f) * weights
+                                 : in_lds ? 2.1f + 0.0002f * table_rows + 0.30f * weights
+                                 : 2.2f + (table_rows <= 16384 ? 0.69f : 0.93f) * weights;
+  const float in_parts = kind == 4 ? 0.7f : in_lds ? 0.9f : kind == 0 && table_rows <= 16384 ? 0.f : kind == 8 ? -0.1f : -0.6f;
+  // The library's rate here is what it reaches, 1.25 PFLOP/s from 100 of its tiles on; below, with less of a risk in the other direction.
   const bool own = npamd_dense_gemm_preferred(M, N, K), many = ceil(M / 256.0) * ceil(N / 256.0) >= 100;
   const float library = many ? 5.f + 2e-9f * M * N * K / 1.25f : (float)library_us(M, N, K);
   const DensePlan p = plan_dense(M, N, K, 0, kDenseMaxSplits);
-  const float host = own ? (p.splits > 1 ? 10.3f : 6.8f) : 33.f;  // of two or three launches
-  // The plan's figures are of products one after the other.  Behind a decode they take a little more: with 0.6 to 0.9 us the line puts every call
-  // of 8 % and more that was measured (tests/test_blocks_line.py) on its side, and more with the sum of its parts as a third launch, but for int4 (product / blocks, us:
-  // int8 431 x 8960 at 390 tokens 21.0 / 17.4, 65536 rows 608 x 4096 at 43 11.7 / 8.8; int4 640 x 7552 at 510 19.7 / 23.3).  Not behind the lookups in
-  // memory of a middle-sized table or of shorter rows, nor behind a decode of codes of four to twelve steps (int4: to six): 65536 rows 320 x 1536 at 422
-  // 9.1 / 10.8, 16384 rows 272 x 8448 at 88 13.1 / 16.0, residual 10144 x 384 at 56 7.9 / 9.5, 576 x 1152 at 271 8.9 / 10.3, int8 2960 x 1664 at 97
-  // 10.8 / 11.9, int4 592 x 1280 at 776 9.6 / 10.3.
-  const bool no_more = kind >= 4 ? K > 768 && K <= (kind == 4 ? 1536 : 3072) : !in_lds && (K <= 3072 || (kind == 0 && table_rows <= 16384));
-  const float behind_decode = no_more ? 0.f : p.splits > 1 && kind != 4 ? 1.75f : 0.75f;
-  const float product = fmaxf(host, decode + (own ? p.us + behind_decode : library));
-  // What the blocks take past their estimate where the product is close: int4 of some steps on compute units that are full, and the second
-  // table of a residual layer whose first the L1s serve.  Decode + product / blocks: int4 8192 x 4096 at 160 tokens 35.5 / 42.0 (38.4 by the
-  // estimate), 592 x 1152 at 731 9.0 / 10.1; residual, 1000 rows, 4112 x 384 at 253 9.6 / 13.1, 2432 x 2048 at 158 13.3 / 16.7, 1904 x 256 at 523 7.7 / 9.9.
-  const int steps = (K + 255) / 256, load = ((N + 15) / 16 * ((M + kGemvTokens - 1) / kGemvTokens) + 255) / 256;
-  const float more = kind == 4 && steps > 4 && load >= 4 ? 0.03f * load * steps : kind == 1 && table_rows > 256 && table_rows <= 2048 ? fmaxf(0.f, 0.3f * load * steps - 1.5f) : 0.f;
-  if (!tile && !in_lds) return 1.03f * (gemv_blocks_long_rows_us(kind, table_rows, M, N, K) + gather + more) < product ? 1 : 0;
-  if (blocks + 1.03f * more >= product) return 0;
+  const float host = own ? (p.splits > 1 ? 10.3f : 7.0f) : 33.f;  // of two or three launches
+  const float product = fmaxf(host, decode + (own ? p.us + (p.splits > 1 ? in_parts : 0.f) : library));
+  if (blocks >= product) return 0;
   if (!tile || (in_lds && M > 256)) return 1;  // past 256 tokens such layers have no tile GEMM
   const int columns = (N + 63) / 64 * ((M + 383) / 384), chunks = K / 64;
   int splits = columns * 10 < 256 * 7 ? 256 / columns : 1;
