@@ -8,6 +8,11 @@ import torch
 from neuropress_amd.transforms.vq_packing import IndexPacking
 
 
+# The dense product's tiles (rows, columns) by their number in NPAMD_DENSE_TILE, as the plan's list has them (test_dense_plan.py).
+DENSE_TILES = {1: (32, 64), 2: (64, 64), 3: (64, 128), 4: (128, 128), 5: (160, 128), 6: (256, 128), 7: (192, 128), 8: (96, 128), 9: (160, 256),
+               10: (192, 256), 11: (256, 224), 12: (256, 256), 13: (96, 64), 14: (192, 192), 15: (64, 128)}  # fmt: skip
+
+
 def gen(seed: int) -> torch.Generator:
     return torch.Generator().manual_seed(seed)
 

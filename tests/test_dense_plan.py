@@ -1,16 +1,24 @@
 """What the dense product's plan chooses, host arithmetic."""
 
+import re
 import time
 
 import pytest
 
-from neuropress_amd import _lib
+from neuropress_amd import _lib, build
+from tests import cases
 
 
 @pytest.mark.parametrize("m,n,k,parts", [(548, 320, 9728, 7), (444, 352, 9856, 8), (601, 432, 9344, 6), (512, 512, 8192, 6)])
 def test_long_k_over_few_tiles(m, n, k, parts):
     """As many parts of K as make one round of 64 x 128 tiles, up to eight: the tile in two groups.  With wide tiles alone 5, 6, 3 and 4 parts, 8 to 15 % slower."""
     assert _lib.load().npamd_dense_gemm_workspace_bytes(m, n, k) == parts * m * n * 4
+
+
+def test_tests_know_every_tile():
+    source = (build.CSRC / "dense_gemm.hip").read_text()
+    rows = re.search(r"kDenseCost\[\] = \{\n(.*?)\n\};", source, re.S).group(1)
+    assert [tuple(map(int, m)) for m in re.findall(r"^\s+\{(\d+), (\d+),", rows, re.M)] == [cases.DENSE_TILES[i] for i in sorted(cases.DENSE_TILES)]
 
 
 # Products (tokens, rows, columns) that one of the two serves faster, by 3 % and more on both types; the last is one that no wide tile takes.

@@ -27,7 +27,7 @@ def dense(monkeypatch):
 
 
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("tile", range(9))
+@pytest.mark.parametrize("tile", [0, *cases.DENSE_TILES])
 def test_dense_product(gpu, dense, tile, act):
     from neuropress_amd import kernels
 

@@ -8,8 +8,7 @@ from tests import cases
 
 pytestmark = pytest.mark.gpu
 
-TILES = {2: (64, 64), 3: (64, 128), 4: (128, 128), 5: (160, 128), 6: (256, 128), 7: (192, 128), 8: (96, 128), 9: (160, 256),
-         10: (192, 256), 11: (256, 224), 12: (256, 256), 13: (96, 64), 14: (192, 192)}  # fmt: skip
+TILES = {number: tile for number, tile in cases.DENSE_TILES.items() if number not in (1, 15)}  # those are the other kernel's
 
 
 @pytest.fixture
@@ -75,3 +74,27 @@ def test_rows_past_a_product(gpu, tuned):
                                         torch.cuda.current_stream().cuda_stream) == 0  # fmt: skip
             assert torch.allclose(y[:m, :n].float(), x.float() @ w.float().T, rtol=2e-3, atol=2e-3)
             assert bool((y[m:] == 7).all()) and bool((y[:, n:] == 7).all()), (tile, n)
+
+
+def large(gpu, m, n, k, act, what):
+    """As `check`, on the GPU in float64."""
+    from neuropress_amd import kernels
+
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=gpu).to(act)
+    w = (torch.randn(n, k, generator=g, device=gpu) * 0.05).to(act)
+    y = kernels.dense_linear(x, w).double()
+    ref, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    tol = ref.abs() * 2.0 ** (-10 if act == torch.float16 else -7) + size * k * 2.0**-24
+    assert bool(((y - ref).abs() <= tol).all()), (what, m, n, k)
+
+
+@pytest.mark.parametrize("tile", sorted(TILES))
+def test_groups_of_row_tiles(gpu, tuned, tile):
+    """Units are counted down the columns of groups of row tiles: several groups, the last of them not full, of several columns, whole and in
+    parts of K.  Groups of 2048 rows (y not much longer than wide) and of four tiles (longer)."""
+    bm, bn = TILES[tile]
+    for splits in (1, 2, 3):
+        tuned(tile, splits)
+        large(gpu, 2048 // bm * bm * 2 + bm + 7, 3800, 256, torch.bfloat16, (tile, splits))
+        large(gpu, 4 * bm * 2 + bm + 9, 2 * bn + 5, 256, torch.float16, (tile, splits))
