@@ -257,9 +257,9 @@ int launch_dense_tile(DenseShape s, hipStream_t st) {
 // The tiles there are and what a launch on each costs, us: fixed + per round of workgroups + hypot(step time, bytes
 // loaded / rate), fitted to 700 shapes of 17 to 4096 rows, 256 to 14336 columns and K of 256 to 14336, fp16 and bf16 (the tile of least
 // estimate is 0.2 % slower than the best of them in the mean, 13 % at most; each tile is there because without it that is 0.4 to 7 % in the mean or 15 % and
-// more on some shape; estimates are within 4 to 9 %).  A round is one tile per compute unit of every die.  What the figures say: a tile of
-// 256 x 256 takes 0.85 us a 64-k step (2048 cycles of MFMAs, at the 1.8 to 2.0 GHz the chip runs at under them) and 7.7 us to start and end; all
-// of them together load at 14 to 36 TB/s from the L2s.
+// more on some shape; estimates are within 4 to 9 %).  A round is one tile per compute unit of every die.  The two legs of the hypot
+// are coefficients of the fit, no times of a unit: together a 64-k step of 256 x 256 on every compute unit takes 1.5 us (4096 x 4096 x 4096), of which its 2048 cycles of MFMAs are 1.0
+// to 1.2 at the 1.7 to 2.0 GHz that the chip runs at under them.
 struct DenseCost {
   int bm, bn, groups;
   float fixed, per_step, per_mb, per_round;
@@ -525,7 +525,8 @@ extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int ta
 // (median, quarters): rounds at least 0.98 full, 64 to 300 GFLOP 1.05 (1.03 to 1.06), to 1600 1.08, past that 1.13; 0.9 to 0.98 full, to 300 GFLOP 0.97 (0.87 to 1.04), to
 // 800 1.03 (0.92 to 1.08), to 1600 1.05, past that 1.08; 0.86 to 0.9 full, past 1600 GFLOP 1.11; less full 0.87 to 0.97 (the library is 10 % and more ahead on one in twenty of those, by
 // no size that tells which: 1024 x 9728 x 14336 239 / 299 us, 1024 x 13824 x 13824 479 / 327).  Rounds of exactly seven eighths are level up to 14336 columns and the library's by 7 % past them, unlike their
-// neighbours (4096 x 14336 x 4096 in bf16 331 to 336 / 336 to 341, fp16 348 to 351 / 352; 4096 x 11008 x 4096, 0.896 full, 405 / 262); so are both types.  Where K is short (512 to 768: 0.81 up to
+// neighbours (4096 x 14336 x 4096 a thousand in a row bf16 329 / 341, fp16 346 / 359, three after a pause 343 to 351 / 347 to 354;
+// 2048 x 14336 x 4096 170 / 174, 179 / 182 and 178 / 178; 4096 x 11008 x 4096, 0.896 full, 405 / 262); there is no difference between the types.  Where K is short (512 to 768: 0.81 up to
 // 64 GFLOP, 1.05 up to 300) or N no multiple of 8 (0.95 up to 300 GFLOP) the line is at 300.  Library / this, us: 4095 x 4096 x 4096 bf16 92.7 / 97.9, 8000 x 4096 x 14336 590 / 695,
 // 2842 x 64000 x 4992 1265 / 1652, 5000 x 128256 x 2048 1957 / 2282; 4096 x 6144 x 4096 174.5 / 177.6 and bf16 166.3 / 157.8, 1646 x 13120 x 11136 690 / 444.
 extern "C" int npamd_dense_gemm_preferred(int M, int N, int K) {

@@ -156,18 +156,18 @@ struct T2ProdVq16 {
 // spreads the reads of 32 columns over the banks.  Wave w decodes the operand pair J = w / 4 of column
 // tile w % 4: in step t the operands of step t + 1 are decoded from registers into the other W slot (ring
 // of two) between the MFMAs, and the bytes of step t + 2 read out of the ring, a barrier ahead of their
-// decoding so that it never waits for LDS.  A line whose last bytes were read in step t - 1 is fetched
-// over from step t on.  The arithmetic is the providers' (providers.hpp): bit for bit the one-pass decode.
+// decoding so that it never waits for LDS.  A line's place is fetched
+// over from behind the first barrier that every wave reaches after the last read of it (kLastRead, kRequest).  The arithmetic is the providers' (providers.hpp): bit for bit the one-pass decode.
 // ---------------------------------------------------------------------------------------------
 template <int ACT, int NBITS, bool ASYM, int MW>
 struct T2ProdQ {
   using P = typename std::conditional<NBITS == 4, Q4Provider<ACT, ASYM>, Q8Provider<ACT, ASYM>>::type;
   using Args = typename P::Args;
   static constexpr int kWRing = 2;
-  // Where the waves meet in a step (see the kernel): in front of its last k group where that is the faster way, us, at its end / inside, 14336 x 4096: fp16 int4 at 200 / 256
-  // / 512 tokens 41.1 / 41.2 / 66.4 and 39.7 / 40.0 / 64.3, int8 41.5 / 42.1 / 69.0 and 40.9 / 41.2 / 67.6; int8 on three row tiles, 300 / 384 tokens, bf16 56.7 / 54.9 and
-  // 55.5 / 54.6, with zero points 60.1 / 62.0 and 58.7 / 61.5, fp16 with zero points 61.6 / 62.2 and 61.4 / 61.9.  One row tile at 48 tokens, where half of the waves only decode,
-  // loses (int4 24.6 and 24.9, int8 23.3 and 24.2; at 128 29.0 and 28.0, 28.9 and 28.8), and a longer decode (bf16, zero points) on two
+  // Where the waves meet in a step (see the kernel): in front of its last k group where that is the faster way.  Ten layers of 2048 x 8192 to 28672 x 8192, time at its end / inside, mean
+  // (least to most): on two row tiles fp16 int4 at 200 / 256 / 512 tokens 1.018 / 1.017 / 1.020 (0.97 to 1.07), int8 1.008 / 1.006 / 1.015 (0.98 to 1.04); on three int8 at 300 / 384 tokens bf16
+  // 1.006 / 1.009 (0.99 to 1.04), with zero points 1.015 / 1.018 (0.98 to 1.06), fp16 with zero points 1.006 / 1.014 (0.98 to 1.05).  14336 x 4096, us: one row tile at 48 tokens, where half
+  // of the waves only decode, loses (int4 24.6 and 24.9, int8 23.3 and 24.2; at 128 29.0 and 28.0, 28.9 and 28.8), and a longer decode (bf16, zero points) on two
   // fills the time that is won: int4 bf16 at 256 / 512 40.2 / 63.2 and 40.2 / 63.8, int8 40.8 / 66.3 and 41.4 / 67.0; int4 on three 53.9 / 54.9 and 53.6 / 55.0.
   static constexpr bool kMeetsInside = MW == 2 ? ACT == NPAMD_F16 && !ASYM : MW == 3 && NBITS == 8 && (ACT == NPAMD_BF16 || ASYM);
   static constexpr int kHandoffBatch = 2;

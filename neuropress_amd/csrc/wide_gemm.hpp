@@ -3,10 +3,10 @@
 // A wave computes 16 MT x 16 NT of the block's tile (MFMA 16x16x32), at most 128 x 64 or 64 x 112: an operand then serves four to eight MFMAs, where waves of
 // 64 x 64 keep LDS as busy as the matrix pipes.  x and W come straight into LDS, rows of 128 bytes, a ring of steps of 64 k; half a step's operands are
 // read between the MFMAs of the half before, and a step's place is loaded again as soon as its second half is in registers: one barrier a step.
-// What bounds it, at 4096 x 14336 x 4096 (bf16, tiles of 256 x 224: 332 us, 1.45 PFLOP/s; the kernel before, 256 x 128 on MFMAs of 32x32x16, 422): the matrix pipes,
-// busy 85 % of the cycles the tiles run, and the power they draw, which holds the clock at 1.7 to 2.0 GHz; 6 us of each round of tiles are its
-// start and its end, half of that the result on its way to memory.
-// What counted, us of the same product: loads right behind the barrier into the place just read, instead of in front of the next one 415 -> 370; spread over 24 of
+// What bounds it, at 4096 x 14336 x 4096 (bf16, tiles of 256 x 224): the matrix pipes, busy 78 % of all cycles, and the power they draw, which holds the clock at
+// 1.7 to 2.0 GHz; 6 us of each round of tiles are its start and its end, half of that the result on its way to memory.  The time goes with the clock: 341 us (1.41 PFLOP/s) each
+// of a thousand in a row, 347 to 354 for three after a pause, 398 to 407 for thirty, the library's product 329, 343 to 351 and 390.
+// What counted, us of that product in one process (the kernel before, 256 x 128 on MFMAs of 32x32x16, 422 there, this one 332): loads right behind the barrier into the place just read, instead of in front of the next one 415 -> 370; spread over 24 of
 // the 64 MFMAs of a step, not one behind each 371 -> 363; 16x16x32 instead of 32x32x16, in as many cycles but less power 388 -> 352; a
 // tile width that fills the last round (256 x 224 for 256 x 256) 352 -> 337.  Tried without gain: four waves of 128 x 128 (one per SIMD: 354), steps of 32 k in
 // four or five places (half lines: 387), a block per compute unit that walks several tiles (358: its stores and the next tile's loads wait
