@@ -9,7 +9,7 @@
 // 32 x 64 in four groups of a wave is for what is left without a tile for every compute unit even at 64 x 64, or is a long chain of steps for few: 8 KiB of operands per
 // step on their way three steps deep (47 x 384 x 8320 unsplit 16.3 us, the library's product 19.0; 90 x 609 x 13312 28).  64 x 128 in two groups of
 // four waves is for long K over few tiles, next to parts of K over blocks: half as many steps one behind the other as in a part of a wide tile.  Decode + product, us, best of all wide
-// tiles and splits / this: 548 x 320 x 9728 20.0 / 17.6, 444 x 352 x 9856 19.7 / 17.2, 370 x 659 x 12800 28.9 / 26.6, 709 x 501 x 10880 30.7 / 25.3, 1160 x 403 x 10112 35.0 / 32.7.
+// tiles and splits / this: 548 x 320 x 9728 20.0 / 17.6, 444 x 352 x 9856 19.7 / 17.2, 370 x 659 x 12800 28.9 / 26.6, 601 x 432 x 9344 22.1 / 19.8.
 //
 // Long reductions over few output tiles leave most of the chip idle all the same, here as in the library.  There K is split over blocks
 // too (`splits` parts of equal length, give or take a step): every block stores its f32 tile to the workspace and splitk_reduce_kernel adds
@@ -279,7 +279,7 @@ constexpr DenseCost kDenseCost[] = {
     {256, 256, 1, 2.163f, 0.853f, 0.073f, 7.682f},
     {96, 64, 1, 1.473f, 0.198f, 0.038f, 2.770f},
     {192, 192, 1, 0.000f, 0.487f, 0.055f, 8.035f},
-    {64, 128, 2, 3.600f, 0.440f, 0.020f, 0.000f},  // the kernel above again; where the plan looks at it
+    {64, 128, 2, 2.000f, 0.400f, 0.040f, 0.000f},  // the kernel above again; where the plan looks at it
 };
 constexpr int kDenseTiles = sizeof(kDenseCost) / sizeof(kDenseCost[0]), kDenseTwoGroups = kDenseTiles - 1;
 
@@ -298,7 +298,7 @@ constexpr int64_t kDenseStrideMax = NPAMD_TILE_MAX_STRIDE;
 constexpr int kDenseMinSplitSteps = 4;  // 64-k steps of a part
 // What a split of this product adds: the reduction kernel and the gap in front of it, and its bytes, us and us per MB (200 shapes of
 // long K, 2 to 16 parts, within 1.4 us in the median).  A ninth part costs the sum another round trip of loads, some 4 us: by itself the plan takes no more than eight.
-constexpr float kDenseSplitFixed = 3.5f, kDenseSplitPerMb = 0.6f;
+constexpr float kDenseSplitFixed = 3.5f, kDenseSplitPerMb = 0.6f, kDenseTwoGroupsPerMb = 0.8f;  // that tile's parts leave a value at a time
 constexpr int kDensePlannedSplits = 8;
 // The same for the tile GEMM's (estimates of npamd_gemv_blocks_preferred).
 constexpr float kSplitFixed = 4.5f, kSplitPerMb = 0.45f;
@@ -313,9 +313,9 @@ void count_tiles(int M, int N, int64_t* tiles, std::index_sequence<I...>) {
   ((tiles[I] = (int64_t)((M - 1) / kDenseCost[I].bm + 1) * ((N - 1) / kDenseCost[I].bn + 1)), ...);
 }
 
-// The tile and split of least estimate.  64 x 128 in two groups is looked at in parts of one round, on up to 40 tiles of at least 320 rows and K from 5120 on: of 74 such
-// products that it takes, behind a decode, 46 are more than 3 % faster than without it (28 more than 8 %) and 17 slower (5), 4.5 % in the mean; with more tiles, on fewer rows, or whole,
-// it loses more calls than it gains.  The wide tiles address their part of the result with 31 bits: with rows of y, or columns, that
+// The tile and split of least estimate.  64 x 128 in two groups is looked at in parts of one round where y has no fewer rows than columns, K from 4096 on; on wider products it loses as
+// many calls as it gains.  Against the tiles of 32x32x16 MFMAs that were here before, behind a decode: of 859 products of 150 to 1700 rows, 256 to 2200 columns and K of 4096 to 14336 55 take
+// more than 6 % longer (104 without the tile, 3 with the best of all tiles and parts) at 0.97 of the time in the mean, of 607 of any size up to 60 GFLOP 19 (47) at 0.914.  The wide tiles address their part of the result with 31 bits: with rows of y, or columns, that
 // could lie further apart than that, the other kernel's.
 //
 // Every call of the band is planned, one at a new token count three times: sizes are divided by constants, and the parts of a tile are looked at only while what they cannot go
@@ -330,7 +330,7 @@ DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits, bool 
   const int only = wide && forced_tile > 0 && forced_tile <= kDenseTiles ? forced_tile - 1 : wide ? -1 : 0;
   int64_t tiles[kDenseTiles];
   count_tiles(M, N, tiles, std::make_index_sequence<kDenseTiles>{});
-  const bool two_groups = only >= 0 || (tiles[kDenseTwoGroups] <= 40 && M >= 320 && steps >= 80);
+  const bool two_groups = only >= 0 || (M >= N && steps >= 64);
   auto load = [&](int i) { return (float)tiles[i] * steps * (kDenseCost[i].bm + kDenseCost[i].bn) * 128e-6f * kDenseCost[i].per_mb; };
   auto look = [&](int i, int splits, int part, float bytes, float sum) {
     const DenseCost& c = kDenseCost[i];
@@ -347,9 +347,10 @@ DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits, bool 
     for (int i = first; i < last; ++i) look(i, 1, steps, load(i), 0.f);
   if (forced_splits == 1 || max_splits < 2) return best;
   const float mb = 4e-6f * M * N;
+  auto per_mb = [](int i) { return i == kDenseTwoGroups ? kDenseTwoGroupsPerMb : kDenseSplitPerMb; };
   if (forced_splits > 1) {
     const int part = (steps + forced_splits - 1) / forced_splits;
-    for (int i = first; i < last; ++i) look(i, forced_splits, part, load(i), kDenseSplitFixed + kDenseSplitPerMb * mb * forced_splits);
+    for (int i = first; i < last; ++i) look(i, forced_splits, part, load(i), kDenseSplitFixed + per_mb(i) * mb * forced_splits);
     return best;
   }
   const int parts = std::min(std::min(max_splits, kDensePlannedSplits), steps / kDenseMinSplitSteps);
@@ -359,7 +360,7 @@ DensePlan plan_dense(int M, int N, int K, int forced_tile, int max_splits, bool 
     const DenseCost& c = kDenseCost[i];
     const float bytes = load(i), least = c.fixed + c.per_round + kDenseSplitFixed + fmaxf(bytes, tiles[i] * steps / (256.f * c.groups) * c.per_step);
     for (int splits = 2; splits <= parts && tiles[i] * splits <= 512; ++splits) {
-      const float sum = kDenseSplitPerMb * mb * splits;
+      const float sum = per_mb(i) * mb * splits;
       if (least + sum >= best.us) break;
       look(i, splits, part_of[splits], bytes, kDenseSplitFixed + sum);
     }
