@@ -416,7 +416,7 @@ extern "C" int npamd_dense_gemm_ragged(const void* x, int64_t ldx, const void* w
 // entry (table_gemm.hip), rather than to decode + product or the tile GEMM.  Up to a round or two of its blocks it is one short launch in the place of two that follow each
 // other; past that every block of tokens decodes its weights again.  All three are estimated.  kind: 0 VQ, 1 residual VQ, 4 and 8 bits
 // per weight.  Codebooks in memory and residual VQ are estimated as with indices that are all as frequent, and with the tables of four layers in turn.  Of 3015 calls
-// near the line, 17 to 4096 tokens, two fifths of them seen by no fit, those that it sends to the slower side lose 0.8 % in the mean of all, 111 of them more than 8 % (the line before this
+// near the line, 17 to 4096 tokens, two fifths of them seen by no fit, those that it sends to the slower side lose 0.8 % in the mean of all, 109 of them more than 8 % (the line before this
 // one, with corrections by format and range of K on the decode's side: 3.2 %, 416).  us, before / blocks, at 64 and 256 tokens: int4 512 x 512 6.9 / 4.0 and 6.9 / 4.1,
 // 1024 x 4096 11.8 / 6.4 and 13.3 / 9.5, 3072 x 3072 14.8 / 8.2; 256 rows 1024 x 1024 7.9 / 4.7 and 8.0 / 5.7, 2048 x 2048 10.4 / 5.7 and 11.1 / 11.2;
 // 4096 rows 1024 x 1024 8.1 / 4.7 and 8.1 / 6.6; 65536 rows 512 x 512 7.0 / 4.2 and 7.1 / 4.8, 1024 x 4096 13.2 / 10.0 and 16.5 / 24.8.
@@ -487,7 +487,8 @@ extern "C" int npamd_gemv_blocks_preferred(int M, int N, int K, int kind, int ta
   const bool in_lds = kind == 0 && table_rows <= 4096;
   if (in_lds && table_rows > 16) blocks = fminf(blocks, plan_table_gemm(M, N, K, table_rows).us);  // up to 16 rows: indices of 4 bits
   // Near the line the blocks' figures are 3 % high at fewer tokens (2483 calls of 17 to 1024 tokens: 0.70 % lost in the mean so, with 1 0.81, with 1.03 1.04), and not past 512.
-  blocks = (M > 512 ? 1.f : 0.97f) * (blocks + gather);
+  // Residual layers with large main tables: between indices that are all as frequent and Zipf's, whose lookups the blocks gain more from (mean loss, uniform / Zipf, 317 calls: 0.94 0.7 / 1.0 %, 0.97 0.5 / 1.7).
+  blocks = (kind == 1 && table_rows > 8192 ? 0.94f : M > 512 ? 1.f : 0.97f) * (blocks + gather);
   // The decode, us: what it takes by itself and per million weights, behind it the product, and what K in parts takes there past the plan's figure (or less).  Fitted to the same calls
   // as the blocks' figures, 0.1 to 45 million weights: within 3 to 5 % in the median, 10 % in nine of ten.
   const float weights = 1e-6f * N * K;
